@@ -384,7 +384,7 @@ def make_rwkv7(dev, fp32=False):
         fwd()
         bwd()
 
-    chunked = not fp32 and ALGO == "chunked"
+    chunked = fp32 or ALGO == "chunked"                            # the fp32 entry points know no other kernels
     kernels = [("rwkv7c_fwd x4 (T=1024 each)" if chunked else "rwkv7_fwd x4 (T=1024 each)", fwd, 7 * eb * C * tok),
                ("rwkv7c_bwd x4" if chunked else "rwkv7_bwd x4", bwd, 13 * eb * C * tok)]
 

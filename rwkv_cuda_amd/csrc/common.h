@@ -177,11 +177,11 @@ int launch_wkv5_bwd_b_split(hipStream_t st, int cross, int B, int T, int C, int 
                             const uint16_t* v, const float* ew, const uint16_t* u, const uint16_t* gy, float* gk32, float* gv32,
                             float* gw32, const float* rdr);
 
-// rwkv7_chunk.hip: chunked rwkv7 kernels (bf16 I/O); s0, sT, dsT, ds0 may be null
-int launch7c_fwd(hipStream_t st, int B, int T, int H, const float* s0, const uint16_t* r, const uint16_t* w, const uint16_t* k,
-                 const uint16_t* v, const uint16_t* a, const uint16_t* b, uint16_t* y, float* sT, float* s, float* sa);
-int launch7c_bwd(hipStream_t st, int B, int T, int H, const uint16_t* r, const uint16_t* w, const uint16_t* k, const uint16_t* v,
-                 const uint16_t* a, const uint16_t* b, const uint16_t* dy, const float* dsT, const float* s, const float* sa,
-                 float* ds0, uint16_t* dr, uint16_t* dw, uint16_t* dk, uint16_t* dv, uint16_t* da, uint16_t* db);
+// rwkv7_chunk.hip: chunked rwkv7 kernels (r..b, y, dy, dr..db are bf16 or, with f32, float); s0, sT, dsT, ds0 may be null
+int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0, const void* r, const void* w, const void* k,
+                 const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa);
+int launch7c_bwd(hipStream_t st, bool f32, int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
+                 const void* a, const void* b, const void* dy, const float* dsT, const float* s, const float* sa,
+                 float* ds0, void* dr, void* dw, void* dk, void* dv, void* da, void* db);
 
 }  // namespace rwkv

@@ -26,6 +26,9 @@
 //            dw_raw = G W_SCALE sig (1 - sig);  P at the end of the call = sum_i dsT o S_T.
 // Every product is an fp32 matrix instruction (no operand is rounded below fp32), so the fp32 outputs sT, ds0 and the
 // saved sa keep the accuracy class of the reference's fp32 recurrence; the bf16 outputs are rounded once at the store.
+// The fp32 mode is therefore the same kernel with fp32 loads and stores (B8 T1024 C4096, forward + backward: 1.20 ms, the
+// step-by-step recurrence on the vector units took 1.94); both are bound by the fp32 matrix pipe and the issue port it shares
+// with the vector instructions of the other two waves of a SIMD.
 //
 // One workgroup of four waves per (batch, head).  A 16x16x4 fp32 matrix instruction takes A[row = lane & 15][k = lane >> 4],
 // B[k = lane >> 4][col = lane & 15] and leaves D[row = 4 (lane >> 4) + v][col = lane & 15] in register v.  The state is
@@ -55,6 +58,8 @@ DEVINL f32x4 ld4(const float* p) { const float4 x = *reinterpret_cast<const floa
 DEVINL void st4(float* p, const f32x4& x) { *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]); }
 constexpr f32x4 ZERO4 = {0.f, 0.f, 0.f, 0.f};
 
+// Element pointers are typed for the bf16 mode; the fp32 mode (the reference's -D_FP32_ build) keeps float pointers in the
+// same fields and its instantiations (F32 = true) read and write them as such.
 struct Args7c {
     int T, H;
     const uint16_t *r, *w, *k, *v, *a, *b, *dy;
@@ -64,6 +69,13 @@ struct Args7c {
     float* s;     // [B,H,T/16][i][j]: state entering each chunk
     float* sa;    // [B,T,H,N]: U
 };
+
+// element base + o as it comes from memory, and its value
+template <bool F32> DEVINL uint32_t ld_raw(const uint16_t* p, size_t base, uint32_t o) {
+    if constexpr (F32) return (reinterpret_cast<const uint32_t*>(p) + base)[o];
+    else return (p + base)[o];
+}
+template <bool F32> DEVINL float widen(uint32_t x) { return F32 ? __uint_as_float(x) : bf2f(static_cast<uint16_t>(x)); }
 
 // the value a lane group g takes from four candidates (register index that depends on the lane group)
 DEVINL float by_group(int g, float x0, float x1, float x2, float x3) { return g == 0 ? x0 : (g == 1 ? x1 : (g == 2 ? x2 : x3)); }
@@ -162,6 +174,7 @@ struct SmemCF {
     float d1[N], dec[N];
 };
 
+template <bool F32>
 __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
     __shared__ SmemCF S;
     const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
@@ -183,7 +196,8 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const size_t o = ((tok0 + static_cast<size_t>(c) * CL + 4 * q + e) * H + h) * N + lane;
-            nx[0][e] = p.w[o]; nx[1][e] = p.r[o]; nx[2][e] = p.k[o]; nx[3][e] = p.v[o]; nx[4][e] = p.a[o]; nx[5][e] = p.b[o];
+            nx[0][e] = ld_raw<F32>(p.w, o, 0); nx[1][e] = ld_raw<F32>(p.r, o, 0); nx[2][e] = ld_raw<F32>(p.k, o, 0);
+            nx[3][e] = ld_raw<F32>(p.v, o, 0); nx[4][e] = ld_raw<F32>(p.a, o, 0); nx[5][e] = ld_raw<F32>(p.b, o, 0);
         }
     };
     fetch(0);
@@ -193,8 +207,9 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
         float lam[4], rr[4], kk[4], vv[4], aa[4], bb[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            lam[e] = W_SCALE * sigmoid_fast(bf2f(nx[0][e]));
-            rr[e] = bf2f(nx[1][e]); kk[e] = bf2f(nx[2][e]); vv[e] = bf2f(nx[3][e]); aa[e] = bf2f(nx[4][e]); bb[e] = bf2f(nx[5][e]);
+            lam[e] = W_SCALE * sigmoid_fast(widen<F32>(nx[0][e]));
+            rr[e] = widen<F32>(nx[1][e]); kk[e] = widen<F32>(nx[2][e]); vv[e] = widen<F32>(nx[3][e]);
+            aa[e] = widen<F32>(nx[4][e]); bb[e] = widen<F32>(nx[5][e]);
         }
         S.part[q][lane] = (lam[0] + lam[1]) + (lam[2] + lam[3]);
         if (c + 1 < nch) fetch(c + 1);
@@ -307,12 +322,13 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
             St[jt] = St[jt] * ld4(&S.dec[16 * jt + 4 * g]) + acc;
         }
         __syncthreads();
-        // ---------------------------------------------------------------- y (bf16) and sa = U (fp32) as whole rows
+        // ---------------------------------------------------------------- y and sa = U (fp32) as whole rows
         {
             const int t = tid >> 4, i4 = (tid & 15) * 4;
             const size_t o = ((tok0 + static_cast<size_t>(c) * CL + t) * H + h) * N + i4;
             const f32x4 y = ld4(&S.Yo[t][i4]);
-            *reinterpret_cast<uint2*>(p.y + o) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
+            if constexpr (F32) st4(reinterpret_cast<float*>(p.y) + o, y);
+            else *reinterpret_cast<uint2*>(p.y + o) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
             st4(p.sa + o, ld4(&S.Uo[t][i4]));
         }
     }
@@ -348,14 +364,17 @@ struct PlanesB {
     float d1[N], d2[N], dec[N];
 };
 constexpr int PK = 72;            // row stride (bf16 elements) of a parked output
+// fp32 outputs are not parked (twice the bytes would not fit the CU's LDS): the waves that finish them store them from
+// registers, 64 bytes of four rows per instruction.
+template <bool F32>
 struct SmemCB {
     PlanesB pl[2];
     float dW[CL][PS];
     float M[CL][TS];                                         // (I - AB)^{-1}
     float AB[CL][TS], AK[CL][TS], RB[CL][TS], RK[CL][TS];
     float dAB[CL][TS], dAK[CL][TS], dRB[CL][TS], dRK[CL][TS];
-    uint16_t park[5][CL][PK];                                // da, dr, db, dk, dw of the chunk whose phase 4 ran last, [token][channel]
-    uint16_t parkv[2][CL][PK];                               // dv, which is ready one visit earlier than the other five
+    uint16_t park[F32 ? 1 : 5][F32 ? 1 : CL][PK];                                // da, dr, db, dk, dw of the chunk whose phase 4 ran last, [token][channel]
+    uint16_t parkv[F32 ? 1 : 2][F32 ? 1 : CL][PK];                               // dv, which is ready one visit earlier than the other five
 };
 
 // tile[t][s] = sum_c X[t][c] Y[s][c] over 64 channels, masked to s < t (strict) or s <= t, stored as [t][s]
@@ -385,8 +404,8 @@ DEVINL void causal_tile(const float (*X)[PS], const float (*Y)[PS], float (*Tl)[
 
 // ---- role P: elementwise preparation (lane = channel, tokens 4 wp + e) one visit ahead, and the row-wise output stores
 struct Prep7 { uint32_t nx[7][4]; float nsa[4]; };
-struct Conv7 { float sg[4], uu[4]; uint32_t pk[6][2]; };      // sigmoid(w), sa, and r k v a b dy as bf16 pairs (tokens 2 z, 2 z + 1)
-DEVINL void bwd_fetch(const Args7c& p, Prep7& x, size_t row0, int wp, int lane, int H, int h) {
+template <bool F32> struct Conv7 { float sg[4], uu[4]; uint32_t pk[6][F32 ? 4 : 2]; };   // sigmoid(w), sa, and r k v a b dy: fp32, or bf16 pairs (tokens 2 z, 2 z + 1)
+template <bool F32> DEVINL void bwd_fetch(const Args7c& p, Prep7& x, size_t row0, int wp, int lane, int H, int h) {
     // wave-uniform base (scalar registers) plus a 32-bit lane offset: no 64-bit address per tensor and token in vector registers
     // (the lane part is hidden from the optimiser: it would otherwise turn every tensor-and-token address into a 64-bit
     // induction variable of the chunk loop, 64 vector registers)
@@ -396,32 +415,42 @@ DEVINL void bwd_fetch(const Args7c& p, Prep7& x, size_t row0, int wp, int lane, 
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const uint32_t o = static_cast<uint32_t>((4 * wp + e) * H) * N + lo;
-        x.nx[0][e] = (p.w + base)[o]; x.nx[1][e] = (p.r + base)[o]; x.nx[2][e] = (p.k + base)[o]; x.nx[3][e] = (p.v + base)[o];
-        x.nx[4][e] = (p.a + base)[o]; x.nx[5][e] = (p.b + base)[o]; x.nx[6][e] = (p.dy + base)[o];
+        const uint16_t* const src[7] = {p.w, p.r, p.k, p.v, p.a, p.b, p.dy};
+#pragma unroll
+        for (int k = 0; k < 7; ++k) x.nx[k][e] = ld_raw<F32>(src[k], base, o);
         x.nsa[e] = (p.sa + base)[o];
     }
 }
 // first half of the preparation: the decay of each token, this wave's decay sum; the other inputs are kept packed so that the
 // registers of x are free for the next fetch
-DEVINL void bwd_convert(PlanesB& O, const Prep7& x, Conv7& y, int wp, int lane) {
+template <bool F32> DEVINL void bwd_convert(PlanesB& O, const Prep7& x, Conv7<F32>& y, int wp, int lane) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) { y.sg[e] = sigmoid_fast(bf2f(x.nx[0][e])); y.uu[e] = x.nsa[e]; }
+    for (int e = 0; e < 4; ++e) { y.sg[e] = sigmoid_fast(widen<F32>(x.nx[0][e])); y.uu[e] = x.nsa[e]; }
 #pragma unroll
-    for (int k = 0; k < 6; ++k)
+    for (int k = 0; k < 6; ++k) {
+        if constexpr (F32) {
 #pragma unroll
-        for (int z = 0; z < 2; ++z) y.pk[k][z] = x.nx[k + 1][2 * z] | (x.nx[k + 1][2 * z + 1] << 16);
+            for (int e = 0; e < 4; ++e) y.pk[k][e] = x.nx[k + 1][e];
+        } else {
+#pragma unroll
+            for (int z = 0; z < 2; ++z) y.pk[k][z] = x.nx[k + 1][2 * z] | (x.nx[k + 1][2 * z + 1] << 16);
+        }
+    }
     O.part[wp][lane] = W_SCALE * ((y.sg[0] + y.sg[1]) + (y.sg[2] + y.sg[3]));
 }
 // second half (after a barrier): the in-chunk factors and every plane
-template <int E0 = 0, int E1 = 4>
-DEVINL void bwd_planes(PlanesB& O, const Conv7& y, int wp, int lane) {
+template <bool F32, int E0 = 0, int E1 = 4>
+DEVINL void bwd_planes(PlanesB& O, const Conv7<F32>& y, int wp, int lane) {
     float cm, cl;
     const float lam[4] = {W_SCALE * y.sg[0], W_SCALE * y.sg[1], W_SCALE * y.sg[2], W_SCALE * y.sg[3]};
     const Factors f = chunk_factors<E0, E1>(lam, O.part, wp, lane, cm, cl);
 #pragma unroll
     for (int e = E0; e < E1; ++e) {
         const int t = 4 * wp + e;
-        auto in = [&](int k) __attribute__((always_inline)) { return (e & 1) ? bf_hi(y.pk[k][e >> 1]) : bf_lo(y.pk[k][e >> 1]); };
+        auto in = [&](int k) __attribute__((always_inline)) {
+            if constexpr (F32) return __uint_as_float(y.pk[k][e]);
+            else return (e & 1) ? bf_hi(y.pk[k][e >> 1]) : bf_lo(y.pk[k][e >> 1]);
+        };
         const float rr = in(0), kk = in(1), vv = in(2), aa = in(3), bb = in(4), gg = in(5);
         O.Ap[t][lane] = aa * f.ea[e];
         O.Rp[t][lane] = rr * f.er[e];
@@ -440,8 +469,8 @@ DEVINL void bwd_planes(PlanesB& O, const Conv7& y, int wp, int lane) {
     }
     if (E0 == 0 && wp == 0) { O.d1[lane] = exp_acc(cm); O.d2[lane] = exp_acc(cl - cm); O.dec[lane] = exp_acc(cl); }
 }
-// da dr db dk dw (and dv) of one chunk leave their parking places as whole rows (256 threads, four channels each)
-DEVINL void bwd_store_rows(const SmemCB& S, int vbuf, const Args7c& p, size_t row0, int tp, int H, int h) {
+// bf16: da dr db dk dw (and dv) of one chunk leave their parking places as whole rows (256 threads, four channels each)
+DEVINL void bwd_store_rows(const SmemCB<false>& S, int vbuf, const Args7c& p, size_t row0, int tp, int H, int h) {
     const int t = tp >> 4, c4 = (tp & 15) * 4;
     const size_t base = (row0 * H + h) * N;
     uint32_t o = static_cast<uint32_t>(t * H) * N + c4;
@@ -452,33 +481,37 @@ DEVINL void bwd_store_rows(const SmemCB& S, int vbuf, const Args7c& p, size_t ro
     put(p.da, &S.park[0][t][c4]); put(p.dr, &S.park[1][t][c4]); put(p.db, &S.park[2][t][c4]); put(p.dk, &S.park[3][t][c4]);
     put(p.dw, &S.park[4][t][c4]); put(p.dv, &S.parkv[vbuf][t][c4]);
 }
-DEVINL void bwd_role_p(SmemCB& S, const Args7c& p, int tid, int w, size_t tok0, int nch, int H, int h) {
+// fp32: element [4 g + v][own] of the chunk whose first row is row0, straight to global memory
+DEVINL void store_f32(uint16_t* dst, size_t row0, int v, uint32_t lane_off, int H, int h, float x) {
+    reinterpret_cast<float*>(dst)[((row0 + v) * H + h) * N + lane_off] = x;
+}
+template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const Args7c& p, int tid, int w, size_t tok0, int nch, int H, int h) {
     const int lane = tid & 63, wp = w - 8, tp = tid - 8 * 64;
     // Raw rows are asked for two visits before they are converted (one visit, of which only two phases lie between the
     // request and the use, is less than the memory system takes under load: the A and B waves then waited for the P waves
     // at two of the three barriers of every visit).  Two register sets take turns; the chunk index is clamped instead of
     // the request being skipped, so that every visit issues the same loads and the waits count the same.
     Prep7 x[2];
-    Conv7 y;
+    Conv7<F32> y;
     auto row_of = [&](int visit) { const int c = nch - 1 - visit; return tok0 + static_cast<size_t>(c > 0 ? c : 0) * CL; };
-    bwd_fetch(p, x[0], row_of(0), wp, lane, H, h);
-    bwd_fetch(p, x[1], row_of(1), wp, lane, H, h);
+    bwd_fetch<F32>(p, x[0], row_of(0), wp, lane, H, h);
+    bwd_fetch<F32>(p, x[1], row_of(1), wp, lane, H, h);
     bwd_convert(S.pl[0], x[0], y, wp, lane);          // visit 0, before the loop
-    bwd_fetch(p, x[0], row_of(2), wp, lane, H, h);
+    bwd_fetch<F32>(p, x[0], row_of(2), wp, lane, H, h);
     __syncthreads();
-    bwd_planes(S.pl[0], y, wp, lane);
+    bwd_planes<F32>(S.pl[0], y, wp, lane);
     __syncthreads();
     auto visit = [&](const int i, auto Z) __attribute__((always_inline)) {     // visit i is chunk nch - 1 - i
         constexpr int z = decltype(Z)::value;        // the set that holds visit i + 1
         const bool next = i + 1 < nch;
         if (next) bwd_convert(S.pl[(i + 1) & 1], x[z], y, wp, lane);
-        bwd_fetch(p, x[z], row_of(i + 3), wp, lane, H, h);
+        bwd_fetch<F32>(p, x[z], row_of(i + 3), wp, lane, H, h);
         __syncthreads();
         // the planes of two of this wave's four tokens in phase 2, the other two in phase 3, in which these waves used to idle
         // while everybody waited for them in phase 2 (nothing reads these planes before the next visit)
-        if (next) bwd_planes<0, 2>(S.pl[(i + 1) & 1], y, wp, lane);
+        if (next) bwd_planes<F32, 0, 2>(S.pl[(i + 1) & 1], y, wp, lane);
         __syncthreads();
-        if (next) bwd_planes<2, 4>(S.pl[(i + 1) & 1], y, wp, lane);
+        if (next) bwd_planes<F32, 2, 4>(S.pl[(i + 1) & 1], y, wp, lane);
         __syncthreads();
     };
     for (int i = 0; i < nch; i += 2) {
@@ -486,10 +519,10 @@ DEVINL void bwd_role_p(SmemCB& S, const Args7c& p, int tid, int w, size_t tok0, 
         if (i + 1 < nch) visit(i + 1, std::integral_constant<int, 0>{});
     }
     __syncthreads();                                 // role B finishes the last chunk
-    bwd_store_rows(S, (nch - 1) & 1, p, tok0, tp, H, h);
+    if constexpr (!F32) bwd_store_rows(S, (nch - 1) & 1, p, tok0, tp, H, h);
 }
 
-DEVINL void bwd_role_a(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
+template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
     const int lane = tid & 63, q = w & 3, l16 = lane & 15, g = lane >> 4;
     const int own = 16 * q + l16;                    // value channel i of this lane's column
     f32x4 dS[4];                                     // dS[i = own][j = 16 jt + 4 g + v]
@@ -541,7 +574,10 @@ DEVINL void bwd_role_a(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
 #pragma unroll
             for (int v = 0; v < 4; ++v) dV = mm(S.RK[4 * g + v][l16], dyop[v], dV);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) S.parkv[i & 1][4 * g + v][own] = f2bf(dV[v]);
+            for (int v = 0; v < 4; ++v) {
+                if constexpr (F32) store_f32(p.dv, tok0 + static_cast<size_t>(nch - 1 - i) * CL, v, static_cast<uint32_t>(4 * g * H) * N + own, H, h, dV[v]);
+                else S.parkv[i & 1][4 * g + v][own] = f2bf(dV[v]);
+            }
 #pragma unroll
             for (int jt = 0; jt < 4; ++jt) {
                 f32x4 acc = accA[jt];
@@ -553,13 +589,15 @@ DEVINL void bwd_role_a(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
         __syncthreads();
         // ---------------------------------------------------------------- phase 3: dAB, dAK (they need dW)
         if (q < 2) causal_tile(S.dW, q == 0 ? O.U : O.V, q == 0 ? S.dAB : S.dAK, true, l16, g);
-        else if (i > 0) {
+        else if constexpr (!F32) {
+          if (i > 0) {
             // The two waves without a tile here carry the finished rows of the visit before to global memory (parked by the
             // B waves in phase 1, dv by this role one visit earlier; both stay as they are until the next visit): the P
             // waves, for which this was a third of a phase that everybody waits for, keep to loads.
             const int tp = tid - 2 * 64;
             bwd_store_rows(S, (i - 1) & 1, p, tok0 + static_cast<size_t>(nch - i) * CL, tp, H, h);
             bwd_store_rows(S, (i - 1) & 1, p, tok0 + static_cast<size_t>(nch - i) * CL, tp + 128, H, h);
+          }
         }
         __syncthreads();
     }
@@ -571,7 +609,7 @@ DEVINL void bwd_role_a(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
     }
 }
 
-DEVINL void bwd_role_b(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, int nch) {
+template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
     const int lane = tid & 63, q = w & 3, l16 = lane & 15, g = lane >> 4;
     const int own = 16 * q + l16;                    // key channel j of this lane's column
     f32x4 dS[4], S0b[4];                             // dS, S0 at [i = 16 ib + 4 g + v][j = own]
@@ -591,8 +629,14 @@ DEVINL void bwd_role_b(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
     };
     float Pj = 0.f;                                  // P at the end of the chunk whose phase 4 comes next
     f32x4 xA = ZERO4, xR = ZERO4, xB = ZERO4, xK = ZERO4;     // state parts of dA', dR', dB', dK', carried into the next visit's phase 1
-    // tile parts, scaling, decay gradient of the chunk whose planes are O; results parked as bf16
-    auto finish = [&](const PlanesB& O) __attribute__((always_inline)) {
+    // tile parts, scaling, decay gradient of the chunk whose planes are O and whose first row is row0; results parked as bf16
+    auto finish = [&](const PlanesB& O, const size_t row0) __attribute__((always_inline)) {
+        uint32_t lo = static_cast<uint32_t>(4 * g * H) * N + own;
+        asm volatile("" : "+v"(lo));
+        auto put = [&](const int k, uint16_t* dst, const int v, const float x) __attribute__((always_inline)) {
+            if constexpr (F32) store_f32(dst, row0, v, lo, H, h, x);
+            else S.park[k][4 * g + v][own] = f2bf(x);
+        };
         const float d1j = O.d1[own], d2j = O.d2[own];
         f32x4 bp, kp, ap, rp;                        // planes at [s or t = 4 g + v][j]
 #pragma unroll
@@ -617,10 +661,10 @@ DEVINL void bwd_role_b(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
             const float dBp = fmaf(d2j, xB[v], tB[v]), dKp = fmaf(d2j, xK[v], tK[v]);
             const float ea = O.EA[t][own], er = O.ER[t][own];
             const float eb = __frcp_rn(er);
-            S.park[0][t][own] = f2bf(dAp * ea);
-            S.park[1][t][own] = f2bf(dRp * er);
-            S.park[2][t][own] = f2bf(dBp * eb);
-            S.park[3][t][own] = f2bf(dKp * eb);
+            put(0, p.da, v, dAp * ea);
+            put(1, p.dr, v, dRp * er);
+            put(2, p.db, v, dBp * eb);
+            put(3, p.dk, v, dKp * eb);
             ada[v] = ap[v] * dAp;
             del[v] = fmaf(rp[v], dRp, -fmaf(bp[v], dBp, kp[v] * dKp));      // r dr - b db - k dk
             dwf[v] = O.DWF[t][own];
@@ -633,7 +677,7 @@ DEVINL void bwd_role_b(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
         for (int v = 3; v >= 0; --v) {
             const float G = Pn + del[v];
             Pn = G + ada[v];
-            S.park[4][4 * g + v][own] = f2bf(G * dwf[v]);
+            put(4, p.dw, v, G * dwf[v]);
         }
         Pj = __shfl(Pn, l16, 64);                    // lane group 0 holds P at the start of the chunk
     };
@@ -644,7 +688,7 @@ DEVINL void bwd_role_b(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
         const int c = nch - 1 - i;
         const PlanesB& O = S.pl[i & 1];
         // ---------------------------------------------------------------- phase 1: finish the previous visit's chunk
-        if (i > 0) finish(S.pl[(i - 1) & 1]);
+        if (i > 0) finish(S.pl[(i - 1) & 1], tok0 + static_cast<size_t>(c + 1) * CL);
         __syncthreads();
         // ---------------------------------------------------------------- phase 2: dY S0, U dS, V dS; dRB, dRK
         if (i == 0 && p.dsT != nullptr) {
@@ -705,47 +749,56 @@ DEVINL void bwd_role_b(SmemCB& S, const Args7c& p, int tid, int w, size_t bh, in
         }
         __syncthreads();
     }
-    finish(S.pl[(nch - 1) & 1]);
+    finish(S.pl[(nch - 1) & 1], tok0);
     __syncthreads();
 }
 
+template <bool F32>
 __global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c p) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    SmemCB& S = *reinterpret_cast<SmemCB*>(smem_raw);
+    SmemCB<F32>& S = *reinterpret_cast<SmemCB<F32>*>(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x, b = blockIdx.y;
     const size_t bh = static_cast<size_t>(b) * p.H + h;
     const size_t tok0 = static_cast<size_t>(b) * p.T;
     const int nch = p.T / CL;
     if (w < 4) bwd_role_a(S, p, tid, w, bh, nch, tok0, p.H, h);
-    else if (w < 8) bwd_role_b(S, p, tid, w, bh, nch);
+    else if (w < 8) bwd_role_b(S, p, tid, w, bh, nch, tok0, p.H, h);
     else bwd_role_p(S, p, tid, w, tok0, nch, p.H, h);
+}
+
+const uint16_t* el(const void* p) { return static_cast<const uint16_t*>(p); }
+uint16_t* el(void* p) { return static_cast<uint16_t*>(p); }
+
+template <bool F32> int start_bwd(hipStream_t st, int B, int H, const Args7c& p) {
+    static_assert(sizeof(SmemCB<F32>) <= 160 * 1024, "the backward's LDS must fit one CU");
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_bwd<F32>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       static_cast<int>(sizeof(SmemCB<F32>)));
+    if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
+    hipLaunchKernelGGL(rwkv7c_bwd<F32>, dim3(H, B), dim3(NTB), sizeof(SmemCB<F32>), st, p);
+    return launch_status();
 }
 
 }  // namespace
 
-
-int launch7c_fwd(hipStream_t st, int B, int T, int H, const float* s0, const uint16_t* r, const uint16_t* w, const uint16_t* k,
-                 const uint16_t* v, const uint16_t* a, const uint16_t* b, uint16_t* y, float* sT, float* s, float* sa) {
+int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0, const void* r, const void* w, const void* k,
+                 const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa) {
     Args7c p{};
-    p.T = T; p.H = H; p.s0 = s0; p.r = r; p.w = w; p.k = k; p.v = v; p.a = a; p.b = b; p.y = y; p.sT = sT; p.s = s; p.sa = sa;
-    hipLaunchKernelGGL(rwkv7c_fwd, dim3(H, B), dim3(NT), 0, st, p);
+    p.T = T; p.H = H; p.s0 = s0; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b); p.y = el(y);
+    p.sT = sT; p.s = s; p.sa = sa;
+    if (f32) hipLaunchKernelGGL(rwkv7c_fwd<true>, dim3(H, B), dim3(NT), 0, st, p);
+    else hipLaunchKernelGGL(rwkv7c_fwd<false>, dim3(H, B), dim3(NT), 0, st, p);
     return launch_status();
 }
 
-int launch7c_bwd(hipStream_t st, int B, int T, int H, const uint16_t* r, const uint16_t* w, const uint16_t* k, const uint16_t* v,
-                 const uint16_t* a, const uint16_t* b, const uint16_t* dy, const float* dsT, const float* s, const float* sa,
-                 float* ds0, uint16_t* dr, uint16_t* dw, uint16_t* dk, uint16_t* dv, uint16_t* da, uint16_t* db) {
+int launch7c_bwd(hipStream_t st, bool f32, int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
+                 const void* a, const void* b, const void* dy, const float* dsT, const float* s, const float* sa,
+                 float* ds0, void* dr, void* dw, void* dk, void* dv, void* da, void* db) {
     Args7c p{};
-    p.T = T; p.H = H; p.r = r; p.w = w; p.k = k; p.v = v; p.a = a; p.b = b; p.dy = dy; p.dsT = dsT;
+    p.T = T; p.H = H; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b); p.dy = el(dy); p.dsT = dsT;
     p.s = const_cast<float*>(s); p.sa = const_cast<float*>(sa); p.ds0 = ds0;
-    p.dr = dr; p.dw = dw; p.dk = dk; p.dv = dv; p.da = da; p.db = db;
-    static_assert(sizeof(SmemCB) <= 160 * 1024, "the backward's LDS must fit one CU");
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_bwd), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       static_cast<int>(sizeof(SmemCB)));
-    if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
-    hipLaunchKernelGGL(rwkv7c_bwd, dim3(H, B), dim3(NTB), sizeof(SmemCB), st, p);
-    return launch_status();
+    p.dr = el(dr); p.dw = el(dw); p.dk = el(dk); p.dv = el(dv); p.da = el(da); p.db = el(db);
+    return f32 ? start_bwd<true>(st, B, H, p) : start_bwd<false>(st, B, H, p);
 }
 
 }  // namespace rwkv
