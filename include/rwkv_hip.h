@@ -238,6 +238,35 @@ int rwkv_wkv5a_backward_ex(void* stream, int B, int T, int C, int H,
                         float* gr, float* gk, float* gv, float* gw1, float* gu1, float* gw2, float* gu2, unsigned flags);
 
 /* ---------------------------------------------------------------------------------------
+ * wkv5 fp32 and wkv5a as everything the wrapper classes do in two calls (wkv5/run.py:469-504, wkv5a/run.py:100-154), head
+ * size 64: raw w in, gradients of the raw parameters summed over the batch out (gw, gu [C]).  Chunked kernels on the fp32
+ * matrix cores: one forward, one reverse sweep.
+ *   `saved` (*_saved_bytes; 0 for another head size, which these entry points refuse with RWKV_ERR_SHAPE): the forward keeps
+ *   the state entering every fourth (wkv5a: second) chunk of 16 tokens for the backward of the same step; NULL for a forward
+ *   without a backward.  `workspace` (*_backward_workspace_bytes): per-batch rows of the parameter gradients.
+ * ------------------------------------------------------------------------------------- */
+size_t rwkv_wkv5f32s_saved_bytes(int B, int T, int C, int H);
+int rwkv_wkv5f32s_forward(void* stream, int B, int T, int C, int H,
+                          const float* r, const float* k, const float* v, const float* w, const float* u, float* y,
+                          void* saved, size_t saved_bytes);
+size_t rwkv_wkv5f32s_backward_workspace_bytes(int B, int T, int C, int H);
+int rwkv_wkv5f32s_backward(void* stream, int B, int T, int C, int H,
+                           const float* r, const float* k, const float* v, const float* w, const float* u, const float* gy,
+                           float* gr, float* gk, float* gv, float* gw, float* gu,
+                           const void* saved, size_t saved_bytes, void* workspace, size_t workspace_bytes);
+size_t rwkv_wkv5as_saved_bytes(int B, int T, int C, int H);
+int rwkv_wkv5as_forward(void* stream, int B, int T, int C, int H,
+                        const float* r, const float* k, const float* v,
+                        const float* w1, const float* u1, const float* w2, const float* u2, float* y,
+                        void* saved, size_t saved_bytes);
+size_t rwkv_wkv5as_backward_workspace_bytes(int B, int T, int C, int H);
+int rwkv_wkv5as_backward(void* stream, int B, int T, int C, int H,
+                         const float* r, const float* k, const float* v,
+                         const float* w1, const float* u1, const float* w2, const float* u2, const float* gy,
+                         float* gr, float* gk, float* gv, float* gw1, float* gu1, float* gw2, float* gu2,
+                         const void* saved, size_t saved_bytes, void* workspace, size_t workspace_bytes);
+
+/* ---------------------------------------------------------------------------------------
  * RWKV-6 wkv, bf16 I/O, per-token decay.  Replaces cuda_forward / cuda_backward of
  * wkv6/cuda/wkv6_op.cpp:5-6 (kernels: wkv6_cuda_v1.cu:6-223).
  *   w = ew = -exp(w_raw), fp32 [B,T,C] (wkv6/run.py:147); the kernel applies exp(ew).

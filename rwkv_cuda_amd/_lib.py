@@ -18,7 +18,7 @@ _INCLUDE = os.path.join(_ROOT, "include")
 LIB_PATH = os.path.join(_HERE, "librwkv_hip.so")
 HASH_PATH = LIB_PATH + ".srchash"        # digest of the sources the library was built from (content, not mtime)
 
-SOURCES = ["abi.hip", "wkv56.hip", "wkv6_fwd.hip", "wkv6_bwd_a.hip", "wkv6_bwd_b.hip", "wkv6_fwd_f.hip", "wkv6_bwd_f.hip", "wkv4.hip", "timex.hip", "rwkv7.hip", "rwkv7_chunk.hip"]
+SOURCES = ["abi.hip", "wkv56.hip", "wkv6_fwd.hip", "wkv6_bwd_a.hip", "wkv6_bwd_b.hip", "wkv6_fwd_f.hip", "wkv6_bwd_f.hip", "wkv4.hip", "timex.hip", "wkv5_f32.hip", "rwkv7.hip", "rwkv7_chunk.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -156,6 +156,14 @@ SIGNATURES = {
     "rwkv_wkv5a_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 8),
     "rwkv_wkv5a_backward": (_I, [_P, _I, _I, _I, _I] + [_P] * 17),
     "rwkv_wkv5a_backward_ex": (_I, [_P, _I, _I, _I, _I] + [_P] * 17 + [_U]),
+    "rwkv_wkv5f32s_saved_bytes": (_Z, [_I, _I, _I, _I]),
+    "rwkv_wkv5f32s_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 6 + [_P, _Z]),
+    "rwkv_wkv5f32s_backward_workspace_bytes": (_Z, [_I, _I, _I, _I]),
+    "rwkv_wkv5f32s_backward": (_I, [_P, _I, _I, _I, _I] + [_P] * 11 + [_P, _Z, _P, _Z]),
+    "rwkv_wkv5as_saved_bytes": (_Z, [_I, _I, _I, _I]),
+    "rwkv_wkv5as_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 8 + [_P, _Z]),
+    "rwkv_wkv5as_backward_workspace_bytes": (_Z, [_I, _I, _I, _I]),
+    "rwkv_wkv5as_backward": (_I, [_P, _I, _I, _I, _I] + [_P] * 15 + [_P, _Z, _P, _Z]),
     "rwkv_wkv6_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 6),
     "rwkv_wkv6_forward_ex": (_I, [_P, _I, _I, _I, _I] + [_P] * 6 + [_U]),
     "rwkv_wkv6_backward_workspace_bytes": (_Z, [_I, _I, _I, _I]),

@@ -1,0 +1,780 @@
+// wkv5 and wkv5a, fp32 I/O, head size 64, in CHUNKED form on the fp32 matrix cores (gfx950, v_mfma_f32_16x16x4_f32).
+//
+// Step form (wkv5/run.py:231-262, wkv5a/run.py:260-289), one head, S[i][j] (i value channel, j key channel):
+//     y_t[i] = sum_j r_t[j] (S_t[i][j] + (u1[j] + u2[i]) k_t[j] v_t[i])       S_{t+1} = S_t o W + v_t k_t^T
+// with W[i][j] = e^{l1[j] + l2[i]}, l = -exp(w_raw); wkv5 has l2 = 0 and u2 = 0 (TWO = false).  The decays are constant in
+// time, so a power that a token of a chunk (L = 16 tokens, local t = 0..15) needs is the same in every chunk: all of them are
+// made once per workgroup and live in registers, each exact to fp32 rounding.  S0 is the state entering the chunk, D the
+// gradient of the state leaving it; o1 = e^{l1}, o2 = e^{l2}; m a reference token (8, the middle, unless the decay is strong):
+//     A[t][s]  = sum_j (r_t o1^{t-m}) (k_s o1^{m-1-s})     B[t][s] = sum_i (gy_t o2^{t-m}) (v_s o2^{m-1-s})          s < t
+//     y_t   = o2^t (r_t o1^t) S0^T        + o2^{t-m} sum_s A[t][s] (v_s o2^{m-1-s})      + bonus
+//     dr_t  = o1^t (gy_t o2^t) S0         + o1^{t-m} sum_s B[t][s] (k_s o1^{m-1-s})      + bonus
+//     dk_t  = o1^{15-t} (v_t o2^{15-t}) D + o1^{m-1-t} sum_s B[s][t] (r_s o1^{s-m})      + bonus
+//     dv_t  = o2^{15-t} (k_t o1^{15-t}) D^T + o2^{m-1-t} sum_s A[s][t] (gy_s o2^{s-m})   + bonus
+//     S_L   = S0 o W^16 + sum_s (v_s o2^{15-s})(k_s o1^{15-s})^T         D_0 = D o W^16 + sum_t (gy_t o2^t)(r_t o1^t)^T
+// Decay gradient: a term (source s, sink t) of the output carries e^{l (t-1-s)}, so d/dl1[j] counts, for every such pair,
+// the tokens strictly between s and t.  Cut at the chunk borders that is a sum of four kinds of products without any
+// cancellation (the difference form used under bf16 outputs loses a digit per decade of T, which fp32 outputs show):
+//     both in the chunk      sum_t r_t o1^{t-m} sum_s (t-1-s) B[t][s] (k_s o1^{m-1-s})
+//     source before, sink in sum_t t r_t dr_t(S0 part)                  source in, sink after  sum_s (15-s) k_s dk_s(D part)
+//     source before, sink after  16 sum_i S0 o W^16 o D
+// Two-sided, the last three are kept per state element (the two middle ones become products over the tokens) and summed
+// over i for l1 and over j for l2 at the end.
+//
+// Strong decays: with one reference in the middle a factor reaches e^{8 |l|}; beyond l = -7 (STRONG) the tiles take a
+// reference in the middle of each half (m = 4, 12) and a pair of tokens of different halves carries o1^8 in addition: a second
+// product for that quadrant, with o1^4 on either side (o1^8 itself may underflow where the whole term is one).  Below l = -17 a decay is taken as e^{-17} = 4e-8, half a unit of the fp32 sum it enters.
+//
+// What bounds it: the fp32 matrix pipe (32 clocks an instruction; 40 per wave and chunk forward, 116 per SIMD backward) and
+// HBM: every tensor crosses it once, plus a saved state every SEG chunks.  B8 T4096 C4096, forward + backward: see the
+// launchers below for what it measured.
+#include "common.h"
+
+namespace rwkv {
+namespace {
+
+constexpr int N = 64;
+constexpr int L = 16;
+constexpr int PS = 68;               // row stride (floats) of a [token][channel] plane
+constexpr int TS = 20;               // row stride (floats) of a 16 x 16 tile
+constexpr int NT = 512;              // forward: waves 0..3 products, 4..7 loads; backward: 0..3 key side, 4..7 value side and loads
+constexpr float STRONG = -7.f, LAM_MIN = -17.f;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+DEVINL f32x4 mm(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+DEVINL f32x4 ld4(const float* p) { const float4 x = *reinterpret_cast<const float4*>(p); return f32x4{x.x, x.y, x.z, x.w}; }
+DEVINL void st4(float* p, const f32x4& x) { *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]); }
+constexpr f32x4 ZERO4 = {0.f, 0.f, 0.f, 0.f};
+
+// states are saved for the backward at the start of every SEG-th chunk; the backward holds the states of a whole segment in
+// registers: 4 chunks one-sided, 2 where the per-element sums and the second side's powers take the room
+template <bool TWO> constexpr int SEG = TWO ? 2 : 4;
+
+struct ArgsC {
+    int T, C, H;
+    const float *r, *k, *v, *gy, *w, *u, *w2, *u2;      // w, w2 raw
+    float *y, *gr, *gk, *gv;
+    float *gw, *gu, *gw2, *gu2;                         // per-batch rows [B][C]
+    float* saved;                                       // [B*H][segments][i][j]
+};
+
+// e^{lam n} for a small integer n, exact to fp32 rounding: the product and the base-2 exponent carry their rounding errors along
+DEVINL float wpow(float lam, float n) {
+    constexpr float L2E_HI = 1.44269502162933349609f, L2E_LO = 1.92596299112661746e-8f, LN2 = 0.69314718055994530942f;
+    const float x = lam * n, lo = fmaf(lam, n, -x);
+    const float t = x * L2E_HI;
+    const float e = fmaf(x, L2E_HI, -t) + fmaf(x, L2E_LO, lo * L2E_HI);
+    const float y = __builtin_amdgcn_exp2f(t);
+    return fmaf(y, e * LN2, y);
+}
+template <int R> DEVINL float row_ror(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + R, 0xf, 0xf, true));
+}
+// sum over the 16 lanes of a row, in all of them
+DEVINL float row_sum(float x) {
+    x += row_ror<8>(x); x += row_ror<4>(x); x += row_ror<2>(x); x += row_ror<1>(x);
+    return x;
+}
+
+struct Head { float lam[N], lam2[N], u[N], u2[N], dec[N], dec2[N]; };
+
+// the head's parameters into LDS (by the first wave); every wave finds out for itself whether a decay is strong
+template <bool TWO> DEVINL bool head_setup(Head& hd, const ArgsC& p, int h, int tid) {
+    const int lane = tid & 63, c = h * N + lane;
+    const float l1 = -expf(p.w[c]), l2 = TWO ? -expf(p.w2[c]) : 0.f;
+    float mn = fminf(l1, l2);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o, 64));
+    if (tid < N) {
+        const float a = fmaxf(l1, LAM_MIN), b = fmaxf(l2, LAM_MIN);
+        hd.lam[lane] = a; hd.dec[lane] = wpow(a, L); hd.u[lane] = p.u[c];
+        hd.lam2[lane] = b; hd.dec2[lane] = wpow(b, L); hd.u2[lane] = TWO ? p.u2[c] : 0.f;
+    }
+    return __builtin_amdgcn_readfirstlane(mn < STRONG ? 1 : 0) != 0;
+}
+// reference token of token t
+DEVINL int ref(bool strong, int t) { return strong ? (t < 8 ? 4 : 12) : 8; }
+
+// One half (32 channels, the 16-channel blocks cb0 and cb0 + 1) of a causal tile sum_c X[t][c] Y[s][c], s < t, with the powers
+// cx (of t = l16) and cy (of s = l16) per channel block and register; w4: half of what pairs across the halves of a strong chunk carry.
+template <bool SCALED>
+DEVINL void half_tile(const float (*X)[PS], const float (*Y)[PS], float (*out)[TS], int cb0, const f32x4 (&cx)[2], const f32x4 (&cy)[2],
+                      const f32x4 (&w4)[2], bool strong, int l16, int g) {
+    f32x4 d[2] = {ZERO4, ZERO4};
+    f32x4 xa[2], ya[2];
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+        xa[z] = ld4(&X[l16][16 * (cb0 + z) + 4 * g]); ya[z] = ld4(&Y[l16][16 * (cb0 + z) + 4 * g]);
+        if constexpr (SCALED) { xa[z] *= cx[z]; ya[z] *= cy[z]; }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int z = 0; z < 2; ++z) d[z] = mm(xa[z][v], ya[z][v], d[z]);
+    f32x4 acc = d[0] + d[1];
+    if (SCALED && strong) {
+        f32x4 o = ZERO4;
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o = mm(xa[z][v] * w4[z][v], ya[z][v] * w4[z][v], o);
+        if (g >= 2 && l16 < 8) acc = o;
+    }
+    // acc[v] = tile[t = 4 g + v][s = l16]
+#pragma unroll
+    for (int v = 0; v < 4; ++v) out[4 * g + v][l16] = l16 < 4 * g + v ? acc[v] : 0.f;
+}
+// the powers half_tile takes for a side with log decays lam
+DEVINL void tile_powers(const float* lam, int cb0, bool strong, int l16, int g, f32x4 (&cx)[2], f32x4 (&cy)[2], f32x4 (&w4)[2]) {
+    const int m = ref(strong, l16);
+#pragma unroll
+    for (int z = 0; z < 2; ++z)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float l = lam[16 * (cb0 + z) + 4 * g + v];
+            cx[z][v] = wpow(l, static_cast<float>(l16 - m));
+            cy[z][v] = wpow(l, static_cast<float>(m - 1 - l16));
+            w4[z][v] = wpow(l, 4.f);
+        }
+}
+// A tile applied to four token rows: sum over slots (token 4 g + v) of a[v] b[v], where pairs of tokens of different halves of a
+// strong chunk take the factor w4 of the output's lane twice; cross: this lane's operand row pairs with the other half.
+DEVINL f32x4 apply(const f32x4& a, const f32x4& b, bool strong, bool cross, float w4) {
+    f32x4 d = ZERO4;
+    if (strong) {
+        f32x4 o = ZERO4;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) { d = mm(cross ? 0.f : a[v], b[v], d); o = mm(cross ? a[v] : 0.f, b[v], o); }
+        return d + o * w4 * w4;
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) d = mm(a[v], b[v], d);
+    return d;
+}
+
+// ---------------------------------------------------------------------------------------------------- forward
+// Waves 0..3 (value channels 16 q + l16): St[jt][v] = S[i = 16 q + l16][j = 16 jt + 4 g + v], as it stands the B operand of a
+// contraction over j.  Waves 4..7 load: chunk c + 2 into LDS while chunk c is worked on (three slots, one barrier a chunk),
+// their global loads four chunks further ahead.  Wave q makes a quarter of the next chunk's tile (16 of the 64 key channels).
+struct SlotF {
+    float r[L][PS], k[L][PS], v[L][PS];
+    float ruk[L], rk[L];
+};
+struct SmemF {
+    Head hd;
+    SlotF slot[3];
+    float part[2][4][L][TS];            // the four waves' parts of the tile, of this chunk and the next
+};
+constexpr int FDEPTH = 4;
+
+template <bool TWO>
+__global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
+    __shared__ SmemF S;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = w & 3, l16 = lane & 15, g = lane >> 4;
+    const int h = blockIdx.x % p.H, b = blockIdx.x / p.H, T = p.T, C = p.C;
+    const int nch = (T + L - 1) / L;
+    const size_t base = static_cast<size_t>(b) * T * C + static_cast<size_t>(h) * N;
+    const bool strong = head_setup<TWO>(S.hd, p, h, tid);
+    __syncthreads();
+    if (w >= 4) {
+        const int tp = tid - 256, row = tp >> 4, c4 = (tp & 15) * 4;
+        const f32x4 u = ld4(&S.hd.u[c4]);
+        f32x4 x[FDEPTH][3];
+        auto fetch = [&](const int c, f32x4 (&d)[3]) __attribute__((always_inline)) {
+            const int cc = min(c, nch - 1);                       // (the same loads in every iteration: see the backward of wkv6)
+            const size_t o = base + static_cast<size_t>(cc) * L * C;
+            const int lo = min(row, T - 1 - cc * L) * C + c4;
+            d[0] = ld4(p.r + o + lo); d[1] = ld4(p.k + o + lo); d[2] = ld4(p.v + o + lo);
+        };
+        auto put = [&](const int c, SlotF& s, const f32x4 (&d)[3]) __attribute__((always_inline)) {
+            const bool ok = c * L + row < T;
+            const f32x4 r = ok ? d[0] : ZERO4, k = ok ? d[1] : ZERO4, v = ok ? d[2] : ZERO4;
+            st4(&s.r[row][c4], r); st4(&s.k[row][c4], k); st4(&s.v[row][c4], v);
+            const f32x4 rk = r * k;
+            const float a = row_sum((rk[0] * u[0] + rk[1] * u[1]) + (rk[2] * u[2] + rk[3] * u[3]));
+            if ((tp & 15) == 0) s.ruk[row] = a;
+            if constexpr (TWO) {
+                const float a2 = row_sum((rk[0] + rk[1]) + (rk[2] + rk[3]));
+                if ((tp & 15) == 0) s.rk[row] = a2;
+            }
+        };
+#pragma unroll
+        for (int z = 0; z < FDEPTH; ++z) fetch(z, x[z]);
+        put(0, S.slot[0], x[0]); fetch(FDEPTH, x[0]);
+        put(1, S.slot[1], x[1]); fetch(FDEPTH + 1, x[1]);
+        __syncthreads();
+        __syncthreads();
+        int sl = 2;
+        for (int c0 = 0; c0 < nch; c0 += FDEPTH) {
+#pragma unroll
+            for (int z = 0; z < FDEPTH; ++z) {
+                const int c = c0 + z;
+                if (c >= nch) break;
+                put(c + 2, S.slot[sl], x[(z + 2) % FDEPTH]);
+                fetch(c + 2 + FDEPTH, x[(z + 2) % FDEPTH]);
+                sl = sl == 2 ? 0 : sl + 1;
+                __syncthreads();
+            }
+        }
+        return;
+    }
+    const int own = 16 * q + l16;
+    // powers: A operands over j (r o1^t, token t = l16; k o1^{15-t}, token 4 g + v), the tile's, the value side's
+    f32x4 crs[4], cke[4], ctx, cty, ct4;
+    {
+        const int m = ref(strong, l16);
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                crs[jt][v] = wpow(S.hd.lam[16 * jt + 4 * g + v], static_cast<float>(l16));
+                cke[jt][v] = wpow(S.hd.lam[16 * jt + l16], static_cast<float>(15 - 4 * g - v));
+            }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float l = S.hd.lam[16 * q + 4 * g + v];
+            ctx[v] = wpow(l, static_cast<float>(l16 - m));
+            cty[v] = wpow(l, static_cast<float>(m - 1 - l16));
+            ct4[v] = wpow(l, 4.f);
+        }
+    }
+    f32x4 c2s = ZERO4, c2m = ZERO4, c2k = ZERO4, c2e = ZERO4;
+    float u2 = 0.f, d2 = 1.f, w24 = 1.f;
+    if constexpr (TWO) {
+        const float l = S.hd.lam2[own];
+        u2 = S.hd.u2[own]; d2 = S.hd.dec2[own]; w24 = wpow(l, 4.f);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = 4 * g + v, m = ref(strong, t);
+            c2s[v] = wpow(l, static_cast<float>(t)); c2e[v] = wpow(l, static_cast<float>(15 - t));
+            c2m[v] = wpow(l, static_cast<float>(t - m)); c2k[v] = wpow(l, static_cast<float>(m - 1 - t));
+        }
+    }
+    auto tile = [&](const SlotF& s, float (*out)[TS]) __attribute__((always_inline)) {
+        const f32x4 xa = ld4(&s.r[l16][16 * q + 4 * g]) * ctx, ya = ld4(&s.k[l16][16 * q + 4 * g]) * cty;
+        f32x4 acc = ZERO4;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc = mm(xa[v], ya[v], acc);
+        if (strong) {
+            f32x4 o = ZERO4;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o = mm(xa[v] * ct4[v], ya[v] * ct4[v], o);
+            if (g >= 2 && l16 < 8) acc = o;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out[4 * g + v][l16] = l16 < 4 * g + v ? acc[v] : 0.f;
+    };
+    const int nseg = (nch + SEG<TWO> - 1) / SEG<TWO>;
+    float* const sv = p.saved != nullptr ? p.saved + static_cast<size_t>(blockIdx.x) * nseg * N * N + own * N + 4 * g : nullptr;
+    f32x4 St[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
+    __syncthreads();                                     // chunks 0 and 1 are there
+    tile(S.slot[0], S.part[0][q]);
+    __syncthreads();
+    int sl = 0;
+    const int lo = 4 * g * C + own;
+    for (int c = 0; c < nch; ++c) {
+        const SlotF& X = S.slot[sl];
+        sl = sl == 2 ? 0 : sl + 1;
+        if (c + 1 < nch) tile(S.slot[sl], S.part[(c + 1) & 1][q]);
+        if (sv != nullptr && c > 0 && c % SEG<TWO> == 0) {
+            float* d = sv + static_cast<size_t>(c / SEG<TWO>) * N * N;
+#pragma unroll
+            for (int jt = 0; jt < 4; ++jt) st4(d + 16 * jt, St[jt]);
+        }
+        f32x4 y2[2] = {ZERO4, ZERO4};
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) {
+            const f32x4 xa = ld4(&X.r[l16][16 * jt + 4 * g]) * crs[jt];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y2[jt & 1] = mm(xa[v], St[jt][v], y2[jt & 1]);
+        }
+        f32x4 vop;                                       // v[token 4 g + v][own]
+#pragma unroll
+        for (int v = 0; v < 4; ++v) vop[v] = X.v[4 * g + v][own];
+        const float (*pt)[L][TS] = S.part[c & 1];
+        const f32x4 at = (ld4(&pt[0][l16][4 * g]) + ld4(&pt[1][l16][4 * g])) + (ld4(&pt[2][l16][4 * g]) + ld4(&pt[3][l16][4 * g]));
+        const f32x4 ruk = ld4(&X.ruk[4 * g]);
+        f32x4 y = y2[0] + y2[1];
+        if constexpr (TWO) {
+            const f32x4 ap = apply(at, vop * c2k, strong, l16 >= 8 && g < 2, w24);
+            y = y * c2s + ap * c2m + vop * (ruk + u2 * ld4(&X.rk[4 * g]));
+        } else {
+            y += vop * ruk;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y = mm(at[v], vop[v], y);
+        }
+        float* const out = p.y + base + static_cast<size_t>(c) * L * C;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (c * L + 4 * g + v < T) (out + static_cast<size_t>(v) * C)[lo] = y[v];
+        const f32x4 ve = TWO ? vop * c2e : vop;
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) {
+            f32x4 acc = St[jt] * ld4(&S.hd.dec[16 * jt + 4 * g]);
+            if constexpr (TWO) acc *= d2;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc = mm(X.k[4 * g + v][16 * jt + l16] * cke[jt][v], ve[v], acc);
+            St[jt] = acc;
+        }
+        __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------- backward
+// One reverse sweep, one barrier a chunk, eight waves:
+//   D, waves 0..3 (key channel j = 16 q + l16): the states of a segment, rebuilt from the saved one, and the gradient state as
+//      S[i = 16 ib + 4 g + v][j]: the B operands of contractions over the value channel.  gr, gk, gw, gu.
+//   E, waves 4..7 (value channel i = 16 q + l16): the gradient state transposed, D[i][j = 16 jt + 4 g + v].  gv; the halves of
+//      the next chunk's two tiles (waves 4, 5 the A tile, 6, 7 the B tile); all loads, SEG chunks ahead of their use.
+// The planes in LDS are the raw inputs: every power is applied to an operand on its way into the matrix instruction, from
+// registers, so that a chunk costs four planes instead of one per power.
+struct SlotB {
+    float r[L][PS], k[L][PS], v[L][PS], g[L][PS];
+    float vg[L], u2vg[L], ruk[L], rk[L];
+};
+template <bool TWO> struct SmemB {
+    Head hd;
+    SlotB slot[2 * SEG<TWO>];
+    float part[2][4][L][TS];            // halves of the tiles A (0, 1) and B (2, 3)
+    float red[4][N];
+};
+
+template <bool TWO>
+DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, int h, int b, size_t base, int nch) {
+    constexpr int G = SEG<TWO>;
+    const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = p.T;
+    const int nseg = (nch + G - 1) / G;
+    const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * nseg * N * N + 4 * g * N + own;
+    const float l1 = S.hd.lam[own], u1 = S.hd.u[own], d1 = S.hd.dec[own], w4 = wpow(l1, 4.f);
+    f32x4 cs, ce, cm, ck, tf;                            // o1^t, o1^{15-t}, o1^{t-m}, o1^{m-1-t} and t for t = 4 g + v
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int t = 4 * g + v, m = ref(strong, t);
+        tf[v] = static_cast<float>(t);
+        cs[v] = wpow(l1, static_cast<float>(t)); ce[v] = wpow(l1, static_cast<float>(15 - t));
+        cm[v] = wpow(l1, static_cast<float>(t - m)); ck[v] = wpow(l1, static_cast<float>(m - 1 - t));
+    }
+    // two-sided: powers of the value side for the A operands gy o2^t, v o2^{15-t} with token l16 / token 4 g + v in the lane
+    f32x4 gx[TWO ? 4 : 1], vx[TWO ? 4 : 1], gup[TWO ? 4 : 1], vup[TWO ? 4 : 1];
+    if constexpr (TWO) {
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float la = S.hd.lam2[16 * ib + 4 * g + v], lb = S.hd.lam2[16 * ib + l16];
+                gx[ib][v] = wpow(la, static_cast<float>(l16)); vx[ib][v] = wpow(la, static_cast<float>(15 - l16));
+                gup[ib][v] = wpow(lb, static_cast<float>(4 * g + v)); vup[ib][v] = wpow(lb, static_cast<float>(15 - 4 * g - v));
+            }
+    }
+    f32x4 St[G][4], Sn[4], dS[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
+    f32x4 accG[TWO ? 4 : 1];
+#pragma unroll
+    for (int e = 0; e < (TWO ? 4 : 1); ++e) accG[e] = ZERO4;
+    float gw = 0.f, gP = 0.f, gu = 0.f;
+    auto fetch_state = [&](const int s) __attribute__((always_inline)) {
+        const float* d = sv + static_cast<size_t>(max(s, 0)) * N * N;
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Sn[ib][v] = s > 0 ? d[(16 * ib + v) * N] : 0.f;      // the sequence starts from nothing
+    };
+    auto decay = [&](const int ib) __attribute__((always_inline)) {
+        if constexpr (TWO) return ld4(&S.hd.dec2[16 * ib + 4 * g]) * d1;
+        else return f32x4{d1, d1, d1, d1};
+    };
+    const int lo = 4 * g * C + own;
+    auto chunk = [&](const int c, const f32x4 (&Sz)[4]) __attribute__((always_inline)) {
+        const SlotB& X = S.slot[c % (2 * G)];
+        const float (*pb)[L][TS] = &S.part[c & 1][2];
+        f32x4 kk, rr, bt;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            kk[v] = X.k[4 * g + v][own]; rr[v] = X.r[4 * g + v][own];
+            bt[v] = pb[0][4 * g + v][l16] + pb[1][4 * g + v][l16];
+        }
+        const f32x4 bm = ld4(&pb[0][l16][4 * g]) + ld4(&pb[1][l16][4 * g]);
+        f32x4 x2[2] = {ZERO4, ZERO4}, z2[2] = {ZERO4, ZERO4};
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+            f32x4 ga = ld4(&X.g[l16][16 * ib + 4 * g]), va = ld4(&X.v[l16][16 * ib + 4 * g]);
+            if constexpr (TWO) { ga *= gx[ib]; va *= vx[ib]; }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                x2[ib & 1] = mm(ga[v], Sz[ib][v], x2[ib & 1]);
+                z2[ib & 1] = mm(va[v], dS[ib][v], z2[ib & 1]);
+            }
+        }
+        const f32x4 km = kk * ck, rm = rr * cm;
+        const bool cx = l16 >= 8 && g < 2, cz = l16 < 8 && g >= 2;
+        f32x4 lag;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) lag[v] = static_cast<float>(l16 - 1) - tf[v];
+        const f32x4 tx = apply(bm, km, strong, cx, w4), tl = apply(bm * lag, km, strong, cx, w4), tz = apply(bt, rm, strong, cz, w4);
+        const f32x4 xs = (x2[0] + x2[1]) * cs, zs = (z2[0] + z2[1]) * ce;
+        const f32x4 vg = ld4(&X.vg[4 * g]);
+        f32x4 bo = vg * u1;
+        if constexpr (TWO) bo += ld4(&X.u2vg[4 * g]);
+        const f32x4 dr = xs + tx * cm + kk * bo, dk = zs + tz * ck + rr * bo;
+        const size_t o = base + static_cast<size_t>(c) * L * C;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (c * L + 4 * g + v < T) {
+                (p.gr + o + static_cast<size_t>(v) * C)[lo] = dr[v];
+                (p.gk + o + static_cast<size_t>(v) * C)[lo] = dk[v];
+            }
+        const f32x4 gu4 = rr * kk * vg, gw4 = rm * tl;
+        gu += (gu4[0] + gu4[1]) + (gu4[2] + gu4[3]);
+        gw += (gw4[0] + gw4[1]) + (gw4[2] + gw4[3]);
+        const f32x4 rs = rr * cs;
+        if constexpr (TWO) {
+            const f32x4 rt = rs * tf, kt = kk * ce * (15.f - tf);
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib) {
+                const f32x4 dec = decay(ib);
+                f32x4 m1 = ZERO4, n1 = ZERO4, acc = dS[ib] * dec;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float ga = X.g[4 * g + v][16 * ib + l16] * gup[ib][v], va = X.v[4 * g + v][16 * ib + l16] * vup[ib][v];
+                    m1 = mm(ga, rt[v], m1);
+                    n1 = mm(va, kt[v], n1);
+                    acc = mm(ga, rs[v], acc);
+                }
+                accG[ib] += Sz[ib] * m1 + dS[ib] * n1 + (16.f * dec) * (Sz[ib] * dS[ib]);
+                dS[ib] = acc;
+            }
+        } else {
+            const f32x4 gs4 = tf * rr * xs + (15.f - tf) * kk * zs;
+            gw += (gs4[0] + gs4[1]) + (gs4[2] + gs4[3]);
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib) {
+                const f32x4 pp = Sz[ib] * dS[ib];
+                gP += (pp[0] + pp[1]) + (pp[2] + pp[3]);
+                f32x4 acc = dS[ib] * d1;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc = mm(X.g[4 * g + v][16 * ib + l16], rs[v], acc);
+                dS[ib] = acc;
+            }
+        }
+    };
+    fetch_state(nseg - 1);
+    __syncthreads();                                     // the top chunks are there
+    __syncthreads();                                     // and the first tiles
+    for (int s = nseg - 1; s >= 0; --s) {
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) St[0][ib] = Sn[ib];
+        fetch_state(s - 1);
+#pragma unroll
+        for (int z = 0; z + 1 < G; ++z) {
+            if (s * G + z + 1 < nch) {
+                const SlotB& X = S.slot[(s * G + z) % (2 * G)];
+                f32x4 ke;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) ke[v] = X.k[4 * g + v][own] * ce[v];
+#pragma unroll
+                for (int ib = 0; ib < 4; ++ib) {
+                    f32x4 acc = St[z][ib] * decay(ib);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        float va = X.v[4 * g + v][16 * ib + l16];
+                        if constexpr (TWO) va *= vup[ib][v];
+                        acc = mm(va, ke[v], acc);
+                    }
+                    St[z + 1][ib] = acc;
+                }
+            }
+        }
+#pragma unroll
+        for (int z = G - 1; z >= 0; --z) {
+            if (s * G + z < nch) {
+                chunk(s * G + z, St[z]);
+                __syncthreads();
+            }
+        }
+    }
+    gw = fmaf(16.f * d1, gP, gw);
+    if constexpr (TWO) {
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                gw += accG[ib][v];
+                const float x = row_sum(accG[ib][v]);
+                if (l16 == 0) S.red[q][16 * ib + 4 * g + v] = x;
+            }
+        __syncthreads();
+    }
+    gw = allreduce_rows(gw); gu = allreduce_rows(gu);
+    if (g == 0) {
+        const float lt = -expf(p.w[h * N + own]);        // (a decay below the smallest one: its gradient is that of the pairs one step apart)
+        const size_t o = static_cast<size_t>(b) * C + h * N + own;
+        p.gw[o] = lt * expf(lt - l1) * gw;
+        p.gu[o] = gu;
+    }
+}
+
+template <bool TWO>
+DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, int h, int b, size_t base, int nch) {
+    constexpr int G = SEG<TWO>;
+    const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = p.T;
+    const int te = 64 * q + lane, row = te >> 4, c4 = (te & 15) * 4;
+    // loads
+    const f32x4 u = ld4(&S.hd.u[c4]), u2c = ld4(&S.hd.u2[c4]);
+    auto fetch = [&](const int c, f32x4 (&d)[4]) __attribute__((always_inline)) {
+        const int cc = max(c, 0);
+        const size_t o = base + static_cast<size_t>(cc) * L * C;
+        const int lo = min(row, T - 1 - cc * L) * C + c4;
+        d[0] = ld4(p.r + o + lo); d[1] = ld4(p.k + o + lo); d[2] = ld4(p.v + o + lo); d[3] = ld4(p.gy + o + lo);
+    };
+    auto put = [&](const int c, const f32x4 (&d)[4]) __attribute__((always_inline)) {
+        SlotB& s = S.slot[c % (2 * G)];
+        const bool ok = c * L + row < T;
+        const f32x4 r = ok ? d[0] : ZERO4, k = ok ? d[1] : ZERO4, v = ok ? d[2] : ZERO4, gy = ok ? d[3] : ZERO4;
+        st4(&s.r[row][c4], r); st4(&s.k[row][c4], k); st4(&s.v[row][c4], v); st4(&s.g[row][c4], gy);
+        const f32x4 rk = r * k, vg = v * gy;
+        const float a = row_sum((rk[0] * u[0] + rk[1] * u[1]) + (rk[2] * u[2] + rk[3] * u[3]));
+        const float e = row_sum((vg[0] + vg[1]) + (vg[2] + vg[3]));
+        if ((te & 15) == 0) { s.ruk[row] = a; s.vg[row] = e; }
+        if constexpr (TWO) {
+            const float a2 = row_sum((rk[0] + rk[1]) + (rk[2] + rk[3]));
+            const float e2 = row_sum((vg[0] * u2c[0] + vg[1] * u2c[1]) + (vg[2] * u2c[2] + vg[3] * u2c[3]));
+            if ((te & 15) == 0) { s.rk[row] = a2; s.u2vg[row] = e2; }
+        }
+    };
+    f32x4 ring[2][4];
+    {
+        f32x4 top[G][4];
+#pragma unroll
+        for (int z = 0; z < G; ++z) fetch(nch - 1 - z, top[z]);
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            // chunk nch - 1 - G is written in the first chunk's phase, from ring[(nch - 1) & 1]
+            if ((nch - 1) & 1) fetch(nch - 1 - G - z, ring[1 - z]);
+            else fetch(nch - 1 - G - z, ring[z]);
+        }
+#pragma unroll
+        for (int z = 0; z < G; ++z)
+            if (nch - 1 - z >= 0) put(nch - 1 - z, top[z]);
+    }
+    // powers: A operands over j, k o1^{15-t} (token l16) and r o1^t (token 4 g + v); the tile half of this wave
+    f32x4 cke[4], crs[4], tx[2], ty[2], t4[2];
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            cke[jt][v] = wpow(S.hd.lam[16 * jt + 4 * g + v], static_cast<float>(15 - l16));
+            crs[jt][v] = wpow(S.hd.lam[16 * jt + l16], static_cast<float>(4 * g + v));
+        }
+    const int cb0 = 2 * (q & 1);
+    tile_powers(q < 2 ? S.hd.lam : S.hd.lam2, cb0, strong, l16, g, tx, ty, t4);
+    auto tile = [&](const int c) __attribute__((always_inline)) {
+        const SlotB& X = S.slot[c % (2 * G)];
+        float (*out)[TS] = S.part[c & 1][q];
+        if (q < 2) half_tile<true>(X.r, X.k, out, cb0, tx, ty, t4, strong, l16, g);
+        else half_tile<TWO>(X.g, X.v, out, cb0, tx, ty, t4, strong, l16, g);
+    };
+    f32x4 c2s = ZERO4, c2e = ZERO4, c2m = ZERO4, c2k = ZERO4;
+    float u2 = 0.f, d2 = 1.f, w24 = 1.f, gw2 = 0.f, gu2 = 0.f;
+    const float l2 = S.hd.lam2[own];
+    if constexpr (TWO) {
+        u2 = S.hd.u2[own]; d2 = S.hd.dec2[own]; w24 = wpow(l2, 4.f);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = 4 * g + v, m = ref(strong, t);
+            c2s[v] = wpow(l2, static_cast<float>(t)); c2e[v] = wpow(l2, static_cast<float>(15 - t));
+            c2m[v] = wpow(l2, static_cast<float>(t - m)); c2k[v] = wpow(l2, static_cast<float>(m - 1 - t));
+        }
+    }
+    f32x4 dT[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
+    const int lo = 4 * g * C + own;
+    auto chunk = [&](const int c, f32x4 (&rg)[4]) __attribute__((always_inline)) {
+        const SlotB& X = S.slot[c % (2 * G)];
+        const float (*pa)[L][TS] = &S.part[c & 1][0];
+        f32x4 go, aT;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) { go[v] = X.g[4 * g + v][own]; aT[v] = pa[0][4 * g + v][l16] + pa[1][4 * g + v][l16]; }
+        f32x4 y2[2] = {ZERO4, ZERO4};
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) {
+            const f32x4 ka = ld4(&X.k[l16][16 * jt + 4 * g]) * cke[jt];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) y2[jt & 1] = mm(ka[v], dT[jt][v], y2[jt & 1]);
+        }
+        const f32x4 ruk = ld4(&X.ruk[4 * g]);
+        f32x4 dv = y2[0] + y2[1];
+        if constexpr (TWO) {
+            const f32x4 rk = ld4(&X.rk[4 * g]), gm = go * c2m;
+            dv = dv * c2e + apply(aT, gm, strong, l16 < 8 && g >= 2, w24) * c2k + go * (ruk + u2 * rk);
+            f32x4 vo, lag;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) { vo[v] = X.v[4 * g + v][own]; lag[v] = static_cast<float>(l16 - 1 - 4 * g - v); }
+            const f32x4 a = ld4(&pa[0][l16][4 * g]) + ld4(&pa[1][l16][4 * g]);
+            const f32x4 w4 = gm * apply(a * lag, vo * c2k, strong, l16 >= 8 && g < 2, w24), u4 = vo * go * rk;
+            gw2 += (w4[0] + w4[1]) + (w4[2] + w4[3]);
+            gu2 += (u4[0] + u4[1]) + (u4[2] + u4[3]);
+        } else {
+            dv += go * ruk;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) dv = mm(aT[v], go[v], dv);
+        }
+        float* const out = p.gv + base + static_cast<size_t>(c) * L * C;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (c * L + 4 * g + v < T) (out + static_cast<size_t>(v) * C)[lo] = dv[v];
+        const f32x4 gs = TWO ? go * c2s : go;
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) {
+            f32x4 acc = dT[jt] * ld4(&S.hd.dec[16 * jt + 4 * g]);
+            if constexpr (TWO) acc *= d2;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc = mm(X.r[4 * g + v][16 * jt + l16] * crs[jt][v], gs[v], acc);
+            dT[jt] = acc;
+        }
+        if (c > 0) tile(c - 1);
+        if (c >= G) put(c - G, rg);
+        fetch(c - G - 2, rg);
+    };
+    __syncthreads();
+    tile(nch - 1);
+    __syncthreads();
+    const int nseg = (nch + G - 1) / G;
+    for (int s = nseg - 1; s >= 0; --s) {
+#pragma unroll
+        for (int z = G - 1; z >= 0; --z) {
+            if (s * G + z < nch) {
+                chunk(s * G + z, ring[z & 1]);
+                __syncthreads();
+            }
+        }
+    }
+    if constexpr (TWO) {
+        __syncthreads();
+        gw2 = allreduce_rows(gw2); gu2 = allreduce_rows(gu2);
+        if (g == 0) {
+            const float lt = -expf(p.w2[h * N + own]);
+            const size_t o = static_cast<size_t>(b) * C + h * N + own;
+            p.gw2[o] = lt * expf(lt - l2) * (gw2 + ((S.red[0][own] + S.red[1][own]) + (S.red[2][own] + S.red[3][own])));
+            p.gu2[o] = gu2;
+        }
+    }
+}
+
+template <bool TWO>
+__global__ __launch_bounds__(NT, 2) void wkv5c_bwd(const ArgsC p) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    SmemB<TWO>& S = *reinterpret_cast<SmemB<TWO>*>(smem_raw);
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = w & 3;
+    const int h = blockIdx.x % p.H, b = blockIdx.x / p.H;
+    const int nch = (p.T + L - 1) / L;
+    const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * N;
+    const bool strong = head_setup<TWO>(S.hd, p, h, tid);
+    __syncthreads();
+    if (w < 4) role_d<TWO>(S, p, strong, q, lane, h, b, base, nch);
+    else role_e<TWO>(S, p, strong, q, lane, h, b, base, nch);
+}
+
+// out[c] = sum over the batch of rows of up to four [B][C] arrays that lie behind each other
+__global__ __launch_bounds__(256) void rows_sum(int B, int C, const float* __restrict__ rows, float* o0, float* o1, float* o2, float* o3) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= C) return;
+    const float* x = rows + static_cast<size_t>(blockIdx.y) * B * C + c;
+    float s = 0.f;
+    for (int b = 0; b < B; ++b) s += x[static_cast<size_t>(b) * C];
+    (blockIdx.y == 0 ? o0 : (blockIdx.y == 1 ? o1 : (blockIdx.y == 2 ? o2 : o3)))[c] = s;
+}
+
+template <bool TWO> size_t saved_bytes(int B, int T, int C, int H) {
+    if (B <= 0 || T <= 0 || H <= 0 || C != H * N) return 0;
+    const size_t nch = (static_cast<size_t>(T) + L - 1) / L;
+    return static_cast<size_t>(B) * H * ((nch + SEG<TWO> - 1) / SEG<TWO>) * N * N * sizeof(float);
+}
+int check(int B, int T, int C, int H) {
+    if (B <= 0 || T <= 0 || H <= 0 || C != H * N) return RWKV_ERR_SHAPE;
+    if (static_cast<long long>(B) * H > 0x7fffffffLL || C > (1 << 26)) return RWKV_ERR_SHAPE;      // 16 rows by a 32-bit offset
+    return RWKV_OK;
+}
+
+template <bool TWO> int start_fwd(void* stream, int B, const ArgsC& p) {
+    hipLaunchKernelGGL(wkv5c_fwd<TWO>, dim3(B * p.H), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
+    return launch_status();
+}
+template <bool TWO> int start_bwd(void* stream, int B, const ArgsC& p, float* rows, float* gw, float* gu, float* gw2, float* gu2) {
+    static_assert(sizeof(SmemB<TWO>) <= 160 * 1024, "the backward's LDS must fit one CU");
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(wkv5c_bwd<TWO>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       static_cast<int>(sizeof(SmemB<TWO>)));
+    if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipLaunchKernelGGL(wkv5c_bwd<TWO>, dim3(B * p.H), dim3(NT), sizeof(SmemB<TWO>), st, p);
+    hipLaunchKernelGGL(rows_sum, dim3((p.C + 255) / 256, TWO ? 4 : 2), dim3(256), 0, st, B, p.C, rows, gw, gu, gw2, gu2);
+    return launch_status();
+}
+
+}  // namespace
+}  // namespace rwkv
+
+using namespace rwkv;
+
+extern "C" {
+
+size_t rwkv_wkv5f32s_saved_bytes(int B, int T, int C, int H) { return saved_bytes<false>(B, T, C, H); }
+size_t rwkv_wkv5as_saved_bytes(int B, int T, int C, int H) { return saved_bytes<true>(B, T, C, H); }
+size_t rwkv_wkv5f32s_backward_workspace_bytes(int B, int T, int C, int H) {
+    return check(B, T, C, H) == RWKV_OK ? 2 * static_cast<size_t>(B) * C * sizeof(float) : 0;
+}
+size_t rwkv_wkv5as_backward_workspace_bytes(int B, int T, int C, int H) {
+    return check(B, T, C, H) == RWKV_OK ? 4 * static_cast<size_t>(B) * C * sizeof(float) : 0;
+}
+
+int rwkv_wkv5f32s_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w,
+                          const float* u, float* y, void* saved, size_t bytes) {
+    if (int e = check(B, T, C, H)) return e;
+    if (int e = check_ptrs({r, k, v, w, u, y})) return e;
+    if (saved != nullptr && (bytes < saved_bytes<false>(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
+    ArgsC p{};
+    p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.saved = static_cast<float*>(saved);
+    return start_fwd<false>(stream, B, p);
+}
+
+int rwkv_wkv5f32s_backward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w,
+                           const float* u, const float* gy, float* gr, float* gk, float* gv, float* gw, float* gu, const void* saved,
+                           size_t bytes, void* workspace, size_t workspace_bytes) {
+    if (int e = check(B, T, C, H)) return e;
+    if (int e = check_ptrs({r, k, v, w, u, gy, gr, gk, gv, gw, gu})) return e;
+    if (saved == nullptr || bytes < saved_bytes<false>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
+    if (workspace == nullptr || workspace_bytes < rwkv_wkv5f32s_backward_workspace_bytes(B, T, C, H)) return RWKV_ERR_WORKSPACE;
+    float* rows = static_cast<float*>(workspace);
+    const size_t m = static_cast<size_t>(B) * C;
+    ArgsC p{};
+    p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv;
+    p.gw = rows; p.gu = rows + m; p.saved = static_cast<float*>(const_cast<void*>(saved));
+    return start_bwd<false>(stream, B, p, rows, gw, gu, nullptr, nullptr);
+}
+
+int rwkv_wkv5as_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
+                        const float* u1, const float* w2, const float* u2, float* y, void* saved, size_t bytes) {
+    if (int e = check(B, T, C, H)) return e;
+    if (int e = check_ptrs({r, k, v, w1, u1, w2, u2, y})) return e;
+    if (saved != nullptr && (bytes < saved_bytes<true>(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
+    ArgsC p{};
+    p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w1; p.u = u1; p.w2 = w2; p.u2 = u2; p.y = y;
+    p.saved = static_cast<float*>(saved);
+    return start_fwd<true>(stream, B, p);
+}
+
+int rwkv_wkv5as_backward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
+                         const float* u1, const float* w2, const float* u2, const float* gy, float* gr, float* gk, float* gv,
+                         float* gw1, float* gu1, float* gw2, float* gu2, const void* saved, size_t bytes, void* workspace,
+                         size_t workspace_bytes) {
+    if (int e = check(B, T, C, H)) return e;
+    if (int e = check_ptrs({r, k, v, w1, u1, w2, u2, gy, gr, gk, gv, gw1, gu1, gw2, gu2})) return e;
+    if (saved == nullptr || bytes < saved_bytes<true>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
+    if (workspace == nullptr || workspace_bytes < rwkv_wkv5as_backward_workspace_bytes(B, T, C, H)) return RWKV_ERR_WORKSPACE;
+    float* rows = static_cast<float*>(workspace);
+    const size_t m = static_cast<size_t>(B) * C;
+    ArgsC p{};
+    p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w1; p.u = u1; p.w2 = w2; p.u2 = u2; p.gy = gy;
+    p.gr = gr; p.gk = gk; p.gv = gv; p.gw = rows; p.gu = rows + m; p.gw2 = rows + 2 * m; p.gu2 = rows + 3 * m;
+    p.saved = static_cast<float*>(const_cast<void*>(saved));
+    return start_bwd<true>(stream, B, p, rows, gw1, gu1, gw2, gu2);
+}
+
+}  // extern "C"
