@@ -242,7 +242,7 @@ int rwkv_wkv5a_backward_ex(void* stream, int B, int T, int C, int H,
  * size 64: raw w in, gradients of the raw parameters summed over the batch out (gw, gu [C]).  Chunked kernels on the fp32
  * matrix cores: one forward, one reverse sweep.
  *   `saved` (*_saved_bytes; 0 for another head size, which these entry points refuse with RWKV_ERR_SHAPE): the forward keeps
- *   the state entering every fourth (wkv5a: second) chunk of 16 tokens for the backward of the same step; NULL for a forward
+ *   the state entering every third (wkv5a: second) chunk of 16 tokens for the backward of the same step; NULL for a forward
  *   without a backward.  `workspace` (*_backward_workspace_bytes): per-batch rows of the parameter gradients.
  * ------------------------------------------------------------------------------------- */
 size_t rwkv_wkv5f32s_saved_bytes(int B, int T, int C, int H);

@@ -21,13 +21,15 @@
 // Two-sided, the last three are kept per state element (the two middle ones become products over the tokens) and summed
 // over i for l1 and over j for l2 at the end.
 //
-// Strong decays: with one reference in the middle a factor reaches e^{8 |l|}; beyond l = -7 (STRONG) the tiles take a
+// Strong decays: with one reference in the middle a factor reaches e^{8 |l|}; beyond l = -7 (LAM_STRONG) the tiles take a
 // reference in the middle of each half (m = 4, 12) and a pair of tokens of different halves carries o1^8 in addition: a second
 // product for that quadrant, with o1^4 on either side (o1^8 itself may underflow where the whole term is one).  Below l = -17 a decay is taken as e^{-17} = 4e-8, half a unit of the fp32 sum it enters.
 //
-// What bounds it: the fp32 matrix pipe (32 clocks an instruction; 40 per wave and chunk forward, 116 per SIMD backward) and
-// HBM: every tensor crosses it once, plus a saved state every SEG chunks.  B8 T4096 C4096, forward + backward: see the
-// launchers below for what it measured.
+// What bounds it.  Forward: HBM (B8 T4096 C4096: 2.9 GB in 0.60 ms; the sequential kernel took 1.3).  Backward: the fp32 matrix
+// instruction, which occupies a SIMD's vector ALU for 32 clocks (99 of them per SIMD and chunk and some 230 vector
+// instructions fill two thirds of its 1.40 ms; the three sequential sweeps took 4.1).  wkv5a: 0.67 + 1.83 ms, 6.2 before.
+#include <stddef.h>
+
 #include "common.h"
 
 namespace rwkv {
@@ -37,18 +39,28 @@ constexpr int N = 64;
 constexpr int L = 16;
 constexpr int PS = 68;               // row stride (floats) of a [token][channel] plane
 constexpr int TS = 20;               // row stride (floats) of a 16 x 16 tile
-constexpr int NT = 512;              // forward: waves 0..3 products, 4..7 loads; backward: 0..3 key side, 4..7 value side and loads
-constexpr float STRONG = -7.f, LAM_MIN = -17.f;
+constexpr int NT = 512;              // forward: waves 0..3 products, 4..7 loads
+constexpr int NTB = 512;             // backward: waves 0..3 D, 4..7 E
+constexpr float LAM_STRONG = -7.f, LAM_MIN = -17.f;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 DEVINL f32x4 mm(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 DEVINL f32x4 ld4(const float* p) { const float4 x = *reinterpret_cast<const float4*>(p); return f32x4{x.x, x.y, x.z, x.w}; }
 DEVINL void st4(float* p, const f32x4& x) { *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]); }
 constexpr f32x4 ZERO4 = {0.f, 0.f, 0.f, 0.f};
+// four floats that need not sit in consecutive registers: for what a wave keeps across its loop (as vectors such values occupy
+// aligned groups of four, and the register allocator spills and reloads whole groups for one of them)
+struct F4 {
+    float a[4];
+    DEVINL float& operator[](int i) { return a[i]; }
+    DEVINL float operator[](int i) const { return a[i]; }
+};
+DEVINL f32x4 operator*(const f32x4& x, const F4& y) { return f32x4{x[0] * y[0], x[1] * y[1], x[2] * y[2], x[3] * y[3]}; }
+DEVINL f32x4 operator*(const F4& y, const f32x4& x) { return x * y; }
 
 // states are saved for the backward at the start of every SEG-th chunk; the backward holds the states of a whole segment in
-// registers: 4 chunks one-sided, 2 where the per-element sums and the second side's powers take the room
-template <bool TWO> constexpr int SEG = TWO ? 2 : 4;
+// registers and two segments' inputs in LDS: 3 chunks one-sided (150 of 160 KB), 2 with the two more planes of the other
+template <bool TWO> constexpr int SEG = TWO ? 2 : 3;
 
 struct ArgsC {
     int T, C, H;
@@ -65,7 +77,9 @@ DEVINL float wpow(float lam, float n) {
     const float t = x * L2E_HI;
     const float e = fmaf(x, L2E_HI, -t) + fmaf(x, L2E_LO, lo * L2E_HI);
     const float y = __builtin_amdgcn_exp2f(t);
-    return fmaf(y, e * LN2, y);
+    float r = fmaf(y, e * LN2, y);
+    asm volatile("" : "+v"(r));        // (a scalar of its own: the compiler packs neighbouring powers into vectors otherwise)
+    return r;
 }
 template <int R> DEVINL float row_ror(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + R, 0xf, 0xf, true));
@@ -90,43 +104,14 @@ template <bool TWO> DEVINL bool head_setup(Head& hd, const ArgsC& p, int h, int 
         hd.lam[lane] = a; hd.dec[lane] = wpow(a, L); hd.u[lane] = p.u[c];
         hd.lam2[lane] = b; hd.dec2[lane] = wpow(b, L); hd.u2[lane] = TWO ? p.u2[c] : 0.f;
     }
-    return __builtin_amdgcn_readfirstlane(mn < STRONG ? 1 : 0) != 0;
+    return __builtin_amdgcn_readfirstlane(mn < LAM_STRONG ? 1 : 0) != 0;
 }
 // reference token of token t
-DEVINL int ref(bool strong, int t) { return strong ? (t < 8 ? 4 : 12) : 8; }
+template <bool STRONG> DEVINL int ref(int t) { return STRONG ? (t < 8 ? 4 : 12) : 8; }
 
-// One half (32 channels, the 16-channel blocks cb0 and cb0 + 1) of a causal tile sum_c X[t][c] Y[s][c], s < t, with the powers
-// cx (of t = l16) and cy (of s = l16) per channel block and register; w4: half of what pairs across the halves of a strong chunk carry.
-template <bool SCALED>
-DEVINL void half_tile(const float (*X)[PS], const float (*Y)[PS], float (*out)[TS], int cb0, const f32x4 (&cx)[2], const f32x4 (&cy)[2],
-                      const f32x4 (&w4)[2], bool strong, int l16, int g) {
-    f32x4 d[2] = {ZERO4, ZERO4};
-    f32x4 xa[2], ya[2];
-#pragma unroll
-    for (int z = 0; z < 2; ++z) {
-        xa[z] = ld4(&X[l16][16 * (cb0 + z) + 4 * g]); ya[z] = ld4(&Y[l16][16 * (cb0 + z) + 4 * g]);
-        if constexpr (SCALED) { xa[z] *= cx[z]; ya[z] *= cy[z]; }
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-#pragma unroll
-        for (int z = 0; z < 2; ++z) d[z] = mm(xa[z][v], ya[z][v], d[z]);
-    f32x4 acc = d[0] + d[1];
-    if (SCALED && strong) {
-        f32x4 o = ZERO4;
-#pragma unroll
-        for (int z = 0; z < 2; ++z)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) o = mm(xa[z][v] * w4[z][v], ya[z][v] * w4[z][v], o);
-        if (g >= 2 && l16 < 8) acc = o;
-    }
-    // acc[v] = tile[t = 4 g + v][s = l16]
-#pragma unroll
-    for (int v = 0; v < 4; ++v) out[4 * g + v][l16] = l16 < 4 * g + v ? acc[v] : 0.f;
-}
 // the powers half_tile takes for a side with log decays lam
-DEVINL void tile_powers(const float* lam, int cb0, bool strong, int l16, int g, f32x4 (&cx)[2], f32x4 (&cy)[2], f32x4 (&w4)[2]) {
-    const int m = ref(strong, l16);
+template <bool STRONG> DEVINL void tile_powers(const float* lam, int cb0, int l16, int g, F4 (&cx)[2], F4 (&cy)[2], F4 (&w4)[2]) {
+    const int m = ref<STRONG>(l16);
 #pragma unroll
     for (int z = 0; z < 2; ++z)
 #pragma unroll
@@ -139,9 +124,9 @@ DEVINL void tile_powers(const float* lam, int cb0, bool strong, int l16, int g, 
 }
 // A tile applied to four token rows: sum over slots (token 4 g + v) of a[v] b[v], where pairs of tokens of different halves of a
 // strong chunk take the factor w4 of the output's lane twice; cross: this lane's operand row pairs with the other half.
-DEVINL f32x4 apply(const f32x4& a, const f32x4& b, bool strong, bool cross, float w4) {
+template <bool STRONG> DEVINL f32x4 apply(const f32x4& a, const f32x4& b, bool cross, float w4) {
     f32x4 d = ZERO4;
-    if (strong) {
+    if constexpr (STRONG) {
         f32x4 o = ZERO4;
 #pragma unroll
         for (int v = 0; v < 4; ++v) { d = mm(cross ? 0.f : a[v], b[v], d); o = mm(cross ? a[v] : 0.f, b[v], o); }
@@ -150,6 +135,18 @@ DEVINL f32x4 apply(const f32x4& a, const f32x4& b, bool strong, bool cross, floa
 #pragma unroll
     for (int v = 0; v < 4; ++v) d = mm(a[v], b[v], d);
     return d;
+}
+
+// four token rows (token 4 g + v) of an output; left: rows from this lane's first on that exist; whole: all of the chunk's do
+DEVINL void store_rows(float* out, int lo, int C, int left, bool whole, const f32x4& x) {
+    if (whole) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) (out + static_cast<size_t>(v) * C)[lo] = x[v];
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (v < left) (out + static_cast<size_t>(v) * C)[lo] = x[v];
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------- forward
@@ -167,62 +164,14 @@ struct SmemF {
 };
 constexpr int FDEPTH = 4;
 
-template <bool TWO>
-__global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
-    __shared__ SmemF S;
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = w & 3, l16 = lane & 15, g = lane >> 4;
-    const int h = blockIdx.x % p.H, b = blockIdx.x / p.H, T = p.T, C = p.C;
-    const int nch = (T + L - 1) / L;
-    const size_t base = static_cast<size_t>(b) * T * C + static_cast<size_t>(h) * N;
-    const bool strong = head_setup<TWO>(S.hd, p, h, tid);
-    __syncthreads();
-    if (w >= 4) {
-        const int tp = tid - 256, row = tp >> 4, c4 = (tp & 15) * 4;
-        const f32x4 u = ld4(&S.hd.u[c4]);
-        f32x4 x[FDEPTH][3];
-        auto fetch = [&](const int c, f32x4 (&d)[3]) __attribute__((always_inline)) {
-            const int cc = min(c, nch - 1);                       // (the same loads in every iteration: see the backward of wkv6)
-            const size_t o = base + static_cast<size_t>(cc) * L * C;
-            const int lo = min(row, T - 1 - cc * L) * C + c4;
-            d[0] = ld4(p.r + o + lo); d[1] = ld4(p.k + o + lo); d[2] = ld4(p.v + o + lo);
-        };
-        auto put = [&](const int c, SlotF& s, const f32x4 (&d)[3]) __attribute__((always_inline)) {
-            const bool ok = c * L + row < T;
-            const f32x4 r = ok ? d[0] : ZERO4, k = ok ? d[1] : ZERO4, v = ok ? d[2] : ZERO4;
-            st4(&s.r[row][c4], r); st4(&s.k[row][c4], k); st4(&s.v[row][c4], v);
-            const f32x4 rk = r * k;
-            const float a = row_sum((rk[0] * u[0] + rk[1] * u[1]) + (rk[2] * u[2] + rk[3] * u[3]));
-            if ((tp & 15) == 0) s.ruk[row] = a;
-            if constexpr (TWO) {
-                const float a2 = row_sum((rk[0] + rk[1]) + (rk[2] + rk[3]));
-                if ((tp & 15) == 0) s.rk[row] = a2;
-            }
-        };
-#pragma unroll
-        for (int z = 0; z < FDEPTH; ++z) fetch(z, x[z]);
-        put(0, S.slot[0], x[0]); fetch(FDEPTH, x[0]);
-        put(1, S.slot[1], x[1]); fetch(FDEPTH + 1, x[1]);
-        __syncthreads();
-        __syncthreads();
-        int sl = 2;
-        for (int c0 = 0; c0 < nch; c0 += FDEPTH) {
-#pragma unroll
-            for (int z = 0; z < FDEPTH; ++z) {
-                const int c = c0 + z;
-                if (c >= nch) break;
-                put(c + 2, S.slot[sl], x[(z + 2) % FDEPTH]);
-                fetch(c + 2 + FDEPTH, x[(z + 2) % FDEPTH]);
-                sl = sl == 2 ? 0 : sl + 1;
-                __syncthreads();
-            }
-        }
-        return;
-    }
+template <bool TWO, bool STRONG>
+DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base, int nch) {
+    const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
     const int own = 16 * q + l16;
     // powers: A operands over j (r o1^t, token t = l16; k o1^{15-t}, token 4 g + v), the tile's, the value side's
-    f32x4 crs[4], cke[4], ctx, cty, ct4;
+    F4 crs[4], cke[4], ctx, cty, ct4;
     {
-        const int m = ref(strong, l16);
+        const int m = ref<STRONG>(l16);
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
@@ -238,14 +187,14 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
             ct4[v] = wpow(l, 4.f);
         }
     }
-    f32x4 c2s = ZERO4, c2m = ZERO4, c2k = ZERO4, c2e = ZERO4;
+    F4 c2s = {}, c2m = {}, c2k = {}, c2e = {};
     float u2 = 0.f, d2 = 1.f, w24 = 1.f;
     if constexpr (TWO) {
         const float l = S.hd.lam2[own];
         u2 = S.hd.u2[own]; d2 = S.hd.dec2[own]; w24 = wpow(l, 4.f);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int t = 4 * g + v, m = ref(strong, t);
+            const int t = 4 * g + v, m = ref<STRONG>(t);
             c2s[v] = wpow(l, static_cast<float>(t)); c2e[v] = wpow(l, static_cast<float>(15 - t));
             c2m[v] = wpow(l, static_cast<float>(t - m)); c2k[v] = wpow(l, static_cast<float>(m - 1 - t));
         }
@@ -255,7 +204,7 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
         f32x4 acc = ZERO4;
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc = mm(xa[v], ya[v], acc);
-        if (strong) {
+        if constexpr (STRONG) {
             f32x4 o = ZERO4;
 #pragma unroll
             for (int v = 0; v < 4; ++v) o = mm(xa[v] * ct4[v], ya[v] * ct4[v], o);
@@ -296,7 +245,7 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
         const f32x4 ruk = ld4(&X.ruk[4 * g]);
         f32x4 y = y2[0] + y2[1];
         if constexpr (TWO) {
-            const f32x4 ap = apply(at, vop * c2k, strong, l16 >= 8 && g < 2, w24);
+            const f32x4 ap = apply<STRONG>(at, vop * c2k, l16 >= 8 && g < 2, w24);
             y = y * c2s + ap * c2m + vop * (ruk + u2 * ld4(&X.rk[4 * g]));
         } else {
             y += vop * ruk;
@@ -304,9 +253,7 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
             for (int v = 0; v < 4; ++v) y = mm(at[v], vop[v], y);
         }
         float* const out = p.y + base + static_cast<size_t>(c) * L * C;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (c * L + 4 * g + v < T) (out + static_cast<size_t>(v) * C)[lo] = y[v];
+        store_rows(out, lo, C, T - c * L - 4 * g, c * L + L <= T, y);
         const f32x4 ve = TWO ? vop * c2e : vop;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
@@ -320,51 +267,175 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
     }
 }
 
+template <bool TWO>
+__global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
+    __shared__ SmemF S;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = w & 3;
+    const int h = blockIdx.x % p.H, b = blockIdx.x / p.H, T = p.T, C = p.C;
+    const int nch = (T + L - 1) / L;
+    const size_t base = static_cast<size_t>(b) * T * C + static_cast<size_t>(h) * N;
+    const bool strong = head_setup<TWO>(S.hd, p, h, tid);
+    __syncthreads();
+    if (w >= 4) {
+        const int tp = tid - 256, row = tp >> 4, c4 = (tp & 15) * 4;
+        const f32x4 u = ld4(&S.hd.u[c4]);
+        f32x4 x[FDEPTH][3];
+        auto fetch = [&](const int c, f32x4 (&d)[3]) __attribute__((always_inline)) {
+            const int cc = min(c, nch - 1);                       // (the same loads in every iteration: see the backward of wkv6)
+            const size_t o = base + static_cast<size_t>(cc) * L * C;
+            const int lo = min(row, T - 1 - cc * L) * C + c4;
+            d[0] = ld4(p.r + o + lo); d[1] = ld4(p.k + o + lo); d[2] = ld4(p.v + o + lo);
+        };
+        auto put = [&](const int c, SlotF& s, const f32x4 (&d)[3]) __attribute__((always_inline)) {
+            f32x4 r = d[0], k = d[1], v = d[2];
+            if (c * L + L > T && c * L + row >= T) { r = ZERO4; k = ZERO4; v = ZERO4; }
+            st4(&s.r[row][c4], r); st4(&s.k[row][c4], k); st4(&s.v[row][c4], v);
+            const f32x4 rk = r * k;
+            const float a = row_sum((rk[0] * u[0] + rk[1] * u[1]) + (rk[2] * u[2] + rk[3] * u[3]));
+            if ((tp & 15) == 0) s.ruk[row] = a;
+            if constexpr (TWO) {
+                const float a2 = row_sum((rk[0] + rk[1]) + (rk[2] + rk[3]));
+                if ((tp & 15) == 0) s.rk[row] = a2;
+            }
+        };
+#pragma unroll
+        for (int z = 0; z < FDEPTH; ++z) fetch(z, x[z]);
+        put(0, S.slot[0], x[0]); fetch(FDEPTH, x[0]);
+        put(1, S.slot[1], x[1]); fetch(FDEPTH + 1, x[1]);
+        __syncthreads();
+        __syncthreads();
+        int sl = 2;
+        for (int c0 = 0; c0 < nch; c0 += FDEPTH) {
+#pragma unroll
+            for (int z = 0; z < FDEPTH; ++z) {
+                const int c = c0 + z;
+                if (c >= nch) break;
+                put(c + 2, S.slot[sl], x[(z + 2) % FDEPTH]);
+                fetch(c + 2 + FDEPTH, x[(z + 2) % FDEPTH]);
+                sl = sl == 2 ? 0 : sl + 1;
+                __syncthreads();
+            }
+        }
+        return;
+    }
+    if (strong) fwd_products<TWO, true>(S, p, q, lane, base, nch);
+    else fwd_products<TWO, false>(S, p, q, lane, base, nch);
+}
+
 // ---------------------------------------------------------------------------------------------------- backward
-// One reverse sweep, one barrier a chunk, eight waves:
-//   D, waves 0..3 (key channel j = 16 q + l16): the states of a segment, rebuilt from the saved one, and the gradient state as
-//      S[i = 16 ib + 4 g + v][j]: the B operands of contractions over the value channel.  gr, gk, gw, gu.
-//   E, waves 4..7 (value channel i = 16 q + l16): the gradient state transposed, D[i][j = 16 jt + 4 g + v].  gv; the halves of
-//      the next chunk's two tiles (waves 4, 5 the A tile, 6, 7 the B tile); all loads, SEG chunks ahead of their use.
-// The planes in LDS are the raw inputs: every power is applied to an operand on its way into the matrix instruction, from
-// registers, so that a chunk costs four planes instead of one per power.
-struct SlotB {
+// One reverse sweep, one barrier a chunk, eight waves, two roles of four:
+//   D, waves 0..3 (key channel j = 16 q + l16): the states of a segment, rebuilt from the saved one, and the gradient state, both
+//      as S[i = 16 ib + 4 g + v][j], the B operands of contractions over the value channel: gr, gk, gw, gu.  The gradient state
+//      goes through LDS to the E waves, which take it transposed (a second copy with an update of its own: 14 % more matrix
+//      instructions).
+//   E, waves 4..7 (value channel i = 16 q + l16): gv; the halves of the next chunk's two tiles (two waves the A tile, two the B
+//      tile); all loads, SEG chunks ahead of their use.
+// (Three roles on twelve waves, S and D apart: 168 registers a wave did not hold them, and no faster without the spills.)
+// The planes in LDS are the raw inputs (two-sided: two scaled ones in addition): a power is applied to an operand on its way
+// into the matrix instruction, from registers, so that a chunk costs four planes instead of one per power.
+template <bool TWO> struct SlotB {
     float r[L][PS], k[L][PS], v[L][PS], g[L][PS];
+    float gs_[TWO ? L : 1][PS], ve_[TWO ? L : 1][PS];       // two-sided: gy o2^t, v o2^{15-t}, which would take 64 registers as powers
     float vg[L], u2vg[L], ruk[L], rk[L];
 };
 template <bool TWO> struct SmemB {
     Head hd;
-    SlotB slot[2 * SEG<TWO>];
+    SlotB<TWO> slot[2 * SEG<TWO>];
     float part[2][4][L][TS];            // halves of the tiles A (0, 1) and B (2, 3)
-    float red[4][N];
+    float ds[2][N][PS];                 // the gradient state of the chunk, for the E waves: [chunk parity][i][j]
+    float red[TWO ? 4 : 1][N];          // two-sided: the waves' sums over j of the per-element gradient
 };
 
-template <bool TWO>
-DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, int h, int b, size_t base, int nch) {
+// LDS by byte offset: the position of the chunk's slot (uniform) plus one of a few per-lane offsets, everything else an
+// immediate of the instruction.  The sum is hidden from the optimiser once per chunk: left alone it keeps (lane offset + field)
+// of every field in a register of its own across the loop, and spills them.
+extern __shared__ __align__(16) unsigned char smem_raw[];
+DEVINL f32x4 lds4(uint32_t o) { return *reinterpret_cast<const f32x4*>(smem_raw + o); }
+DEVINL float lds1(uint32_t o) { return *reinterpret_cast<const float*>(smem_raw + o); }
+DEVINL uint32_t hide(uint32_t o) { asm volatile("" : "+v"(o)); return o; }
+constexpr uint32_t ROWB = PS * 4, TROWB = TS * 4, TILEB = L * TROWB;
+// rows 4 g + v, v = 0..3, of one column
+template <uint32_t STRIDE = ROWB> DEVINL f32x4 col4(uint32_t o) { return f32x4{lds1(o), lds1(o + STRIDE), lds1(o + 2 * STRIDE), lds1(o + 3 * STRIDE)}; }
+template <bool TWO> struct At {                            // byte offsets within LDS and within a slot
+    using M = SmemB<TWO>;
+    using B = SlotB<TWO>;
+    static constexpr uint32_t DEC2 = offsetof(M, hd) + offsetof(Head, dec2), PART = offsetof(M, part), DS = offsetof(M, ds), DSB = sizeof(M::ds) / 2;
+    static constexpr uint32_t R = offsetof(B, r), K = offsetof(B, k), V = offsetof(B, v), GY = offsetof(B, g);
+    static constexpr uint32_t GS = TWO ? offsetof(B, gs_) : GY, VE = TWO ? offsetof(B, ve_) : V;       // gy o2^t, v o2^{15-t}
+    static constexpr uint32_t VG = offsetof(B, vg), U2VG = offsetof(B, u2vg), RUK = offsetof(B, ruk), RK = offsetof(B, rk);
+    static DEVINL uint32_t slot(int c) { return offsetof(M, slot) + static_cast<uint32_t>(c % (2 * SEG<TWO>)) * sizeof(B); }
+    static DEVINL uint32_t tile(int c, int half) { return PART + static_cast<uint32_t>((c & 1) * 4 + half) * TILEB; }
+    static DEVINL uint32_t ds(int c) { return DS + static_cast<uint32_t>(c & 1) * DSB; }
+};
+
+// One half (32 channels, two 16-channel blocks) of a causal tile sum_c X[t][c] Y[s][c], s < t, from the plane rows at x and y to
+// the tile column at out, with the powers cx (of t = l16) and cy (of s = l16) per channel block and register; w4: half of what
+// pairs across the halves of a strong chunk carry.
+template <bool SCALED, bool STRONG>
+DEVINL void half_tile(uint32_t x, uint32_t y, uint32_t out, const F4 (&cx)[2], const F4 (&cy)[2], const F4 (&w4)[2], int l16, int g) {
+    f32x4 d[2] = {ZERO4, ZERO4};
+    f32x4 xa[2], ya[2];
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+        xa[z] = lds4(x + 64 * z); ya[z] = lds4(y + 64 * z);
+        if constexpr (SCALED) { xa[z] = xa[z] * cx[z]; ya[z] = ya[z] * cy[z]; }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int z = 0; z < 2; ++z) d[z] = mm(xa[z][v], ya[z][v], d[z]);
+    f32x4 acc = d[0] + d[1];
+    if constexpr (SCALED && STRONG) {
+        f32x4 o = ZERO4;
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) o = mm(xa[z][v] * w4[z][v], ya[z][v] * w4[z][v], o);
+        if (g >= 2 && l16 < 8) acc = o;
+    }
+    // acc[v] = tile[t = 4 g + v][s = l16]
+#pragma unroll
+    for (int v = 0; v < 4; ++v) *reinterpret_cast<float*>(smem_raw + out + v * TROWB) = l16 < 4 * g + v ? acc[v] : 0.f;
+}
+// the gradient state from the D waves' layout, x[ib][v] = D[i = 16 ib + 4 g + v][j = own], to LDS as rows
+DEVINL void hand_over(uint32_t o, const f32x4 (&x)[4]) {
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) *reinterpret_cast<float*>(smem_raw + o + (16 * ib + v) * ROWB) = x[ib][v];
+}
+DEVINL float sum4(const f32x4& x) { return (x[0] + x[1]) + (x[2] + x[3]); }
+// two-sided: a lane's per-element sums acc[i = 16 ib + 4 g + v][j] summed over the wave's sixteen j
+DEVINL void reduce_cols(float* red, const f32x4 (&acc)[4], int l16, int g) {
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float x = row_sum(acc[ib][v]);
+            if (l16 == 0) red[16 * ib + 4 * g + v] = x;
+        }
+}
+DEVINL void store_chunk(float* p, size_t base, int c, int g, int own, int C, int T, const f32x4& x) {
+    store_rows(p + base + static_cast<size_t>(c) * L * C, 4 * g * C + own, C, T - c * L - 4 * g, c * L + L <= T, x);
+}
+
+template <bool TWO, bool STRONG>
+DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b, size_t base, int nch) {
     constexpr int G = SEG<TWO>;
+    using A = At<TWO>;
     const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = p.T;
+    const uint32_t orow = l16 * ROWB + 16 * g, ocol = 4 * g * ROWB + 4 * own, oall = 4 * g * ROWB + 4 * l16;      // [l16][4 g ..], [4 g + v][own], [4 g + v][l16]
+    const uint32_t otr = l16 * TROWB + 16 * g, otc = 4 * g * TROWB + 4 * l16;
     const int nseg = (nch + G - 1) / G;
     const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * nseg * N * N + 4 * g * N + own;
     const float l1 = S.hd.lam[own], u1 = S.hd.u[own], d1 = S.hd.dec[own], w4 = wpow(l1, 4.f);
-    f32x4 cs, ce, cm, ck, tf;                            // o1^t, o1^{15-t}, o1^{t-m}, o1^{m-1-t} and t for t = 4 g + v
+    F4 cs, ce, cm, ck, tf, tr15, lag;                    // o1^t, o1^{15-t}, o1^{t-m}, o1^{m-1-t}, t, 15 - t for t = 4 g + v; t' - 1 - t for t' = l16
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        const int t = 4 * g + v, m = ref(strong, t);
-        tf[v] = static_cast<float>(t);
+        const int t = 4 * g + v, m = ref<STRONG>(t);
+        tf[v] = static_cast<float>(t); tr15[v] = static_cast<float>(15 - t); lag[v] = static_cast<float>(l16 - 1 - t);
         cs[v] = wpow(l1, static_cast<float>(t)); ce[v] = wpow(l1, static_cast<float>(15 - t));
         cm[v] = wpow(l1, static_cast<float>(t - m)); ck[v] = wpow(l1, static_cast<float>(m - 1 - t));
-    }
-    // two-sided: powers of the value side for the A operands gy o2^t, v o2^{15-t} with token l16 / token 4 g + v in the lane
-    f32x4 gx[TWO ? 4 : 1], vx[TWO ? 4 : 1], gup[TWO ? 4 : 1], vup[TWO ? 4 : 1];
-    if constexpr (TWO) {
-#pragma unroll
-        for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float la = S.hd.lam2[16 * ib + 4 * g + v], lb = S.hd.lam2[16 * ib + l16];
-                gx[ib][v] = wpow(la, static_cast<float>(l16)); vx[ib][v] = wpow(la, static_cast<float>(15 - l16));
-                gup[ib][v] = wpow(lb, static_cast<float>(4 * g + v)); vup[ib][v] = wpow(lb, static_cast<float>(15 - 4 * g - v));
-            }
     }
     f32x4 St[G][4], Sn[4], dS[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
     f32x4 accG[TWO ? 4 : 1];
@@ -379,85 +450,74 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, 
             for (int v = 0; v < 4; ++v) Sn[ib][v] = s > 0 ? d[(16 * ib + v) * N] : 0.f;      // the sequence starts from nothing
     };
     auto decay = [&](const int ib) __attribute__((always_inline)) {
-        if constexpr (TWO) return ld4(&S.hd.dec2[16 * ib + 4 * g]) * d1;
+        if constexpr (TWO) return lds4(hide(16 * g) + A::DEC2 + 64 * ib) * d1;
         else return f32x4{d1, d1, d1, d1};
     };
-    const int lo = 4 * g * C + own;
-    auto chunk = [&](const int c, const f32x4 (&Sz)[4]) __attribute__((always_inline)) {
-        const SlotB& X = S.slot[c % (2 * G)];
-        const float (*pb)[L][TS] = &S.part[c & 1][2];
-        f32x4 kk, rr, bt;
+    // rows of the value side for the next chunk, asked for before the barrier that ends this one (they have been there since
+    // long ago; the first matrix instructions after a barrier would wait for all waves' reads at once)
+    f32x4 gx[4], vx[4];
+    auto rows = [&](const int c) __attribute__((always_inline)) {
+        const uint32_t xr = hide(A::slot(max(c, 0)) + orow);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            kk[v] = X.k[4 * g + v][own]; rr[v] = X.r[4 * g + v][own];
-            bt[v] = pb[0][4 * g + v][l16] + pb[1][4 * g + v][l16];
-        }
-        const f32x4 bm = ld4(&pb[0][l16][4 * g]) + ld4(&pb[1][l16][4 * g]);
+        for (int ib = 0; ib < 4; ++ib) { gx[ib] = lds4(xr + A::GS + 64 * ib); vx[ib] = lds4(xr + A::VE + 64 * ib); }
+    };
+    auto chunk = [&](const int c, const f32x4 (&Sz)[4]) __attribute__((always_inline)) {
+        const uint32_t sx = A::slot(c), xc = hide(sx + ocol), xd = hide(sx + oall), xg = hide(sx + 16 * g);
+        const uint32_t tr = hide(A::tile(c, 2) + otr), tc = hide(A::tile(c, 2) + otc);
         f32x4 x2[2] = {ZERO4, ZERO4}, z2[2] = {ZERO4, ZERO4};
 #pragma unroll
         for (int ib = 0; ib < 4; ++ib) {
-            f32x4 ga = ld4(&X.g[l16][16 * ib + 4 * g]), va = ld4(&X.v[l16][16 * ib + 4 * g]);
-            if constexpr (TWO) { ga *= gx[ib]; va *= vx[ib]; }
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                x2[ib & 1] = mm(ga[v], Sz[ib][v], x2[ib & 1]);
-                z2[ib & 1] = mm(va[v], dS[ib][v], z2[ib & 1]);
+                x2[ib & 1] = mm(gx[ib][v], Sz[ib][v], x2[ib & 1]);
+                z2[ib & 1] = mm(vx[ib][v], dS[ib][v], z2[ib & 1]);
             }
         }
-        const f32x4 km = kk * ck, rm = rr * cm;
-        const bool cx = l16 >= 8 && g < 2, cz = l16 < 8 && g >= 2;
-        f32x4 lag;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) lag[v] = static_cast<float>(l16 - 1) - tf[v];
-        const f32x4 tx = apply(bm, km, strong, cx, w4), tl = apply(bm * lag, km, strong, cx, w4), tz = apply(bt, rm, strong, cz, w4);
-        const f32x4 xs = (x2[0] + x2[1]) * cs, zs = (z2[0] + z2[1]) * ce;
-        const f32x4 vg = ld4(&X.vg[4 * g]);
-        f32x4 bo = vg * u1;
-        if constexpr (TWO) bo += ld4(&X.u2vg[4 * g]);
-        const f32x4 dr = xs + tx * cm + kk * bo, dk = zs + tz * ck + rr * bo;
-        const size_t o = base + static_cast<size_t>(c) * L * C;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (c * L + 4 * g + v < T) {
-                (p.gr + o + static_cast<size_t>(v) * C)[lo] = dr[v];
-                (p.gk + o + static_cast<size_t>(v) * C)[lo] = dk[v];
-            }
-        const f32x4 gu4 = rr * kk * vg, gw4 = rm * tl;
-        gu += (gu4[0] + gu4[1]) + (gu4[2] + gu4[3]);
-        gw += (gw4[0] + gw4[1]) + (gw4[2] + gw4[3]);
+        const f32x4 kk = col4(xc + A::K), rr = col4(xc + A::R);
         const f32x4 rs = rr * cs;
         if constexpr (TWO) {
-            const f32x4 rt = rs * tf, kt = kk * ce * (15.f - tf);
+            const f32x4 rt = rs * tf, kt = kk * ce * tr15;
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) {
-                const f32x4 dec = decay(ib);
+                const f32x4 ga = col4(xd + A::GS + 64 * ib), va = col4(xd + A::VE + 64 * ib), dec = decay(ib);
                 f32x4 m1 = ZERO4, n1 = ZERO4, acc = dS[ib] * dec;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const float ga = X.g[4 * g + v][16 * ib + l16] * gup[ib][v], va = X.v[4 * g + v][16 * ib + l16] * vup[ib][v];
-                    m1 = mm(ga, rt[v], m1);
-                    n1 = mm(va, kt[v], n1);
-                    acc = mm(ga, rs[v], acc);
-                }
-                accG[ib] += Sz[ib] * m1 + dS[ib] * n1 + (16.f * dec) * (Sz[ib] * dS[ib]);
+                for (int v = 0; v < 4; ++v) { m1 = mm(ga[v], rt[v], m1); n1 = mm(va[v], kt[v], n1); acc = mm(ga[v], rs[v], acc); }
+                accG[ib] += Sz[ib] * (m1 + (16.f * dec) * dS[ib]) + dS[ib] * n1;
                 dS[ib] = acc;
             }
         } else {
-            const f32x4 gs4 = tf * rr * xs + (15.f - tf) * kk * zs;
-            gw += (gs4[0] + gs4[1]) + (gs4[2] + gs4[3]);
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) {
-                const f32x4 pp = Sz[ib] * dS[ib];
-                gP += (pp[0] + pp[1]) + (pp[2] + pp[3]);
+                const f32x4 ga = col4(xd + A::GS + 64 * ib);
+                gP += sum4(Sz[ib] * dS[ib]);
                 f32x4 acc = dS[ib] * d1;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc = mm(X.g[4 * g + v][16 * ib + l16], rs[v], acc);
+                for (int v = 0; v < 4; ++v) acc = mm(ga[v], rs[v], acc);
                 dS[ib] = acc;
             }
         }
+        if (c > 0) hand_over(hide(A::ds(c - 1) + ocol), dS);
+        if constexpr (!TWO) rows(c - 1);
+        const f32x4 bm = lds4(tr) + lds4(tr + TILEB), bt = col4<TROWB>(tc) + col4<TROWB>(tc + TILEB);
+        const f32x4 km = kk * ck, rm = rr * cm;
+        const bool cx = l16 >= 8 && g < 2, cz = l16 < 8 && g >= 2;
+        const f32x4 tx = apply<STRONG>(bm, km, cx, w4), tl = apply<STRONG>(bm * lag, km, cx, w4), tz = apply<STRONG>(bt, rm, cz, w4);
+        const f32x4 xs = (x2[0] + x2[1]) * cs, zs = (z2[0] + z2[1]) * ce;
+        const f32x4 vg = lds4(xg + A::VG);
+        f32x4 bo = vg * u1;
+        if constexpr (TWO) bo += lds4(xg + A::U2VG);
+        gu += sum4(rr * kk * vg);
+        gw += sum4(rm * tl);
+        if constexpr (!TWO) gw += sum4(rr * xs * tf + kk * zs * tr15);
+        store_chunk(p.gr, base, c, g, own, C, T, xs + tx * cm + kk * bo);
+        store_chunk(p.gk, base, c, g, own, C, T, zs + tz * ck + rr * bo);
+        if constexpr (TWO) rows(c - 1);                  // (earlier, under the products above, the registers do not reach for this)
     };
     fetch_state(nseg - 1);
+    hand_over(A::ds(nch - 1) + ocol, dS);
     __syncthreads();                                     // the top chunks are there
+    rows(nch - 1);
     __syncthreads();                                     // and the first tiles
     for (int s = nseg - 1; s >= 0; --s) {
 #pragma unroll
@@ -466,27 +526,23 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, 
 #pragma unroll
         for (int z = 0; z + 1 < G; ++z) {
             if (s * G + z + 1 < nch) {
-                const SlotB& X = S.slot[(s * G + z) % (2 * G)];
-                f32x4 ke;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) ke[v] = X.k[4 * g + v][own] * ce[v];
+                const uint32_t sx = A::slot(s * G + z), xc = hide(sx + ocol), xd = hide(sx + oall);
+                const f32x4 ke = col4(xc + A::K) * ce;
 #pragma unroll
                 for (int ib = 0; ib < 4; ++ib) {
+                    const f32x4 va = col4(xd + A::VE + 64 * ib);
                     f32x4 acc = St[z][ib] * decay(ib);
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        float va = X.v[4 * g + v][16 * ib + l16];
-                        if constexpr (TWO) va *= vup[ib][v];
-                        acc = mm(va, ke[v], acc);
-                    }
+                    for (int v = 0; v < 4; ++v) acc = mm(va[v], ke[v], acc);
                     St[z + 1][ib] = acc;
                 }
             }
         }
 #pragma unroll
         for (int z = G - 1; z >= 0; --z) {
-            if (s * G + z < nch) {
-                chunk(s * G + z, St[z]);
+            const int c = s * G + z;
+            if (c < nch) {
+                chunk(c, St[z]);
                 __syncthreads();
             }
         }
@@ -494,15 +550,10 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, 
     gw = fmaf(16.f * d1, gP, gw);
     if constexpr (TWO) {
 #pragma unroll
-        for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                gw += accG[ib][v];
-                const float x = row_sum(accG[ib][v]);
-                if (l16 == 0) S.red[q][16 * ib + 4 * g + v] = x;
-            }
-        __syncthreads();
+        for (int ib = 0; ib < 4; ++ib) gw += sum4(accG[ib]);
+        reduce_cols(S.red[q], accG, l16, g);
     }
+    __syncthreads();
     gw = allreduce_rows(gw); gu = allreduce_rows(gu);
     if (g == 0) {
         const float lt = -expf(p.w[h * N + own]);        // (a decay below the smallest one: its gradient is that of the pairs one step apart)
@@ -512,13 +563,26 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, 
     }
 }
 
-template <bool TWO>
-DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, int h, int b, size_t base, int nch) {
+template <bool TWO, bool STRONG>
+DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b, size_t base, int nch) {
     constexpr int G = SEG<TWO>;
+    using A = At<TWO>;
     const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = p.T;
+    const uint32_t orow = l16 * ROWB + 16 * g, ocol = 4 * g * ROWB + 4 * own;                // [l16][4 g ..], [4 g + v][own]
+    const uint32_t otr = l16 * TROWB + 16 * g, otc = 4 * g * TROWB + 4 * l16, odt = own * ROWB + 16 * g;
     const int te = 64 * q + lane, row = te >> 4, c4 = (te & 15) * 4;
-    // loads
-    const f32x4 u = ld4(&S.hd.u[c4]), u2c = ld4(&S.hd.u2[c4]);
+    // loads: chunk c - G is written in the phase of chunk c, out of registers that asked for it G phases before
+    F4 u, u2c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { u[e] = S.hd.u[c4 + e]; u2c[e] = S.hd.u2[c4 + e]; }
+    F4 pgs = {}, pve = {};
+    if constexpr (TWO) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            pgs[e] = wpow(S.hd.lam2[c4 + e], static_cast<float>(row));
+            pve[e] = wpow(S.hd.lam2[c4 + e], static_cast<float>(15 - row));
+        }
+    }
     auto fetch = [&](const int c, f32x4 (&d)[4]) __attribute__((always_inline)) {
         const int cc = max(c, 0);
         const size_t o = base + static_cast<size_t>(cc) * L * C;
@@ -526,150 +590,135 @@ DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, bool strong, int q, int lane, 
         d[0] = ld4(p.r + o + lo); d[1] = ld4(p.k + o + lo); d[2] = ld4(p.v + o + lo); d[3] = ld4(p.gy + o + lo);
     };
     auto put = [&](const int c, const f32x4 (&d)[4]) __attribute__((always_inline)) {
-        SlotB& s = S.slot[c % (2 * G)];
-        const bool ok = c * L + row < T;
-        const f32x4 r = ok ? d[0] : ZERO4, k = ok ? d[1] : ZERO4, v = ok ? d[2] : ZERO4, gy = ok ? d[3] : ZERO4;
+        SlotB<TWO>& s = S.slot[c % (2 * G)];
+        f32x4 r = d[0], k = d[1], v = d[2], gy = d[3];
+        if (c * L + L > T && c * L + row >= T) { r = ZERO4; k = ZERO4; v = ZERO4; gy = ZERO4; }
         st4(&s.r[row][c4], r); st4(&s.k[row][c4], k); st4(&s.v[row][c4], v); st4(&s.g[row][c4], gy);
+        if constexpr (TWO) { st4(&s.gs_[row][c4], gy * pgs); st4(&s.ve_[row][c4], v * pve); }
         const f32x4 rk = r * k, vg = v * gy;
-        const float a = row_sum((rk[0] * u[0] + rk[1] * u[1]) + (rk[2] * u[2] + rk[3] * u[3]));
-        const float e = row_sum((vg[0] + vg[1]) + (vg[2] + vg[3]));
+        const float a = row_sum(sum4(rk * u)), e = row_sum(sum4(vg));
         if ((te & 15) == 0) { s.ruk[row] = a; s.vg[row] = e; }
         if constexpr (TWO) {
-            const float a2 = row_sum((rk[0] + rk[1]) + (rk[2] + rk[3]));
-            const float e2 = row_sum((vg[0] * u2c[0] + vg[1] * u2c[1]) + (vg[2] * u2c[2] + vg[3] * u2c[3]));
+            const float a2 = row_sum(sum4(rk)), e2 = row_sum(sum4(vg * u2c));
             if ((te & 15) == 0) { s.rk[row] = a2; s.u2vg[row] = e2; }
         }
     };
-    f32x4 ring[2][4];
+    f32x4 ring[G][4];
     {
         f32x4 top[G][4];
 #pragma unroll
         for (int z = 0; z < G; ++z) fetch(nch - 1 - z, top[z]);
 #pragma unroll
-        for (int z = 0; z < 2; ++z) {
-            // chunk nch - 1 - G is written in the first chunk's phase, from ring[(nch - 1) & 1]
-            if ((nch - 1) & 1) fetch(nch - 1 - G - z, ring[1 - z]);
-            else fetch(nch - 1 - G - z, ring[z]);
-        }
-#pragma unroll
         for (int z = 0; z < G; ++z)
             if (nch - 1 - z >= 0) put(nch - 1 - z, top[z]);
     }
-    // powers: A operands over j, k o1^{15-t} (token l16) and r o1^t (token 4 g + v); the tile half of this wave
-    f32x4 cke[4], crs[4], tx[2], ty[2], t4[2];
+    // the segment's position of chunk c - G is that of chunk c: its registers are ring[c % G]
+    const int ctop = nch - 1 - (nch - 1) % G;            // first chunk of the top segment
+#pragma unroll
+    for (int z = 0; z < G; ++z) fetch(ctop + z < nch ? ctop + z - G : ctop + z - 2 * G, ring[z]);
+
+    // powers: the A operand k o1^{15-t} (token l16); the tile half of this wave
+    F4 cke[4], tx[2], ty[2], t4[2], lag;
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            cke[jt][v] = wpow(S.hd.lam[16 * jt + 4 * g + v], static_cast<float>(15 - l16));
-            crs[jt][v] = wpow(S.hd.lam[16 * jt + l16], static_cast<float>(4 * g + v));
-        }
+        for (int v = 0; v < 4; ++v) cke[jt][v] = wpow(S.hd.lam[16 * jt + 4 * g + v], static_cast<float>(15 - l16));
     const int cb0 = 2 * (q & 1);
-    tile_powers(q < 2 ? S.hd.lam : S.hd.lam2, cb0, strong, l16, g, tx, ty, t4);
+    tile_powers<STRONG>(q < 2 ? S.hd.lam : S.hd.lam2, cb0, l16, g, tx, ty, t4);
     auto tile = [&](const int c) __attribute__((always_inline)) {
-        const SlotB& X = S.slot[c % (2 * G)];
-        float (*out)[TS] = S.part[c & 1][q];
-        if (q < 2) half_tile<true>(X.r, X.k, out, cb0, tx, ty, t4, strong, l16, g);
-        else half_tile<TWO>(X.g, X.v, out, cb0, tx, ty, t4, strong, l16, g);
+        const uint32_t xr = hide(A::slot(c) + orow + 64 * cb0), out = hide(A::tile(c, q) + otc);
+        if (q < 2) half_tile<true, STRONG>(xr + A::R, xr + A::K, out, tx, ty, t4, l16, g);
+        else half_tile<TWO, STRONG>(xr + A::GY, xr + A::V, out, tx, ty, t4, l16, g);
     };
-    f32x4 c2s = ZERO4, c2e = ZERO4, c2m = ZERO4, c2k = ZERO4;
-    float u2 = 0.f, d2 = 1.f, w24 = 1.f, gw2 = 0.f, gu2 = 0.f;
+    F4 c2e = {}, c2m = {}, c2k = {};
+    float u2 = 0.f, w24 = 1.f, gw2 = 0.f, gu2 = 0.f;
     const float l2 = S.hd.lam2[own];
     if constexpr (TWO) {
-        u2 = S.hd.u2[own]; d2 = S.hd.dec2[own]; w24 = wpow(l2, 4.f);
+        u2 = S.hd.u2[own]; w24 = wpow(l2, 4.f);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int t = 4 * g + v, m = ref(strong, t);
-            c2s[v] = wpow(l2, static_cast<float>(t)); c2e[v] = wpow(l2, static_cast<float>(15 - t));
+            const int t = 4 * g + v, m = ref<STRONG>(t);
+            c2e[v] = wpow(l2, static_cast<float>(15 - t));
             c2m[v] = wpow(l2, static_cast<float>(t - m)); c2k[v] = wpow(l2, static_cast<float>(m - 1 - t));
+            lag[v] = static_cast<float>(l16 - 1 - t);
         }
     }
-    f32x4 dT[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
-    const int lo = 4 * g * C + own;
-    auto chunk = [&](const int c, f32x4 (&rg)[4]) __attribute__((always_inline)) {
-        const SlotB& X = S.slot[c % (2 * G)];
-        const float (*pa)[L][TS] = &S.part[c & 1][0];
+    __syncthreads();
+    tile(nch - 1);
+    __syncthreads();
+    auto chunk = [&](const int c) __attribute__((always_inline)) {
+        const uint32_t sx = A::slot(c), xr = hide(sx + orow), xc = hide(sx + ocol), xg = hide(sx + 16 * g);
+        const uint32_t dt0 = hide(A::ds(c) + odt), tc = hide(A::tile(c, 0) + otc);
         f32x4 go, aT;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { go[v] = X.g[4 * g + v][own]; aT[v] = pa[0][4 * g + v][l16] + pa[1][4 * g + v][l16]; }
         f32x4 y2[2] = {ZERO4, ZERO4};
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
-            const f32x4 ka = ld4(&X.k[l16][16 * jt + 4 * g]) * cke[jt];
+            const f32x4 ka = lds4(xr + A::K + 64 * jt) * cke[jt], dt = lds4(dt0 + 64 * jt);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) y2[jt & 1] = mm(ka[v], dT[jt][v], y2[jt & 1]);
+            for (int v = 0; v < 4; ++v) y2[jt & 1] = mm(ka[v], dt[v], y2[jt & 1]);
         }
-        const f32x4 ruk = ld4(&X.ruk[4 * g]);
+        go = col4(xc + A::GY); aT = col4<TROWB>(tc) + col4<TROWB>(tc + TILEB);
+        const f32x4 ruk = lds4(xg + A::RUK);
         f32x4 dv = y2[0] + y2[1];
         if constexpr (TWO) {
-            const f32x4 rk = ld4(&X.rk[4 * g]), gm = go * c2m;
-            dv = dv * c2e + apply(aT, gm, strong, l16 < 8 && g >= 2, w24) * c2k + go * (ruk + u2 * rk);
-            f32x4 vo, lag;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) { vo[v] = X.v[4 * g + v][own]; lag[v] = static_cast<float>(l16 - 1 - 4 * g - v); }
-            const f32x4 a = ld4(&pa[0][l16][4 * g]) + ld4(&pa[1][l16][4 * g]);
-            const f32x4 w4 = gm * apply(a * lag, vo * c2k, strong, l16 >= 8 && g < 2, w24), u4 = vo * go * rk;
-            gw2 += (w4[0] + w4[1]) + (w4[2] + w4[3]);
-            gu2 += (u4[0] + u4[1]) + (u4[2] + u4[3]);
+            const f32x4 rk = lds4(xg + A::RK), gm = go * c2m, vo = col4(xc + A::V);
+            dv = dv * c2e + apply<STRONG>(aT, gm, l16 < 8 && g >= 2, w24) * c2k + go * (ruk + u2 * rk);
+            const uint32_t tr = hide(A::tile(c, 0) + otr);
+            const f32x4 a = lds4(tr) + lds4(tr + TILEB);
+            gw2 += sum4(gm * apply<STRONG>(a * lag, vo * c2k, l16 >= 8 && g < 2, w24));
+            gu2 += sum4(vo * go * rk);
         } else {
             dv += go * ruk;
 #pragma unroll
             for (int v = 0; v < 4; ++v) dv = mm(aT[v], go[v], dv);
         }
-        float* const out = p.gv + base + static_cast<size_t>(c) * L * C;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (c * L + 4 * g + v < T) (out + static_cast<size_t>(v) * C)[lo] = dv[v];
-        const f32x4 gs = TWO ? go * c2s : go;
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) {
-            f32x4 acc = dT[jt] * ld4(&S.hd.dec[16 * jt + 4 * g]);
-            if constexpr (TWO) acc *= d2;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc = mm(X.r[4 * g + v][16 * jt + l16] * crs[jt][v], gs[v], acc);
-            dT[jt] = acc;
-        }
+        store_chunk(p.gv, base, c, g, own, C, T, dv);
         if (c > 0) tile(c - 1);
-        if (c >= G) put(c - G, rg);
-        fetch(c - G - 2, rg);
     };
-    __syncthreads();
-    tile(nch - 1);
-    __syncthreads();
-    const int nseg = (nch + G - 1) / G;
-    for (int s = nseg - 1; s >= 0; --s) {
+    for (int s = (nch - 1) / G; s >= 0; --s) {
 #pragma unroll
         for (int z = G - 1; z >= 0; --z) {
-            if (s * G + z < nch) {
-                chunk(s * G + z, ring[z & 1]);
+            const int c = s * G + z;
+            if (c < nch) {
+                chunk(c);
+                if (c >= G) put(c - G, ring[z]);
+                fetch(c - 2 * G, ring[z]);
                 __syncthreads();
             }
         }
     }
+    __syncthreads();
     if constexpr (TWO) {
-        __syncthreads();
         gw2 = allreduce_rows(gw2); gu2 = allreduce_rows(gu2);
         if (g == 0) {
             const float lt = -expf(p.w2[h * N + own]);
             const size_t o = static_cast<size_t>(b) * C + h * N + own;
-            p.gw2[o] = lt * expf(lt - l2) * (gw2 + ((S.red[0][own] + S.red[1][own]) + (S.red[2][own] + S.red[3][own])));
+#pragma unroll
+            for (int z = 0; z < 4; ++z) gw2 += S.red[z][own];
+            p.gw2[o] = lt * expf(lt - l2) * gw2;
             p.gu2[o] = gu2;
         }
     }
 }
 
+template <bool TWO, bool STRONG>
+DEVINL void bwd_roles(SmemB<TWO>& S, const ArgsC& p, int w, int lane, int h, int b, size_t base, int nch) {
+    const int q = w & 3;
+    if (w < 4) role_d<TWO, STRONG>(S, p, q, lane, h, b, base, nch);
+    else role_e<TWO, STRONG>(S, p, q, lane, h, b, base, nch);
+}
+
 template <bool TWO>
-__global__ __launch_bounds__(NT, 2) void wkv5c_bwd(const ArgsC p) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
+__global__ __launch_bounds__(NTB, 2) void wkv5c_bwd(const ArgsC p) {
     SmemB<TWO>& S = *reinterpret_cast<SmemB<TWO>*>(smem_raw);
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = w & 3;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x % p.H, b = blockIdx.x / p.H;
     const int nch = (p.T + L - 1) / L;
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * N;
     const bool strong = head_setup<TWO>(S.hd, p, h, tid);
     __syncthreads();
-    if (w < 4) role_d<TWO>(S, p, strong, q, lane, h, b, base, nch);
-    else role_e<TWO>(S, p, strong, q, lane, h, b, base, nch);
+    if (strong) bwd_roles<TWO, true>(S, p, w, lane, h, b, base, nch);
+    else bwd_roles<TWO, false>(S, p, w, lane, h, b, base, nch);
 }
 
 // out[c] = sum over the batch of rows of up to four [B][C] arrays that lie behind each other
@@ -703,7 +752,7 @@ template <bool TWO> int start_bwd(void* stream, int B, const ArgsC& p, float* ro
                                                        static_cast<int>(sizeof(SmemB<TWO>)));
     if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(wkv5c_bwd<TWO>, dim3(B * p.H), dim3(NT), sizeof(SmemB<TWO>), st, p);
+    hipLaunchKernelGGL(wkv5c_bwd<TWO>, dim3(B * p.H), dim3(NTB), sizeof(SmemB<TWO>), st, p);
     hipLaunchKernelGGL(rows_sum, dim3((p.C + 255) / 256, TWO ? 4 : 2), dim3(256), 0, st, B, p.C, rows, gw, gu, gw2, gu2);
     return launch_status();
 }
