@@ -1,24 +1,19 @@
-"""Plumbing shared by the operator wrappers: tensor checks, stream and device handling."""
+"""The two ways from Python into the library: the operators as C++ autograd functions, and single C-ABI entry points."""
 
 import torch
 
 from . import _lib
 
-
-def require(cond, msg):
-    # the reference uses bare asserts (e.g. wkv6_state/run.py:84-100); an AssertionError keeps that contract
-    if not cond:
-        raise AssertionError(msg)
+_ops = None
 
 
-def check_tensors(tensors, dtype, names):
-    dev = tensors[0].device
-    require(dev.type == "cuda", "tensors must live on a HIP device: there is no CPU path")
-    for t, n in zip(tensors, names):
-        require(t.dtype == dtype, f"{n}.dtype must be {dtype}, got {t.dtype}")
-        require(t.is_contiguous(), f"{n} must be contiguous")
-        require(t.device == dev, f"{n} is on {t.device}, expected {dev}")
-    return dev
+def ops():
+    """The C++ autograd functions (csrc/autograd.cpp); loads the extension once."""
+    global _ops
+    if _ops is None:
+        from . import binding
+        _ops = binding.load().ops
+    return _ops
 
 
 def call(name, dev, *args):

@@ -10,6 +10,9 @@ csrc/binding.cpp is that shim for all nine extensions at once, calling the C ABI
     torch.ops.rwkv7_statepassing_clampw.forward(s0, r, w, k, v, a, b, y, sT, s, sa)
 
 build() compiles with torch.utils.cpp_extension (the same route as the reference) and keeps the result in-tree.
+
+csrc/autograd.cpp, in the same extension, holds the operators as C++ autograd functions (`ext.ops.*`): what the classes of
+this package's operator modules call.
 """
 import importlib.machinery
 import importlib.util
@@ -36,7 +39,7 @@ def _compile(verbose):
     rocm = os.environ.get("ROCM_HOME", "/opt/rocm")
     cpp_extension.load(
         name=NAME,
-        sources=[os.path.join(_HERE, "csrc", "binding.cpp")],
+        sources=[os.path.join(_HERE, "csrc", f) for f in ("binding.cpp", "autograd.cpp")],
         extra_include_paths=[os.path.join(os.path.dirname(_HERE), "include"), os.path.join(rocm, "include")],
         extra_cflags=["-O2", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"],
         # the dollar signs survive ninja and the shell as a literal $ORIGIN: the extension finds librwkv_hip.so beside itself
@@ -49,7 +52,7 @@ def _compile(verbose):
 
 
 def build(verbose=False):
-    """Compile csrc/binding.cpp against the built librwkv_hip.so with torch.utils.cpp_extension and keep the result
+    """Compile csrc/binding.cpp and csrc/autograd.cpp against the built librwkv_hip.so with torch.utils.cpp_extension and keep the result
     in-tree.  The compile runs in a child process: cpp_extension.load also loads what it built, and a TORCH_LIBRARY
     namespace can be registered only once per process, so the caller's process must load the in-tree copy alone."""
     if not os.path.exists(_lib.LIB_PATH):
@@ -59,7 +62,7 @@ def build(verbose=False):
     if verbose or res.returncode != 0:
         print(res.stdout, flush=True)
     if res.returncode != 0:
-        raise RuntimeError("building csrc/binding.cpp failed")
+        raise RuntimeError("building csrc/binding.cpp and csrc/autograd.cpp failed")
     shutil.copyfile(os.path.join(_BUILD_DIR, NAME + ".so"), SO_PATH)
     return SO_PATH
 

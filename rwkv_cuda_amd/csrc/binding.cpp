@@ -312,6 +312,8 @@ void r7_backward(Tensor& r, Tensor& w, Tensor& k, Tensor& v, Tensor& a, Tensor& 
 
 }  // namespace
 
+void bind_autograd(pybind11::module_& m);        // autograd.cpp: submodule `ops`
+
 // One Python extension module with a submodule per reference extension: `ext.wkv6state.forward(...)` is what
 // `wkv6state_cuda.forward(...)` is in wkv6_state/run.py:77,103.
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -331,6 +333,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     sub("rwkv7_clampw", &r7_forward, &r7_backward);
     sub("rwkv7_state_clampw", &r7s_forward, &r7s_backward);
     sub("rwkv7_statepassing_clampw", &r7sp_forward, &r7sp_backward);
+    bind_autograd(m);
 }
 
 TORCH_LIBRARY(wkv, m) { m.def("forward", wkv_forward); m.def("backward", wkv_backward); }

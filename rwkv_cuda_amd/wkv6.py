@@ -2,8 +2,8 @@
 
 import torch
 
-from . import _lib, options
-from ._call import call, check_tensors, require
+from . import options
+from ._call import ops
 
 HEAD_SIZE = 64          # the size the matrix-core kernels are written for; any size up to MAX_HEAD_SIZE runs
 MAX_HEAD_SIZE = 128
@@ -12,41 +12,12 @@ MAX_HEAD_SIZE = 128
 class WKV_6(torch.autograd.Function):
     """Same signature as WKV_6, wkv6/run.py:128-170: r,k,v,w[B,T,C], u[H,N] bf16, w raw.
     The reference wrapper computes ew = -exp(w.float()) (:147) and its kernel applies exp(ew); here the raw
-    w goes straight to the kernels (rwkv_wkv6raw_*), which evaluate the same two exponentials in fp32.
+    w goes straight to the kernels, which evaluate the same two exponentials in fp32.
     The fp32-ew entry points rwkv_wkv6_forward/backward stay available for callers of the C ABI."""
 
     @staticmethod
-    def forward(ctx, B, T, C, H, r, k, v, w, u):
-        with torch.no_grad():
-            dev = check_tensors((r, k, v, w, u), torch.bfloat16, "rkvwu")
-            require(C % H == 0 and C // H <= MAX_HEAD_SIZE, "C must be a multiple of H with a head size of at most 128")
-            require(r.numel() == B * T * C, "shape mismatch")
-            ctx.B, ctx.T, ctx.C, ctx.H = B, T, C, H
-            ctx.flags = options.current_flags()
-            y = torch.empty((B, T, C), device=dev, dtype=torch.bfloat16)
-            # the forward keeps the state entering every 64th token for the backward's single reverse sweep (no bytes for
-            # head sizes and options that take the two-sweep kernels)
-            nsaved = _lib.load().rwkv_wkv6f_saved_bytes(B, T, C, H)
-            saved = torch.empty(nsaved, device=dev, dtype=torch.uint8)
-            call("rwkv_wkv6f_forward", dev, B, T, C, H, r, k, v, w, u, None, y, saved if nsaved else None, nsaved, ctx.flags)
-            ctx.save_for_backward(r, k, v, w, u, saved)
-            return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        with torch.no_grad():
-            B, T, C, H = ctx.B, ctx.T, ctx.C, ctx.H
-            r, k, v, w, u, saved = ctx.saved_tensors
-            gy = gy.contiguous()
-            dev = check_tensors((gy,), torch.bfloat16, ("gy",))
-            new = lambda *shape: torch.empty(shape, device=dev, dtype=torch.bfloat16)
-            gr, gk, gv, gw = new(B, T, C), new(B, T, C), new(B, T, C), new(B, T, C)
-            gu = new(H, C // H)                               # summed over the batch by the library (:169)
-            nbytes = _lib.load().rwkv_wkv6f_backward_saved_workspace_bytes(B, T, C, H)
-            ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-            call("rwkv_wkv6f_backward_saved", dev, B, T, C, H, r, k, v, w, u, None, gy, gr, gk, gv, gw, gu, None,
-                 saved if saved.numel() else None, saved.numel(), ws, nbytes, ctx.flags)
-            return (None, None, None, None, gr, gk, gv, gw, gu)
+    def apply(B, T, C, H, r, k, v, w, u):
+        return ops().wkv6(B, T, C, H, r, k, v, w, u, options.current_flags())
 
 
 def RUN_CUDA(B, T, C, H, r, k, v, w, u):
