@@ -129,6 +129,8 @@ SIGNATURES = {
     "rwkv_timex_forward": (_I, [_P, _P, _P, _P, _F, _I, _I, _I]),
     "rwkv_timex_backward": (_I, [_P] * 6 + [_I, _I, _I]),
     "rwkv_timex_backward_sum": (_I, [_P] * 6 + [_I, _I, _I]),
+    "rwkv_timex_backward_ws_bytes": (_Z, [_I, _I, _I]),
+    "rwkv_timex_backward_ws": (_I, [_P] * 6 + [_I, _I, _I] + [_P, _Z]),
     "rwkv_wkv5_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 6),
     "rwkv_wkv5_forward_ex": (_I, [_P, _I, _I, _I, _I] + [_P] * 6 + [_U]),
     "rwkv_wkv5_forward_workspace_bytes": (_Z, [_I, _I, _I, _I]),

@@ -111,7 +111,7 @@ struct Wkv4 : Function<Wkv4> {
 Tensor wkv4_op(int64_t B, int64_t T, int64_t C, const Tensor& w, const Tensor& u, const Tensor& k, const Tensor& v) { return Wkv4::apply(B, T, C, w, u, k, v); }
 
 // --------------------------------------------------------------------------------------------- depthwise_conv1d (run.py:76-102)
-constexpr int64_t T_MAX = 4096, T_SUM_MAX = 1024;      // rwkv_timex_backward_sum: T % 32 == 0 and T <= 1024
+constexpr int64_t T_MAX = 4096;
 struct TimeX : Function<TimeX> {
     static Tensor forward(AutogradContext* ctx, const Tensor& w_, const Tensor& k_, int64_t B, int64_t C, int64_t T, double eps) {
         require(T % 4 == 0 && T <= T_MAX, "require T % 4 == 0 and T <= T_MAX");
@@ -130,15 +130,10 @@ struct TimeX : Function<TimeX> {
         const Tensor &w = s[0], &k = s[1], gx = g[0].contiguous();
         const int B = i32(get(ctx, "B")), T = i32(get(ctx, "T")), C = i32(get(ctx, "C"));
         const Guard guard(w.device());
-        Tensor gk = at::empty({B, C, T}, k.options()), gw;
-        if (T % 32 == 0 && T <= T_SUM_MAX) {             // the sum over the batch of run.py:102 happens in the kernel
-            gw = at::empty({C, T}, k.options());
-            ok(rwkv_timex_backward_sum(stream_of(w), P(w), P(k), P(gx), P(gw), P(gk), B, C, T), false);
-        } else {
-            Tensor rows = at::empty({B, C, T}, k.options());
-            ok(rwkv_timex_backward(stream_of(w), P(w), P(k), P(gx), P(rows), P(gk), B, C, T), false);
-            gw = rows.sum(0);
-        }
+        Tensor gk = at::empty({B, C, T}, k.options()), gw = at::empty({C, T}, k.options());      // the sum over the batch of run.py:102 happens in the library
+        const size_t n = rwkv_timex_backward_ws_bytes(B, C, T);
+        const Tensor ws = n > 0 ? bytes(k, n) : Tensor();
+        ok(rwkv_timex_backward_ws(stream_of(w), P(w), P(k), P(gx), P(gw), P(gk), B, C, T, P(ws), n), false);
         return {gw, gk, NONE, NONE, NONE, NONE};
     }
 };

@@ -5,74 +5,14 @@
 //   gk[b,c,u] =       sum_{t>=u} wr[t-u] g[b,c,t]
 //   gw[b,c,T-1-d] =   sum_{u}    g[b,c,u+d] k[b,c,u]         (per batch; the wrapper sums over b)
 //
-// conv / corr kernels: one workgroup per (channel, group of BB batch rows).  The reversed
-// kernel row wr (with four leading zeros, so taps of negative lag read 0 and the diagonal block
-// needs no mask) and the BB input rows sit in LDS; a thread owns 4 consecutive outputs for all
-// BB rows and walks the lags 4 at a time: two 16-byte LDS reads give the 7 taps it needs, one
-// broadcast 16-byte read per row gives the inputs, 16 FMAs per row follow.
-// gw kernel: one workgroup per (b,c) row; a thread owns 4 consecutive lags d.
+// Three families on fp16 matrix instructions at fp32 accuracy (two fp16 terms per operand): timex_conv_h2 / timex_gw_sum_h2
+// for whole tiles of 32 steps and full batches, timex_conv_any / timex_gw_any for every other length and batch size.
+// timex_gw (vector units) makes the per-batch gw of the reference's signature: one workgroup per (b,c) row; a thread owns 4
+// consecutive lags d.
 #include "common.h"
 
 namespace rwkv {
 namespace {
-
-constexpr int BB = 8;
-
-// MIRROR = false: out[t] = eps + sum_{u<=t} wr[t-u] in[u]      (forward)
-// MIRROR = true : out[u] =       sum_{t>=u} wr[t-u] in[t]      (gk)
-template <bool MIRROR>
-__global__ __launch_bounds__(1024) void timex_conv(const float* __restrict__ w, const float* __restrict__ in,
-                                                  float* __restrict__ out, float eps, int B, int C, int T) {
-    extern __shared__ float lds[];
-    float* wr = lds;                 // [T + 4], wr[4 + d] = w[c][T-1-d], wr[0..3] = 0
-    float* rows = lds + T + 4;       // [BB][T]
-    const int c = blockIdx.x, b0 = blockIdx.y * BB, tid = threadIdx.x;
-    const int nthr = T >> 2;
-
-    for (int i = tid; i < 4; i += nthr) wr[i] = 0.f;
-    for (int d = tid; d < T; d += nthr) wr[4 + d] = w[static_cast<size_t>(c) * T + (T - 1 - d)];
-#pragma unroll
-    for (int r = 0; r < BB; ++r) {
-        const int b = b0 + r;
-        float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (b < B) x = *reinterpret_cast<const float4*>(in + (static_cast<size_t>(b) * C + c) * T + 4 * tid);
-        *reinterpret_cast<float4*>(rows + r * T + 4 * tid) = x;
-    }
-    __syncthreads();
-
-    const int o0 = 4 * tid;          // first output index of this thread
-    float acc[BB][4];
-#pragma unroll
-    for (int r = 0; r < BB; ++r)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) acc[r][a] = MIRROR ? 0.f : eps;
-
-    const int lo = MIRROR ? o0 : 0, hi = MIRROR ? T - 4 : o0;
-    for (int s4 = lo; s4 <= hi; s4 += 4) {
-        const int d0 = MIRROR ? s4 - o0 : o0 - s4;                   // >= 0, multiple of 4
-        const float4 wl = *reinterpret_cast<const float4*>(wr + d0);       // lags d0-4 .. d0-1
-        const float4 wh = *reinterpret_cast<const float4*>(wr + d0 + 4);   // lags d0   .. d0+3
-        const float wv[8] = {wl.x, wl.y, wl.z, wl.w, wh.x, wh.y, wh.z, wh.w};
-#pragma unroll
-        for (int r = 0; r < BB; ++r) {
-            const float4 x4 = *reinterpret_cast<const float4*>(rows + r * T + s4);
-            const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    // forward: lag = (o0+a) - (s4+e) = d0 + a - e;  mirror: lag = (s4+e) - (o0+a) = d0 + e - a
-                    acc[r][a] = fmaf(wv[4 + (MIRROR ? e - a : a - e)], xv[e], acc[r][a]);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < BB; ++r) {
-        const int b = b0 + r;
-        if (b < B)
-            *reinterpret_cast<float4*>(out + (static_cast<size_t>(b) * C + c) * T + o0) =
-                make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
-    }
-}
 
 // gw[row][T-1-d] = sum_u g[row][u+d] k[row][u]
 __global__ __launch_bounds__(1024) void timex_gw(const float* __restrict__ k, const float* __restrict__ g,
@@ -139,6 +79,7 @@ constexpr int NCU = 256;               // workgroups of the persistent kernels: 
 // LDS: 2 x 32 x (T + 16) x 2 + 4 x (T + 96) x 2 + 64 bytes = 142 144 of 163 840 at T = 1024, the longest T this form takes.
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 constexpr int T_H2_MAX = 1024;
+constexpr int T_ANY = 4096;            // the longest sequence of the kernels for any shape
 constexpr int T_H2_MID = 768;          // up to here a lane holds 3 pieces (16 bytes each) of each of its four rows while they are in flight, beyond 4
 __host__ __device__ inline int h2_row_stride(int T) { return T + 16; }           // elements; (T + 16) / 2 dwords = 8 or 24 mod 32
 __host__ __device__ inline int h2_line_len(int T) { return T + ((T & 32) ? 64 : 96); }    // half of it = 16 mod 32 dwords: the shifted copy sits 16 banks away
@@ -622,16 +563,381 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
     }
 }
 
+// ------------------------------------------------------------------------------------ any length, any batch size
+// The same products with the columns taken from time as well as from the batch.  With t = 32 a + i the convolution of a row is
+//     out[32 a + i] = sum_{d <= a} sum_j W_d[i][j] in[32 (a - d) + j],     W_d[i][j] = wr[32 d + i - j],
+// so for every block lag d one 32 x 32 Toeplitz matrix meets ALL 32-step blocks of all rows: a column is a pair (block a, row
+// b), numbered a Bg + b in a unit of Bg batch rows of one channel, and 32 consecutive columns are a tile of one matrix
+// instruction.  Two rows of 1500 steps fill three column tiles, where a tile of 32 batch rows would be empty but for two.
+// A tile's columns differ in a by at most 31 / Bg: d runs to the largest a, and blocks before a row's start (mirror: after its
+// end) read as zeros, of which every row has zb behind it.  The kernel gradient is the same contraction turned round:
+//     gw[lag 32 d + i - j] = sum over the diagonals of M_d[i][j] = sum_columns g[32 a + i] k[32 (a - d) + j],
+// K slots are columns, sixteen an instruction, g and k operands by transposing LDS reads whose lanes point at blocks of their
+// own.  Rows lie in LDS as blocks of 32 + 8 fp16 (80 bytes: 16-byte reads of neighbouring columns fall on different banks if a
+// row has an odd number of blocks), 512 threads, at most 80 KB and 128 registers: two workgroups share a CU, one converts
+// its rows while the other multiplies.  Bound by LDS reads (4 KB per column tile and block lag, and 4 KB for the Toeplitz
+// operand that a wave's two tiles share).  B13 C384 T1500: 58 us a convolution, 101 us the kernel gradient; the vector-unit
+// kernels that these replace took 315 / 286 and, with the sum over the batch, 243 us.
+constexpr int BLK = 40;                // fp16 elements of a block in LDS, 32 of them data
+constexpr int LDS_ANY = 80 * 1024;     // two workgroups per CU
+constexpr int PZ = 32;                 // zeros in front of the forward line (lags beyond the last tap, of rows past T)
+constexpr int CONV_PIECES = 8, GW_PIECES = 4;   // 16-byte pieces a thread stages (per tensor): Bg nt 8 / 512 at most
+
+struct AnyGeom {
+    int nt, bg, zb, pitch;             // blocks of a row, rows of a unit, zero blocks behind a row, nt + zb (odd)
+    __host__ __device__ size_t plane() const { return static_cast<size_t>(zb + bg * pitch) * BLK; }     // elements
+};
+inline AnyGeom any_geom(int T, int bg, int span) {        // span: how many blocks the columns of one operand may differ by
+    AnyGeom q;
+    q.nt = (T + 31) / 32; q.bg = bg;
+    q.zb = (span + bg - 1) / bg;
+    q.zb += (q.nt + q.zb + 1) & 1;
+    q.pitch = q.nt + q.zb;
+    return q;
+}
+inline size_t conv_any_lds(const AnyGeom& q) { return (2 * q.plane() + 4 * static_cast<size_t>(h2_line_len(32 * q.nt))) * 2 + 64; }
+inline size_t gw_any_lds(const AnyGeom& q) { return 4 * q.plane() * 2 + static_cast<size_t>(q.nt) * 256 + 64; }
+
+// rows b0 .. of channel c as 16-byte pieces: piece idx = tid + 512 i <-> (row, four steps)
+template <int NP> struct Stager {
+    float4 x[NP];
+    DEVINL void fetch(const float* __restrict__ in, const AnyGeom& q, int c, int b0, int B, int C, int T) {
+        const int per = 8 * q.nt, total = q.bg * per;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            const int idx = static_cast<int>(threadIdx.x) + TXT * i;
+            if (idx < total) {
+                const int b = idx / per, t = 4 * (idx - b * per);
+                if (b0 + b < B && t < T) x[i] = *reinterpret_cast<const float4*>(in + (static_cast<size_t>(b0 + b) * C + c) * T + t);
+            }
+        }
+    }
+    DEVINL float largest() const {
+        float m = 0.f;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) m = max_abs4(m, x[i]);
+        return wave_max(m);
+    }
+    DEVINL void store(uint16_t* rp, const AnyGeom& q, float up) const {
+        const int per = 8 * q.nt, total = q.bg * per;
+        const size_t pl = q.plane();
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const int idx = static_cast<int>(threadIdx.x) + TXT * i;
+            if (idx < total) {
+                const int b = idx / per, r = idx - b * per;
+                uint16_t* d = rp + (q.zb + b * q.pitch + (r >> 3)) * BLK + 4 * (r & 7);
+                const H2x4 y = split2x4(x[i], up);
+                *reinterpret_cast<uint2*>(d) = y.h;
+                *reinterpret_cast<uint2*>(d + pl) = y.l;
+            }
+        }
+    }
+};
+// the blocks in front of the first row and behind every row
+DEVINL void zero_blocks(uint16_t* rp, const AnyGeom& q) {
+    const int n = q.zb * (q.bg + 1) * (BLK / 8);
+    const size_t pl = q.plane();
+    for (int i = threadIdx.x; i < n; i += TXT) {
+        const int blk = i / (BLK / 8), e = i - blk * (BLK / 8), row = blk / q.zb, z = blk - row * q.zb;      // row 0: the front
+        uint16_t* d = rp + (row * q.pitch + z) * BLK + 8 * e;
+        *reinterpret_cast<uint4*>(d) = make_uint4(0, 0, 0, 0);
+        *reinterpret_cast<uint4*>(d + pl) = make_uint4(0, 0, 0, 0);
+    }
+}
+
+template <bool MIRROR>
+__global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict__ w, const float* __restrict__ in, float* __restrict__ out,
+                                                         float eps, int B, int C, int T, int ng, const AnyGeom q) {
+    extern __shared__ __align__(16) float lds[];
+    const int Tp = 32 * q.nt, xl = h2_line_len(Tp), plane = static_cast<int>(q.plane());
+    uint16_t* rp = reinterpret_cast<uint16_t*>(lds);                    // [2][plane]
+    uint16_t* al = rp + 2 * plane;                                      // [2 planes][2 copies][xl]
+    float* red = reinterpret_cast<float*>(al + 4 * xl);                 // [2][8]
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, kh = lane >> 5;
+    const int c = blockIdx.x / ng, b0 = (blockIdx.x - c * ng) * q.bg;
+    float unscale;
+    {
+        Stager<CONV_PIECES> st;
+        st.fetch(in, q, c, b0, B, C, T);
+        float wr[T_ANY / TXT], mw = 0.f;
+#pragma unroll
+        for (int z = 0; z < T_ANY / TXT; ++z) {
+            const int tau = z * TXT + tid;
+            wr[z] = tau < T ? w[static_cast<size_t>(c) * T + tau] : 0.f;
+            mw = fmaxf(mw, fabsf(wr[z]));
+        }
+        for (int i = tid; i < 2 * xl; i += TXT) reinterpret_cast<uint32_t*>(al)[i] = 0;
+        zero_blocks(rp, q);
+        const float mx = st.largest();
+        mw = wave_max(mw);
+        if (lane == 0) { red[wv] = mx; red[8 + wv] = mw; }
+        __syncthreads();
+        float ax = 0.f, aw = 0.f;
+#pragma unroll
+        for (int i = 0; i < TXW; ++i) { ax = fmaxf(ax, red[i]); aw = fmaxf(aw, red[8 + i]); }
+        const Pow2 sx = scale_for(ax), sw = scale_for(aw);
+        unscale = sx.down * sw.down;
+        st.store(rp, q, sx.up);
+        // tap tau (lag T-1-tau) sits at line position PZ + tau (forward) or 31 + lag (mirror); the rest is zero
+#pragma unroll
+        for (int z = 0; z < T_ANY / TXT; ++z) {
+            const int tau = z * TXT + tid;
+            if (tau < T) {
+                const H2 a = split2(wr[z] * sw.up);
+                const int pos = MIRROR ? 31 + (T - 1 - tau) : PZ + tau;
+                const uint16_t pl[2] = {a.h, a.l};
+#pragma unroll
+                for (int p = 0; p < 2; ++p) { al[(2 * p) * xl + pos] = pl[p]; al[(2 * p + 1) * xl + pos - 1] = pl[p]; }
+            }
+        }
+        __syncthreads();
+    }
+    // Column tiles in the order of decreasing work go to the waves back and forth: ranks wv and 15 - wv, at most two a wave, the
+    // shorter one along with the longer one (they share the Toeplitz operand) as far as it goes.
+    const int ncol = q.nt * q.bg, ntile = (ncol + 31) >> 5;
+    int tile[2], nd[2];
+    const uint16_t* bp[2];
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+        const int rank = z == 0 ? wv : 2 * TXW - 1 - wv;
+        tile[z] = MIRROR ? rank : ntile - 1 - rank;
+        nd[z] = rank < ntile ? (MIRROR ? q.nt - 32 * tile[z] / q.bg : min(32 * tile[z] + 31, ncol - 1) / q.bg + 1) : 0;
+        const int col = min(32 * max(tile[z], 0) + ln, ncol - 1), a = col / q.bg, b = col - a * q.bg;
+        bp[z] = rp + (q.zb + b * q.pitch + a) * BLK + 8 * kh;
+    }
+    const int start = (MIRROR ? 31 - ln : PZ + T - 1 - ln) + 8 * kh;    // forward: line[start - 32 d + j], mirror: line[start + 32 d + j]
+    const uint32_t* ap = reinterpret_cast<const uint32_t*>(al + (start & 1) * xl) + (start >> 1);
+    f32x16 acc[2];
+#pragma unroll
+    for (int z = 0; z < 2; ++z)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[z][v] = 0.f;
+    auto run = [&](auto NTL, const int d0, const int d1) __attribute__((always_inline)) {
+        constexpr int NT_ = decltype(NTL)::value;
+        for (int d = d0; d < d1; ++d) {
+            const int o = MIRROR ? d : -d;
+            f16x8 fa[2][2], fb[NT_][2][2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    const uint32_t* a4 = ap + 16 * o + 8 * ks + p * xl;          // a plane is 2 xl elements = xl dwords
+                    fa[ks][p] = __builtin_bit_cast(f16x8, make_uint4(a4[0], a4[1], a4[2], a4[3]));
+                }
+#pragma unroll
+            for (int z = 0; z < NT_; ++z)
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p)
+                        fb[z][ks][p] = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4*>(bp[z] + BLK * o + 16 * ks + p * plane));
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int term = 0; term < 3; ++term)
+#pragma unroll
+                    for (int z = 0; z < NT_; ++z)
+                        acc[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[ks][term == 2], fb[z][ks][term == 1], acc[z], 0, 0, 0);
+        }
+    };
+    run(std::integral_constant<int, 2>{}, 0, nd[1]);
+    run(std::integral_constant<int, 1>{}, nd[1], nd[0]);
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+        const int col = 32 * tile[z] + ln, a = col / q.bg, b = col - a * q.bg;
+        if (nd[z] > 0 && col < ncol && b0 + b < B) {
+            float* o = out + (static_cast<size_t>(b0 + b) * C + c) * T;
+#pragma unroll
+            for (int v4 = 0; v4 < 4; ++v4) {
+                const int t = 32 * a + 8 * v4 + 4 * kh;
+                const float e = MIRROR ? 0.f : eps;
+                if (t < T)
+                    *reinterpret_cast<float4*>(o + t) = make_float4(fmaf(acc[z][4 * v4], unscale, e), fmaf(acc[z][4 * v4 + 1], unscale, e),
+                                                                    fmaf(acc[z][4 * v4 + 2], unscale, e), fmaf(acc[z][4 * v4 + 3], unscale, e));
+            }
+        }
+    }
+}
+
+// the sum of a finished 32 x 32 tile of lag tile d over its diagonals, into diag[64 d ..] (entry l: lag 32 d + l - 31)
+DEVINL void add_diagonals(float* diag, const f32x16& acc, int d, float unscale, int ln, int kh) {
+    float pos = 0.f, neg = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int t = 8 * (v >> 2) + 4 * kh + (v & 3);
+        const float y = __shfl(acc[v], (kh << 5) | ((t - ln) & 31), 64);
+        if (t >= ln) pos += y; else neg += y;
+    }
+    pos += __shfl_xor(pos, 32, 64);
+    neg += __shfl_xor(neg, 32, 64);
+    if (kh == 0) diag[64 * d + 31 + ln] += pos * unscale;
+    else if (ln >= 1) diag[64 * d + ln - 1] += neg * unscale;
+}
+
+// one workgroup: channel c = blockIdx.x, batch groups blockIdx.y, blockIdx.y + gridDim.y, ...; out[blockIdx.y][c][T]
+__global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__ k, const float* __restrict__ g, float* __restrict__ out,
+                                                       int B, int C, int T, int ng, const AnyGeom q) {
+    extern __shared__ __align__(16) float lds[];
+    const int plane = static_cast<int>(q.plane());
+    uint16_t* gp = reinterpret_cast<uint16_t*>(lds);            // [2][plane]
+    uint16_t* kp = gp + 2 * plane;                              // [2][plane]
+    float* diag = reinterpret_cast<float*>(kp + 2 * plane);     // [nt][64]
+    float* red = diag + 64 * q.nt;                              // [2][8]
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ln = lane & 31, kh = lane >> 5, l16 = lane & 15;
+    const int c = blockIdx.x, ncol = q.nt * q.bg, nsteps = (ncol + 15) >> 4;
+    for (int i = tid; i < 64 * q.nt; i += TXT) diag[i] = 0.f;
+    zero_blocks(gp, q);
+    zero_blocks(kp, q);
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)gp));
+    const uint32_t k_off = 4u * static_cast<uint32_t>(plane), pl_b = 2u * static_cast<uint32_t>(plane);
+    const int db = 16 % q.bg, step_b = 2 * BLK * (db * q.pitch + 16 / q.bg), wrap_b = 2 * BLK * (1 - q.bg * q.pitch);
+    for (int grp = blockIdx.y; grp < ng; grp += gridDim.y) {
+        const int b0 = grp * q.bg;
+        float unscale;
+        {
+            Stager<GW_PIECES> sg, sk;
+            sg.fetch(g, q, c, b0, B, C, T);
+            sk.fetch(k, q, c, b0, B, C, T);
+            const float mg = sg.largest(), mk = sk.largest();
+            if (lane == 0) { red[wv] = mg; red[8 + wv] = mk; }
+            __syncthreads();               // (everybody is also done with the group before)
+            float ag = 0.f, ak = 0.f;
+#pragma unroll
+            for (int i = 0; i < TXW; ++i) { ag = fmaxf(ag, red[i]); ak = fmaxf(ak, red[8 + i]); }
+            const Pow2 ug = scale_for(ag), uk = scale_for(ak);
+            unscale = ug.down * uk.down;
+            sg.store(gp, q, ug.up);
+            sk.store(kp, q, uk.up);
+            __syncthreads();
+        }
+        // lag tile d takes the columns from d Bg on; tiles in the order of decreasing work go to the waves back and forth, four at
+        // a time (their g operand is the same)
+        for (int set = 0; 32 * set < q.nt; ++set) {
+            const int dd[4] = {32 * set + wv, 32 * set + 15 - wv, 32 * set + 16 + wv, 32 * set + 31 - wv};
+            if (dd[0] >= q.nt) break;
+            f32x16 acc[4];
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[z][v] = 0.f;
+            int s = (dd[0] * q.bg) >> 4;
+            // this lane's columns in the two transposing reads of a step: K slots 8 kh + (l16 >> 2) and four on
+            int bb[2];
+            uint32_t at[2];
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const int col = 16 * s + 8 * kh + (l16 >> 2) + 4 * z, a = col / q.bg;
+                bb[z] = col - a * q.bg;
+                at[z] = lds0 + 2u * static_cast<uint32_t>((q.zb + bb[z] * q.pitch + a) * BLK + 16 * (ln >> 4) + 4 * (l16 & 3));
+            }
+            auto operand = [&](const uint32_t o) __attribute__((always_inline)) {
+                const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_ptr)(at[0] + o));
+                const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_ptr)(at[1] + o));
+                const uint2 x = __builtin_bit_cast(uint2, lo), y = __builtin_bit_cast(uint2, hi);
+                return __builtin_bit_cast(f16x8, make_uint4(x.x, x.y, y.x, y.y));
+            };
+            auto run = [&](auto NTL, const int end) __attribute__((always_inline)) {
+                constexpr int NT_ = decltype(NTL)::value;
+                for (; s < end; ++s) {
+                    f16x8 fg[2];
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) fg[p] = operand(p * pl_b);
+#pragma unroll
+                    for (int z0 = 0; z0 < NT_; z0 += 2) {             // (two at a time: the four tiles' operands together would not fit 128 registers)
+                        f16x8 fk[2][2];
+#pragma unroll
+                        for (int z = z0; z < NT_ && z < z0 + 2; ++z)
+#pragma unroll
+                            for (int p = 0; p < 2; ++p) fk[z - z0][p] = operand(k_off + p * pl_b - 2u * BLK * static_cast<uint32_t>(dd[z]));
+#pragma unroll
+                        for (int term = 0; term < 3; ++term)
+#pragma unroll
+                            for (int z = z0; z < NT_ && z < z0 + 2; ++z)
+                                acc[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fg[term == 2], fk[z - z0][term == 1], acc[z], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int z = 0; z < 2; ++z) {
+                        at[z] += step_b; bb[z] += db;
+                        if (bb[z] >= q.bg) { bb[z] -= q.bg; at[z] += wrap_b; }
+                    }
+                }
+            };
+            auto from = [&](const int z) { return dd[z] < q.nt ? (dd[z] * q.bg) >> 4 : nsteps; };
+            run(std::integral_constant<int, 1>{}, from(1));
+            run(std::integral_constant<int, 2>{}, from(2));
+            run(std::integral_constant<int, 3>{}, from(3));
+            run(std::integral_constant<int, 4>{}, nsteps);
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+                if (dd[z] < q.nt) add_diagonals(diag, acc[z], dd[z], unscale, ln, kh);     // a lag tile belongs to one wave
+        }
+    }
+    __syncthreads();
+    float* o = out + (static_cast<size_t>(blockIdx.y) * C + c) * T;
+    for (int x = tid; x < T; x += TXT) {        // lag = 32 d + e comes from tile d (diagonal e) and tile d + 1 (diagonal e - 32)
+        const int lag = T - 1 - x, d = lag >> 5, e = lag & 31;
+        o[x] = diag[64 * d + 31 + e] + (d + 1 < q.nt ? diag[64 * (d + 1) + e - 1] : 0.f);
+    }
+}
+// out[x] = sum of n parts that lie `size` floats apart, four elements a thread
+__global__ __launch_bounds__(256) void timex_add_parts(const float4* __restrict__ part, float4* __restrict__ out, size_t size4, int n) {
+    const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= size4) return;
+    float4 a = part[i];
+    for (int z = 1; z < n; ++z) {
+        const float4 x = part[i + z * size4];
+        a.x += x.x; a.y += x.y; a.z += x.z; a.w += x.w;
+    }
+    out[i] = a;
+}
+
+// Batch rows of a unit.  Convolution: what finishes first by a count of matrix clocks (48 per column tile and block lag on a
+// CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (two a wave) and 80 KB.
+AnyGeom conv_any_geom(int B, int C, int T) {
+    AnyGeom best{};
+    double cost = 1e300;
+    for (int bg = 1; bg <= B && bg <= 32; ++bg) {
+        const AnyGeom q = any_geom(T, bg, 31);
+        const int ncol = q.nt * bg, ntile = (ncol + 31) / 32;
+        if (ntile > 2 * TXW || conv_any_lds(q) > LDS_ANY || 8 * ncol > CONV_PIECES * TXT) { if (bg > 1) break; }
+        long long pairs = 0;
+        for (int t = 0; t < ntile; ++t) pairs += (32 * t + 31 < ncol ? 32 * t + 31 : ncol - 1) / bg + 1;
+        const long long units = static_cast<long long>(C) * ((B + bg - 1) / bg);
+        const double x = static_cast<double>((units + 2 * NCU - 1) / (2 * NCU)) * (48.0 * pairs + 0.1 * bg * T + 3000.0);
+        if (x < cost) { cost = x; best = q; }
+    }
+    return best;
+}
+AnyGeom gw_any_geom(int B, int T) {
+    AnyGeom best = any_geom(T, 1, 15);
+    for (int bg = 2; bg <= B && bg <= 32; ++bg) {
+        const AnyGeom q = any_geom(T, bg, 15);
+        if (gw_any_lds(q) > LDS_ANY || 8 * q.nt * bg > GW_PIECES * TXT) break;
+        best = q;
+    }
+    return best;
+}
+// batch groups that work side by side (their sums are added by a second kernel): as many as it takes for two workgroups per CU
+int gw_any_parts(int B, int C, const AnyGeom& q) {
+    const int ng = (B + q.bg - 1) / q.bg, want = (2 * NCU + C - 1) / C;
+    return ng < want ? ng : want;
+}
+
 constexpr int T_MAX = 4096;
 
 int check_tx(int B, int C, int T) {
     if (B <= 0 || C <= 0 || T <= 0) return RWKV_ERR_SHAPE;
     if (T % 4 != 0 || T > T_MAX) return RWKV_ERR_SHAPE;
-    if ((B + BB - 1) / BB > 65535) return RWKV_ERR_SHAPE;
+    if (B > 8 * 65535) return RWKV_ERR_SHAPE;
     return RWKV_OK;
 }
 
-// The matrix-core path pays off once the 32 columns of a product are mostly real batch rows.
+// Whole tiles of steps and enough batch rows for the 32 columns of a product: the kernels whose operands are shared best.  B32
+// C768 T768 forward: 58 us here, 64 with the kernel for any shape.
 bool use_mfma(int B, int T) { return T % 32 == 0 && T <= T_MFMA_MAX && B >= 8; }
 int conv_grid(int B, int C) {
     const long long units = static_cast<long long>(C) * ((B + MROWS - 1) / MROWS);
@@ -651,18 +957,21 @@ template <typename K> int raise_lds_limit(K kernel, size_t bytes) {
 
 using namespace rwkv;
 
-// gk = the mirrored convolution of gwk with w.
-int launch_gk(void* stream, const float* w, const float* gwk, float* gk, int B, int C, int T) {
+// the convolution (forward) or its mirror (gk = the mirrored convolution of gwk with w)
+template <bool MIRROR> int launch_conv(void* stream, const float* w, const float* in, float* out, float eps, int B, int C, int T) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
     if (use_mfma(B, T)) {
         const size_t lds = h2_lds_bytes(T);
-        auto kernel = T <= T_H2_MID ? timex_conv_h2<true, T_H2_MID / 256> : timex_conv_h2<true, T_H2_MAX / 256>;
+        auto kernel = T <= T_H2_MID ? timex_conv_h2<MIRROR, T_H2_MID / 256> : timex_conv_h2<MIRROR, T_H2_MAX / 256>;
         if (int e = raise_lds_limit(kernel, lds)) return e;
-        hipLaunchKernelGGL(kernel, dim3(conv_grid(B, C)), dim3(TXT), lds, static_cast<hipStream_t>(stream), w, gwk, gk, 0.0f, B, C, T);
+        hipLaunchKernelGGL(kernel, dim3(conv_grid(B, C)), dim3(TXT), lds, st, w, in, out, eps, B, C, T);
     } else {
-        const size_t lds = (static_cast<size_t>(BB + 1) * T + 4) * sizeof(float);
-        if (int e = raise_lds_limit(timex_conv<true>, lds)) return e;
-        hipLaunchKernelGGL(timex_conv<true>, dim3(C, (B + BB - 1) / BB), dim3(T / 4), lds,
-                           static_cast<hipStream_t>(stream), w, gwk, gk, 0.0f, B, C, T);
+        const AnyGeom q = conv_any_geom(B, C, T);
+        const size_t lds = conv_any_lds(q);
+        const int ng = (B + q.bg - 1) / q.bg;
+        if (static_cast<long long>(C) * ng > 0x7fffffffLL) return RWKV_ERR_SHAPE;
+        if (int e = raise_lds_limit(timex_conv_any<MIRROR>, lds)) return e;
+        hipLaunchKernelGGL(timex_conv_any<MIRROR>, dim3(C * ng), dim3(TXT), lds, st, w, in, out, eps, B, C, T, ng, q);
     }
     return RWKV_OK;
 }
@@ -672,17 +981,7 @@ extern "C" {
 int rwkv_timex_forward(void* stream, const float* w, const float* k, float* x, float eps, int B, int C, int T) {
     if (int e = check_tx(B, C, T)) return e;
     if (int e = check_ptrs({w, k, x})) return e;
-    if (use_mfma(B, T)) {
-        const size_t lds = h2_lds_bytes(T);
-        auto kernel = T <= T_H2_MID ? timex_conv_h2<false, T_H2_MID / 256> : timex_conv_h2<false, T_H2_MAX / 256>;
-        if (int e = raise_lds_limit(kernel, lds)) return e;
-        hipLaunchKernelGGL(kernel, dim3(conv_grid(B, C)), dim3(TXT), lds, static_cast<hipStream_t>(stream), w, k, x, eps, B, C, T);
-        return launch_status();
-    }
-    const size_t lds = (static_cast<size_t>(BB + 1) * T + 4) * sizeof(float);
-    if (int e = raise_lds_limit(timex_conv<false>, lds)) return e;
-    hipLaunchKernelGGL(timex_conv<false>, dim3(C, (B + BB - 1) / BB), dim3(T / 4), lds,
-                       static_cast<hipStream_t>(stream), w, k, x, eps, B, C, T);
+    if (int e = launch_conv<false>(stream, w, k, x, eps, B, C, T)) return e;
     return launch_status();
 }
 
@@ -691,7 +990,7 @@ int rwkv_timex_backward(void* stream, const float* w, const float* k, const floa
     if (int e = check_tx(B, C, T)) return e;
     if (int e = check_ptrs({w, k, gwk, gw, gk})) return e;
     if (static_cast<long long>(B) * C > 0x7fffffffLL) return RWKV_ERR_SHAPE;
-    if (int e = launch_gk(stream, w, gwk, gk, B, C, T)) return e;
+    if (int e = launch_conv<true>(stream, w, gwk, gk, 0.0f, B, C, T)) return e;
     hipLaunchKernelGGL(timex_gw, dim3(B * C), dim3(T / 4), (2 * static_cast<size_t>(T) + 4) * sizeof(float),
                        static_cast<hipStream_t>(stream), k, gwk, gw, T);
     return launch_status();
@@ -702,12 +1001,39 @@ int rwkv_timex_backward_sum(void* stream, const float* w, const float* k, const 
     if (int e = check_tx(B, C, T)) return e;
     if (T % 32 != 0 || T > T_MFMA_MAX) return RWKV_ERR_SHAPE;
     if (int e = check_ptrs({w, k, gwk, gw_sum, gk})) return e;
-    if (int e = launch_gk(stream, w, gwk, gk, B, C, T)) return e;
+    if (int e = launch_conv<true>(stream, w, gwk, gk, 0.0f, B, C, T)) return e;
     // (any batch size: a pass takes 16 rows, rows past the batch count as zero)
     const size_t lds_gw = gw_h2_lds_bytes(T);
     auto kernel = T <= T_H2_MID ? timex_gw_sum_h2<T_H2_MID / 256> : timex_gw_sum_h2<T_H2_MAX / 256>;
     if (int e = raise_lds_limit(kernel, lds_gw)) return e;
     hipLaunchKernelGGL(kernel, dim3(C < NCU ? C : NCU), dim3(TXT), lds_gw, static_cast<hipStream_t>(stream), k, gwk, gw_sum, B, C, T);
+    return launch_status();
+}
+
+size_t rwkv_timex_backward_ws_bytes(int B, int C, int T) {
+    if (check_tx(B, C, T) != RWKV_OK || (T % 32 == 0 && T <= T_MFMA_MAX)) return 0;
+    const int parts = gw_any_parts(B, C, gw_any_geom(B, T));
+    return parts <= 1 ? 0 : static_cast<size_t>(parts) * C * T * sizeof(float);
+}
+
+int rwkv_timex_backward_ws(void* stream, const float* w, const float* k, const float* gwk, float* gw_sum, float* gk, int B, int C, int T,
+                           void* workspace, size_t workspace_bytes) {
+    if (int e = check_tx(B, C, T)) return e;
+    if (T % 32 == 0 && T <= T_MFMA_MAX) return rwkv_timex_backward_sum(stream, w, k, gwk, gw_sum, gk, B, C, T);
+    if (int e = check_ptrs({w, k, gwk, gw_sum, gk})) return e;
+    const AnyGeom q = gw_any_geom(B, T);
+    const int ng = (B + q.bg - 1) / q.bg, parts = gw_any_parts(B, C, q);
+    if (parts > 1 && (workspace == nullptr || workspace_bytes < rwkv_timex_backward_ws_bytes(B, C, T) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+    if (int e = launch_conv<true>(stream, w, gwk, gk, 0.0f, B, C, T)) return e;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const size_t lds = gw_any_lds(q);
+    if (int e = raise_lds_limit(timex_gw_any, lds)) return e;
+    hipLaunchKernelGGL(timex_gw_any, dim3(C, parts), dim3(TXT), lds, st, k, gwk, parts > 1 ? static_cast<float*>(workspace) : gw_sum, B, C, T, ng, q);
+    if (parts > 1) {
+        const size_t n4 = static_cast<size_t>(C) * T / 4;
+        hipLaunchKernelGGL(timex_add_parts, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, st,
+                           static_cast<const float4*>(workspace), reinterpret_cast<float4*>(gw_sum), n4, parts);
+    }
     return launch_status();
 }
 
