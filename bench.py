@@ -172,7 +172,7 @@ def make_wkv6(dev, state, B=8):
 
 def make_wkv5(dev, H=32, N=64):
     """N = 64: the matrix-core kernels at B8 T4096 C2048; N = 128: wkv5_bf16/run.py:17-22 as shipped (B8 T4096 C4096),
-    which runs on the same kernels with every head taken as four heads of 64 (two launches per kernel, fp32 terms added)."""
+    a workgroup per whole head (with --algo sweeps or no states kept: four heads of 64, two launches per kernel, fp32 terms added)."""
     from rwkv_cuda_amd import _lib, synth
     from rwkv_cuda_amd._call import call
     lib = _lib.load()
@@ -192,7 +192,7 @@ def make_wkv5(dev, H=32, N=64):
     ew = (-torch.exp(w.float())).contiguous()
     eew = torch.exp(ew).contiguous()
 
-    one_sweep = N == 64 and ALGO == "chunked"
+    one_sweep = ALGO == "chunked"
     if one_sweep:
         nsaved = lib.rwkv_wkv5s_saved_bytes(B, T, C, H)
         saved = torch.empty(nsaved, device=dev, dtype=torch.uint8)
@@ -217,8 +217,9 @@ def make_wkv5(dev, H=32, N=64):
         return run
 
     if one_sweep:
-        kernels = [("wkv6_fwd_fused<head decay> (keeps states)", fwd1, 8 * C * tok),       # r k v -> y
-                   ("wkv6_bwd_fused<head decay> (+ batch sums)", bwd1, 14 * C * tok)]      # r k v gy -> gr gk gv
+        names = ("wkv6_fwd_fused<head decay>", "wkv6_bwd_fused<head decay>") if N == 64 else ("wkv5b_fwd", "wkv5b_bwd")
+        kernels = [(names[0] + " (keeps states)", fwd1, 8 * C * tok),       # r k v -> y
+                   (names[1] + " (+ batch sums)", bwd1, 14 * C * tok)]      # r k v gy -> gr gk gv
     elif N == 64:
         kernels = [("wkv6_fwd_ws<head decay>", lambda: call("rwkv_wkv5_forward_ex", dev, B, T, C, H, r, k, v, eew, u, y, FLAGS), 8 * C * tok),
                    ("wkv6_bwd_a_ws<head decay>", bwd(1), 10 * C * tok),           # r k v gy -> gr (+ fp32 workspace)

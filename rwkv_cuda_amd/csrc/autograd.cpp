@@ -249,7 +249,7 @@ Tensor wkv5a_op(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
 // --------------------------------------------------------------------------------------------- wkv5, bf16 (wkv5_bf16/run.py:44-88)
 struct Wkv5Bf16 : Function<Wkv5Bf16> {
     static Tensor forward(AutogradContext* ctx, int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& r, const Tensor& k, const Tensor& v,
-                          const Tensor& w, const Tensor& u, int64_t flags) {
+                          const Tensor& w, const Tensor& u, int64_t flags, bool grad) {
         check({{&r, "r"}, {&k, "k"}, {&v, "v"}, {&w, "w"}, {&u, "u"}}, BF, r);
         check_head(C, H);
         require(r.numel() == B * T * C && k.numel() == r.numel() && v.numel() == r.numel() && w.numel() == C && u.numel() == C, "shape mismatch");
@@ -257,14 +257,17 @@ struct Wkv5Bf16 : Function<Wkv5Bf16> {
         const Dims d = dims(B, T, C, H);
         // ew = -exp(w.float()), eew = exp(ew) (:63-64) are made by the library into `decay` = [eew | ew]
         Tensor decay = at::empty({2 * C}, r.options().dtype(F32)), y = at::empty({B, T, C}, r.options());
-        const size_t n = C == H * HEAD ? rwkv_wkv5s_saved_bytes(d.B, d.T, d.C, d.H) : 0;
+        const bool whole = C == H * MAX_HEAD && flags == 0;
+        const size_t n = C == H * HEAD || whole ? rwkv_wkv5s_saved_bytes(d.B, d.T, d.C, d.H) : 0;
         if (n > 0) {
-            // head size 64: one forward and one reverse sweep; the forward keeps the state entering every 64th token
-            Tensor saved = bytes(r, n);
-            ok(rwkv_wkv5s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(saved), n, flags), true);
-            ctx->save_for_backward({r, k, v, decay, u, w, saved});
+            // head sizes 64 and 128: one forward and one reverse sweep; the forward keeps the state entering every 64th token
+            // (at 128 only if a backward can follow)
+            const bool keep = grad || !whole;
+            const Tensor saved = keep ? bytes(r, n) : Tensor();
+            ok(rwkv_wkv5s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(saved), keep ? n : 0, flags), true);
+            if (keep) ctx->save_for_backward({r, k, v, decay, u, w, saved});
         } else {
-            // heads of 128 channels run as four heads of 64 whose fp32 terms need scratch; every other size needs none
+            // heads of 128 channels with options run as four heads of 64 whose fp32 terms need scratch; every other size needs none
             const size_t nf = rwkv_wkv5_forward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, nf < 16 ? 16 : nf);
             ok(rwkv_wkv5raw_forward_ws(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(ws), nf, flags), true);
@@ -284,7 +287,8 @@ struct Wkv5Bf16 : Function<Wkv5Bf16> {
         Tensor gw = at::empty({d.H, d.C / d.H}, o), gu = at::empty({d.H, d.C / d.H}, o);       // summed over the batch by the library (:86-87)
         if (s.size() > 5) {
             const Tensor &w = s[5], &saved = s[6];
-            const size_t n = rwkv_wkv5s_backward_workspace_bytes(d.B, d.T, d.C, d.H);
+            // (at head size 128 without options the per-batch rows of gw and gu are all)
+            const size_t n = d.C == d.H * MAX_HEAD ? 4 * static_cast<size_t>(d.B) * d.C : rwkv_wkv5s_backward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, n);
             ok(rwkv_wkv5s_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(decay), P(u), P(gy), P(gr), P(gk), P(gv), P(gw), P(gu),
                                    P(saved), saved.numel(), P(ws), n, flags), false);
@@ -294,11 +298,11 @@ struct Wkv5Bf16 : Function<Wkv5Bf16> {
             ok(rwkv_wkv5raw_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(decay), P(u), P(gy), P(gr), P(gk), P(gv), P(gw), P(gu),
                                      P(ws), n, flags), false);
         }
-        return {NONE, NONE, NONE, NONE, gr, gk, gv, gw, gu, NONE};
+        return {NONE, NONE, NONE, NONE, gr, gk, gv, gw, gu, NONE, NONE};
     }
 };
 Tensor wkv5_bf16_op(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& w, const Tensor& u, int64_t flags) {
-    return Wkv5Bf16::apply(B, T, C, H, r, k, v, w, u, flags);
+    return Wkv5Bf16::apply(B, T, C, H, r, k, v, w, u, flags, wants_grad({&r, &k, &v, &w, &u}));
 }
 
 // ------------------------------------------------------- wkv6 and wkv6_state, bf16 (wkv6/run.py:128-170, wkv6_state/run.py:80-124)

@@ -176,6 +176,15 @@ int launch_wkv5_bwd_a_split(hipStream_t st, int cross, int B, int T, int C, int 
 int launch_wkv5_bwd_b_split(hipStream_t st, int cross, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k,
                             const uint16_t* v, const float* ew, const uint16_t* u, const uint16_t* gy, float* gk32, float* gv32,
                             float* gw32, const float* rdr);
+// wkv5_bf.hip: wkv5, bf16, heads of 128 channels, whole heads, decays of any strength; w raw.  saved (may be null in the forward):
+// the states for the backward; gw, gu: per-batch rows [B][C].
+constexpr int WKV5B_MAX_C = 1 << 24;           // byte offsets within 32 rows are 32-bit
+size_t wkv5b_saved_bytes(int B, int T, int C, int H);
+int launch_wkv5b_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
+                     const uint16_t* u, uint16_t* y, float* decay, float* saved);
+int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
+                     const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu,
+                     const float* saved);
 
 // rwkv7_chunk.hip: chunked rwkv7 kernels (r..b, y, dy, dr..db are bf16 or, with f32, float); s0, sT, dsT, ds0 may be null
 int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0, const void* r, const void* w, const void* k,

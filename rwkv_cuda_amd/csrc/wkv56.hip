@@ -1355,7 +1355,16 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H, const rw
 
 // ---- wkv5 (head size 64) on the one-sweep pair: the raw decay of a channel stands in for every token's, its gradient is
 //      summed over the tokens inside the kernel.  `decay` = [eew | ew] is made for the kernels that redo flagged heads.
-size_t rwkv_wkv5s_saved_bytes(int B, int T, int C, int H) { return rwkv_wkv6f_saved_bytes(B, T, C, H); }
+// heads of 128 channels: one workgroup holds a whole head (wkv5_bf.hip)
+namespace {
+bool whole_head_ok(int C, int H, unsigned flags) { return C == H * N_SPLIT && !(flags & (RWKV_FLAG_SWEEPS | RWKV_PASS_ALL)) && C <= WKV5B_MAX_C; }
+size_t whole_head_ws_bytes(int B, int C) { return 2 * round16(static_cast<size_t>(B) * C * sizeof(uint16_t)); }
+}  // namespace
+
+size_t rwkv_wkv5s_saved_bytes(int B, int T, int C, int H) {
+    if (check_dims(B, T, C, H) == RWKV_OK && whole_head_ok(C, H, 0u)) return wkv5b_saved_bytes(B, T, C, H);
+    return rwkv_wkv6f_saved_bytes(B, T, C, H);
+}
 
 int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16* r, const rwkv_bf16* k, const rwkv_bf16* v,
                        const rwkv_bf16* w_raw, const rwkv_bf16* u, rwkv_bf16* y, float* decay, void* saved, size_t saved_bytes,
@@ -1363,6 +1372,14 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
     if (int e = check_dims(B, T, C, H)) return e;
     if (int e = check_ptrs({r, k, v, w_raw, u, y, decay}, C == H * N)) return e;
     const hipStream_t st = static_cast<hipStream_t>(stream);
+    if (whole_head_ok(C, H, flags)) {
+        const int e = check_ptrs({r, k, v, w_raw, u, y, decay});
+        if (e == RWKV_OK) {
+            if (saved != nullptr && (saved_bytes < wkv5b_saved_bytes(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
+            return launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved));
+        }
+        if (saved != nullptr) return e;
+    }
     if (!fused_ok(T, C, H, flags) || saved == nullptr) {
         hipLaunchKernelGGL(wkv5_decay_transform, dim3((C + 255) / 256), dim3(256), 0, st, C, w_raw, decay);
         return rwkv_wkv5_forward_ex(stream, B, T, C, H, r, k, v, decay, u, y, flags);
@@ -1400,6 +1417,16 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
                         rwkv_bf16* gk, rwkv_bf16* gv, rwkv_bf16* gw, rwkv_bf16* gu, const void* saved, size_t saved_bytes,
                         void* workspace, size_t workspace_bytes, unsigned flags) {
     if (int e = check_dims(B, T, C, H)) return e;
+    if (whole_head_ok(C, H, flags) && saved != nullptr) {
+        if (int e = check_ptrs({r, k, v, w_raw, decay, u, gy, gr, gk, gv, gw, gu})) return e;
+        if (saved_bytes < wkv5b_saved_bytes(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
+        if (workspace == nullptr || workspace_bytes < whole_head_ws_bytes(B, C) || !aligned16(workspace)) return RWKV_ERR_WORKSPACE;
+        uint16_t* pw = static_cast<uint16_t*>(workspace);                                 // per-batch gw, then per-batch gu
+        uint16_t* pu = pw + whole_head_ws_bytes(B, C) / 4;
+        if (int e = launch_wkv5b_bwd(static_cast<hipStream_t>(stream), B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved))) return e;
+        hipLaunchKernelGGL(bf16_batch_sum, dim3((C + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), B, C, pw, gw, pu, gu);
+        return launch_status();
+    }
     if (workspace == nullptr || workspace_bytes < rwkv_wkv5s_backward_workspace_bytes(B, T, C, H) || !aligned16(workspace))
         return RWKV_ERR_WORKSPACE;
     if (!fused_ok(T, C, H, flags) || saved == nullptr)

@@ -1,0 +1,900 @@
+// wkv5, bf16 I/O, whole heads of N = 128 channels in one workgroup: one forward and one reverse sweep in chunks of
+// L = 32 tokens on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16), for decays of any strength.
+//
+// Step form (wkv5_bf16/cuda/wkv5_cuda.cu), one head, S[i][j] (i value channel, j key channel), o = e^l, l = -exp(w_raw):
+//     y_t[i] = sum_j r_t[j] (S_t[i][j] + u[j] k_t[j] v_t[i])       S_{t+1} = S_t o + v_t k_t^T
+// The decay is constant in time, so the powers a token of a chunk (local t = 0..31) needs are the same in every chunk and are
+// made once per workgroup.  S0 is the state entering the chunk, D the gradient of the state leaving it, m a reference token:
+//     A[t][s] = sum_j (r_t o^{t-m}) (k_s o^{m-1-s})  (s < t), A[t][t] = sum_j r_t u k_t        B[t][s] = gy_t . v_s  (s < t)
+//     y_t  = (r_t o^t) S0^T + sum_s A[t][s] v_s
+//     gr_t = o^t (gy_t S0) + o^{t-m} sum_s B[t][s] (k_s o^{m-1-s}) + u k_t (v_t . gy_t)
+//     gk_t = o^{31-t} (v_t D) + o^{m-1-t} sum_s B[s][t] (r_s o^{s-m}) + u r_t (v_t . gy_t)
+//     gv_t = (k_t o^{31-t}) D^T + sum_s A[s][t] gy_s
+//     S_L = S0 o^32 + sum_s v_s (k_s o^{31-s})^T           D_0 = D o^32 + sum_t gy_t (r_t o^t)^T
+// A term (source s, sink t) of the output carries o^(tokens strictly between), so d/dl counts those tokens: t for sources before
+// the chunk, 31 - s for sinks after it, 32 where both lie outside, t - 1 - s inside (the tile B with this weight; taken apart into
+// (t - 16) - (s - 15) the sums would cancel, and two hi / lo products differ by 1e-5 where the true gradient is zero).
+// Operands: fp32 values as hi + lo bf16 (16 mantissa bits), three products where both sides are fp32; r, k, v, gy are exact.
+//
+// Strong decays.  A factor reaches e^{|l| d}, d the distance of a token from its reference.  The forward has one reference in the
+// middle (its planes serve the state products too), up to |l| = 4.5.  The backward refers to the middle of the half that the
+// output's token lies in (m = 8, 24; a tile's quadrant across the halves to 16): d is 8 and |l| may reach 9, for one more
+// operand per tile.  Heads beyond that take a reference per 8 tokens (m = 4, 12, 20, 28); a pair of tokens d such blocks apart
+// then carries o^{8 d} in addition: a product per distance, half of the factor on either side (o^{8 d} may underflow where the
+// whole term is one).  Below l = -17 a decay is taken as e^{-17} = 4e-8.
+// Handing such heads to step-by-step kernels, as the kernels before did, made one strong channel in 4096 cost more than
+// everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 ms with.
+//
+// What bounds it (B8 T4096 C4096: one workgroup per CU).  Forward 0.52 ms for 2.1 GB, half of them the saved states: HBM (4.1 TB/s;
+// 0.82 ms as four heads of 64).  Backward 1.03 ms: the D waves, some 1600 vector and 170 matrix instructions a chunk, and their
+// waits for the saved state (2.95 ms as two sweeps over four heads of 64, whose fp32 terms went through memory).  Both together
+// 6.56 -> 1.49 ms where a channel's decay was strong, 3.87 -> 1.48 where none was.
+#include <stddef.h>
+
+#include "wkv6_fused.h"
+
+namespace rwkv {
+namespace {
+
+constexpr int NTH = 512;             // waves 0..3 hold states, 4..7 load and prepare
+constexpr float LAM_STRONG_F = -4.5f, LAM_STRONG_B = -9.f, LAM_MIN = -17.f;
+constexpr f32x4 ZERO4 = {0.f, 0.f, 0.f, 0.f};
+
+struct ArgsW {
+    int T, C, H;
+    const uint16_t *r, *k, *v, *w, *u, *gy;      // w raw
+    uint16_t *y, *gr, *gk, *gv, *gw, *gu;        // gw, gu: per-batch rows [B][C]
+    float* decay;                                // [e^l | l], 2 C floats (forward)
+    float* saved;                                // [B*H][ceil(chunks / 2)][j][i]: the state entering every even chunk
+};
+
+extern __shared__ __align__(16) unsigned char smem_raw[];
+
+// Sizes of one head.  A wave owns CT tiles of 16 channels; a row of 2 N bytes is loaded in PIECES of 16 bytes.
+template <int HN> struct G {
+    static constexpr int CT = HN / 64, KS = HN / 32, NB16 = HN / 16, PARTS = HN / 32;
+    static constexpr int PIECES = HN / 8, ROWS = 256 / PIECES, PASSES = L / ROWS;
+    static constexpr uint32_t ROW = 2 * HN + 16, PLANE = L * ROW;
+    static constexpr uint32_t LAM = 0, U = 4 * HN, BASE = 8 * HN;
+    static constexpr uint32_t PART = 3 * 1024;                                   // the three quadrants of a tile, fp32, as the lanes hold them
+    // forward: three slots of planes R' hi, lo, K' hi, lo, V and sum r u k; two sets of tile parts
+    static constexpr uint32_t FRH = 0, FRL = PLANE, FKH = 2 * PLANE, FKL = 3 * PLANE, FV = 4 * PLANE, FRUK = 5 * PLANE, FSLOT = FRUK + 4 * L;
+    static constexpr uint32_t FPART = BASE + 3 * FSLOT, FTOTAL = FPART + 2 * PARTS * PART;
+    // backward: two slots of planes r, k, v, gy and two scalars a token; the gradient state hi, lo [j][i]; one set of tile parts
+    static constexpr uint32_t R = 0, K = PLANE, V = 2 * PLANE, GY = 3 * PLANE, VG = 4 * PLANE, RUK = VG + 4 * L, SLOT = RUK + 4 * L;
+    static constexpr uint32_t DSH = BASE + 2 * SLOT, DSL = DSH + HN * ROW, BPART = DSL + HN * ROW, BTOTAL = BPART + PARTS * PART;
+};
+static_assert(G<128>::FTOTAL <= 160 * 1024 && G<128>::BTOTAL <= 160 * 1024, "LDS of one CU");
+
+DEVINL float lds_f(uint32_t o) { return lds_ld<float>(o); }
+
+// e^{lam n} for a small integer n, exact to fp32 rounding: the product and the base-2 exponent carry their rounding errors along
+DEVINL float wpow(float lam, float n) {
+    constexpr float L2E_HI = 1.44269502162933349609f, L2E_LO = 1.92596299112661746e-8f, LN2F = 0.69314718055994530942f;
+    const float x = lam * n, lo = fmaf(lam, n, -x);
+    const float t = x * L2E_HI;
+    const float e = fmaf(x, L2E_HI, -t) + fmaf(x, L2E_LO, lo * L2E_HI);
+    const float y = __builtin_amdgcn_exp2f(t);
+    float r = fmaf(y, e * LN2F, y);
+    asm volatile("" : "+v"(r));
+    return r;
+}
+DEVINL float wpow(float lam, int n) { return wpow(lam, static_cast<float>(n)); }
+
+template <int CTRL> DEVINL float dpp(float x) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true)); }
+// sum over groups of 8 or 16 lanes, in all of them
+template <int LANES> DEVINL float lanes_sum(float x) {
+    x += dpp<0xB1>(x); x += dpp<0x4E>(x); x += dpp<0x141>(x);      // lane ^ 1, lane ^ 2, mirrored within eight
+    if constexpr (LANES == 16) x += dpp<0x140>(x);                // mirrored within sixteen
+    return x;
+}
+// eight fp32 values -> hi and lo operands
+struct Op2 { bf16x8 h, l; };
+DEVINL Op2 split8(const float (&x)[8]) {
+    const HL a = hilo2k(x[0], x[1]), b = hilo2k(x[2], x[3]), c = hilo2k(x[4], x[5]), d = hilo2k(x[6], x[7]);
+    return {as_op(a.h, b.h, c.h, d.h), as_op(a.l, b.l, c.l, d.l)};
+}
+DEVINL Op2 split8(const f32x4& x, const f32x4& y) { const float f[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]}; return split8(f); }
+DEVINL f32x4 mm3(const Op2& a, const Op2& b, f32x4 c) { return mfma(a.l, b.h, mfma(a.h, b.l, mfma(a.h, b.h, c))); }
+DEVINL void unpack(const bf16x8& x, float (&f)[8]) { unpack8(__builtin_bit_cast(uint4, x), f); }
+DEVINL Op2 scaled(const bf16x8& x, const float (&p)[8]) {
+    float f[8];
+    unpack(x, f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] *= p[e];
+    return split8(f);
+}
+// Operand with the 32 rows (tokens) of a plane along K in accumulator order: slot (g, e) <-> row 16 (e >> 2) + 4 g + (e & 3), lane
+// <-> column.  a: element [4 g + (l16 >> 2)][col + 4 (l16 & 3)].
+template <uint32_t ROW> DEVINL bf16x8 ld_tra(const lds_t a) {
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_ptr)(a));
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_ptr)(a + 16 * ROW));
+    const u32x2 x = __builtin_bit_cast(u32x2, lo), y = __builtin_bit_cast(u32x2, hi);
+    return as_op(x[0], x[1], y[0], y[1]);
+}
+DEVINL int slot_token(int g, int e) { return 16 * (e >> 2) + 4 * g + (e & 3); }
+
+// The head's parameters into LDS (by the first wave); every wave finds out for itself whether a decay is strong.
+template <int HN> DEVINL bool head_setup(const ArgsW& p, lds_t sb, int h, int b, int tid, float limit) {
+    const int lane = tid & 63;
+    float mn = 0.f;
+#pragma unroll
+    for (int z = 0; z < HN / 64; ++z) {
+        const int n = 64 * z + lane, c = h * HN + n;
+        const float l = -expf(bf2f(p.w[c]));
+        mn = fminf(mn, l);
+        if (tid < 64) {
+            lds_st<float>(sb + G<HN>::LAM + 4 * n, fmaxf(l, LAM_MIN));
+            lds_st<float>(sb + G<HN>::U + 4 * n, bf2f(p.u[c]));
+            if (p.decay != nullptr && b == 0) { p.decay[c] = expf(l); p.decay[p.C + c] = l; }
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o, 64));
+    return __builtin_amdgcn_readfirstlane(mn < limit ? 1 : 0) != 0;
+}
+
+// Rows of a [token][channel] tensor from one token on, as a buffer: reads of rows that do not exist give zeros, stores to them are
+// dropped, so the ends of a sequence cost no branches and no masks (an offset of 32 rows stays below 2^31: WKV5B_MAX_C).
+typedef __amdgpu_buffer_rsrc_t rows_t;
+DEVINL rows_t rows_of(const uint16_t* first, int left, int C) {
+    // (the two limits become one vector instruction: its result has to come back for the descriptor)
+    const int rows = __builtin_amdgcn_readfirstlane(min(max(left, 0), L));
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(first), 0, rows * C * 2, 0x00027000);
+}
+DEVINL uint4 load16(rows_t r, int o) { return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0)); }
+
+// A 16 x 16 tile of a bf16 output: rows (tokens) 4 g + v, lane = column.  Neighbouring lanes exchange halves, so that each stores
+// pairs of columns: even lanes rows 4 g, 4 g + 1, odd lanes the other two.  o: byte offset of the lane's first row and column.
+DEVINL int tile_offset(int l16, int g, int C) { return (4 * g + 2 * (l16 & 1)) * 2 * C + 2 * (l16 & ~1); }
+DEVINL void store_tile(rows_t out, int o, int C, int l16, const f32x4& x) {
+    const bool odd = l16 & 1;
+    const float r0 = dpp<0xB1>(odd ? x[0] : x[2]), r1 = dpp<0xB1>(odd ? x[1] : x[3]);
+    const uint32_t a = cvt2(odd ? r0 : x[0], odd ? x[2] : r0), b = cvt2(odd ? r1 : x[1], odd ? x[3] : r1);
+    __builtin_amdgcn_raw_buffer_store_b32(a, out, o, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(b, out, o + 2 * C, 0, 0);
+}
+
+// One wave's part (32 channels of the contraction) of a causal tile D[snk][src] = sum_j x_snk y_src, src <= snk, lane = src or snk
+// (LANE_SNK): three quadrants (row tile, lane tile).  x, y: two operands each (token tiles).
+template <bool LANE_SNK> struct Quad {       // {row tile, lane tile} of quadrant z
+    static constexpr int ROWT[3] = {0, LANE_SNK ? 0 : 1, 1}, LANET[3] = {0, LANE_SNK ? 1 : 0, 1};
+};
+// lane and row token of a tile element, whether it is strictly causal
+template <bool LANE_SNK> DEVINL bool causal(int z, int l16, int row) {
+    const int a = 16 * Quad<LANE_SNK>::ROWT[z] + row, b = 16 * Quad<LANE_SNK>::LANET[z] + l16;
+    return LANE_SNK ? a < b : b < a;
+}
+// the part, masked, with `diag` (of the lane's token in the lane tile) on its diagonal, to LDS
+template <bool LANE_SNK> DEVINL void put_part(lds_t out, const f32x4 (&q)[3], const float (&diag)[2], int lane) {
+    const int l16 = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+        f32x4 x;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            x[v] = causal<LANE_SNK>(z, l16, 4 * g + v) ? q[z][v] : 0.f;
+            if (Quad<LANE_SNK>::ROWT[z] == Quad<LANE_SNK>::LANET[z]) x[v] = l16 == 4 * g + v ? diag[Quad<LANE_SNK>::LANET[z]] : x[v];
+        }
+        lds_st<f32x4>(out + 1024 * z + 16 * lane, x);
+    }
+}
+// the parts added up and split: operands of the two lane tiles (slots: the row tokens in accumulator order)
+template <bool LANE_SNK, int PARTS, uint32_t PART> DEVINL void take_parts(lds_t in, int lane, Op2 (&a)[2]) {
+    f32x4 s[3];
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+        s[z] = lds_ld<f32x4>(in + 1024 * z + 16 * lane);
+#pragma unroll
+        for (int i = 1; i < PARTS; ++i) s[z] += lds_ld<f32x4>(in + i * PART + 1024 * z + 16 * lane);
+    }
+    // lane is the sink: sources of tile 0 for both lane tiles, of tile 1 for the second; lane is the source: the other way round
+    if constexpr (LANE_SNK) { a[0] = split8(s[0], ZERO4); a[1] = split8(s[1], s[2]); }
+    else { a[0] = split8(s[0], s[1]); a[1] = split8(ZERO4, s[2]); }
+}
+// powers for a tile part, channel ch0 + e: of token 16 z + l16, x as the sink, y as the source; they are those of the token in its
+// half (strong: in its 8 tokens) and serve both.  cx, cy: as sink of the second and source of the first half of a pair across
+// them; strong: w4 = o^4.
+template <bool STRONG> struct TilePowers { float px[8], py[8], cx[STRONG ? 1 : 8], cy[STRONG ? 1 : 8], w4[STRONG ? 8 : 1]; };
+template <bool STRONG> DEVINL void tile_powers(TilePowers<STRONG>& t, lds_t lam, int l16) {
+    const int m = STRONG ? 8 * (l16 >> 3) + 4 : 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float l = lds_f(lam + 4 * e);
+        t.px[e] = wpow(l, l16 - m); t.py[e] = wpow(l, m - 1 - l16);
+        if constexpr (STRONG) t.w4[e] = wpow(l, 4);
+        else { t.cx[e] = wpow(l, l16); t.cy[e] = wpow(l, 15 - l16); }
+    }
+}
+// tile part from raw rows (operands of the two token tiles)
+template <bool LANE_SNK, bool STRONG> DEVINL void raw_part(const bf16x8 (&r)[2], const bf16x8 (&k)[2], const TilePowers<STRONG>& t, int lane, f32x4 (&q)[3]) {
+    using Q = Quad<LANE_SNK>;
+    if constexpr (!STRONG) {
+#pragma unroll
+        for (int z = 0; z < 3; ++z) {
+            const bool across = Q::ROWT[z] != Q::LANET[z];
+            const int snk = LANE_SNK ? Q::LANET[z] : Q::ROWT[z], src = LANE_SNK ? Q::ROWT[z] : Q::LANET[z];
+            const Op2 x = scaled(r[snk], across ? t.cx : t.px), y = scaled(k[src], across ? t.cy : t.py);
+            q[z] = LANE_SNK ? mm3(y, x, ZERO4) : mm3(x, y, ZERO4);
+        }
+    } else {
+        const int l16 = lane & 15, g = lane >> 4;
+        float fx[8], fy[8];
+#pragma unroll
+        for (int z = 0; z < 3; ++z) q[z] = ZERO4;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            fx[e] = t.px[e]; fy[e] = t.py[e];
+            asm volatile("" : "+v"(fx[e]), "+v"(fy[e]));   // (the products below are the same in every chunk: 48 registers across the loop)
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            __builtin_amdgcn_sched_barrier(0);
+            const Op2 x[2] = {scaled(r[0], fx), scaled(r[1], fx)}, y[2] = {scaled(k[0], fy), scaled(k[1], fy)};
+#pragma unroll
+            for (int z = 0; z < 3; ++z) {
+                const f32x4 o = LANE_SNK ? mm3(y[Q::ROWT[z]], x[Q::LANET[z]], ZERO4) : mm3(x[Q::ROWT[z]], y[Q::LANET[z]], ZERO4);
+                const int rb = 2 * Q::ROWT[z] + (g >> 1), lb = 2 * Q::LANET[z] + (l16 >> 3);
+                const bool on = (LANE_SNK ? lb - rb : rb - lb) == d;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) q[z][v] = on ? o[v] : q[z][v];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { fx[e] *= t.w4[e]; fy[e] *= t.w4[e]; }
+        }
+    }
+}
+// NA tiles applied to an operand: sum over the row tokens (slots) of tile x operand, for one lane tile.  b: the operand, x scaled by
+// pf.  Strong: per distance d of the blocks of 8 tokens, with o^{4 d} on the operand and on the result (o^{8 d} may underflow where
+// the whole term is one); w4: o^4 of the output's lane, which is the operand's.
+template <bool LANE_SNK, bool STRONG, int NA>
+DEVINL void apply(const Op2 (&a)[NA], const Op2& b, const bf16x8& x, const float (&pf)[8], int lane_tile, int lane, float w4, f32x4 (&out)[NA]) {
+    if constexpr (!STRONG) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) out[i] = mm3(a[i], b, ZERO4);
+    } else {
+        const int l16 = lane & 15, g = lane >> 4, lb = 2 * lane_tile + (l16 >> 3), d0 = LANE_SNK ? lb - (g >> 1) : (g >> 1) - lb, d1 = d0 + (LANE_SNK ? -2 : 2);
+        float f = 1.f;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) out[i] = ZERO4;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            __builtin_amdgcn_sched_barrier(0);           // one distance after the other: side by side they take too many registers
+            float pd[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) pd[e] = pf[e] * f;
+            const Op2 bd = d == 0 ? b : scaled(x, pd);
+            const bool on0 = d0 == d, on1 = d1 == d;
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                const uint4 ah = __builtin_bit_cast(uint4, a[i].h), al = __builtin_bit_cast(uint4, a[i].l);
+                const Op2 ad = {as_op(on0 ? ah.x : 0u, on0 ? ah.y : 0u, on1 ? ah.z : 0u, on1 ? ah.w : 0u),
+                                as_op(on0 ? al.x : 0u, on0 ? al.y : 0u, on1 ? al.z : 0u, on1 ? al.w : 0u)};
+                out[i] += mm3(ad, bd, ZERO4) * f;
+            }
+            f *= w4;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------- forward
+// Waves 0..3 hold St[ct][jt][v] = S[j = 16 jt + 4 g + v][i = own], as it stands the B operand of a contraction over j.  Waves 4..7
+// load (two chunks ahead of the planes, the planes two chunks ahead of their use) and make the next chunk's tile in parts of 32
+// key channels.  One barrier a chunk.
+// Planes: R' = r o^{t-16}, K' = k o^{15-t} (they serve the tile, the state times o^16 on its way in and out of the update); strong:
+// r o^t, k o^{31-t}, and the tile is made from the raw rows.
+template <int HN, bool STRONG> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int q, int lane, size_t base, int nch) {
+    using A = G<HN>;
+    constexpr int CT = A::CT, KS = A::KS, NJ = A::NB16;
+    const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    float dd[NJ][4];                                     // o^16; strong: o^32
+#pragma unroll
+    for (int jt = 0; jt < NJ; ++jt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dd[jt][v] = wpow(lds_f(sb + A::LAM + 4 * (16 * jt + 4 * g + v)), STRONG ? 32 : 16);
+    f32x4 St[CT][NJ];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int jt = 0; jt < NJ; ++jt) St[ct][jt] = ZERO4;
+    const int nseg = (nch + 1) / 2;
+    float* const sv = p.saved != nullptr ? p.saved + static_cast<size_t>(blockIdx.x) * nseg * HN * HN + 16 * CT * q + l16 + 4 * g * HN : nullptr;
+    uint16_t* const out = p.y + base + 16 * CT * q;
+    const int to = tile_offset(l16, g, C);
+    const lds_t orow = sb + A::BASE + l16 * A::ROW + 8 * g, otr = sb + A::BASE + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3);
+    __syncthreads();                                     // chunks 0 and 1 are there
+    __syncthreads();                                     // and the first tile
+    int sl = 0;
+    for (int c = 0; c < nch; ++c) {
+        lds_t xr = orow + sl * A::FSLOT, xt = otr + sl * A::FSLOT;
+        opaque(xr); opaque(xt);
+        sl = sl == 2 ? 0 : sl + 1;
+        if (sv != nullptr && (c & 1) == 0) {
+            float* const d = sv + static_cast<size_t>(c >> 1) * HN * HN;
+#pragma unroll
+            for (int jt = 0; jt < NJ; ++jt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct) d[(16 * jt + v) * HN + 16 * ct] = St[ct][jt][v];
+        }
+        f32x4 Y[2][CT];
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) Y[tt][ct] = ZERO4;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            Op2 x[2];
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                x[tt].h = ld_acc(xr + A::FRH + 16 * tt * A::ROW + 64 * ks);
+                x[tt].l = ld_acc(xr + A::FRL + 16 * tt * A::ROW + 64 * ks);
+            }
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                if constexpr (!STRONG) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) { St[ct][2 * ks][v] *= dd[2 * ks][v]; St[ct][2 * ks + 1][v] *= dd[2 * ks + 1][v]; }
+                }
+                const Op2 s = split8(St[ct][2 * ks], St[ct][2 * ks + 1]);
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt) Y[tt][ct] = mm3(x[tt], s, Y[tt][ct]);
+            }
+        }
+        bf16x8 vo[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) vo[ct] = ld_tra<A::ROW>(xt + A::FV + 32 * (CT * q + ct));
+        Op2 at[2];
+        take_parts<true, A::PARTS, A::PART>(sb + A::FPART + (c & 1) * (A::PARTS * A::PART), lane, at);
+        const rows_t o = rows_of(out + static_cast<size_t>(c) * L * C, T - c * L, C);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const f32x4 y = mfma(at[tt].l, vo[ct], mfma(at[tt].h, vo[ct], Y[tt][ct]));
+                store_tile(o, to + 32 * tt * C + 32 * ct, C, l16, y);
+            }
+#pragma unroll
+        for (int jt = 0; jt < NJ; ++jt) {
+            const bf16x8 kh = ld_tra<A::ROW>(xt + A::FKH + 32 * jt), kl = ld_tra<A::ROW>(xt + A::FKL + 32 * jt);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                f32x4 s = St[ct][jt];
+                if constexpr (STRONG) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s[v] *= dd[jt][v];
+                }
+                s = mfma(kl, vo[ct], mfma(kh, vo[ct], s));
+                if constexpr (!STRONG) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s[v] *= dd[jt][v];
+                }
+                St[ct][jt] = s;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <int HN, bool STRONG> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int tp, size_t base, int nch) {
+    using A = G<HN>;
+    constexpr int NP = A::PASSES;
+    const int lane = tp & 63, q = tp >> 6, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    const int row0 = tp / A::PIECES, c8 = (tp % A::PIECES) * 8;
+    float u[8], pr[NP][8], pk[NP][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float l = lds_f(sb + A::LAM + 4 * (c8 + e));
+        u[e] = lds_f(sb + A::U + 4 * (c8 + e));
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+            const int t = row0 + z * A::ROWS;
+            pr[z][e] = wpow(l, STRONG ? t : t - 16);
+            pk[z][e] = wpow(l, STRONG ? 31 - t : 15 - t);
+        }
+    }
+    [[maybe_unused]] TilePowers<STRONG> tpw;
+    if constexpr (STRONG) tile_powers(tpw, sb + A::LAM + 4 * (32 * (q % A::PARTS) + 8 * g), l16);
+    uint4 x[2][3][NP];
+    auto fetch = [&](const int c, uint4 (&d)[3][NP]) __attribute__((always_inline)) {
+        const int cc = min(c, nch - 1);                  // (the same loads in every iteration)
+        const size_t o = base + static_cast<size_t>(cc) * L * C;
+        const int left = T - c * L;
+        const rows_t r = rows_of(p.r + o, left, C), k = rows_of(p.k + o, left, C), v = rows_of(p.v + o, left, C);
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+            const int lo = 2 * ((row0 + z * A::ROWS) * C + c8);
+            d[0][z] = load16(r, lo); d[1][z] = load16(k, lo); d[2][z] = load16(v, lo);
+        }
+    };
+    auto put = [&](const int sl, const uint4 (&d)[3][NP]) __attribute__((always_inline)) {
+        const lds_t s = sb + A::BASE + sl * A::FSLOT;
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+            const int t = row0 + z * A::ROWS;
+            float r[8], k[8], a = 0.f;
+            unpack8(d[0][z], r); unpack8(d[1][z], k);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { a = fmaf(r[e] * u[e], k[e], a); r[e] *= pr[z][e]; k[e] *= pk[z][e]; }
+            const Op2 ro = split8(r), ko = split8(k);
+            const lds_t o = s + t * A::ROW + 2 * c8;
+            lds_st<bf16x8>(o + A::FRH, ro.h); lds_st<bf16x8>(o + A::FRL, ro.l);
+            lds_st<bf16x8>(o + A::FKH, ko.h); lds_st<bf16x8>(o + A::FKL, ko.l);
+            lds_st<bf16x8>(o + A::FV, op4(d[2][z]));
+            a = lanes_sum<A::PIECES>(a);
+            if (c8 == 0) lds_st<float>(s + A::FRUK + 4 * t, a);
+        }
+    };
+    auto tile = [&](const int c, const int sl) __attribute__((always_inline)) {
+        if (q >= A::PARTS) return;
+        f32x4 qd[3];
+        const lds_t s = sb + A::BASE + sl * A::FSLOT;
+        if constexpr (STRONG) {
+            const size_t co = base + static_cast<size_t>(c) * L * C;
+            const rows_t rr = rows_of(p.r + co, T - c * L, C), kk = rows_of(p.k + co, T - c * L, C);
+            bf16x8 r[2], k[2];
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const int o = 2 * ((16 * z + l16) * C + 32 * q + 8 * g);
+                r[z] = op4(load16(rr, o)); k[z] = op4(load16(kk, o));
+            }
+            raw_part<true, true>(r, k, tpw, lane, qd);
+        } else {
+            Op2 xo[2], yo[2];
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const lds_t o = s + (16 * z + l16) * A::ROW + 64 * q + 16 * g;
+                xo[z] = {ld_op(o + A::FRH), ld_op(o + A::FRL)};
+                yo[z] = {ld_op(o + A::FKH), ld_op(o + A::FKL)};
+            }
+#pragma unroll
+            for (int z = 0; z < 3; ++z) qd[z] = mm3(yo[Quad<true>::ROWT[z]], xo[Quad<true>::LANET[z]], ZERO4);
+        }
+        const float diag[2] = {q == 0 ? lds_f(s + A::FRUK + 4 * l16) : 0.f, q == 0 ? lds_f(s + A::FRUK + 4 * (16 + l16)) : 0.f};
+        put_part<true>(sb + A::FPART + ((c & 1) * A::PARTS + q) * A::PART, qd, diag, lane);
+    };
+    fetch(0, x[0]); fetch(1, x[1]);
+    put(0, x[0]); fetch(2, x[0]);
+    put(1, x[1]); fetch(3, x[1]);
+    __syncthreads();
+    tile(0, 0);
+    __syncthreads();
+    int sl = 2;
+    for (int c0 = 0; c0 < nch; c0 += 2) {
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            const int c = c0 + z;
+            if (c >= nch) break;
+            put(sl, x[z]);
+            fetch(c + 4, x[z]);
+            if (c + 1 < nch) tile(c + 1, sl == 0 ? 2 : sl - 1);
+            sl = sl == 2 ? 0 : sl + 1;
+            __syncthreads();
+        }
+    }
+}
+
+template <int HN>
+__global__ __launch_bounds__(NTH, 2) void wkv5b_fwd(const ArgsW p) {
+    const lds_t sb = lds_of(smem_raw);
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = (p.T + L - 1) / L;
+    const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
+    const bool strong = head_setup<HN>(p, sb, h, b, tid, LAM_STRONG_F);
+    __syncthreads();
+    if (w < 4) {
+        if (strong) fwd_states<HN, true>(p, sb, w, tid & 63, base, nch);
+        else fwd_states<HN, false>(p, sb, w, tid & 63, base, nch);
+    } else {
+        if (strong) fwd_loads<HN, true>(p, sb, tid - 256, base, nch);
+        else fwd_loads<HN, false>(p, sb, tid - 256, base, nch);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------- backward
+// One reverse sweep, two barriers a chunk, two roles of four waves:
+//   D, waves 0..3 (key channels j): the gradient state dS[ct][ib][v] = D[i = 16 ib + 4 g + v][j = own], the B operand of contractions
+//      over the value channel: gk in the first half of a chunk; gr, the gradient state's update and the decay gradient in the second.
+//      The saved state passes through in tiles (an odd chunk's is one update away from the saved one, made on the way).  The tile B is
+//      made by each of these waves in both orientations: its operands are the rows that the state products read anyway, and an
+//      accumulator with the summed tokens in its registers is an operand as it stands.
+//   E, waves 4..7 (value channels i): first half: the loads, the rows of the next chunk to LDS, this chunk's tile A in parts; second
+//      half: gv, for which the D waves left their gradient state in LDS (hi, lo) in the first.
+template <bool LANE_SNK> DEVINL void mask(f32x4 (&b)[3], int l16, int g) {
+#pragma unroll
+    for (int z = 0; z < 3; ++z)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) b[z][v] = causal<LANE_SNK>(z, l16, 4 * g + v) ? b[z][v] : 0.f;
+}
+
+template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, int h, int b, size_t base, int nch) {
+    using A = G<HN>;
+    constexpr int CT = A::CT, KS = A::KS, NI = A::NB16;
+    const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    // Powers of a set of eight slots, token 16 a + 4 g + b: a base per lane times o^b times o^{16 a} (or the reverse); the eight would
+    // take the registers that the states need.  Bases: cb of o^{t-m}, kb of o^{m-1-t}, m the middle of the token's half (strong: of
+    // its 8 tokens).
+    float l[CT], u[CT], o1[CT], o2[CT], o3[CT], o8[CT], o16[CT], o32[CT], cb[CT], kb[CT];
+    f32x4 dS[CT][NI];
+    float gw[CT], gP[CT], gu[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int j = 16 * (CT * q + ct) + l16;
+        l[ct] = lds_f(sb + A::LAM + 4 * j); u[ct] = lds_f(sb + A::U + 4 * j);
+        o1[ct] = wpow(l[ct], 1); o2[ct] = wpow(l[ct], 2); o3[ct] = wpow(l[ct], 3); o8[ct] = wpow(l[ct], 8); o16[ct] = wpow(l[ct], 16); o32[ct] = wpow(l[ct], 32);
+        cb[ct] = wpow(l[ct], STRONG ? 4 * (g & 1) - 4 : 4 * g - 8);
+        kb[ct] = wpow(l[ct], STRONG ? -4 * (g & 1) : 4 - 4 * g);
+#pragma unroll
+        for (int ib = 0; ib < NI; ++ib) dS[ct][ib] = ZERO4;
+        gw[ct] = gP[ct] = gu[ct] = 0.f;
+    }
+    // (hidden: hoisted out of the loop the powers and token numbers would take registers all the same)
+    auto hide = [](float x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); return x; };
+    auto up = [&](int ct, float base, bool span, float (&f)[8]) __attribute__((always_inline)) {
+        base = hide(base);
+        f[0] = base; f[1] = base * o1[ct]; f[2] = base * o2[ct]; f[3] = base * o3[ct];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[4 + e] = span ? f[e] * o16[ct] : f[e];
+    };
+    auto down = [&](int ct, float base, bool span, float (&f)[8]) __attribute__((always_inline)) {
+        base = hide(base);
+        f[4] = base * o3[ct]; f[5] = base * o2[ct]; f[6] = base * o1[ct]; f[7] = base;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = span ? f[4 + e] * o16[ct] : f[4 + e];
+    };
+    auto to_ref = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { up(ct, cb[ct], false, f); };                                    // o^{t-m}
+    auto from_ref = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { down(ct, kb[ct], false, f); };                                // o^{m-1-t}
+    auto from_start = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { up(ct, STRONG ? wpow(hide(l[ct]), 4 * g) : cb[ct] * o8[ct], true, f); };            // o^t
+    auto to_end = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { down(ct, STRONG ? wpow(hide(l[ct]), 12 - 4 * g) : kb[ct] * o8[ct], true, f); };         // o^{31-t}
+    // The operands that a tile's lane tiles 0 and 1 are applied to, referred to the middle of the lane's half whichever half a slot's
+    // token lies in.  f: the powers of the token in its own half.  Only the far pair (sinks of the second half for a source of the
+    // first, or sources of the first for a sink of the second) takes o^16; the slots on the wrong side of the lane tile meet zeros.
+    auto tile_operands = [&](int ct, bool sinks, const bf16x8& x, const float (&f)[8], Op2 (&o)[2]) __attribute__((always_inline)) {
+        float fx[8], ff[4];
+        unpack(x, fx);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) fx[e] *= f[e];
+        o[0] = o[1] = split8(fx);
+        if constexpr (!STRONG) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ff[e] = (sinks ? fx[4 + e] : fx[e]) * o16[ct];
+            const HL a = hilo2k(ff[0], ff[1]), b = hilo2k(ff[2], ff[3]);
+            Op2& w = o[sinks ? 0 : 1];
+            const uint4 h = __builtin_bit_cast(uint4, w.h), lo = __builtin_bit_cast(uint4, w.l);
+            w = sinks ? Op2{as_op(h.x, h.y, a.h, b.h), as_op(lo.x, lo.y, a.l, b.l)} : Op2{as_op(a.h, b.h, h.z, h.w), as_op(a.l, b.l, lo.z, lo.w)};
+        }
+    };
+    const float t0 = static_cast<float>(4 * g);
+    const int to = tile_offset(l16, g, C);
+    const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * (nch / 2) * HN * HN + (16 * CT * q + l16) * HN + 4 * g;
+    auto fetch_state = [&](int c, int ks, f32x4 (&s)[CT][2]) __attribute__((always_inline)) {
+        const float* const d = sv + static_cast<size_t>(c >> 1) * HN * HN + 32 * ks;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int z = 0; z < 2; ++z) s[ct][z] = *reinterpret_cast<const f32x4*>(d + 16 * ct * HN + 16 * z);
+    };
+    auto chunk = [&](auto odd_, const int c) __attribute__((always_inline)) {
+        constexpr bool ODD = decltype(odd_)::value;
+        const lds_t sx = sb + A::BASE + (ODD ? A::SLOT : 0);
+        lds_t xr = sx + l16 * A::ROW + 8 * g, xt = sx + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3), xs = sx + 16 * g;
+        lds_t ho = sb + A::DSH + (16 * CT * q + l16) * A::ROW + 8 * g;
+        opaque(xr); opaque(xt); opaque(xs); opaque(ho);
+        const size_t co = base + static_cast<size_t>(c) * L * C + 16 * CT * q;
+        const rows_t gk_ = rows_of(p.gk + co, T - c * L, C), gr_ = rows_of(p.gr + co, T - c * L, C);
+        // ---- first half: gk
+        f32x4 Z[2][CT], Bt[3] = {ZERO4, ZERO4, ZERO4}, Ct[3] = {ZERO4, ZERO4, ZERO4};
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) { Z[0][ct] = ZERO4; Z[1][ct] = ZERO4; }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            bf16x8 va[2], ga[2];
+#pragma unroll
+            for (int z = 0; z < 2; ++z) { va[z] = ld_acc(xr + A::V + 16 * z * A::ROW + 64 * ks); ga[z] = ld_acc(xr + A::GY + 16 * z * A::ROW + 64 * ks); }
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const Op2 s = split8(dS[ct][2 * ks], dS[ct][2 * ks + 1]);
+                const uint4 hi = __builtin_bit_cast(uint4, s.h), lo = __builtin_bit_cast(uint4, s.l);
+                const lds_t o = ho + 16 * ct * A::ROW + 64 * ks;
+                lds_st<u32x2>(o, u32x2{hi.x, hi.y}); lds_st<u32x2>(o + 32, u32x2{hi.z, hi.w});
+                lds_st<u32x2>(o + (A::DSL - A::DSH), u32x2{lo.x, lo.y}); lds_st<u32x2>(o + (A::DSL - A::DSH) + 32, u32x2{lo.z, lo.w});
+#pragma unroll
+                for (int z = 0; z < 2; ++z) Z[z][ct] = mfma(va[z], s.l, mfma(va[z], s.h, Z[z][ct]));
+            }
+#pragma unroll
+            for (int z = 0; z < 3; ++z) {
+                Bt[z] = mfma(ga[Quad<false>::ROWT[z]], va[Quad<false>::LANET[z]], Bt[z]);         // rows: sinks, lane: source
+                Ct[z] = mfma(va[Quad<true>::ROWT[z]], ga[Quad<true>::LANET[z]], Ct[z]);           // rows: sources, lane: sink
+            }
+        }
+        mask<false>(Bt, l16, g); mask<true>(Ct, l16, g);
+        f32x4 Lt[3];                                     // the tile weighted with the tokens between, for the decay gradient
+        {
+            const float lag = hide(t0 - static_cast<float>(l16 + 1));
+#pragma unroll
+            for (int z = 0; z < 3; ++z)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) Lt[z][v] = Bt[z][v] * (lag + static_cast<float>(16 * (Quad<false>::ROWT[z] - Quad<false>::LANET[z]) + v));
+        }
+        const Op2 ba[2] = {split8(Bt[0], Bt[1]), split8(ZERO4, Bt[2])}, la[2] = {split8(Lt[0], Lt[1]), split8(ZERO4, Lt[2])}, ca[2] = {split8(Ct[0], ZERO4), split8(Ct[1], Ct[2])};
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const bf16x8 rT = ld_tra<A::ROW>(xt + A::R + 32 * (CT * q + ct)), kT = ld_tra<A::ROW>(xt + A::K + 32 * (CT * q + ct));
+            const f32x4 vg0 = lds_ld<f32x4>(xs + A::VG), vg1 = lds_ld<f32x4>(xs + A::VG + 64);
+            float r[8], k[8], pe[8], pf[8], pm[8];
+            unpack(rT, r); unpack(kT, k);
+            Op2 ro[2];
+            to_ref(ct, pm);
+            tile_operands(ct, true, rT, pm, ro);
+            from_ref(ct, pf);
+            to_end(ct, pe);
+            const float w4 = STRONG ? o2[ct] * o2[ct] : 1.f;
+            const float th = hide(t0);
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const Op2 tiles[2] = {ba[z], la[z]};
+                f32x4 tz[2];
+                apply<false, STRONG>(tiles, ro[z], rT, pm, z, lane, w4, tz);
+                f32x4 o;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int e = 4 * z + v;
+                    const float zs = Z[z][ct][v] * pe[e], ti = tz[0][v] * pf[e], vg = z ? vg1[v] : vg0[v], t = th + static_cast<float>(16 * z + v);
+                    gw[ct] = fmaf(k[e], (31.f - t) * zs + tz[1][v] * pf[e], gw[ct]);
+                    const float rv = r[e] * vg;
+                    gu[ct] = fmaf(rv, k[e], gu[ct]);
+                    o[v] = fmaf(rv, u[ct], zs + ti);
+                }
+                store_tile(gk_, to + 32 * z * C + 32 * ct, C, l16, o);
+            }
+        }
+        f32x4 Sn[2][CT][2];
+        fetch_state(c, 0, Sn[0]);
+        fetch_state(c, 1, Sn[1]);
+        __syncthreads();                                 // the rows of the chunk before are there, the gradient state is handed over
+        // ---- second half: gr, update
+        const lds_t qt = sb + A::BASE + (ODD ? 0 : A::SLOT) + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3);
+        Op2 rs[CT], kp[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            float f[8];
+            from_start(ct, f);
+            rs[ct] = scaled(ld_tra<A::ROW>(xt + A::R + 32 * (CT * q + ct)), f);
+            if constexpr (ODD) {
+                to_end(ct, f);
+                kp[ct] = scaled(ld_tra<A::ROW>(qt + A::K + 32 * (CT * q + ct)), f);
+            }
+        }
+        f32x4 X[2][CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) { X[0][ct] = ZERO4; X[1][ct] = ZERO4; }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            bf16x8 ga[2];
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const bf16x8 gt = ld_tra<A::ROW>(xt + A::GY + 64 * ks + 32 * z);
+                bf16x8 vt;
+                if constexpr (ODD) vt = ld_tra<A::ROW>(qt + A::V + 64 * ks + 32 * z);
+                ga[z] = ld_acc(xr + A::GY + 16 * z * A::ROW + 64 * ks);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                    f32x4& s = Sn[ks & 1][ct][z];
+                    f32x4& d = dS[ct][2 * ks + z];
+                    if constexpr (ODD) s = mfma(vt, kp[ct].l, mfma(vt, kp[ct].h, s * o32[ct]));
+                    gP[ct] += (s[0] * d[0] + s[1] * d[1]) + (s[2] * d[2] + s[3] * d[3]);
+                    d = mfma(gt, rs[ct].l, mfma(gt, rs[ct].h, d * o32[ct]));
+                }
+            }
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const Op2 s = split8(Sn[ks & 1][ct][0], Sn[ks & 1][ct][1]);
+#pragma unroll
+                for (int z = 0; z < 2; ++z) X[z][ct] = mfma(ga[z], s.l, mfma(ga[z], s.h, X[z][ct]));
+            }
+            if (ks + 2 < KS) fetch_state(c, ks + 2, Sn[ks & 1]);
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const bf16x8 rT = ld_tra<A::ROW>(xt + A::R + 32 * (CT * q + ct)), kT = ld_tra<A::ROW>(xt + A::K + 32 * (CT * q + ct));
+            const f32x4 vg0 = lds_ld<f32x4>(xs + A::VG), vg1 = lds_ld<f32x4>(xs + A::VG + 64);
+            float r[8], k[8], ps[8], pf[8], pm[8];
+            unpack(rT, r); unpack(kT, k);
+            Op2 ko[2];
+            from_ref(ct, pm);
+            tile_operands(ct, false, kT, pm, ko);
+            to_ref(ct, pf);
+            from_start(ct, ps);
+            const float w4 = STRONG ? o2[ct] * o2[ct] : 1.f;
+            const float th = hide(t0);
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const Op2 tiles[1] = {ca[z]};
+                f32x4 tx[1];
+                apply<true, STRONG>(tiles, ko[z], kT, pm, z, lane, w4, tx);
+                f32x4 o;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int e = 4 * z + v;
+                    const float x = X[z][ct][v] * ps[e], ti = tx[0][v] * pf[e], vg = z ? vg1[v] : vg0[v], t = th + static_cast<float>(16 * z + v);
+                    gw[ct] = fmaf(r[e] * t, x, gw[ct]);
+                    o[v] = fmaf(k[e] * vg, u[ct], x + ti);
+                }
+                store_tile(gr_, to + 32 * z * C + 32 * ct, C, l16, o);
+            }
+        }
+        __syncthreads();
+    };
+    __syncthreads();                                     // the top chunk is there
+    for (int c = nch - 1; c >= 0; c -= 2) {
+        chunk(std::true_type{}, c);
+        chunk(std::false_type{}, c - 1);
+    }
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int c = h * HN + 16 * (CT * q + ct) + l16;
+        const float sw = allreduce_rows(fmaf(32.f * o32[ct], gP[ct], gw[ct])), su = allreduce_rows(gu[ct]);
+        if (g == 0) {
+            const float lt = -expf(bf2f(p.w[c]));        // (a decay below the smallest one: its gradient is that of the pairs one step apart)
+            const float f = expf(lt - l[ct]);            // zero long before lt leaves fp32's range
+            p.gw[static_cast<size_t>(b) * C + c] = f2bf(f > 0.f ? lt * f * sw : 0.f);
+            p.gu[static_cast<size_t>(b) * C + c] = f2bf(su);
+        }
+    }
+}
+
+template <int HN, bool STRONG> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, size_t base, int nch) {
+    using A = G<HN>;
+    constexpr int CT = A::CT, KS = A::KS, NP = A::PASSES;
+    const int q = __builtin_amdgcn_readfirstlane(te >> 6), lane = te & 63, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    const int row0 = te / A::PIECES, c8 = (te % A::PIECES) * 8, to = tile_offset(l16, g, C);
+    float u[8], cke[2][KS][8];                           // cke: o^{31-t} of token 16 tt + l16, channel 32 ks + 8 g + e
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        u[e] = lds_f(sb + A::U + 4 * (c8 + e));
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const float l = lds_f(sb + A::LAM + 4 * (32 * ks + 8 * g + e));
+            cke[0][ks][e] = wpow(l, 31 - l16); cke[1][ks][e] = wpow(l, 15 - l16);
+        }
+    }
+    TilePowers<STRONG> tp;
+    tile_powers(tp, sb + A::LAM + 4 * (32 * (q % A::PARTS) + 8 * g), l16);
+    auto fetch = [&](const int c, uint4 (&d)[4][NP]) __attribute__((always_inline)) {
+        const int cc = max(c, 0);
+        const size_t o = base + static_cast<size_t>(cc) * L * C;
+        const int left = T - cc * L;
+        const rows_t r = rows_of(p.r + o, left, C), k = rows_of(p.k + o, left, C), v = rows_of(p.v + o, left, C), gy = rows_of(p.gy + o, left, C);
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+            const int lo = 2 * ((row0 + z * A::ROWS) * C + c8);
+            d[0][z] = load16(r, lo); d[1][z] = load16(k, lo); d[2][z] = load16(v, lo); d[3][z] = load16(gy, lo);
+        }
+    };
+    auto put = [&](const int sl, const uint4 (&d)[4][NP]) __attribute__((always_inline)) {
+        const lds_t s = sb + A::BASE + sl * A::SLOT;
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+            const int t = row0 + z * A::ROWS;
+            const lds_t o = s + t * A::ROW + 2 * c8;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lds_st<bf16x8>(o + i * A::PLANE, op4(d[i][z]));
+            float r[8], k[8], v[8], gy[8], a = 0.f, b = 0.f;
+            unpack8(d[0][z], r); unpack8(d[1][z], k); unpack8(d[2][z], v); unpack8(d[3][z], gy);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { a = fmaf(r[e] * u[e], k[e], a); b = fmaf(v[e], gy[e], b); }
+            a = lanes_sum<A::PIECES>(a); b = lanes_sum<A::PIECES>(b);
+            if (c8 == 0) { lds_st<float>(s + A::RUK + 4 * t, a); lds_st<float>(s + A::VG + 4 * t, b); }
+        }
+    };
+    uint4 ring[2][4][NP];
+    {
+        uint4 top[4][NP];
+        fetch(nch - 1, top);
+        fetch(nch - 2, ring[0]);                         // chunk c rides in ring[c & 1]
+        fetch(nch - 3, ring[1]);
+        put(1, top);
+    }
+    auto chunk = [&](auto odd_, const int c) __attribute__((always_inline)) {
+        constexpr bool ODD = decltype(odd_)::value;
+        constexpr int PREV = ODD ? 0 : 1;
+        const lds_t sx = sb + A::BASE + (ODD ? A::SLOT : 0);
+        // ---- first half
+        if (q < A::PARTS) {
+            lds_t o = sx + l16 * A::ROW + 64 * q + 16 * g;
+            opaque(o);
+            const bf16x8 r[2] = {ld_op(o + A::R), ld_op(o + A::R + 16 * A::ROW)}, k[2] = {ld_op(o + A::K), ld_op(o + A::K + 16 * A::ROW)};
+            f32x4 qd[3];
+            raw_part<false, STRONG>(r, k, tp, lane, qd);
+            const float diag[2] = {q == 0 ? lds_f(sx + A::RUK + 4 * l16) : 0.f, q == 0 ? lds_f(sx + A::RUK + 4 * (16 + l16)) : 0.f};
+            put_part<false>(sb + A::BPART + q * A::PART, qd, diag, lane);
+        }
+        put(PREV, ring[PREV]);                           // (chunk 0: rows that nobody reads)
+        fetch(c - 3, ring[PREV]);
+        __syncthreads();
+        // ---- second half: gv
+        lds_t xo = sx + l16 * A::ROW + 16 * g, ht = sb + A::DSH + (8 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3) + 32 * CT * q;
+        lds_t xt = sx + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3) + 32 * CT * q;
+        opaque(xo); opaque(ht); opaque(xt);
+        f32x4 O[2][CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) { O[0][ct] = ZERO4; O[1][ct] = ZERO4; }
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const Op2 ke[2] = {scaled(ld_op(xo + A::K + 64 * ks), cke[0][ks]), scaled(ld_op(xo + A::K + 16 * A::ROW + 64 * ks), cke[1][ks])};
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const Op2 s = {ld_tr(ht + 32 * ks * A::ROW + 32 * ct, A::ROW), ld_tr(ht + (A::DSL - A::DSH) + 32 * ks * A::ROW + 32 * ct, A::ROW)};
+#pragma unroll
+                for (int z = 0; z < 2; ++z) O[z][ct] = mm3(ke[z], s, O[z][ct]);
+            }
+        }
+        Op2 at[2];
+        take_parts<false, A::PARTS, A::PART>(sb + A::BPART, lane, at);
+        const rows_t out = rows_of(p.gv + base + static_cast<size_t>(c) * L * C + 16 * CT * q, T - c * L, C);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const bf16x8 go = ld_tra<A::ROW>(xt + A::GY + 32 * ct);
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const f32x4 o = mfma(at[z].l, go, mfma(at[z].h, go, O[z][ct]));
+                store_tile(out, to + 32 * z * C + 32 * ct, C, l16, o);
+            }
+        }
+        __syncthreads();
+    };
+    __syncthreads();
+    for (int c = nch - 1; c >= 0; c -= 2) {
+        chunk(std::true_type{}, c);
+        chunk(std::false_type{}, c - 1);
+    }
+}
+
+template <int HN>
+__global__ __launch_bounds__(NTH, 2) void wkv5b_bwd(const ArgsW p) {
+    const lds_t sb = lds_of(smem_raw);
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = 2 * ((p.T + 2 * L - 1) / (2 * L));      // whole pairs (a last chunk without tokens adds zeros)
+    const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
+    const bool strong = head_setup<HN>(p, sb, h, b, tid, LAM_STRONG_B);
+    __syncthreads();
+    if (w < 4) {
+        if (strong) role_d<HN, true>(p, sb, w, tid & 63, h, b, base, nch);
+        else role_d<HN, false>(p, sb, w, tid & 63, h, b, base, nch);
+    } else {
+        if (strong) role_e<HN, true>(p, sb, tid - 256, base, nch);
+        else role_e<HN, false>(p, sb, tid - 256, base, nch);
+    }
+}
+
+template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, uint32_t lds) {
+    if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); e != hipSuccess) {
+        g_last_hip_error = static_cast<int>(e);
+        return RWKV_ERR_LAUNCH;
+    }
+    hipLaunchKernelGGL(kernel, dim3(B * p.H), dim3(NTH), lds, st, p);
+    return launch_status();
+}
+
+}  // namespace
+
+size_t wkv5b_saved_bytes(int B, int T, int C, int H) {
+    const size_t nch = (static_cast<size_t>(T) + L - 1) / L, n = C / H;
+    return static_cast<size_t>(B) * H * ((nch + 1) / 2) * n * n * sizeof(float);
+}
+int launch_wkv5b_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
+                     const uint16_t* u, uint16_t* y, float* decay, float* saved) {
+    ArgsW p{};
+    p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.decay = decay; p.saved = saved;
+    return launch(wkv5b_fwd<128>, st, B, p, G<128>::FTOTAL);
+}
+int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
+                     const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu, const float* saved) {
+    ArgsW p{};
+    p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv; p.gw = gw; p.gu = gu;
+    p.saved = const_cast<float*>(saved);
+    return launch(wkv5b_bwd<128>, st, B, p, G<128>::BTOTAL);
+}
+
+}  // namespace rwkv

@@ -1,0 +1,58 @@
+"""GPU: bf16 wkv5 with heads of 128 channels, a workgroup per head (rwkv_wkv5s_*, what wkv5_bf16.RUN_CUDA runs), against the fp64
+oracle where it can go wrong: one token, whole chunks (32 tokens) and pairs of them (a saved state each) and one off, and decays
+of every strength: slow ones, some beyond what one reference token per chunk carries, and ones whose powers leave fp32's range
+within a few steps.  The bar is that of the other bf16 kernels: no further from fp64 than fp32 arithmetic with rounded outputs."""
+import pytest
+import torch
+
+from oracle import wkv56 as O
+from rwkv_cuda_amd import synth, wkv5_bf16
+from _gpu_util import DEV, assert_no_worse
+
+pytestmark = pytest.mark.gpu
+N = 128
+
+
+def _run(B, T, C, H, r, k, v, w, u, gy):
+    t = [x.to(DEV).requires_grad_(True) for x in (r, k, v, w, u)]
+    y = wkv5_bf16.RUN_CUDA(B, T, C, H, *t)
+    y.backward(gy.to(DEV))
+    with torch.no_grad():                                   # a forward that keeps no states
+        assert torch.equal(wkv5_bf16.RUN_CUDA(B, T, C, H, *t), y)
+    return [y.detach()] + [x.grad for x in t]
+
+
+def _decays(kind, w):
+    if kind == "usual":
+        return w
+    g = torch.Generator().manual_seed(5)
+    lo, hi = {"strong": (1.0, 4.0), "slow": (-8.0, -4.0), "mixed": (-6.0, 3.0)}[kind]      # exp(-exp(4)) = 2e-24 a step
+    return (torch.rand(w.shape, generator=g) * (hi - lo) + lo).to(w.dtype)
+
+
+@pytest.mark.parametrize("decays", ["usual", "slow", "mixed", "strong"])
+@pytest.mark.parametrize("T", [1, 2, 31, 32, 33, 63, 64, 65, 96, 97, 130, 260])
+def test_wkv5_whole_heads(lib, T, decays):
+    B, H = 2, 2
+    C = H * N
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=900 + T)
+    w = _decays(decays, w)
+    print(f"\nwkv5 N=128 T={T} {decays}", flush=True)
+    ref = O.wkv5_grads(B, T, C, H, r, k, v, w, u, gy)
+    emu = O.emulate_wkv5_bf16(B, T, C, H, r, k, v, w, u, gy)
+    for name, a, e, g in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, _run(B, T, C, H, r, k, v, w, u, gy)):
+        assert_no_worse(name, a, e.reshape(a.shape), g.reshape(a.shape))
+
+
+def test_one_strong_head_among_others_changes_nothing_else(lib):
+    """Every workgroup picks its powers by its own head: the heads without a strong channel give the same bits."""
+    B, T, H = 2, 100, 3
+    C = H * N
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=31)
+    a = _run(B, T, C, H, r, k, v, w, u, gy)
+    w = w.clone()
+    w.view(H, N)[1, 70] = 2.5
+    b = _run(B, T, C, H, r, k, v, w, u, gy)
+    for x, y in zip(a[:4], b[:4]):
+        x, y = x.view(B, T, H, N), y.view(B, T, H, N)
+        assert torch.equal(x[:, :, 0], y[:, :, 0]) and torch.equal(x[:, :, 2], y[:, :, 2]) and not torch.equal(x[:, :, 1], y[:, :, 1])
