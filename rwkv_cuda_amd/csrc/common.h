@@ -176,7 +176,8 @@ int launch_wkv5_bwd_a_split(hipStream_t st, int cross, int B, int T, int C, int 
 int launch_wkv5_bwd_b_split(hipStream_t st, int cross, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k,
                             const uint16_t* v, const float* ew, const uint16_t* u, const uint16_t* gy, float* gk32, float* gv32,
                             float* gw32, const float* rdr);
-// wkv5_bf.hip: wkv5, bf16, heads of 128 channels, whole heads, decays of any strength; w raw.  saved (may be null in the forward):
+// wkv5_bf.hip: wkv5, bf16, heads of 128 or 64 channels, whole heads, decays of any strength; w raw.  Size 64: only layers with a
+// strong decay (strong_layer, wkv6_fused.h), the others belong to the one-sweep kernels above and the launch returns at once.  saved (may be null in the forward):
 // the states for the backward; gw, gu: per-batch rows [B][C].
 constexpr int WKV5B_MAX_C = 1 << 24;           // byte offsets within 32 rows are 32-bit
 size_t wkv5b_saved_bytes(int B, int T, int C, int H);

@@ -1358,12 +1358,16 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H, const rw
 // heads of 128 channels: one workgroup holds a whole head (wkv5_bf.hip)
 namespace {
 bool whole_head_ok(int C, int H, unsigned flags) { return C == H * N_SPLIT && !(flags & (RWKV_FLAG_SWEEPS | RWKV_PASS_ALL)) && C <= WKV5B_MAX_C; }
+bool fused5_ok(int T, int C, int H, unsigned flags) { return fused_ok(T, C, H, flags) && C <= WKV5B_MAX_C; }
 size_t whole_head_ws_bytes(int B, int C) { return 2 * round16(static_cast<size_t>(B) * C * sizeof(uint16_t)); }
 }  // namespace
 
 size_t rwkv_wkv5s_saved_bytes(int B, int T, int C, int H) {
-    if (check_dims(B, T, C, H) == RWKV_OK && whole_head_ok(C, H, 0u)) return wkv5b_saved_bytes(B, T, C, H);
-    return rwkv_wkv6f_saved_bytes(B, T, C, H);
+    if (check_dims(B, T, C, H) != RWKV_OK) return 0;
+    if (whole_head_ok(C, H, 0u)) return wkv5b_saved_bytes(B, T, C, H);
+    // head size 64: a layer keeps the states of the one-sweep kernels or, with a strong decay, those of wkv5_bf.hip
+    const size_t n = rwkv_wkv6f_saved_bytes(B, T, C, H);
+    return n == 0 || C > WKV5B_MAX_C ? 0 : (n < wkv5b_saved_bytes(B, T, C, H) ? wkv5b_saved_bytes(B, T, C, H) : n);
 }
 
 int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16* r, const rwkv_bf16* k, const rwkv_bf16* v,
@@ -1380,7 +1384,7 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         }
         if (saved != nullptr) return e;
     }
-    if (!fused_ok(T, C, H, flags) || saved == nullptr) {
+    if (!fused5_ok(T, C, H, flags) || saved == nullptr) {
         hipLaunchKernelGGL(wkv5_decay_transform, dim3((C + 255) / 256), dim3(256), 0, st, C, w_raw, decay);
         return rwkv_wkv5_forward_ex(stream, B, T, C, H, r, k, v, decay, u, y, flags);
     }
@@ -1399,7 +1403,7 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, NB, TB, local, logdec, s32, decay)) return e;
     } else if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, 1, 0, nullptr, nullptr, nullptr, decay)) return e;
-    return launch_wkv6_fwd_chunk(st, W_HEAD, B, T, C, H, r, k, v, decay, u, nullptr, y, static_cast<char*>(saved), flg);
+    return launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved));
 }
 
 size_t rwkv_wkv5s_backward_workspace_bytes(int B, int T, int C, int H) {
@@ -1429,14 +1433,13 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
     }
     if (workspace == nullptr || workspace_bytes < rwkv_wkv5s_backward_workspace_bytes(B, T, C, H) || !aligned16(workspace))
         return RWKV_ERR_WORKSPACE;
-    if (!fused_ok(T, C, H, flags) || saved == nullptr)
+    if (!fused5_ok(T, C, H, flags) || saved == nullptr)
         return rwkv_wkv5raw_backward(stream, B, T, C, H, r, k, v, decay, u, gy, gr, gk, gv, gw, gu, workspace, workspace_bytes, flags);
     if (int e = check_ptrs({r, k, v, w_raw, decay, u, gy, gr, gk, gv, gw, gu})) return e;
     if (saved_bytes < rwkv_wkv5s_saved_bytes(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     char* wsb = static_cast<char*>(workspace);
     const size_t n = round16(rwkv_wkv5_backward_workspace_bytes(B, T, C, H));
-    float* rdr = static_cast<float*>(workspace);
     uint16_t* pw = reinterpret_cast<uint16_t*>(wsb + n);                                  // per-batch gw, then per-batch gu
     uint16_t* pu = pw + static_cast<size_t>(B) * C;
     int* flg = reinterpret_cast<int*>(wsb + round16(rwkv_wkv5raw_backward_workspace_bytes(B, T, C, H)));
@@ -1454,10 +1457,8 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
                                           NB, TB, local, logdec, ds32, gu32, pw, gw32)) return e;
     } else if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, nullptr, pu, nullptr, static_cast<const char*>(saved), flg,
                                              1, 0, nullptr, nullptr, nullptr, nullptr, pw, nullptr)) return e;
-    // heads whose decay the mid-point factors cannot carry: the two sweeps redo them (their per-batch gw, gu rows included)
-    const float* ew = decay + C;
-    if (int e = launch_wkv6_bwd_a_chunk(st, W_HEAD, B, T, C, H, r, k, v, ew, u, nullptr, gy, gr, pu, rdr, flg)) return e;
-    if (int e = launch_wkv6_bwd_b_chunk(st, W_HEAD, B, T, C, H, r, k, v, ew, u, nullptr, gy, gk, gv, pw, nullptr, rdr, flg)) return e;
+    // a layer with a decay that the mid-point factors cannot carry
+    if (int e = launch_wkv5b_bwd(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved))) return e;
     hipLaunchKernelGGL(bf16_batch_sum, dim3((C + 255) / 256), dim3(256), 0, st, B, C, pw, gw, pu, gu);
     return launch_status();
 }

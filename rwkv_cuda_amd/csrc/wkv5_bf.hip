@@ -1,4 +1,4 @@
-// wkv5, bf16 I/O, whole heads of N = 128 channels in one workgroup: one forward and one reverse sweep in chunks of
+// wkv5, bf16 I/O, whole heads of N = 128 or 64 channels in one workgroup: one forward and one reverse sweep in chunks of
 // L = 32 tokens on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16), for decays of any strength.
 //
 // Step form (wkv5_bf16/cuda/wkv5_cuda.cu), one head, S[i][j] (i value channel, j key channel), o = e^l, l = -exp(w_raw):
@@ -17,13 +17,14 @@
 // Operands: fp32 values as hi + lo bf16 (16 mantissa bits), three products where both sides are fp32; r, k, v, gy are exact.
 //
 // Strong decays.  A factor reaches e^{|l| d}, d the distance of a token from its reference.  The forward has one reference in the
-// middle (its planes serve the state products too), up to |l| = 4.5.  The backward refers to the middle of the half that the
-// output's token lies in (m = 8, 24; a tile's quadrant across the halves to 16): d is 8 and |l| may reach 9, for one more
-// operand per tile.  Heads beyond that take a reference per 8 tokens (m = 4, 12, 20, 28); a pair of tokens d such blocks apart
+// middle (its planes serve the state products too), up to |l| = 4.5, and makes its tiles from raw rows beyond.  These, and the
+// backward always, refer to the middle of the half that the output's token lies in (m = 8, 24; a tile's quadrant across the halves
+// to 16): d is 8 and |l| may reach 9, for one more operand per tile.  Heads beyond that take a reference per 8 tokens (m = 4, 12, 20, 28); a pair of tokens d such blocks apart
 // then carries o^{8 d} in addition: a product per distance, half of the factor on either side (o^{8 d} may underflow where the
 // whole term is one).  Below l = -17 a decay is taken as e^{-17} = 4e-8.
 // Handing such heads to step-by-step kernels, as the kernels before did, made one strong channel in 4096 cost more than
-// everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 ms with.
+// everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 ms with.  That is why layers of 64-channel
+// heads come here as well once they have such a channel (0.74 ms at B8 T4096 C2048 where they took 1.66 ms).
 //
 // What bounds it (B8 T4096 C4096: one workgroup per CU).  Forward 0.52 ms for 2.1 GB, half of them the saved states: HBM (4.1 TB/s;
 // 0.82 ms as four heads of 64).  Backward 1.03 ms: the D waves, some 1600 vector and 170 matrix instructions a chunk, and their
@@ -37,7 +38,8 @@ namespace rwkv {
 namespace {
 
 constexpr int NTH = 512;             // waves 0..3 hold states, 4..7 load and prepare
-constexpr float LAM_STRONG_F = -4.5f, LAM_STRONG_B = -9.f, LAM_MIN = -17.f;
+constexpr float LAM_MID = -4.5f, LAM_HALF = -9.f, LAM_MIN = -17.f;      // strongest log decay for one reference, for one per half; taken at most
+enum { REF_MID, REF_HALF, REF_8 };
 constexpr f32x4 ZERO4 = {0.f, 0.f, 0.f, 0.f};
 
 struct ArgsW {
@@ -114,8 +116,8 @@ template <uint32_t ROW> DEVINL bf16x8 ld_tra(const lds_t a) {
 }
 DEVINL int slot_token(int g, int e) { return 16 * (e >> 2) + 4 * g + (e & 3); }
 
-// The head's parameters into LDS (by the first wave); every wave finds out for itself whether a decay is strong.
-template <int HN> DEVINL bool head_setup(const ArgsW& p, lds_t sb, int h, int b, int tid, float limit) {
+// The head's parameters into LDS (by the first wave); every wave finds out for itself what its strongest log decay is.
+template <int HN> DEVINL float head_setup(const ArgsW& p, lds_t sb, int h, int b, int tid) {
     const int lane = tid & 63;
     float mn = 0.f;
 #pragma unroll
@@ -131,7 +133,7 @@ template <int HN> DEVINL bool head_setup(const ArgsW& p, lds_t sb, int h, int b,
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o, 64));
-    return __builtin_amdgcn_readfirstlane(mn < limit ? 1 : 0) != 0;
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, mn)));
 }
 
 // Rows of a [token][channel] tensor from one token on, as a buffer: reads of rows that do not exist give zeros, stores to them are
@@ -281,8 +283,8 @@ DEVINL void apply(const Op2 (&a)[NA], const Op2& b, const bf16x8& x, const float
 // Waves 0..3 hold St[ct][jt][v] = S[j = 16 jt + 4 g + v][i = own], as it stands the B operand of a contraction over j.  Waves 4..7
 // load (two chunks ahead of the planes, the planes two chunks ahead of their use) and make the next chunk's tile in parts of 32
 // key channels.  One barrier a chunk.
-// Planes: R' = r o^{t-16}, K' = k o^{15-t} (they serve the tile, the state times o^16 on its way in and out of the update); strong:
-// r o^t, k o^{31-t}, and the tile is made from the raw rows.
+// Planes: R' = r o^{t-16}, K' = k o^{15-t} (they serve the tile, the state times o^16 on its way in and out of the update); strong
+// decays: r o^t, k o^{31-t}, and the tile is made from the raw rows (read once more, from L2).
 template <int HN, bool STRONG> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int q, int lane, size_t base, int nch) {
     using A = G<HN>;
     constexpr int CT = A::CT, KS = A::KS, NJ = A::NB16;
@@ -377,8 +379,9 @@ template <int HN, bool STRONG> DEVINL void fwd_states(const ArgsW& p, lds_t sb, 
     }
 }
 
-template <int HN, bool STRONG> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int tp, size_t base, int nch) {
+template <int HN, int REF> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int tp, size_t base, int nch) {
     using A = G<HN>;
+    constexpr bool RAW = REF != REF_MID, STRONG = REF == REF_8;       // the tile is made from raw rows
     constexpr int NP = A::PASSES;
     const int lane = tp & 63, q = tp >> 6, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
     const int row0 = tp / A::PIECES, c8 = (tp % A::PIECES) * 8;
@@ -390,12 +393,12 @@ template <int HN, bool STRONG> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, i
 #pragma unroll
         for (int z = 0; z < NP; ++z) {
             const int t = row0 + z * A::ROWS;
-            pr[z][e] = wpow(l, STRONG ? t : t - 16);
-            pk[z][e] = wpow(l, STRONG ? 31 - t : 15 - t);
+            pr[z][e] = wpow(l, RAW ? t : t - 16);
+            pk[z][e] = wpow(l, RAW ? 31 - t : 15 - t);
         }
     }
     [[maybe_unused]] TilePowers<STRONG> tpw;
-    if constexpr (STRONG) tile_powers(tpw, sb + A::LAM + 4 * (32 * (q % A::PARTS) + 8 * g), l16);
+    if constexpr (RAW) tile_powers(tpw, sb + A::LAM + 4 * (32 * (q % A::PARTS) + 8 * g), l16);
     uint4 x[2][3][NP];
     auto fetch = [&](const int c, uint4 (&d)[3][NP]) __attribute__((always_inline)) {
         const int cc = min(c, nch - 1);                  // (the same loads in every iteration)
@@ -430,7 +433,7 @@ template <int HN, bool STRONG> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, i
         if (q >= A::PARTS) return;
         f32x4 qd[3];
         const lds_t s = sb + A::BASE + sl * A::FSLOT;
-        if constexpr (STRONG) {
+        if constexpr (RAW) {
             const size_t co = base + static_cast<size_t>(c) * L * C;
             const rows_t rr = rows_of(p.r + co, T - c * L, C), kk = rows_of(p.k + co, T - c * L, C);
             bf16x8 r[2], k[2];
@@ -439,7 +442,7 @@ template <int HN, bool STRONG> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, i
                 const int o = 2 * ((16 * z + l16) * C + 32 * q + 8 * g);
                 r[z] = op4(load16(rr, o)); k[z] = op4(load16(kk, o));
             }
-            raw_part<true, true>(r, k, tpw, lane, qd);
+            raw_part<true, STRONG>(r, k, tpw, lane, qd);
         } else {
             Op2 xo[2], yo[2];
 #pragma unroll
@@ -481,14 +484,16 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_fwd(const ArgsW p) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = (p.T + L - 1) / L;
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
-    const bool strong = head_setup<HN>(p, sb, h, b, tid, LAM_STRONG_F);
+    if (HN == 64 && !strong_layer(p.w, p.C, tid & 63)) return;      // the one-sweep kernels of wkv6 have done this layer
+    const float lmin = head_setup<HN>(p, sb, h, b, tid);
     __syncthreads();
     if (w < 4) {
-        if (strong) fwd_states<HN, true>(p, sb, w, tid & 63, base, nch);
+        if (lmin < LAM_MID) fwd_states<HN, true>(p, sb, w, tid & 63, base, nch);
         else fwd_states<HN, false>(p, sb, w, tid & 63, base, nch);
     } else {
-        if (strong) fwd_loads<HN, true>(p, sb, tid - 256, base, nch);
-        else fwd_loads<HN, false>(p, sb, tid - 256, base, nch);
+        if (lmin < LAM_HALF) fwd_loads<HN, REF_8>(p, sb, tid - 256, base, nch);
+        else if (lmin < LAM_MID) fwd_loads<HN, REF_HALF>(p, sb, tid - 256, base, nch);
+        else fwd_loads<HN, REF_MID>(p, sb, tid - 256, base, nch);
     }
 }
 
@@ -558,7 +563,7 @@ template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int 
         o[0] = o[1] = split8(fx);
         if constexpr (!STRONG) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ff[e] = (sinks ? fx[4 + e] : fx[e]) * o16[ct];
+            for (int e = 0; e < 4; ++e) ff[e] = (sinks ? fx[4 + e] : fx[e]) * o8[ct] * o8[ct];      // (o^16 may underflow where this does not)
             const HL a = hilo2k(ff[0], ff[1]), b = hilo2k(ff[2], ff[3]);
             Op2& w = o[sinks ? 0 : 1];
             const uint4 h = __builtin_bit_cast(uint4, w.h), lo = __builtin_bit_cast(uint4, w.l);
@@ -857,7 +862,8 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_bwd(const ArgsW p) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = 2 * ((p.T + 2 * L - 1) / (2 * L));      // whole pairs (a last chunk without tokens adds zeros)
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
-    const bool strong = head_setup<HN>(p, sb, h, b, tid, LAM_STRONG_B);
+    if (HN == 64 && !strong_layer(p.w, p.C, tid & 63)) return;
+    const bool strong = head_setup<HN>(p, sb, h, b, tid) < LAM_HALF;
     __syncthreads();
     if (w < 4) {
         if (strong) role_d<HN, true>(p, sb, w, tid & 63, h, b, base, nch);
@@ -887,14 +893,14 @@ int launch_wkv5b_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t*
                      const uint16_t* u, uint16_t* y, float* decay, float* saved) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.decay = decay; p.saved = saved;
-    return launch(wkv5b_fwd<128>, st, B, p, G<128>::FTOTAL);
+    return C == H * 64 ? launch(wkv5b_fwd<64>, st, B, p, G<64>::FTOTAL) : launch(wkv5b_fwd<128>, st, B, p, G<128>::FTOTAL);
 }
 int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
                      const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu, const float* saved) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv; p.gw = gw; p.gu = gu;
     p.saved = const_cast<float*>(saved);
-    return launch(wkv5b_bwd<128>, st, B, p, G<128>::BTOTAL);
+    return C == H * 64 ? launch(wkv5b_bwd<64>, st, B, p, G<64>::BTOTAL) : launch(wkv5b_bwd<128>, st, B, p, G<128>::BTOTAL);
 }
 
 }  // namespace rwkv

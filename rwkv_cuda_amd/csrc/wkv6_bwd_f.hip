@@ -840,6 +840,13 @@ __global__ __launch_bounds__(NTG) void wkv6_bwd_fused(const ArgsG arg) {
     const int t0 = blk * arg.TB;
     const size_t base = (static_cast<size_t>(b) * arg.T + t0) * arg.C + static_cast<size_t>(h) * N;
     const size_t bh = bhx, bq = bh * arg.NB + blk;
+    if constexpr (WMODE == W_HEAD) {
+        const uint16_t* w = static_cast<const uint16_t*>(arg.w);
+        if (strong_layer(w, arg.C, tid & 63)) {
+            if (tid < 64 && blk == 0) flag_strong_head(arg.flags, bh, w, h, tid);
+            return;
+        }
+    }
     ArgsG a = arg;
     a.T = arg.T - t0 < arg.TB ? arg.T - t0 : arg.TB;
     const int nsegs = ((arg.T + L - 1) / L + 1) / 2;                // saved states of a whole sequence

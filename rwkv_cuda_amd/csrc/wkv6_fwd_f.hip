@@ -516,6 +516,12 @@ __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
     const int t0 = blk * arg.TB;
     const size_t base = (static_cast<size_t>(b) * arg.T + t0) * arg.C + static_cast<size_t>(h) * N;
     const size_t bh = bhx, bq = bh * arg.NB + blk;
+    if constexpr (HD) {
+        if (strong_layer(arg.w, arg.C, tid & 63)) {
+            if (tid < 64 && blk == 0) flag_strong_head(arg.flags, bh, arg.w, h, tid);
+            return;
+        }
+    }
     ArgsQ a = arg;
     a.T = arg.T - t0 < arg.TB ? arg.T - t0 : arg.TB;
     const int nseg = ((arg.T + L - 1) / L + 1) / 2;                 // saved states of a whole sequence

@@ -56,3 +56,33 @@ def test_one_strong_head_among_others_changes_nothing_else(lib):
     for x, y in zip(a[:4], b[:4]):
         x, y = x.view(B, T, H, N), y.view(B, T, H, N)
         assert torch.equal(x[:, :, 0], y[:, :, 0]) and torch.equal(x[:, :, 2], y[:, :, 2]) and not torch.equal(x[:, :, 1], y[:, :, 1])
+
+
+@pytest.mark.parametrize("decays", ["mixed", "strong"])
+@pytest.mark.parametrize("T", [1, 31, 33, 64, 97, 260])
+def test_wkv5_head_size_64_with_a_strong_decay(lib, T, decays):
+    """Head size 64 belongs to the one-sweep kernels until one channel of the layer decays too fast for them."""
+    B, H = 2, 3
+    C = H * 64
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=1200 + T)
+    w = _decays(decays, w)
+    print(f"\nwkv5 N=64 T={T} {decays}", flush=True)
+    ref = O.wkv5_grads(B, T, C, H, r, k, v, w, u, gy)
+    emu = O.emulate_wkv5_bf16(B, T, C, H, r, k, v, w, u, gy)
+    for name, a, e, g in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, _run(B, T, C, H, r, k, v, w, u, gy)):
+        assert_no_worse(name, a, e.reshape(a.shape), g.reshape(a.shape))
+
+
+@pytest.mark.parametrize("w1", [1.3125, 1.3203125, 1.5, 2.1875, 2.203125, 2.84375])
+@pytest.mark.parametrize("head", [64, 128])
+def test_wkv5_around_the_thresholds(lib, head, w1):
+    """One channel at the decays where the kernels (one-sweep or whole heads), or the reference tokens, change."""
+    B, T, H = 1, 70, 2
+    C = H * head
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=77)
+    w = w.clamp(max=1.25)
+    w.view(-1)[head + 9] = w1
+    ref = O.wkv5_grads(B, T, C, H, r, k, v, w, u, gy)
+    emu = O.emulate_wkv5_bf16(B, T, C, H, r, k, v, w, u, gy)
+    for name, a, e, g in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, _run(B, T, C, H, r, k, v, w, u, gy)):
+        assert_no_worse(name, a, e.reshape(a.shape), g.reshape(a.shape))
