@@ -436,6 +436,14 @@ int rwkv7_statepassing_backward_ex(void* stream, int B, int T, int H,
                                    rwkv_bf16* dr, rwkv_bf16* dw, rwkv_bf16* dk, rwkv_bf16* dv,
                                    rwkv_bf16* da, rwkv_bf16* db, unsigned flags);
 
+/* A forward that no backward follows, of all three ops in both modes: as rwkv7_statepassing_forward_ex without flags, but
+ * nothing is kept in `s` and `sa`.  fp32: 0 for bf16 r..b and y, 1 for
+ * fp32; s0 and sT may be NULL (zero initial state; not written).  y and sT are bit for bit those of the other entry points.
+ * No counterpart in the reference, whose forward always keeps both (rwkv7_statepassing_clampw.cu:67-73). */
+int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float* s0,
+                       const void* r, const void* w, const void* k, const void* v, const void* a, const void* b,
+                       void* y, float* sT);
+
 /* The two siblings of the state-passing op, served by the same kernels:
  *   rwkv7_state_*  : initial state s0 and its gradient ds0, no final state.  Replaces cuda_forward /
  *                    cuda_backward of rwkv7_fast_fused/cuda/rwkv7_state_clampw.cpp:10,17.

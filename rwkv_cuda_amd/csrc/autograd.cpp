@@ -376,7 +376,7 @@ Tensor wkv6_state_op(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& r
 // whose layout belongs to the library.  The backward must run with the flags of the forward (the kernel families lay `s` out
 // differently), so they ride on the context.
 variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a,
-                        const Tensor& b, int64_t flags, bool passing, bool flat) {
+                        const Tensor& b, int64_t flags, bool passing, bool flat, bool grad) {
     const auto dt = r.scalar_type();
     require(dt == BF || dt == F32, "r.dtype must be bfloat16 or float32, got " + str(dt));
     require(r.dim() == 3 || r.dim() == 4, "r..b are [B,T,H,64] or [B,T,H*64]");
@@ -394,8 +394,14 @@ variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r,
     const auto f32 = r.options().dtype(F32);
     Tensor y = flat ? at::empty({B, T, H * HEAD}, r.options()) : at::empty({B, T, H, HEAD}, r.options());
     Tensor sT = passing ? at::empty({B, H, HEAD, HEAD}, f32) : Tensor();
-    Tensor s = at::empty({B, H, T / CHUNK7, HEAD, HEAD}, f32), sa = at::empty({B, T, H, HEAD}, f32);
     void* st = stream_of(r);
+    if (!grad && (dt != BF || !(flags & RWKV_FLAG_SWEEPS))) {
+        // no backward can follow: nothing is kept for one
+        ok(rwkv7_forward_only(st, b_, t_, h_, dt == F32, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT)), true);
+        if (passing) return {y, sT};
+        return {y};
+    }
+    Tensor s = at::empty({B, H, T / CHUNK7, HEAD, HEAD}, f32), sa = at::empty({B, T, H, HEAD}, f32);
     if (dt == BF)
         ok(rwkv7_statepassing_forward_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)), true);
     else if (passing) ok(rwkv7_statepassing_forward_f32(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa)), true);
@@ -430,32 +436,33 @@ variable_list rwkv7_grads(AutogradContext* ctx, const Tensor& dy_, const Tensor&
 }
 struct Rwkv7Passing : Function<Rwkv7Passing> {
     static variable_list forward(AutogradContext* ctx, const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a,
-                                 const Tensor& b, int64_t flags, bool) { return rwkv7_run(ctx, s0, r, w, k, v, a, b, flags, true, true); }
+                                 const Tensor& b, int64_t flags, bool grad) { return rwkv7_run(ctx, s0, r, w, k, v, a, b, flags, true, true, grad); }
     static variable_list backward(AutogradContext* ctx, variable_list g) { return rwkv7_grads(ctx, g[0], g[1], true); }
 };
 struct Rwkv7State : Function<Rwkv7State> {
     static variable_list forward(AutogradContext* ctx, const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a,
-                                 const Tensor& b, int64_t flags, bool flat) { return rwkv7_run(ctx, s0, r, w, k, v, a, b, flags, false, flat); }
-    static variable_list backward(AutogradContext* ctx, variable_list g) { return rwkv7_grads(ctx, g[0], NONE, true); }
+                                 const Tensor& b, int64_t flags, bool flat, bool grad) { return rwkv7_run(ctx, s0, r, w, k, v, a, b, flags, false, flat, grad); }
+    static variable_list backward(AutogradContext* ctx, variable_list g) { variable_list x = rwkv7_grads(ctx, g[0], NONE, true); x.push_back(NONE); return x; }
 };
 struct Rwkv7 : Function<Rwkv7> {
     static variable_list forward(AutogradContext* ctx, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b,
-                                 int64_t flags, bool flat) { return rwkv7_run(ctx, NONE, r, w, k, v, a, b, flags, false, flat); }
+                                 int64_t flags, bool flat, bool grad) { return rwkv7_run(ctx, NONE, r, w, k, v, a, b, flags, false, flat, grad); }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
         variable_list x = rwkv7_grads(ctx, g[0], NONE, false);
         x.erase(x.begin());
+        x.push_back(NONE);
         return x;
     }
 };
 std::tuple<Tensor, Tensor> rwkv7_passing_op(const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b, int64_t flags) {
-    variable_list o = Rwkv7Passing::apply(s0, r, w, k, v, a, b, flags, true);
+    variable_list o = Rwkv7Passing::apply(s0, r, w, k, v, a, b, flags, wants_grad({&s0, &r, &w, &k, &v, &a, &b}));
     return {o[0], o[1]};
 }
 Tensor rwkv7_state_op(const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b, int64_t flags, bool flat) {
-    return Rwkv7State::apply(s0, r, w, k, v, a, b, flags, flat)[0];
+    return Rwkv7State::apply(s0, r, w, k, v, a, b, flags, flat, wants_grad({&s0, &r, &w, &k, &v, &a, &b}))[0];
 }
 Tensor rwkv7_op(const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b, int64_t flags, bool flat) {
-    return Rwkv7::apply(r, w, k, v, a, b, flags, flat)[0];
+    return Rwkv7::apply(r, w, k, v, a, b, flags, flat, wants_grad({&r, &w, &k, &v, &a, &b}))[0];
 }
 
 }  // namespace

@@ -436,6 +436,15 @@ int rwkv7_statepassing_backward_ex(void* stream, int B, int T, int H, const rwkv
     return bf16_bwd(stream, flags, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
+// A forward that no backward follows: the chunked kernels without their stores of `s` and `sa`.
+int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float* s0, const void* r, const void* w, const void* k,
+                       const void* v, const void* a, const void* b, void* y, float* sT) {
+    if (int e = check7(B, T, H)) return e;
+    if (int e = check_ptrs({r, w, k, v, a, b, y})) return e;
+    if (!aligned16(s0) || !aligned16(sT)) return RWKV_ERR_ALIGN;
+    return launch7c_fwd(static_cast<hipStream_t>(stream), fp32 != 0, B, T, H, s0, r, w, k, v, a, b, y, sT, nullptr, nullptr);
+}
+
 // ---- fp32 I/O: what the reference builds from the same sources with -D_FP32_ (rwkv7_cuda_benchmark.py:102-126 and the
 // same lines of its _state and _state_passing siblings).  The chunked kernels, whose arithmetic is fp32 in either mode: only
 // loads and stores differ.

@@ -174,7 +174,12 @@ struct SmemCF {
     float d1[N], dec[N];
 };
 
-template <bool F32>
+// KEEP: `s` and `sa` are written for a backward, 20 bytes per element beside the 14 of a bf16 forward's inputs and output.  Without
+// (no backward can follow) B8 T1024 C4096 takes 353 us instead of 383, and none of the 672 MB; one chunk of 32 heads, the call
+// included, 7.9 instead of 9.4.  The rest is the fp32 matrix pipe plus the vector instructions, which hardly overlap with it: the
+// state's products moved ahead of the barrier behind the inverse, or the waits for stores taken out of the loop, did not make it
+// faster (384 and 394 us).
+template <bool F32, bool KEEP>
 __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
     __shared__ SmemCF S;
     const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
@@ -230,7 +235,7 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
         }
         if (q == 0) { S.d1[lane] = exp_acc(cm); S.dec[lane] = exp_acc(cl); }
         // the state entering the chunk, for the backward
-        {
+        if constexpr (KEEP) {
             float* slot = p.s + (bh * nch + c) * N * N + static_cast<size_t>(i_own) * N + 4 * g;
 #pragma unroll
             for (int jt = 0; jt < 4; ++jt) st4(slot + 16 * jt, St[jt]);
@@ -310,7 +315,10 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
             for (int v = 0; v < 4; ++v) Y = mm(rk[v], vop[v], Y);
         }
 #pragma unroll
-        for (int v = 0; v < 4; ++v) { S.Yo[4 * g + v][i_own] = Y[v]; S.Uo[4 * g + v][i_own] = U[v]; }
+        for (int v = 0; v < 4; ++v) {
+            S.Yo[4 * g + v][i_own] = Y[v];
+            if constexpr (KEEP) S.Uo[4 * g + v][i_own] = U[v];
+        }
         // ---------------------------------------------------------------- S^T = diag(dec) S^T + (B' d2)^T U + (K' d2)^T V
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
@@ -329,7 +337,7 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
             const f32x4 y = ld4(&S.Yo[t][i4]);
             if constexpr (F32) st4(reinterpret_cast<float*>(p.y) + o, y);
             else *reinterpret_cast<uint2*>(p.y + o) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
-            st4(p.sa + o, ld4(&S.Uo[t][i4]));
+            if constexpr (KEEP) st4(p.sa + o, ld4(&S.Uo[t][i4]));
         }
     }
     if (p.sT != nullptr) {
@@ -786,8 +794,8 @@ int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0,
     Args7c p{};
     p.T = T; p.H = H; p.s0 = s0; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b); p.y = el(y);
     p.sT = sT; p.s = s; p.sa = sa;
-    if (f32) hipLaunchKernelGGL(rwkv7c_fwd<true>, dim3(H, B), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(rwkv7c_fwd<false>, dim3(H, B), dim3(NT), 0, st, p);
+    const auto kernel = s != nullptr ? (f32 ? rwkv7c_fwd<true, true> : rwkv7c_fwd<false, true>) : (f32 ? rwkv7c_fwd<true, false> : rwkv7c_fwd<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(H, B), dim3(NT), 0, st, p);
     return launch_status();
 }
 

@@ -200,3 +200,24 @@ def test_rwkv7_backward_uses_the_kernel_family_of_its_forward(lib):
     got = [y.detach().view(B, T, H, 64), S.detach()] + [x.grad for x in t]
     for name, a_, e, g in zip(NAMES, ref, emu, got):
         assert_no_worse("sweeps forward, backward after the block: " + name, a_, e, g)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,H", [(1, 16, 1), (2, 48, 3), (3, 160, 2)])
+def test_rwkv7_forward_without_gradients_is_bit_identical(lib, B, T, H, dtype):
+    """Where no backward can follow the kernels keep no states: the same outputs, bit for bit, for all three siblings, at one,
+    an odd and an even number of chunks."""
+    print(f"\nrwkv7 forward only B={B} T={T} H={H} {dtype}", flush=True)
+    s0, r, w, k, v, a, b, _, _ = synth.rwkv7_inputs(B, T, H, 64, seed=37)
+    s0 = s0.to(DEV)
+    x = [t.to(DEV, dtype).view(B, T, H * 64) for t in (r, w, k, v, a, b)]
+    xg = [t.clone().requires_grad_(True) for t in x]
+    y, sT = R.RWKV7_STATE_PASSING_CLAMPW_CUDA(s0, *xg)
+    assert y.requires_grad and sT.requires_grad
+    want = [y, sT, R.RWKV7_STATE_CLAMPW_CUDA(s0, *xg), R.RWKV7_CLAMPW_CUDA(*xg)]
+    for args in (x, xg):                                  # nothing asks for a gradient; gradients are off
+        with torch.set_grad_enabled(args is x):
+            got = [*R.RWKV7_STATE_PASSING_CLAMPW_CUDA(s0, *args), R.RWKV7_STATE_CLAMPW_CUDA(s0, *args), R.RWKV7_CLAMPW_CUDA(*args)]
+        for g, e in zip(got, want):
+            assert not g.requires_grad and torch.equal(g, e.detach())
+    torch.cuda.synchronize()
