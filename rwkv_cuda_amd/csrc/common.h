@@ -115,6 +115,24 @@ DEVINL void allreduce2_rows(float& x, float& y) {
     x = u; y = w;                                 // [X, X, X, X], [Y, Y, Y, Y]
 }
 
+// ----------------------------------------------------------------------------- wkv5: decays that are too fast for chunks
+// wkv5's chunked kernels carry powers e^{l d} of a channel's log decay l = -exp(w) over a few tokens, in both directions.  A head
+// with one channel beyond what they carry (fp32 wkv5c_*: l < -17, where the powers of half a chunk still stay inside fp32) runs
+// step by step instead (wkv5_steps_*, wkv56.hip).  A decay that is no number counts as one of these: the steps hand it on
+// as the operator does.  Chunked and step kernels decide by the same test, for the channels of the head from c0 on.
+constexpr float W_STEPS_F32 = 2.8332133f;      // ln 17
+template <bool F32, int HN> DEVINL bool steps_head(const void* w, const void* w2, const int c0) {
+    bool on = false;
+#pragma unroll
+    for (int z = 0; z < HN / 64; ++z) {
+        const int c = c0 + 64 * z + (threadIdx.x & 63);
+        static_assert(F32, "fp32");
+        on |= !(static_cast<const float*>(w)[c] <= W_STEPS_F32);
+        if (w2 != nullptr) on |= !(static_cast<const float*>(w2)[c] <= W_STEPS_F32);
+    }
+    return __ballot(on) != 0ull;
+}
+
 // ----------------------------------------------------------------------------- host checks
 extern thread_local int g_last_hip_error;
 
@@ -176,6 +194,14 @@ int launch_wkv5_bwd_a_split(hipStream_t st, int cross, int B, int T, int C, int 
 int launch_wkv5_bwd_b_split(hipStream_t st, int cross, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k,
                             const uint16_t* v, const float* ew, const uint16_t* u, const uint16_t* gy, float* gk32, float* gv32,
                             float* gw32, const float* rdr);
+// wkv56.hip: the heads of an fp32 wkv5 (wkv5a: w2, u2 not null) layer of 64-channel heads that the chunked kernels leave out; gw, gu,
+// gw2, gu2: per-batch rows [B][C]
+int launch_wkv5f32_steps_fwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
+                             const float* u, const float* w2, const float* u2, float* y);
+int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
+                             const float* u, const float* w2, const float* u2, const float* gy, float* gr, float* gk, float* gv,
+                             float* gw, float* gu, float* gw2, float* gu2);
+
 // wkv5_bf.hip: wkv5, bf16, heads of 128 or 64 channels, whole heads, decays of any strength; w raw.  Size 64: only layers with a
 // strong decay (strong_layer, wkv6_fused.h), the others belong to the one-sweep kernels above and the launch returns at once.  saved (may be null in the forward):
 // the states for the backward; gw, gu: per-batch rows [B][C].

@@ -514,6 +514,7 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
 // each, so every sum of the recurrence is a private loop over LDS-broadcast vectors plus one or two cross-lane adds.
 // Same passes, formulas, rounding points and workspace as the sweeps above; hn (the head size, 1..NP) is a run-time
 // value, NP the padded size the registers are unrolled for.
+// STEPS (wkv5 only): w (w2) are the raw decays and GR carries Q in either precision, so that no pass needs another's workspace.
 constexpr int GTC = 16;          // time steps per staged chunk
 
 // The step loops below are unrolled over a thread's part of a state row.  Left alone, the compiler issues all of the LDS
@@ -534,12 +535,13 @@ template <int NP, int PARTS> struct RowGeom {
 };
 
 // staged vectors of one chunk; the ones a pass does not use shrink to one row
-template <int NP, int PARTS, int PASS, bool F32, bool TWO> struct SmemRows {
+template <int NP, int PARTS, int PASS, bool F32, bool TWO, bool STEPS = false> struct SmemRows {
     static constexpr int LEN = RowGeom<NP, PARTS>::LEN;
-    static constexpr bool kF = (PASS == P_GK && !F32) || (TWO && PASS == P_GR);     // gw factor, or w2[i] gy[i]
+    static constexpr bool kScan = PASS == P_GK && !F32 && !STEPS;
+    static constexpr bool kF = kScan || (TWO && PASS == P_GR);                      // gw factor, or w2[i] gy[i]
     alignas(16) float r[GTC][LEN], k[GTC][LEN], w[GTC][LEN];
     alignas(16) float v[PASS != P_GV ? GTC : 1][LEN], g[PASS != P_FWD ? GTC : 1][LEN];
-    alignas(16) float f[kF ? GTC : 1][LEN], rdr[(PASS == P_GK && !F32) ? GTC : 1][LEN];
+    alignas(16) float f[kF ? GTC : 1][LEN], rdr[kScan ? GTC : 1][LEN];
     float dot[GTC], dot2[TWO ? GTC : 1], dot3[TWO ? GTC : 1];
     alignas(16) float u[LEN], u2[TWO ? LEN : 4], w2[TWO ? LEN : 4];
 };
@@ -553,17 +555,22 @@ template <int PARTS> DEVINL float parts_sum(float x) {
     return x;
 }
 
-template <int NP, int PARTS, int PASS, int WMODE, bool F32, bool TWO = false>
-__global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const Args a, const int hn) {
+template <int NP, int PARTS, int PASS, int WMODE, bool F32, bool TWO, bool STEPS>
+DEVINL void rows_body(SmemRows<NP, PARTS, PASS, F32, TWO, STEPS>& S, const Args& a, const int hn) {
     static_assert(!F32 || WMODE == W_HEAD, "fp32 I/O exists for wkv5 only");
+    static_assert(!STEPS || WMODE == W_HEAD, "raw decays per channel");
     static_assert(!TWO || F32, "the two-sided op is fp32 only");
     using G = RowGeom<NP, PARTS>;
     constexpr int EL = G::EL, SLOT = G::SLOT;
     constexpr bool REV = (PASS == P_GK || PASS == P_GV);
     constexpr bool ROW_I = (PASS == P_FWD || PASS == P_GV);     // row = value channel, registers = key channels
-    constexpr bool DIRECT_GW = F32 && PASS == P_GR;             // as in wkv_sweep: the fp32 op carries Q = dS/dw
-    constexpr bool SCAN_GW = !F32 && PASS == P_GK;
-    __shared__ SmemRows<NP, PARTS, PASS, F32, TWO> S;
+    constexpr bool DIRECT_GW = (F32 || STEPS) && PASS == P_GR;  // as in wkv_sweep: the fp32 op carries Q = dS/dw
+    constexpr bool SCAN_GW = SmemRows<NP, PARTS, PASS, F32, TWO, STEPS>::kScan;
+    // the log decay and the decay of a channel of this layer
+    auto log_decay = [](const float* ew, const void* raw, int c) { return STEPS ? -expf(load1<F32>(static_cast<const uint16_t*>(raw), c)) : ew[c]; };
+    auto decay = [](const void* w, int c) { return STEPS ? expf(-expf(load1<F32>(static_cast<const uint16_t*>(w), c))) : static_cast<const float*>(w)[c]; };
+    // d decay / d raw = decay x log decay, zero where the decay is (the log decay may have left fp32's range there)
+    auto decay_grad = [](float lw, float w) { return STEPS && w == 0.f ? 0.f : lw * w; };
 
     const int tid = threadIdx.x;
     const int row = tid / PARTS, part = tid % PARTS;            // threads beyond NP * PARTS (NP * PARTS < 64) only idle
@@ -589,11 +596,14 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
         S.u[cat] = chan ? load1<F32>(a.u, h * hn + cn) : 0.f;
         if constexpr (TWO) {
             S.u2[cat] = chan ? load1<F32>(a.u2, h * hn + cn) : 0.f;
-            S.w2[cat] = chan ? a.w2[h * hn + cn] : 1.f;
+            S.w2[cat] = chan ? decay(a.w2, h * hn + cn) : 1.f;
         }
     }
-    const float w_chan = (WMODE == W_HEAD && chan) ? static_cast<const float*>(a.w)[h * hn + cn] : 1.f;     // stager's channel
-    const float w_row = (WMODE == W_HEAD && live) ? static_cast<const float*>(a.w)[h * hn + row] : 1.f;     // this row's channel
+    float w_chan = 1.f, w_row = 1.f;                            // stager's channel, this row's channel
+    if constexpr (WMODE == W_HEAD) {
+        if (chan) w_chan = decay(a.w, h * hn + cn);
+        if (live) w_row = decay(a.w, h * hn + row);
+    }
     float St[EL], Q[DIRECT_GW ? EL : 1];
 #pragma unroll
     for (int e = 0; e < EL; ++e) St[e] = 0.f;
@@ -605,7 +615,7 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
     float u2_row = 0.f, w2_row = 1.f, gu2_acc = 0.f;
     if constexpr (TWO) {
         u2_row = live ? load1<F32>(a.u2, h * hn + row) : 0.f;
-        w2_row = live ? a.w2[h * hn + row] : 1.f;
+        w2_row = live ? decay(a.w2, h * hn + row) : 1.f;
 #pragma unroll
         for (int e = 0; e < (GW2 ? EL : 1); ++e) A[e] = 0.f;
     }
@@ -739,7 +749,7 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
                     if constexpr (DIRECT_GW) gw_acc = fmaf(rr, acc2, gw_acc);
                     if (ok) {
                         store1<F32>(a.gr, off, TWO ? fmaf(kk, fmaf(uu, dot, S.dot2[t]), acc) : fmaf(uu * kk, dot, acc));
-                        if constexpr (!F32) a.rdr[off] = rr * acc;
+                        if constexpr (!F32 && !STEPS) a.rdr[off] = rr * acc;
                     }
                 } else {
                     if (ok) store1<F32>(a.gk, off, TWO ? fmaf(rr, fmaf(uu, dot, S.dot2[t]), acc) : fmaf(uu * rr, dot, acc));
@@ -759,7 +769,7 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
     if constexpr (PASS == P_GR) {
         if (writer) {
             store1<F32>(a.gu, pc, gu_acc);
-            if constexpr (DIRECT_GW) store1<F32>(a.gw, pc, a.ew_head[h * hn + row] * w_row * gw_acc);     // d eew / d w_raw = eew * ew
+            if constexpr (DIRECT_GW) store1<F32>(a.gw, pc, decay_grad(log_decay(a.ew_head, a.w, h * hn + row), w_row) * gw_acc);     // d eew / d w_raw = eew * ew
         }
         if constexpr (GW2) {
             // gu2: the staging groups' partial sums, one row of LDS per group
@@ -784,7 +794,7 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
                     for (int q = 0; q < (NP < GTC ? NP : GTC); ++q) tot += S.k[q][cat];
             }
             if (tid < NP && chan)
-                store1<F32>(a.gw2, static_cast<size_t>(b) * a.C + static_cast<size_t>(h) * hn + cn, a.ew2_head[h * hn + cn] * a.w2[h * hn + cn] * tot);
+                store1<F32>(a.gw2, static_cast<size_t>(b) * a.C + static_cast<size_t>(h) * hn + cn, decay_grad(log_decay(a.ew2_head, a.w2, h * hn + cn), decay(a.w2, h * hn + cn)) * tot);
         }
     }
     if constexpr (PASS == P_GK) {
@@ -799,6 +809,33 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
             for (int e = 0; e < EL; ++e) if (o0 + e < hn) a.gs[(bh * hn + o0 + e) * hn + row] = f2bf(St[e]);
         }
     }
+}
+
+template <int NP, int PARTS, int PASS, int WMODE, bool F32, bool TWO = false>
+__global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const Args a, const int hn) {
+    __shared__ SmemRows<NP, PARTS, PASS, F32, TWO> S;
+    rows_body<NP, PARTS, PASS, WMODE, F32, TWO, false>(S, a, hn);
+}
+
+// The heads of a wkv5 layer whose decay the chunked kernels do not carry (steps_head, common.h), step by step; all other
+// workgroups return at once.  Backward: the three passes, which need nothing of each other, side by side.
+template <int NP, int PARTS, bool F32, bool TWO>
+__global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_fwd(const Args a, const int hn) {
+    if (!steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP)) return;
+    __shared__ SmemRows<NP, PARTS, P_FWD, F32, TWO, true> S;
+    rows_body<NP, PARTS, P_FWD, W_HEAD, F32, TWO, true>(S, a, hn);
+}
+template <int NP, int PARTS, bool F32, bool TWO>
+__global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_bwd(const Args a, const int hn) {
+    if (!steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP)) return;
+    __shared__ union {
+        SmemRows<NP, PARTS, P_GR, F32, TWO, true> gr;
+        SmemRows<NP, PARTS, P_GV, F32, TWO, true> gv;
+        SmemRows<NP, PARTS, P_GK, F32, TWO, true> gk;
+    } S;
+    if (blockIdx.y == 0) rows_body<NP, PARTS, P_GR, W_HEAD, F32, TWO, true>(S.gr, a, hn);
+    else if (blockIdx.y == 1) rows_body<NP, PARTS, P_GV, W_HEAD, F32, TWO, true>(S.gv, a, hn);
+    else rows_body<NP, PARTS, P_GK, W_HEAD, F32, TWO, true>(S.gk, a, hn);
 }
 
 constexpr int MAX_HEAD = 128;
@@ -969,7 +1006,32 @@ int launch_bwd_split(hipStream_t st, int B, int T, int C, int H, const uint16_t*
     return launch_status();
 }
 
+const uint16_t* as_elems(const float* p) { return reinterpret_cast<const uint16_t*>(p); }
+uint16_t* out_elems(float* p) { return reinterpret_cast<uint16_t*>(p); }
+
 }  // namespace
+
+int launch_wkv5f32_steps_fwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
+                             const float* u, const float* w2, const float* u2, float* y) {
+    Args a{};
+    a.T = T; a.C = H * N; a.H = H; a.r = as_elems(r); a.k = as_elems(k); a.v = as_elems(v); a.w = w; a.u = as_elems(u); a.w2 = w2;
+    a.u2 = as_elems(u2); a.y = out_elems(y);
+    const auto kernel = w2 != nullptr ? wkv5_steps_fwd<64, 4, true, true> : wkv5_steps_fwd<64, 4, true, false>;
+    hipLaunchKernelGGL(kernel, dim3(B * H), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    return launch_status();
+}
+int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
+                             const float* u, const float* w2, const float* u2, const float* gy, float* gr, float* gk, float* gv,
+                             float* gw, float* gu, float* gw2, float* gu2) {
+    Args a{};
+    a.T = T; a.C = H * N; a.H = H; a.r = as_elems(r); a.k = as_elems(k); a.v = as_elems(v); a.w = w; a.u = as_elems(u); a.w2 = w2;
+    a.u2 = as_elems(u2); a.gy = as_elems(gy); a.gr = out_elems(gr); a.gk = out_elems(gk); a.gv = out_elems(gv); a.gw = out_elems(gw);
+    a.gu = out_elems(gu); a.gw2 = out_elems(gw2); a.gu2 = out_elems(gu2);
+    const auto kernel = w2 != nullptr ? wkv5_steps_bwd<64, 4, true, true> : wkv5_steps_bwd<64, 4, true, false>;
+    hipLaunchKernelGGL(kernel, dim3(B * H, 3), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    return launch_status();
+}
+
 }  // namespace rwkv
 
 using namespace rwkv;
@@ -1021,11 +1083,7 @@ int rwkv_wkv5_backward_ex(void* stream, int B, int T, int C, int H, const rwkv_b
     return launch_bwd<W_HEAD>(static_cast<hipStream_t>(stream), B, a, flags);
 }
 
-// ---- wkv5, fp32 I/O: the sequential fp32 sweeps only (the chunked kernels work to bf16-I/O accuracy)
-namespace {
-const uint16_t* as_elems(const float* p) { return reinterpret_cast<const uint16_t*>(p); }
-uint16_t* out_elems(float* p) { return reinterpret_cast<uint16_t*>(p); }
-}  // namespace
+// ---- wkv5, fp32 I/O, behind the reference's own signature: the sequential fp32 sweeps
 
 int rwkv_wkv5f32_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v,
                          const float* eew, const float* u, float* y) {

@@ -23,7 +23,8 @@
 //
 // Strong decays: with one reference in the middle a factor reaches e^{8 |l|}; beyond l = -7 (LAM_STRONG) the tiles take a
 // reference in the middle of each half (m = 4, 12) and a pair of tokens of different halves carries o1^8 in addition: a second
-// product for that quadrant, with o1^4 on either side (o1^8 itself may underflow where the whole term is one).  Below l = -17 a decay is taken as e^{-17} = 4e-8, half a unit of the fp32 sum it enters.
+// product for that quadrant, with o1^4 on either side (o1^8 itself may underflow where the whole term is one).  Heads with a
+// channel below l = -17, or one that is no number, are left to wkv5_steps_* (steps_head, common.h).
 //
 // What bounds it.  Forward: HBM (B8 T4096 C4096: 2.9 GB in 0.60 ms; the sequential kernel took 1.3).  Backward: the fp32 matrix
 // instruction, which occupies a SIMD's vector ALU for 32 clocks (99 of them per SIMD and chunk and some 230 vector
@@ -41,7 +42,7 @@ constexpr int PS = 68;               // row stride (floats) of a [token][channel
 constexpr int TS = 20;               // row stride (floats) of a 16 x 16 tile
 constexpr int NT = 512;              // forward: waves 0..3 products, 4..7 loads
 constexpr int NTB = 512;             // backward: waves 0..3 D, 4..7 E
-constexpr float LAM_STRONG = -7.f, LAM_MIN = -17.f;
+constexpr float LAM_STRONG = -7.f;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 DEVINL f32x4 mm(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
@@ -100,9 +101,8 @@ template <bool TWO> DEVINL bool head_setup(Head& hd, const ArgsC& p, int h, int 
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o, 64));
     if (tid < N) {
-        const float a = fmaxf(l1, LAM_MIN), b = fmaxf(l2, LAM_MIN);
-        hd.lam[lane] = a; hd.dec[lane] = wpow(a, L); hd.u[lane] = p.u[c];
-        hd.lam2[lane] = b; hd.dec2[lane] = wpow(b, L); hd.u2[lane] = TWO ? p.u2[c] : 0.f;
+        hd.lam[lane] = l1; hd.dec[lane] = wpow(l1, L); hd.u[lane] = p.u[c];
+        hd.lam2[lane] = l2; hd.dec2[lane] = wpow(l2, L); hd.u2[lane] = TWO ? p.u2[c] : 0.f;
     }
     return __builtin_amdgcn_readfirstlane(mn < LAM_STRONG ? 1 : 0) != 0;
 }
@@ -274,6 +274,7 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
     const int h = blockIdx.x % p.H, b = blockIdx.x / p.H, T = p.T, C = p.C;
     const int nch = (T + L - 1) / L;
     const size_t base = static_cast<size_t>(b) * T * C + static_cast<size_t>(h) * N;
+    if (steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, h * N)) return;
     const bool strong = head_setup<TWO>(S.hd, p, h, tid);
     __syncthreads();
     if (w >= 4) {
@@ -556,9 +557,8 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
     __syncthreads();
     gw = allreduce_rows(gw); gu = allreduce_rows(gu);
     if (g == 0) {
-        const float lt = -expf(p.w[h * N + own]);        // (a decay below the smallest one: its gradient is that of the pairs one step apart)
         const size_t o = static_cast<size_t>(b) * C + h * N + own;
-        p.gw[o] = lt * expf(lt - l1) * gw;
+        p.gw[o] = l1 * gw;
         p.gu[o] = gu;
     }
 }
@@ -691,11 +691,10 @@ DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
     if constexpr (TWO) {
         gw2 = allreduce_rows(gw2); gu2 = allreduce_rows(gu2);
         if (g == 0) {
-            const float lt = -expf(p.w2[h * N + own]);
             const size_t o = static_cast<size_t>(b) * C + h * N + own;
 #pragma unroll
             for (int z = 0; z < 4; ++z) gw2 += S.red[z][own];
-            p.gw2[o] = lt * expf(lt - l2) * gw2;
+            p.gw2[o] = l2 * gw2;
             p.gu2[o] = gu2;
         }
     }
@@ -715,6 +714,7 @@ __global__ __launch_bounds__(NTB, 2) void wkv5c_bwd(const ArgsC p) {
     const int h = blockIdx.x % p.H, b = blockIdx.x / p.H;
     const int nch = (p.T + L - 1) / L;
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * N;
+    if (steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, h * N)) return;
     const bool strong = head_setup<TWO>(S.hd, p, h, tid);
     __syncthreads();
     if (strong) bwd_roles<TWO, true>(S, p, w, lane, h, b, base, nch);
@@ -744,7 +744,7 @@ int check(int B, int T, int C, int H) {
 
 template <bool TWO> int start_fwd(void* stream, int B, const ArgsC& p) {
     hipLaunchKernelGGL(wkv5c_fwd<TWO>, dim3(B * p.H), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
-    return launch_status();
+    return launch_wkv5f32_steps_fwd(static_cast<hipStream_t>(stream), B, p.T, p.H, p.r, p.k, p.v, p.w, p.u, p.w2, p.u2, p.y);
 }
 template <bool TWO> int start_bwd(void* stream, int B, const ArgsC& p, float* rows, float* gw, float* gu, float* gw2, float* gu2) {
     static_assert(sizeof(SmemB<TWO>) <= 160 * 1024, "the backward's LDS must fit one CU");
@@ -753,6 +753,7 @@ template <bool TWO> int start_bwd(void* stream, int B, const ArgsC& p, float* ro
     if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
     hipStream_t st = static_cast<hipStream_t>(stream);
     hipLaunchKernelGGL(wkv5c_bwd<TWO>, dim3(B * p.H), dim3(NTB), sizeof(SmemB<TWO>), st, p);
+    if (int e = launch_wkv5f32_steps_bwd(st, B, p.T, p.H, p.r, p.k, p.v, p.w, p.u, p.w2, p.u2, p.gy, p.gr, p.gk, p.gv, p.gw, p.gu, p.gw2, p.gu2)) return e;
     hipLaunchKernelGGL(rows_sum, dim3((p.C + 255) / 256, TWO ? 4 : 2), dim3(256), 0, st, B, p.C, rows, gw, gu, gw2, gu2);
     return launch_status();
 }

@@ -1,0 +1,78 @@
+"""GPU: wkv5 and wkv5a heads with a decay that is too fast for the powers of the chunked kernels, or is no number.  They run step
+by step, so the decay that acts is the true one, which shows where nothing else hides it (tokens without a key or value of
+their own), and a NaN parameter reaches the outputs and its gradient.
+
+Tolerance: fp32, 1e-5 of an element, not of the largest one: an output here is a handful of products of fp32 factors, with a
+decay whose log (at most 90) is rounded to fp32: 90 x 6e-8."""
+import pytest
+import torch
+
+from oracle import wkv56 as O
+from oracle import wkv5a as A
+from rwkv_cuda_amd import wkv5, wkv5a
+from _gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+def _f32_inputs(B, T, H, seed):
+    g = torch.Generator().manual_seed(seed)
+    rnd = lambda *s: torch.rand(*s, generator=g) * 2 - 1
+    return [rnd(B, T, H * 64) for _ in range(3)] + [rnd(H, 64) for _ in range(4)] + [rnd(B, T, H * 64)]
+
+
+def _run_f32(two, r, k, v, w1, u1, w2, u2, gy):
+    B, T, C = r.shape
+    H = w1.shape[0]
+    t = [x.to(DEV).requires_grad_(True) for x in ((r, k, v, w1, u1, w2, u2) if two else (r, k, v, w1.reshape(C), u1.reshape(C)))]
+    y = wkv5a.CUDA_1(*t) if two else wkv5.RUN_CUDA(B, T, C, H, *t)
+    y.backward(gy.to(DEV))
+    return [y.detach().cpu()] + [x.grad.cpu() for x in t]
+
+
+@pytest.mark.parametrize("two", [False, True])
+def test_fp32_fast_decays_act_as_they_are(lib, two):
+    B, T, H = 2, 50, 3
+    C = H * 64
+    r, k, v, w1, u1, w2, u2, gy = _f32_inputs(B, T, H, 11)
+    w1[0] = torch.linspace(2.80, 2.84, 64)           # either side of the border
+    w1[1, 7], w1[1, 20] = 3.0, 4.5                   # e^-20 and e^-90 a step among ordinary channels
+    if two:
+        w2[2, 30] = 3.0
+    k.view(B, T, H, 64)[:, 17::3] = 0                # pairs of tokens without a key: what is left of the state is all they see
+    k.view(B, T, H, 64)[:, 18::3] = 0
+    r, k, v, w1, u1, w2, u2, gy = [x.double() for x in (r, k, v, w1, u1, w2, u2, gy)]
+    ref = A.grads(B, T, C, H, r, k, v, w1, u1, w2, u2, gy) if two else O.wkv5_grads(B, T, C, H, r, k, v, w1.reshape(C), u1.reshape(C), gy)
+    got = _run_f32(two, *[x.float() for x in (r, k, v, w1, u1, w2, u2, gy)])
+    for name, a, x in zip(["y", "gr", "gk", "gv", "gw1", "gu1", "gw2", "gu2"], ref, got):
+        a, x = a.reshape(x.shape), x.double()
+        e = float((a - x).abs().max() / a.abs().max())
+        print(f"  {name}: max {e:.1e}", flush=True)
+        assert e <= 1e-5, name
+    # a head whose channels are all fast and a token without keys: y is e^l times a product, far below the other tokens'
+    w1 = torch.full((H, 64), 3.2, dtype=torch.float64)
+    w2 = torch.full((H, 64), -30.0, dtype=torch.float64)
+    args = (r, k, v, w1, u1, w2, u2)
+    ref = A.grads(B, T, C, H, *args, gy) if two else O.wkv5_grads(B, T, C, H, r, k, v, w1.reshape(C), u1.reshape(C), gy)
+    got = _run_f32(two, *[x.float() for x in (*args, gy)])
+    a, x = ref[0].reshape(B, T, C)[:, 18::3], got[0].double()[:, 18::3]       # two steps behind the last key
+    assert 0 < float(a.abs().max()) < 1e-9
+    assert float((a - x).abs().max() / a.abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("two", [False, True])
+def test_fp32_nan_decay_is_not_swallowed(lib, two):
+    B, T, H = 1, 40, 3
+    x = _f32_inputs(B, T, H, 12)
+    clean = _run_f32(two, *x)
+    for i in ([3, 5] if two else [3]):
+        x[i] = x[i].clone()
+        x[i][1, 9] = float("nan")
+        got = _run_f32(two, *x)
+        y, c = (z[0].view(B, T, H, 64) for z in (got, clean))
+        # a decay of key channel 9 meets every output of the head, one of value channel 9 its own
+        hit = y[:, 1:, 1] if i == 3 else y[:, 1:, 1, 9]
+        assert torch.isnan(hit).all() and torch.equal(y[:, :, 0], c[:, :, 0]) and torch.equal(y[:, :, 2], c[:, :, 2])
+        g = got[4 if i == 3 else 6].view(H, 64)
+        assert torch.isnan(g[1, 9]) and torch.isfinite(g[0]).all() and torch.isfinite(g[2]).all()
+        x[i] = torch.nan_to_num(x[i])
