@@ -53,6 +53,8 @@ struct Args {
     const uint16_t* u2;
     uint16_t *gw2, *gu2;
     float* rdr;           // workspace [B,T,C] fp32: r * dr'
+    // wkv5_steps_* only: flag words [B*H][8] of the one-sweep kernels (the second may be null)
+    const int *flags, *flags2;
 };
 
 template <int PASS> struct Smem {
@@ -819,15 +821,26 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
 
 // The heads of a wkv5 layer whose decay the chunked kernels do not carry (steps_head, common.h), step by step; all other
 // workgroups return at once.  Backward: the three passes, which need nothing of each other, side by side.
+// bf16, heads of 64, in a layer without a strong decay: the heads that a one-sweep kernel has given up (its flag words, of the
+// forward and in the backward of both directions: such a forward has left no states).
+template <int NP, bool F32, bool TWO> DEVINL bool steps_for(const Args& a) {
+    if constexpr (!F32) {
+        if (strong_layer(static_cast<const uint16_t*>(a.w), a.C, threadIdx.x & 63)) return false;
+        const int lane = threadIdx.x & 63;
+        int x = lane < 8 ? a.flags[8 * blockIdx.x + lane] : 0;
+        if (a.flags2 != nullptr && lane < 8) x |= a.flags2[8 * blockIdx.x + lane];
+        return __ballot(x != 0) != 0ull;
+    } else return steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP);
+}
 template <int NP, int PARTS, bool F32, bool TWO>
 __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_fwd(const Args a, const int hn) {
-    if (!steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP)) return;
+    if (!steps_for<NP, F32, TWO>(a)) return;
     __shared__ SmemRows<NP, PARTS, P_FWD, F32, TWO, true> S;
     rows_body<NP, PARTS, P_FWD, W_HEAD, F32, TWO, true>(S, a, hn);
 }
 template <int NP, int PARTS, bool F32, bool TWO>
 __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_bwd(const Args a, const int hn) {
-    if (!steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP)) return;
+    if (!steps_for<NP, F32, TWO>(a)) return;
     __shared__ union {
         SmemRows<NP, PARTS, P_GR, F32, TWO, true> gr;
         SmemRows<NP, PARTS, P_GV, F32, TWO, true> gv;
@@ -1020,6 +1033,24 @@ int launch_wkv5f32_steps_fwd(hipStream_t st, int B, int T, int H, const float* r
     hipLaunchKernelGGL(kernel, dim3(B * H), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
     return launch_status();
 }
+namespace {
+int launch_wkv5_steps_fwd(hipStream_t st, int B, int T, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
+                          const uint16_t* w, const uint16_t* u, uint16_t* y, const int* flags) {
+    Args a{};
+    a.T = T; a.C = H * N; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.y = y; a.flags = flags;
+    hipLaunchKernelGGL((wkv5_steps_fwd<64, 4, false, false>), dim3(B * H), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    return launch_status();
+}
+int launch_wkv5_steps_bwd(hipStream_t st, int B, int T, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
+                          const uint16_t* w, const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv,
+                          uint16_t* gw, uint16_t* gu, const int* flags_fwd, const int* flags_bwd) {
+    Args a{};
+    a.T = T; a.C = H * N; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.gy = gy; a.gr = gr; a.gk = gk; a.gv = gv; a.gw = gw;
+    a.gu = gu; a.flags = flags_fwd; a.flags2 = flags_bwd;
+    hipLaunchKernelGGL((wkv5_steps_bwd<64, 4, false, false>), dim3(B * H, 3), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    return launch_status();
+}
+}  // namespace
 int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
                              const float* u, const float* w2, const float* u2, const float* gy, float* gr, float* gk, float* gv,
                              float* gw, float* gu, float* gw2, float* gu2) {
@@ -1412,7 +1443,8 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H, const rw
 }
 
 // ---- wkv5 (head size 64) on the one-sweep pair: the raw decay of a channel stands in for every token's, its gradient is
-//      summed over the tokens inside the kernel.  `decay` = [eew | ew] is made for the kernels that redo flagged heads.
+//      summed over the tokens inside the kernel.  A layer with a strong decay belongs to wkv5_bf.hip; heads that a one-sweep
+//      kernel gives up run step by step.
 // heads of 128 channels: one workgroup holds a whole head (wkv5_bf.hip)
 namespace {
 bool whole_head_ok(int C, int H, unsigned flags) { return C == H * N_SPLIT && !(flags & (RWKV_FLAG_SWEEPS | RWKV_PASS_ALL)) && C <= WKV5B_MAX_C; }
@@ -1461,7 +1493,9 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, NB, TB, local, logdec, s32, decay)) return e;
     } else if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, 1, 0, nullptr, nullptr, nullptr, decay)) return e;
-    return launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved));
+    // the heads given up (before wkv5_bf.hip, whose states may lie where the flag words are), then a strong layer
+    if (int e = launch_wkv5_steps_fwd(st, B, T, H, r, k, v, w_raw, u, y, flg)) return e;
+    return launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, nullptr, static_cast<float*>(saved));
 }
 
 size_t rwkv_wkv5s_backward_workspace_bytes(int B, int T, int C, int H) {
@@ -1515,8 +1549,10 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
                                           NB, TB, local, logdec, ds32, gu32, pw, gw32)) return e;
     } else if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, nullptr, pu, nullptr, static_cast<const char*>(saved), flg,
                                              1, 0, nullptr, nullptr, nullptr, nullptr, pw, nullptr)) return e;
-    // a layer with a decay that the mid-point factors cannot carry
+    // a layer with a decay that the mid-point factors cannot carry, then the heads given up
     if (int e = launch_wkv5b_bwd(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved))) return e;
+    const int* flg_fwd = reinterpret_cast<const int*>(static_cast<const char*>(saved) + saved_states_bytes(B, T, H));
+    if (int e = launch_wkv5_steps_bwd(st, B, T, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, flg_fwd, flg)) return e;
     hipLaunchKernelGGL(bf16_batch_sum, dim3((C + 255) / 256), dim3(256), 0, st, B, C, pw, gw, pu, gu);
     return launch_status();
 }

@@ -31,7 +31,7 @@
 // chunk n-it, the SD and E waves do the products of chunk n+1-it, and the P waves finish chunk n+2-it.
 //
 // A chunk in which some channel decays by more than e^-60 over either half cannot use the mid-point factors.  Such a
-// (batch, head) is flagged in `flags` and the caller reruns it with the two-sweep kernels, which have a step-by-step path.
+// (batch, head) is flagged in `flags` and the caller reruns it with the two-sweep kernels, which have a step-by-step path (wkv5: with wkv5_steps_bwd).
 #include "wkv6_fused.h"
 
 namespace rwkv {

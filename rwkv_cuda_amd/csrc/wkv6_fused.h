@@ -71,23 +71,8 @@ DEVINL void split16(const f32x4 (&x)[4], const float s, bf16x8 (&h)[2], bf16x8 (
     }
 }
 
-// wkv5 (one decay per channel): whether any channel of the layer decays faster than the mid-point factors of these kernels carry
-// (16 tokens by more than e^-60: w > 1.32; the threshold is the bfloat16 below).  One such channel moves the whole layer to
-// wkv5_bf.hip, whose workgroups take any decay: redoing the one head after the others would cost the time of the longest
-// sequence once more (B8 T4096 C2048, forward + backward: 0.54 ms here, 0.74 ms there, 1.66 ms with the one head redone step by
-// step).  Every wave looks at every channel (C is a multiple of 64), so all come to the same answer.
-DEVINL bool strong_decay(const float w) { return w > 1.3125f; }
-DEVINL bool strong_layer(const uint16_t* w, const int C, const int lane) {
-    bool strong = false;
-    for (int c = lane * 8; c < C; c += 512) {
-        float f[8];
-        unpack8(*reinterpret_cast<const uint4*>(w + c), f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) strong |= strong_decay(f[e]);
-    }
-    return __ballot(strong) != 0ull;
-}
-// the head's words of the flag array in a layer that is left to wkv5_bf.hip: set if a channel of its own is the reason
+// the head's words of the flag array in a wkv5 layer that is left to wkv5_bf.hip: set if a channel of its own is the reason (in
+// such a layer nothing depends on them)
 DEVINL void flag_strong_head(int* flags, const size_t bh, const uint16_t* w, const int h, const int lane) {
     const bool strong = __ballot(strong_decay(bf2f(w[h * N + lane]))) != 0ull;
     if (lane < 8) flags[bh * 8 + lane] = strong ? 1 : 0;

@@ -19,7 +19,7 @@
 // loaded them, and y leaves through an LDS tile.
 //
 // A chunk in which some channel decays by more than e^-60 over either half cannot use the mid-point factors.  Such a
-// (batch, head) is flagged in `flags` and the caller reruns it with wkv6_fwd_ws, which has a step-by-step path.
+// (batch, head) is flagged in `flags` and the caller reruns it with wkv6_fwd_ws, which has a step-by-step path (wkv5: with wkv5_steps_fwd).
 #include "wkv6_fused.h"
 
 namespace rwkv {
@@ -519,6 +519,12 @@ __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
     if constexpr (HD) {
         if (strong_layer(arg.w, arg.C, tid & 63)) {
             if (tid < 64 && blk == 0) flag_strong_head(arg.flags, bh, arg.w, h, tid);
+            if (tid < 64 && blk == 0 && b == 0) {
+                const int c = h * N + tid;
+                const float ew = -expf(bf2f(arg.w[c]));
+                arg.decay_out[c] = expf(ew);
+                arg.decay_out[arg.C + c] = ew;
+            }
             return;
         }
     }

@@ -2,15 +2,16 @@
 by step, so the decay that acts is the true one, which shows where nothing else hides it (tokens without a key or value of
 their own), and a NaN parameter reaches the outputs and its gradient.
 
-Tolerance: fp32, 1e-5 of an element, not of the largest one: an output here is a handful of products of fp32 factors, with a
+Tolerance: bf16 outputs, the bar of the other bf16 kernels (no further from fp64 than fp32 steps with rounded outputs).  fp32, 1e-5 of an element, not of the largest one: an output here is a handful of products of fp32 factors, with a
 decay whose log (at most 90) is rounded to fp32: 90 x 6e-8."""
 import pytest
 import torch
 
 from oracle import wkv56 as O
 from oracle import wkv5a as A
-from rwkv_cuda_amd import wkv5, wkv5a
-from _gpu_util import DEV
+from rwkv_cuda_amd import synth, wkv5, wkv5a
+from rwkv_cuda_amd._call import call
+from _gpu_util import DEV, assert_no_worse
 
 pytestmark = pytest.mark.gpu
 
@@ -76,3 +77,32 @@ def test_fp32_nan_decay_is_not_swallowed(lib, two):
         g = got[4 if i == 3 else 6].view(H, 64)
         assert torch.isnan(g[1, 9]) and torch.isfinite(g[0]).all() and torch.isfinite(g[2]).all()
         x[i] = torch.nan_to_num(x[i])
+
+
+@pytest.mark.parametrize("B,T,H", [(2, 100, 3), (1, 300, 2)])
+def test_bf16_head_that_the_forward_gave_up_is_redone_by_the_backward(lib, B, T, H):
+    """A one-sweep forward that gives a head up says so in the head's flag words behind the saved states, and leaves no states worth
+    anything: here both are written by hand.  (1, 300, 2) runs as blocks of time."""
+    C = H * 64
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=70 + T)
+    w = w.clamp(max=1.25)
+    ref = O.wkv5_grads(B, T, C, H, r, k, v, w, u, gy)
+    emu = O.emulate_wkv5_bf16(B, T, C, H, r, k, v, w, u, gy)
+    d = [x.to(DEV) for x in (r, k, v, w, u, gy)]
+    bf = dict(device=DEV, dtype=torch.bfloat16)
+    y, decay = torch.empty(B, T, C, **bf), torch.empty(2 * C, device=DEV)
+    nsv = lib.rwkv_wkv5s_saved_bytes(B, T, C, H)
+    saved = torch.empty(nsv, device=DEV, dtype=torch.uint8)
+    call("rwkv_wkv5s_forward", DEV, B, T, C, H, *d[:5], y, decay, saved, nsv, 0)
+    per_head = (T + 63) // 64 * 64 * 64 * 3
+    at = B * H * per_head                                           # the flag words, eight a head
+    assert int(saved[at:at + 32 * B * H].max()) == 0
+    saved[(B * H - 1) * per_head:at] = 0x41                         # the last head
+    saved[at + 32 * (B * H - 1)] = 1
+    gr, gk, gv = (torch.empty(B, T, C, **bf) for _ in range(3))
+    gw, gu = torch.empty(H, 64, **bf), torch.empty(H, 64, **bf)
+    n = lib.rwkv_wkv5s_backward_workspace_bytes(B, T, C, H)
+    ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+    call("rwkv_wkv5s_backward", DEV, B, T, C, H, d[0], d[1], d[2], d[3], decay, d[4], d[5], gr, gk, gv, gw, gu, saved, nsv, ws, n, 0)
+    for name, a, e, x in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, [y, gr, gk, gv, gw, gu]):
+        assert_no_worse(name, a, e.reshape(a.shape), x.reshape(a.shape))
