@@ -117,27 +117,29 @@ DEVINL void allreduce2_rows(float& x, float& y) {
 
 // ----------------------------------------------------------------------------- wkv5: decays that are too fast for chunks
 // wkv5's chunked kernels carry powers e^{l d} of a channel's log decay l = -exp(w) over a few tokens, in both directions.  A head
-// with one channel beyond what they carry (fp32 wkv5c_*: l < -17, where the powers of half a chunk still stay inside fp32) runs step by step instead (wkv5_steps_*, wkv56.hip).  A decay that is no
+// with one channel beyond what they carry (fp32 wkv5c_*: l < -17, where the powers of half a chunk still stay inside fp32; bf16
+// wkv5b_*: l < -9, half a chunk of twice the length) runs step by step instead (wkv5_steps_*, wkv56.hip).  A decay that is no
 // number counts as one of these: the steps hand it on as the operator does.  Chunked and step kernels decide by the same test,
 // for the channels of the head from c0 on.
-constexpr float W_STEPS_F32 = 2.8332133f;      // ln 17
+constexpr float W_STEPS_F32 = 2.8332133f, W_STEPS_BF16 = 2.1875f;      // ln 17; e^2.1875 = 8.91, the last bfloat16 below ln 9
 template <bool F32, int HN> DEVINL bool steps_head(const void* w, const void* w2, const int c0) {
     bool on = false;
 #pragma unroll
     for (int z = 0; z < HN / 64; ++z) {
         const int c = c0 + 64 * z + (threadIdx.x & 63);
-        static_assert(F32, "fp32");
-        on |= !(static_cast<const float*>(w)[c] <= W_STEPS_F32);
-        if (w2 != nullptr) on |= !(static_cast<const float*>(w2)[c] <= W_STEPS_F32);
+        if constexpr (F32) on |= !(static_cast<const float*>(w)[c] <= W_STEPS_F32);
+        else on |= !(bf2f(static_cast<const uint16_t*>(w)[c]) <= W_STEPS_BF16);
+        if (F32 && w2 != nullptr) on |= !(static_cast<const float*>(w2)[c] <= W_STEPS_F32);
     }
     return __ballot(on) != 0ull;
 }
 // bf16, heads of 64: whether any channel of the layer decays faster than the mid-point factors of the one-sweep kernels
-// (wkv6_fwd_f.hip, wkv6_bwd_f.hip) carry (16 tokens by more than e^-60: w > 1.32; the threshold is the bfloat16 below).  One such channel moves the whole layer to wkv5_bf.hip: redoing the one head after the others would cost the time of the
+// (wkv6_fwd_f.hip, wkv6_bwd_f.hip) carry (16 tokens by more than e^-60: w > 1.32; the threshold is the bfloat16 below), or is no
+// number.  One such channel moves the whole layer to wkv5_bf.hip: redoing the one head after the others would cost the time of the
 // longest sequence once more (B8 T4096 C2048, forward + backward: 0.54 ms in one sweep, 0.74 ms there, 1.66 ms with the one head
-// redone step by step).  Every wave looks at every channel (C is a multiple of 64), so
+// redone step by step, as a head beyond W_STEPS_BF16 still is).  Every wave looks at every channel (C is a multiple of 64), so
 // all come to the same answer.
-DEVINL bool strong_decay(const float w) { return w > 1.3125f; }
+DEVINL bool strong_decay(const float w) { return !(w <= 1.3125f); }
 DEVINL bool strong_layer(const uint16_t* w, const int C, const int lane) {
     bool strong = false;
     for (int c = lane * 8; c < C; c += 512) {
@@ -219,7 +221,8 @@ int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r
                              float* gw, float* gu, float* gw2, float* gu2);
 
 // wkv5_bf.hip: wkv5, bf16, heads of 128 or 64 channels, whole heads, decays of any strength; w raw.  Size 64: only layers with a
-// strong decay (strong_layer), the others belong to the one-sweep kernels above and the launch returns at once.  saved (may be null in the forward):
+// strong decay (strong_layer), the others belong to the one-sweep kernels above and the launch returns at once, and of a strong
+// layer only the heads that do not run step by step (steps_head).  saved (may be null in the forward):
 // the states for the backward; gw, gu: per-batch rows [B][C].
 constexpr int WKV5B_MAX_C = 1 << 24;           // byte offsets within 32 rows are 32-bit
 size_t wkv5b_saved_bytes(int B, int T, int C, int H);

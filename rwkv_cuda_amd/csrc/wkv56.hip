@@ -824,13 +824,15 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
 // bf16, heads of 64, in a layer without a strong decay: the heads that a one-sweep kernel has given up (its flag words, of the
 // forward and in the backward of both directions: such a forward has left no states).
 template <int NP, bool F32, bool TWO> DEVINL bool steps_for(const Args& a) {
-    if constexpr (!F32) {
-        if (strong_layer(static_cast<const uint16_t*>(a.w), a.C, threadIdx.x & 63)) return false;
-        const int lane = threadIdx.x & 63;
-        int x = lane < 8 ? a.flags[8 * blockIdx.x + lane] : 0;
-        if (a.flags2 != nullptr && lane < 8) x |= a.flags2[8 * blockIdx.x + lane];
-        return __ballot(x != 0) != 0ull;
-    } else return steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP);
+    if constexpr (!F32 && NP == 64) {
+        if (!strong_layer(static_cast<const uint16_t*>(a.w), a.C, threadIdx.x & 63)) {
+            const int lane = threadIdx.x & 63;
+            int x = lane < 8 ? a.flags[8 * blockIdx.x + lane] : 0;
+            if (a.flags2 != nullptr && lane < 8) x |= a.flags2[8 * blockIdx.x + lane];
+            return __ballot(x != 0) != 0ull;
+        }
+    }
+    return steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP);
 }
 template <int NP, int PARTS, bool F32, bool TWO>
 __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_fwd(const Args a, const int hn) {
@@ -1443,8 +1445,8 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H, const rw
 }
 
 // ---- wkv5 (head size 64) on the one-sweep pair: the raw decay of a channel stands in for every token's, its gradient is
-//      summed over the tokens inside the kernel.  A layer with a strong decay belongs to wkv5_bf.hip; heads that a one-sweep
-//      kernel gives up run step by step.
+//      summed over the tokens inside the kernel.  A layer with a strong decay belongs to wkv5_bf.hip; heads that neither can do
+//      run step by step.
 // heads of 128 channels: one workgroup holds a whole head (wkv5_bf.hip)
 namespace {
 bool whole_head_ok(int C, int H, unsigned flags) { return C == H * N_SPLIT && !(flags & (RWKV_FLAG_SWEEPS | RWKV_PASS_ALL)) && C <= WKV5B_MAX_C; }
@@ -1493,7 +1495,7 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, NB, TB, local, logdec, s32, decay)) return e;
     } else if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, 1, 0, nullptr, nullptr, nullptr, decay)) return e;
-    // the heads given up (before wkv5_bf.hip, whose states may lie where the flag words are), then a strong layer
+    // the heads that run step by step (before wkv5_bf.hip, whose states may lie where the flag words are), then a strong layer
     if (int e = launch_wkv5_steps_fwd(st, B, T, H, r, k, v, w_raw, u, y, flg)) return e;
     return launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, nullptr, static_cast<float*>(saved));
 }
@@ -1549,7 +1551,7 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
                                           NB, TB, local, logdec, ds32, gu32, pw, gw32)) return e;
     } else if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, nullptr, pu, nullptr, static_cast<const char*>(saved), flg,
                                              1, 0, nullptr, nullptr, nullptr, nullptr, pw, nullptr)) return e;
-    // a layer with a decay that the mid-point factors cannot carry, then the heads given up
+    // a layer with a decay that the mid-point factors cannot carry, then the heads that run step by step
     if (int e = launch_wkv5b_bwd(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved))) return e;
     const int* flg_fwd = reinterpret_cast<const int*>(static_cast<const char*>(saved) + saved_states_bytes(B, T, H));
     if (int e = launch_wkv5_steps_bwd(st, B, T, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, flg_fwd, flg)) return e;

@@ -484,7 +484,8 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_fwd(const ArgsW p) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = (p.T + L - 1) / L;
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
-    if (HN == 64 && !strong_layer(p.w, p.C, tid & 63)) return;      // the one-sweep kernels of wkv6 have done this layer
+    // the one-sweep kernels of wkv6 have done this layer, or this head runs step by step
+    if (HN == 64 && (!strong_layer(p.w, p.C, tid & 63) || steps_head<false, HN>(p.w, nullptr, h * HN))) return;
     const float lmin = head_setup<HN>(p, sb, h, b, tid);
     __syncthreads();
     if (w < 4) {
@@ -862,7 +863,7 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_bwd(const ArgsW p) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = 2 * ((p.T + 2 * L - 1) / (2 * L));      // whole pairs (a last chunk without tokens adds zeros)
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
-    if (HN == 64 && !strong_layer(p.w, p.C, tid & 63)) return;
+    if (HN == 64 && (!strong_layer(p.w, p.C, tid & 63) || steps_head<false, HN>(p.w, nullptr, h * HN))) return;
     const bool strong = head_setup<HN>(p, sb, h, b, tid) < LAM_HALF;
     __syncthreads();
     if (w < 4) {

@@ -9,7 +9,7 @@ import torch
 
 from oracle import wkv56 as O
 from oracle import wkv5a as A
-from rwkv_cuda_amd import synth, wkv5, wkv5a
+from rwkv_cuda_amd import synth, wkv5, wkv5_bf16, wkv5a
 from rwkv_cuda_amd._call import call
 from _gpu_util import DEV, assert_no_worse
 
@@ -77,6 +77,51 @@ def test_fp32_nan_decay_is_not_swallowed(lib, two):
         g = got[4 if i == 3 else 6].view(H, 64)
         assert torch.isnan(g[1, 9]) and torch.isfinite(g[0]).all() and torch.isfinite(g[2]).all()
         x[i] = torch.nan_to_num(x[i])
+
+
+def _run_bf16(B, T, C, H, r, k, v, w, u, gy):
+    t = [x.to(DEV).requires_grad_(True) for x in (r, k, v, w, u)]
+    y = wkv5_bf16.RUN_CUDA(B, T, C, H, *t)
+    y.backward(gy.to(DEV))
+    with torch.no_grad():
+        assert torch.equal(wkv5_bf16.RUN_CUDA(B, T, C, H, *t).view(torch.int16), y.view(torch.int16))
+    return [y.detach().cpu()] + [x.grad.cpu() for x in t]
+
+
+@pytest.mark.parametrize("B,T,H,N", [(2, 50, 3, 64), (1, 300, 2, 64)])
+def test_bf16_fast_decays_act_as_they_are(lib, B, T, H, N):
+    """(1, 300, 2, 64) runs as blocks of time where no decay is strong."""
+    C = H * N
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=60 + T)
+    w = w.clone()
+    w[0] = 3.0                                       # e^-20 a step
+    w[1, 3], w[1, 9] = 2.1875, 1.5                   # the last decay of the chunked kernels
+    k = k.clone()
+    k.view(B, T, H, N)[:, 17::3] = 0
+    k.view(B, T, H, N)[:, 18::3] = 0
+    ref = O.wkv5_grads(B, T, C, H, r, k, v, w, u, gy)
+    emu = O.emulate_wkv5_bf16(B, T, C, H, r, k, v, w, u, gy)
+    got = _run_bf16(B, T, C, H, r, k, v, w, u, gy)
+    for name, a, e, x in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, got):
+        assert_no_worse(name, a, e.reshape(a.shape), x.reshape(a.shape))
+    a, e, x = (z.view(B, T, H, N)[:, 18::3, 0] for z in (ref[0], emu[0], got[0]))        # two steps behind the last key
+    assert 0 < float(a.abs().max()) < 1e-6
+    assert_no_worse("y behind the last key", a / a.abs().max(), e.double() / a.abs().max(), x.double() / a.abs().max())
+
+
+@pytest.mark.parametrize("B,T,H,N", [(2, 50, 3, 64), (1, 300, 3, 64)])
+def test_bf16_nan_decay_is_not_swallowed(lib, B, T, H, N):
+    C = H * N
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=90 + T)
+    w = w.clone()
+    w[0, 5] = 1.5                                    # (head 0: a layer of the whole-head kernels either way)
+    clean = _run_bf16(B, T, C, H, r, k, v, w, u, gy)
+    w[1, 9] = float("nan")
+    got = _run_bf16(B, T, C, H, r, k, v, w, u, gy)
+    y, c = (z[0].view(B, T, H, N) for z in (got, clean))
+    assert torch.isnan(y[:, 32:, 1]).all() and torch.equal(y[:, :, 0], c[:, :, 0]) and torch.equal(y[:, :, 2], c[:, :, 2])
+    gw = got[4].view(H, N)
+    assert torch.isnan(gw[1, 9]) and torch.isfinite(gw[0]).all() and torch.isfinite(gw[2]).all()
 
 
 @pytest.mark.parametrize("B,T,H", [(2, 100, 3), (1, 300, 2)])
