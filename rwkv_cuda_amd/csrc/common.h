@@ -220,9 +220,9 @@ int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r
                              const float* u, const float* w2, const float* u2, const float* gy, float* gr, float* gk, float* gv,
                              float* gw, float* gu, float* gw2, float* gu2);
 
-// wkv5_bf.hip: wkv5, bf16, heads of 128 or 64 channels, whole heads, decays of any strength; w raw.  Size 64: only layers with a
-// strong decay (strong_layer), the others belong to the one-sweep kernels above and the launch returns at once, and of a strong
-// layer only the heads that do not run step by step (steps_head).  saved (may be null in the forward):
+// wkv5_bf.hip: wkv5, bf16, heads of 128 or 64 channels, whole heads; w raw.  Size 64: only layers with a
+// strong decay (strong_layer), the others belong to the one-sweep kernels above and the launch returns at once.
+// Heads that run step by step (steps_head) are left out.  saved (may be null in the forward):
 // the states for the backward; gw, gu: per-batch rows [B][C].
 constexpr int WKV5B_MAX_C = 1 << 24;           // byte offsets within 32 rows are 32-bit
 size_t wkv5b_saved_bytes(int B, int T, int C, int H);

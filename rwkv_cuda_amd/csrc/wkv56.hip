@@ -1036,20 +1036,23 @@ int launch_wkv5f32_steps_fwd(hipStream_t st, int B, int T, int H, const float* r
     return launch_status();
 }
 namespace {
-int launch_wkv5_steps_fwd(hipStream_t st, int B, int T, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
+// bf16, heads of 64 or 128 channels (128: flags are not read)
+int launch_wkv5_steps_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
                           const uint16_t* w, const uint16_t* u, uint16_t* y, const int* flags) {
     Args a{};
-    a.T = T; a.C = H * N; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.y = y; a.flags = flags;
-    hipLaunchKernelGGL((wkv5_steps_fwd<64, 4, false, false>), dim3(B * H), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    a.T = T; a.C = C; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.y = y; a.flags = flags;
+    if (C == H * N) hipLaunchKernelGGL((wkv5_steps_fwd<64, 4, false, false>), dim3(B * H), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    else hipLaunchKernelGGL((wkv5_steps_fwd<128, 4, false, false>), dim3(B * H), dim3(RowGeom<128, 4>::NTHREADS), 0, st, a, N_SPLIT);
     return launch_status();
 }
-int launch_wkv5_steps_bwd(hipStream_t st, int B, int T, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
+int launch_wkv5_steps_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
                           const uint16_t* w, const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv,
                           uint16_t* gw, uint16_t* gu, const int* flags_fwd, const int* flags_bwd) {
     Args a{};
-    a.T = T; a.C = H * N; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.gy = gy; a.gr = gr; a.gk = gk; a.gv = gv; a.gw = gw;
+    a.T = T; a.C = C; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.gy = gy; a.gr = gr; a.gk = gk; a.gv = gv; a.gw = gw;
     a.gu = gu; a.flags = flags_fwd; a.flags2 = flags_bwd;
-    hipLaunchKernelGGL((wkv5_steps_bwd<64, 4, false, false>), dim3(B * H, 3), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    if (C == H * N) hipLaunchKernelGGL((wkv5_steps_bwd<64, 4, false, false>), dim3(B * H, 3), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    else hipLaunchKernelGGL((wkv5_steps_bwd<128, 4, false, false>), dim3(B * H, 3), dim3(RowGeom<128, 4>::NTHREADS), 0, st, a, N_SPLIT);
     return launch_status();
 }
 }  // namespace
@@ -1472,7 +1475,8 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         const int e = check_ptrs({r, k, v, w_raw, u, y, decay});
         if (e == RWKV_OK) {
             if (saved != nullptr && (saved_bytes < wkv5b_saved_bytes(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
-            return launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved));
+            if (int e2 = launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved))) return e2;
+            return launch_wkv5_steps_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, nullptr);
         }
         if (saved != nullptr) return e;
     }
@@ -1496,7 +1500,7 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, NB, TB, local, logdec, s32, decay)) return e;
     } else if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, 1, 0, nullptr, nullptr, nullptr, decay)) return e;
     // the heads that run step by step (before wkv5_bf.hip, whose states may lie where the flag words are), then a strong layer
-    if (int e = launch_wkv5_steps_fwd(st, B, T, H, r, k, v, w_raw, u, y, flg)) return e;
+    if (int e = launch_wkv5_steps_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, flg)) return e;
     return launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, nullptr, static_cast<float*>(saved));
 }
 
@@ -1522,6 +1526,7 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
         uint16_t* pw = static_cast<uint16_t*>(workspace);                                 // per-batch gw, then per-batch gu
         uint16_t* pu = pw + whole_head_ws_bytes(B, C) / 4;
         if (int e = launch_wkv5b_bwd(static_cast<hipStream_t>(stream), B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved))) return e;
+        if (int e = launch_wkv5_steps_bwd(static_cast<hipStream_t>(stream), B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, nullptr, nullptr)) return e;
         hipLaunchKernelGGL(bf16_batch_sum, dim3((C + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), B, C, pw, gw, pu, gu);
         return launch_status();
     }
@@ -1554,7 +1559,7 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
     // a layer with a decay that the mid-point factors cannot carry, then the heads that run step by step
     if (int e = launch_wkv5b_bwd(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved))) return e;
     const int* flg_fwd = reinterpret_cast<const int*>(static_cast<const char*>(saved) + saved_states_bytes(B, T, H));
-    if (int e = launch_wkv5_steps_bwd(st, B, T, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, flg_fwd, flg)) return e;
+    if (int e = launch_wkv5_steps_bwd(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, flg_fwd, flg)) return e;
     hipLaunchKernelGGL(bf16_batch_sum, dim3((C + 255) / 256), dim3(256), 0, st, B, C, pw, gw, pu, gu);
     return launch_status();
 }

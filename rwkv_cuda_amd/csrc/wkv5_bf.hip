@@ -1,5 +1,5 @@
 // wkv5, bf16 I/O, whole heads of N = 128 or 64 channels in one workgroup: one forward and one reverse sweep in chunks of
-// L = 32 tokens on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16), for decays of any strength.
+// L = 32 tokens on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16), for decays up to e^-9 a step.
 //
 // Step form (wkv5_bf16/cuda/wkv5_cuda.cu), one head, S[i][j] (i value channel, j key channel), o = e^l, l = -exp(w_raw):
 //     y_t[i] = sum_j r_t[j] (S_t[i][j] + u[j] k_t[j] v_t[i])       S_{t+1} = S_t o + v_t k_t^T
@@ -19,12 +19,12 @@
 // Strong decays.  A factor reaches e^{|l| d}, d the distance of a token from its reference.  The forward has one reference in the
 // middle (its planes serve the state products too), up to |l| = 4.5, and makes its tiles from raw rows beyond.  These, and the
 // backward always, refer to the middle of the half that the output's token lies in (m = 8, 24; a tile's quadrant across the halves
-// to 16): d is 8 and |l| may reach 9, for one more operand per tile.  Heads beyond that take a reference per 8 tokens (m = 4, 12, 20, 28); a pair of tokens d such blocks apart
-// then carries o^{8 d} in addition: a product per distance, half of the factor on either side (o^{8 d} may underflow where the
-// whole term is one).  Below l = -17 a decay is taken as e^{-17} = 4e-8.
-// Handing such heads to step-by-step kernels, as the kernels before did, made one strong channel in 4096 cost more than
-// everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 ms with.  That is why layers of 64-channel
-// heads come here as well once they have such a channel (0.74 ms at B8 T4096 C2048 where they took 1.66 ms).
+// to 16): d is 8 and |l| may reach 9, for one more operand per tile.  A head beyond that, or with a decay that is no number, is left
+// to wkv5_steps_* (steps_head, common.h): with a reference per 8 tokens, and a product for each distance of two such blocks, the
+// loops spill hundreds of registers, and decays below e^-17 are out of reach all the same.
+// Handing every head with a strong decay (|l| > 3.7) to step-by-step kernels, as the kernels before did, made one such channel in
+// 4096 cost more than everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 ms with.  That is why
+// layers of 64-channel heads come here as well once they have such a channel (0.74 ms at B8 T4096 C2048 where they took 1.66 ms).
 //
 // What bounds it (B8 T4096 C4096: one workgroup per CU).  Forward 0.52 ms for 2.1 GB, half of them the saved states: HBM (4.1 TB/s;
 // 0.82 ms as four heads of 64).  Backward 1.03 ms: the D waves, some 1600 vector and 170 matrix instructions a chunk, and their
@@ -38,8 +38,7 @@ namespace rwkv {
 namespace {
 
 constexpr int NTH = 512;             // waves 0..3 hold states, 4..7 load and prepare
-constexpr float LAM_MID = -4.5f, LAM_HALF = -9.f, LAM_MIN = -17.f;      // strongest log decay for one reference, for one per half; taken at most
-enum { REF_MID, REF_HALF, REF_8 };
+constexpr float LAM_MID = -4.5f;     // strongest log decay for one reference (one per half: W_STEPS_BF16)
 constexpr f32x4 ZERO4 = {0.f, 0.f, 0.f, 0.f};
 
 struct ArgsW {
@@ -126,7 +125,7 @@ template <int HN> DEVINL float head_setup(const ArgsW& p, lds_t sb, int h, int b
         const float l = -expf(bf2f(p.w[c]));
         mn = fminf(mn, l);
         if (tid < 64) {
-            lds_st<float>(sb + G<HN>::LAM + 4 * n, fmaxf(l, LAM_MIN));
+            lds_st<float>(sb + G<HN>::LAM + 4 * n, l);
             lds_st<float>(sb + G<HN>::U + 4 * n, bf2f(p.u[c]));
             if (p.decay != nullptr && b == 0) { p.decay[c] = expf(l); p.decay[p.C + c] = l; }
         }
@@ -195,87 +194,25 @@ template <bool LANE_SNK, int PARTS, uint32_t PART> DEVINL void take_parts(lds_t 
     else { a[0] = split8(s[0], s[1]); a[1] = split8(ZERO4, s[2]); }
 }
 // powers for a tile part, channel ch0 + e: of token 16 z + l16, x as the sink, y as the source; they are those of the token in its
-// half (strong: in its 8 tokens) and serve both.  cx, cy: as sink of the second and source of the first half of a pair across
-// them; strong: w4 = o^4.
-template <bool STRONG> struct TilePowers { float px[8], py[8], cx[STRONG ? 1 : 8], cy[STRONG ? 1 : 8], w4[STRONG ? 8 : 1]; };
-template <bool STRONG> DEVINL void tile_powers(TilePowers<STRONG>& t, lds_t lam, int l16) {
-    const int m = STRONG ? 8 * (l16 >> 3) + 4 : 8;
+// half and serve both.  cx, cy: as sink of the second and source of the first half of a pair across them.
+struct TilePowers { float px[8], py[8], cx[8], cy[8]; };
+DEVINL void tile_powers(TilePowers& t, lds_t lam, int l16) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const float l = lds_f(lam + 4 * e);
-        t.px[e] = wpow(l, l16 - m); t.py[e] = wpow(l, m - 1 - l16);
-        if constexpr (STRONG) t.w4[e] = wpow(l, 4);
-        else { t.cx[e] = wpow(l, l16); t.cy[e] = wpow(l, 15 - l16); }
+        t.px[e] = wpow(l, l16 - 8); t.py[e] = wpow(l, 7 - l16);
+        t.cx[e] = wpow(l, l16); t.cy[e] = wpow(l, 15 - l16);
     }
 }
 // tile part from raw rows (operands of the two token tiles)
-template <bool LANE_SNK, bool STRONG> DEVINL void raw_part(const bf16x8 (&r)[2], const bf16x8 (&k)[2], const TilePowers<STRONG>& t, int lane, f32x4 (&q)[3]) {
+template <bool LANE_SNK> DEVINL void raw_part(const bf16x8 (&r)[2], const bf16x8 (&k)[2], const TilePowers& t, f32x4 (&q)[3]) {
     using Q = Quad<LANE_SNK>;
-    if constexpr (!STRONG) {
 #pragma unroll
-        for (int z = 0; z < 3; ++z) {
-            const bool across = Q::ROWT[z] != Q::LANET[z];
-            const int snk = LANE_SNK ? Q::LANET[z] : Q::ROWT[z], src = LANE_SNK ? Q::ROWT[z] : Q::LANET[z];
-            const Op2 x = scaled(r[snk], across ? t.cx : t.px), y = scaled(k[src], across ? t.cy : t.py);
-            q[z] = LANE_SNK ? mm3(y, x, ZERO4) : mm3(x, y, ZERO4);
-        }
-    } else {
-        const int l16 = lane & 15, g = lane >> 4;
-        float fx[8], fy[8];
-#pragma unroll
-        for (int z = 0; z < 3; ++z) q[z] = ZERO4;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            fx[e] = t.px[e]; fy[e] = t.py[e];
-            asm volatile("" : "+v"(fx[e]), "+v"(fy[e]));   // (the products below are the same in every chunk: 48 registers across the loop)
-        }
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            __builtin_amdgcn_sched_barrier(0);
-            const Op2 x[2] = {scaled(r[0], fx), scaled(r[1], fx)}, y[2] = {scaled(k[0], fy), scaled(k[1], fy)};
-#pragma unroll
-            for (int z = 0; z < 3; ++z) {
-                const f32x4 o = LANE_SNK ? mm3(y[Q::ROWT[z]], x[Q::LANET[z]], ZERO4) : mm3(x[Q::ROWT[z]], y[Q::LANET[z]], ZERO4);
-                const int rb = 2 * Q::ROWT[z] + (g >> 1), lb = 2 * Q::LANET[z] + (l16 >> 3);
-                const bool on = (LANE_SNK ? lb - rb : rb - lb) == d;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) q[z][v] = on ? o[v] : q[z][v];
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) { fx[e] *= t.w4[e]; fy[e] *= t.w4[e]; }
-        }
-    }
-}
-// NA tiles applied to an operand: sum over the row tokens (slots) of tile x operand, for one lane tile.  b: the operand, x scaled by
-// pf.  Strong: per distance d of the blocks of 8 tokens, with o^{4 d} on the operand and on the result (o^{8 d} may underflow where
-// the whole term is one); w4: o^4 of the output's lane, which is the operand's.
-template <bool LANE_SNK, bool STRONG, int NA>
-DEVINL void apply(const Op2 (&a)[NA], const Op2& b, const bf16x8& x, const float (&pf)[8], int lane_tile, int lane, float w4, f32x4 (&out)[NA]) {
-    if constexpr (!STRONG) {
-#pragma unroll
-        for (int i = 0; i < NA; ++i) out[i] = mm3(a[i], b, ZERO4);
-    } else {
-        const int l16 = lane & 15, g = lane >> 4, lb = 2 * lane_tile + (l16 >> 3), d0 = LANE_SNK ? lb - (g >> 1) : (g >> 1) - lb, d1 = d0 + (LANE_SNK ? -2 : 2);
-        float f = 1.f;
-#pragma unroll
-        for (int i = 0; i < NA; ++i) out[i] = ZERO4;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            __builtin_amdgcn_sched_barrier(0);           // one distance after the other: side by side they take too many registers
-            float pd[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pd[e] = pf[e] * f;
-            const Op2 bd = d == 0 ? b : scaled(x, pd);
-            const bool on0 = d0 == d, on1 = d1 == d;
-#pragma unroll
-            for (int i = 0; i < NA; ++i) {
-                const uint4 ah = __builtin_bit_cast(uint4, a[i].h), al = __builtin_bit_cast(uint4, a[i].l);
-                const Op2 ad = {as_op(on0 ? ah.x : 0u, on0 ? ah.y : 0u, on1 ? ah.z : 0u, on1 ? ah.w : 0u),
-                                as_op(on0 ? al.x : 0u, on0 ? al.y : 0u, on1 ? al.z : 0u, on1 ? al.w : 0u)};
-                out[i] += mm3(ad, bd, ZERO4) * f;
-            }
-            f *= w4;
-        }
+    for (int z = 0; z < 3; ++z) {
+        const bool across = Q::ROWT[z] != Q::LANET[z];
+        const int snk = LANE_SNK ? Q::LANET[z] : Q::ROWT[z], src = LANE_SNK ? Q::ROWT[z] : Q::LANET[z];
+        const Op2 x = scaled(r[snk], across ? t.cx : t.px), y = scaled(k[src], across ? t.cy : t.py);
+        q[z] = LANE_SNK ? mm3(y, x, ZERO4) : mm3(x, y, ZERO4);
     }
 }
 
@@ -283,17 +220,17 @@ DEVINL void apply(const Op2 (&a)[NA], const Op2& b, const bf16x8& x, const float
 // Waves 0..3 hold St[ct][jt][v] = S[j = 16 jt + 4 g + v][i = own], as it stands the B operand of a contraction over j.  Waves 4..7
 // load (two chunks ahead of the planes, the planes two chunks ahead of their use) and make the next chunk's tile in parts of 32
 // key channels.  One barrier a chunk.
-// Planes: R' = r o^{t-16}, K' = k o^{15-t} (they serve the tile, the state times o^16 on its way in and out of the update); strong
-// decays: r o^t, k o^{31-t}, and the tile is made from the raw rows (read once more, from L2).
-template <int HN, bool STRONG> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int q, int lane, size_t base, int nch) {
+// Planes: R' = r o^{t-16}, K' = k o^{15-t} (they serve the tile, the state times o^16 on its way in and out of the update); RAW, for
+// strong decays: r o^t, k o^{31-t}, and the tile is made from the raw rows (read once more, from L2).
+template <int HN, bool RAW> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int q, int lane, size_t base, int nch) {
     using A = G<HN>;
     constexpr int CT = A::CT, KS = A::KS, NJ = A::NB16;
     const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
-    float dd[NJ][4];                                     // o^16; strong: o^32
+    float dd[NJ][4];                                     // o^16; RAW: o^32
 #pragma unroll
     for (int jt = 0; jt < NJ; ++jt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) dd[jt][v] = wpow(lds_f(sb + A::LAM + 4 * (16 * jt + 4 * g + v)), STRONG ? 32 : 16);
+        for (int v = 0; v < 4; ++v) dd[jt][v] = wpow(lds_f(sb + A::LAM + 4 * (16 * jt + 4 * g + v)), RAW ? 32 : 16);
     f32x4 St[CT][NJ];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)
@@ -335,7 +272,7 @@ template <int HN, bool STRONG> DEVINL void fwd_states(const ArgsW& p, lds_t sb, 
             }
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
-                if constexpr (!STRONG) {
+                if constexpr (!RAW) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) { St[ct][2 * ks][v] *= dd[2 * ks][v]; St[ct][2 * ks + 1][v] *= dd[2 * ks + 1][v]; }
                 }
@@ -363,12 +300,12 @@ template <int HN, bool STRONG> DEVINL void fwd_states(const ArgsW& p, lds_t sb, 
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
                 f32x4 s = St[ct][jt];
-                if constexpr (STRONG) {
+                if constexpr (RAW) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) s[v] *= dd[jt][v];
                 }
                 s = mfma(kl, vo[ct], mfma(kh, vo[ct], s));
-                if constexpr (!STRONG) {
+                if constexpr (!RAW) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) s[v] *= dd[jt][v];
                 }
@@ -379,9 +316,8 @@ template <int HN, bool STRONG> DEVINL void fwd_states(const ArgsW& p, lds_t sb, 
     }
 }
 
-template <int HN, int REF> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int tp, size_t base, int nch) {
+template <int HN, bool RAW> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int tp, size_t base, int nch) {
     using A = G<HN>;
-    constexpr bool RAW = REF != REF_MID, STRONG = REF == REF_8;       // the tile is made from raw rows
     constexpr int NP = A::PASSES;
     const int lane = tp & 63, q = tp >> 6, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
     const int row0 = tp / A::PIECES, c8 = (tp % A::PIECES) * 8;
@@ -397,7 +333,7 @@ template <int HN, int REF> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int t
             pk[z][e] = wpow(l, RAW ? 31 - t : 15 - t);
         }
     }
-    [[maybe_unused]] TilePowers<STRONG> tpw;
+    [[maybe_unused]] TilePowers tpw;
     if constexpr (RAW) tile_powers(tpw, sb + A::LAM + 4 * (32 * (q % A::PARTS) + 8 * g), l16);
     uint4 x[2][3][NP];
     auto fetch = [&](const int c, uint4 (&d)[3][NP]) __attribute__((always_inline)) {
@@ -442,7 +378,7 @@ template <int HN, int REF> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int t
                 const int o = 2 * ((16 * z + l16) * C + 32 * q + 8 * g);
                 r[z] = op4(load16(rr, o)); k[z] = op4(load16(kk, o));
             }
-            raw_part<true, STRONG>(r, k, tpw, lane, qd);
+            raw_part<true>(r, k, tpw, qd);
         } else {
             Op2 xo[2], yo[2];
 #pragma unroll
@@ -484,17 +420,16 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_fwd(const ArgsW p) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = (p.T + L - 1) / L;
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
-    // the one-sweep kernels of wkv6 have done this layer, or this head runs step by step
-    if (HN == 64 && (!strong_layer(p.w, p.C, tid & 63) || steps_head<false, HN>(p.w, nullptr, h * HN))) return;
-    const float lmin = head_setup<HN>(p, sb, h, b, tid);
+    if (HN == 64 && !strong_layer(p.w, p.C, tid & 63)) return;      // the one-sweep kernels of wkv6 have done this layer
+    const float lmin = head_setup<HN>(p, sb, h, b, tid);            // (the decays of every head go to p.decay)
+    if (steps_head<false, HN>(p.w, nullptr, h * HN)) return;
     __syncthreads();
     if (w < 4) {
         if (lmin < LAM_MID) fwd_states<HN, true>(p, sb, w, tid & 63, base, nch);
         else fwd_states<HN, false>(p, sb, w, tid & 63, base, nch);
     } else {
-        if (lmin < LAM_HALF) fwd_loads<HN, REF_8>(p, sb, tid - 256, base, nch);
-        else if (lmin < LAM_MID) fwd_loads<HN, REF_HALF>(p, sb, tid - 256, base, nch);
-        else fwd_loads<HN, REF_MID>(p, sb, tid - 256, base, nch);
+        if (lmin < LAM_MID) fwd_loads<HN, true>(p, sb, tid - 256, base, nch);
+        else fwd_loads<HN, false>(p, sb, tid - 256, base, nch);
     }
 }
 
@@ -514,13 +449,12 @@ template <bool LANE_SNK> DEVINL void mask(f32x4 (&b)[3], int l16, int g) {
         for (int v = 0; v < 4; ++v) b[z][v] = causal<LANE_SNK>(z, l16, 4 * g + v) ? b[z][v] : 0.f;
 }
 
-template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, int h, int b, size_t base, int nch) {
+template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, int h, int b, size_t base, int nch) {
     using A = G<HN>;
     constexpr int CT = A::CT, KS = A::KS, NI = A::NB16;
     const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
     // Powers of a set of eight slots, token 16 a + 4 g + b: a base per lane times o^b times o^{16 a} (or the reverse); the eight would
-    // take the registers that the states need.  Bases: cb of o^{t-m}, kb of o^{m-1-t}, m the middle of the token's half (strong: of
-    // its 8 tokens).
+    // take the registers that the states need.  Bases: cb of o^{t-m}, kb of o^{m-1-t}, m the middle of the token's half.
     float l[CT], u[CT], o1[CT], o2[CT], o3[CT], o8[CT], o16[CT], o32[CT], cb[CT], kb[CT];
     f32x4 dS[CT][NI];
     float gw[CT], gP[CT], gu[CT];
@@ -529,8 +463,8 @@ template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int 
         const int j = 16 * (CT * q + ct) + l16;
         l[ct] = lds_f(sb + A::LAM + 4 * j); u[ct] = lds_f(sb + A::U + 4 * j);
         o1[ct] = wpow(l[ct], 1); o2[ct] = wpow(l[ct], 2); o3[ct] = wpow(l[ct], 3); o8[ct] = wpow(l[ct], 8); o16[ct] = wpow(l[ct], 16); o32[ct] = wpow(l[ct], 32);
-        cb[ct] = wpow(l[ct], STRONG ? 4 * (g & 1) - 4 : 4 * g - 8);
-        kb[ct] = wpow(l[ct], STRONG ? -4 * (g & 1) : 4 - 4 * g);
+        cb[ct] = wpow(l[ct], 4 * g - 8);
+        kb[ct] = wpow(l[ct], 4 - 4 * g);
 #pragma unroll
         for (int ib = 0; ib < NI; ++ib) dS[ct][ib] = ZERO4;
         gw[ct] = gP[ct] = gu[ct] = 0.f;
@@ -551,8 +485,8 @@ template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int 
     };
     auto to_ref = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { up(ct, cb[ct], false, f); };                                    // o^{t-m}
     auto from_ref = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { down(ct, kb[ct], false, f); };                                // o^{m-1-t}
-    auto from_start = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { up(ct, STRONG ? wpow(hide(l[ct]), 4 * g) : cb[ct] * o8[ct], true, f); };            // o^t
-    auto to_end = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { down(ct, STRONG ? wpow(hide(l[ct]), 12 - 4 * g) : kb[ct] * o8[ct], true, f); };         // o^{31-t}
+    auto from_start = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { up(ct, cb[ct] * o8[ct], true, f); };            // o^t
+    auto to_end = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { down(ct, kb[ct] * o8[ct], true, f); };            // o^{31-t}
     // The operands that a tile's lane tiles 0 and 1 are applied to, referred to the middle of the lane's half whichever half a slot's
     // token lies in.  f: the powers of the token in its own half.  Only the far pair (sinks of the second half for a source of the
     // first, or sources of the first for a sink of the second) takes o^16; the slots on the wrong side of the lane tile meet zeros.
@@ -562,24 +496,23 @@ template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int 
 #pragma unroll
         for (int e = 0; e < 8; ++e) fx[e] *= f[e];
         o[0] = o[1] = split8(fx);
-        if constexpr (!STRONG) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ff[e] = (sinks ? fx[4 + e] : fx[e]) * o8[ct] * o8[ct];      // (o^16 may underflow where this does not)
-            const HL a = hilo2k(ff[0], ff[1]), b = hilo2k(ff[2], ff[3]);
-            Op2& w = o[sinks ? 0 : 1];
-            const uint4 h = __builtin_bit_cast(uint4, w.h), lo = __builtin_bit_cast(uint4, w.l);
-            w = sinks ? Op2{as_op(h.x, h.y, a.h, b.h), as_op(lo.x, lo.y, a.l, b.l)} : Op2{as_op(a.h, b.h, h.z, h.w), as_op(a.l, b.l, lo.z, lo.w)};
-        }
+        for (int e = 0; e < 4; ++e) ff[e] = (sinks ? fx[4 + e] : fx[e]) * o8[ct] * o8[ct];      // (o^16 may underflow where this does not)
+        const HL a = hilo2k(ff[0], ff[1]), b = hilo2k(ff[2], ff[3]);
+        Op2& w = o[sinks ? 0 : 1];
+        const uint4 h = __builtin_bit_cast(uint4, w.h), lo = __builtin_bit_cast(uint4, w.l);
+        w = sinks ? Op2{as_op(h.x, h.y, a.h, b.h), as_op(lo.x, lo.y, a.l, b.l)} : Op2{as_op(a.h, b.h, h.z, h.w), as_op(a.l, b.l, lo.z, lo.w)};
     };
     const float t0 = static_cast<float>(4 * g);
     const int to = tile_offset(l16, g, C);
-    const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * (nch / 2) * HN * HN + (16 * CT * q + l16) * HN + 4 * g;
+    const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * (nch / 2) * HN * HN;
+    const uint32_t so = (16 * CT * q + l16) * HN + 4 * g;         // (a scalar base and one lane offset)
     auto fetch_state = [&](int c, int ks, f32x4 (&s)[CT][2]) __attribute__((always_inline)) {
         const float* const d = sv + static_cast<size_t>(c >> 1) * HN * HN + 32 * ks;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-            for (int z = 0; z < 2; ++z) s[ct][z] = *reinterpret_cast<const f32x4*>(d + 16 * ct * HN + 16 * z);
+            for (int z = 0; z < 2; ++z) s[ct][z] = *reinterpret_cast<const f32x4*>(d + 16 * ct * HN + 16 * z + so);
     };
     auto chunk = [&](auto odd_, const int c) __attribute__((always_inline)) {
         constexpr bool ODD = decltype(odd_)::value;
@@ -635,13 +568,10 @@ template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int 
             tile_operands(ct, true, rT, pm, ro);
             from_ref(ct, pf);
             to_end(ct, pe);
-            const float w4 = STRONG ? o2[ct] * o2[ct] : 1.f;
             const float th = hide(t0);
 #pragma unroll
             for (int z = 0; z < 2; ++z) {
-                const Op2 tiles[2] = {ba[z], la[z]};
-                f32x4 tz[2];
-                apply<false, STRONG>(tiles, ro[z], rT, pm, z, lane, w4, tz);
+                const f32x4 tz[2] = {mm3(ba[z], ro[z], ZERO4), mm3(la[z], ro[z], ZERO4)};
                 f32x4 o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
@@ -712,18 +642,15 @@ template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int 
             tile_operands(ct, false, kT, pm, ko);
             to_ref(ct, pf);
             from_start(ct, ps);
-            const float w4 = STRONG ? o2[ct] * o2[ct] : 1.f;
             const float th = hide(t0);
 #pragma unroll
             for (int z = 0; z < 2; ++z) {
-                const Op2 tiles[1] = {ca[z]};
-                f32x4 tx[1];
-                apply<true, STRONG>(tiles, ko[z], kT, pm, z, lane, w4, tx);
+                const f32x4 tx = mm3(ca[z], ko[z], ZERO4);
                 f32x4 o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const int e = 4 * z + v;
-                    const float x = X[z][ct][v] * ps[e], ti = tx[0][v] * pf[e], vg = z ? vg1[v] : vg0[v], t = th + static_cast<float>(16 * z + v);
+                    const float x = X[z][ct][v] * ps[e], ti = tx[v] * pf[e], vg = z ? vg1[v] : vg0[v], t = th + static_cast<float>(16 * z + v);
                     gw[ct] = fmaf(r[e] * t, x, gw[ct]);
                     o[v] = fmaf(k[e] * vg, u[ct], x + ti);
                 }
@@ -742,30 +669,27 @@ template <int HN, bool STRONG> DEVINL void role_d(const ArgsW& p, lds_t sb, int 
         const int c = h * HN + 16 * (CT * q + ct) + l16;
         const float sw = allreduce_rows(fmaf(32.f * o32[ct], gP[ct], gw[ct])), su = allreduce_rows(gu[ct]);
         if (g == 0) {
-            const float lt = -expf(bf2f(p.w[c]));        // (a decay below the smallest one: its gradient is that of the pairs one step apart)
-            const float f = expf(lt - l[ct]);            // zero long before lt leaves fp32's range
-            p.gw[static_cast<size_t>(b) * C + c] = f2bf(f > 0.f ? lt * f * sw : 0.f);
+            p.gw[static_cast<size_t>(b) * C + c] = f2bf(l[ct] * sw);
             p.gu[static_cast<size_t>(b) * C + c] = f2bf(su);
         }
     }
 }
 
-template <int HN, bool STRONG> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, size_t base, int nch) {
+template <int HN> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, size_t base, int nch) {
     using A = G<HN>;
     constexpr int CT = A::CT, KS = A::KS, NP = A::PASSES;
     const int q = __builtin_amdgcn_readfirstlane(te >> 6), lane = te & 63, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
     const int row0 = te / A::PIECES, c8 = (te % A::PIECES) * 8, to = tile_offset(l16, g, C);
-    float u[8], cke[2][KS][8];                           // cke: o^{31-t} of token 16 tt + l16, channel 32 ks + 8 g + e
+    float cke[2][KS][8];                                 // o^{31-t} of token 16 tt + l16, channel 32 ks + 8 g + e
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        u[e] = lds_f(sb + A::U + 4 * (c8 + e));
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const float l = lds_f(sb + A::LAM + 4 * (32 * ks + 8 * g + e));
             cke[0][ks][e] = wpow(l, 31 - l16); cke[1][ks][e] = wpow(l, 15 - l16);
         }
     }
-    TilePowers<STRONG> tp;
+    TilePowers tp;
     tile_powers(tp, sb + A::LAM + 4 * (32 * (q % A::PARTS) + 8 * g), l16);
     auto fetch = [&](const int c, uint4 (&d)[4][NP]) __attribute__((always_inline)) {
         const int cc = max(c, 0);
@@ -780,6 +704,7 @@ template <int HN, bool STRONG> DEVINL void role_e(const ArgsW& p, lds_t sb, int 
     };
     auto put = [&](const int sl, const uint4 (&d)[4][NP]) __attribute__((always_inline)) {
         const lds_t s = sb + A::BASE + sl * A::SLOT;
+        const f32x4 u[2] = {lds_ld<f32x4>(sb + A::U + 4 * c8), lds_ld<f32x4>(sb + A::U + 4 * c8 + 16)};      // (registers for these across the loop would spill others)
 #pragma unroll
         for (int z = 0; z < NP; ++z) {
             const int t = row0 + z * A::ROWS;
@@ -789,7 +714,7 @@ template <int HN, bool STRONG> DEVINL void role_e(const ArgsW& p, lds_t sb, int 
             float r[8], k[8], v[8], gy[8], a = 0.f, b = 0.f;
             unpack8(d[0][z], r); unpack8(d[1][z], k); unpack8(d[2][z], v); unpack8(d[3][z], gy);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) { a = fmaf(r[e] * u[e], k[e], a); b = fmaf(v[e], gy[e], b); }
+            for (int e = 0; e < 8; ++e) { a = fmaf(r[e] * u[e >> 2][e & 3], k[e], a); b = fmaf(v[e], gy[e], b); }
             a = lanes_sum<A::PIECES>(a); b = lanes_sum<A::PIECES>(b);
             if (c8 == 0) { lds_st<float>(s + A::RUK + 4 * t, a); lds_st<float>(s + A::VG + 4 * t, b); }
         }
@@ -812,7 +737,7 @@ template <int HN, bool STRONG> DEVINL void role_e(const ArgsW& p, lds_t sb, int 
             opaque(o);
             const bf16x8 r[2] = {ld_op(o + A::R), ld_op(o + A::R + 16 * A::ROW)}, k[2] = {ld_op(o + A::K), ld_op(o + A::K + 16 * A::ROW)};
             f32x4 qd[3];
-            raw_part<false, STRONG>(r, k, tp, lane, qd);
+            raw_part<false>(r, k, tp, qd);
             const float diag[2] = {q == 0 ? lds_f(sx + A::RUK + 4 * l16) : 0.f, q == 0 ? lds_f(sx + A::RUK + 4 * (16 + l16)) : 0.f};
             put_part<false>(sb + A::BPART + q * A::PART, qd, diag, lane);
         }
@@ -863,16 +788,11 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_bwd(const ArgsW p) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = 2 * ((p.T + 2 * L - 1) / (2 * L));      // whole pairs (a last chunk without tokens adds zeros)
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
-    if (HN == 64 && (!strong_layer(p.w, p.C, tid & 63) || steps_head<false, HN>(p.w, nullptr, h * HN))) return;
-    const bool strong = head_setup<HN>(p, sb, h, b, tid) < LAM_HALF;
+    if ((HN == 64 && !strong_layer(p.w, p.C, tid & 63)) || steps_head<false, HN>(p.w, nullptr, h * HN)) return;
+    head_setup<HN>(p, sb, h, b, tid);
     __syncthreads();
-    if (w < 4) {
-        if (strong) role_d<HN, true>(p, sb, w, tid & 63, h, b, base, nch);
-        else role_d<HN, false>(p, sb, w, tid & 63, h, b, base, nch);
-    } else {
-        if (strong) role_e<HN, true>(p, sb, tid - 256, base, nch);
-        else role_e<HN, false>(p, sb, tid - 256, base, nch);
-    }
+    if (w < 4) role_d<HN>(p, sb, w, tid & 63, h, b, base, nch);
+    else role_e<HN>(p, sb, tid - 256, base, nch);
 }
 
 template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, uint32_t lds) {

@@ -88,7 +88,7 @@ def _run_bf16(B, T, C, H, r, k, v, w, u, gy):
     return [y.detach().cpu()] + [x.grad.cpu() for x in t]
 
 
-@pytest.mark.parametrize("B,T,H,N", [(2, 50, 3, 64), (1, 300, 2, 64)])
+@pytest.mark.parametrize("B,T,H,N", [(2, 50, 3, 64), (1, 300, 2, 64), (2, 50, 3, 128), (1, 100, 2, 128)])
 def test_bf16_fast_decays_act_as_they_are(lib, B, T, H, N):
     """(1, 300, 2, 64) runs as blocks of time where no decay is strong."""
     C = H * N
@@ -109,7 +109,7 @@ def test_bf16_fast_decays_act_as_they_are(lib, B, T, H, N):
     assert_no_worse("y behind the last key", a / a.abs().max(), e.double() / a.abs().max(), x.double() / a.abs().max())
 
 
-@pytest.mark.parametrize("B,T,H,N", [(2, 50, 3, 64), (1, 300, 3, 64)])
+@pytest.mark.parametrize("B,T,H,N", [(2, 50, 3, 64), (1, 300, 3, 64), (2, 70, 3, 128)])
 def test_bf16_nan_decay_is_not_swallowed(lib, B, T, H, N):
     C = H * N
     r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=90 + T)
