@@ -306,10 +306,11 @@ Tensor wkv5_bf16_op(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& r,
 }
 
 // ------------------------------------------------------- wkv6 and wkv6_state, bf16 (wkv6/run.py:128-170, wkv6_state/run.py:80-124)
-// (s: the initial state, undefined for wkv6)
-variable_list wkv6_grads(AutogradContext* ctx, const Tensor& gy_, const Tensor& s0) {
+// (s: the initial state, undefined for wkv6; the saved variables are taken once: hooks on them run per taking, and a checkpoint
+// refuses a second one)
+variable_list wkv6_grads(AutogradContext* ctx, const Tensor& gy_, bool state) {
     const auto s = ctx->get_saved_variables();
-    const Tensor &r = s[0], &k = s[1], &v = s[2], &w = s[3], &u = s[4], &saved = s[5], gy = gy_.contiguous();
+    const Tensor &r = s[0], &k = s[1], &v = s[2], &w = s[3], &u = s[4], &saved = s[5], s0 = state ? s[6] : Tensor(), gy = gy_.contiguous();
     const Dims d = get_dims(ctx);
     const Guard guard(r.device());
     const auto o = r.options();
@@ -347,7 +348,7 @@ struct Wkv6 : Function<Wkv6> {
         return wkv6_run(ctx, B, T, C, H, r, k, v, w, u, NONE, flags);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g) {
-        variable_list x = wkv6_grads(ctx, g[0], NONE);
+        variable_list x = wkv6_grads(ctx, g[0], false);
         x.erase(x.begin() + 9);
         return x;
     }
@@ -360,7 +361,7 @@ struct Wkv6State : Function<Wkv6State> {
         require(s.numel() == B * C * (C / H), "shape mismatch");
         return wkv6_run(ctx, B, T, C, H, r, k, v, w, u, s, flags);
     }
-    static variable_list backward(AutogradContext* ctx, variable_list g) { return wkv6_grads(ctx, g[0], ctx->get_saved_variables()[6]); }
+    static variable_list backward(AutogradContext* ctx, variable_list g) { return wkv6_grads(ctx, g[0], true); }
 };
 Tensor wkv6_op(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& w, const Tensor& u, int64_t flags) {
     return Wkv6::apply(B, T, C, H, r, k, v, w, u, flags);
