@@ -421,7 +421,7 @@ variable_list rwkv7_grads(AutogradContext* ctx, const Tensor& dy_, const Tensor&
     const int B = i32(get(ctx, "B")), T = i32(get(ctx, "T")), H = i32(get(ctx, "H"));
     const Guard guard(r.device());
     Tensor ds0 = state ? at::empty({B, H, HEAD, HEAD}, r.options().dtype(F32)) : Tensor(), d[6];
-    for (Tensor& t : d) t = at::empty(r.sizes(), r.options());
+    for (int i = 0; i < 6; ++i) d[i] = at::empty(x[i].sizes(), r.options());       // (each input may have come in either shape)
     void* st = stream_of(r);
     if (r.scalar_type() == BF)
         ok(rwkv7_statepassing_backward_ex(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]),

@@ -78,3 +78,16 @@ def test_checkpoint_and_saved_tensor_hooks(lib, op):
     got = _grads(out, t)
     assert all(torch.equal(a, b) for a, b in zip(want, got))
     assert count and all(n == 1 for n in count.values()), count
+
+
+@pytest.mark.parametrize("op", ["rwkv7_none", "rwkv7_state", "rwkv7_passing", "rwkv7_passing_f32"])
+def test_rwkv7_gradients_have_the_shapes_of_their_inputs(lib, op):
+    """The functions take r as [B,T,C]; the others may be [B,T,H,64] as well, the same memory."""
+    f, x = _case(op)
+    want = _grads(f(*(t := [z.to(DEV).requires_grad_(True) for z in x])), t)
+    first = len(x) - 6
+    y = [z.view(B, T, H, 64) if i in (first + 1, first + 4) else z for i, z in enumerate(x)]
+    got = _grads(f(*(t := [z.to(DEV).requires_grad_(True) for z in y])), t)
+    n = len(want) - len(x)
+    for a, b, z in zip(want[n:], got[n:], y):
+        assert b.shape == z.shape and torch.equal(a.reshape(z.shape), b)
