@@ -372,17 +372,18 @@ Tensor wkv6_state_op(int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& r
 }
 
 // --------------------------------------------- rwkv7 clamp-w (rwkv7_cuda_benchmark_state_passing.py:75-103, _state.py:75-102, .py:76-100)
-// One body for the three siblings: s0 may be undefined (no state), passing = the final state is an output too.  r..b are
-// [B,T,H,64] or [B,T,H*64] (the same memory); y has the shape `flat` asks for.  The checkpoint tensors `s` and `sa` are scratch
+// One body for the three siblings: s0 may be undefined (no state), passing = the final state is an output too.  r is
+// [B,T,H*64] (flat: the functions) or [B,T,H,64] (the classes), the others either (the same memory); y has the shape of r, with
+// `passing` always [B,T,H*64].  The checkpoint tensors `s` and `sa` are scratch
 // whose layout belongs to the library.  The backward must run with the flags of the forward (the kernel families lay `s` out
 // differently), so they ride on the context.
 variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a,
                         const Tensor& b, int64_t flags, bool passing, bool flat, bool grad) {
     const auto dt = r.scalar_type();
     require(dt == BF || dt == F32, "r.dtype must be bfloat16 or float32, got " + str(dt));
-    require(r.dim() == 3 || r.dim() == 4, "r..b are [B,T,H,64] or [B,T,H*64]");
-    require(r.dim() == 3 ? r.size(2) % HEAD == 0 : r.size(3) == HEAD, "head size must be 64");
-    const int64_t B = r.size(0), T = r.size(1), H = r.dim() == 3 ? r.size(2) / HEAD : r.size(2);
+    require(r.dim() == (flat ? 3 : 4), flat ? "r must be [B,T,H*64]" : "r must be [B,T,H,64]");
+    require(flat ? r.size(2) % HEAD == 0 : r.size(3) == HEAD, "head size must be 64");
+    const int64_t B = r.size(0), T = r.size(1), H = flat ? r.size(2) / HEAD : r.size(2);
     require(T % CHUNK7 == 0, "T must be a multiple of CHUNK_LEN");
     check({{&r, "r"}, {&w, "w"}, {&k, "k"}, {&v, "v"}, {&a, "a"}, {&b, "b"}}, dt, r);
     for (const Tensor* x : {&w, &k, &v, &a, &b}) require(x->numel() == r.numel(), "shape mismatch");
@@ -393,7 +394,7 @@ variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r,
     const Guard guard(r.device());
     const int b_ = i32(B), t_ = i32(T), h_ = i32(H);
     const auto f32 = r.options().dtype(F32);
-    Tensor y = flat ? at::empty({B, T, H * HEAD}, r.options()) : at::empty({B, T, H, HEAD}, r.options());
+    Tensor y = flat || passing ? at::empty({B, T, H * HEAD}, r.options()) : at::empty({B, T, H, HEAD}, r.options());
     Tensor sT = passing ? at::empty({B, H, HEAD, HEAD}, f32) : Tensor();
     void* st = stream_of(r);
     if (!grad && (dt != BF || !(flags & RWKV_FLAG_SWEEPS))) {
@@ -437,8 +438,8 @@ variable_list rwkv7_grads(AutogradContext* ctx, const Tensor& dy_, const Tensor&
 }
 struct Rwkv7Passing : Function<Rwkv7Passing> {
     static variable_list forward(AutogradContext* ctx, const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a,
-                                 const Tensor& b, int64_t flags, bool grad) { return rwkv7_run(ctx, s0, r, w, k, v, a, b, flags, true, true, grad); }
-    static variable_list backward(AutogradContext* ctx, variable_list g) { return rwkv7_grads(ctx, g[0], g[1], true); }
+                                 const Tensor& b, int64_t flags, bool flat, bool grad) { return rwkv7_run(ctx, s0, r, w, k, v, a, b, flags, true, flat, grad); }
+    static variable_list backward(AutogradContext* ctx, variable_list g) { variable_list x = rwkv7_grads(ctx, g[0], g[1], true); x.push_back(NONE); return x; }
 };
 struct Rwkv7State : Function<Rwkv7State> {
     static variable_list forward(AutogradContext* ctx, const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a,
@@ -455,8 +456,8 @@ struct Rwkv7 : Function<Rwkv7> {
         return x;
     }
 };
-std::tuple<Tensor, Tensor> rwkv7_passing_op(const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b, int64_t flags) {
-    variable_list o = Rwkv7Passing::apply(s0, r, w, k, v, a, b, flags, wants_grad({&s0, &r, &w, &k, &v, &a, &b}));
+std::tuple<Tensor, Tensor> rwkv7_passing_op(const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b, int64_t flags, bool flat) {
+    variable_list o = Rwkv7Passing::apply(s0, r, w, k, v, a, b, flags, flat, wants_grad({&s0, &r, &w, &k, &v, &a, &b}));
     return {o[0], o[1]};
 }
 Tensor rwkv7_state_op(const Tensor& s0, const Tensor& r, const Tensor& w, const Tensor& k, const Tensor& v, const Tensor& a, const Tensor& b, int64_t flags, bool flat) {

@@ -19,11 +19,11 @@ class RWKV7_STATE_PASSING_CLAMPW_CUDA_OP(torch.autograd.Function):
 
     @staticmethod
     def apply(s0, r, w, k, v, a, b):
-        return ops().rwkv7_passing(s0, r, w, k, v, a, b, options.current_flags())
+        return ops().rwkv7_passing(s0, r, w, k, v, a, b, options.current_flags(), False)
 
 
 def RWKV7_STATE_PASSING_CLAMPW_CUDA(s0, r, w, k, v, a, b):
-    return ops().rwkv7_passing(s0, r, w, k, v, a, b, options.current_flags())
+    return ops().rwkv7_passing(s0, r, w, k, v, a, b, options.current_flags(), True)
 
 
 class RWKV7_STATE_CLAMPW_CUDA_OP(torch.autograd.Function):

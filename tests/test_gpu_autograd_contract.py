@@ -91,3 +91,17 @@ def test_rwkv7_gradients_have_the_shapes_of_their_inputs(lib, op):
     n = len(want) - len(x)
     for a, b, z in zip(want[n:], got[n:], y):
         assert b.shape == z.shape and torch.equal(a.reshape(z.shape), b)
+
+
+def test_rwkv7_functions_and_classes_take_r_in_their_own_shape(lib):
+    for op, cls in (("rwkv7_none", R.RWKV7_CLAMPW_CUDA_OP), ("rwkv7_state", R.RWKV7_STATE_CLAMPW_CUDA_OP), ("rwkv7_passing", R.RWKV7_STATE_PASSING_CLAMPW_CUDA_OP)):
+        f, x = _case(op)
+        t = [z.to(DEV) for z in x]
+        n = len(t) - 6
+        heads = t[:n] + [z.view(B, T, H, 64) for z in t[n:]]
+        y, z = f(*t), cls.apply(*heads)
+        y, z = (y[0], z[0]) if op == "rwkv7_passing" else (y, z)
+        assert y.shape == (B, T, C) and z.shape == ((B, T, C) if op == "rwkv7_passing" else (B, T, H, 64)) and torch.equal(y, z.view(B, T, C))
+        for call, args in ((f, heads), (cls.apply, t)):
+            with pytest.raises((AssertionError, ValueError)):
+                call(*args)
