@@ -249,7 +249,8 @@ int rwkv_wkv5a_backward_ex(void* stream, int B, int T, int C, int H,
  * matrix cores: one forward, one reverse sweep.
  *   `saved` (*_saved_bytes; 0 for another head size, which these entry points refuse with RWKV_ERR_SHAPE): the forward keeps
  *   the state entering every third (wkv5a: second) chunk of 16 tokens for the backward of the same step; NULL for a forward
- *   without a backward.  `workspace` (*_backward_workspace_bytes): per-batch rows of the parameter gradients.
+ *   without a backward.  `workspace` (*_backward_workspace_bytes): per-batch rows of the parameter gradients.  The raw decays
+ *   (w, w1, w2) may have any alignment.
  * ------------------------------------------------------------------------------------- */
 size_t rwkv_wkv5f32s_saved_bytes(int B, int T, int C, int H);
 int rwkv_wkv5f32s_forward(void* stream, int B, int T, int C, int H,

@@ -777,7 +777,8 @@ size_t rwkv_wkv5as_backward_workspace_bytes(int B, int T, int C, int H) {
 int rwkv_wkv5f32s_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w,
                           const float* u, float* y, void* saved, size_t bytes) {
     if (int e = check(B, T, C, H)) return e;
-    if (int e = check_ptrs({r, k, v, w, u, y})) return e;
+    if (int e = check_ptrs({r, k, v, u, y})) return e;
+    if (int e = check_ptrs({w}, false)) return e;
     if (saved != nullptr && (bytes < saved_bytes<false>(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.saved = static_cast<float*>(saved);
@@ -788,7 +789,8 @@ int rwkv_wkv5f32s_backward(void* stream, int B, int T, int C, int H, const float
                            const float* u, const float* gy, float* gr, float* gk, float* gv, float* gw, float* gu, const void* saved,
                            size_t bytes, void* workspace, size_t workspace_bytes) {
     if (int e = check(B, T, C, H)) return e;
-    if (int e = check_ptrs({r, k, v, w, u, gy, gr, gk, gv, gw, gu})) return e;
+    if (int e = check_ptrs({r, k, v, u, gy, gr, gk, gv, gw, gu})) return e;
+    if (int e = check_ptrs({w}, false)) return e;
     if (saved == nullptr || bytes < saved_bytes<false>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
     if (workspace == nullptr || workspace_bytes < rwkv_wkv5f32s_backward_workspace_bytes(B, T, C, H)) return RWKV_ERR_WORKSPACE;
     float* rows = static_cast<float*>(workspace);
@@ -802,7 +804,8 @@ int rwkv_wkv5f32s_backward(void* stream, int B, int T, int C, int H, const float
 int rwkv_wkv5as_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
                         const float* u1, const float* w2, const float* u2, float* y, void* saved, size_t bytes) {
     if (int e = check(B, T, C, H)) return e;
-    if (int e = check_ptrs({r, k, v, w1, u1, w2, u2, y})) return e;
+    if (int e = check_ptrs({r, k, v, u1, u2, y})) return e;
+    if (int e = check_ptrs({w1, w2}, false)) return e;
     if (saved != nullptr && (bytes < saved_bytes<true>(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w1; p.u = u1; p.w2 = w2; p.u2 = u2; p.y = y;
@@ -815,7 +818,8 @@ int rwkv_wkv5as_backward(void* stream, int B, int T, int C, int H, const float* 
                          float* gw1, float* gu1, float* gw2, float* gu2, const void* saved, size_t bytes, void* workspace,
                          size_t workspace_bytes) {
     if (int e = check(B, T, C, H)) return e;
-    if (int e = check_ptrs({r, k, v, w1, u1, w2, u2, gy, gr, gk, gv, gw1, gu1, gw2, gu2})) return e;
+    if (int e = check_ptrs({r, k, v, u1, u2, gy, gr, gk, gv, gw1, gu1, gw2, gu2})) return e;
+    if (int e = check_ptrs({w1, w2}, false)) return e;
     if (saved == nullptr || bytes < saved_bytes<true>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
     if (workspace == nullptr || workspace_bytes < rwkv_wkv5as_backward_workspace_bytes(B, T, C, H)) return RWKV_ERR_WORKSPACE;
     float* rows = static_cast<float*>(workspace);

@@ -105,3 +105,19 @@ def test_rwkv7_functions_and_classes_take_r_in_their_own_shape(lib):
         for call, args in ((f, heads), (cls.apply, t)):
             with pytest.raises((AssertionError, ValueError)):
                 call(*args)
+
+
+@pytest.mark.parametrize("op", ["wkv5", "wkv5a"])
+def test_fp32_decays_of_any_alignment(lib, op):
+    """A decay may be a view at an odd offset of a larger parameter."""
+    f, x = _case(op)
+    want = _grads(f(*(t := [z.to(DEV).requires_grad_(True) for z in x])), t)
+    t = []
+    for i, z in enumerate(x):
+        z = z.to(DEV)
+        if i in (3, 5):
+            z = torch.cat([z.new_zeros(1), z.reshape(-1)])[1:].view(z.shape)
+            assert z.data_ptr() % 16 == 4
+        t.append(z.requires_grad_(True))
+    got = _grads(f(*t), t)
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
