@@ -129,7 +129,8 @@ int rwkv_wkv4raw_backward(void* stream, int B, int T, int C,
  *   T must be a multiple of 4 (same as the reference); B is unrestricted.
  *   With T % 32 == 0, T <= 1024 and B >= 8 the sums run on the matrix cores with every fp32 operand carried as two fp16
  *   terms (22 mantissa bits, scaled by a power of two per 32 batch rows): errors against fp64 are those of an fp32 loop
- *   (1e-7 of the outputs' scale), but a product is not the bit pattern of the fp32 product.
+ *   (1e-7 of the outputs' scale), but a product is not the bit pattern of the fp32 product.  Other shapes carry an operand as
+ *   three bf16 terms (all 24 bits, fp32's range): every element within the error bound of an fp32 loop.
  * ------------------------------------------------------------------------------------- */
 int rwkv_timex_forward(void* stream, const float* w, const float* k, float* x, float eps, int B, int C, int T);
 int rwkv_timex_backward(void* stream, const float* w, const float* k, const float* gwk,

@@ -5,8 +5,8 @@
 //   gk[b,c,u] =       sum_{t>=u} wr[t-u] g[b,c,t]
 //   gw[b,c,T-1-d] =   sum_{u}    g[b,c,u+d] k[b,c,u]         (per batch; the wrapper sums over b)
 //
-// Three families on fp16 matrix instructions at fp32 accuracy (two fp16 terms per operand): timex_conv_h2 / timex_gw_sum_h2
-// for whole tiles of 32 steps and full batches, timex_conv_any / timex_gw_any for every other length and batch size.
+// Two families on the matrix cores at fp32 accuracy: timex_conv_h2 / timex_gw_sum_h2 (two fp16 terms per operand) for whole tiles
+// of 32 steps and full batches, timex_conv_any / timex_gw_any (three bf16 terms) for every other length and batch size.
 // timex_gw (vector units) makes the per-batch gw of the reference's signature: one workgroup per (b,c) row; a thread owns 4
 // consecutive lags d.
 #include "common.h"
@@ -573,15 +573,27 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // end) read as zeros, of which every row has zb behind it.  The kernel gradient is the same contraction turned round:
 //     gw[lag 32 d + i - j] = sum over the diagonals of M_d[i][j] = sum_columns g[32 a + i] k[32 (a - d) + j],
 // K slots are columns, sixteen an instruction, g and k operands by transposing LDS reads whose lanes point at blocks of their
-// own.  Rows lie in LDS as blocks of 32 + 8 fp16 (80 bytes: 16-byte reads of neighbouring columns fall on different banks if a
-// row has an odd number of blocks), 512 threads, at most 80 KB and 128 registers: two workgroups share a CU, one converts
-// its rows while the other multiplies.  Bound by LDS reads (4 KB per column tile and block lag, and 4 KB for the Toeplitz
-// operand that a wave's two tiles share).  B13 C384 T1500: 58 us a convolution, 101 us the kernel gradient; the vector-unit
-// kernels that these replace took 315 / 286 and, with the sum over the batch, 243 us.
-constexpr int BLK = 40;                // fp16 elements of a block in LDS, 32 of them data
+// own.
+// Operands are THREE bf16 terms, x = h + m + l (each the nearest of what is left: all 24 bits of x), and a product is
+//     x y = h h' + h m' + m h' + m m' + h l' + l h'            (the terms left out are below 2^-24 of the product, 2^-26 rms)
+// with fp32's exponents.  The five small products have accumulators of their own: the sum of the large ones, whose roundings are
+// what is left of an error, rounds once an instruction.  Nothing is scaled, so nothing is scaled and an element's accuracy does not depend on its neighbours: short rows, rows
+// that grow late and batches of unequal rows come out as from an fp32 loop, which two fp16 terms under a common power of two
+// (half the products, 58 and 101 us where these take 95 and 111) do not give.  A unit with an element that is no number, infinite or beyond
+// bf16's largest is done by such a loop (a matrix product would carry it to earlier steps: zero times infinity).
+// Rows lie in LDS as blocks of 32 + 8 terms (80 bytes: 16-byte reads of neighbouring columns fall on different banks if a
+// row has an odd number of blocks), 512 threads, 128 registers, and up to T = 2900 (gradient) and 3360 at most 80 KB: two
+// workgroups share a CU, one converts its rows while the other multiplies; longer rows take a CU each.  B13 C384 T1500:
+// 95 us a convolution, 111 us the kernel gradient, relative errors 1.8e-7 and 1.0e-7; the fp32 loops on the vector units that
+// these replace took 315 / 286 and, with the sum over the batch, 243 us, with 5.6e-7.
+constexpr int BLK = 40;                // elements of a block in LDS, 32 of them data
 constexpr int LDS_ANY = 80 * 1024;     // two workgroups per CU
 constexpr int PZ = 32;                 // zeros in front of the forward line (lags beyond the last tap, of rows past T)
 constexpr int CONV_PIECES = 8, GW_PIECES = 4;   // 16-byte pieces a thread stages (per tensor): Bg nt 8 / 512 at most
+constexpr int NPL = 3;                 // planes: terms of an operand
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+// the six products of two operands, the small ones first
+constexpr int TERM_A[6] = {2, 0, 1, 1, 0, 0}, TERM_B[6] = {0, 2, 1, 0, 1, 0};
 
 struct AnyGeom {
     int nt, bg, zb, pitch;             // blocks of a row, rows of a unit, zero blocks behind a row, nt + zb (odd)
@@ -595,42 +607,69 @@ inline AnyGeom any_geom(int T, int bg, int span) {        // span: how many bloc
     q.pitch = q.nt + q.zb;
     return q;
 }
-inline size_t conv_any_lds(const AnyGeom& q) { return (2 * q.plane() + 4 * static_cast<size_t>(h2_line_len(32 * q.nt))) * 2 + 64; }
-inline size_t gw_any_lds(const AnyGeom& q) { return 4 * q.plane() * 2 + static_cast<size_t>(q.nt) * 256 + 64; }
+inline size_t conv_any_lds(const AnyGeom& q) { return (NPL * q.plane() + 2 * NPL * static_cast<size_t>(h2_line_len(32 * q.nt))) * 2 + 16; }
+inline size_t gw_any_lds(const AnyGeom& q) { return 2 * NPL * q.plane() * 2 + static_cast<size_t>(q.nt) * 256 + 16; }
 
+// an element that three bf16 terms do not carry: its nearest bf16 is not finite
+DEVINL bool beyond_terms(float x) { return (__float_as_uint(x) & 0x7fffffffu) >= 0x7f7f8000u; }
+DEVINL bool beyond_terms(const float4& v) { return beyond_terms(v.x) | beyond_terms(v.y) | beyond_terms(v.z) | beyond_terms(v.w); }
+// v = p[0] + p[1] + p[2], four elements as packed pairs
+struct B3x4 { uint2 p[NPL]; };
+DEVINL B3x4 split3x4(float4 v) {
+    B3x4 r;
+#pragma unroll
+    for (int z = 0; z < NPL; ++z) {
+        r.p[z] = make_uint2(pack_bf2(v.x, v.y), pack_bf2(v.z, v.w));
+        v.x -= bf_lo(r.p[z].x); v.y -= bf_hi(r.p[z].x); v.z -= bf_lo(r.p[z].y); v.w -= bf_hi(r.p[z].y);
+    }
+    return r;
+}
+// whether any thread of the workgroup says so; red: one word, zeroed by thread 0 at least one barrier before; takes one barrier
+DEVINL bool any_thread(bool x, int* red) {
+    if (__ballot(x) != 0ull && (threadIdx.x & 63) == 0) *red = 1;
+    __syncthreads();
+    return *red != 0;
+}
+
+// threadIdx.x, hidden from the optimiser: it would keep the addresses of every piece across the loops of timex_gw_any, in scratch
+DEVINL int own_thread() {
+    int t = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(t));
+    return t;
+}
 // rows b0 .. of channel c as 16-byte pieces: piece idx = tid + 512 i <-> (row, four steps)
 template <int NP> struct Stager {
     float4 x[NP];
     DEVINL void fetch(const float* __restrict__ in, const AnyGeom& q, int c, int b0, int B, int C, int T) {
-        const int per = 8 * q.nt, total = q.bg * per;
+        const int per = 8 * q.nt, total = q.bg * per, tid = own_thread();
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
             x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            const int idx = static_cast<int>(threadIdx.x) + TXT * i;
+            const int idx = tid + TXT * i;
             if (idx < total) {
                 const int b = idx / per, t = 4 * (idx - b * per);
                 if (b0 + b < B && t < T) x[i] = *reinterpret_cast<const float4*>(in + (static_cast<size_t>(b0 + b) * C + c) * T + t);
             }
         }
     }
-    DEVINL float largest() const {
-        float m = 0.f;
+    DEVINL bool beyond() const {
+        bool on = false;
 #pragma unroll
-        for (int i = 0; i < NP; ++i) m = max_abs4(m, x[i]);
-        return wave_max(m);
+        for (int i = 0; i < NP; ++i) on |= beyond_terms(x[i]);
+        return on;
     }
-    DEVINL void store(uint16_t* rp, const AnyGeom& q, float up) const {
-        const int per = 8 * q.nt, total = q.bg * per;
+    DEVINL void store(uint16_t* rp, const AnyGeom& q) const {
+        const int per = 8 * q.nt, total = q.bg * per, tid = own_thread();
         const size_t pl = q.plane();
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-            const int idx = static_cast<int>(threadIdx.x) + TXT * i;
+            const int idx = tid + TXT * i;
             if (idx < total) {
                 const int b = idx / per, r = idx - b * per;
                 uint16_t* d = rp + (q.zb + b * q.pitch + (r >> 3)) * BLK + 4 * (r & 7);
-                const H2x4 y = split2x4(x[i], up);
-                *reinterpret_cast<uint2*>(d) = y.h;
-                *reinterpret_cast<uint2*>(d + pl) = y.l;
+                const B3x4 y = split3x4(x[i]);
+#pragma unroll
+                for (int p = 0; p < NPL; ++p) *reinterpret_cast<uint2*>(d + p * pl) = y.p[p];
             }
         }
     }
@@ -642,8 +681,8 @@ DEVINL void zero_blocks(uint16_t* rp, const AnyGeom& q) {
     for (int i = threadIdx.x; i < n; i += TXT) {
         const int blk = i / (BLK / 8), e = i - blk * (BLK / 8), row = blk / q.zb, z = blk - row * q.zb;      // row 0: the front
         uint16_t* d = rp + (row * q.pitch + z) * BLK + 8 * e;
-        *reinterpret_cast<uint4*>(d) = make_uint4(0, 0, 0, 0);
-        *reinterpret_cast<uint4*>(d + pl) = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int p = 0; p < NPL; ++p) *reinterpret_cast<uint4*>(d + p * pl) = make_uint4(0, 0, 0, 0);
     }
 }
 
@@ -652,44 +691,49 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
                                                          float eps, int B, int C, int T, int ng, const AnyGeom q) {
     extern __shared__ __align__(16) float lds[];
     const int Tp = 32 * q.nt, xl = h2_line_len(Tp), plane = static_cast<int>(q.plane());
-    uint16_t* rp = reinterpret_cast<uint16_t*>(lds);                    // [2][plane]
-    uint16_t* al = rp + 2 * plane;                                      // [2 planes][2 copies][xl]
-    float* red = reinterpret_cast<float*>(al + 4 * xl);                 // [2][8]
+    uint16_t* rp = reinterpret_cast<uint16_t*>(lds);                    // [NPL][plane]
+    uint16_t* al = rp + NPL * plane;                                    // [NPL planes][2 copies][xl]
+    int* red = reinterpret_cast<int*>(al + 2 * NPL * xl);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, kh = lane >> 5;
     const int c = blockIdx.x / ng, b0 = (blockIdx.x - c * ng) * q.bg;
-    float unscale;
     {
         Stager<CONV_PIECES> st;
         st.fetch(in, q, c, b0, B, C, T);
-        float wr[T_ANY / TXT], mw = 0.f;
+        float wr[T_ANY / TXT];
+        bool beyond = st.beyond();
 #pragma unroll
         for (int z = 0; z < T_ANY / TXT; ++z) {
             const int tau = z * TXT + tid;
             wr[z] = tau < T ? w[static_cast<size_t>(c) * T + tau] : 0.f;
-            mw = fmaxf(mw, fabsf(wr[z]));
+            beyond |= beyond_terms(wr[z]);
         }
-        for (int i = tid; i < 2 * xl; i += TXT) reinterpret_cast<uint32_t*>(al)[i] = 0;
+        for (int i = tid; i < NPL * xl; i += TXT) reinterpret_cast<uint32_t*>(al)[i] = 0;
         zero_blocks(rp, q);
-        const float mx = st.largest();
-        mw = wave_max(mw);
-        if (lane == 0) { red[wv] = mx; red[8 + wv] = mw; }
+        if (tid == 0) *red = 0;
         __syncthreads();
-        float ax = 0.f, aw = 0.f;
-#pragma unroll
-        for (int i = 0; i < TXW; ++i) { ax = fmaxf(ax, red[i]); aw = fmaxf(aw, red[8 + i]); }
-        const Pow2 sx = scale_for(ax), sw = scale_for(aw);
-        unscale = sx.down * sw.down;
-        st.store(rp, q, sx.up);
+        if (any_thread(beyond, red)) {
+            for (int i = tid; i < q.bg * T; i += TXT) {
+                const int b = i / T, t = i - b * T;
+                if (b0 + b >= B) break;
+                const size_t row = (static_cast<size_t>(b0 + b) * C + c) * T;
+                const float *x = in + row, *wl = w + static_cast<size_t>(c) * T + T - 1;       // wl[-lag]
+                float acc = 0.f;
+                if constexpr (MIRROR) { for (int s = t; s < T; ++s) acc = fmaf(wl[t - s], x[s], acc); }
+                else { for (int s = 0; s <= t; ++s) acc = fmaf(wl[s - t], x[s], acc); }
+                out[row + t] = MIRROR ? acc : acc + eps;
+            }
+            return;
+        }
+        st.store(rp, q);
         // tap tau (lag T-1-tau) sits at line position PZ + tau (forward) or 31 + lag (mirror); the rest is zero
 #pragma unroll
         for (int z = 0; z < T_ANY / TXT; ++z) {
             const int tau = z * TXT + tid;
             if (tau < T) {
-                const H2 a = split2(wr[z] * sw.up);
+                const B3x4 a = split3x4(make_float4(wr[z], 0.f, 0.f, 0.f));
                 const int pos = MIRROR ? 31 + (T - 1 - tau) : PZ + tau;
-                const uint16_t pl[2] = {a.h, a.l};
 #pragma unroll
-                for (int p = 0; p < 2; ++p) { al[(2 * p) * xl + pos] = pl[p]; al[(2 * p + 1) * xl + pos - 1] = pl[p]; }
+                for (int p = 0; p < NPL; ++p) { al[(2 * p) * xl + pos] = static_cast<uint16_t>(a.p[p].x); al[(2 * p + 1) * xl + pos - 1] = static_cast<uint16_t>(a.p[p].x); }
             }
         }
         __syncthreads();
@@ -709,37 +753,36 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
     }
     const int start = (MIRROR ? 31 - ln : PZ + T - 1 - ln) + 8 * kh;    // forward: line[start - 32 d + j], mirror: line[start + 32 d + j]
     const uint32_t* ap = reinterpret_cast<const uint32_t*>(al + (start & 1) * xl) + (start >> 1);
-    f32x16 acc[2];
+    f32x16 acc[2], low[2];          // the products of the first terms, which are what rounds; the other five
 #pragma unroll
     for (int z = 0; z < 2; ++z)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[z][v] = 0.f;
+        for (int v = 0; v < 16; ++v) { acc[z][v] = 0.f; low[z][v] = 0.f; }
     auto run = [&](auto NTL, const int d0, const int d1) __attribute__((always_inline)) {
         constexpr int NT_ = decltype(NTL)::value;
         for (int d = d0; d < d1; ++d) {
             const int o = MIRROR ? d : -d;
-            f16x8 fa[2][2], fb[NT_][2][2];
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
+            for (int ks = 0; ks < 2; ++ks) {
+                bf16x8 fa[NPL], fb[NT_][NPL];
 #pragma unroll
-                for (int p = 0; p < 2; ++p) {
+                for (int p = 0; p < NPL; ++p) {
                     const uint32_t* a4 = ap + 16 * o + 8 * ks + p * xl;          // a plane is 2 xl elements = xl dwords
-                    fa[ks][p] = __builtin_bit_cast(f16x8, make_uint4(a4[0], a4[1], a4[2], a4[3]));
+                    fa[p] = __builtin_bit_cast(bf16x8, make_uint4(a4[0], a4[1], a4[2], a4[3]));
                 }
 #pragma unroll
-            for (int z = 0; z < NT_; ++z)
+                for (int z = 0; z < NT_; ++z)
 #pragma unroll
-                for (int ks = 0; ks < 2; ++ks)
+                    for (int p = 0; p < NPL; ++p)
+                        fb[z][p] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(bp[z] + BLK * o + 16 * ks + p * plane));
 #pragma unroll
-                    for (int p = 0; p < 2; ++p)
-                        fb[z][ks][p] = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4*>(bp[z] + BLK * o + 16 * ks + p * plane));
+                for (int term = 0; term < 6; ++term)
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                for (int term = 0; term < 3; ++term)
-#pragma unroll
-                    for (int z = 0; z < NT_; ++z)
-                        acc[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[ks][term == 2], fb[z][ks][term == 1], acc[z], 0, 0, 0);
+                    for (int z = 0; z < NT_; ++z) {
+                        f32x16& sum = term == 5 ? acc[z] : low[z];
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[TERM_A[term]], fb[z][TERM_B[term]], sum, 0, 0, 0);
+                    }
+            }
         }
     };
     run(std::integral_constant<int, 2>{}, 0, nd[1]);
@@ -752,17 +795,17 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
 #pragma unroll
             for (int v4 = 0; v4 < 4; ++v4) {
                 const int t = 32 * a + 8 * v4 + 4 * kh;
-                const float e = MIRROR ? 0.f : eps;
-                if (t < T)
-                    *reinterpret_cast<float4*>(o + t) = make_float4(fmaf(acc[z][4 * v4], unscale, e), fmaf(acc[z][4 * v4 + 1], unscale, e),
-                                                                    fmaf(acc[z][4 * v4 + 2], unscale, e), fmaf(acc[z][4 * v4 + 3], unscale, e));
+                float x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = (acc[z][4 * v4 + e] + low[z][4 * v4 + e]) + (MIRROR ? 0.f : eps);
+                if (t < T) *reinterpret_cast<float4*>(o + t) = make_float4(x[0], x[1], x[2], x[3]);
             }
         }
     }
 }
 
 // the sum of a finished 32 x 32 tile of lag tile d over its diagonals, into diag[64 d ..] (entry l: lag 32 d + l - 31)
-DEVINL void add_diagonals(float* diag, const f32x16& acc, int d, float unscale, int ln, int kh) {
+DEVINL void add_diagonals(float* diag, const f32x16& acc, int d, int ln, int kh) {
     float pos = 0.f, neg = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
@@ -772,8 +815,8 @@ DEVINL void add_diagonals(float* diag, const f32x16& acc, int d, float unscale, 
     }
     pos += __shfl_xor(pos, 32, 64);
     neg += __shfl_xor(neg, 32, 64);
-    if (kh == 0) diag[64 * d + 31 + ln] += pos * unscale;
-    else if (ln >= 1) diag[64 * d + ln - 1] += neg * unscale;
+    if (kh == 0) diag[64 * d + 31 + ln] += pos;
+    else if (ln >= 1) diag[64 * d + ln - 1] += neg;
 }
 
 // one workgroup: channel c = blockIdx.x, batch groups blockIdx.y, blockIdx.y + gridDim.y, ...; out[blockIdx.y][c][T]
@@ -781,10 +824,10 @@ __global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__
                                                        int B, int C, int T, int ng, const AnyGeom q) {
     extern __shared__ __align__(16) float lds[];
     const int plane = static_cast<int>(q.plane());
-    uint16_t* gp = reinterpret_cast<uint16_t*>(lds);            // [2][plane]
-    uint16_t* kp = gp + 2 * plane;                              // [2][plane]
-    float* diag = reinterpret_cast<float*>(kp + 2 * plane);     // [nt][64]
-    float* red = diag + 64 * q.nt;                              // [2][8]
+    uint16_t* gp = reinterpret_cast<uint16_t*>(lds);            // [NPL][plane]
+    uint16_t* kp = gp + NPL * plane;                            // [NPL][plane]
+    float* diag = reinterpret_cast<float*>(kp + NPL * plane);   // [nt][64]
+    int* red = reinterpret_cast<int*>(diag + 64 * q.nt);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ln = lane & 31, kh = lane >> 5, l16 = lane & 15;
     const int c = blockIdx.x, ncol = q.nt * q.bg, nsteps = (ncol + 15) >> 4;
@@ -792,37 +835,42 @@ __global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__
     zero_blocks(gp, q);
     zero_blocks(kp, q);
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)gp));
-    const uint32_t k_off = 4u * static_cast<uint32_t>(plane), pl_b = 2u * static_cast<uint32_t>(plane);
+    const uint32_t k_off = 2u * NPL * static_cast<uint32_t>(plane), pl_b = 2u * static_cast<uint32_t>(plane);
     const int db = 16 % q.bg, step_b = 2 * BLK * (db * q.pitch + 16 / q.bg), wrap_b = 2 * BLK * (1 - q.bg * q.pitch);
     for (int grp = blockIdx.y; grp < ng; grp += gridDim.y) {
         const int b0 = grp * q.bg;
-        float unscale;
         {
             Stager<GW_PIECES> sg, sk;
             sg.fetch(g, q, c, b0, B, C, T);
             sk.fetch(k, q, c, b0, B, C, T);
-            const float mg = sg.largest(), mk = sk.largest();
-            if (lane == 0) { red[wv] = mg; red[8 + wv] = mk; }
-            __syncthreads();               // (everybody is also done with the group before)
-            float ag = 0.f, ak = 0.f;
-#pragma unroll
-            for (int i = 0; i < TXW; ++i) { ag = fmaxf(ag, red[i]); ak = fmaxf(ak, red[8 + i]); }
-            const Pow2 ug = scale_for(ag), uk = scale_for(ak);
-            unscale = ug.down * uk.down;
-            sg.store(gp, q, ug.up);
-            sk.store(kp, q, uk.up);
+            __syncthreads();               // everybody is done with the group before
+            if (tid == 0) *red = 0;
+            __syncthreads();
+            if (any_thread(sg.beyond() | sk.beyond(), red)) {
+                for (int lag = tid; lag < T; lag += TXT) {
+                    float acc = 0.f;
+                    for (int b = b0; b < B && b < b0 + q.bg; ++b) {
+                        const size_t row = (static_cast<size_t>(b) * C + c) * T;
+                        for (int u = 0; u + lag < T; ++u) acc = fmaf(g[row + u + lag], k[row + u], acc);
+                    }
+                    diag[64 * (lag >> 5) + 31 + (lag & 31)] += acc;
+                }
+                continue;
+            }
+            sg.store(gp, q);
+            sk.store(kp, q);
             __syncthreads();
         }
-        // lag tile d takes the columns from d Bg on; tiles in the order of decreasing work go to the waves back and forth, four at
+        // lag tile d takes the columns from d Bg on; tiles in the order of decreasing work go to the waves back and forth, two at
         // a time (their g operand is the same)
-        for (int set = 0; 32 * set < q.nt; ++set) {
-            const int dd[4] = {32 * set + wv, 32 * set + 15 - wv, 32 * set + 16 + wv, 32 * set + 31 - wv};
+        for (int set = 0; 16 * set < q.nt; ++set) {
+            const int dd[2] = {16 * set + wv, 16 * set + 15 - wv};
             if (dd[0] >= q.nt) break;
-            f32x16 acc[4];
+            f32x16 acc[2], low[2];          // as in timex_conv_any
 #pragma unroll
-            for (int z = 0; z < 4; ++z)
+            for (int z = 0; z < 2; ++z)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[z][v] = 0.f;
+                for (int v = 0; v < 16; ++v) { acc[z][v] = 0.f; low[z][v] = 0.f; }
             int s = (dd[0] * q.bg) >> 4;
             // this lane's columns in the two transposing reads of a step: K slots 8 kh + (l16 >> 2) and four on
             int bb[2];
@@ -837,28 +885,26 @@ __global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__
                 const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_ptr)(at[0] + o));
                 const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_ptr)(at[1] + o));
                 const uint2 x = __builtin_bit_cast(uint2, lo), y = __builtin_bit_cast(uint2, hi);
-                return __builtin_bit_cast(f16x8, make_uint4(x.x, x.y, y.x, y.y));
+                return __builtin_bit_cast(bf16x8, make_uint4(x.x, x.y, y.x, y.y));
             };
             auto run = [&](auto NTL, const int end) __attribute__((always_inline)) {
                 constexpr int NT_ = decltype(NTL)::value;
                 for (; s < end; ++s) {
-                    f16x8 fg[2];
+                    bf16x8 fg[NPL];
 #pragma unroll
-                    for (int p = 0; p < 2; ++p) fg[p] = operand(p * pl_b);
+                    for (int p = 0; p < NPL; ++p) fg[p] = operand(p * pl_b);
+                    bf16x8 fk[NT_][NPL];
 #pragma unroll
-                    for (int z0 = 0; z0 < NT_; z0 += 2) {             // (two at a time: the four tiles' operands together would not fit 128 registers)
-                        f16x8 fk[2][2];
+                    for (int z = 0; z < NT_; ++z)
 #pragma unroll
-                        for (int z = z0; z < NT_ && z < z0 + 2; ++z)
+                        for (int p = 0; p < NPL; ++p) fk[z][p] = operand(k_off + p * pl_b - 2u * BLK * static_cast<uint32_t>(dd[z]));
 #pragma unroll
-                            for (int p = 0; p < 2; ++p) fk[z - z0][p] = operand(k_off + p * pl_b - 2u * BLK * static_cast<uint32_t>(dd[z]));
+                    for (int term = 0; term < 6; ++term)
 #pragma unroll
-                        for (int term = 0; term < 3; ++term)
-#pragma unroll
-                            for (int z = z0; z < NT_ && z < z0 + 2; ++z)
-                                acc[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fg[term == 2], fk[z - z0][term == 1], acc[z], 0, 0, 0);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
+                        for (int z = 0; z < NT_; ++z) {
+                            f32x16& sum = term == 5 ? acc[z] : low[z];
+                            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg[TERM_A[term]], fk[z][TERM_B[term]], sum, 0, 0, 0);
+                        }
 #pragma unroll
                     for (int z = 0; z < 2; ++z) {
                         at[z] += step_b; bb[z] += db;
@@ -866,14 +912,11 @@ __global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__
                     }
                 }
             };
-            auto from = [&](const int z) { return dd[z] < q.nt ? (dd[z] * q.bg) >> 4 : nsteps; };
-            run(std::integral_constant<int, 1>{}, from(1));
-            run(std::integral_constant<int, 2>{}, from(2));
-            run(std::integral_constant<int, 3>{}, from(3));
-            run(std::integral_constant<int, 4>{}, nsteps);
+            run(std::integral_constant<int, 1>{}, dd[1] < q.nt ? (dd[1] * q.bg) >> 4 : nsteps);
+            run(std::integral_constant<int, 2>{}, nsteps);
 #pragma unroll
-            for (int z = 0; z < 4; ++z)
-                if (dd[z] < q.nt) add_diagonals(diag, acc[z], dd[z], unscale, ln, kh);     // a lag tile belongs to one wave
+            for (int z = 0; z < 2; ++z)
+                if (dd[z] < q.nt) add_diagonals(diag, acc[z] + low[z], dd[z], ln, kh);     // a lag tile belongs to one wave
         }
     }
     __syncthreads();
@@ -895,8 +938,9 @@ __global__ __launch_bounds__(256) void timex_add_parts(const float4* __restrict_
     out[i] = a;
 }
 
-// Batch rows of a unit.  Convolution: what finishes first by a count of matrix clocks (48 per column tile and block lag on a
-// CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (two a wave) and 80 KB.
+// Batch rows of a unit.  Convolution: what finishes first by a count of matrix clocks (96 per column tile and block lag on a
+// CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (two a wave) and 80 KB
+// (a single row may have more).
 AnyGeom conv_any_geom(int B, int C, int T) {
     AnyGeom best{};
     double cost = 1e300;
@@ -907,7 +951,7 @@ AnyGeom conv_any_geom(int B, int C, int T) {
         long long pairs = 0;
         for (int t = 0; t < ntile; ++t) pairs += (32 * t + 31 < ncol ? 32 * t + 31 : ncol - 1) / bg + 1;
         const long long units = static_cast<long long>(C) * ((B + bg - 1) / bg);
-        const double x = static_cast<double>((units + 2 * NCU - 1) / (2 * NCU)) * (48.0 * pairs + 0.1 * bg * T + 3000.0);
+        const double x = static_cast<double>((units + 2 * NCU - 1) / (2 * NCU)) * (96.0 * pairs + 0.15 * bg * T + 3000.0);
         if (x < cost) { cost = x; best = q; }
     }
     return best;

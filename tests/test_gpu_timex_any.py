@@ -2,8 +2,9 @@
 oracle: one block of steps, a block and a piece, odd numbers of blocks, the longest sequence, batches of one row up to more than
 one unit, batch groups that are summed by a second kernel and ones that are not.
 
-Tolerance: the fp32 ops' bar of 1e-5.  An operand keeps 22 bits (a product 2^-21), sums are fp32: n products leave about
-sqrt(n) 2^-24 + 2^-21 of their scale, 1e-6 at n = 4096 x 33."""
+Tolerance: the fp32 ops' bar of 1e-5, and element by element the bound of an fp32 loop: n products leave at most n 2^-24 of the
+sum of their magnitudes.  An operand keeps its 24 bits, a product loses less than 2^-23, and a matrix instruction adds sixteen products
+at a time in six parts: fewer roundings than the loop has."""
 import pytest
 import torch
 
@@ -52,7 +53,7 @@ def test_reference_signature_gives_per_batch_kernel_gradients(lib):
 
 
 def test_rows_of_very_different_size(lib):
-    """A unit shares one power of two: the small rows of a unit keep their accuracy down to 2^-28 of its largest element."""
+    """The rows of a unit do not meet."""
     B, C, T = 6, 2, 500
     w, k, g = synth.timex_inputs(B, C, T, seed=4)
     scale = torch.tensor([1.0, 1e-4, 1e3, 1e-2, 1.0, 1e-3]).view(B, 1, 1)
@@ -62,3 +63,58 @@ def test_rows_of_very_different_size(lib):
     x.backward((g * scale).to(DEV))
     for b in range(B):
         assert max_rel_to_peak(out[b], x[b].detach().double().cpu()) <= 1e-5 and max_rel_to_peak(gk[b], t[1].grad[b].double().cpu()) <= 1e-5, b
+
+
+def _abs_sums(w, k, g, B, C, T):
+    """What the fp32 bound is taken of, and how many products each sum has."""
+    out, gw, gk = OT.grads(w.abs(), k.abs(), g.abs(), B, C, T)
+    n = torch.arange(1, T + 1, dtype=torch.float64)
+    return (out, n), (gw, B * n), (gk, n.flip(0))
+
+
+@pytest.mark.parametrize("spike", [None, 1e6, 3.4e38])
+@pytest.mark.parametrize("B,T", [(3, 4), (1, 36), (3, 60), (2, 500), (5, 1500), (2, 4096)])
+def test_every_element_within_the_bound_of_an_fp32_loop(lib, B, T, spike):
+    """Also in rows that are small until one large element (beyond bf16's range, too), which the elements before it do not see."""
+    C = 2
+    print(f"\ntimex any bound B={B} T={T} spike={spike}", flush=True)
+    w, k, g = (x.clamp(-0.9, 0.9) for x in synth.timex_inputs(B, C, T, seed=3 * B + T))
+    if spike is not None:
+        m = T // 2
+        k[:, :, :m] *= 1e-7
+        k[0, :, m] = spike              # (in one row: its product with |w|, |g| <= 0.9 is below fp32's largest number, that of three rows is not)
+        g[:, :, m + 1:] *= 1e-7
+    ref = OT.grads(w, k, g, B, C, T)
+    t = [x.to(DEV).requires_grad_(True) for x in (w, k)]
+    x = depthwise_conv1d.RUN_CUDA(*t, B, C, T, 0.0)
+    x.backward(g.to(DEV))
+    for name, a, got, (mag, n) in zip(("x", "gw", "gk"), ref, (x, t[0].grad, t[1].grad), _abs_sums(w, k, g, B, C, T)):
+        worst = ((got.detach().double().cpu() - a).abs() / ((n + 4) * 2.0 ** -24 * mag + 1e-38)).max().item()
+        print(f"  {name}: worst element at {worst:.3f} of the bound", flush=True)
+        assert worst <= 1, name
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("T", [60, 1500])
+def test_an_element_that_is_no_number_stays_where_it_acts(lib, T, bad):
+    """Not in other rows, in earlier outputs, or (mirrored) in later gradients."""
+    B, C = 5, 2
+    t0, t1 = T // 2 + 3, T // 3
+    w, k, g = synth.timex_inputs(B, C, T, seed=T)
+    kb, gb = k.clone(), g.clone()
+    kb[1, 0, t0] = bad
+    gb[3, 1, t1] = bad
+    ref = OT.grads(w, k, g, B, C, T)
+    t = [x.to(DEV).requires_grad_(True) for x in (w, kb)]
+    x = depthwise_conv1d.RUN_CUDA(*t, B, C, T, 0.0)
+    x.backward(gb.to(DEV))
+    x, gw, gk = x.detach().double().cpu(), t[0].grad.double().cpu(), t[1].grad.double().cpu()
+    hit_x = torch.zeros(B, C, T, dtype=torch.bool)
+    hit_x[1, 0, t0:] = True
+    hit_k = torch.zeros(B, C, T, dtype=torch.bool)
+    hit_k[3, 1, :t1 + 1] = True
+    lag = torch.arange(T - 1, -1, -1)
+    hit_w = torch.stack([lag <= T - 1 - t0, lag <= t1])
+    for name, a, got, hit in (("x", ref[0], x, hit_x), ("gw", ref[1], gw, hit_w), ("gk", ref[2], gk, hit_k)):
+        assert torch.equal(~torch.isfinite(got), hit), name
+        assert max_rel_to_peak(a[~hit], got[~hit]) <= 1e-5, name
