@@ -14,6 +14,7 @@ build() compiles with torch.utils.cpp_extension (the same route as the reference
 csrc/autograd.cpp, in the same extension, holds the operators as C++ autograd functions (`ext.ops.*`): what the classes of
 this package's operator modules call.
 """
+import hashlib
 import importlib.machinery
 import importlib.util
 import os
@@ -28,7 +29,18 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 SO_PATH = os.path.join(_HERE, NAME + ".so")
 _BUILD_DIR = os.path.join(_HERE, "build", NAME)
 
+_SOURCES = [os.path.join(_HERE, "csrc", f) for f in ("binding.cpp", "autograd.cpp")]
+
 _ext = None
+
+
+def source_hash():
+    """Digest of what the extension is compiled from; the extension carries the one it was compiled with."""
+    h = hashlib.sha256()
+    for path in _SOURCES + [os.path.join(os.path.dirname(_HERE), "include", "rwkv_hip.h")]:
+        with open(path, "rb") as f:
+            h.update(os.path.basename(path).encode() + b"\0" + f.read())
+    return h.hexdigest()
 
 
 def _compile(verbose):
@@ -39,9 +51,9 @@ def _compile(verbose):
     rocm = os.environ.get("ROCM_HOME", "/opt/rocm")
     cpp_extension.load(
         name=NAME,
-        sources=[os.path.join(_HERE, "csrc", f) for f in ("binding.cpp", "autograd.cpp")],
+        sources=_SOURCES,
         extra_include_paths=[os.path.join(os.path.dirname(_HERE), "include"), os.path.join(rocm, "include")],
-        extra_cflags=["-O2", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"],
+        extra_cflags=["-O2", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-DRWKV_BINDING_SOURCE_HASH={source_hash()}"],
         # the dollar signs survive ninja and the shell as a literal $ORIGIN: the extension finds librwkv_hip.so beside itself
         extra_ldflags=[f"-L{_HERE}", "-lrwkv_hip", "-Wl,-rpath,\\$$ORIGIN:\\$$ORIGIN/../..", f"-L{torch_lib}", "-lc10_hip", "-ltorch_hip",
                        f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64"],
@@ -67,6 +79,18 @@ def build(verbose=False):
     return SO_PATH
 
 
+def _check(mod):
+    """Every operator's host code is in the extension: one built from other sources than those beside it would run yesterday's
+    checks, workspace sizes and saved tensors with today's kernels, and one built against another version of the C ABI would
+    resolve its symbols lazily and fail, or misbehave, at call time."""
+    have, want = getattr(mod, "abi_version", None), _lib.load().rwkv_abi_version()
+    if have != want:
+        raise RuntimeError(f"{SO_PATH} was built against ABI version {have}, librwkv_hip.so is version {want}: "
+                           "rebuild it (rwkv_cuda_amd.binding.build())")
+    if getattr(mod, "source_hash", None) != source_hash():
+        raise RuntimeError(f"{SO_PATH} was built from different sources: rebuild it (rwkv_cuda_amd.binding.build())")
+
+
 def load():
     """Import the in-tree extension (registers the torch.ops libraries as a side effect)."""
     global _ext
@@ -83,11 +107,7 @@ def load():
     spec = importlib.util.spec_from_loader(NAME, loader)
     mod = importlib.util.module_from_spec(spec)
     loader.exec_module(mod)
-    # a shim built against another version of the C ABI would resolve its symbols lazily and fail, or misbehave, at call time
-    have, want = getattr(mod, "abi_version", None), _lib.load().rwkv_abi_version()
-    if have != want:
-        raise RuntimeError(f"{SO_PATH} was built against ABI version {have}, librwkv_hip.so is version {want}: "
-                           "rebuild it (rwkv_cuda_amd.binding.build())")
+    _check(mod)
     sys.modules[NAME] = mod
     _ext = mod
     return mod

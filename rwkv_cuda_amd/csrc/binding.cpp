@@ -319,6 +319,9 @@ void bind_autograd(pybind11::module_& m);        // autograd.cpp: submodule `ops
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     // the ABI this shim was compiled against; binding.load() compares it with the library's
     m.attr("abi_version") = RWKV_ABI_VERSION;
+#define RWKV_TEXT_(x) #x
+#define RWKV_TEXT(x) RWKV_TEXT_(x)
+    m.attr("source_hash") = RWKV_TEXT(RWKV_BINDING_SOURCE_HASH);      // binding.py compares it with the sources beside the extension
     auto sub = [&](const char* name, auto fwd, auto bwd) {
         auto s = m.def_submodule(name);
         s.def("forward", fwd);

@@ -102,3 +102,18 @@ def test_reference_style_extension_loads_and_registers_its_ops(lib):
     c = torch.zeros(4)
     with pytest.raises(RuntimeError, match="HIP device"):
         ext.wkv.forward(1, 1, 4, c, c, c, c, c)
+
+
+def test_extension_from_other_sources_is_refused(lib):
+    """Every operator's host code is in the extension, so an old one beside new sources may not load: not one without a digest,
+    not one with another."""
+    from types import SimpleNamespace
+
+    from rwkv_cuda_amd import binding
+    mod = binding.load()
+    assert mod.source_hash == binding.source_hash() and len(mod.source_hash) == 64
+    binding._check(mod)
+    abi = lib.rwkv_abi_version()
+    for old in (SimpleNamespace(abi_version=abi), SimpleNamespace(abi_version=abi, source_hash="0" * 64)):
+        with pytest.raises(RuntimeError, match="different sources"):
+            binding._check(old)
