@@ -365,27 +365,21 @@ def make_rwkv7(dev, fp32=False):
         st = s0
         for i in range(4):
             rr, ww, kk, vv, aa, bb, _ = seg[i]
-            if fp32:
-                call("rwkv7_statepassing_forward_f32", dev, B, TS, H, st, rr, ww, kk, vv, aa, bb, ys[i], sTs[i], ss[i], sas[i])
-            else:
-                call("rwkv7_statepassing_forward_ex", dev, B, TS, H, st, rr, ww, kk, vv, aa, bb, ys[i], sTs[i], ss[i], sas[i], FLAGS)
+            call(f"rwkv7_statepassing_forward{sfx}_ex", dev, B, TS, H, st, rr, ww, kk, vv, aa, bb, ys[i], sTs[i], ss[i], sas[i], FLAGS)
             st = sTs[i]
 
     def bwd():
         g = dsT
         for i in (3, 2, 1, 0):
             rr, ww, kk, vv, aa, bb, dd = seg[i]
-            if fp32:
-                call("rwkv7_statepassing_backward_f32", dev, B, TS, H, rr, ww, kk, vv, aa, bb, dd, g, ss[i], sas[i], ds[i], *grads[i])
-            else:
-                call("rwkv7_statepassing_backward_ex", dev, B, TS, H, rr, ww, kk, vv, aa, bb, dd, g, ss[i], sas[i], ds[i], *grads[i], FLAGS)
+            call(f"rwkv7_statepassing_backward{sfx}_ex", dev, B, TS, H, rr, ww, kk, vv, aa, bb, dd, g, ss[i], sas[i], ds[i], *grads[i], FLAGS)
             g = ds[i]
 
     def step():
         fwd()
         bwd()
 
-    chunked = fp32 or ALGO == "chunked"                            # the fp32 entry points know no other kernels
+    chunked = ALGO == "chunked"
     kernels = [("rwkv7c_fwd x4 (T=1024 each)" if chunked else "rwkv7_fwd x4 (T=1024 each)", fwd, 7 * eb * C * tok),
                ("rwkv7c_bwd x4" if chunked else "rwkv7_bwd x4", bwd, 13 * eb * C * tok)]
 

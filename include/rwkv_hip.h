@@ -485,6 +485,16 @@ int rwkv7_statepassing_backward_f32(void* stream, int B, int T, int H,
                                     const float* a, const float* b, const float* dy, const float* dsT,
                                     const float* s, const float* sa, float* ds0,
                                     float* dr, float* dw, float* dk, float* dv, float* da, float* db);
+/* as rwkv7_statepassing_*_ex: flags, missing tensors, and the pairing rule */
+int rwkv7_statepassing_forward_f32_ex(void* stream, int B, int T, int H,
+                                      const float* s0, const float* r, const float* w, const float* k,
+                                      const float* v, const float* a, const float* b,
+                                      float* y, float* sT, float* s, float* sa, unsigned flags);
+int rwkv7_statepassing_backward_f32_ex(void* stream, int B, int T, int H,
+                                       const float* r, const float* w, const float* k, const float* v,
+                                       const float* a, const float* b, const float* dy, const float* dsT,
+                                       const float* s, const float* sa, float* ds0,
+                                       float* dr, float* dw, float* dk, float* dv, float* da, float* db, unsigned flags);
 int rwkv7_state_forward_f32(void* stream, int B, int T, int H,
                             const float* s0, const float* r, const float* w, const float* k,
                             const float* v, const float* a, const float* b, float* y, float* s, float* sa);

@@ -397,7 +397,7 @@ variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r,
     Tensor y = flat || passing ? at::empty({B, T, H * HEAD}, r.options()) : at::empty({B, T, H, HEAD}, r.options());
     Tensor sT = passing ? at::empty({B, H, HEAD, HEAD}, f32) : Tensor();
     void* st = stream_of(r);
-    if (!grad && (dt != BF || !(flags & RWKV_FLAG_SWEEPS))) {
+    if (!grad && !(flags & RWKV_FLAG_SWEEPS)) {
         // no backward can follow: nothing is kept for one
         ok(rwkv7_forward_only(st, b_, t_, h_, dt == F32, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT)), true);
         if (passing) return {y, sT};
@@ -406,9 +406,8 @@ variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r,
     Tensor s = at::empty({B, H, T / CHUNK7, HEAD, HEAD}, f32), sa = at::empty({B, T, H, HEAD}, f32);
     if (dt == BF)
         ok(rwkv7_statepassing_forward_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)), true);
-    else if (passing) ok(rwkv7_statepassing_forward_f32(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa)), true);
-    else if (s0.defined()) ok(rwkv7_state_forward_f32(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(s), P(sa)), true);
-    else ok(rwkv7_forward_f32(st, b_, t_, h_, P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(s), P(sa)), true);
+    else
+        ok(rwkv7_statepassing_forward_f32_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)), true);
     ctx->save_for_backward({r, w, k, v, a, b, s, sa});
     put(ctx, {{"B", B}, {"T", T}, {"H", H}, {"flags", flags}});
     if (passing) return {y, sT};
@@ -427,13 +426,9 @@ variable_list rwkv7_grads(AutogradContext* ctx, const Tensor& dy_, const Tensor&
     if (r.scalar_type() == BF)
         ok(rwkv7_statepassing_backward_ex(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]),
                                           P(d[3]), P(d[4]), P(d[5]), static_cast<unsigned>(get(ctx, "flags"))), false);
-    else if (dsT.defined())
-        ok(rwkv7_statepassing_backward_f32(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]),
-                                           P(d[3]), P(d[4]), P(d[5])), false);
-    else if (state)
-        ok(rwkv7_state_backward_f32(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]), P(d[3]), P(d[4]), P(d[5])), false);
     else
-        ok(rwkv7_backward_f32(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(s), P(sa), P(d[0]), P(d[1]), P(d[2]), P(d[3]), P(d[4]), P(d[5])), false);
+        ok(rwkv7_statepassing_backward_f32_ex(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]),
+                                              P(d[3]), P(d[4]), P(d[5]), static_cast<unsigned>(get(ctx, "flags"))), false);
     return {ds0, d[0], d[1], d[2], d[3], d[4], d[5], NONE, NONE};
 }
 struct Rwkv7Passing : Function<Rwkv7Passing> {

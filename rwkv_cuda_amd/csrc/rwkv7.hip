@@ -28,6 +28,8 @@ constexpr int NT = NW * 64;
 constexpr int JW = 16;
 constexpr float W_SCALE = -0.6065306597f;   // -exp(-0.5)
 
+// Element pointers are typed for the bf16 mode; the fp32 mode (the reference's -D_FP32_ build) stores float pointers in
+// the same fields and its kernels (F32 = true) read them back as such through ldg4 / stg4.
 struct Args7 {
     int T, H;
     const uint16_t *r, *w, *k, *v, *a, *b, *dy;
@@ -48,8 +50,23 @@ DEVINL uint2 pack4(const float (&f)[4]) {
 }
 DEVINL void st4(float* dst, const float (&f)[4]) { *reinterpret_cast<float4*>(dst) = make_float4(f[0], f[1], f[2], f[3]); }
 // four consecutive elements as they come from memory
-DEVINL uint2 ldg4(const uint16_t* p, size_t o) { return *reinterpret_cast<const uint2*>(p + o); }
-DEVINL void stg4(uint16_t* p, size_t o, const float (&f)[4]) { *reinterpret_cast<uint2*>(p + o) = pack4(f); }
+template <bool F32> struct Raw4;
+template <> struct Raw4<false> { uint2 q; };
+template <> struct Raw4<true> { float4 q; };
+template <bool F32> DEVINL Raw4<F32> ldg4(const uint16_t* p, size_t o) {
+    Raw4<F32> x;
+    if constexpr (F32) x.q = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p) + o);
+    else x.q = *reinterpret_cast<const uint2*>(p + o);
+    return x;
+}
+template <bool F32> DEVINL void widen4(const Raw4<F32>& x, float (&f)[4]) {
+    if constexpr (F32) { f[0] = x.q.x; f[1] = x.q.y; f[2] = x.q.z; f[3] = x.q.w; }
+    else unpack4(x.q, f);
+}
+template <bool F32> DEVINL void stg4(uint16_t* p, size_t o, const float (&f)[4]) {
+    if constexpr (F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(p) + o) = make_float4(f[0], f[1], f[2], f[3]);
+    else *reinterpret_cast<uint2*>(p + o) = pack4(f);
+}
 DEVINL void ld16(float (&f)[16], const float* src) {          // 16 consecutive floats, 16-byte aligned (LDS)
 #pragma unroll
     for (int e = 0; e < 16; e += 4) {
@@ -64,6 +81,7 @@ struct SmemF {
     float y[CL][N], sa[CL][N];
 };
 
+template <bool F32>
 __global__ __launch_bounds__(NT) void rwkv7_fwd(const Args7 p) {
     __shared__ SmemF S;
     const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6, lo = lane & 15, hi = lane >> 4;
@@ -86,11 +104,11 @@ __global__ __launch_bounds__(NT) void rwkv7_fwd(const Args7 p) {
     }
 
     const int nchunks = T / CL;
-    uint2 gr, gw, gk, gv, ga, gb;
+    Raw4<F32> gr, gw, gk, gv, ga, gb;
     auto prefetch = [&](int c) {
         const size_t o = off(c * CL + st);
-        gr = ldg4(p.r, o); gw = ldg4(p.w, o); gk = ldg4(p.k, o);
-        gv = ldg4(p.v, o); ga = ldg4(p.a, o); gb = ldg4(p.b, o);
+        gr = ldg4<F32>(p.r, o); gw = ldg4<F32>(p.w, o); gk = ldg4<F32>(p.k, o);
+        gv = ldg4<F32>(p.v, o); ga = ldg4<F32>(p.a, o); gb = ldg4<F32>(p.b, o);
     };
     prefetch(0);
 
@@ -98,12 +116,12 @@ __global__ __launch_bounds__(NT) void rwkv7_fwd(const Args7 p) {
         __syncthreads();
         {
             float f[4];
-            unpack4(gr, f); st4(&S.r[st][sj], f);
-            unpack4(gk, f); st4(&S.k[st][sj], f);
-            unpack4(gv, f); st4(&S.v[st][sj], f);
-            unpack4(ga, f); st4(&S.a[st][sj], f);
-            unpack4(gb, f); st4(&S.b[st][sj], f);
-            unpack4(gw, f);
+            widen4<F32>(gr, f); st4(&S.r[st][sj], f);
+            widen4<F32>(gk, f); st4(&S.k[st][sj], f);
+            widen4<F32>(gv, f); st4(&S.v[st][sj], f);
+            widen4<F32>(ga, f); st4(&S.a[st][sj], f);
+            widen4<F32>(gb, f); st4(&S.b[st][sj], f);
+            widen4<F32>(gw, f);
 #pragma unroll
             for (int e = 0; e < 4; ++e) f[e] = __expf(W_SCALE / (1.0f + __expf(-f[e])));
             st4(&S.w[st][sj], f);
@@ -143,7 +161,7 @@ __global__ __launch_bounds__(NT) void rwkv7_fwd(const Args7 p) {
         {
             const size_t o = off(c * CL + st);
             float f[4] = {S.y[st][sj], S.y[st][sj + 1], S.y[st][sj + 2], S.y[st][sj + 3]};
-            stg4(p.y, o, f);
+            stg4<F32>(p.y, o, f);
             *reinterpret_cast<float4*>(p.sa + o) = *reinterpret_cast<const float4*>(&S.sa[st][sj]);
         }
     }
@@ -165,6 +183,7 @@ struct SmemB {
     float dSb[2][N];
 };
 
+template <bool F32>
 __global__ __launch_bounds__(NT) void rwkv7_bwd(const Args7 p) {
     __shared__ SmemB S;
     const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6, lo = lane & 15, hi = lane >> 4;
@@ -193,12 +212,12 @@ __global__ __launch_bounds__(NT) void rwkv7_bwd(const Args7 p) {
     }
 
     const int nchunks = T / CL;
-    uint2 gr, gw, gk, gv, ga, gb, gdy;
+    Raw4<F32> gr, gw, gk, gv, ga, gb, gdy;
     float4 gsa;
     auto prefetch = [&](int c) {
         const size_t o = off(c * CL + st);
-        gr = ldg4(p.r, o); gw = ldg4(p.w, o); gk = ldg4(p.k, o); gv = ldg4(p.v, o);
-        ga = ldg4(p.a, o); gb = ldg4(p.b, o); gdy = ldg4(p.dy, o);
+        gr = ldg4<F32>(p.r, o); gw = ldg4<F32>(p.w, o); gk = ldg4<F32>(p.k, o); gv = ldg4<F32>(p.v, o);
+        ga = ldg4<F32>(p.a, o); gb = ldg4<F32>(p.b, o); gdy = ldg4<F32>(p.dy, o);
         gsa = *reinterpret_cast<const float4*>(p.sa + o);
     };
     prefetch(nchunks - 1);
@@ -207,14 +226,14 @@ __global__ __launch_bounds__(NT) void rwkv7_bwd(const Args7 p) {
         __syncthreads();
         {
             float f[4], g[4];
-            unpack4(gr, f); st4(&S.r[st][sj], f);
-            unpack4(gk, f); st4(&S.k[st][sj], f);
-            unpack4(gv, f); st4(&S.v[st][sj], f);
-            unpack4(ga, f); st4(&S.a[st][sj], f);
-            unpack4(gb, f); st4(&S.b[st][sj], f);
-            unpack4(gdy, f); st4(&S.dy[st][sj], f);
+            widen4<F32>(gr, f); st4(&S.r[st][sj], f);
+            widen4<F32>(gk, f); st4(&S.k[st][sj], f);
+            widen4<F32>(gv, f); st4(&S.v[st][sj], f);
+            widen4<F32>(ga, f); st4(&S.a[st][sj], f);
+            widen4<F32>(gb, f); st4(&S.b[st][sj], f);
+            widen4<F32>(gdy, f); st4(&S.dy[st][sj], f);
             *reinterpret_cast<float4*>(&S.sa[st][sj]) = gsa;
-            unpack4(gw, f);
+            widen4<F32>(gw, f);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float sig = 1.0f / (1.0f + __expf(-f[e]));
@@ -293,14 +312,14 @@ __global__ __launch_bounds__(NT) void rwkv7_bwd(const Args7 p) {
             const size_t o = off(c * CL + st);
             auto put = [&](uint16_t* dst, const float (*src)[N]) {
                 float f[4] = {src[st][sj], src[st][sj + 1], src[st][sj + 2], src[st][sj + 3]};
-                stg4(dst, o, f);
+                stg4<F32>(dst, o, f);
             };
             put(p.dr, S.dr); put(p.dw, S.dw); put(p.dk, S.dk);
             put(p.dv, S.dv); put(p.db, S.db);
             float f[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) f[e] = (S.da[st][0][sj + e] + S.da[st][1][sj + e]) + (S.da[st][2][sj + e] + S.da[st][3][sj + e]);
-            stg4(p.da, o, f);
+            stg4<F32>(p.da, o, f);
         }
     }
     if (p.ds0 != nullptr) {
@@ -318,40 +337,47 @@ int check7(int B, int T, int H) {
     return RWKV_OK;
 }
 
-int launch7_fwd(void* stream, int B, int T, int H, const float* s0, const uint16_t* r, const uint16_t* w, const uint16_t* k,
-                const uint16_t* v, const uint16_t* a, const uint16_t* b, uint16_t* y, float* sT, float* s, float* sa) {
+const uint16_t* el(const void* p) { return static_cast<const uint16_t*>(p); }
+uint16_t* el(void* p) { return static_cast<uint16_t*>(p); }
+
+// r..b, y (and dy, dr..db below) are bf16 or, with f32, float
+int launch7_fwd(void* stream, bool f32, int B, int T, int H, const float* s0, const void* r, const void* w,
+                const void* k, const void* v, const void* a, const void* b, void* y,
+                float* sT, float* s, float* sa) {
     Args7 p{};
-    p.T = T; p.H = H; p.s0 = s0; p.r = r; p.w = w; p.k = k; p.v = v; p.a = a; p.b = b; p.y = y; p.sT = sT; p.s = s; p.sa = sa;
-    hipLaunchKernelGGL(rwkv7_fwd, dim3(H, B), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
+    p.T = T; p.H = H; p.s0 = s0; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b);
+    p.y = el(y); p.sT = sT; p.s = s; p.sa = sa;
+    if (f32) hipLaunchKernelGGL(rwkv7_fwd<true>, dim3(H, B), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
+    else hipLaunchKernelGGL(rwkv7_fwd<false>, dim3(H, B), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
     return launch_status();
 }
 
-int launch7_bwd(void* stream, int B, int T, int H, const uint16_t* r, const uint16_t* w, const uint16_t* k, const uint16_t* v,
-                const uint16_t* a, const uint16_t* b, const uint16_t* dy, const float* dsT, const float* s, const float* sa,
-                float* ds0, uint16_t* dr, uint16_t* dw, uint16_t* dk, uint16_t* dv, uint16_t* da, uint16_t* db) {
+int launch7_bwd(void* stream, bool f32, int B, int T, int H, const void* r, const void* w, const void* k,
+                const void* v, const void* a, const void* b, const void* dy, const float* dsT,
+                const float* s, const float* sa, float* ds0, void* dr, void* dw, void* dk,
+                void* dv, void* da, void* db) {
     Args7 p{};
-    p.T = T; p.H = H; p.r = r; p.w = w; p.k = k; p.v = v; p.a = a; p.b = b; p.dy = dy;
+    p.T = T; p.H = H; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b); p.dy = el(dy);
     p.dsT = dsT; p.s = const_cast<float*>(s); p.sa = const_cast<float*>(sa);
-    p.ds0 = ds0; p.dr = dr; p.dw = dw; p.dk = dk; p.dv = dv; p.da = da; p.db = db;
-    hipLaunchKernelGGL(rwkv7_bwd, dim3(H, B), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
+    p.ds0 = ds0; p.dr = el(dr); p.dw = el(dw); p.dk = el(dk); p.dv = el(dv); p.da = el(da); p.db = el(db);
+    if (f32) hipLaunchKernelGGL(rwkv7_bwd<true>, dim3(H, B), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
+    else hipLaunchKernelGGL(rwkv7_bwd<false>, dim3(H, B), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
     return launch_status();
 }
 
-// bf16 mode: the chunked matrix-core kernels (rwkv7_chunk.hip) unless RWKV_FLAG_SWEEPS asks for the step kernels above.
+// The chunked matrix-core kernels (rwkv7_chunk.hip) unless RWKV_FLAG_SWEEPS asks for the step kernels above, in either mode.
 // The two families lay out the scratch tensor `s` differently, so a backward must get the flags of its forward.
 constexpr unsigned DEFAULT7 = 0u;                   // what the entry points without a flags argument run: the chunked kernels
-int bf16_fwd(void* stream, unsigned flags, int B, int T, int H, const float* s0, const rwkv_bf16* r, const rwkv_bf16* w,
-             const rwkv_bf16* k, const rwkv_bf16* v, const rwkv_bf16* a, const rwkv_bf16* b, rwkv_bf16* y, float* sT,
-             float* s, float* sa) {
-    if (flags & RWKV_FLAG_SWEEPS) return launch7_fwd(stream, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
-    return launch7c_fwd(static_cast<hipStream_t>(stream), false, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
+int run_fwd(void* stream, bool f32, unsigned flags, int B, int T, int H, const float* s0, const void* r, const void* w, const void* k,
+            const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa) {
+    if (flags & RWKV_FLAG_SWEEPS) return launch7_fwd(stream, f32, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
+    return launch7c_fwd(static_cast<hipStream_t>(stream), f32, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
 }
-int bf16_bwd(void* stream, unsigned flags, int B, int T, int H, const rwkv_bf16* r, const rwkv_bf16* w, const rwkv_bf16* k,
-             const rwkv_bf16* v, const rwkv_bf16* a, const rwkv_bf16* b, const rwkv_bf16* dy, const float* dsT,
-             const float* s, const float* sa, float* ds0, rwkv_bf16* dr, rwkv_bf16* dw, rwkv_bf16* dk, rwkv_bf16* dv,
-             rwkv_bf16* da, rwkv_bf16* db) {
-    if (flags & RWKV_FLAG_SWEEPS) return launch7_bwd(stream, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
-    return launch7c_bwd(static_cast<hipStream_t>(stream), false, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
+int run_bwd(void* stream, bool f32, unsigned flags, int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
+            const void* a, const void* b, const void* dy, const float* dsT, const float* s, const float* sa, float* ds0, void* dr,
+            void* dw, void* dk, void* dv, void* da, void* db) {
+    if (flags & RWKV_FLAG_SWEEPS) return launch7_bwd(stream, f32, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
+    return launch7c_bwd(static_cast<hipStream_t>(stream), f32, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
 }  // namespace
@@ -366,7 +392,7 @@ int rwkv7_statepassing_forward(void* stream, int B, int T, int H, const float* s
                                const rwkv_bf16* b, rwkv_bf16* y, float* sT, float* s, float* sa) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({s0, r, w, k, v, a, b, y, sT, s, sa})) return e;
-    return bf16_fwd(stream, DEFAULT7, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
+    return run_fwd(stream, false, DEFAULT7, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
 }
 
 int rwkv7_statepassing_backward(void* stream, int B, int T, int H, const rwkv_bf16* r, const rwkv_bf16* w,
@@ -376,7 +402,7 @@ int rwkv7_statepassing_backward(void* stream, int B, int T, int H, const rwkv_bf
                                 rwkv_bf16* da, rwkv_bf16* db) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db})) return e;
-    return bf16_bwd(stream, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
+    return run_bwd(stream, false, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
 // Initial state with its gradient, no final state: the same kernels without the sT store and with dsT = 0.
@@ -385,7 +411,7 @@ int rwkv7_state_forward(void* stream, int B, int T, int H, const float* s0, cons
                         rwkv_bf16* y, float* s, float* sa) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({s0, r, w, k, v, a, b, y, s, sa})) return e;
-    return bf16_fwd(stream, DEFAULT7, B, T, H, s0, r, w, k, v, a, b, y, nullptr, s, sa);
+    return run_fwd(stream, false, DEFAULT7, B, T, H, s0, r, w, k, v, a, b, y, nullptr, s, sa);
 }
 
 int rwkv7_state_backward(void* stream, int B, int T, int H, const rwkv_bf16* r, const rwkv_bf16* w,
@@ -394,7 +420,7 @@ int rwkv7_state_backward(void* stream, int B, int T, int H, const rwkv_bf16* r, 
                          rwkv_bf16* dw, rwkv_bf16* dk, rwkv_bf16* dv, rwkv_bf16* da, rwkv_bf16* db) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, ds0, dr, dw, dk, dv, da, db})) return e;
-    return bf16_bwd(stream, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, ds0, dr, dw, dk, dv, da, db);
+    return run_bwd(stream, false, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
 // No state on either side: zero initial state, no final state, no state gradients.
@@ -402,7 +428,7 @@ int rwkv7_forward(void* stream, int B, int T, int H, const rwkv_bf16* r, const r
                   const rwkv_bf16* v, const rwkv_bf16* a, const rwkv_bf16* b, rwkv_bf16* y, float* s, float* sa) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, y, s, sa})) return e;
-    return bf16_fwd(stream, DEFAULT7, B, T, H, nullptr, r, w, k, v, a, b, y, nullptr, s, sa);
+    return run_fwd(stream, false, DEFAULT7, B, T, H, nullptr, r, w, k, v, a, b, y, nullptr, s, sa);
 }
 
 int rwkv7_backward(void* stream, int B, int T, int H, const rwkv_bf16* r, const rwkv_bf16* w, const rwkv_bf16* k,
@@ -411,7 +437,7 @@ int rwkv7_backward(void* stream, int B, int T, int H, const rwkv_bf16* r, const 
                    rwkv_bf16* db) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, dr, dw, dk, dv, da, db})) return e;
-    return bf16_bwd(stream, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, nullptr, dr, dw, dk, dv, da, db);
+    return run_bwd(stream, false, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, nullptr, dr, dw, dk, dv, da, db);
 }
 
 // The state-passing op with per-call flags; s0, sT (forward) and dsT, ds0 (backward) may be NULL, which makes these two
@@ -422,7 +448,7 @@ int rwkv7_statepassing_forward_ex(void* stream, int B, int T, int H, const float
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, y, s, sa})) return e;
     if (!aligned16(s0) || !aligned16(sT)) return RWKV_ERR_ALIGN;
-    return bf16_fwd(stream, flags, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
+    return run_fwd(stream, false, flags, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
 }
 
 int rwkv7_statepassing_backward_ex(void* stream, int B, int T, int H, const rwkv_bf16* r, const rwkv_bf16* w,
@@ -433,7 +459,7 @@ int rwkv7_statepassing_backward_ex(void* stream, int B, int T, int H, const rwkv
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, dr, dw, dk, dv, da, db})) return e;
     if (!aligned16(dsT) || !aligned16(ds0)) return RWKV_ERR_ALIGN;
-    return bf16_bwd(stream, flags, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
+    return run_bwd(stream, false, flags, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
 // A forward that no backward follows: the chunked kernels without their stores of `s` and `sa`.
@@ -453,7 +479,7 @@ int rwkv7_statepassing_forward_f32(void* stream, int B, int T, int H, const floa
                                    float* sT, float* s, float* sa) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({s0, r, w, k, v, a, b, y, sT, s, sa})) return e;
-    return launch7c_fwd(static_cast<hipStream_t>(stream), true, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
+    return run_fwd(stream, true, DEFAULT7, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
 }
 
 int rwkv7_statepassing_backward_f32(void* stream, int B, int T, int H, const float* r, const float* w, const float* k,
@@ -462,7 +488,7 @@ int rwkv7_statepassing_backward_f32(void* stream, int B, int T, int H, const flo
                                     float* dv, float* da, float* db) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db})) return e;
-    return launch7c_bwd(static_cast<hipStream_t>(stream), true, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
+    return run_bwd(stream, true, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
 int rwkv7_state_forward_f32(void* stream, int B, int T, int H, const float* s0, const float* r, const float* w,
@@ -470,7 +496,7 @@ int rwkv7_state_forward_f32(void* stream, int B, int T, int H, const float* s0, 
                             float* sa) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({s0, r, w, k, v, a, b, y, s, sa})) return e;
-    return launch7c_fwd(static_cast<hipStream_t>(stream), true, B, T, H, s0, r, w, k, v, a, b, y, nullptr, s, sa);
+    return run_fwd(stream, true, DEFAULT7, B, T, H, s0, r, w, k, v, a, b, y, nullptr, s, sa);
 }
 
 int rwkv7_state_backward_f32(void* stream, int B, int T, int H, const float* r, const float* w, const float* k,
@@ -479,14 +505,14 @@ int rwkv7_state_backward_f32(void* stream, int B, int T, int H, const float* r, 
                              float* db) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, ds0, dr, dw, dk, dv, da, db})) return e;
-    return launch7c_bwd(static_cast<hipStream_t>(stream), true, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, ds0, dr, dw, dk, dv, da, db);
+    return run_bwd(stream, true, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
 int rwkv7_forward_f32(void* stream, int B, int T, int H, const float* r, const float* w, const float* k,
                       const float* v, const float* a, const float* b, float* y, float* s, float* sa) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, y, s, sa})) return e;
-    return launch7c_fwd(static_cast<hipStream_t>(stream), true, B, T, H, nullptr, r, w, k, v, a, b, y, nullptr, s, sa);
+    return run_fwd(stream, true, DEFAULT7, B, T, H, nullptr, r, w, k, v, a, b, y, nullptr, s, sa);
 }
 
 int rwkv7_backward_f32(void* stream, int B, int T, int H, const float* r, const float* w, const float* k,
@@ -494,7 +520,27 @@ int rwkv7_backward_f32(void* stream, int B, int T, int H, const float* r, const 
                        const float* sa, float* dr, float* dw, float* dk, float* dv, float* da, float* db) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, dr, dw, dk, dv, da, db})) return e;
-    return launch7c_bwd(static_cast<hipStream_t>(stream), true, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, nullptr, dr, dw, dk, dv, da, db);
+    return run_bwd(stream, true, DEFAULT7, B, T, H, r, w, k, v, a, b, dy, nullptr, s, sa, nullptr, dr, dw, dk, dv, da, db);
+}
+
+// The state-passing op with per-call flags; s0, sT (forward) and dsT, ds0 (backward) may be NULL, as in the bf16 mode.
+int rwkv7_statepassing_forward_f32_ex(void* stream, int B, int T, int H, const float* s0, const float* r, const float* w,
+                                      const float* k, const float* v, const float* a, const float* b, float* y, float* sT,
+                                      float* s, float* sa, unsigned flags) {
+    if (int e = check7(B, T, H)) return e;
+    if (int e = check_ptrs({r, w, k, v, a, b, y, s, sa})) return e;
+    if (!aligned16(s0) || !aligned16(sT)) return RWKV_ERR_ALIGN;
+    return run_fwd(stream, true, flags, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa);
+}
+
+int rwkv7_statepassing_backward_f32_ex(void* stream, int B, int T, int H, const float* r, const float* w, const float* k,
+                                       const float* v, const float* a, const float* b, const float* dy, const float* dsT,
+                                       const float* s, const float* sa, float* ds0, float* dr, float* dw, float* dk,
+                                       float* dv, float* da, float* db, unsigned flags) {
+    if (int e = check7(B, T, H)) return e;
+    if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, dr, dw, dk, dv, da, db})) return e;
+    if (!aligned16(dsT) || !aligned16(ds0)) return RWKV_ERR_ALIGN;
+    return run_bwd(stream, true, flags, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db);
 }
 
 }  // extern "C"

@@ -221,3 +221,26 @@ def test_rwkv7_forward_without_gradients_is_bit_identical(lib, B, T, H, dtype):
         for g, e in zip(got, want):
             assert not g.requires_grad and torch.equal(g, e.detach())
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("B,T,H", [(1, 16, 1), (2, 80, 3)])
+def test_fp32_sweeps_option_runs_the_step_kernels(lib, B, T, H):
+    """The option chooses the kernels in the fp32 mode too, for the backward that follows as well, and without gradients."""
+    N = 64
+    args = _fp32_inputs(B, T, H, 91)
+    s0, r, w, k, v, a, b, dy, dsT = args
+    ref = O.grads(*args)
+    emu = O.backward_hand(*args, dtype=torch.float32, invert=True)
+    out = {}
+    for algo in ("chunked", "sweeps"):
+        t = [x.to(DEV).requires_grad_(True) for x in (s0, *(x.reshape(B, T, H * N) for x in (r, w, k, v, a, b)))]
+        with options.algorithm(algo):
+            y, sT = R.RWKV7_STATE_PASSING_CLAMPW_CUDA(*t)
+            with torch.no_grad():
+                y1, sT1 = R.RWKV7_STATE_PASSING_CLAMPW_CUDA(*t)
+        assert torch.equal(y, y1) and torch.equal(sT, sT1)
+        g = torch.autograd.grad([y, sT], t, [dy.to(DEV).view(B, T, H * N), dsT.to(DEV)])
+        out[algo] = [x.detach().double().cpu() for x in (y, sT, *g)]
+        for name, want, e, got in zip(NAMES, ref, emu, out[algo]):
+            assert_fp32_mode(f"{algo} {name}", want.reshape(got.shape), e.reshape(got.shape), got)
+    assert not torch.equal(out["chunked"][0], out["sweeps"][0])
