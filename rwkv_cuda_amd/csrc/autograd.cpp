@@ -47,21 +47,26 @@ void check(std::initializer_list<std::pair<const Tensor*, const char*>> ts, c10:
 void check_head(int64_t C, int64_t H) {
     require(H > 0 && C % H == 0 && C / H <= MAX_HEAD, "C must be a multiple of H with a head size of at most 128");
 }
+// the package's own error type, in either direction: the engine's threads, which run the backwards, do not hold the interpreter's lock
+[[noreturn]] void fail(const std::string& msg) {
+    const py::gil_scoped_acquire lock;
+    PyErr_SetString(py::module_::import("rwkv_cuda_amd._lib").attr("RwkvHipError").ptr(), msg.c_str());
+    throw py::error_already_set();
+}
 // sizes as the C ABI takes them
-int i32(int64_t x) { TORCH_CHECK(x > 0 && x <= std::numeric_limits<int>::max(), "size ", x, " is outside 1 .. 2147483647"); return static_cast<int>(x); }
+int i32(int64_t x) {
+    if (x <= 0 || x > std::numeric_limits<int>::max()) fail("size " + std::to_string(x) + " is outside 1 .. 2147483647");
+    return static_cast<int>(x);
+}
 struct Dims { int B, T, C, H; };
 Dims dims(int64_t B, int64_t T, int64_t C, int64_t H) { return {i32(B), i32(T), i32(C), i32(H)}; }
 
 void* stream_of(const Tensor& t) { return static_cast<void*>(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream()); }
-void ok(int status, bool forward) {
+void ok(int status) {
     if (status == RWKV_OK) return;
     std::string msg = "librwkv_hip: status " + std::to_string(status) + ": " + rwkv_strerror(status);
     if (status == RWKV_ERR_LAUNCH) msg += " (hipError " + std::to_string(rwkv_last_hip_error()) + ")";
-    if (forward) {
-        PyErr_SetString(py::module_::import("rwkv_cuda_amd._lib").attr("RwkvHipError").ptr(), msg.c_str());
-        throw py::error_already_set();
-    }
-    TORCH_CHECK(false, msg);
+    fail(msg);
 }
 
 // typed pointers; an undefined tensor is NULL
@@ -90,7 +95,7 @@ struct Wkv4 : Function<Wkv4> {
         const Guard guard(w.device());
         Tensor y = at::empty({B, T, C}, k.options());
         // w = -exp(w) of the reference wrapper (:95) happens inside the kernels
-        ok(rwkv_wkv4raw_forward(stream_of(w), i32(B), i32(T), i32(C), P(w), P(u), P(k), P(v), P(y)), true);
+        ok(rwkv_wkv4raw_forward(stream_of(w), i32(B), i32(T), i32(C), P(w), P(u), P(k), P(v), P(y)));
         ctx->save_for_backward({w, u, k, v});
         put(ctx, {{"B", B}, {"T", T}, {"C", C}});
         return y;
@@ -104,7 +109,7 @@ struct Wkv4 : Function<Wkv4> {
         Tensor gk = at::empty({B, T, C}, w.options()), gv = at::empty({B, T, C}, w.options());
         const size_t n = rwkv_wkv4raw_backward_workspace_bytes(B, T, C);
         Tensor ws = bytes(w, n);
-        ok(rwkv_wkv4raw_backward(stream_of(w), B, T, C, P(w), P(u), P(k), P(v), P(gy), P(gw), P(gu), P(gk), P(gv), P(ws), n), false);
+        ok(rwkv_wkv4raw_backward(stream_of(w), B, T, C, P(w), P(u), P(k), P(v), P(gy), P(gw), P(gu), P(gk), P(gv), P(ws), n));
         return {NONE, NONE, NONE, gw, gu, gk, gv};
     }
 };
@@ -120,7 +125,7 @@ struct TimeX : Function<TimeX> {
         require(w.numel() == C * T && k.numel() == B * C * T, "shape mismatch");
         const Guard guard(w.device());
         Tensor x = at::empty({B, C, T}, k.options());
-        ok(rwkv_timex_forward(stream_of(w), P(w), P(k), P(x), static_cast<float>(eps), i32(B), i32(C), i32(T)), true);
+        ok(rwkv_timex_forward(stream_of(w), P(w), P(k), P(x), static_cast<float>(eps), i32(B), i32(C), i32(T)));
         ctx->save_for_backward({w, k});
         put(ctx, {{"B", B}, {"T", T}, {"C", C}});
         return x;
@@ -133,7 +138,7 @@ struct TimeX : Function<TimeX> {
         Tensor gk = at::empty({B, C, T}, k.options()), gw = at::empty({C, T}, k.options());      // the sum over the batch of run.py:102 happens in the library
         const size_t n = rwkv_timex_backward_ws_bytes(B, C, T);
         const Tensor ws = n > 0 ? bytes(k, n) : Tensor();
-        ok(rwkv_timex_backward_ws(stream_of(w), P(w), P(k), P(gx), P(gw), P(gk), B, C, T, P(ws), n), false);
+        ok(rwkv_timex_backward_ws(stream_of(w), P(w), P(k), P(gx), P(gw), P(gk), B, C, T, P(ws), n));
         return {gw, gk, NONE, NONE, NONE, NONE};
     }
 };
@@ -155,11 +160,11 @@ struct Wkv5F32 : Function<Wkv5F32> {
         if (chunked) {
             const size_t n = grad ? rwkv_wkv5f32s_saved_bytes(d.B, d.T, d.C, d.H) : 0;
             const Tensor saved = grad ? bytes(r, n) : Tensor();
-            ok(rwkv_wkv5f32s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(saved), n), true);
+            ok(rwkv_wkv5f32s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(saved), n));
             if (grad) ctx->save_for_backward({r, k, v, w, u, saved});
         } else {
             const Tensor ew = w.exp().neg_(), eew = ew.exp();
-            ok(rwkv_wkv5f32_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(eew), P(u), P(y)), true);
+            ok(rwkv_wkv5f32_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(eew), P(u), P(y)));
             if (grad) ctx->save_for_backward({r, k, v, w, u, eew, ew});
         }
         put(ctx, {{"B", B}, {"T", T}, {"C", C}, {"H", H}, {"chunked", chunked}});
@@ -178,10 +183,10 @@ struct Wkv5F32 : Function<Wkv5F32> {
             const size_t n = rwkv_wkv5f32s_backward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, n);
             ok(rwkv_wkv5f32s_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(gy), P(gr), P(gk), P(gv), P(gw), P(gu),
-                                      P(saved), saved.numel(), P(ws), n), false);
+                                      P(saved), saved.numel(), P(ws), n));
         } else {
             Tensor pw = at::empty({d.B, d.C}, o), pu = at::empty({d.B, d.C}, o);
-            ok(rwkv_wkv5f32_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(s[5]), P(s[6]), P(u), P(gy), P(gr), P(gk), P(gv), P(pw), P(pu)), false);
+            ok(rwkv_wkv5f32_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(s[5]), P(s[6]), P(u), P(gy), P(gr), P(gk), P(gv), P(pw), P(pu)));
             gw = pw.sum(0).view(w.sizes()); gu = pu.sum(0).view(u.sizes());
         }
         return {NONE, NONE, NONE, NONE, gr, gk, gv, gw, gu, NONE, NONE};
@@ -208,11 +213,11 @@ struct Wkv5A : Function<Wkv5A> {
         if (chunked) {
             const size_t n = grad ? rwkv_wkv5as_saved_bytes(d.B, d.T, d.C, d.H) : 0;
             const Tensor saved = grad ? bytes(r, n) : Tensor();
-            ok(rwkv_wkv5as_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w1), P(u1), P(w2), P(u2), P(y), P(saved), n), true);
+            ok(rwkv_wkv5as_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w1), P(u1), P(w2), P(u2), P(y), P(saved), n));
             if (grad) ctx->save_for_backward({r, k, v, w1, u1, w2, u2, saved});
         } else {
             const Tensor ew1 = w1.exp().neg_(), eew1 = ew1.exp(), ew2 = w2.exp().neg_(), eew2 = ew2.exp();
-            ok(rwkv_wkv5a_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(eew1), P(u1), P(eew2), P(u2), P(y)), true);
+            ok(rwkv_wkv5a_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(eew1), P(u1), P(eew2), P(u2), P(y)));
             if (grad) ctx->save_for_backward({r, k, v, w1, u1, w2, u2, eew1, ew1, eew2, ew2});
         }
         put(ctx, {{"B", B}, {"T", T}, {"C", C}, {"H", H}, {"chunked", chunked}});
@@ -232,11 +237,11 @@ struct Wkv5A : Function<Wkv5A> {
             const size_t n = rwkv_wkv5as_backward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, n);
             ok(rwkv_wkv5as_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w1), P(u1), P(w2), P(u2), P(gy), P(gr), P(gk), P(gv),
-                                    P(gp[0]), P(gp[1]), P(gp[2]), P(gp[3]), P(saved), saved.numel(), P(ws), n), false);
+                                    P(gp[0]), P(gp[1]), P(gp[2]), P(gp[3]), P(saved), saved.numel(), P(ws), n));
         } else {
             for (Tensor& x : gp) x = at::empty({d.B, d.C}, o);
             ok(rwkv_wkv5a_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(s[7]), P(s[8]), P(u1), P(s[9]), P(s[10]), P(u2), P(gy),
-                                   P(gr), P(gk), P(gv), P(gp[0]), P(gp[1]), P(gp[2]), P(gp[3])), false);
+                                   P(gr), P(gk), P(gv), P(gp[0]), P(gp[1]), P(gp[2]), P(gp[3])));
             for (Tensor& x : gp) x = x.sum(0).view(w1.sizes());
         }
         return {gr, gk, gv, gp[0], gp[1], gp[2], gp[3], NONE, NONE};
@@ -264,13 +269,13 @@ struct Wkv5Bf16 : Function<Wkv5Bf16> {
             // (at 128 only if a backward can follow)
             const bool keep = grad || !whole;
             const Tensor saved = keep ? bytes(r, n) : Tensor();
-            ok(rwkv_wkv5s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(saved), keep ? n : 0, flags), true);
+            ok(rwkv_wkv5s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(saved), keep ? n : 0, flags));
             if (keep) ctx->save_for_backward({r, k, v, decay, u, w, saved});
         } else {
             // heads of 128 channels with options run as four heads of 64 whose fp32 terms need scratch; every other size needs none
             const size_t nf = rwkv_wkv5_forward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, nf < 16 ? 16 : nf);
-            ok(rwkv_wkv5raw_forward_ws(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(ws), nf, flags), true);
+            ok(rwkv_wkv5raw_forward_ws(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(ws), nf, flags));
             ctx->save_for_backward({r, k, v, decay, u});
         }
         put(ctx, {{"B", B}, {"T", T}, {"C", C}, {"H", H}, {"flags", flags}});
@@ -291,12 +296,12 @@ struct Wkv5Bf16 : Function<Wkv5Bf16> {
             const size_t n = d.C == d.H * MAX_HEAD ? 4 * static_cast<size_t>(d.B) * d.C : rwkv_wkv5s_backward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, n);
             ok(rwkv_wkv5s_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(decay), P(u), P(gy), P(gr), P(gk), P(gv), P(gw), P(gu),
-                                   P(saved), saved.numel(), P(ws), n, flags), false);
+                                   P(saved), saved.numel(), P(ws), n, flags));
         } else {
             const size_t n = rwkv_wkv5raw_backward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, n);
             ok(rwkv_wkv5raw_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(decay), P(u), P(gy), P(gr), P(gk), P(gv), P(gw), P(gu),
-                                     P(ws), n, flags), false);
+                                     P(ws), n, flags));
         }
         return {NONE, NONE, NONE, NONE, gr, gk, gv, gw, gu, NONE, NONE};
     }
@@ -320,7 +325,7 @@ variable_list wkv6_grads(AutogradContext* ctx, const Tensor& gy_, bool state) {
     const size_t n = rwkv_wkv6f_backward_saved_workspace_bytes(d.B, d.T, d.C, d.H);
     Tensor ws = bytes(r, n);
     ok(rwkv_wkv6f_backward_saved(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(s0), P(gy), P(gr), P(gk), P(gv), P(gw), P(gu), P(gs),
-                                 saved.numel() > 0 ? P(saved) : Ptr{nullptr}, saved.numel(), P(ws), n, static_cast<unsigned>(get(ctx, "flags"))), false);
+                                 saved.numel() > 0 ? P(saved) : Ptr{nullptr}, saved.numel(), P(ws), n, static_cast<unsigned>(get(ctx, "flags"))));
     return {NONE, NONE, NONE, NONE, gr, gk, gv, gw, gu, gs, NONE};
 }
 Tensor wkv6_run(AutogradContext* ctx, int64_t B, int64_t T, int64_t C, int64_t H, const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& w,
@@ -336,7 +341,7 @@ Tensor wkv6_run(AutogradContext* ctx, int64_t B, int64_t T, int64_t C, int64_t H
     const size_t n = rwkv_wkv6f_saved_bytes(d.B, d.T, d.C, d.H);
     Tensor saved = bytes(r, n);
     ok(rwkv_wkv6f_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(s), P(y), n > 0 ? P(saved) : Ptr{nullptr}, n,
-                          static_cast<unsigned>(flags)), true);
+                          static_cast<unsigned>(flags)));
     if (s.defined()) ctx->save_for_backward({r, k, v, w, u, saved, s});
     else ctx->save_for_backward({r, k, v, w, u, saved});
     put(ctx, {{"B", B}, {"T", T}, {"C", C}, {"H", H}, {"flags", flags}});
@@ -399,15 +404,15 @@ variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r,
     void* st = stream_of(r);
     if (!grad && !(flags & RWKV_FLAG_SWEEPS)) {
         // no backward can follow: nothing is kept for one
-        ok(rwkv7_forward_only(st, b_, t_, h_, dt == F32, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT)), true);
+        ok(rwkv7_forward_only(st, b_, t_, h_, dt == F32, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT)));
         if (passing) return {y, sT};
         return {y};
     }
     Tensor s = at::empty({B, H, T / CHUNK7, HEAD, HEAD}, f32), sa = at::empty({B, T, H, HEAD}, f32);
     if (dt == BF)
-        ok(rwkv7_statepassing_forward_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)), true);
+        ok(rwkv7_statepassing_forward_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)));
     else
-        ok(rwkv7_statepassing_forward_f32_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)), true);
+        ok(rwkv7_statepassing_forward_f32_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)));
     ctx->save_for_backward({r, w, k, v, a, b, s, sa});
     put(ctx, {{"B", B}, {"T", T}, {"H", H}, {"flags", flags}});
     if (passing) return {y, sT};
@@ -425,10 +430,10 @@ variable_list rwkv7_grads(AutogradContext* ctx, const Tensor& dy_, const Tensor&
     void* st = stream_of(r);
     if (r.scalar_type() == BF)
         ok(rwkv7_statepassing_backward_ex(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]),
-                                          P(d[3]), P(d[4]), P(d[5]), static_cast<unsigned>(get(ctx, "flags"))), false);
+                                          P(d[3]), P(d[4]), P(d[5]), static_cast<unsigned>(get(ctx, "flags"))));
     else
         ok(rwkv7_statepassing_backward_f32_ex(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]),
-                                              P(d[3]), P(d[4]), P(d[5]), static_cast<unsigned>(get(ctx, "flags"))), false);
+                                              P(d[3]), P(d[4]), P(d[5]), static_cast<unsigned>(get(ctx, "flags"))));
     return {ds0, d[0], d[1], d[2], d[3], d[4], d[5], NONE, NONE};
 }
 struct Rwkv7Passing : Function<Rwkv7Passing> {

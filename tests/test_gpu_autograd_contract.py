@@ -5,6 +5,7 @@ import torch
 from torch.utils.checkpoint import checkpoint
 
 from rwkv_cuda_amd import depthwise_conv1d, rwkv7_fast_fused as R, synth, wkv, wkv5, wkv5_bf16, wkv5a, wkv6, wkv6_state
+from rwkv_cuda_amd._lib import RwkvHipError
 from _gpu_util import DEV
 
 pytestmark = pytest.mark.gpu
@@ -121,3 +122,22 @@ def test_fp32_decays_of_any_alignment(lib, op):
         t.append(z.requires_grad_(True))
     got = _grads(f(*t), t)
     assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_errors_of_either_direction_are_the_packages_own(lib, op):
+    """No tokens, and an upstream gradient off the 16-byte grid: refused by the host code, in the backward on a thread of the engine."""
+    f, x = _case(op)
+    t = [z.to(DEV).requires_grad_(True) for z in x]
+    out = f(*t)
+    out = out if isinstance(out, tuple) else (out,)
+    up = [torch.ones_like(o) for o in out]
+    up[0] = torch.cat([up[0].new_zeros(1), up[0].reshape(-1)])[1:].view(up[0].shape)
+    assert up[0].data_ptr() % 16 != 0
+    with pytest.raises(RwkvHipError, match="align"):
+        torch.autograd.grad(out, t, up)
+    if op.startswith(("wkv5", "wkv6")) and op != "wkv5a":
+        empty = [z.detach()[:, :0].contiguous() if z.dim() == 3 else z.detach() for z in t]
+        module, h = {"wkv5": (wkv5, H), "wkv5_bf16": (wkv5_bf16, H), "wkv5_bf16_128": (wkv5_bf16, H // 2), "wkv6": (wkv6, H), "wkv6_state": (wkv6_state, H)}[op]
+        with pytest.raises(RwkvHipError):
+            module.RUN_CUDA(B, 0, C, h, *empty)
