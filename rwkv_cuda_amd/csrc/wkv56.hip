@@ -823,7 +823,15 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
 // workgroups return at once.  Backward: the three passes, which need nothing of each other, side by side.
 // bf16, heads of 64, in a layer without a strong decay: the heads that a one-sweep kernel has given up (its flag words, of the
 // forward and in the backward of both directions: such a forward has left no states).
-template <int NP, bool F32, bool TWO> DEVINL bool steps_for(const Args& a) {
+// fp32: also the heads whose inputs are not all finite, which the chunked kernels mark by a NaN in the first element of each output
+// (wkv5_f32.hip); out: the one that this workgroup would write.
+template <int NP, bool F32, bool TWO> DEVINL bool steps_for(const Args& a, const uint16_t* out) {
+    if constexpr (F32) {
+        const size_t first = static_cast<size_t>(blockIdx.x / a.H) * a.T * a.C + static_cast<size_t>(blockIdx.x % a.H) * NP;
+        const float x = reinterpret_cast<const float*>(out)[first];
+        __syncthreads();                                 // all waves have it before one of them writes
+        if (x != x) return true;
+    }
     if constexpr (!F32 && NP == 64) {
         if (!strong_layer(static_cast<const uint16_t*>(a.w), a.C, threadIdx.x & 63)) {
             const int lane = threadIdx.x & 63;
@@ -836,13 +844,13 @@ template <int NP, bool F32, bool TWO> DEVINL bool steps_for(const Args& a) {
 }
 template <int NP, int PARTS, bool F32, bool TWO>
 __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_fwd(const Args a, const int hn) {
-    if (!steps_for<NP, F32, TWO>(a)) return;
+    if (!steps_for<NP, F32, TWO>(a, a.y)) return;
     __shared__ SmemRows<NP, PARTS, P_FWD, F32, TWO, true> S;
     rows_body<NP, PARTS, P_FWD, W_HEAD, F32, TWO, true>(S, a, hn);
 }
 template <int NP, int PARTS, bool F32, bool TWO>
 __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_bwd(const Args a, const int hn) {
-    if (!steps_for<NP, F32, TWO>(a)) return;
+    if (!steps_for<NP, F32, TWO>(a, blockIdx.y == 0 ? a.gr : (blockIdx.y == 1 ? a.gv : a.gk))) return;
     __shared__ union {
         SmemRows<NP, PARTS, P_GR, F32, TWO, true> gr;
         SmemRows<NP, PARTS, P_GV, F32, TWO, true> gv;

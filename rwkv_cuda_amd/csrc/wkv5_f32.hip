@@ -26,6 +26,12 @@
 // product for that quadrant, with o1^4 on either side (o1^8 itself may underflow where the whole term is one).  Heads with a
 // channel below l = -17, or one that is no number, are left to wkv5_steps_* (steps_head, common.h).
 //
+// Inputs that are no number, or infinite: a tile product multiplies what it leaves out by zero, which would carry them to up to 15
+// tokens that they do not act on (earlier outputs, later gradients).  The waves that load note them (one multiply-add an element;
+// wkv5 B8 T4096 C4096, forward + backward, 2.03 -> 2.04 ms), and a head that has any is marked by a NaN in the first element of each of its outputs, which wkv5_steps_*
+// look at: they do it over, step by step.  (The mark costs no workspace and no entry point, and a head whose first output is a NaN
+// by itself is merely done twice.)
+//
 // What bounds it.  Forward: HBM (B8 T4096 C4096: 2.9 GB in 0.60 ms; the sequential kernel took 1.3).  Backward: the fp32 matrix
 // instruction, which occupies a SIMD's vector ALU for 32 clocks (99 of them per SIMD and chunk and some 230 vector
 // instructions fill two thirds of its 1.40 ms; the three sequential sweeps took 4.1).  wkv5a: 0.67 + 1.83 ms, 6.2 before.
@@ -92,6 +98,16 @@ DEVINL float row_sum(float x) {
 }
 
 struct Head { float lam[N], lam2[N], u[N], u2[N], dec[N], dec2[N]; };
+
+// whether any element is no number, or infinite
+DEVINL bool not_finite(const f32x4& a, const f32x4& b, const f32x4& c, const f32x4& d = ZERO4) {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s = fmaf(a[e], 0.f, fmaf(b[e], 0.f, fmaf(c[e], 0.f, fmaf(d[e], 0.f, s))));
+    return s != 0.f;
+}
+// the mark, by the lane that has written this element before
+DEVINL void mark(float* first) { *first = __builtin_nanf(""); }
 
 // the head's parameters into LDS (by the first wave); every wave finds out for itself whether a decay is strong
 template <bool TWO> DEVINL bool head_setup(Head& hd, const ArgsC& p, int h, int tid) {
@@ -161,6 +177,7 @@ struct SmemF {
     Head hd;
     SlotF slot[3];
     float part[2][4][L][TS];            // the four waves' parts of the tile, of this chunk and the next
+    int marked;
 };
 constexpr int FDEPTH = 4;
 
@@ -265,6 +282,7 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base,
         }
         __syncthreads();
     }
+    if (q == 0 && lane == 0 && S.marked) mark(p.y + base);
 }
 
 template <bool TWO>
@@ -276,6 +294,7 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
     const size_t base = static_cast<size_t>(b) * T * C + static_cast<size_t>(h) * N;
     if (steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, h * N)) return;
     const bool strong = head_setup<TWO>(S.hd, p, h, tid);
+    if (tid == 0) S.marked = 0;
     __syncthreads();
     if (w >= 4) {
         const int tp = tid - 256, row = tp >> 4, c4 = (tp & 15) * 4;
@@ -291,6 +310,7 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
             f32x4 r = d[0], k = d[1], v = d[2];
             if (c * L + L > T && c * L + row >= T) { r = ZERO4; k = ZERO4; v = ZERO4; }
             st4(&s.r[row][c4], r); st4(&s.k[row][c4], k); st4(&s.v[row][c4], v);
+            if (not_finite(r, k, v)) S.marked = 1;
             const f32x4 rk = r * k;
             const float a = row_sum((rk[0] * u[0] + rk[1] * u[1]) + (rk[2] * u[2] + rk[3] * u[3]));
             if ((tp & 15) == 0) s.ruk[row] = a;
@@ -345,6 +365,7 @@ template <bool TWO> struct SmemB {
     float part[2][4][L][TS];            // halves of the tiles A (0, 1) and B (2, 3)
     float ds[2][N][PS];                 // the gradient state of the chunk, for the E waves: [chunk parity][i][j]
     float red[TWO ? 4 : 1][N];          // two-sided: the waves' sums over j of the per-element gradient
+    int marked;
 };
 
 // LDS by byte offset: the position of the chunk's slot (uniform) plus one of a few per-lane offsets, everything else an
@@ -561,6 +582,7 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
         p.gw[o] = l1 * gw;
         p.gu[o] = gu;
     }
+    if (q == 0 && lane == 0 && S.marked) { mark(p.gr + base); mark(p.gk + base); }
 }
 
 template <bool TWO, bool STRONG>
@@ -594,6 +616,7 @@ DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
         f32x4 r = d[0], k = d[1], v = d[2], gy = d[3];
         if (c * L + L > T && c * L + row >= T) { r = ZERO4; k = ZERO4; v = ZERO4; gy = ZERO4; }
         st4(&s.r[row][c4], r); st4(&s.k[row][c4], k); st4(&s.v[row][c4], v); st4(&s.g[row][c4], gy);
+        if (not_finite(r, k, v, gy)) S.marked = 1;
         if constexpr (TWO) { st4(&s.gs_[row][c4], gy * pgs); st4(&s.ve_[row][c4], v * pve); }
         const f32x4 rk = r * k, vg = v * gy;
         const float a = row_sum(sum4(rk * u)), e = row_sum(sum4(vg));
@@ -688,6 +711,7 @@ DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
         }
     }
     __syncthreads();
+    if (q == 0 && lane == 0 && S.marked) mark(p.gv + base);
     if constexpr (TWO) {
         gw2 = allreduce_rows(gw2); gu2 = allreduce_rows(gu2);
         if (g == 0) {
@@ -716,6 +740,7 @@ __global__ __launch_bounds__(NTB, 2) void wkv5c_bwd(const ArgsC p) {
     const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * N;
     if (steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, h * N)) return;
     const bool strong = head_setup<TWO>(S.hd, p, h, tid);
+    if (tid == 0) S.marked = 0;
     __syncthreads();
     if (strong) bwd_roles<TWO, true>(S, p, w, lane, h, b, base, nch);
     else bwd_roles<TWO, false>(S, p, w, lane, h, b, base, nch);

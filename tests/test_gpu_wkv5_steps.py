@@ -151,3 +151,29 @@ def test_bf16_head_that_the_forward_gave_up_is_redone_by_the_backward(lib, B, T,
     call("rwkv_wkv5s_backward", DEV, B, T, C, H, d[0], d[1], d[2], d[3], decay, d[4], d[5], gr, gk, gv, gw, gu, saved, nsv, ws, n, 0)
     for name, a, e, x in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, [y, gr, gk, gv, gw, gu]):
         assert_no_worse(name, a, e.reshape(a.shape), x.reshape(a.shape))
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("two", [False, True])
+def test_fp32_elements_that_are_not_finite_stay_where_they_act(lib, two, bad):
+    """In the middle of a chunk, one input at a time: the outputs and gradients that meet the element are not finite, all others of
+    its head are what they are without it, and other heads keep their bits."""
+    B, T, H, h, t0, c0 = 2, 60, 3, 1, 23, 9
+    x = _f32_inputs(B, T, H, 13)
+    clean = [z.view(-1, T, H, 64) for z in _run_f32(two, *x)[:4]]
+    t = torch.arange(T)
+    upto, since, at = t <= t0, t >= t0, t == t0
+    every, one = torch.ones(64, dtype=torch.bool), torch.arange(64) == c0
+    # input -> (tokens, channels) of y, gr, gk, gv that it reaches
+    reach = {0: [(at, every), None, (upto, one), (upto, every)], 1: [(since, every), (since, one), None, (at, every)],
+             2: [(since, one), (since, every), (at, every), None], 7: [None, (at, every), (upto, every), (upto, one)]}
+    for i, hits in reach.items():
+        y = list(x)
+        y[i] = x[i].clone()
+        y[i].view(B, T, H, 64)[1, t0, h, c0] = bad
+        got = [z.view(-1, T, H, 64) for z in _run_f32(two, *y)[:4]]
+        for name, a, g, hit in zip(("y", "gr", "gk", "gv"), clean, got, hits):
+            want = torch.zeros(T, 64, dtype=torch.bool) if hit is None else hit[0][:, None] & hit[1][None, :]
+            assert torch.equal(~torch.isfinite(g[1, :, h]), want), (i, name)
+            assert float((a[1, :, h] - g[1, :, h])[~want].abs().max() / a.abs().max()) <= 1e-5, (i, name)
+            assert torch.equal(a[0], g[0]) and torch.equal(a[1, :, [0, 2]], g[1, :, [0, 2]]), (i, name)
