@@ -1,6 +1,7 @@
 """GPU: the chunked fp32 kernels of wkv5 and wkv5a (head size 64) against the fp64 oracle, where they can go wrong: sequences of
-one token, of whole chunks (16 tokens), of whole segments between saved states (64 and 32 tokens) and one off, and decays of
-every strength up to those whose powers leave fp32's range within a chunk.
+one token, of whole chunks (16 tokens), of whole segments between saved states (48 and 32 tokens) and one off, and decays of
+every strength: up to the limit of the chunks' powers ("fast": the tiles with a reference per half chunk) and beyond it ("strong":
+half of the channels, so that nearly every head runs step by step).
 
 Tolerance: the fp32 ops' bar of 1e-5, relative to the largest element and to the RMS.  A sum of n fp32 products carries about
 sqrt(n) 6e-8; n is at most a few hundred here, and each product has up to six rounded factors: 2e-6.  wkv5a's slow decays
@@ -15,7 +16,7 @@ from rwkv_cuda_amd import options, wkv5, wkv5a
 from _gpu_util import DEV
 
 pytestmark = pytest.mark.gpu
-TS = [1, 2, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 81, 200]
+TS = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 81, 95, 96, 97, 143, 144, 145, 200]
 
 
 def _check(names, ref, got):
@@ -32,12 +33,12 @@ def _check(names, ref, got):
 def _inputs(B, T, H, seed, decays):
     g = torch.Generator().manual_seed(seed)
     rnd = lambda *s, lo=-1.0, hi=1.0: torch.rand(*s, generator=g) * (hi - lo) + lo
-    lo, hi = {"usual": (-1.0, 1.0), "slow": (-8.0, 1.0), "strong": (1.0, 3.5)}[decays]      # exp(-exp(3.5)) = 4e-15 a step
+    lo, hi = {"usual": (-1.0, 1.0), "slow": (-8.0, 1.0), "fast": (1.0, 2.83), "strong": (1.0, 3.5)}[decays]      # exp(-exp(3.5)) = 4e-15 a step
     C = H * 64
     return [rnd(B, T, C) for _ in range(3)], [rnd(H, 64, lo=lo, hi=hi), rnd(H, 64), rnd(H, 64, lo=lo, hi=hi), rnd(H, 64)], rnd(B, T, C)
 
 
-@pytest.mark.parametrize("decays", ["usual", "strong"])
+@pytest.mark.parametrize("decays", ["usual", "fast", "strong"])
 @pytest.mark.parametrize("T", TS)
 def test_wkv5(lib, T, decays):
     B, H = 2, 3
@@ -54,7 +55,7 @@ def test_wkv5(lib, T, decays):
         assert torch.equal(wkv5.RUN_CUDA(B, T, C, H, *t), y)
 
 
-@pytest.mark.parametrize("decays", ["usual", "slow", "strong"])
+@pytest.mark.parametrize("decays", ["usual", "slow", "fast", "strong"])
 @pytest.mark.parametrize("T", TS)
 def test_wkv5a(lib, T, decays):
     B, H = 2, 2
@@ -69,7 +70,7 @@ def test_wkv5a(lib, T, decays):
 
 
 def test_one_fast_channel_among_slow_ones(lib):
-    """A head takes the references of the strong case as a whole: its ordinary channels must not suffer."""
+    """A head takes the references of the fast case, or the steps, as a whole: its ordinary channels must not suffer."""
     B, T, H = 1, 70, 2
     C = H * 64
     (r, k, v), (w, u, _, _), gy = _inputs(B, T, H, 5, "usual")

@@ -1,7 +1,7 @@
 """GPU: bf16 wkv5 with heads of 128 channels, a workgroup per head (rwkv_wkv5s_*, what wkv5_bf16.RUN_CUDA runs), against the fp64
 oracle where it can go wrong: one token, whole chunks (32 tokens) and pairs of them (a saved state each) and one off, and decays
-of every strength: slow ones, some beyond what one reference token per chunk carries, and ones whose powers leave fp32's range
-within a few steps.  The bar is that of the other bf16 kernels: no further from fp64 than fp32 arithmetic with rounded outputs."""
+of every strength: slow ones, some beyond what one reference token per chunk carries ("fast": up to the limit of one per half a
+chunk), and ones beyond that, whose heads run step by step ("mixed", "strong": nearly all heads).  The bar is that of the other bf16 kernels: no further from fp64 than fp32 arithmetic with rounded outputs."""
 import pytest
 import torch
 
@@ -26,11 +26,11 @@ def _decays(kind, w):
     if kind == "usual":
         return w
     g = torch.Generator().manual_seed(5)
-    lo, hi = {"strong": (1.0, 4.0), "slow": (-8.0, -4.0), "mixed": (-6.0, 3.0)}[kind]      # exp(-exp(4)) = 2e-24 a step
+    lo, hi = {"fast": (-1.0, 2.18), "strong": (1.0, 4.0), "slow": (-8.0, -4.0), "mixed": (-6.0, 3.0)}[kind]      # exp(-exp(4)) = 2e-24 a step
     return (torch.rand(w.shape, generator=g) * (hi - lo) + lo).to(w.dtype)
 
 
-@pytest.mark.parametrize("decays", ["usual", "slow", "mixed", "strong"])
+@pytest.mark.parametrize("decays", ["usual", "slow", "fast", "mixed", "strong"])
 @pytest.mark.parametrize("T", [1, 2, 31, 32, 33, 63, 64, 65, 96, 97, 130, 260])
 def test_wkv5_whole_heads(lib, T, decays):
     B, H = 2, 2
@@ -58,7 +58,7 @@ def test_one_strong_head_among_others_changes_nothing_else(lib):
         assert torch.equal(x[:, :, 0], y[:, :, 0]) and torch.equal(x[:, :, 2], y[:, :, 2]) and not torch.equal(x[:, :, 1], y[:, :, 1])
 
 
-@pytest.mark.parametrize("decays", ["mixed", "strong"])
+@pytest.mark.parametrize("decays", ["fast", "mixed", "strong"])
 @pytest.mark.parametrize("T", [1, 31, 33, 64, 97, 260])
 def test_wkv5_head_size_64_with_a_strong_decay(lib, T, decays):
     """Head size 64 belongs to the one-sweep kernels until one channel of the layer decays too fast for them."""
