@@ -243,7 +243,8 @@ def make_wkv5(dev, H=32, N=64):
 
 
 def make_wkv5_fp32(dev):
-    """The fp32 wkv5 op at the reference's own benchmark shape (wkv5/run.py:395-399)."""
+    """The fp32 wkv5 op at the reference's own benchmark shape (wkv5/run.py:395-399): what the Python operator runs, one sweep each
+    way; with --algo sweeps the sequential sweeps behind the reference's signature."""
     from rwkv_cuda_amd import _lib
     from rwkv_cuda_amd._call import call
     lib = _lib.load()
@@ -258,8 +259,15 @@ def make_wkv5_fp32(dev):
     tok = B * T
     ew = (-torch.exp(w)).contiguous()
     eew = torch.exp(ew).contiguous()
+    saved, ws = (torch.empty(n(B, T, C, H), device=dev, dtype=torch.uint8) for n in (lib.rwkv_wkv5f32s_saved_bytes, lib.rwkv_wkv5f32s_backward_workspace_bytes))
+    fwd1 = lambda: call("rwkv_wkv5f32s_forward", dev, B, T, C, H, r, k, v, w, u, y, saved, saved.numel())
+    bwd1 = lambda: call("rwkv_wkv5f32s_backward", dev, B, T, C, H, r, k, v, w, u, gy, gr, gk, gv, gw[0], gu[0], saved, saved.numel(), ws, ws.numel())
 
     def step():
+        if ALGO == "chunked":
+            fwd1()
+            bwd1()
+            return gw[0], gu[0]
         ew_ = (-torch.exp(w)).contiguous()
         eew_ = torch.exp(ew_).contiguous()
         call("rwkv_wkv5f32_forward", dev, B, T, C, H, r, k, v, eew_, u, y)
@@ -275,6 +283,8 @@ def make_wkv5_fp32(dev):
                ("wkv_sweep<gr+gu+gw, fp32 I/O>", bwd(1), 20 * C * tok),       # r k v gy -> gr
                ("wkv_sweep<gv, fp32 I/O>", bwd(2), 16 * C * tok),             # r k gy -> gv
                ("wkv_sweep<gk, fp32 I/O>", bwd(4), 20 * C * tok)]             # r k v gy -> gk
+    if ALGO == "chunked":
+        kernels = [("wkv5c_fwd (keeps states)", fwd1, 16 * C * tok), ("wkv5c_bwd (+ batch sums)", bwd1, 28 * C * tok)]
 
     def cpu_baseline(t_cpu=128):
         from oracle import wkv56 as O
@@ -292,7 +302,7 @@ def make_wkv5_fp32(dev):
 
 
 def make_wkv5a(dev):
-    """wkv5a (two-sided decay and bonus, fp32) at the reference's timing shape (wkv5a/run.py:62-66)."""
+    """wkv5a (two-sided decay and bonus, fp32) at the reference's timing shape (wkv5a/run.py:62-66); kernels as for fp32 wkv5."""
     from rwkv_cuda_amd import _lib
     from rwkv_cuda_amd._call import call
     lib = _lib.load()
@@ -308,8 +318,16 @@ def make_wkv5a(dev):
     tok = B * T
     dec = lambda w: ((-torch.exp(w)).contiguous(), torch.exp(-torch.exp(w)).contiguous())
     (ew1, eew1), (ew2, eew2) = dec(w1), dec(w2)
+    saved, ws = (torch.empty(n(B, T, C, H), device=dev, dtype=torch.uint8) for n in (lib.rwkv_wkv5as_saved_bytes, lib.rwkv_wkv5as_backward_workspace_bytes))
+    grads1 = [x[0] for x in (gw1, gu1, gw2, gu2)]
+    fwd1 = lambda: call("rwkv_wkv5as_forward", dev, B, T, C, H, r, k, v, w1, u1, w2, u2, y, saved, saved.numel())
+    bwd1 = lambda: call("rwkv_wkv5as_backward", dev, B, T, C, H, r, k, v, w1, u1, w2, u2, gy, gr, gk, gv, *grads1, saved, saved.numel(), ws, ws.numel())
 
     def step():
+        if ALGO == "chunked":
+            fwd1()
+            bwd1()
+            return grads1
         (a1, b1), (a2, b2) = dec(w1), dec(w2)
         call("rwkv_wkv5a_forward", dev, B, T, C, H, r, k, v, b1, u1, b2, u2, y)
         call("rwkv_wkv5a_backward", dev, B, T, C, H, r, k, v, b1, a1, u1, b2, a2, u2, gy, gr, gk, gv, gw1, gu1, gw2, gu2)
@@ -324,6 +342,8 @@ def make_wkv5a(dev):
                ("wkv_sweep<gr+gu+gw, two-sided>", bwd(1), 20 * C * tok),
                ("wkv_sweep<gv, two-sided>", bwd(2), 16 * C * tok),
                ("wkv_sweep<gk, two-sided>", bwd(4), 20 * C * tok)]
+    if ALGO == "chunked":
+        kernels = [("wkv5c_fwd, two-sided (keeps states)", fwd1, 16 * C * tok), ("wkv5c_bwd, two-sided (+ batch sums)", bwd1, 28 * C * tok)]
 
     def cpu_baseline(t_cpu=128):
         from oracle import wkv5a as A
