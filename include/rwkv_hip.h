@@ -62,8 +62,16 @@ int rwkv_hbm_probe(void* stream, int mode, const void* src, void* dst, size_t by
 /* Per-call options of the *_ex entry points below (no counterpart in the reference).  Every *_ex function is its
  * reference-signature sibling plus a trailing `flags` word; the sibling is the same call with flags = 0.  Nothing here is
  * process-wide: two threads may run different algorithms or pass subsets at the same time.
- *   RWKV_FLAG_SWEEPS : wkv5 / wkv6 / wkv6_state run the sequential fp32 recurrence kernels instead of the chunked
- *                      matrix-core kernels (second algorithm; the parity anchor of the chunked kernels).
+ *   RWKV_FLAG_SWEEPS : wkv5 / wkv6 / wkv6_state and the rwkv7 state-passing op (bf16 and fp32) run the sequential fp32
+ *                      recurrence kernels instead of the chunked matrix-core kernels (second algorithm; the parity anchor
+ *                      of the chunked kernels).
+ *
+ * Inputs that are not finite.  The bf16 chunked kernels (wkv5, wkv6, wkv6_state) and the chunked rwkv7 kernels, fp32 mode
+ * included, multiply what a causal tile leaves out by zero: a NaN or an infinity in an input reaches, besides all that it acts
+ * on, outputs of the tokens before it (and gradients of those after it) within its chunk of 16 (rwkv7) or 32 tokens of its
+ * head; so do the two-term fp16 kernels of depthwise_conv1d, within 32 steps of a unit of 32 batch rows of a channel.  The
+ * sequential kernels, those of fp32 wkv5 and wkv5a, and the three-term kernels of depthwise_conv1d keep it to where it acts.
+ *
  *   RWKV_PASS_*      : restrict a backward to a subset of its kernels so that a profiler can time one kernel per call
  *                      (no pass bit set = all of them).  Sequential kernels: GR (gr, gu, workspace), GV (gv), GK (gk, gw,
  *                      gs; reads the workspace GR left).  Chunked kernels: GR selects the first sweep (gr, gu, workspace),
@@ -250,8 +258,9 @@ int rwkv_wkv5a_backward_ex(void* stream, int B, int T, int C, int H,
  * matrix cores: one forward, one reverse sweep.
  *   `saved` (*_saved_bytes; 0 for another head size, which these entry points refuse with RWKV_ERR_SHAPE): the forward keeps
  *   the state entering every third (wkv5a: second) chunk of 16 tokens for the backward of the same step; NULL for a forward
- *   without a backward.  `workspace` (*_backward_workspace_bytes): per-batch rows of the parameter gradients.  The raw decays
- *   (w, w1, w2) may have any alignment.
+ *   without a backward: 16 KB per head and 48 (wkv5a: 32) tokens, 721 MB (1.07 GB) at B8 T4096 C4096.  `workspace`
+ *   (*_backward_workspace_bytes): per-batch rows of the parameter gradients.  The raw decays (w, w1, w2) may have any alignment.
+ *   Heads with a decay below e^-17 a step, a decay that is no number, or an input that is not finite run step by step.
  * ------------------------------------------------------------------------------------- */
 size_t rwkv_wkv5f32s_saved_bytes(int B, int T, int C, int H);
 int rwkv_wkv5f32s_forward(void* stream, int B, int T, int C, int H,
@@ -357,7 +366,9 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H,
  * floats) left by the forward for the backward, gw, gu [H,N] summed over time and batch out.  The decay of a channel
  * stands in for every token's decay in the kernels of rwkv_wkv6f_*, and its gradient is added up over the tokens inside
  * the kernel.  Head size 128: one workgroup holds a whole head; the forward may go without `saved` (nothing is kept then),
- * and the backward needs no more workspace than 4 B C bytes.  Other head sizes, RWKV_FLAG_SWEEPS / RWKV_PASS_* or (size 64)
+ * and the backward needs no more workspace than 4 B C bytes.  Heads with a decay below e^-9 a step, or one that is no number,
+ * run step by step, at both sizes.  `saved`: 64 KB (size 64: 16 KB, for any layer) per head and 64 tokens, 1.07 GB at B8 T4096
+ * C4096 (268 MB at C2048).  Other head sizes, RWKV_FLAG_SWEEPS / RWKV_PASS_* or (size 64)
  * saved = NULL: rwkv_wkv5raw_forward / _backward. */
 size_t rwkv_wkv5s_saved_bytes(int B, int T, int C, int H);
 int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H,
@@ -475,7 +486,7 @@ int rwkv7_backward(void* stream, int B, int T, int H,
 
 /* fp32 I/O for the three rwkv7 ops: what the reference builds from the same sources with -D_FP32_, where `bf` is float
  * (rwkv7_clampw.cu:3-7, rwkv7_cuda_benchmark.py:102-126, and the same lines of the _state and _state_passing siblings).
- * Same arguments as the bf16 entry points with every bf16 tensor fp32; same kernels and fp32 arithmetic. */
+ * Same arguments as the bf16 entry points with every bf16 tensor fp32; same (chunked) kernels and fp32 arithmetic. */
 int rwkv7_statepassing_forward_f32(void* stream, int B, int T, int H,
                                    const float* s0, const float* r, const float* w, const float* k,
                                    const float* v, const float* a, const float* b,

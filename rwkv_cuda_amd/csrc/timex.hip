@@ -577,9 +577,9 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // Operands are THREE bf16 terms, x = h + m + l (each the nearest of what is left: all 24 bits of x), and a product is
 //     x y = h h' + h m' + m h' + m m' + h l' + l h'            (the terms left out are below 2^-24 of the product, 2^-26 rms)
 // with fp32's exponents.  The five small products have accumulators of their own: the sum of the large ones, whose roundings are
-// what is left of an error, rounds once an instruction.  Nothing is scaled, so nothing is scaled and an element's accuracy does not depend on its neighbours: short rows, rows
-// that grow late and batches of unequal rows come out as from an fp32 loop, which two fp16 terms under a common power of two
-// (half the products, 58 and 101 us where these take 95 and 111) do not give.  A unit with an element that is no number, infinite or beyond
+// what is left of an error, rounds once an instruction.  Nothing is scaled, so an element's accuracy does not depend on its
+// neighbours: short rows, rows that grow late and batches of unequal rows come out as from an fp32 loop, which two fp16 terms
+// under a common power of two (half the products, 58 and 101 us where these take 95 and 111) do not give.  A unit with an element that is no number, infinite or beyond
 // bf16's largest is done by such a loop (a matrix product would carry it to earlier steps: zero times infinity).
 // Rows lie in LDS as blocks of 32 + 8 terms (80 bytes: 16-byte reads of neighbouring columns fall on different banks if a
 // row has an odd number of blocks), 512 threads, 128 registers, and up to T = 2900 (gradient) and 3360 at most 80 KB: two

@@ -28,9 +28,9 @@
 //
 // Inputs that are no number, or infinite: a tile product multiplies what it leaves out by zero, which would carry them to up to 15
 // tokens that they do not act on (earlier outputs, later gradients).  The waves that load note them (one multiply-add an element;
-// wkv5 B8 T4096 C4096, forward + backward, 2.03 -> 2.04 ms), and a head that has any is marked by a NaN in the first element of each of its outputs, which wkv5_steps_*
-// look at: they do it over, step by step.  (The mark costs no workspace and no entry point, and a head whose first output is a NaN
-// by itself is merely done twice.)
+// wkv5 B8 T4096 C4096, forward + backward, 2.03 -> 2.04 ms), and a head that has any is marked by a NaN in the first element of
+// each of its outputs, which wkv5_steps_* look at: they do it over, step by step.  (The mark costs no workspace and no entry
+// point, and a head whose first output is a NaN by itself is merely done twice.)
 //
 // What bounds it.  Forward: HBM (B8 T4096 C4096: 2.9 GB in 0.60 ms; the sequential kernel took 1.3).  Backward: the fp32 matrix
 // instruction, which occupies a SIMD's vector ALU for 32 clocks (99 of them per SIMD and chunk and some 230 vector

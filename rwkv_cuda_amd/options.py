@@ -1,4 +1,4 @@
-"""Per-call kernel options for the wkv5 / wkv6 / wkv6_state wrappers.
+"""Per-call kernel options for the wkv5 (bf16 and fp32) / wkv5a / wkv6 / wkv6_state wrappers and the rwkv7 state-passing op.
 
 The C ABI takes them as the `flags` word of its *_ex entry points; nothing is process-wide there.  On the Python side a
 `with algorithm("sweeps"):` block selects the sequential kernels for every forward issued inside it by this thread; the
