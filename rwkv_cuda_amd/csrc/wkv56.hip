@@ -116,13 +116,18 @@ template <bool F32> DEVINL void store1(uint16_t* p, size_t i, float x) {
     else p[i] = f2bf(x);
 }
 
+// wkv5: a channel's log decay from the raw parameter; d decay / d raw from the two, zero where the decay is (the log decay may have
+// left fp32's range there)
+template <bool F32> DEVINL float raw_log_decay(const void* raw, int c) { return -expf(load1<F32>(static_cast<const uint16_t*>(raw), c)); }
+template <bool STEPS> DEVINL float decay_grad(float lw, float w) { return STEPS && w == 0.f ? 0.f : lw * w; }
+
 template <bool F32> struct Staged {
     Raw8<F32> r, k, v, g;
     uint4 w0, w1;
     float4 rdr0, rdr1;
 };
 
-template <int PASS, int WMODE, bool F32>
+template <int PASS, int WMODE, bool F32, bool STEPS>
 DEVINL void prefetch(Staged<F32>& p, const Args& a, size_t base, int c0, int st, int sj) {
     const int t = c0 + st;
     const bool ok = t < a.T;
@@ -139,7 +144,7 @@ DEVINL void prefetch(Staged<F32>& p, const Args& a, size_t base, int c0, int st,
         p.w0 = ok ? *reinterpret_cast<const uint4*>(w) : z;
         p.w1 = ok ? *reinterpret_cast<const uint4*>(w + 4) : z;
     }
-    if constexpr (PASS == P_GK && !F32) {
+    if constexpr (PASS == P_GK && !F32 && !STEPS) {
         const float4 zf = make_float4(0.f, 0.f, 0.f, 0.f);
         p.rdr0 = ok ? *reinterpret_cast<const float4*>(a.rdr + off) : zf;
         p.rdr1 = ok ? *reinterpret_cast<const float4*>(a.rdr + off + 4) : zf;
@@ -157,7 +162,7 @@ DEVINL void ld8f(const float* src, float (&f)[8]) {
 }
 
 // registers -> LDS (fp32), plus the per-step scalar `dot`
-template <int PASS, int WMODE, bool F32, bool TWO>
+template <int PASS, int WMODE, bool F32, bool TWO, bool STEPS>
 DEVINL void commit(Smem<PASS>& S, const Staged<F32>& p, const Args& a, int c0, int st, int sj) {
     const bool ok = (c0 + st) < a.T;
     float fr[8], fk[8], fv[8], fg[8];
@@ -190,7 +195,7 @@ DEVINL void commit(Smem<PASS>& S, const Staged<F32>& p, const Args& a, int c0, i
             st8(&S.f[st][sj], fw);
         }
     }
-    if constexpr (PASS == P_GK && !F32) {
+    if constexpr (PASS == P_GK && !F32 && !STEPS) {
         *reinterpret_cast<float4*>(&S.rdr[st][sj]) = p.rdr0;
         *reinterpret_cast<float4*>(&S.rdr[st][sj + 4]) = p.rdr1;
     }
@@ -230,13 +235,16 @@ DEVINL void commit(Smem<PASS>& S, const Staged<F32>& p, const Args& a, int c0, i
     }
 }
 
-template <int PASS, int WMODE, bool F32 = false, bool TWO = false>
-__global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
+// STEPS (wkv5 only): w (w2) are the raw decays and GR carries Q in either precision, so that no pass needs another's workspace.
+template <int PASS, int WMODE, bool F32, bool TWO, bool STEPS>
+DEVINL void sweep_body(Smem<PASS>& S, const Args& a) {
+    static_assert(!STEPS || WMODE == W_HEAD, "raw decays per channel");
     static_assert(!F32 || WMODE == W_HEAD, "fp32 I/O exists for wkv5 only");
     static_assert(!TWO || F32, "the two-sided op is fp32 only, as in the reference (wkv5a_cuda_v1a2.cu:5)");
     constexpr bool REV = (PASS == P_GK || PASS == P_GV);
     constexpr bool SHAPE_F = (PASS == P_FWD || PASS == P_GV);
-    __shared__ Smem<PASS> S;
+    auto log_decay = [](const float* ew, const void* raw, int c) { return STEPS ? raw_log_decay<F32>(raw, c) : ew[c]; };
+    auto decay = [](const void* w, int c) { return STEPS ? expf(raw_log_decay<F32>(w, c)) : static_cast<const float*>(w)[c]; };
 
     const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
     const int b = blockIdx.x / a.H, h = blockIdx.x % a.H;
@@ -250,7 +258,7 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
     if constexpr (TWO) {
         if (tid < N) {
             S.u2[tid] = load1<F32>(a.u2, h * N + tid);
-            S.w2[tid] = a.w2[h * N + tid];
+            S.w2[tid] = decay(a.w2, h * N + tid);
         }
     }
 
@@ -274,8 +282,7 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
     // time-constant decay (wkv5)
     float w_const = 1.f;
     if constexpr (WMODE == W_HEAD) {
-        const float* eew = static_cast<const float*>(a.w) + h * N;
-        w_const = SHAPE_F ? eew[rowslot] : eew[lane];
+        w_const = decay(a.w, h * N + (SHAPE_F ? rowslot : lane));
     }
 #pragma unroll
     for (int e = 0; e < JW; ++e) asm volatile("" : "+v"(St[e]));
@@ -288,14 +295,12 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
     constexpr bool REGW = TWO || (WMODE == W_HEAD && SHAPE_F);
     float wreg[REGW ? JW : 1];
     if constexpr (TWO) {
-        const float* w1 = static_cast<const float*>(a.w) + h * N;
-        const float* w2 = a.w2 + h * N;
 #pragma unroll
-        for (int e = 0; e < JW; ++e) wreg[e] = SHAPE_F ? w1[q * JW + e] * w2[lane] : w1[lane] * w2[q * JW + e];
+        for (int e = 0; e < JW; ++e)
+            wreg[e] = SHAPE_F ? decay(a.w, h * N + q * JW + e) * decay(a.w2, h * N + lane) : decay(a.w, h * N + lane) * decay(a.w2, h * N + q * JW + e);
     } else if constexpr (REGW) {
-        const float* eew = static_cast<const float*>(a.w) + h * N;
 #pragma unroll
-        for (int e = 0; e < JW; ++e) wreg[e] = eew[q * JW + e];
+        for (int e = 0; e < JW; ++e) wreg[e] = decay(a.w, h * N + q * JW + e);
     }
     if constexpr (REGW) {
 #pragma unroll
@@ -309,8 +314,8 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
     // fp32 I/O: the P recurrence above loses a digit per decade of T to cancellation, which bf16 outputs hide and
     // fp32 outputs do not.  GR carries Q = dS/dw instead (Q_{t+1} = S_t + w Q_t, the reference's second recurrence,
     // wkv5/run.py:249-252) and sums gw[j] = sum_t r_t[j] sum_i gy_t[i] Q_t[i,j] per lane; GK then makes gk only.
-    constexpr bool DIRECT_GW = F32 && PASS == P_GR;
-    constexpr bool SCAN_GW = !F32 && PASS == P_GK;
+    constexpr bool DIRECT_GW = (F32 || STEPS) && PASS == P_GR;
+    constexpr bool SCAN_GW = !F32 && !STEPS && PASS == P_GK;
     float Q[DIRECT_GW ? JW : 1];
 #pragma unroll
     for (int e = 0; e < (DIRECT_GW ? JW : 1); ++e) Q[e] = 0.f;
@@ -327,15 +332,15 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
     const int nchunks = (a.T + TC - 1) / TC;
     const bool stager = tid < NSTAGE;                       // whole waves
     Staged<F32> pre;
-    if (stager) prefetch<PASS, WMODE, F32>(pre, a, base, (REV ? nchunks - 1 : 0) * TC, st, sj);
+    if (stager) prefetch<PASS, WMODE, F32, STEPS>(pre, a, base, (REV ? nchunks - 1 : 0) * TC, st, sj);
     __syncthreads();                                        // S.u (u2, w2) visible
 
     for (int ci = 0; ci < nchunks; ++ci) {
         const int c0 = (REV ? nchunks - 1 - ci : ci) * TC;
         __syncthreads();                                    // previous epilogue is done with LDS
-        if (stager) commit<PASS, WMODE, F32, TWO>(S, pre, a, c0, st, sj);
+        if (stager) commit<PASS, WMODE, F32, TWO, STEPS>(S, pre, a, c0, st, sj);
         __syncthreads();
-        if (stager && ci + 1 < nchunks) prefetch<PASS, WMODE, F32>(pre, a, base, (REV ? nchunks - 2 - ci : ci + 1) * TC, st, sj);
+        if (stager && ci + 1 < nchunks) prefetch<PASS, WMODE, F32, STEPS>(pre, a, base, (REV ? nchunks - 2 - ci : ci + 1) * TC, st, sj);
 
         // ---- TC sequential steps
 #pragma unroll 4
@@ -416,7 +421,7 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
             }
             if (ok) {
                 store8<F32>(a.gr, off, out);
-                if constexpr (!F32) {
+                if constexpr (!F32 && !STEPS) {
                     *reinterpret_cast<float4*>(a.rdr + off) = make_float4(rdr[0], rdr[1], rdr[2], rdr[3]);
                     *reinterpret_cast<float4*>(a.rdr + off + 4) = make_float4(rdr[4], rdr[5], rdr[6], rdr[7]);
                 }
@@ -470,8 +475,7 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
                 float s = 0.f;
 #pragma unroll
                 for (int w = 0; w < NW; ++w) s += S.part[w][0][tid];
-                const float eew = static_cast<const float*>(a.w)[h * N + tid];   // d eew / d w_raw = eew * ew
-                store1<F32>(a.gw, static_cast<size_t>(b) * a.C + h * N + tid, a.ew_head[h * N + tid] * eew * s);
+                store1<F32>(a.gw, static_cast<size_t>(b) * a.C + h * N + tid, decay_grad<STEPS>(log_decay(a.ew_head, a.w, h * N + tid), decay(a.w, h * N + tid)) * s);
             }
         }
         if constexpr (TWO) {
@@ -491,7 +495,7 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
             if (tid < N) {                                                        // tid = i
                 float s = 0.f;
                 for (int j = 0; j < N; ++j) s += S.part[tid / JW][tid % JW][(j + tid) & (N - 1)];
-                store1<F32>(a.gw2, static_cast<size_t>(b) * a.C + h * N + tid, a.ew2_head[h * N + tid] * a.w2[h * N + tid] * s);
+                store1<F32>(a.gw2, static_cast<size_t>(b) * a.C + h * N + tid, decay_grad<STEPS>(log_decay(a.ew2_head, a.w2, h * N + tid), decay(a.w2, h * N + tid)) * s);
             }
         }
     }
@@ -509,6 +513,12 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
     }
 }
 
+template <int PASS, int WMODE, bool F32 = false, bool TWO = false>
+__global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
+    __shared__ Smem<PASS> S;
+    sweep_body<PASS, WMODE, F32, TWO, false>(S, a);
+}
+
 // ----------------------------------------------------------------------------------------------------------------------
 // Head sizes other than 64 (the reference builds its kernels with -D_N_=HEAD_SIZE: wkv5_bf16/run.py:21 ships 128, the
 // self-checks of wkv5/run.py, wkv6/run.py and wkv6_state/run.py use 2, 4 and 8).  One workgroup per (batch, head).  A row
@@ -516,7 +526,7 @@ __global__ __launch_bounds__(NT) void wkv_sweep(const Args a) {
 // each, so every sum of the recurrence is a private loop over LDS-broadcast vectors plus one or two cross-lane adds.
 // Same passes, formulas, rounding points and workspace as the sweeps above; hn (the head size, 1..NP) is a run-time
 // value, NP the padded size the registers are unrolled for.
-// STEPS (wkv5 only): w (w2) are the raw decays and GR carries Q in either precision, so that no pass needs another's workspace.
+// STEPS: as in sweep_body.
 constexpr int GTC = 16;          // time steps per staged chunk
 
 // The step loops below are unrolled over a thread's part of a state row.  Left alone, the compiler issues all of the LDS
@@ -569,10 +579,8 @@ DEVINL void rows_body(SmemRows<NP, PARTS, PASS, F32, TWO, STEPS>& S, const Args&
     constexpr bool DIRECT_GW = (F32 || STEPS) && PASS == P_GR;  // as in wkv_sweep: the fp32 op carries Q = dS/dw
     constexpr bool SCAN_GW = SmemRows<NP, PARTS, PASS, F32, TWO, STEPS>::kScan;
     // the log decay and the decay of a channel of this layer
-    auto log_decay = [](const float* ew, const void* raw, int c) { return STEPS ? -expf(load1<F32>(static_cast<const uint16_t*>(raw), c)) : ew[c]; };
-    auto decay = [](const void* w, int c) { return STEPS ? expf(-expf(load1<F32>(static_cast<const uint16_t*>(w), c))) : static_cast<const float*>(w)[c]; };
-    // d decay / d raw = decay x log decay, zero where the decay is (the log decay may have left fp32's range there)
-    auto decay_grad = [](float lw, float w) { return STEPS && w == 0.f ? 0.f : lw * w; };
+    auto log_decay = [](const float* ew, const void* raw, int c) { return STEPS ? raw_log_decay<F32>(raw, c) : ew[c]; };
+    auto decay = [](const void* w, int c) { return STEPS ? expf(raw_log_decay<F32>(w, c)) : static_cast<const float*>(w)[c]; };
 
     const int tid = threadIdx.x;
     const int row = tid / PARTS, part = tid % PARTS;            // threads beyond NP * PARTS (NP * PARTS < 64) only idle
@@ -771,7 +779,7 @@ DEVINL void rows_body(SmemRows<NP, PARTS, PASS, F32, TWO, STEPS>& S, const Args&
     if constexpr (PASS == P_GR) {
         if (writer) {
             store1<F32>(a.gu, pc, gu_acc);
-            if constexpr (DIRECT_GW) store1<F32>(a.gw, pc, decay_grad(log_decay(a.ew_head, a.w, h * hn + row), w_row) * gw_acc);     // d eew / d w_raw = eew * ew
+            if constexpr (DIRECT_GW) store1<F32>(a.gw, pc, decay_grad<STEPS>(log_decay(a.ew_head, a.w, h * hn + row), w_row) * gw_acc);     // d eew / d w_raw = eew * ew
         }
         if constexpr (GW2) {
             // gu2: the staging groups' partial sums, one row of LDS per group
@@ -796,7 +804,7 @@ DEVINL void rows_body(SmemRows<NP, PARTS, PASS, F32, TWO, STEPS>& S, const Args&
                     for (int q = 0; q < (NP < GTC ? NP : GTC); ++q) tot += S.k[q][cat];
             }
             if (tid < NP && chan)
-                store1<F32>(a.gw2, static_cast<size_t>(b) * a.C + static_cast<size_t>(h) * hn + cn, decay_grad(log_decay(a.ew2_head, a.w2, h * hn + cn), decay(a.w2, h * hn + cn)) * tot);
+                store1<F32>(a.gw2, static_cast<size_t>(b) * a.C + static_cast<size_t>(h) * hn + cn, decay_grad<STEPS>(log_decay(a.ew2_head, a.w2, h * hn + cn), decay(a.w2, h * hn + cn)) * tot);
         }
     }
     if constexpr (PASS == P_GK) {
@@ -820,7 +828,9 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
 }
 
 // The heads of a wkv5 layer whose decay the chunked kernels do not carry (steps_head, common.h), step by step; all other
-// workgroups return at once.  Backward: the three passes, which need nothing of each other, side by side.
+// workgroups return at once.  Backward: the three passes, which need nothing of each other, side by side.  Heads of 64 on the body
+// of wkv_sweep (a layer of B8 T4096 with one such head: bf16 3.1 ms, fp32 C4096 5.0 ms; on the rows above 4.2 and more), those of
+// 128 on the rows.
 // bf16, heads of 64, in a layer without a strong decay: the heads that a one-sweep kernel has given up (its flag words, of the
 // forward and in the backward of both directions: such a forward has left no states).
 // fp32: also the heads whose inputs are not all finite, which the chunked kernels mark by a NaN in the first element of each output
@@ -842,23 +852,32 @@ template <int NP, bool F32, bool TWO> DEVINL bool steps_for(const Args& a, const
     }
     return steps_head<F32, NP>(a.w, TWO ? a.w2 : nullptr, (blockIdx.x % a.H) * NP);
 }
-template <int NP, int PARTS, bool F32, bool TWO>
-__global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_fwd(const Args a, const int hn) {
-    if (!steps_for<NP, F32, TWO>(a, a.y)) return;
-    __shared__ SmemRows<NP, PARTS, P_FWD, F32, TWO, true> S;
-    rows_body<NP, PARTS, P_FWD, W_HEAD, F32, TWO, true>(S, a, hn);
+template <bool F32, bool TWO> __global__ __launch_bounds__(NT) void wkv5_steps_fwd(const Args a) {
+    if (!steps_for<N, F32, TWO>(a, a.y)) return;
+    __shared__ Smem<P_FWD> S;
+    sweep_body<P_FWD, W_HEAD, F32, TWO, true>(S, a);
 }
-template <int NP, int PARTS, bool F32, bool TWO>
-__global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv5_steps_bwd(const Args a, const int hn) {
-    if (!steps_for<NP, F32, TWO>(a, blockIdx.y == 0 ? a.gr : (blockIdx.y == 1 ? a.gv : a.gk))) return;
-    __shared__ union {
-        SmemRows<NP, PARTS, P_GR, F32, TWO, true> gr;
-        SmemRows<NP, PARTS, P_GV, F32, TWO, true> gv;
-        SmemRows<NP, PARTS, P_GK, F32, TWO, true> gk;
-    } S;
-    if (blockIdx.y == 0) rows_body<NP, PARTS, P_GR, W_HEAD, F32, TWO, true>(S.gr, a, hn);
-    else if (blockIdx.y == 1) rows_body<NP, PARTS, P_GV, W_HEAD, F32, TWO, true>(S.gv, a, hn);
-    else rows_body<NP, PARTS, P_GK, W_HEAD, F32, TWO, true>(S.gk, a, hn);
+template <bool F32, bool TWO> __global__ __launch_bounds__(NT) void wkv5_steps_bwd(const Args a) {
+    if (!steps_for<N, F32, TWO>(a, blockIdx.y == 0 ? a.gr : (blockIdx.y == 1 ? a.gv : a.gk))) return;
+    __shared__ union { Smem<P_GR> gr; Smem<P_GV> gv; Smem<P_GK> gk; } S;
+    if (blockIdx.y == 0) sweep_body<P_GR, W_HEAD, F32, TWO, true>(S.gr, a);
+    else if (blockIdx.y == 1) sweep_body<P_GV, W_HEAD, F32, TWO, true>(S.gv, a);
+    else sweep_body<P_GK, W_HEAD, F32, TWO, true>(S.gk, a);
+}
+// heads of 128 channels, bf16
+using Geom128 = RowGeom<128, 4>;
+template <int PASS> using Smem128 = SmemRows<128, 4, PASS, false, false, true>;
+__global__ __launch_bounds__(Geom128::NTHREADS) void wkv5_steps_fwd_128(const Args a) {
+    if (!steps_for<128, false, false>(a, a.y)) return;
+    __shared__ Smem128<P_FWD> S;
+    rows_body<128, 4, P_FWD, W_HEAD, false, false, true>(S, a, 128);
+}
+__global__ __launch_bounds__(Geom128::NTHREADS) void wkv5_steps_bwd_128(const Args a) {
+    if (!steps_for<128, false, false>(a, a.gr)) return;
+    __shared__ union { Smem128<P_GR> gr; Smem128<P_GV> gv; Smem128<P_GK> gk; } S;
+    if (blockIdx.y == 0) rows_body<128, 4, P_GR, W_HEAD, false, false, true>(S.gr, a, 128);
+    else if (blockIdx.y == 1) rows_body<128, 4, P_GV, W_HEAD, false, false, true>(S.gv, a, 128);
+    else rows_body<128, 4, P_GK, W_HEAD, false, false, true>(S.gk, a, 128);
 }
 
 constexpr int MAX_HEAD = 128;
@@ -1039,8 +1058,8 @@ int launch_wkv5f32_steps_fwd(hipStream_t st, int B, int T, int H, const float* r
     Args a{};
     a.T = T; a.C = H * N; a.H = H; a.r = as_elems(r); a.k = as_elems(k); a.v = as_elems(v); a.w = w; a.u = as_elems(u); a.w2 = w2;
     a.u2 = as_elems(u2); a.y = out_elems(y);
-    const auto kernel = w2 != nullptr ? wkv5_steps_fwd<64, 4, true, true> : wkv5_steps_fwd<64, 4, true, false>;
-    hipLaunchKernelGGL(kernel, dim3(B * H), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    const auto kernel = w2 != nullptr ? wkv5_steps_fwd<true, true> : wkv5_steps_fwd<true, false>;
+    hipLaunchKernelGGL(kernel, dim3(B * H), dim3(NT), 0, st, a);
     return launch_status();
 }
 namespace {
@@ -1049,8 +1068,8 @@ int launch_wkv5_steps_fwd(hipStream_t st, int B, int T, int C, int H, const uint
                           const uint16_t* w, const uint16_t* u, uint16_t* y, const int* flags) {
     Args a{};
     a.T = T; a.C = C; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.y = y; a.flags = flags;
-    if (C == H * N) hipLaunchKernelGGL((wkv5_steps_fwd<64, 4, false, false>), dim3(B * H), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
-    else hipLaunchKernelGGL((wkv5_steps_fwd<128, 4, false, false>), dim3(B * H), dim3(RowGeom<128, 4>::NTHREADS), 0, st, a, N_SPLIT);
+    if (C == H * N) hipLaunchKernelGGL((wkv5_steps_fwd<false, false>), dim3(B * H), dim3(NT), 0, st, a);
+    else hipLaunchKernelGGL(wkv5_steps_fwd_128, dim3(B * H), dim3(Geom128::NTHREADS), 0, st, a);
     return launch_status();
 }
 int launch_wkv5_steps_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
@@ -1059,8 +1078,8 @@ int launch_wkv5_steps_bwd(hipStream_t st, int B, int T, int C, int H, const uint
     Args a{};
     a.T = T; a.C = C; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.gy = gy; a.gr = gr; a.gk = gk; a.gv = gv; a.gw = gw;
     a.gu = gu; a.flags = flags_fwd; a.flags2 = flags_bwd;
-    if (C == H * N) hipLaunchKernelGGL((wkv5_steps_bwd<64, 4, false, false>), dim3(B * H, 3), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
-    else hipLaunchKernelGGL((wkv5_steps_bwd<128, 4, false, false>), dim3(B * H, 3), dim3(RowGeom<128, 4>::NTHREADS), 0, st, a, N_SPLIT);
+    if (C == H * N) hipLaunchKernelGGL((wkv5_steps_bwd<false, false>), dim3(B * H, 3), dim3(NT), 0, st, a);
+    else hipLaunchKernelGGL(wkv5_steps_bwd_128, dim3(B * H, 3), dim3(Geom128::NTHREADS), 0, st, a);
     return launch_status();
 }
 }  // namespace
@@ -1071,8 +1090,8 @@ int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r
     a.T = T; a.C = H * N; a.H = H; a.r = as_elems(r); a.k = as_elems(k); a.v = as_elems(v); a.w = w; a.u = as_elems(u); a.w2 = w2;
     a.u2 = as_elems(u2); a.gy = as_elems(gy); a.gr = out_elems(gr); a.gk = out_elems(gk); a.gv = out_elems(gv); a.gw = out_elems(gw);
     a.gu = out_elems(gu); a.gw2 = out_elems(gw2); a.gu2 = out_elems(gu2);
-    const auto kernel = w2 != nullptr ? wkv5_steps_bwd<64, 4, true, true> : wkv5_steps_bwd<64, 4, true, false>;
-    hipLaunchKernelGGL(kernel, dim3(B * H, 3), dim3(RowGeom<64, 4>::NTHREADS), 0, st, a, N);
+    const auto kernel = w2 != nullptr ? wkv5_steps_bwd<true, true> : wkv5_steps_bwd<true, false>;
+    hipLaunchKernelGGL(kernel, dim3(B * H, 3), dim3(NT), 0, st, a);
     return launch_status();
 }
 

@@ -23,13 +23,14 @@
 // to wkv5_steps_* (steps_head, common.h): with a reference per 8 tokens, and a product for each distance of two such blocks, the
 // loops spill hundreds of registers, and decays below e^-17 are out of reach all the same.
 // Handing every head with a strong decay (|l| > 3.7) to step-by-step kernels, as the kernels before did, made one such channel in
-// 4096 cost more than everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 ms with.  That is why
-// layers of 64-channel heads come here as well once they have such a channel (0.74 ms at B8 T4096 C2048 where they took 1.66 ms).
+// 4096 cost more than everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 to 11.3 ms with.  That is
+// why layers of 64-channel heads come here as well once they have such a channel (B8 T4096 C2048: 0.60 ms with a channel at
+// l = -4.5, 0.70 at -8.6, where they took 1.7 to 3.8 ms).
 //
-// What bounds it (B8 T4096 C4096: one workgroup per CU).  Forward 0.52 ms for 2.1 GB, half of them the saved states: HBM (4.1 TB/s;
-// 0.82 ms as four heads of 64).  Backward 1.03 ms: the D waves, some 1600 vector and 170 matrix instructions a chunk, and their
+// What bounds it (B8 T4096 C4096: one workgroup per CU).  Forward 0.43 ms for 2.1 GB, half of them the saved states: HBM (5.0 TB/s;
+// 0.82 ms as four heads of 64).  Backward 1.05 ms: the D waves, some 1600 vector and 170 matrix instructions a chunk, and their
 // waits for the saved state (2.95 ms as two sweeps over four heads of 64, whose fp32 terms went through memory).  Both together
-// 6.56 -> 1.49 ms where a channel's decay was strong, 3.87 -> 1.48 where none was.
+// 6.56 -> 1.47 ms where a channel's decay was strong, 3.83 -> 1.48 where none was.
 #include <stddef.h>
 
 #include "wkv6_fused.h"
