@@ -24,35 +24,33 @@
 //     da = dA' e^{c_t - c_m}, dr = dR' e^{c_{t+1} - c_m}, db = dB' e^{c_m - c_{t+1}}, dk likewise
 //     decay: with P_t = sum_i dS_t o S_t per key channel,  G_t = P_{t+1} + r dr - b db - k dk,  P_t = G_t + a da,
 //            dw_raw = G W_SCALE sig (1 - sig);  P at the end of the call = sum_i dsT o S_T.
-// Every product is an fp32 matrix instruction (no operand is rounded below fp32), so the fp32 outputs sT, ds0 and the
-// saved sa keep the accuracy class of the reference's fp32 recurrence; the bf16 outputs are rounded once at the store.
-// The fp32 mode is therefore the same kernel with fp32 loads and stores (B8 T1024 C4096, forward + backward: 1.20 ms, the
-// step-by-step recurrence on the vector units took 1.94); both are bound by the fp32 matrix pipe and the issue port it shares
-// with the vector instructions of the other two waves of a SIMD.
+// Every product takes all 24 bits of its operands, so the fp32 outputs sT, ds0 and the saved sa keep the accuracy class of the
+// reference's fp32 recurrence; the bf16 outputs are rounded once at the store.  The fp32 mode is therefore the same kernel with fp32
+// loads and stores.  Products are split ones (split3.h) but for the tiles from A', R', B', K', which are fp32 matrix instructions:
+// their operands enter one product each, and splitting those costs what the instructions cost.
 //
-// One workgroup of four waves per (batch, head).  A 16x16x4 fp32 matrix instruction takes A[row = lane & 15][k = lane >> 4],
+// One workgroup per (batch, head).  A 16x16x4 fp32 matrix instruction takes A[row = lane & 15][k = lane >> 4],
 // B[k = lane >> 4][col = lane & 15] and leaves D[row = 4 (lane >> 4) + v][col = lane & 15] in register v.  The state is
 // kept TRANSPOSED in accumulator registers, S^T tile jt of wave q: register v of lane (l16, g) = S[i = 16 q + l16][j = 16 jt + 4 g + v].
-// K slots may be assigned to channels (or tokens) in any order as long as both operands agree, so with slot g <-> channel
-// 16 jt + 4 g + v in step (jt, v) an accumulator register IS the B operand of that step, and an accumulator tile whose rows
-// are tokens (U, W, dU, dW) is the B operand of a contraction over tokens with slot g <-> token 4 g + v.  Nothing is ever
-// transposed through LDS except the gradient state for the two products that contract over the value channel.
+// K slots may be assigned to channels (or tokens) in any order as long as both operands agree, so accumulator registers, split, are the
+// B operand of the next product: two state tiles of a contraction over 32 channels, U, W, dU, dW of one over 16 tokens.  Nothing is
+// transposed through LDS but by reads that transpose.
 //
 // Private layout of the interface's scratch tensors: `s` slot c holds the state ENTERING chunk c as [i][j] fp32 (the
 // reference stores the state leaving it; the backward here needs the entering one and never inverts a step), `sa` is U.
-#include "common.h"
+#include <stddef.h>
+
+#include "split3.h"
 
 namespace rwkv {
 namespace {
 
 constexpr int N = 64;
 constexpr int CL = RWKV7_CHUNK_LEN;
-constexpr int NT = 256;
 constexpr int PS = 68;            // row stride (floats) of a [token][channel] plane
 constexpr int TS = 20;            // row stride (floats) of a 16 x 16 tile
 constexpr float W_SCALE = -0.6065306597f;   // -exp(-0.5), rwkv7_statepassing_clampw.cu:16
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 DEVINL f32x4 mm(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 DEVINL f32x4 ld4(const float* p) { const float4 x = *reinterpret_cast<const float4*>(p); return f32x4{x.x, x.y, x.z, x.w}; }
 DEVINL void st4(float* p, const f32x4& x) { *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]); }
@@ -71,9 +69,11 @@ struct Args7c {
 };
 
 // element base + o as it comes from memory, and its value
+// (a scalar base and one 32-bit byte offset a lane)
 template <bool F32> DEVINL uint32_t ld_raw(const uint16_t* p, size_t base, uint32_t o) {
-    if constexpr (F32) return (reinterpret_cast<const uint32_t*>(p) + base)[o];
-    else return (p + base)[o];
+    const char* const b = reinterpret_cast<const char*>(p) + base * (F32 ? 4 : 2);
+    if constexpr (F32) return *reinterpret_cast<const uint32_t*>(b + o * 4u);
+    else return *reinterpret_cast<const uint16_t*>(b + o * 2u);
 }
 template <bool F32> DEVINL float widen(uint32_t x) { return F32 ? __uint_as_float(x) : bf2f(static_cast<uint16_t>(x)); }
 
@@ -83,6 +83,7 @@ DEVINL float by_group(int g, float x0, float x1, float x2, float x3) { return g 
 // Rows of M = (I - AB)^{-1}: lane (l16 = r) gets m[s] = M[r][s] from the column recurrence M[r][s] = [r == s] + sum_{t>s} M[r][t] AB[t][s].
 // ABt[s][t] = AB[t][s] is read with wave-uniform addresses (LDS broadcast).
 DEVINL void inverse_rows(const float (*ABt)[TS], int r, float (&m)[CL]) {
+    asm volatile("" : "+v"(r));            // (or sixteen comparisons with it live in registers across the caller's loop)
     m[CL - 1] = r == CL - 1 ? 1.f : 0.f;
 #pragma unroll
     for (int s = CL - 2; s >= 0; --s) {
@@ -99,6 +100,7 @@ DEVINL void inverse_rows(const float (*ABt)[TS], int r, float (&m)[CL]) {
 }
 // Columns of the same M: lane (l16 = c) gets m[t] = M[t][c] from the row recurrence M[t][c] = [t == c] + sum_{s<t} AB[t][s] M[s][c].
 DEVINL void inverse_cols(const float (*AB)[TS], int c, float (&m)[CL]) {
+    asm volatile("" : "+v"(c));            // (or sixteen comparisons with it live in registers across the caller's loop)
     m[0] = c == 0 ? 1.f : 0.f;
 #pragma unroll
     for (int t = 1; t < CL; ++t) {
@@ -128,7 +130,6 @@ DEVINL float exp_acc(float x) {
 // Every exponent is formed as a direct sum of the lam between the token and its reference point (never as a difference of
 // two long cumulative sums), so its absolute error -- the factor's relative error -- scales with the exponent itself.
 struct Factors { float ea[4], er[4], eb[4], es[4], ee[4]; };   // e^{c_t - c_m}, e^{c_{t+1} - c_m}, e^{c_m - c_{t+1}}, e^{c_t}, e^{c_L - c_{t+1}}
-template <int E0 = 0, int E1 = 4>
 DEVINL Factors chunk_factors(const float (&lam)[4], const float (*part)[N], int q, int j, float& cm_out, float& cl_out) {
     const float p0 = part[0][j], p1 = part[1][j], p2 = part[2][j], p3 = part[3][j];
     const float cm = p0 + p1, cl = (p0 + p1) + (p2 + p3);
@@ -144,7 +145,7 @@ DEVINL Factors chunk_factors(const float (&lam)[4], const float (*part)[N], int 
     for (int e = 3; e >= 0; --e) suf[e] = suf[e + 1] + lam[e];
     Factors f = {};
 #pragma unroll
-    for (int e = E0; e < E1; ++e) {                // (the exponentials of the tokens asked for; the sums above are cheap)
+    for (int e = 0; e < 4; ++e) {                  // (a caller pays for the factors that it takes)
         // c_t - c_m and c_{t+1} - c_m
         const float xt = q < 2 ? -(suf[e] + gap) : gap + pre[e];
         const float xn = q < 2 ? -(suf[e + 1] + gap) : gap + pre[e + 1];
@@ -160,67 +161,92 @@ DEVINL Factors chunk_factors(const float (&lam)[4], const float (*part)[N], int 
     return f;
 }
 
-DEVINL float sigmoid_fast(float x) { return __frcp_rn(1.f + __expf(-x)); }
+// (a Newton step behind the hardware reciprocal instead of a full division, a sixth of the vector instructions that turn inputs into
+// planes; the exponent stops short of overflow, where the step would make a NaN, and a NaN passes)
+DEVINL float sigmoid_fast(float x) {
+    const float t = x * -1.44269504088896340736f;
+    const float d = 1.f + __builtin_amdgcn_exp2f(t > 126.f ? 126.f : t);
+    const float y = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, y, 1.f), y, y);
+}
 
+// tile[t][s] = sum_c X[t][c] Y[s][c] over 64 channels, masked to s < t (strict) or s <= t: register v <-> t = 4 g + v, lane <-> s, or
+// (ROWS) register v <-> s = 4 g + v, lane <-> t
+template <bool ROWS> DEVINL f32x4 causal_acc(const float (*X)[PS], const float (*Y)[PS], bool strict, int l16, int g) {
+    f32x4 part[2] = {ZERO4, ZERO4};               // two independent chains
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+        const f32x4 xa = ld4(&X[l16][16 * cb + 4 * g]), yb = ld4(&Y[l16][16 * cb + 4 * g]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) part[cb & 1] = ROWS ? mm(yb[v], xa[v], part[cb & 1]) : mm(xa[v], yb[v], part[cb & 1]);
+    }
+    f32x4 acc = part[0] + part[1];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int t = ROWS ? l16 : 4 * g + v, s = ROWS ? 4 * g + v : l16;
+        acc[v] = (strict ? s < t : s <= t) ? acc[v] : 0.f;
+    }
+    return acc;
+}
 // ---------------------------------------------------------------------------------------------------- forward
+// One workgroup of eight waves per (batch, head), two of them on a CU, two roles with their own loops and two barriers a chunk:
+//          phase X                                                   | phase Y
+//   S:     (a e^{c_t}) S0^T, (r e^{c_{t+1}}) S0^T; rows of the chunk  | AK V, U, RK V + RB U, the state
+//          before and the state entering to memory                    |
+//   P:     causal tiles and the inverse of this chunk; decay sums of  | factors, planes of the next chunk
+//          the next                                                   |
+// A plane that one phase writes and the other reads needs no second copy (k, b carried to the chunk's end and dec, which S reads while P writes, do).
+// The P waves make the tiles on the fp32 matrix instructions, all other products are split ones (split3.h).
+constexpr int NTF = 8 * 64;        // waves 0..3 role S, 4..7 role P
 struct SmemCF {
-    float Ap[CL][PS], Rp[CL][PS], Bp[CL][PS], Kp[CL][PS], V[CL][PS];
-    float Be[CL][PS], Ke[CL][PS];      // b, k carried to the end of the chunk: e^{c_L - c_{s+1}}
-    float As[CL][PS];                  // a referred to the start of the chunk: e^{c_t}
+    float Ap[CL][PS], Rp[CL][PS], Bp[CL][PS], Kp[CL][PS];      // referred to the middle of the chunk: the tiles
     float Yo[CL][PS], Uo[CL][PS];
-    float ABt[CL][TS], AK[CL][TS], RB[CL][TS], RK[CL][TS];
-    float M[CL][TS];                   // (I - AB)^{-1}, rows by the wave that made AB
+    float ABt[CL][TS];
     float part[4][N];
-    float d1[N], dec[N];
+    float dec[2][N];
 };
+// three-term planes and tiles behind it: a e^{c_t}, r e^{c_{t+1}}, k and b carried to the end of the chunk (e^{c_L - c_{s+1}}), v (one term
+// where it is bf16), AK, RB, RK, (I - AB)^{-1}
+constexpr uint32_t F_AS = (sizeof(SmemCF) + 31) / 32 * 32, F_RS = F_AS + PLANE3, F_KB = F_RS + PLANE3, F_V = F_KB + 2 * PAIR3;
+template <bool F32> constexpr uint32_t F_MA = F_V + (F32 ? PLANE3 : TERM);      // (I - AB)^{-1} and AK
+template <bool F32> constexpr uint32_t F_RKB = F_MA<F32> + TPAIR3;                // RK and RB
+template <bool F32> constexpr uint32_t F_TOTAL = F_RKB<F32> + TPAIR3;
+static_assert(F_TOTAL<true> <= 80 * 1024, "two workgroups a CU");
 
-// KEEP: `s` and `sa` are written for a backward, 20 bytes per element beside the 14 of a bf16 forward's inputs and output.  Without
-// (no backward can follow) B8 T1024 C4096 takes 353 us instead of 383, and none of the 672 MB; one chunk of 32 heads, the call
-// included, 7.9 instead of 9.4.  The rest is the fp32 matrix pipe plus the vector instructions, which hardly overlap with it: the
-// state's products moved ahead of the barrier behind the inverse, or the waits for stores taken out of the loop, did not make it
-// faster (384 and 394 us).
-template <bool F32, bool KEEP>
-__global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
-    __shared__ SmemCF S;
-    const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
-    const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
-    const int nch = T / CL;
-    const size_t bh = static_cast<size_t>(b) * H + h;
-    const size_t tok0 = static_cast<size_t>(b) * T;                       // first token row of this batch
-    const int i_own = 16 * q + l16;
-
-    // state, transposed tiles: St[jt][v] = S[i_own][16 jt + 4 g + v]
-    f32x4 St[4];
-#pragma unroll
-    for (int jt = 0; jt < 4; ++jt)
-        St[jt] = p.s0 != nullptr ? ld4(p.s0 + bh * N * N + static_cast<size_t>(i_own) * N + 16 * jt + 4 * g) : ZERO4;
-
-    // prep role: channel j = lane, tokens 4 q + e
+template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args7c& p, int q, int lane, size_t tok0, int nch, int h) {
+    const int l16 = lane & 15, g = lane >> 4, H = p.H;
+    // channel j = lane, tokens 4 q + e
     uint32_t nx[6][4];
-    auto fetch = [&](int c) __attribute__((always_inline)) {
+    auto fetch = [&](int c) __attribute__((always_inline)) {         // (clamped, so that every chunk issues the same loads)
+        const size_t base = ((tok0 + static_cast<size_t>(c < nch ? c : nch - 1) * CL) * H + h) * N;
+        uint32_t lo = lane;
+        asm volatile("" : "+v"(lo));
+        const uint16_t* const src[6] = {p.w, p.r, p.k, p.v, p.a, p.b};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const size_t o = ((tok0 + static_cast<size_t>(c) * CL + 4 * q + e) * H + h) * N + lane;
-            nx[0][e] = ld_raw<F32>(p.w, o, 0); nx[1][e] = ld_raw<F32>(p.r, o, 0); nx[2][e] = ld_raw<F32>(p.k, o, 0);
-            nx[3][e] = ld_raw<F32>(p.v, o, 0); nx[4][e] = ld_raw<F32>(p.a, o, 0); nx[5][e] = ld_raw<F32>(p.b, o, 0);
-        }
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) nx[k][e] = ld_raw<F32>(src[k], base, static_cast<uint32_t>((4 * q + e) * H) * N + lo);
     };
-    fetch(0);
-
-    for (int c = 0; c < nch; ++c) {
-        // ---------------------------------------------------------------- prep: decay sums, scaled operand planes
-        float lam[4], rr[4], kk[4], vv[4], aa[4], bb[4];
+    float lam[4], rr[4], kk[4], aa[4], bb[4];
+    [[maybe_unused]] float vv[4];
+    [[maybe_unused]] uint32_t vb[4];
+    auto convert = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             lam[e] = W_SCALE * sigmoid_fast(widen<F32>(nx[0][e]));
-            rr[e] = widen<F32>(nx[1][e]); kk[e] = widen<F32>(nx[2][e]); vv[e] = widen<F32>(nx[3][e]);
+            // (a value of its own: the product could join an addition in one of the two copies of this code and not in the other, and a
+            // sequence cut into calls would no longer give the same bits)
+            asm volatile("" : "+v"(lam[e]));
+            rr[e] = widen<F32>(nx[1][e]); kk[e] = widen<F32>(nx[2][e]);
+            if constexpr (F32) vv[e] = widen<F32>(nx[3][e]); else vb[e] = nx[3][e];
             aa[e] = widen<F32>(nx[4][e]); bb[e] = widen<F32>(nx[5][e]);
         }
         S.part[q][lane] = (lam[0] + lam[1]) + (lam[2] + lam[3]);
-        if (c + 1 < nch) fetch(c + 1);
-        __syncthreads();
+    };
+    auto planes = [&](const int slot) __attribute__((always_inline)) {
         float cm, cl;
         const Factors f = chunk_factors(lam, S.part, q, lane, cm, cl);
+        f32x4 as, rs, ke, be;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int t = 4 * q + e;
@@ -228,12 +254,86 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
             S.Rp[t][lane] = rr[e] * f.er[e];
             S.Bp[t][lane] = bb[e] * f.eb[e];
             S.Kp[t][lane] = kk[e] * f.eb[e];
-            S.As[t][lane] = aa[e] * f.es[e];
-            S.Be[t][lane] = bb[e] * f.ee[e];
-            S.Ke[t][lane] = kk[e] * f.ee[e];
-            S.V[t][lane] = vv[e];
+            as[e] = aa[e] * f.es[e];
+            rs[e] = rr[e] * (f.es[e] * __expf(lam[e]));
+            ke[e] = kk[e] * f.ee[e];
+            be[e] = bb[e] * f.ee[e];
         }
-        if (q == 0) { S.d1[lane] = exp_acc(cm); S.dec[lane] = exp_acc(cl); }
+        const lds_t o = sb + piece(lane, q);
+        put3(o + F_AS, split3(as)); put3(o + F_RS, split3(rs));
+        put_pair<TERM2>(sb + F_KB + slot * PAIR3 + piece2(lane, q), split3(ke), split3(be));
+        if constexpr (F32) put3(o + F_V, split3(f32x4{vv[0], vv[1], vv[2], vv[3]}));
+        else lds_st<u32x2>(o + F_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
+        if (q == 0) S.dec[slot][lane] = exp_acc(cl);
+    };
+    fetch(0);
+    convert();
+    fetch(1);
+    __syncthreads();
+    planes(0);
+    __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+        // ---------------------------------------------------------------- phase X
+        {
+            const float (*X)[PS] = q < 2 ? S.Ap : S.Rp;
+            const float (*Y)[PS] = (q & 1) ? S.Kp : S.Bp;
+            f32x4 x;
+            if (q == 0) {
+                st4(&S.ABt[l16][4 * g], causal_acc<false>(X, Y, true, l16, g));
+                // this wave wrote AB itself (LDS keeps a wave's accesses in order): the inverse once, for all four S waves
+                float m[CL];
+                inverse_rows(S.ABt, l16, m);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) x[v] = by_group(g, m[v], m[4 + v], m[8 + v], m[12 + v]);
+            } else x = causal_acc<true>(X, Y, q == 1, l16, g);
+            // (one store with a selected address, as in the backward)
+            put_half<TTERM2>(sb + piece2(l16, g) + (q == 0 ? F_MA<F32> : (q == 1 ? F_MA<F32> + 8 : (q == 2 ? F_RKB<F32> + 8 : F_RKB<F32>))), split3(x));
+        }
+        convert();
+        fetch(c + 2);
+        __syncthreads();
+        // ---------------------------------------------------------------- phase Y
+        planes((c + 1) & 1);
+        __syncthreads();
+    }
+}
+
+template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb, const Args7c& p, int q, int tid, size_t bh, size_t tok0, int nch, int h) {
+    const int lane = tid & 63, l16 = lane & 15, g = lane >> 4, H = p.H;
+    const int i_own = 16 * q + l16;
+    // state, transposed tiles: St[jt][v] = S[i_own][16 jt + 4 g + v]
+    f32x4 St[4];
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt)
+        St[jt] = p.s0 != nullptr ? ld4(p.s0 + bh * N * N + static_cast<size_t>(i_own) * N + 16 * jt + 4 * g) : ZERO4;
+    // y and sa = U (fp32) of chunk c as whole rows
+    auto store_rows = [&](const int c) __attribute__((always_inline)) {
+        const int t = tid >> 4, i4 = (tid & 15) * 4;
+        const size_t o = ((tok0 + static_cast<size_t>(c) * CL + t) * H + h) * N + i4;
+        const f32x4 y = ld4(&S.Yo[t][i4]);
+        if constexpr (F32) st4(reinterpret_cast<float*>(p.y) + o, y);
+        else *reinterpret_cast<uint2*>(p.y + o) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
+        if constexpr (KEEP) st4(p.sa + o, ld4(&S.Uo[t][i4]));
+    };
+    const Tr tr = tr_bases(sb, l16, g);
+    const lds_t pp = sb + piece2(l16, g), vp = sb + F_V + piece(i_own, g);
+    auto load_v = [&]() __attribute__((always_inline)) {
+        if constexpr (F32) return get3(vp); else return lds_ld<u32x2>(vp);
+    };
+    __syncthreads();
+    __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+        // ---------------------------------------------------------------- phase X: what needs no tile
+        const auto vop = load_v();                   // V[s = 4 g + v][i_own]
+        Sum2 W = SUM0, Y = SUM0;
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) {
+            const Op3 st = join(split3(St[2 * hb]), split3(St[2 * hb + 1]));
+            add32(W, get3_tr(F_AS, tr, hb), st);
+            add32(Y, get3_tr(F_RS, tr, hb), st);
+        }
+        here(W); here(Y);
+        if (c > 0) store_rows(c - 1);
         // the state entering the chunk, for the backward
         if constexpr (KEEP) {
             float* slot = p.s + (bh * nch + c) * N * N + static_cast<size_t>(i_own) * N + 4 * g;
@@ -241,110 +341,54 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
             for (int jt = 0; jt < 4; ++jt) st4(slot + 16 * jt, St[jt]);
         }
         __syncthreads();
-        // ---------------------------------------------------------------- one causal tile per wave
-        {
-            const float (*X)[PS] = q < 2 ? S.Ap : S.Rp;
-            const float (*Y)[PS] = (q & 1) ? S.Kp : S.Bp;
-            f32x4 acc = ZERO4;
-#pragma unroll
-            for (int jb = 0; jb < 4; ++jb) {
-                const f32x4 xa = ld4(&X[l16][16 * jb + 4 * g]), yb = ld4(&Y[l16][16 * jb + 4 * g]);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc = mm(xa[v], yb[v], acc);
-            }
-            // acc[v] = tile[t = 4 g + v][s = l16]
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int t = 4 * g + v;
-                acc[v] = (q < 2 ? l16 < t : l16 <= t) ? acc[v] : 0.f;
-            }
-            if (q == 0) {
-                st4(&S.ABt[l16][4 * g], acc);
-                // this wave wrote AB itself (LDS keeps a wave's accesses in order): the inverse once, for all four waves
-                float m[CL];
-                inverse_rows(S.ABt, l16, m);
-                if (g == 0)
-#pragma unroll
-                    for (int s4 = 0; s4 < CL; s4 += 4) st4(&S.M[l16][s4], f32x4{m[s4], m[s4 + 1], m[s4 + 2], m[s4 + 3]});
-            } else {
-                float (*Tl)[TS] = q == 1 ? S.AK : (q == 2 ? S.RB : S.RK);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) Tl[4 * g + v][l16] = acc[v];
-            }
-        }
-        __syncthreads();
-        // ---------------------------------------------------------------- W = (a e^{c_t}) S0^T + AK V, value channels of this wave
-        f32x4 vop;                                   // V[s = 4 g + v][i_own]
-#pragma unroll
-        for (int v = 0; v < 4; ++v) vop[v] = S.V[4 * g + v][i_own];
-        f32x4 W = ZERO4;
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) {
-            const f32x4 xa = ld4(&S.As[l16][16 * jt + 4 * g]);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) W = mm(xa[v], St[jt][v], W);
-        }
-        {
-            const f32x4 ak = ld4(&S.AK[l16][4 * g]);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) W = mm(ak[v], vop[v], W);
-        }
-        // ---------------------------------------------------------------- U = (I - AB)^{-1} W
-        f32x4 U = ZERO4;
-        {
-            const f32x4 mr = ld4(&S.M[l16][4 * g]);   // M[t = l16][s = 4 g + v]
-#pragma unroll
-            for (int v = 0; v < 4; ++v) U = mm(mr[v], W[v], U);
-        }
-        // ---------------------------------------------------------------- Y = R' (d1 S0^T) + RB U + RK V
-        f32x4 Sd[4];
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) Sd[jt] = St[jt] * ld4(&S.d1[16 * jt + 4 * g]);
-        f32x4 Y = ZERO4;
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) {
-            const f32x4 xa = ld4(&S.Rp[l16][16 * jt + 4 * g]);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Y = mm(xa[v], Sd[jt][v], Y);
-        }
-        {
-            const f32x4 rb = ld4(&S.RB[l16][4 * g]), rk = ld4(&S.RK[l16][4 * g]);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Y = mm(rb[v], U[v], Y);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Y = mm(rk[v], vop[v], Y);
-        }
+        // ---------------------------------------------------------------- phase Y
+        add16(W, get_half<TTERM2>(pp + F_MA<F32> + 8), vop);
+        Sum2 Us = SUM0;
+        add16(Us, get_half<TTERM2>(pp + F_MA<F32>), split3(total(W)));
+        const f32x4 U = total(Us);
+        const Op3 vu = join(as3(vop), split3(U));        // V and U share the instructions of what follows
+        add32(Y, get_pair<TTERM2>(pp + F_RKB<F32>), vu);
+        const f32x4 y = total(Y);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            S.Yo[4 * g + v][i_own] = Y[v];
+            S.Yo[4 * g + v][i_own] = y[v];
             if constexpr (KEEP) S.Uo[4 * g + v][i_own] = U[v];
         }
-        // ---------------------------------------------------------------- S^T = diag(dec) S^T + (B' d2)^T U + (K' d2)^T V
+        const lds_t kb = pp + F_KB + (c & 1) * PAIR3;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
-            f32x4 acc = ZERO4;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc = mm(S.Be[4 * g + v][16 * jt + l16], U[v], acc);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc = mm(S.Ke[4 * g + v][16 * jt + l16], vop[v], acc);
-            St[jt] = St[jt] * ld4(&S.dec[16 * jt + 4 * g]) + acc;
+            Sum2 x = SUM0;
+            add32(x, get_pair<TERM2>(kb + 1024 * jt), vu);
+            St[jt] = St[jt] * ld4(&S.dec[c & 1][16 * jt + 4 * g]) + total(x);
         }
         __syncthreads();
-        // ---------------------------------------------------------------- y and sa = U (fp32) as whole rows
-        {
-            const int t = tid >> 4, i4 = (tid & 15) * 4;
-            const size_t o = ((tok0 + static_cast<size_t>(c) * CL + t) * H + h) * N + i4;
-            const f32x4 y = ld4(&S.Yo[t][i4]);
-            if constexpr (F32) st4(reinterpret_cast<float*>(p.y) + o, y);
-            else *reinterpret_cast<uint2*>(p.y + o) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
-            if constexpr (KEEP) st4(p.sa + o, ld4(&S.Uo[t][i4]));
-        }
     }
+    store_rows(nch - 1);
     if (p.sT != nullptr) {
         float* dst = p.sT + bh * N * N + static_cast<size_t>(i_own) * N + 4 * g;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) st4(dst + 16 * jt, St[jt]);
     }
+}
+
+// KEEP: `s` and `sa` are written for a backward, 20 bytes per element beside the 14 of a bf16 forward's inputs and output.
+// What bounds it: issue.  B8 T1024 C4096, one call: 398 us with every product on the fp32 matrix instructions, in four waves that did
+// everything in turn between four barriers; 390 in two roles of four waves; 335 with split products, since the fp32 instructions
+// (96 a wave and chunk) held the vector unit for half of the time.  Vector instructions are now most of it, two thirds of them in the
+// P waves.  fp32 mode 396 -> 360.  Errors against 64 bits, T256, before -> now: y 1.8 -> 1.4e-7, sT 6.9 -> 6.0e-8 (slow decays
+// 1.5e-7 -> 9e-8).
+template <bool F32, bool KEEP>
+__global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c p) {
+    extern __shared__ __align__(32) unsigned char smem_raw[];
+    SmemCF& S = *reinterpret_cast<SmemCF*>(smem_raw);
+    const lds_t sb = lds_of(smem_raw);
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = blockIdx.x, b = blockIdx.y;
+    const int nch = p.T / CL;
+    const size_t bh = static_cast<size_t>(b) * p.H + h;
+    const size_t tok0 = static_cast<size_t>(b) * p.T;                 // first token row of this batch
+    if (w < 4) fwd_role_s<F32, KEEP>(S, sb, p, w, tid, bh, tok0, nch, h);
+    else fwd_role_p<F32>(S, sb, p, w - 4, tid & 63, tok0, nch, h);
 }
 
 // ---------------------------------------------------------------------------------------------------- backward
@@ -358,56 +402,90 @@ __global__ __launch_bounds__(NT, 2) void rwkv7c_fwd(const Args7c p) {
 //                them, scan the decay gradient and park the results; they run one phase behind the A waves.
 //   waves 8..11 ("P"): fetch the seven input rows and `sa` two chunks ahead, convert them and build the operand planes
 //                (double-buffered).  The finished gradient rows leave LDS-staged, as whole rows, through A waves 2 and 3.
-// The gradient state is therefore kept twice (both copies get the same update); nothing is transposed through LDS.
+// The gradient state is therefore kept twice (both copies get the same update).
+// What bounds it: issue, and waits for LDS and at barriers.  B8 T1024 C4096, one call: 762 us with fp32 matrix instructions (962 a
+// chunk, 57 % of a SIMD's time in which it could issue no vector instruction), 676 with split products (fp32 mode 811 -> 844 in a
+// trace of few calls, 797 -> 770 among others: its 24 rows a chunk leave from registers, 64 bytes at a time).  Of that, causal tiles
+// and the inverse moved from phase 1, where everybody waited for wave 0, into the phase 3 before: 727 -> 676.  Errors against 64 bits,
+// T256, before -> now: ds0 1.55e-7 -> 8e-8, dr 1.5 -> 1.1e-7, dk 1.6 -> 1.2e-7, dv 1.5 -> 1.4e-7, da 2.3 -> 1.9e-7, db 2.4 -> 1.8e-7.
 constexpr int NTB = 12 * 64;       // waves 0..3 role A, 4..7 role B, 8..11 role P
 
-// Everything that is a function of one chunk's inputs alone; two copies: the P waves fill one while the A and B waves work on the other.
+// Everything that is a function of one chunk's inputs alone; two copies (but for the planes that only phase 1 reads): the P waves fill
+// one while the A and B waves work on the other.
 struct PlanesB {
     float Ap[CL][PS], Rp[CL][PS], Bp[CL][PS], Kp[CL][PS];   // referred to the middle of the chunk (tiles, dA' .. dK')
-    float As[CL][PS], Rs[CL][PS];                            // a e^{c_t}, r e^{c_{t+1}}: the state-gradient update
-    float Bd[CL][PS], Kd[CL][PS];                            // b, k times e^{c_L - c_{s+1}}: dU, dV, S_T
-    float V[CL][PS], dY[CL][PS], U[CL][PS];
     float EA[CL][PS], ER[CL][PS], DWF[CL][PS];               // e^{c_t - c_m}, e^{c_{t+1} - c_m}, W_SCALE sig (1 - sig)
-    float part[4][N];
     float d1[N], d2[N], dec[N];
 };
+static_assert(offsetof(PlanesB, Rp) == 4 * CL * PS && offsetof(PlanesB, d1) == 7 * 4 * CL * PS && offsetof(PlanesB, dec) == offsetof(PlanesB, d1) + 8 * N, "role B's addresses");
 constexpr int PK = 72;            // row stride (bf16 elements) of a parked output
 // fp32 outputs are not parked (twice the bytes would not fit the CU's LDS): the waves that finish them store them from
 // registers, 64 bytes of four rows per instruction.
 template <bool F32>
 struct SmemCB {
     PlanesB pl[2];
-    float dW[CL][PS];
-    float M[CL][TS];                                         // (I - AB)^{-1}
-    float AB[CL][TS], AK[CL][TS], RB[CL][TS], RK[CL][TS];
-    float dAB[CL][TS], dAK[CL][TS], dRB[CL][TS], dRK[CL][TS];
+    float part[4][N];
+    float AB[CL][TS];
     uint16_t park[F32 ? 1 : 5][F32 ? 1 : CL][PK];                                // da, dr, db, dk, dw of the chunk whose phase 4 ran last, [token][channel]
     uint16_t parkv[F32 ? 1 : 2][F32 ? 1 : CL][PK];                               // dv, which is ready one visit earlier than the other five
 };
-
-// tile[t][s] = sum_c X[t][c] Y[s][c] over 64 channels, masked to s < t (strict) or s <= t, stored as [t][s]
-DEVINL void causal_tile(const float (*X)[PS], const float (*Y)[PS], float (*Tl)[TS], bool strict, int l16, int g) {
-    f32x4 part[2] = {ZERO4, ZERO4};               // two independent chains
+// three-term planes and tiles behind it.  Two copies: r e^{c_{t+1}} and a e^{c_t} (RA, the state-gradient update), U, v and dy (one term
+// each where they are bf16).  One: b, k times e^{c_L - c_{s+1}} (dU, dV), dW, and the tiles, each as the lanes of its products hold
+// it: the transposes of (I - AB)^{-1} and RB (MB), RK and AK (RKA); by rows (over s) dAB and dAK for dA', dRB and dRK for dR'; by columns (over t)
+// dAB and dRB for dB', dAK and dRK for dK'.
+template <bool F32> struct LB {
+    static constexpr uint32_t TWO = (sizeof(SmemCB<F32>) + 31) / 32 * 32, EX = F32 ? PLANE3 : TERM;      // from TWO on
+    static constexpr uint32_t RA = 0, U = PAIR3, V = U + PLANE3, DY = V + EX, SLOT = DY + EX;
+    static constexpr uint32_t ONE = TWO + 2 * SLOT;                                                         // from ONE on
+    static constexpr uint32_t BD = 0, KD = PLANE3, DW = 2 * PLANE3, MB = 3 * PLANE3, RKA = MB + TPAIR3;
+    static constexpr uint32_t A_ROWS = RKA + TPAIR3, R_ROWS = A_ROWS + TPAIR3, B_COLS = R_ROWS + TPAIR3, K_COLS = B_COLS + TPAIR3, BYTES = ONE + K_COLS + TPAIR3;
+};
+// A lane's addresses in one of the two regions
+struct LaneB { Tr tr; lds_t rows[2], own, pair, own_pair; };
+DEVINL LaneB lane_bases(lds_t base, int l16, int g, int own) {
+    LaneB b{tr_bases(base, l16, g), {base + piece(l16, g), base + (piece(l16, g) ^ 16u)}, base + piece(own, g), base + piece2(l16, g), base + piece2(own, g)};
+    opaque(b.tr.a); opaque(b.tr.b); opaque(b.rows[0]); opaque(b.rows[1]); opaque(b.own); opaque(b.pair); opaque(b.own_pair);
+    return b;
+}
+// v, dy: four tokens of a channel, and over channels
+template <bool F32> DEVINL auto exact_piece(lds_t a) { if constexpr (F32) return get3(a); else return lds_ld<u32x2>(a); }
+template <bool F32> DEVINL auto exact_tr(uint32_t plane, const Tr& o, int hb) { if constexpr (F32) return get3_tr(plane, o, hb); else return ld_tr16(o, plane, hb); }
+// causal_acc from three-term planes (or, not three, exact ones): rows of the result from a, columns from b; transposed: tokens s along
+// the rows.  All but the planes' addresses is uniform: the waves that make different tiles share the code.
+DEVINL f32x4 causal_split(const Tr& o, lds_t a, bool a3, lds_t b, bool b3, bool transposed, bool strict, int l16, int g) {
+    Sum2 sum = SUM0;
+    const Tr oa{o.a + a, o.b + a}, ob{o.a + b, o.b + b};
+    const bf16x8 ah[2] = {ld_tr16(oa, 0, 0), ld_tr16(oa, 0, 1)}, bh[2] = {ld_tr16(ob, 0, 0), ld_tr16(ob, 0, 1)};
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-        const f32x4 xa = ld4(&X[l16][16 * cb + 4 * g]), yb = ld4(&Y[l16][16 * cb + 4 * g]);
+    for (int hb = 0; hb < 2; ++hb) sum.hi = mmb(ah[hb], bh[hb], sum.hi);
+    if (a3) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) part[cb & 1] = mm(xa[v], yb[v], part[cb & 1]);
+        for (int hb = 0; hb < 2; ++hb) {
+            const bf16x8 am = ld_tr16(oa, TERM, hb);
+            sum.lo = mmb(ld_tr16(oa, 2 * TERM, hb), bh[hb], sum.lo);
+            if (b3) sum.lo = mmb(am, ld_tr16(ob, TERM, hb), sum.lo);
+            sum.lo = mmb(am, bh[hb], sum.lo);
+        }
     }
-    const f32x4 acc = part[0] + part[1];
+    if (b3) {
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) sum.lo = mmb(ah[hb], ld_tr16(ob, TERM, hb), mmb(ah[hb], ld_tr16(ob, 2 * TERM, hb), sum.lo));
+    }
+    f32x4 acc = total(sum);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        const int t = 4 * g + v;
-        Tl[t][l16] = (strict ? l16 < t : l16 <= t) ? acc[v] : 0.f;
+        const int r = 4 * g + v, t = transposed ? l16 : r, s = transposed ? r : l16;
+        acc[v] = (strict ? s < t : s <= t) ? acc[v] : 0.f;
     }
+    return acc;
 }
 
 // Per visit i (chunks in descending order) every wave passes three barriers; role B trails role A by one phase, so that
 // both always have matrix work in the same phase:
 //          phase 1                          | phase 2                                   | phase 3
-//   A:     tile, M, tile-free parts of (i)   | dU, dW, dV, state update of (i)           | dAB, dAK of (i)
-//   B:     tile parts + epilogue of (i - 1)  | dY S0, U dS, V dS, dRB, dRK of (i)        | dW S0, state update of (i)
-//   P:     raw inputs -> decay sums (i + 1)  | factors, planes (i + 1)                   | -
+//   A:     state parts of dU, dV of (i)      | dU, dW, dV, state update of (i)           | dAB, dAK of (i), both ways; tile, M of (i + 1)
+//   B:     other tile parts, rest of (i - 1) | dY S0, U dS, V dS, dRB, dRK of (i)        | dW S0, state update, dr of (i)
+//   P:     decay sums, U, v, dy (i + 1)      | fp32 planes (i + 1)                       | other three-term planes (i + 1)
 // (the rows of visit i - 1 leave in phase 3, through the two A waves that have no tile there)
 
 // ---- role P: elementwise preparation (lane = channel, tokens 4 wp + e) one visit ahead, and the row-wise output stores
@@ -431,7 +509,7 @@ template <bool F32> DEVINL void bwd_fetch(const Args7c& p, Prep7& x, size_t row0
 }
 // first half of the preparation: the decay of each token, this wave's decay sum; the other inputs are kept packed so that the
 // registers of x are free for the next fetch
-template <bool F32> DEVINL void bwd_convert(PlanesB& O, const Prep7& x, Conv7<F32>& y, int wp, int lane) {
+template <bool F32> DEVINL void bwd_convert(float (*part)[N], const Prep7& x, Conv7<F32>& y, int wp, int lane) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) { y.sg[e] = sigmoid_fast(widen<F32>(x.nx[0][e])); y.uu[e] = x.nsa[e]; }
 #pragma unroll
@@ -444,38 +522,66 @@ template <bool F32> DEVINL void bwd_convert(PlanesB& O, const Prep7& x, Conv7<F3
             for (int z = 0; z < 2; ++z) y.pk[k][z] = x.nx[k + 1][2 * z] | (x.nx[k + 1][2 * z + 1] << 16);
         }
     }
-    O.part[wp][lane] = W_SCALE * ((y.sg[0] + y.sg[1]) + (y.sg[2] + y.sg[3]));
+    part[wp][lane] = W_SCALE * ((y.sg[0] + y.sg[1]) + (y.sg[2] + y.sg[3]));
 }
-// second half (after a barrier): the in-chunk factors and every plane
-template <bool F32, int E0 = 0, int E1 = 4>
-DEVINL void bwd_planes(PlanesB& O, const Conv7<F32>& y, int wp, int lane) {
+// second half (after a barrier), in two parts, each with the factors that it needs: the fp32 planes; three-term planes
+template <bool F32> struct In7 {
+    const Conv7<F32>& y;
+    DEVINL float operator()(int k, int e) const {
+        if constexpr (F32) return __uint_as_float(y.pk[k][e]);
+        else return (e & 1) ? bf_hi(y.pk[k][e >> 1]) : bf_lo(y.pk[k][e >> 1]);
+    }
+};
+template <bool F32> DEVINL void bwd_planes(PlanesB& O, const float (*part)[N], const Conv7<F32>& y, int wp, int lane) {
     float cm, cl;
     const float lam[4] = {W_SCALE * y.sg[0], W_SCALE * y.sg[1], W_SCALE * y.sg[2], W_SCALE * y.sg[3]};
-    const Factors f = chunk_factors<E0, E1>(lam, O.part, wp, lane, cm, cl);
+    const Factors f = chunk_factors(lam, part, wp, lane, cm, cl);
+    const In7<F32> in{y};
 #pragma unroll
-    for (int e = E0; e < E1; ++e) {
+    for (int e = 0; e < 4; ++e) {
         const int t = 4 * wp + e;
-        auto in = [&](int k) __attribute__((always_inline)) {
-            if constexpr (F32) return __uint_as_float(y.pk[k][e]);
-            else return (e & 1) ? bf_hi(y.pk[k][e >> 1]) : bf_lo(y.pk[k][e >> 1]);
-        };
-        const float rr = in(0), kk = in(1), vv = in(2), aa = in(3), bb = in(4), gg = in(5);
-        O.Ap[t][lane] = aa * f.ea[e];
-        O.Rp[t][lane] = rr * f.er[e];
-        O.Bp[t][lane] = bb * f.eb[e];
-        O.Kp[t][lane] = kk * f.eb[e];
-        O.As[t][lane] = aa * f.es[e];
-        O.Rs[t][lane] = rr * (f.es[e] * __expf(lam[e]));
-        O.Bd[t][lane] = bb * f.ee[e];
-        O.Kd[t][lane] = kk * f.ee[e];
-        O.V[t][lane] = vv;
-        O.dY[t][lane] = gg;
-        O.U[t][lane] = y.uu[e];
+        O.Ap[t][lane] = in(3, e) * f.ea[e];
+        O.Rp[t][lane] = in(0, e) * f.er[e];
+        O.Bp[t][lane] = in(4, e) * f.eb[e];
+        O.Kp[t][lane] = in(1, e) * f.eb[e];
         O.EA[t][lane] = f.ea[e];
         O.ER[t][lane] = f.er[e];
         O.DWF[t][lane] = W_SCALE * y.sg[e] * (1.f - y.sg[e]);
     }
-    if (E0 == 0 && wp == 0) { O.d1[lane] = exp_acc(cm); O.d2[lane] = exp_acc(cl - cm); O.dec[lane] = exp_acc(cl); }
+    if (wp == 0) { O.d1[lane] = exp_acc(cm); O.d2[lane] = exp_acc(cl - cm); O.dec[lane] = exp_acc(cl); }
+}
+// sb: LDS base, slot: offset of the chunk's copy
+template <bool F32> DEVINL void bwd_planes3(const lds_t sb, const lds_t slot, const float (*part)[N], const Conv7<F32>& y, int wp, int lane) {
+    using O = LB<F32>;
+    float cm, cl;
+    const float lam[4] = {W_SCALE * y.sg[0], W_SCALE * y.sg[1], W_SCALE * y.sg[2], W_SCALE * y.sg[3]};
+    const Factors f = chunk_factors(lam, part, wp, lane, cm, cl);
+    const In7<F32> in{y};
+    f32x4 as, rs, bd, kd;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        as[e] = in(3, e) * f.es[e];
+        rs[e] = in(0, e) * (f.es[e] * __expf(lam[e]));
+        bd[e] = in(4, e) * f.ee[e];
+        kd[e] = in(1, e) * f.ee[e];
+    }
+    const lds_t o = sb + O::ONE + piece(lane, wp);
+    put_pair<TERM2>(sb + O::TWO + slot + O::RA + piece2(lane, wp), split3(rs), split3(as));
+    put3(o + O::BD, split3(bd)); put3(o + O::KD, split3(kd));
+}
+// U, v and dy, which no factor enters
+template <bool F32> DEVINL void bwd_planes_raw(const lds_t sb, const lds_t slot, const Conv7<F32>& y, int wp, int lane) {
+    using O = LB<F32>;
+    const In7<F32> in{y};
+    const lds_t o = sb + O::TWO + slot + piece(lane, wp);
+    put3(o + O::U, split3(f32x4{y.uu[0], y.uu[1], y.uu[2], y.uu[3]}));
+    if constexpr (F32) {
+        put3(o + O::V, split3(f32x4{in(2, 0), in(2, 1), in(2, 2), in(2, 3)}));
+        put3(o + O::DY, split3(f32x4{in(5, 0), in(5, 1), in(5, 2), in(5, 3)}));
+    } else {
+        lds_st<u32x2>(o + O::V, u32x2{y.pk[2][0], y.pk[2][1]});
+        lds_st<u32x2>(o + O::DY, u32x2{y.pk[5][0], y.pk[5][1]});
+    }
 }
 // bf16: da dr db dk dw (and dv) of one chunk leave their parking places as whole rows (256 threads, four channels each)
 DEVINL void bwd_store_rows(const SmemCB<false>& S, int vbuf, const Args7c& p, size_t row0, int tp, int H, int h) {
@@ -491,9 +597,9 @@ DEVINL void bwd_store_rows(const SmemCB<false>& S, int vbuf, const Args7c& p, si
 }
 // fp32: element [4 g + v][own] of the chunk whose first row is row0, straight to global memory
 DEVINL void store_f32(uint16_t* dst, size_t row0, int v, uint32_t lane_off, int H, int h, float x) {
-    reinterpret_cast<float*>(dst)[((row0 + v) * H + h) * N + lane_off] = x;
+    *reinterpret_cast<float*>(reinterpret_cast<char*>(dst) + ((row0 + v) * H + h) * N * 4 + lane_off * 4u) = x;
 }
-template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const Args7c& p, int tid, int w, size_t tok0, int nch, int H, int h) {
+template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t tok0, int nch, int H, int h) {
     const int lane = tid & 63, wp = w - 8, tp = tid - 8 * 64;
     // Raw rows are asked for two visits before they are converted (one visit, of which only two phases lie between the
     // request and the use, is less than the memory system takes under load: the A and B waves then waited for the P waves
@@ -504,22 +610,23 @@ template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const Args7c& p, int 
     auto row_of = [&](int visit) { const int c = nch - 1 - visit; return tok0 + static_cast<size_t>(c > 0 ? c : 0) * CL; };
     bwd_fetch<F32>(p, x[0], row_of(0), wp, lane, H, h);
     bwd_fetch<F32>(p, x[1], row_of(1), wp, lane, H, h);
-    bwd_convert(S.pl[0], x[0], y, wp, lane);          // visit 0, before the loop
+    bwd_convert(S.part, x[0], y, wp, lane);           // visit 0, before the loop
     bwd_fetch<F32>(p, x[0], row_of(2), wp, lane, H, h);
     __syncthreads();
-    bwd_planes<F32>(S.pl[0], y, wp, lane);
+    bwd_planes<F32>(S.pl[0], S.part, y, wp, lane);
+    bwd_planes3<F32>(sb, 0, S.part, y, wp, lane);
+    bwd_planes_raw<F32>(sb, 0, y, wp, lane);
     __syncthreads();
     auto visit = [&](const int i, auto Z) __attribute__((always_inline)) {     // visit i is chunk nch - 1 - i
         constexpr int z = decltype(Z)::value;        // the set that holds visit i + 1
         const bool next = i + 1 < nch;
-        if (next) bwd_convert(S.pl[(i + 1) & 1], x[z], y, wp, lane);
+        if (next) bwd_convert(S.part, x[z], y, wp, lane);
         bwd_fetch<F32>(p, x[z], row_of(i + 3), wp, lane, H, h);
+        if (next) bwd_planes_raw<F32>(sb, ((i + 1) & 1) * LB<F32>::SLOT, y, wp, lane);
         __syncthreads();
-        // the planes of two of this wave's four tokens in phase 2, the other two in phase 3, in which these waves used to idle
-        // while everybody waited for them in phase 2 (nothing reads these planes before the next visit)
-        if (next) bwd_planes<F32, 0, 2>(S.pl[(i + 1) & 1], y, wp, lane);
+        if (next) bwd_planes<F32>(S.pl[(i + 1) & 1], S.part, y, wp, lane);
         __syncthreads();
-        if (next) bwd_planes<F32, 2, 4>(S.pl[(i + 1) & 1], y, wp, lane);
+        if (next) bwd_planes3<F32>(sb, ((i + 1) & 1) * LB<F32>::SLOT, S.part, y, wp, lane);
         __syncthreads();
     };
     for (int i = 0; i < nch; i += 2) {
@@ -530,57 +637,59 @@ template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const Args7c& p, int 
     if constexpr (!F32) bwd_store_rows(S, (nch - 1) & 1, p, tok0, tp, H, h);
 }
 
-template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
+template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
     const int lane = tid & 63, q = w & 3, l16 = lane & 15, g = lane >> 4;
     const int own = 16 * q + l16;                    // value channel i of this lane's column
     f32x4 dS[4];                                     // dS[i = own][j = 16 jt + 4 g + v]
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
         dS[jt] = p.dsT != nullptr ? ld4(p.dsT + bh * N * N + static_cast<size_t>(own) * N + 16 * jt + 4 * g) : ZERO4;
-    __syncthreads();
-    __syncthreads();
-    for (int i = 0; i < nch; ++i) {
-        const PlanesB& O = S.pl[i & 1];
-        // ---------------------------------------------------------------- phase 1: the parts of dU, dV, dS that need no tile; a causal tile; M
-        // (a chain of dependent matrix instructions runs slower than independent ones: two partial sums each)
-        f32x4 dyop, dUp[2] = {ZERO4, ZERO4}, dVp[2] = {ZERO4, ZERO4}, accA[4];
+    using L = LB<F32>;
+    const LaneB one = lane_bases(sb + L::ONE, l16, g, own);
+    const Tr base_tr = tr_bases(sb, l16, g);
+    // a causal tile of a visit, and M
+    auto tiles = [&](const PlanesB& O) __attribute__((always_inline)) {
+        const f32x4 acc = causal_acc<false>(q < 2 ? O.Ap : O.Rp, (q & 1) ? O.Kp : O.Bp, q < 2, l16, g);
+        f32x4 x = acc;
+        if (q == 0) {                            // this wave wrote AB itself: LDS keeps a wave's accesses in order
 #pragma unroll
-        for (int v = 0; v < 4; ++v) dyop[v] = O.dY[4 * g + v][own];           // dY[tau = 4 g + v][i]
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) {
-            const f32x4 xb = ld4(&O.Bd[l16][16 * jt + 4 * g]), xk = ld4(&O.Kd[l16][16 * jt + 4 * g]);
-            f32x4 acc = ZERO4;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                dUp[jt & 1] = mm(xb[v], dS[jt][v], dUp[jt & 1]);
-                dVp[jt & 1] = mm(xk[v], dS[jt][v], dVp[jt & 1]);
-                acc = mm(O.Rs[4 * g + v][16 * jt + l16], dyop[v], acc);
-            }
-            accA[jt] = acc;
-        }
-        causal_tile(q < 2 ? O.Ap : O.Rp, (q & 1) ? O.Kp : O.Bp, q == 0 ? S.AB : (q == 1 ? S.AK : (q == 2 ? S.RB : S.RK)), q < 2, l16, g);
-        if (q == 0) {                                // this wave wrote AB itself: LDS keeps a wave's accesses in order
+            for (int v = 0; v < 4; ++v) S.AB[4 * g + v][l16] = acc[v];
             float m[CL];
             inverse_cols(S.AB, l16, m);
-            if (g == 0)
 #pragma unroll
-                for (int t = 0; t < CL; ++t) S.M[t][l16] = m[t];
+            for (int v = 0; v < 4; ++v) x[v] = by_group(g, m[v], m[4 + v], m[8 + v], m[12 + v]);
         }
-        f32x4 dU = dUp[0] + dUp[1], dV = dVp[0] + dVp[1];
+        // (one store with a selected address: with one in each of the branches the compiler merged them and left the address undefined
+        // on one way there)
+        put_half<TTERM2>(one.pair + (q == 0 ? L::MB : (q == 1 ? L::RKA + 8 : (q == 2 ? L::MB + 8 : L::RKA))), split3(x));
+    };
+    __syncthreads();
+    __syncthreads();
+    tiles(S.pl[0]);
+    for (int i = 0; i < nch; ++i) {
+        const PlanesB& O = S.pl[i & 1];
+        const LaneB two = lane_bases(sb + L::TWO + (i & 1) * L::SLOT, l16, g, own);
+        // ---------------------------------------------------------------- phase 1: the parts of dU, dV that need no tile
+        Sum2 dUs = SUM0, dVs = SUM0;
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) {
+            const Op3 st = join(split3(dS[2 * hb]), split3(dS[2 * hb + 1]));
+            add32(dUs, get3_tr(L::BD, one.tr, hb), st);
+            add32(dVs, get3_tr(L::KD, one.tr, hb), st);
+        }
+        here(dUs); here(dVs);
         __syncthreads();
         // ---------------------------------------------------------------- phase 2: dU, dW = M^T dU, dV, the gradient state
         {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) dU = mm(S.RB[4 * g + v][l16], dyop[v], dU);
-            f32x4 dW = ZERO4;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) dW = mm(S.M[4 * g + v][l16], dU[v], dW);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) S.dW[4 * g + v][own] = dW[v];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) dV = mm(S.AK[4 * g + v][l16], dW[v], dV);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) dV = mm(S.RK[4 * g + v][l16], dyop[v], dV);
+            const auto dyop = exact_piece<F32>(two.own + L::DY);             // dY[tau = 4 g + v][i]
+            add16(dUs, get_half<TTERM2>(one.pair + L::MB + 8), dyop);
+            Sum2 dWs = SUM0;
+            add16(dWs, get_half<TTERM2>(one.pair + L::MB), split3(total(dUs)));
+            const B3 dW = split3(total(dWs));
+            put3(one.own + L::DW, dW);
+            const Op3 yw = join(as3(dyop), dW);          // dY and dW share the instructions of what follows
+            add32(dVs, get_pair<TTERM2>(one.pair + L::RKA), yw);
+            const f32x4 dV = total(dVs);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if constexpr (F32) store_f32(p.dv, tok0 + static_cast<size_t>(nch - 1 - i) * CL, v, static_cast<uint32_t>(4 * g * H) * N + own, H, h, dV[v]);
@@ -588,18 +697,23 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const Args7c& p, int 
             }
 #pragma unroll
             for (int jt = 0; jt < 4; ++jt) {
-                f32x4 acc = accA[jt];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc = mm(O.As[4 * g + v][16 * jt + l16], dW[v], acc);
-                dS[jt] = dS[jt] * ld4(&O.dec[16 * jt + 4 * g]) + acc;
+                Sum2 x = SUM0;
+                add32(x, get_pair<TERM2>(two.pair + L::RA + 1024 * jt), yw);
+                dS[jt] = dS[jt] * ld4(&O.dec[16 * jt + 4 * g]) + total(x);
             }
         }
         __syncthreads();
-        // ---------------------------------------------------------------- phase 3: dAB, dAK (they need dW)
-        if (q < 2) causal_tile(S.dW, q == 0 ? O.U : O.V, q == 0 ? S.dAB : S.dAK, true, l16, g);
-        else if constexpr (!F32) {
-          if (i > 0) {
-            // The two waves without a tile here carry the finished rows of the visit before to global memory (parked by the
+        // ---------------------------------------------------------------- phase 3: dAB (q even), dAK (they need dW), by rows and by columns
+        {
+            const lds_t w = L::ONE + L::DW, o = L::TWO + (i & 1) * L::SLOT + (q & 1 ? L::V : L::U);
+            const bool o3 = F32 || (q & 1) == 0, byrow = q < 2;
+            const f32x4 t = causal_split(base_tr, byrow ? o : w, byrow ? o3 : true, byrow ? w : o, byrow ? true : o3, byrow, true, l16, g);
+            put_half<TTERM2>(one.pair + (q == 0 ? L::A_ROWS : (q == 1 ? L::A_ROWS + 8 : (q == 2 ? L::B_COLS : L::K_COLS))), split3(t));
+        }
+        if (i + 1 < nch) tiles(S.pl[(i + 1) & 1]);
+        if constexpr (!F32) {
+          if (q >= 2 && i > 0) {
+            // Two waves carry the finished rows of the visit before to global memory (parked by the
             // B waves in phase 1, dv by this role one visit earlier; both stay as they are until the next visit): the P
             // waves, for which this was a third of a phase that everybody waits for, keep to loads.
             const int tp = tid - 2 * 64;
@@ -617,9 +731,12 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const Args7c& p, int 
     }
 }
 
-template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
+template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
     const int lane = tid & 63, q = w & 3, l16 = lane & 15, g = lane >> 4;
     const int own = 16 * q + l16;                    // key channel j of this lane's column
+    using L = LB<F32>;
+    const LaneB one = lane_bases(sb + L::ONE, l16, g, own);
+    const Tr base_tr = tr_bases(sb, l16, g);
     f32x4 dS[4], S0b[4];                             // dS, S0 at [i = 16 ib + 4 g + v][j = own]
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib)
@@ -628,54 +745,61 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const Args7c& p, int 
             dS[ib][v] = p.dsT != nullptr ? p.dsT[bh * N * N + static_cast<size_t>(16 * ib + 4 * g + v) * N + own] : 0.f;
     auto fetch_state = [&](int c) __attribute__((always_inline)) {
         const float* slot = p.s + (bh * nch + c) * N * N;
-        uint32_t o = static_cast<uint32_t>(4 * g) * N + own;
+        uint32_t o = static_cast<uint32_t>(4 * g * N + own) * 4u;
         asm volatile("" : "+v"(o));
+        const char* const at = reinterpret_cast<const char*>(slot);
 #pragma unroll
         for (int ib = 0; ib < 4; ++ib)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) S0b[ib][v] = slot[o + (16 * ib + v) * N];
+            for (int v = 0; v < 4; ++v) S0b[ib][v] = *reinterpret_cast<const float*>(at + (16 * ib + v) * N * 4 + o);
     };
+    // fp32 planes of a visit, element [4 g + v][own] of plane k; d1, d2, dec of the own channel; parked outputs
+    lds_t fl = sb + static_cast<uint32_t>(4 * g * PS + own) * 4, cl = sb + 7 * 4 * CL * PS + 4 * own;
+    [[maybe_unused]] lds_t park = sb + static_cast<uint32_t>(offsetof(SmemCB<F32>, park)) + static_cast<uint32_t>(4 * g * PK + own) * 2;
+    opaque(fl); opaque(cl); opaque(park);
+    auto planes_of = [&](int visit) __attribute__((always_inline)) { return static_cast<lds_t>((visit & 1) * sizeof(PlanesB)); };
+    auto plane = [&](lds_t O, int k, int v) __attribute__((always_inline)) { return lds_ld<float>(fl + O + 4 * PS * (CL * k + v)); };
+    auto chan = [&](lds_t O, int k) __attribute__((always_inline)) { return lds_ld<float>(cl + O + 4 * N * k); };
     float Pj = 0.f;                                  // P at the end of the chunk whose phase 4 comes next
-    f32x4 xA = ZERO4, xR = ZERO4, xB = ZERO4, xK = ZERO4;     // state parts of dA', dR', dB', dK', carried into the next visit's phase 1
+    f32x4 xA = ZERO4, xB = ZERO4, xK = ZERO4, dRp = ZERO4;    // state parts of dA', dB', dK', and dR', carried into the next visit's phase 1
+    Op3 bk;                                          // and B', K' as an operand
+    // a contraction over 16 with a pair of tiles (one after the other: the registers do not hold the operands of all of them)
+    auto tile2 = [&](uint32_t pair, const Op3& b) __attribute__((always_inline)) {
+        Sum2 s = SUM0;
+        add32(s, get_pair<TTERM2>(one.pair + pair), b);
+        __builtin_amdgcn_sched_barrier(0);
+        return total(s);
+    };
     // tile parts, scaling, decay gradient of the chunk whose planes are O and whose first row is row0; results parked as bf16
-    auto finish = [&](const PlanesB& O, const size_t row0) __attribute__((always_inline)) {
-        uint32_t lo = static_cast<uint32_t>(4 * g * H) * N + own;
+    auto finish = [&](const lds_t O, const size_t row0) __attribute__((always_inline)) {
+        [[maybe_unused]] uint32_t lo = static_cast<uint32_t>(4 * g * H) * N + own;
         asm volatile("" : "+v"(lo));
         auto put = [&](const int k, uint16_t* dst, const int v, const float x) __attribute__((always_inline)) {
             if constexpr (F32) store_f32(dst, row0, v, lo, H, h, x);
-            else S.park[k][4 * g + v][own] = f2bf(x);
+            else lds_st<uint16_t>(park + 2 * PK * (CL * k + v), f2bf(x));
         };
-        const float d1j = O.d1[own], d2j = O.d2[own];
+        const float d1j = chan(O, 0), d2j = chan(O, 1);
         f32x4 bp, kp, ap, rp;                        // planes at [s or t = 4 g + v][j]
 #pragma unroll
-        for (int v = 0; v < 4; ++v) { bp[v] = O.Bp[4 * g + v][own]; kp[v] = O.Kp[4 * g + v][own]; ap[v] = O.Ap[4 * g + v][own]; rp[v] = O.Rp[4 * g + v][own]; }
-        f32x4 tA = ZERO4, tR = ZERO4, tB = ZERO4, tK = ZERO4;
-        const f32x4 dab = ld4(&S.dAB[l16][4 * g]), dak = ld4(&S.dAK[l16][4 * g]), drb = ld4(&S.dRB[l16][4 * g]), drk = ld4(&S.dRK[l16][4 * g]);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            tA = mm(dab[v], bp[v], tA); tR = mm(drb[v], bp[v], tR);
-            tB = mm(S.dAB[4 * g + v][l16], ap[v], tB); tK = mm(S.dAK[4 * g + v][l16], ap[v], tK);
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            tA = mm(dak[v], kp[v], tA); tR = mm(drk[v], kp[v], tR);
-            tB = mm(S.dRB[4 * g + v][l16], rp[v], tB); tK = mm(S.dRK[4 * g + v][l16], rp[v], tK);
-        }
+        for (int v = 0; v < 4; ++v) { bp[v] = plane(O, 2, v); kp[v] = plane(O, 3, v); ap[v] = plane(O, 0, v); rp[v] = plane(O, 1, v); }
+        const f32x4 tA = tile2(L::A_ROWS, bk);
+        const Op3 ar = join(split3(ap), split3(rp));
+        const f32x4 tB = tile2(L::B_COLS, ar), tK = tile2(L::K_COLS, ar);
         float del[4], ada[4], dwf[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int t = 4 * g + v;
-            const float dAp = fmaf(d1j, xA[v], tA[v]), dRp = fmaf(d1j, xR[v], tR[v]);
+            const float dAp = fmaf(d1j, xA[v], tA[v]);
             const float dBp = fmaf(d2j, xB[v], tB[v]), dKp = fmaf(d2j, xK[v], tK[v]);
-            const float ea = O.EA[t][own], er = O.ER[t][own];
-            const float eb = __frcp_rn(er);
+            const float ea = plane(O, 4, v), er = plane(O, 5, v);
+            float eb = __builtin_amdgcn_rcpf(er);                               // (er is between e^-4.9 and e^4.9)
+            eb = fmaf(fmaf(-er, eb, 1.f), eb, eb);
             put(0, p.da, v, dAp * ea);
-            put(1, p.dr, v, dRp * er);
+            put(1, p.dr, v, dRp[v] * er);
             put(2, p.db, v, dBp * eb);
             put(3, p.dk, v, dKp * eb);
             ada[v] = ap[v] * dAp;
-            del[v] = fmaf(rp[v], dRp, -fmaf(bp[v], dBp, kp[v] * dKp));      // r dr - b db - k dk
-            dwf[v] = O.DWF[t][own];
+            del[v] = fmaf(rp[v], dRp[v], -fmaf(bp[v], dBp, kp[v] * dKp));      // r dr - b db - k dk
+            dwf[v] = plane(O, 6, v);
         }
         // G_t = P_{t+1} + del_t,  P_t = G_t + a da:  suffix sums over t = 4 g + v, later lane groups first
         const float tot = (del[0] + ada[0]) + (del[1] + ada[1]) + (del[2] + ada[2]) + (del[3] + ada[3]);
@@ -694,22 +818,21 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const Args7c& p, int 
     __syncthreads();
     for (int i = 0; i < nch; ++i) {
         const int c = nch - 1 - i;
-        const PlanesB& O = S.pl[i & 1];
+        const lds_t O = planes_of(i);
+        const LaneB two = lane_bases(sb + L::TWO + (i & 1) * L::SLOT, l16, g, own);
         // ---------------------------------------------------------------- phase 1: finish the previous visit's chunk
-        if (i > 0) finish(S.pl[(i - 1) & 1], tok0 + static_cast<size_t>(c + 1) * CL);
-        __syncthreads();
-        // ---------------------------------------------------------------- phase 2: dY S0, U dS, V dS; dRB, dRK
-        if (i == 0 && p.dsT != nullptr) {
+        if (i > 0) finish(planes_of(i - 1), tok0 + static_cast<size_t>(c + 1) * CL);
+        else if (p.dsT != nullptr) {
             // P at the end of the call: sum_i dsT o S_T with S_T = S0 dec + U^T (B' d2) + V^T (K' d2) of the last chunk
-            const float decj = O.dec[own];
+            const float decj = chan(O, 2);
+            const Op3 bdk = join(get3(one.own + L::BD), get3(one.own + L::KD));
             float pp = 0.f;
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) {
-                f32x4 acc = ZERO4;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc = mm(O.U[4 * g + v][16 * ib + l16], O.Bd[4 * g + v][own], acc);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc = mm(O.V[4 * g + v][16 * ib + l16], O.Kd[4 * g + v][own], acc);
+                const lds_t o = two.rows[ib & 1] + 512 * ib;
+                Sum2 x = SUM0;
+                add32(x, join(get3(o + L::U), as3(exact_piece<F32>(o + L::V))), bdk);
+                const f32x4 acc = total(x);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) pp = fmaf(dS[ib][v], fmaf(S0b[ib][v], decj, acc[v]), pp);
             }
@@ -717,73 +840,94 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const Args7c& p, int 
             pp += __shfl_xor(pp, 32, 64);
             Pj = pp;
         }
+        __syncthreads();
+        // ---------------------------------------------------------------- phase 2: dY S0, U dS, V dS; dRB (q even), dRK, by rows and by columns
+        auto ya = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::DY, two.tr, hb); };
+        auto ua = [&](int hb) __attribute__((always_inline)) { return get3_tr(L::U, two.tr, hb); };
+        auto va = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::V, two.tr, hb); };
+        Op3 s0[2];
+        f32x4 xR;
         {
-            f32x4 pr[2] = {ZERO4, ZERO4}, pb[2] = {ZERO4, ZERO4}, pk[2] = {ZERO4, ZERO4};   // two partial sums each: independent chains
+            Sum2 pr = SUM0, pb = SUM0, pk = SUM0;
 #pragma unroll
-            for (int ib = 0; ib < 4; ++ib) {
-                const f32x4 ya = ld4(&O.dY[l16][16 * ib + 4 * g]), ua = ld4(&O.U[l16][16 * ib + 4 * g]), va = ld4(&O.V[l16][16 * ib + 4 * g]);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    pr[ib & 1] = mm(ya[v], S0b[ib][v], pr[ib & 1]);
-                    pb[ib & 1] = mm(ua[v], dS[ib][v], pb[ib & 1]);
-                    pk[ib & 1] = mm(va[v], dS[ib][v], pk[ib & 1]);
-                }
+            for (int hb = 0; hb < 2; ++hb) {
+                s0[hb] = join(split3(S0b[2 * hb]), split3(S0b[2 * hb + 1]));
+                const Op3 ds = join(split3(dS[2 * hb]), split3(dS[2 * hb + 1]));
+                add32(pr, ya(hb), s0[hb]);
+                add32(pb, ua(hb), ds);
+                add32(pk, va(hb), ds);
             }
-            xR = pr[0] + pr[1]; xB = pb[0] + pb[1]; xK = pk[0] + pk[1];
+            xR = total(pr); xB = total(pb); xK = total(pk);
         }
-        if (q >= 2) causal_tile(O.dY, q == 2 ? O.U : O.V, q == 2 ? S.dRB : S.dRK, false, l16, g);
+        {
+            const lds_t copy = L::TWO + (i & 1) * L::SLOT, y = copy + L::DY, o = copy + (q & 1 ? L::V : L::U);
+            const bool o3 = F32 || (q & 1) == 0, byrow = q < 2;
+            const f32x4 t = causal_split(base_tr, byrow ? o : y, byrow ? o3 : F32, byrow ? y : o, byrow ? F32 : o3, byrow, false, l16, g);
+            put_half<TTERM2>(one.pair + (q == 0 ? L::R_ROWS : (q == 1 ? L::R_ROWS + 8 : (q == 2 ? L::B_COLS + 8 : L::K_COLS + 8))), split3(t));
+        }
         __syncthreads();
         // ---------------------------------------------------------------- phase 3: dW S0; the gradient state
         {
-            const float decj = O.dec[own];
-            f32x4 rs, as;
+            const float decj = chan(O, 2);
+            const Op3 ra = get_pair<TERM2>(two.own_pair + L::RA);
+            Sum2 pa = SUM0;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) { rs[v] = O.Rs[4 * g + v][own]; as[v] = O.As[4 * g + v][own]; }
-            f32x4 pa[2] = {ZERO4, ZERO4};
+            for (int hb = 0; hb < 2; ++hb) add32(pa, get3_tr(L::DW, one.tr, hb), s0[hb]);
+            xA = total(pa);
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) {
-                const f32x4 wa = ld4(&S.dW[l16][16 * ib + 4 * g]);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) pa[ib & 1] = mm(wa[v], S0b[ib][v], pa[ib & 1]);
-                f32x4 acc = ZERO4;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc = mm(O.dY[4 * g + v][16 * ib + l16], rs[v], acc);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc = mm(S.dW[4 * g + v][16 * ib + l16], as[v], acc);
-                dS[ib] = dS[ib] * decj + acc;
+                Sum2 x = SUM0;
+                add32(x, join(as3(exact_piece<F32>(two.rows[ib & 1] + 512 * ib + L::DY)), get3(one.rows[ib & 1] + 512 * ib + L::DW)), ra);
+                dS[ib] = dS[ib] * decj + total(x);
             }
-            xA = pa[0] + pa[1];
+            // dR' needs no tile of this phase; B', K' stay for dA'
+            f32x4 bp, kp;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) { bp[v] = plane(O, 2, v); kp[v] = plane(O, 3, v); }
+            bk = join(split3(bp), split3(kp));
+            const f32x4 tR = tile2(L::R_ROWS, bk);
+            const float d1j = chan(O, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) dRp[v] = fmaf(d1j, xR[v], tR[v]);
             if (c > 0) fetch_state(c - 1);
         }
         __syncthreads();
     }
-    finish(S.pl[(nch - 1) & 1], tok0);
+    finish(planes_of(nch - 1), tok0);
     __syncthreads();
 }
 
 template <bool F32>
 __global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c p) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
+    extern __shared__ __align__(32) unsigned char smem_raw[];
     SmemCB<F32>& S = *reinterpret_cast<SmemCB<F32>*>(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x, b = blockIdx.y;
     const size_t bh = static_cast<size_t>(b) * p.H + h;
     const size_t tok0 = static_cast<size_t>(b) * p.T;
     const int nch = p.T / CL;
-    if (w < 4) bwd_role_a(S, p, tid, w, bh, nch, tok0, p.H, h);
-    else if (w < 8) bwd_role_b(S, p, tid, w, bh, nch, tok0, p.H, h);
-    else bwd_role_p(S, p, tid, w, tok0, nch, p.H, h);
+    const lds_t sb = lds_of(smem_raw);
+    if (w < 4) bwd_role_a(S, sb, p, tid, w, bh, nch, tok0, p.H, h);
+    else if (w < 8) bwd_role_b(S, sb, p, tid, w, bh, nch, tok0, p.H, h);
+    else bwd_role_p(S, sb, p, tid, w, tok0, nch, p.H, h);
 }
 
 const uint16_t* el(const void* p) { return static_cast<const uint16_t*>(p); }
 uint16_t* el(void* p) { return static_cast<uint16_t*>(p); }
 
-template <bool F32> int start_bwd(hipStream_t st, int B, int H, const Args7c& p) {
-    static_assert(sizeof(SmemCB<F32>) <= 160 * 1024, "the backward's LDS must fit one CU");
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_bwd<F32>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       static_cast<int>(sizeof(SmemCB<F32>)));
+template <bool F32, bool KEEP> int start_fwd(hipStream_t st, int B, int H, const Args7c& p) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_fwd<F32, KEEP>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       static_cast<int>(F_TOTAL<F32>));
     if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
-    hipLaunchKernelGGL(rwkv7c_bwd<F32>, dim3(H, B), dim3(NTB), sizeof(SmemCB<F32>), st, p);
+    rwkv7c_fwd<F32, KEEP><<<dim3(H, B), dim3(NTF), F_TOTAL<F32>, st>>>(p);
+    return launch_status();
+}
+template <bool F32> int start_bwd(hipStream_t st, int B, int H, const Args7c& p) {
+    static_assert(LB<F32>::BYTES <= 160 * 1024, "the backward's LDS must fit one CU");
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_bwd<F32>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       static_cast<int>(LB<F32>::BYTES));
+    if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
+    hipLaunchKernelGGL(rwkv7c_bwd<F32>, dim3(H, B), dim3(NTB), LB<F32>::BYTES, st, p);
     return launch_status();
 }
 
@@ -794,9 +938,8 @@ int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0,
     Args7c p{};
     p.T = T; p.H = H; p.s0 = s0; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b); p.y = el(y);
     p.sT = sT; p.s = s; p.sa = sa;
-    const auto kernel = s != nullptr ? (f32 ? rwkv7c_fwd<true, true> : rwkv7c_fwd<false, true>) : (f32 ? rwkv7c_fwd<true, false> : rwkv7c_fwd<false, false>);
-    hipLaunchKernelGGL(kernel, dim3(H, B), dim3(NT), 0, st, p);
-    return launch_status();
+    if (s != nullptr) return f32 ? start_fwd<true, true>(st, B, H, p) : start_fwd<false, true>(st, B, H, p);
+    return f32 ? start_fwd<true, false>(st, B, H, p) : start_fwd<false, false>(st, B, H, p);
 }
 
 int launch7c_bwd(hipStream_t st, bool f32, int B, int T, int H, const void* r, const void* w, const void* k, const void* v,

@@ -1,4 +1,6 @@
 """GPU parity: rwkv7 clamp-w with state passing through the C ABI against the CPU oracle."""
+import math
+
 import pytest
 import torch
 
@@ -244,3 +246,32 @@ def test_fp32_sweeps_option_runs_the_step_kernels(lib, B, T, H):
         for name, want, e, got in zip(NAMES, ref, emu, out[algo]):
             assert_fp32_mode(f"{algo} {name}", want.reshape(got.shape), e.reshape(got.shape), got)
     assert not torch.equal(out["chunked"][0], out["sweeps"][0])
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("T", [16, 32, 48, 112])
+@pytest.mark.parametrize("shift", [-6.0, 0.5, 6.0])
+def test_fp32_state_keeps_24_bits(T, f32, shift):
+    """One, two, three and seven chunks, slow to strong decays: the fp32 state against the step form in 64 bits.  Bound: a factor of the
+    last chunk carries about 1e-7 (an exponential's last bit and a product's rounding), a sum of 16 terms and of two products as much."""
+    B, H, N = 2, 3, 64
+    g = torch.Generator().manual_seed(T)
+    n = lambda *s: torch.randn(*s, generator=g)
+    kk = torch.nn.functional.normalize(n(B, T, H, N), dim=-1)
+    s0 = n(B, H, N, N) * 0.1
+    x = [n(B, T, H, N) * 0.5, n(B, T, H, N) + shift, n(B, T, H, N) * 0.5, n(B, T, H, N) * 0.5, -kk, kk * torch.sigmoid(n(B, T, H, N))]
+    x = [t.to(torch.float32 if f32 else torch.bfloat16) for t in x]
+    r, w, k, v, a, b = (t.double() for t in x)
+    S = s0.double()
+    d = torch.exp(-math.exp(-0.5) * torch.sigmoid(w))
+    ys = []
+    for t in range(T):
+        sa = S @ a[:, t, :, :, None]
+        S = S * d[:, t, :, None, :] + sa * b[:, t, :, None, :] + v[:, t, :, :, None] * k[:, t, :, None, :]
+        ys.append((S @ r[:, t, :, :, None])[..., 0])
+    dev = [t.cuda().view(B, T, H * N) for t in x]
+    with torch.no_grad():
+        y, sT = R.RWKV7_STATE_PASSING_CLAMPW_CUDA(s0.cuda(), *dev)
+    rel = lambda p, q: ((p.double().cpu().reshape(q.shape) - q).norm() / q.norm()).item()
+    assert rel(sT, S) <= 2e-7
+    assert rel(y, torch.stack(ys, 1)) <= (4e-7 if f32 else 2.0 ** -8)
