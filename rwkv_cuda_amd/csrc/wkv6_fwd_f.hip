@@ -547,23 +547,39 @@ __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
     else role_tiles<LOCAL>(S, a, lane, w, bh, n, nit);
 }
 
-// States entering the blocks from the local results, one workgroup of 256 threads per (batch, head), 16 consecutive key
-// channels of one value channel per thread.  Forward (reverse = 0): S = s0; out[blk] = S; S <- S 2^logdec[blk] + local[blk].
+// States entering the blocks from the local results, four key channels of one value channel per thread, a quarter of a (batch,
+// head) per workgroup of 256.  Forward (reverse = 0): S = s0; out[blk] = S; S <- S 2^logdec[blk] + local[blk].
 // Reverse: the same from the last block down, from zero: what enters a block from above.
+// It is there for few (batch, head) pairs, so what bounds it is latency: 16 bytes a lane, side by side, and the reads of SCAN_AHEAD
+// blocks, of which none depends on another, in flight together.  B1 H32, 8 blocks: 5.1 us (launch, one round of reads, the stores); with sixteen channels a thread (a quarter
+// of the workgroups, 64 bytes between lanes) and the reads of one block at a time 11.
+constexpr int SCAN_AHEAD = 8, SCAN_WG = N * N / (4 * 256);
 __global__ __launch_bounds__(256) void wkv6_scan(const float* __restrict__ local, const float* __restrict__ logdec, const uint16_t* __restrict__ s0,
                                                  float* __restrict__ out, const int NB, const int reverse) {
-    const size_t bh = blockIdx.x;
-    const int e = threadIdx.x * 16, j0 = e % N;
-    float x[16];
+    const size_t bh = blockIdx.x / SCAN_WG;
+    const int e = ((blockIdx.x % SCAN_WG) * 256 + threadIdx.x) * 4, j0 = e % N;
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+    if (s0 != nullptr && !reverse) {
+        const uint2 s = *reinterpret_cast<const uint2*>(s0 + bh * (N * N) + e);
+        x = f32x4{bf_lo(s.x), bf_hi(s.x), bf_lo(s.y), bf_hi(s.y)};
+    }
+    for (int i0 = 0; i0 < NB; i0 += SCAN_AHEAD) {
+        f32x4 d[SCAN_AHEAD], y[SCAN_AHEAD];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) x[q] = (s0 != nullptr && !reverse) ? bf2f(s0[bh * (N * N) + e + q]) : 0.f;
-    for (int i = 0; i < NB; ++i) {
-        const int blk = reverse ? NB - 1 - i : i;
-        const size_t o = (bh * NB + blk) * (N * N) + e;
+        for (int z = 0; z < SCAN_AHEAD; ++z) {          // (past the last block: its values once more, not used)
+            const int i = i0 + z < NB ? i0 + z : NB - 1;
+            const size_t blk = bh * NB + (reverse ? NB - 1 - i : i);
+            d[z] = *reinterpret_cast<const f32x4*>(logdec + blk * N + j0);
+            y[z] = *reinterpret_cast<const f32x4*>(local + blk * (N * N) + e);
+        }
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            out[o + q] = x[q];
-            x[q] = fmaf(x[q], exp2_fast(logdec[(bh * NB + blk) * N + j0 + q]), local[o + q]);
+        for (int z = 0; z < SCAN_AHEAD; ++z) {
+            const int i = i0 + z;
+            if (i < NB) {
+                *reinterpret_cast<f32x4*>(out + (bh * NB + (reverse ? NB - 1 - i : i)) * (N * N) + e) = x;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) x[q] = fmaf(x[q], exp2_fast(d[z][q]), y[z][q]);
+            }
         }
     }
 }
@@ -586,7 +602,7 @@ int launch_wkv6_fwd_fused(hipStream_t st, int B, int T, int C, int H, const uint
     a.NB = NB; a.TB = TB; a.blk_state = blk_state; a.blk_decay = blk_decay;
     if (head_decay) hipLaunchKernelGGL((wkv6_fwd_fused<true, true>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
     else hipLaunchKernelGGL((wkv6_fwd_fused<true, false>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
-    hipLaunchKernelGGL(wkv6_scan, dim3(B * H), dim3(256), 0, st, blk_state, blk_decay, s0, s32, NB, 0);
+    hipLaunchKernelGGL(wkv6_scan, dim3(B * H * SCAN_WG), dim3(256), 0, st, blk_state, blk_decay, s0, s32, NB, 0);
     a.blk_state = nullptr; a.blk_decay = nullptr; a.s32 = s32;
     if (head_decay) hipLaunchKernelGGL((wkv6_fwd_fused<false, true>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
     else hipLaunchKernelGGL((wkv6_fwd_fused<false, false>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
@@ -595,7 +611,7 @@ int launch_wkv6_fwd_fused(hipStream_t st, int B, int T, int C, int H, const uint
 
 // reverse scan for the backward (wkv6_bwd_f.hip): out[blk] = what enters block blk from above
 int launch_wkv6_scan_reverse(hipStream_t st, int BH, int NB, const float* local, const float* logdec, float* out) {
-    hipLaunchKernelGGL(wkv6_scan, dim3(BH), dim3(256), 0, st, local, logdec, static_cast<const uint16_t*>(nullptr), out, NB, 1);
+    hipLaunchKernelGGL(wkv6_scan, dim3(BH * SCAN_WG), dim3(256), 0, st, local, logdec, static_cast<const uint16_t*>(nullptr), out, NB, 1);
     return launch_status();
 }
 

@@ -92,6 +92,19 @@ def test_few_sequences_run_as_blocks_with_a_scan(lib, B, H, state):
         assert float(gw[:, 0].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("T", [1140, 2040, 2170])
+def test_scan_over_more_blocks_than_it_reads_at_once(lib, T):
+    """9, 16 and 17 blocks of 128 tokens: the scan reads eight of them together."""
+    B, H = 1, 2
+    r, k, v, w, u, gy, s0 = synth.wkv6_inputs(B, T, H * 64, H, seed=T, state=True)
+    ref = O.wkv6_grads(B, T, H * 64, H, r, k, v, w, u, gy, s0=s0)
+    emu = O.emulate_wkv6_bf16(B, T, H * 64, H, r, k, v, w, u, gy, s0=s0)
+    got, handed_back = run_pair(lib, B, T, H, r, k, v, w, u, s0, gy, saved_fill=0x7f)
+    assert handed_back == 0
+    for name, a, e, g in zip(NAMES, ref, emu, got):
+        assert_no_worse(f"T{T} {name}", a, e, g)
+
+
 def test_one_sweep_hands_strong_decays_to_the_two_sweep_kernels(lib):
     """Decays so strong that a channel loses more than e^-60 over 16 tokens: those (batch, head) pairs are flagged by the
     one-sweep kernel and redone by the two-sweep kernels, whose chunks have a step-by-step path; the others are not."""
