@@ -1457,18 +1457,19 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H, const rw
     int* flg = reinterpret_cast<int*>(wsb + round16(rwkv_wkv6f_backward_workspace_bytes(B, T, C, H)));
     int TB;
     const int NB = scan_blocks(B, T, H, &TB, flags);
+    float* gu32 = nullptr;                // several blocks: gu of each in fp32, which the first sweep adds up where it has nothing to redo
     if (NB > 1) {
         const size_t nq = static_cast<size_t>(B) * H * NB;
         float* local = reinterpret_cast<float*>(reinterpret_cast<char*>(flg) + round16(static_cast<size_t>(B) * H * 8 * sizeof(int)));
         float* ds32 = local + nq * 64 * 64;
         float* logdec = ds32 + nq * 64 * 64;
-        float* gu32 = logdec + nq * 64;
+        gu32 = logdec + nq * 64;
         zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w, u, gy, gr, gk, gv, gw, pu, gs, static_cast<const char*>(saved), flg,
                                           NB, TB, local, logdec, ds32, gu32)) return e;
     } else if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w, u, gy, gr, gk, gv, gw, pu, gs, static_cast<const char*>(saved), flg)) return e;
     // (batch, head) pairs with a decay the mid-point factors cannot carry: the two sweeps redo them, all others return at once
-    if (int e = launch_wkv6_bwd_a_chunk(st, W_RAW, B, T, C, H, r, k, v, w, u, s, gy, gr, pu, rdr, flg)) return e;
+    if (int e = launch_wkv6_bwd_a_chunk(st, W_RAW, B, T, C, H, r, k, v, w, u, s, gy, gr, pu, rdr, flg, gu32, NB)) return e;
     // (the second sweep's workgroups of batch row 0 first add the per-batch gu rows up: they are complete by then, and a
     //  launch of its own for that costs as much as any other, about 5 us)
     return launch_wkv6_bwd_b_chunk(st, W_RAW, B, T, C, H, r, k, v, w, u, s, gy, gk, gv, gw, gs, rdr, flg, pu, gu);

@@ -475,8 +475,14 @@ DEVINL void bwa_state(SmemA2& S, const ArgsB& a, const int tid, const size_t bas
 template <int WMODE, int SPLIT = 0>
 __global__ __launch_bounds__(NTA) void wkv6_bwd_a_ws(const ArgsB a) {
     __shared__ SmemA2 S;
-    if (skip_unflagged(a.only_flagged, blockIdx.x)) return;
     const int tid = threadIdx.x;
+    if (skip_unflagged(a.only_flagged, blockIdx.x)) {
+        if (SPLIT == 0 && a.gu_parts != nullptr && tid < N) {
+            const size_t i = static_cast<size_t>(blockIdx.x) * N + tid, n = static_cast<size_t>(gridDim.x) * N;     // C = H N
+            a.gu[i] = f2bf(block_sum(a.gu_parts, a.gu_blocks, n, i));
+        }
+        return;
+    }
     const int b = blockIdx.x / a.H, h = blockIdx.x % a.H;
     const int hk = SPLIT != 0 ? h ^ a.cross : h;       // the block of 64 channels that r, k, w, u come from and gr, gu go to
     const size_t vbase = static_cast<size_t>(b) * a.T * a.C + static_cast<size_t>(h) * N;
@@ -503,10 +509,11 @@ __global__ __launch_bounds__(NTA) void wkv6_bwd_a_ws(const ArgsB a) {
 int launch_wkv6_bwd_a_chunk(hipStream_t st, int wmode, int B, int T, int C, int H, const uint16_t* r,
                             const uint16_t* k, const uint16_t* v, const void* w, const uint16_t* u,
                             const uint16_t* s0, const uint16_t* gy, uint16_t* gr, uint16_t* gu, float* rdr,
-                            const int* only_flagged) {
+                            const int* only_flagged, const float* gu_parts, int gu_blocks) {
     ArgsB a{};
     a.T = T; a.C = C; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.s0 = s0; a.gy = gy;
     a.gr = gr; a.gu = gu; a.rdr = rdr; a.only_flagged = only_flagged;
+    a.gu_parts = gu_parts; a.gu_blocks = gu_blocks;
     if (wmode == W_RAW) hipLaunchKernelGGL(wkv6_bwd_a_ws<W_RAW>, dim3(B * H), dim3(NTA), 0, st, a);
     else if (wmode == W_EW) hipLaunchKernelGGL(wkv6_bwd_a_ws<W_EW>, dim3(B * H), dim3(NTA), 0, st, a);
     else hipLaunchKernelGGL(wkv6_bwd_a_ws<W_HEAD>, dim3(B * H), dim3(NTA), 0, st, a);

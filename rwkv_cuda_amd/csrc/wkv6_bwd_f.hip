@@ -879,13 +879,12 @@ __global__ __launch_bounds__(NTG) void wkv6_bwd_fused(const ArgsG arg) {
     }
 }
 
-// gu of a batch row from its blocks: out[b][c] = bf16(sum_blk part[blk][b][c])
-__global__ __launch_bounds__(256) void gu_block_sum(const int NB, const size_t n, const float* __restrict__ part, uint16_t* __restrict__ out) {
+// wkv5: gu and gw of a batch row from its blocks: out[b][c] = bf16(sum_blk part[blk][b][c]) (wkv6: the kernel that comes next does it)
+__global__ __launch_bounds__(256) void block_sums(const int NB, const size_t n, const float* __restrict__ pu, uint16_t* __restrict__ gu,
+                                                  const float* __restrict__ pw, uint16_t* __restrict__ gw) {
     const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
     if (i >= n) return;
-    float x = 0.f;
-    for (int blk = 0; blk < NB; ++blk) x += part[blk * n + i];
-    out[i] = f2bf(x);
+    (blockIdx.y == 0 ? gu : gw)[i] = f2bf(block_sum(blockIdx.y == 0 ? pu : pw, NB, n, i));
 }
 
 }  // namespace
@@ -913,9 +912,10 @@ int launch_wkv6_bwd_fused(hipStream_t st, int B, int T, int C, int H, const uint
     if (gwp != nullptr) a.gw32 = gw32;
     if (hd) hipLaunchKernelGGL((wkv6_bwd_fused<W_HEAD, false>), dim3(B * H * NB), dim3(NTG), 0, st, a);
     else hipLaunchKernelGGL((wkv6_bwd_fused<W_RAW, false>), dim3(B * H * NB), dim3(NTG), 0, st, a);
-    const size_t n = static_cast<size_t>(B) * C;
-    hipLaunchKernelGGL(gu_block_sum, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, NB, n, gu32, gu);
-    if (gwp != nullptr) hipLaunchKernelGGL(gu_block_sum, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, NB, n, gw32, gwp);
+    if (hd) {
+        const size_t n = static_cast<size_t>(B) * C;
+        hipLaunchKernelGGL(block_sums, dim3(static_cast<unsigned>((n + 255) / 256), 2), dim3(256), 0, st, NB, n, gu32, gu, gw32, gwp);
+    }
     return launch_status();
 }
 

@@ -101,6 +101,10 @@ struct ArgsB {
     // when not null: [B*H][8]; a workgroup runs only if one of its eight words is not zero (the (batch, head) pairs that
     // the one-sweep backward has handed back)
     const int* only_flagged;
+    // when not null (sweep A only): gu of the (batch, head) pairs that it skips, which ran as gu_blocks blocks of time: fp32 terms
+    // [block][B][C], added up and rounded once
+    const float* gu_parts;
+    int gu_blocks;
     // when not null (sweep B only): out[c] = bf16(sum_b float(in[b][c])), the sum of per-batch-row partials over the batch
     // (torch.sum(gu, 0) of the wrapper), done by the workgroups of batch row 0 before anything else.  `in` must be
     // complete when the kernel starts: sweep B does not write it.
@@ -112,6 +116,18 @@ DEVINL bool skip_unflagged(const int* f, const int bh) {
     if (f == nullptr) return false;
     const int4 x = *reinterpret_cast<const int4*>(f + 8 * bh), y = *reinterpret_cast<const int4*>(f + 8 * bh + 4);
     return (x.x | x.y | x.z | x.w | y.x | y.y | y.z | y.w) == 0;
+}
+// element i of a sum over nb blocks that lie n apart; eight reads in flight (one at a time each waits for memory, 0.5 us)
+DEVINL float block_sum(const float* __restrict__ part, const int nb, const size_t n, const size_t i) {
+    float s = 0.f;
+    for (int z0 = 0; z0 < nb; z0 += 8) {
+        float x[8];
+#pragma unroll
+        for (int z = 0; z < 8; ++z) x[z] = part[static_cast<size_t>(z0 + z < nb ? z0 + z : nb - 1) * n + i];
+#pragma unroll
+        for (int z = 0; z < 8; ++z) s += z0 + z < nb ? x[z] : 0.f;
+    }
+    return s;
 }
 
 // A head of 128 channels as four heads of 64 (SPLIT = true, wkv5 only).  With the key channels j and the value channels
