@@ -93,6 +93,9 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
     //  row at every token - a cache hit - so that all prep waves run the same loads and the waits count the same)
     const char* __restrict__ pB = reinterpret_cast<const char*>(lower ? (HD ? a.w + h * N : a.w + base) : a.v + base);   // w | v
     const uint32_t bmask = (HD && lower) ? 127u : ~0u;
+    // LOCAL: a state takes no r.  Its rows are not read (the loads stay, of one row that hits the cache, for the same reason), R' is not made
+    // and neither is the diagonal of A.  B1 T3001 C2048: 24.5 -> 20.8 us with the reads and this arithmetic left out.
+    const uint32_t amask = (LOCAL && lower) ? 127u : ~0u;
     const uint32_t row_b = 2u * static_cast<uint32_t>(a.C);                                     // bytes from a token to the next
     uint32_t offA = (8 * (w & 3) + (lane >> 3)) * row_b + 16 * (lane & 7);                      // rows 8 (w & 3) .. +7
     const uint32_t lastA = static_cast<uint32_t>(a.T - 1) * row_b + 16 * (lane & 7);
@@ -113,7 +116,7 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
     Raw ring[DEPTH];                       // DEPTH chunks ahead
     auto fetch = [&](const int c, Raw& x) __attribute__((always_inline)) {
         const uint32_t o = min(static_cast<uint32_t>(c * L) * row_b + offA, lastA);
-        x.a = *reinterpret_cast<const u32x4*>(pA + o);
+        x.a = *reinterpret_cast<const u32x4*>(pA + (o & amask));
         x.b = *reinterpret_cast<const u32x4*>(pB + (o & bmask));
     };
     // the rows of chunk c into the slot: r, k, w where the R' hi, K' hi, R' lo planes will be (staging), v in place
@@ -219,9 +222,10 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
         }
         // (the stores side by side, with no load between them: the compiler then pairs them, two planes or two rows an instruction)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) { lds_st<uint32_t>(so + O_RPH + e * 16 * ROW_B + b_tp, r0[e].h); lds_st<uint32_t>(so + O_RPL + e * 16 * ROW_B + b_tp, r0[e].l); }
+        for (int e = 0; e < (LOCAL ? 0 : 2); ++e) { lds_st<uint32_t>(so + O_RPH + e * 16 * ROW_B + b_tp, r0[e].h); lds_st<uint32_t>(so + O_RPL + e * 16 * ROW_B + b_tp, r0[e].l); }
 #pragma unroll
         for (int e = 0; e < 2; ++e) { lds_st<uint32_t>(so + O_KPH + e * 16 * ROW_B + b_tp, k0[e].h); lds_st<uint32_t>(so + O_KPL + e * 16 * ROW_B + b_tp, k0[e].l); }
+        if constexpr (LOCAL) return;
         allreduce2_rows(ruk[0], ruk[1]);                       // sums over the four channel pairs of this wave
         if (jq == 0) { lds_st<float>(so + O_RUK + w * (4 * L) + b_l, ruk[0]); lds_st<float>(so + O_RUK + w * (4 * L) + 64 + b_l, ruk[1]); }
     };
