@@ -47,6 +47,7 @@ constexpr int DEPTH = 2;           // chunks that the prep waves load ahead (fou
 constexpr int KEPT = 3;            // iterations between the preparation of a chunk and its finishing
 constexpr int TRIP = 6;            // iterations per trip of the prep loop: a multiple of both, so that the registers of the
                                    // loads in flight and of what is kept for the finishing have fixed names (no copies)
+template <bool LOCAL> constexpr int trip = LOCAL ? DEPTH : TRIP;      // (LOCAL: nothing is finished)
 constexpr int TQ = 20;             // causal tiles [t][s], 32 bf16 and 16 bytes of padding: 80 B (16-byte reads of 16 rows hit all banks once)
 
 struct alignas(16) SlotG {
@@ -166,7 +167,7 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
     //  run the same loads and the waits count the same; the decay itself is read once, below)
     const char* __restrict__ pB = reinterpret_cast<const char*>(lower ? (HD ? static_cast<const uint16_t*>(a.w) + h * N : static_cast<const uint16_t*>(a.w) + base) : a.v + base);   // w | v
     // LOCAL: a gradient state takes no k and no v (as in wkv6_fwd_f.hip: one row of them that hits the cache, and no K').  B1 T3001 C2048:
-    // 27.1 -> 22.9 us.
+    // 27.1 -> 22.9 us, 19.3 with two iterations past the last chunk instead of up to eight.
     const uint32_t amask = (LOCAL && !lower) ? 127u : ~0u, bmask = (lower ? HD : LOCAL) ? 127u : ~0u;
     const char* __restrict__ pC = reinterpret_cast<const char*>(a.gy + base);
     const uint32_t row_b = 2u * static_cast<uint32_t>(a.C);                                     // bytes from a token to the next
@@ -372,8 +373,10 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
     __builtin_amdgcn_sched_barrier(0);
     // DEPTH iterations per trip, no stage with loads or ring registers skipped: a way round one, or round the second half,
     // would be one more way into the next wait, on which the registers it waits for are the newest loads (the count then
-    // covers everything).  Below chunk 0 the stages run on rows that all count as dead, into the planes of a slot that
-    // nobody reads any more (c < 0: the slot of chunk c + 3, whose products were done in the iteration before).
+    // covers everything).  Below chunk 0 the rows that are staged all count as dead, in the planes of a slot that nobody reads any
+    // more (c < 0: the slot of chunk c + 3, whose products were done in the iteration before), and nothing is prepared (which neither
+    // loads nor touches the ring).
+    constexpr int TRIP = trip<LOCAL>;
     for (int it0 = 0; it0 < nit; it0 += TRIP)
         static_for<TRIP>([&](auto Z) {
             constexpr int z = decltype(Z)::value % DEPTH, zk = decltype(Z)::value % KEPT;
@@ -398,7 +401,7 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
             }
             __builtin_amdgcn_sched_barrier(0);
             met_ok = meet_wait(&S.met[0], 8u * (it + 1)) && met_ok;        // all rows of chunk cp are staged
-            if ((cut && it == 0) || cp < 0) prep(cp, hq[zk], part); else prep(cp, hq[zk], full);
+            if (cut && it == 0) prep(cp, hq[zk], part); else if (cp >= 0) prep(cp, hq[zk], full);
             __syncthreads();
         });
     // (a meeting that never completed, which the counting excludes, would leave this head to the two-sweep kernels)
@@ -869,7 +872,7 @@ __global__ __launch_bounds__(NTG) void wkv6_bwd_fused(const ArgsG arg) {
     if (tid < 4) S.met[tid] = 0;
     __syncthreads();
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, w = wid & 3;
-    const int nit = (n + 3 + TRIP - 1) / TRIP * TRIP;      // iterations of the pipeline: n + 3, in whole trips of the prep loop
+    const int nit = (n + (LOCAL ? 2 : 3) + trip<LOCAL> - 1) / trip<LOCAL> * trip<LOCAL>;      // iterations of the pipeline: n + 3 (nothing to finish: n + 2), in whole trips of the prep loop
     if (wid < 8) role_prep<WMODE, LOCAL>(S, a, lane, wid, base, h, bh, n, nit);
     else if (wid < 12) role_sd<WMODE, LOCAL>(S, a, lane, w, bh, n, nit);
     else {

@@ -94,7 +94,7 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
     const char* __restrict__ pB = reinterpret_cast<const char*>(lower ? (HD ? a.w + h * N : a.w + base) : a.v + base);   // w | v
     const uint32_t bmask = (HD && lower) ? 127u : ~0u;
     // LOCAL: a state takes no r.  Its rows are not read (the loads stay, of one row that hits the cache, for the same reason), R' is not made
-    // and neither is the diagonal of A.  B1 T3001 C2048: 24.5 -> 20.8 us with the reads and this arithmetic left out.
+    // and neither is the diagonal of A.  B1 T3001 C2048: 24.5 -> 20.8 us, 18.9 with nothing prepared past the end.
     const uint32_t amask = (LOCAL && lower) ? 127u : ~0u;
     const uint32_t row_b = 2u * static_cast<uint32_t>(a.C);                                     // bytes from a token to the next
     uint32_t offA = (8 * (w & 3) + (lane >> 3)) * row_b + 16 * (lane & 7);                      // rows 8 (w & 3) .. +7
@@ -251,7 +251,8 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
     __builtin_amdgcn_sched_barrier(0);
     // DEPTH iterations per trip, nothing in them skipped: a way round a stage, or round the second half, would be one more
     // way into the next wait, on which the registers it waits for are the newest loads (the count then covers everything).
-    // Past the last chunk the stages run on rows that all count as dead, into a slot nobody reads.
+    // Past the last chunk the rows that are staged all count as dead, in a slot nobody reads, and nothing is prepared (which neither loads
+    // nor touches the ring).
     for (int it0 = 0; it0 < nit; it0 += DEPTH)
         static_for<DEPTH>([&](auto Z) {
             constexpr int z = decltype(Z)::value;
@@ -265,7 +266,7 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
             if constexpr (!LOCAL) store_y(it >= 3 ? it - 3 : 0, it >= 3);
             __builtin_amdgcn_sched_barrier(0);
             met_ok = meet_wait(&S.met[0], 8u * (it + 1)) && met_ok;      // all eight waves have staged their rows of chunk it
-            if (it >= n - 1) prep(it, part); else prep(it, full);
+            if (it < n - 1) prep(it, full); else if (it < n) prep(it, part);
             __syncthreads();
         });
     // (a meeting that never completed, which the counting excludes, would leave the results of this head to the other kernel)
@@ -545,7 +546,7 @@ __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
     if (tid == 0) S.met[0] = 0;
     __syncthreads();
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, w = wid & 3;
-    const int nit = (n + 2 + DEPTH) & ~(DEPTH - 1);        // iterations of the pipeline: n + 3, in whole trips of the prep loop
+    const int nit = (n + (LOCAL ? 1 : 2) + DEPTH) & ~(DEPTH - 1);        // iterations of the pipeline: n + 3 (no y to store: n + 2), in whole trips of the prep loop
     if (wid < 8) role_prep<LOCAL, HD>(S, a, lane, wid, base, h, bh, n, nit);
     else if (wid < 12) role_state<LOCAL>(S, a, lane, w, bh, n, nit);
     else role_tiles<LOCAL>(S, a, lane, w, bh, n, nit);
