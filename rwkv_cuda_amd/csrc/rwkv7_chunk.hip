@@ -1,4 +1,4 @@
-// RWKV-7 "clamp-w" generalised delta rule in CHUNKED form on the matrix cores (gfx950, v_mfma_f32_16x16x4_f32).
+// RWKV-7 "clamp-w" generalised delta rule in CHUNKED form on the matrix cores (gfx950).
 //
 // Step form (rwkv7_fast_fused/cuda/rwkv7_statepassing_clampw.cu:20-187), one head, S[i][j] (i value, j key):
 //     sa_t = S_t a_t;   S_{t+1} = S_t diag(w_t) + sa_t b_t^T + v_t k_t^T;   y_t = S_{t+1} r_t;   w_t = exp(W_SCALE sigmoid(w_raw_t))
