@@ -260,8 +260,9 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
             be[e] = bb[e] * f.ee[e];
         }
         const lds_t o = sb + piece(lane, q);
-        put3(o + F_AS, split3(as)); put3(o + F_RS, split3(rs));
-        put_pair<TERM2>(sb + F_KB + slot * PAIR3 + piece2(lane, q), split3(ke), split3(be));
+        // (no factor is above 1: what comes from bf16 inputs stays within bf16's range)
+        put3(o + F_AS, split3<!F32>(as)); put3(o + F_RS, split3<!F32>(rs));
+        put_pair<TERM2>(sb + F_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(ke), split3<!F32>(be));
         if constexpr (F32) put3(o + F_V, split3(f32x4{vv[0], vv[1], vv[2], vv[3]}));
         else lds_st<u32x2>(o + F_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
         if (q == 0) S.dec[slot][lane] = exp_acc(cl);
@@ -566,8 +567,9 @@ template <bool F32> DEVINL void bwd_planes3(const lds_t sb, const lds_t slot, co
         kd[e] = in(1, e) * f.ee[e];
     }
     const lds_t o = sb + O::ONE + piece(lane, wp);
-    put_pair<TERM2>(sb + O::TWO + slot + O::RA + piece2(lane, wp), split3(rs), split3(as));
-    put3(o + O::BD, split3(bd)); put3(o + O::KD, split3(kd));
+    // (no factor is above 1: what comes from bf16 inputs stays within bf16's range)
+    put_pair<TERM2>(sb + O::TWO + slot + O::RA + piece2(lane, wp), split3<!F32>(rs), split3<!F32>(as));
+    put3(o + O::BD, split3<!F32>(bd)); put3(o + O::KD, split3<!F32>(kd));
 }
 // U, v and dy, which no factor enters
 template <bool F32> DEVINL void bwd_planes_raw(const lds_t sb, const lds_t slot, const Conv7<F32>& y, int wp, int lane) {

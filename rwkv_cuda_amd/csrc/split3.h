@@ -1,13 +1,14 @@
 // fp32 products on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16): an fp32 value as three bf16 terms, x = h + m + l (rounded to
-// nearest, every remainder exact: all 24 bits), a product as the six that count, hh + hm + mh + mm + hl + lh; those left out are
-// below 2^-26 of it.  Accumulation is fp32 either way.
+// nearest, every remainder exact), a product as the six that count, hh + hm + mh + mm + hl + lh; those left out are at most 2^-24 of it,
+// 2^-27 in the root mean square.  Accumulation is fp32 either way.  All 24 bits from 2^-110 up to the largest fp32; what is smaller
+// is kept to 2^-134 (the last term falls among bf16's subnormals).
 //
 // Why not v_mfma_f32_16x16x4_f32: it holds the vector unit.  Per SIMD, one wave issuing matrix and another vector instructions, cycles
 // for 16 matrix and 64 vector ones: fp32 573 and 329 alone, 882 together; bf16 292 and 308 alone, 478 together.  16 tokens of a
 // contraction are four fp32 instructions (143 cycles, none left for anything else) or three of these (55, of which the vector unit
 // loses 30); splitting costs 5.5 vector instructions an element, once for all products that it enters.
 //
-// An infinite element has remainders that are no numbers: what it enters is NaN, where fp32 instructions would give an infinity or NaN.
+// An infinity has a remainder that is no number: what it enters is NaN, where fp32 instructions would give an infinity or NaN.
 #pragma once
 #include "common.h"
 
@@ -38,14 +39,24 @@ DEVINL uint32_t round2(float a, float b) {
     asm("" : "+v"(r));
     return r;
 }
-// four values, three terms
+// The pair with an infinity replaced by the largest bf16 of its sign, in all of 16-bit integers: what is beyond 0x7f7f on the positive
+// side, on the negative one what is beyond 0xff7f as unsigned numbers.  (Two instructions a pair; the values held to that bound before
+// they are rounded cost the backward registers: fp32 mode 904 us, this 817, nothing of the kind 796, which gave NaN for a finite
+// input at B8 T1024 C4096; bf16 641, 623, 601.  A wave that looks for such values first and branches: 842 and 624.)
+DEVINL uint32_t finite2(uint32_t r) {
+    asm("v_pk_min_i16 %0, %0, %1\n\tv_pk_min_u16 %0, %0, %2" : "+v"(r) : "s"(0x7f7f7f7fu), "s"(0xff7fff7fu));
+    return r;
+}
+// four values, three terms.  A value beyond the largest bf16, (2 - 2^-7) 2^127, would round to an infinity, and its remainders were no
+// numbers: its first term is that largest one and the others take the rest (below 2^120, so still exact).  BOUNDED: there is none.
 struct B3 { u32x2 h, m, l; };
-DEVINL B3 split3(const f32x4& x) {
+template <bool BOUNDED = false> DEVINL B3 split3(const f32x4& x) {
     B3 o;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         float a = x[2 * i], b = x[2 * i + 1];
-        o.h[i] = round2(a, b);
+        if constexpr (BOUNDED) o.h[i] = round2(a, b);
+        else o.h[i] = finite2(round2(a, b));
         a -= bf_lo(o.h[i]); b -= bf_hi(o.h[i]);
         o.m[i] = round2(a, b);
         a -= bf_lo(o.m[i]); b -= bf_hi(o.m[i]);

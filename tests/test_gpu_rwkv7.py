@@ -275,3 +275,33 @@ def test_fp32_state_keeps_24_bits(T, f32, shift):
     rel = lambda p, q: ((p.double().cpu().reshape(q.shape) - q).norm() / q.norm()).item()
     assert rel(sT, S) <= 2e-7
     assert rel(y, torch.stack(ys, 1)) <= (4e-7 if f32 else 2.0 ** -8)
+
+
+FLT_MAX = torch.finfo(torch.float32).max
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("f32,name,t", [(False, "s0", 3), (False, "dsT", 3), (True, "s0", 3), (True, "dsT", 3), (True, "r", 23), (True, "k", 23), (True, "v", 16),
+                                        (True, "v", 31), (True, "b", 23), (True, "dy", 16), (True, "dy", 31)])
+def test_finite_values_beyond_the_largest_bf16(f32, name, t, sign):
+    """The largest fp32 value as one element of an input (s0 and dsT are fp32 in either mode): results are finite where the step form's
+    are in fp32, and as accurate as without it.  Bound of an fp32 result: one element carries the norm, so its roundings do not average out;
+    32 of them at 2^-24 (decays over 48 steps, sums and splits).  A bf16 result: its own rounding."""
+    B, T, H, N = 1, 48, 1, 64
+    s0, r, w, k, v, a, b, dy, dsT = synth.rwkv7_inputs(B, T, H, N, seed=7)
+    x = dict(s0=s0, r=r, w=w, k=k, v=v, a=a, b=b, dy=dy, dsT=dsT)
+    dt = torch.float32 if f32 else torch.bfloat16
+    x = {n: (z if n == "w" else z * 2.0 ** -9).to(z.dtype if n in ("s0", "dsT") else dt) for n, z in x.items()}          # no product overflows
+    if name in ("s0", "dsT"):
+        x[name][0, 0, t, 5] = sign * FLT_MAX
+    else:
+        x[name][0, t, 0, 5] = sign * FLT_MAX
+    args = [x[n] for n in ("s0", "r", "w", "k", "v", "a", "b", "dy", "dsT")]
+    ref = O.grads(*args)
+    assert all(float(z.abs().max()) < FLT_MAX * 1.0001 for z in ref)
+    got = _run(args)
+    for n, want, g in zip(NAMES, ref, got):
+        assert bool(g.isfinite().all()), n
+        e = ((g.double().cpu() - want).norm() / want.norm()).item()
+        print(f"  {n}: {e:.2e}", flush=True)
+        assert e <= (2.0 ** -19 if g.dtype == torch.float32 else 2.0 ** -8), (n, e)

@@ -1,0 +1,79 @@
+"""CPU: the split products of the chunked rwkv7 kernels (csrc/split3.h), restated in numpy.
+
+An fp32 operand is three bf16 terms, x = h + m + l, each the nearest bf16 of the exact remainder, the first one never an
+infinity; a product is the six of the nine that count.  Checked here: over which range the three terms hold all 24 bits, what
+happens at its ends, and what the three products left out are worth."""
+import numpy as np
+import pytest
+
+FLT_MAX, BF_MAX = np.finfo(np.float32).max, np.float32((2 - 2.0 ** -7) * 2.0 ** 127)
+
+
+def to_bf16(x):
+    """Nearest bf16, ties to even, as fp32."""
+    u = x.astype(np.float32).view(np.uint32).astype(np.uint64)
+    return (((u + 0x7fff + ((u >> 16) & 1)) & 0xffff0000).astype(np.uint32)).view(np.float32)
+
+
+def finite(h):
+    """finite2 of split3.h: the same minima over 16-bit integers."""
+    b = (h.view(np.uint32) >> 16).astype(np.uint16)
+    b = np.minimum(b.view(np.int16), np.int16(0x7f7f)).view(np.uint16)
+    b = np.minimum(b, np.uint16(0xff7f))
+    return (b.astype(np.uint32) << 16).view(np.float32)
+
+
+def split3(x):
+    x = np.asarray(x, np.float32)
+    h = finite(to_bf16(x))
+    r = x - h
+    m = to_bf16(r)
+    return h, m, to_bf16(r - m)
+
+
+def values(lo, hi, n=200000, seed=0):
+    """Magnitudes spread over the logarithm, random significands and signs."""
+    rng = np.random.default_rng(seed)
+    x = np.ldexp(rng.uniform(1, 2, n), rng.integers(lo, hi, n)).astype(np.float32)
+    return x * rng.choice(np.float32([-1, 1]), n)
+
+
+def test_three_terms_hold_all_24_bits():
+    x = values(-110, 128)
+    x = np.concatenate([x, np.float32([FLT_MAX, -FLT_MAX, BF_MAX, -BF_MAX, 2.0 ** -110, 0.0])])
+    edge = np.arange(0x7f7f0000, 0x7f800000, dtype=np.uint32).view(np.float32)          # around and beyond the largest bf16
+    for v in (x, edge, -edge):
+        h, m, l = split3(v)
+        assert np.all(np.isfinite(h)) and np.all(np.isfinite(m)) and np.all(np.isfinite(l))
+        assert np.array_equal(h.astype(np.float64) + m + l, v.astype(np.float64))
+
+
+def test_the_first_term_is_the_nearest_bf16_up_to_the_largest():
+    x = values(-126, 128)
+    x = x[np.abs(x) <= BF_MAX]
+    assert np.array_equal(split3(x)[0], to_bf16(x))
+    assert np.array_equal(split3(np.float32([FLT_MAX, -FLT_MAX]))[0], np.float32([BF_MAX, -BF_MAX]))
+
+
+def test_smaller_values_lose_bits_to_the_spacing_of_bf16_subnormals():
+    x = values(-126, -110)
+    h, m, l = split3(x)
+    err = np.abs(h.astype(np.float64) + m + l - x.astype(np.float64))
+    assert err.max() <= 2.0 ** -134 and err.max() > 0          # half of 2^-133
+
+
+@pytest.mark.parametrize("v", [np.inf, -np.inf, np.nan])
+def test_an_infinity_or_nan_is_not_finite_in_its_remainders(v):
+    with np.errstate(invalid="ignore"):
+        h, m, l = split3(np.float32([v]))
+        assert np.isnan((h.astype(np.float64) + m + l)[0])
+
+
+def test_products_left_out():
+    """m l' + l m' + l l' against the whole product: at most 2^-24, 2^-27 in the root mean square."""
+    x, y = values(-1, 1, seed=1), values(-1, 1, seed=2)
+    (h, m, l), (p, q, s) = ([t.astype(np.float64) for t in split3(v)] for v in (x, y))
+    exact = x.astype(np.float64) * y
+    six = h * p + h * q + m * p + m * q + h * s + l * p
+    rel = np.abs(six - exact) / np.abs(exact)
+    assert rel.max() <= 2.0 ** -24 and np.sqrt((rel ** 2).mean()) <= 2.0 ** -27
