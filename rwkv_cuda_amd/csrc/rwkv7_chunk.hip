@@ -162,12 +162,12 @@ DEVINL Factors chunk_factors(const float (&lam)[4], const float (*part)[N], int 
 }
 
 // (a Newton step behind the hardware reciprocal instead of a full division, a sixth of the vector instructions that turn inputs into
-// planes; the exponent stops short of overflow, where the step would make a NaN, and a NaN passes)
+// planes.  A quarter of the denominator, since the reciprocal flushes what is below 2^-126; an overflown exponential leaves zero, and
+// so no decay gradient, where the step by itself would make a NaN; a NaN passes by y)
 DEVINL float sigmoid_fast(float x) {
-    const float t = x * -1.44269504088896340736f;
-    const float d = 1.f + __builtin_amdgcn_exp2f(t > 126.f ? 126.f : t);
+    const float d = fmaf(__builtin_amdgcn_exp2f(x * -1.44269504088896340736f), 0.25f, 0.25f);
     const float y = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, y, 1.f), y, y);
+    return 0.25f * fmaf(fmaf(-fminf(d, 3.40282346638528859812e38f), y, 1.f), y, y);
 }
 
 // tile[t][s] = sum_c X[t][c] Y[s][c] over 64 channels, masked to s < t (strict) or s <= t: register v <-> t = 4 g + v, lane <-> s, or

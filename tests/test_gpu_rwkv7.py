@@ -305,3 +305,28 @@ def test_finite_values_beyond_the_largest_bf16(f32, name, t, sign):
         e = ((g.double().cpu() - want).norm() / want.norm()).item()
         print(f"  {n}: {e:.2e}", flush=True)
         assert e <= (2.0 ** -19 if g.dtype == torch.float32 else 2.0 ** -8), (n, e)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_no_decay_has_no_decay_gradient(lib, dtype):
+    """w = -inf, or so low that e^-w overflows: sigmoid(w) is zero, the step keeps the state, and dw is zero and not merely small; where
+    sigmoid(w) is subnormal (spacing 2^-149, so 2^-22 of 4e-39) dw is still right."""
+    B, T, H, N = 1, 32, 2, 64
+    s0, r, w, k, v, a, b, dy, dsT = synth.rwkv7_inputs(B, T, H, N, seed=8)
+    w[:, 3, :, 7], w[:, 16, :, 8], w[:, 31, :, 9] = -math.inf, -120.0, -3e38
+    w[:, 7], w[:, 20] = -88.5, -87.5          # (bf16 holds both)
+    off = w < -100
+    args = [s0, *(x.to(dtype) for x in (r, w, k, v, a, b, dy)), dsT]
+    got = _run(args)
+    assert float(got[NAMES.index("dw")].cpu()[off].abs().max()) == 0.0
+    ref = O.grads(*args)
+    dw, want = got[NAMES.index("dw")].double().cpu(), ref[NAMES.index("dw")]
+    rel, spacing = (2e-5, 2.0 ** -149) if dtype == torch.float32 else (2.0 ** -8, 2.0 ** -133)        # (of subnormal results)
+    for t in (7, 20):
+        assert float((dw[:, t] - want[:, t]).norm()) <= rel * float(want[:, t].norm()) + spacing * math.sqrt(want[:, t].numel()), t
+    emu = O.emulate_bf16(*args) if dtype == torch.bfloat16 else O.backward_hand(*args, dtype=torch.float32)
+    for name, x, e, g in zip(NAMES, ref, emu, got):
+        if dtype == torch.bfloat16:
+            assert_no_worse(name, x, e, g)
+        else:
+            assert_fp32_mode(name, x, e, g)
