@@ -7,6 +7,7 @@ import torch
 from oracle import rwkv7 as O
 from oracle import err_ratio
 from rwkv_cuda_amd import options, synth, rwkv7_fast_fused as R
+from rwkv_cuda_amd._call import call
 from _gpu_util import DEV, assert_no_worse
 
 pytestmark = pytest.mark.gpu
@@ -251,30 +252,46 @@ def test_fp32_sweeps_option_runs_the_step_kernels(lib, B, T, H):
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("T", [16, 32, 48, 112])
 @pytest.mark.parametrize("shift", [-6.0, 0.5, 6.0])
-def test_fp32_state_keeps_24_bits(T, f32, shift):
-    """One, two, three and seven chunks, slow to strong decays: the fp32 state against the step form in 64 bits.  Bound: a factor of the
-    last chunk carries about 1e-7 (an exponential's last bit and a product's rounding), a sum of 16 terms and of two products as much."""
+@pytest.mark.parametrize("end", [False, True])
+def test_fp32_results_keep_24_bits(lib, T, f32, shift, end):
+    """One, two, three and seven chunks, slow to strong decays, with and without a gradient of the final state: every fp32 result (y and
+    the gradients are fp32 in the fp32 mode alone) against the step form in 64 bits.  Bound: each factor, sum and product of a chunk
+    leaves about half a unit in the last place, 2^-24, four to eight of them in a result: 4e-7.  (Products without their second-order
+    terms, m m', h l', l h', would leave 4.5e-6.)  dw = G sig (1 - sig): G is a difference that is carried through the call, 3e-7 a
+    chunk at most, adding up as a random walk; 1 - sig is rounded at 2^-25 and about e^-w."""
     B, H, N = 2, 3, 64
     g = torch.Generator().manual_seed(T)
     n = lambda *s: torch.randn(*s, generator=g)
     kk = torch.nn.functional.normalize(n(B, T, H, N), dim=-1)
-    s0 = n(B, H, N, N) * 0.1
-    x = [n(B, T, H, N) * 0.5, n(B, T, H, N) + shift, n(B, T, H, N) * 0.5, n(B, T, H, N) * 0.5, -kk, kk * torch.sigmoid(n(B, T, H, N))]
+    s0, dsT = n(B, H, N, N) * 0.1, n(B, H, N, N) * 0.1
+    x = [n(B, T, H, N) * 0.5, n(B, T, H, N) + shift, n(B, T, H, N) * 0.5, n(B, T, H, N) * 0.5, -kk, kk * torch.sigmoid(n(B, T, H, N)), n(B, T, H, N)]
     x = [t.to(torch.float32 if f32 else torch.bfloat16) for t in x]
-    r, w, k, v, a, b = (t.double() for t in x)
-    S = s0.double()
+    S, r, w, k, v, a, b = p = [t.double().requires_grad_(True) for t in (s0, *x[:6])]
     d = torch.exp(-math.exp(-0.5) * torch.sigmoid(w))
-    ys = []
+    ys, sas = [], []
     for t in range(T):
-        sa = S @ a[:, t, :, :, None]
-        S = S * d[:, t, :, None, :] + sa * b[:, t, :, None, :] + v[:, t, :, :, None] * k[:, t, :, None, :]
-        ys.append((S @ r[:, t, :, :, None])[..., 0])
-    dev = [t.cuda().view(B, T, H * N) for t in x]
-    with torch.no_grad():
-        y, sT = R.RWKV7_STATE_PASSING_CLAMPW_CUDA(s0.cuda(), *dev)
-    rel = lambda p, q: ((p.double().cpu().reshape(q.shape) - q).norm() / q.norm()).item()
-    assert rel(sT, S) <= 2e-7
-    assert rel(y, torch.stack(ys, 1)) <= (4e-7 if f32 else 2.0 ** -8)
+        sas.append((S * a[:, t, :, None, :]).sum(-1))
+        S = S * d[:, t, :, None, :] + sas[-1][..., None] * b[:, t, :, None, :] + v[:, t, :, :, None] * k[:, t, :, None, :]
+        ys.append((S * r[:, t, :, None, :]).sum(-1))
+    y = torch.stack(ys, 1)
+    grads = torch.autograd.grad([y, S] if end else [y], p, [x[6].double(), dsT.double()] if end else [x[6].double()])
+    want = dict(zip(("y", "sT", "sa", "ds0", "dr", "dw", "dk", "dv", "da", "db"), (y.detach(), S.detach(), torch.stack(sas, 1).detach(), *grads)))
+    dev = [t.to(DEV) for t in (s0, *x)]
+    new = lambda *s: torch.full(s, math.nan, device=DEV)
+    like = lambda: torch.full_like(dev[1], math.nan)
+    got = dict(y=like(), sT=new(B, H, N, N), s=new(B, H, T // 16, N, N), sa=new(B, T, H, N), ds0=new(B, H, N, N), **{z: like() for z in ("dr", "dw", "dk", "dv", "da", "db")})
+    sfx = "_f32" if f32 else ""
+    call(f"rwkv7_statepassing_forward{sfx}_ex", DEV, B, T, H, *dev[:7], got["y"], got["sT"], got["s"], got["sa"], 0)
+    call(f"rwkv7_statepassing_backward{sfx}_ex", DEV, B, T, H, *dev[1:], dsT.to(DEV) if end else None, got["s"], got["sa"],
+         *(got[z] for z in ("ds0", "dr", "dw", "dk", "dv", "da", "db")), 0)
+    with torch.no_grad():                                   # the forward that keeps nothing: the same bits
+        y1, sT1 = R.RWKV7_STATE_PASSING_CLAMPW_CUDA(dev[0], *(t.view(B, T, H * N) for t in dev[1:7]))
+    assert torch.equal(y1.view_as(got["y"]), got["y"]) and torch.equal(sT1, got["sT"])
+    for z, q in want.items():
+        e = ((got[z].double().cpu() - q).norm() / q.norm()).item()
+        print(f"  {z}: {e:.2e}", flush=True)
+        dw = 3e-7 * max(1.0, T / 16) ** 0.5 * 2 + 2.0 ** -25 * math.exp(shift + 1)
+        assert e <= (2.0 ** -8 if got[z].dtype == torch.bfloat16 else dw if z == "dw" else 4e-7), (z, e)
 
 
 FLT_MAX = torch.finfo(torch.float32).max
