@@ -69,7 +69,9 @@ int rwkv_hbm_probe(void* stream, int mode, const void* src, void* dst, size_t by
  * Inputs that are not finite.  The bf16 chunked kernels (wkv5, wkv6, wkv6_state) and the chunked rwkv7 kernels, fp32 mode
  * included, multiply what a causal tile leaves out by zero: a NaN or an infinity in an input reaches, besides all that it acts
  * on, outputs of the tokens before it (and gradients of those after it) within its chunk of 16 (rwkv7) or 32 tokens of its
- * head; so do the two-term fp16 kernels of depthwise_conv1d, within 32 steps of a unit of 32 batch rows of a channel.  The
+ * head; so do the two-term fp16 kernels of depthwise_conv1d, within 32 steps of a unit of 32 batch rows of a channel.  What the
+ * chunked rwkv7 kernels make of an infinity is NaN in most places where the recurrence has an infinity (a product takes an fp32
+ * value as three bf16 terms, and an infinity has no finite remainder); finite values up to the largest fp32 act as they are.  The
  * sequential kernels, those of fp32 wkv5 and wkv5a, and the three-term kernels of depthwise_conv1d keep it to where it acts.
  *
  *   RWKV_PASS_*      : restrict a backward to a subset of its kernels so that a profiler can time one kernel per call

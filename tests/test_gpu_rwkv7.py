@@ -347,3 +347,32 @@ def test_no_decay_has_no_decay_gradient(lib, dtype):
             assert_no_worse(name, x, e, g)
         else:
             assert_fp32_mode(name, x, e, g)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("name", ["r", "k", "v", "a", "b", "s0"])
+@pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
+def test_where_an_infinity_reaches(lib, dtype, name, value):
+    """One infinity or NaN among the inputs: what is not finite in the step form is not finite here (NaN where that has an infinity, as the
+    header says), nothing before its chunk is touched, and neither are other heads and batch rows, gradients included."""
+    B, T, H, N = 2, 48, 2, 64
+    s0, r, w, k, v, a, b, dy, dsT = synth.rwkv7_inputs(B, T, H, N, seed=9)
+    x = dict(s0=s0, r=r, w=w, k=k, v=v, a=a, b=b, dy=dy, dsT=dsT)
+    x = {n: z.to(torch.float32 if n in ("s0", "dsT") else dtype) for n, z in x.items()}
+    clean = _run(list(x.values()))
+    x[name] = x[name].clone()
+    if name == "s0":
+        x[name][0, 0, 3, 5] = value
+    else:
+        x[name][0, 23, 0, 5] = value
+    got = _run(list(x.values()))
+    step = O.recurrent(*(x[n].double() for n in ("s0", "r", "w", "k", "v", "a", "b")))
+    for want, g in zip(step, got):
+        assert not bool((~want.isfinite() & g.cpu().isfinite()).any())
+    assert not bool(got[0][0, 23, 0].isfinite().all())
+    if name != "s0":
+        assert torch.equal(got[0][:, :16], clean[0][:, :16])
+    for n, c, g in zip(NAMES, clean, got):
+        per_head = (lambda z: z) if n in ("sT", "ds0") else (lambda z: z.transpose(1, 2))         # [B, H, ...]
+        c, g = per_head(c), per_head(g)
+        assert torch.equal(c[1], g[1]) and torch.equal(c[0, 1], g[0, 1]), n
