@@ -26,8 +26,10 @@
 //            dw_raw = G W_SCALE sig (1 - sig);  P at the end of the call = sum_i dsT o S_T.
 // Every product takes all 24 bits of its operands, so the fp32 outputs sT, ds0 and the saved sa keep the accuracy class of the
 // reference's fp32 recurrence; the bf16 outputs are rounded once at the store.  The fp32 mode is therefore the same kernel with fp32
-// loads and stores.  Products are split ones (split3.h) but for the tiles from A', R', B', K', which are fp32 matrix instructions:
-// their operands enter one product each, and splitting those costs what the instructions cost.
+// loads and stores.  Products are split ones (split3.h) but for the tiles AB, AK, RB, RK in both directions, which are fp32 matrix
+// instructions, 16 a wave and chunk.  Each of A', R', B', K' enters two of them.  Split operands were not built: the wave that makes a
+// tile would split both of its sides, 176 vector instructions beside 12 matrix ones, or read them from LDS split, and the backward,
+// whose B waves split those planes for products of their own, has 1 KB of LDS left where two copies of them take 14 KB more.
 //
 // One workgroup per (batch, head).  A 16x16x4 fp32 matrix instruction takes A[row = lane & 15][k = lane >> 4],
 // B[k = lane >> 4][col = lane & 15] and leaves D[row = 4 (lane >> 4) + v][col = lane & 15] in register v.  The state is
@@ -375,9 +377,9 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
 // KEEP: `s` and `sa` are written for a backward, 20 bytes per element beside the 14 of a bf16 forward's inputs and output.
 // What bounds it: issue.  B8 T1024 C4096, one call: 398 us with every product on the fp32 matrix instructions, in four waves that did
 // everything in turn between four barriers; 390 in two roles of four waves; 335 with split products, since the fp32 instructions
-// (96 a wave and chunk) held the vector unit for half of the time.  Vector instructions are now most of it, two thirds of them in the
-// P waves.  fp32 mode 396 -> 360.  Errors against 64 bits, T256, before -> now: y 1.8 -> 1.4e-7, sT 6.9 -> 6.0e-8 (slow decays
-// 1.5e-7 -> 9e-8).
+// (96 a wave and chunk) held the vector unit for half of the time.  The first of these forms and this one in alternation on one
+// machine: bf16 391 -> 327 us, fp32 mode 396 -> 379.  Vector instructions now issue 67 % of a SIMD's time, matrix ones about a third.
+// Errors against 64 bits, T16 to T1024, slow to strong decays, largest, before -> now: y 2.4 -> 1.7e-7, sT 1.6 -> 1.0e-7, sa 2.3 -> 1.7e-7.
 template <bool F32, bool KEEP>
 __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c p) {
     extern __shared__ __align__(32) unsigned char smem_raw[];
@@ -405,10 +407,14 @@ __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c p) {
 //                (double-buffered).  The finished gradient rows leave LDS-staged, as whole rows, through A waves 2 and 3.
 // The gradient state is therefore kept twice (both copies get the same update).
 // What bounds it: issue, and waits for LDS and at barriers.  B8 T1024 C4096, one call: 762 us with fp32 matrix instructions (962 a
-// chunk, 57 % of a SIMD's time in which it could issue no vector instruction), 676 with split products (fp32 mode 811 -> 844 in a
-// trace of few calls, 797 -> 770 among others: its 24 rows a chunk leave from registers, 64 bytes at a time).  Of that, causal tiles
-// and the inverse moved from phase 1, where everybody waited for wave 0, into the phase 3 before: 727 -> 676.  Errors against 64 bits,
-// T256, before -> now: ds0 1.55e-7 -> 8e-8, dr 1.5 -> 1.1e-7, dk 1.6 -> 1.2e-7, dv 1.5 -> 1.4e-7, da 2.3 -> 1.9e-7, db 2.4 -> 1.8e-7.
+// chunk, 57 % of a SIMD's time in which it could issue no vector instruction), 676 with split products.  Of that, causal tiles
+// and the inverse moved from phase 1, where everybody waited for wave 0, into the phase 3 before: 727 -> 676.  Both forms in alternation
+// on one machine: bf16 714 -> 636 us, vector instructions issuing 62 % of a SIMD's time.  The fp32 mode gained nothing, 796 -> 829 (and
+// 797 -> 805 on another): its 24 rows a chunk leave from registers, 64 bytes at a time, and it splits v and dy as well; forward and
+// backward together 1188 -> 1188 there, 1190 -> 1165 on the other.
+// Errors against 64 bits, T16 to T1024, slow to strong decays, largest, before -> now: ds0 1.8 -> 1.0e-7, dr 1.9 -> 1.3e-7, dk 2.1 ->
+// 1.3e-7, dv 2.2 -> 1.7e-7, da 3.0 -> 2.2e-7, db 3.2 -> 2.1e-7; dw 3.2 -> 2.4e-6 at T1024 and usual decays, 7.3 -> 6.9e-6 at decays near
+// e^-0.6, where 1 - sig has few digits.
 constexpr int NTB = 12 * 64;       // waves 0..3 role A, 4..7 role B, 8..11 role P
 
 // Everything that is a function of one chunk's inputs alone; two copies (but for the planes that only phase 1 reads): the P waves fill
@@ -427,7 +433,7 @@ struct SmemCB {
     PlanesB pl[2];
     float part[4][N];
     float AB[CL][TS];
-    uint16_t park[F32 ? 1 : 5][F32 ? 1 : CL][PK];                                // da, dr, db, dk, dw of the chunk whose phase 4 ran last, [token][channel]
+    uint16_t park[F32 ? 1 : 5][F32 ? 1 : CL][PK];                                // da, dr, db, dk, dw of the chunk that role B finished last, [token][channel]
     uint16_t parkv[F32 ? 1 : 2][F32 ? 1 : CL][PK];                               // dv, which is ready one visit earlier than the other five
 };
 // three-term planes and tiles behind it.  Two copies: r e^{c_{t+1}} and a e^{c_t} (RA, the state-gradient update), U, v and dy (one term
@@ -762,7 +768,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     auto planes_of = [&](int visit) __attribute__((always_inline)) { return static_cast<lds_t>((visit & 1) * sizeof(PlanesB)); };
     auto plane = [&](lds_t O, int k, int v) __attribute__((always_inline)) { return lds_ld<float>(fl + O + 4 * PS * (CL * k + v)); };
     auto chan = [&](lds_t O, int k) __attribute__((always_inline)) { return lds_ld<float>(cl + O + 4 * N * k); };
-    float Pj = 0.f;                                  // P at the end of the chunk whose phase 4 comes next
+    float Pj = 0.f;                                  // P at the end of the chunk that is finished next
     f32x4 xA = ZERO4, xB = ZERO4, xK = ZERO4, dRp = ZERO4;    // state parts of dA', dB', dK', and dR', carried into the next visit's phase 1
     Op3 bk;                                          // and B', K' as an operand
     // a contraction over 16 with a pair of tiles (one after the other: the registers do not hold the operands of all of them)

@@ -1,12 +1,13 @@
 // fp32 products on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16): an fp32 value as three bf16 terms, x = h + m + l (rounded to
 // nearest, every remainder exact), a product as the six that count, hh + hm + mh + mm + hl + lh; those left out are at most 2^-24 of it,
-// 2^-27 in the root mean square.  Accumulation is fp32 either way.  All 24 bits from 2^-110 up to the largest fp32; what is smaller
-// is kept to 2^-134 (the last term falls among bf16's subnormals).
+// 2^-27 in the root mean square.  Accumulation is fp32 either way.  All 24 bits from 2^-110 up to the largest fp32; what is smaller,
+// a value (its last term falls among bf16's subnormals) or a product, is kept to about 2^-134.
 //
 // Why not v_mfma_f32_16x16x4_f32: it holds the vector unit.  Per SIMD, one wave issuing matrix and another vector instructions, cycles
-// for 16 matrix and 64 vector ones: fp32 573 and 329 alone, 882 together; bf16 292 and 308 alone, 478 together.  16 tokens of a
-// contraction are four fp32 instructions (143 cycles, none left for anything else) or three of these (55, of which the vector unit
-// loses 30); splitting costs 5.5 vector instructions an element, once for all products that it enters.
+// for 16 matrix and 64 vector ones: fp32 573 and 329 alone, 882 together; bf16 292 and 308 alone, 478 together.  16 elements of a
+// contraction are four fp32 instructions (143 cycles, none left for anything else) or, two by two, three of these (55, of which the
+// vector unit loses 30); 16 alone take four, two where one side is exact in bf16.  Splitting costs 5.5 vector instructions an element,
+// 6.5 where infinite first terms have to be ruled out, once for all products that it enters.
 //
 // An infinity has a remainder that is no number: what it enters is NaN, where fp32 instructions would give an infinity or NaN.
 #pragma once
@@ -83,10 +84,8 @@ DEVINL void add32(Sum2& s, const Op3& a, const Op3& b) {
     s.lo = mmb(a.h, b.m, s.lo);
     s.hi = mmb(a.h, b.h, s.hi);
 }
-// one side, or both, exact in bf16
+// one side exact in bf16
 DEVINL void add32(Sum2& s, const bf16x8& a, const Op3& b) { s.lo = mmb(a, b.m, mmb(a, b.l, s.lo)); s.hi = mmb(a, b.h, s.hi); }
-DEVINL void add32(Sum2& s, const Op3& a, const bf16x8& b) { s.lo = mmb(a.m, b, mmb(a.l, b, s.lo)); s.hi = mmb(a.h, b, s.hi); }
-DEVINL void add32(Sum2& s, const bf16x8& a, const bf16x8& b) { s.hi = mmb(a, b, s.hi); }
 // Contraction over 16, four elements a lane on either side: the halves of an instruction's 32 slots take different terms.
 DEVINL void add16(Sum2& s, const B3& a, const B3& b) {
     const u32x2 z = {0u, 0u};
