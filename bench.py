@@ -51,8 +51,10 @@ TRAFFIC_MEASURED = {
     "wkv_sweep<gr+gu+gw, fp32 I/O>": 2148e6 + 537e6,
     "wkv_sweep<gr+gu+gw, two-sided>": 2148e6 + 537e6,
     # profiles/rwkv7_chunk_kernels_B8_T4096_C4096.md (four calls of T = 1024)
-    "rwkv7c_fwd x4 (T=1024 each)": 4 * (411.2e6 + 746.6e6),
-    "rwkv7c_bwd x4": 4 * (1149.7e6 + 411.0e6),
+    "rwkv7c_fwd x4 (T=1024 each)": 4 * (411.3e6 + 746.6e6),
+    "rwkv7c_bwd x4": 4 * (1150.3e6 + 411.6e6),
+    "rwkv7c_fwd<fp32> x4 (T=1024 each)": 4 * (814.4e6 + 813.7e6),
+    "rwkv7c_bwd<fp32> x4": 4 * (1638.1e6 + 822.6e6),
     # profiles/wkv5_split_kernels_B8_T4096_C4096_N128.md (both launches of a kernel and the sums that follow them)
     "wkv6_fwd_ws<head decay, split> x2": (805.7e6 + 536.9e6) + (1342.5e6 + 268.5e6),
     "wkv6_bwd_a_ws<head decay, split> x2": (1095.4e6 + 1334.3e6) + (1638.6e6 + 1065.4e6),
@@ -400,8 +402,9 @@ def make_rwkv7(dev, fp32=False):
         bwd()
 
     chunked = ALGO == "chunked"
-    kernels = [("rwkv7c_fwd x4 (T=1024 each)" if chunked else "rwkv7_fwd x4 (T=1024 each)", fwd, 7 * eb * C * tok),
-               ("rwkv7c_bwd x4" if chunked else "rwkv7_bwd x4", bwd, 13 * eb * C * tok)]
+    mode = "<fp32>" if fp32 else ""
+    kernels = [(f"rwkv7c_fwd{mode} x4 (T=1024 each)" if chunked else f"rwkv7_fwd{mode} x4 (T=1024 each)", fwd, 7 * eb * C * tok),
+               (f"rwkv7c_bwd{mode} x4" if chunked else f"rwkv7_bwd{mode} x4", bwd, 13 * eb * C * tok)]
 
     def cpu_baseline(t_cpu=64):
         from oracle import rwkv7 as O
