@@ -41,12 +41,16 @@ DEVINL uint32_t round2(float a, float b) {
     return r;
 }
 // The pair with an infinity replaced by the largest bf16 of its sign, in all of 16-bit integers: what is beyond 0x7f7f on the positive
-// side, on the negative one what is beyond 0xff7f as unsigned numbers.  (Two instructions a pair; the values held to that bound before
-// they are rounded cost the backward registers: fp32 mode 904 us, this 817, nothing of the kind 796, which gave NaN for a finite
-// input at B8 T1024 C4096; bf16 641, 623, 601.  A wave that looks for such values first and branches: 842 and 624.)
+// side, on the negative one what is beyond 0xff7f as unsigned numbers.  Two instructions a pair: B8 T1024 C4096, backward, fp32 mode
+// 802 -> 826 us, bf16 613 -> 638; forward 376 -> 382 and 319 -> 327.  (Values held to that bound before they are rounded cost the
+// backward registers: 796 -> 904 and 601 -> 641.  Looking for such values first and branching: 842 and 624.)  Not as inline assembly: a
+// matrix instruction has to stay two wait states behind a vector instruction that writes its operand, and the compiler, which sees
+// to that, does not look into assembly.
 DEVINL uint32_t finite2(uint32_t r) {
-    asm("v_pk_min_i16 %0, %0, %1\n\tv_pk_min_u16 %0, %0, %2" : "+v"(r) : "s"(0x7f7f7f7fu), "s"(0xff7fff7fu));
-    return r;
+    typedef short i16x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const i16x2 p = __builtin_elementwise_min(__builtin_bit_cast(i16x2, r), i16x2{0x7f7f, 0x7f7f});
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, p), u16x2{0xff7f, 0xff7f}));
 }
 // four values, three terms.  A value beyond the largest bf16, (2 - 2^-7) 2^127, would round to an infinity, and its remainders were no
 // numbers: its first term is that largest one and the others take the rest (below 2^120, so still exact).  BOUNDED: there is none.

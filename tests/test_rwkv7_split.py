@@ -3,9 +3,13 @@
 An fp32 operand is three bf16 terms, x = h + m + l, each the nearest bf16 of the exact remainder, the first one never an
 infinity; a product is the six of the nine that count.  Checked here: over which range the three terms hold all 24 bits, what
 happens at its ends, and what the three products left out are worth."""
+import os
+import re
+
 import numpy as np
 import pytest
 
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rwkv_cuda_amd", "csrc")
 FLT_MAX, BF_MAX = np.finfo(np.float32).max, np.float32((2 - 2.0 ** -7) * 2.0 ** 127)
 
 
@@ -77,3 +81,14 @@ def test_products_left_out():
     six = h * p + h * q + m * p + m * q + h * s + l * p
     rel = np.abs(six - exact) / np.abs(exact)
     assert rel.max() <= 2.0 ** -24 and np.sqrt((rel ** 2).mean()) <= 2.0 ** -27
+
+
+@pytest.mark.parametrize("name", ["split3.h", "rwkv7_chunk.hip"])
+def test_no_instruction_is_inline_assembly(name):
+    """Operands of matrix instructions are made here.  Such an instruction needs two wait states after the vector instruction that writes
+    its operand; the compiler inserts them, but not for an instruction inside assembly.  Empty asm statements (values kept from the
+    optimiser) are no instruction."""
+    with open(os.path.join(CSRC, name)) as f:
+        text = re.sub(r"//[^\n]*", "", f.read())
+    bodies = re.findall(r"\basm\b(?:\s+volatile)?\s*\(\s*\"([^\"]*)\"", text)
+    assert bodies and all(b == "" for b in bodies), bodies
