@@ -42,12 +42,12 @@ HIPCC_FLAGS = [
 # and of the diagonal sums, none touched inside its product loops.)
 # wkv5c_bwd runs at the register limit too (256, eight waves a CU) and keeps a few values that a wave needs once a chunk in scratch:
 # these and no more.
-# rwkv7c_bwd: addresses and other values that its B waves need a few times a chunk (fp32 mode: of its stores).
+# rwkv7c_bwd: a reload in the chunk loop waits for the state that the same wave has asked for, so none.
 # The one-sweep kernels let the compiler count their waits: a spill inside their loops would put scratch traffic between a
 # prefetch and its use (and a forward variant that spilled eleven registers gave wrong results): none may spill.
 SPILL_LIMIT = {"wkv6_bwd_fused": 0, "wkv6_fwd_fused": 0, "wkv6_fwd_ws": 0, "wkv6_bwd_a_ws": 0, "wkv6_bwd_b_wsILi0E": 3, "wkv6_bwd_b_wsILi1E": 1, "wkv6_bwd_b_wsILi2E": 1,
                "wkv_rows": 0, "wkv5_steps": 0, "wkv5b_fwd": 0, "wkv5b_bwd": 0, "wkv5c_fwd": 0, "wkv5c_bwdILb0E": 6, "wkv5c_bwdILb1E": 9, "wkv4_fwd_reg": 0, "wkv4_bwd_reg": 0, "timex_conv_h2": 0, "timex_gw_sum_h2": 0,
-               "timex_conv_any": 0, "timex_gw_any": 2, "rwkv7c_fwd": 0, "rwkv7c_bwdILb0E": 1, "rwkv7c_bwdILb1E": 26}
+               "timex_conv_any": 0, "timex_gw_any": 2, "rwkv7c_fwd": 0, "rwkv7c_bwd": 0}
 
 _lib = None
 

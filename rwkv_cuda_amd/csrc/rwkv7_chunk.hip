@@ -454,6 +454,10 @@ DEVINL LaneB lane_bases(lds_t base, int l16, int g, int own) {
     opaque(b.tr.a); opaque(b.tr.b); opaque(b.rows[0]); opaque(b.rows[1]); opaque(b.own); opaque(b.pair); opaque(b.own_pair);
     return b;
 }
+// The same lane's addresses in another region, d bytes on (modulo 2^32): an addition each, where bases of its own would be spilled
+DEVINL LaneB moved(const LaneB& b, lds_t d) {
+    return {{b.tr.a + d, b.tr.b + d}, {b.rows[0] + d, b.rows[1] + d}, b.own + d, b.pair + d, b.own_pair + d};
+}
 // v, dy: four tokens of a channel, and over channels
 template <bool F32> DEVINL auto exact_piece(lds_t a) { if constexpr (F32) return get3(a); else return lds_ld<u32x2>(a); }
 template <bool F32> DEVINL auto exact_tr(uint32_t plane, const Tr& o, int hb) { if constexpr (F32) return get3_tr(plane, o, hb); else return ld_tr16(o, plane, hb); }
@@ -603,9 +607,10 @@ DEVINL void bwd_store_rows(const SmemCB<false>& S, int vbuf, const Args7c& p, si
     put(p.da, &S.park[0][t][c4]); put(p.dr, &S.park[1][t][c4]); put(p.db, &S.park[2][t][c4]); put(p.dk, &S.park[3][t][c4]);
     put(p.dw, &S.park[4][t][c4]); put(p.dv, &S.parkv[vbuf][t][c4]);
 }
-// fp32: element [4 g + v][own] of the chunk whose first row is row0, straight to global memory
-DEVINL void store_f32(uint16_t* dst, size_t row0, int v, uint32_t lane_off, int H, int h, float x) {
-    *reinterpret_cast<float*>(reinterpret_cast<char*>(dst) + ((row0 + v) * H + h) * N * 4 + lane_off * 4u) = x;
+// fp32: element `first` + o straight to global memory.  (One scalar base a tensor and the row in the lane's offset: with a base for each
+// of the twenty rows that a B wave stores the scalar registers were spilled.)
+DEVINL void store_f32(uint16_t* dst, size_t first, uint32_t o, float x) {
+    *reinterpret_cast<float*>(reinterpret_cast<char*>(dst) + first * 4 + o * 4u) = x;
 }
 template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t tok0, int nch, int H, int h) {
     const int lane = tid & 63, wp = w - 8, tp = tid - 8 * 64;
@@ -676,7 +681,7 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
     tiles(S.pl[0]);
     for (int i = 0; i < nch; ++i) {
         const PlanesB& O = S.pl[i & 1];
-        const LaneB two = lane_bases(sb + L::TWO + (i & 1) * L::SLOT, l16, g, own);
+        const LaneB two = moved(one, L::TWO + (i & 1) * L::SLOT - L::ONE);
         // ---------------------------------------------------------------- phase 1: the parts of dU, dV that need no tile
         Sum2 dUs = SUM0, dVs = SUM0;
 #pragma unroll
@@ -700,7 +705,7 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
             const f32x4 dV = total(dVs);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                if constexpr (F32) store_f32(p.dv, tok0 + static_cast<size_t>(nch - 1 - i) * CL, v, static_cast<uint32_t>(4 * g * H) * N + own, H, h, dV[v]);
+                if constexpr (F32) store_f32(p.dv, ((tok0 + static_cast<size_t>(nch - 1 - i) * CL) * H + h) * N, static_cast<uint32_t>((4 * g + v) * H) * N + own, dV[v]);
                 else S.parkv[i & 1][4 * g + v][own] = f2bf(dV[v]);
             }
 #pragma unroll
@@ -739,11 +744,18 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
     }
 }
 
+// The lane's number, worked out where it is used.  (What is derived from threadIdx is kept in registers across the chunk loop, and where
+// those do not last, in scratch: a reload waits for all loads under way, the next state among them.)
+DEVINL uint32_t lane_again() {
+    uint32_t all = ~0u;
+    asm volatile("" : "+s"(all));
+    return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
+}
 template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
     const int lane = tid & 63, q = w & 3, l16 = lane & 15, g = lane >> 4;
     const int own = 16 * q + l16;                    // key channel j of this lane's column
     using L = LB<F32>;
-    const LaneB one = lane_bases(sb + L::ONE, l16, g, own);
+    LaneB one = lane_bases(sb + L::ONE, l16, g, own);
     const Tr base_tr = tr_bases(sb, l16, g);
     f32x4 dS[4], S0b[4];                             // dS, S0 at [i = 16 ib + 4 g + v][j = own]
 #pragma unroll
@@ -753,8 +765,8 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             dS[ib][v] = p.dsT != nullptr ? p.dsT[bh * N * N + static_cast<size_t>(16 * ib + 4 * g + v) * N + own] : 0.f;
     auto fetch_state = [&](int c) __attribute__((always_inline)) {
         const float* slot = p.s + (bh * nch + c) * N * N;
-        uint32_t o = static_cast<uint32_t>(4 * g * N + own) * 4u;
-        asm volatile("" : "+v"(o));
+        const uint32_t me = lane_again();
+        const uint32_t o = ((me >> 4) * (4 * N) + 16 * q + (me & 15)) * 4u;
         const char* const at = reinterpret_cast<const char*>(slot);
 #pragma unroll
         for (int ib = 0; ib < 4; ++ib)
@@ -780,10 +792,11 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     };
     // tile parts, scaling, decay gradient of the chunk whose planes are O and whose first row is row0; results parked as bf16
     auto finish = [&](const lds_t O, const size_t row0) __attribute__((always_inline)) {
-        [[maybe_unused]] uint32_t lo = static_cast<uint32_t>(4 * g * H) * N + own;
-        asm volatile("" : "+v"(lo));
+        const uint32_t me = lane_again();
+        [[maybe_unused]] const uint32_t lo = (me >> 4) * static_cast<uint32_t>(4 * H * N) + 16 * q + (me & 15);
+        [[maybe_unused]] const size_t first = (row0 * H + h) * N;
         auto put = [&](const int k, uint16_t* dst, const int v, const float x) __attribute__((always_inline)) {
-            if constexpr (F32) store_f32(dst, row0, v, lo, H, h, x);
+            if constexpr (F32) store_f32(dst, first, lo + static_cast<uint32_t>(v * H) * N, x);
             else lds_st<uint16_t>(park + 2 * PK * (CL * k + v), f2bf(x));
         };
         const float d1j = chan(O, 0), d2j = chan(O, 1);
@@ -811,7 +824,8 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         }
         // G_t = P_{t+1} + del_t,  P_t = G_t + a da:  suffix sums over t = 4 g + v, later lane groups first
         const float tot = (del[0] + ada[0]) + (del[1] + ada[1]) + (del[2] + ada[2]) + (del[3] + ada[3]);
-        const float t1 = __shfl_down(tot, 16, 64), t2 = __shfl_down(tot, 32, 64), t3 = __shfl_down(tot, 48, 64);
+        auto of_lane = [](uint32_t l, float x) __attribute__((always_inline)) { return __int_as_float(__builtin_amdgcn_ds_bpermute(static_cast<int>(4 * l), __float_as_int(x))); };
+        const float t1 = of_lane(me + 16, tot), t2 = of_lane(me + 32, tot), t3 = of_lane(me + 48, tot);
         float Pn = Pj + (g < 3 ? t1 : 0.f) + (g < 2 ? t2 : 0.f) + (g < 1 ? t3 : 0.f);     // P after this lane's last token
 #pragma unroll
         for (int v = 3; v >= 0; --v) {
@@ -819,7 +833,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             Pn = G + ada[v];
             put(4, p.dw, v, G * dwf[v]);
         }
-        Pj = __shfl(Pn, l16, 64);                    // lane group 0 holds P at the start of the chunk
+        Pj = of_lane(me & 15, Pn);                   // lane group 0 holds P at the start of the chunk
     };
     fetch_state(nch - 1);
     __syncthreads();
@@ -827,7 +841,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     for (int i = 0; i < nch; ++i) {
         const int c = nch - 1 - i;
         const lds_t O = planes_of(i);
-        const LaneB two = lane_bases(sb + L::TWO + (i & 1) * L::SLOT, l16, g, own);
+        const LaneB two = moved(one, L::TWO + (i & 1) * L::SLOT - L::ONE);
         // ---------------------------------------------------------------- phase 1: finish the previous visit's chunk
         if (i > 0) finish(planes_of(i - 1), tok0 + static_cast<size_t>(c + 1) * CL);
         else if (p.dsT != nullptr) {
@@ -901,6 +915,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         }
         __syncthreads();
     }
+    opaque(one.pair);                                // (or the tiles' addresses are kept from before the loop, in scratch)
     finish(planes_of(nch - 1), tok0);
     __syncthreads();
 }
