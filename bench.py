@@ -52,9 +52,9 @@ TRAFFIC_MEASURED = {
     "wkv_sweep<gr+gu+gw, two-sided>": 2148e6 + 537e6,
     # profiles/rwkv7_chunk_kernels_B8_T4096_C4096.md (four calls of T = 1024)
     "rwkv7c_fwd x4 (T=1024 each)": 4 * (411.3e6 + 746.6e6),
-    "rwkv7c_bwd x4": 4 * (1150.3e6 + 411.6e6),
+    "rwkv7c_bwd x4": 4 * (1149.8e6 + 411.0e6),
     "rwkv7c_fwd<fp32> x4 (T=1024 each)": 4 * (814.4e6 + 813.7e6),
-    "rwkv7c_bwd<fp32> x4": 4 * (1638.1e6 + 822.6e6),
+    "rwkv7c_bwd<fp32> x4": 4 * (1620.8e6 + 813.7e6),
     # profiles/wkv5_split_kernels_B8_T4096_C4096_N128.md (both launches of a kernel and the sums that follow them)
     "wkv6_fwd_ws<head decay, split> x2": (805.7e6 + 536.9e6) + (1342.5e6 + 268.5e6),
     "wkv6_bwd_a_ws<head decay, split> x2": (1095.4e6 + 1334.3e6) + (1638.6e6 + 1065.4e6),

@@ -378,7 +378,7 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
 // What bounds it: issue.  B8 T1024 C4096, one call: 398 us with every product on the fp32 matrix instructions, in four waves that did
 // everything in turn between four barriers; 390 in two roles of four waves; 335 with split products, since the fp32 instructions
 // (96 a wave and chunk) held the vector unit for half of the time.  The first of these forms and this one in alternation on one
-// machine: bf16 385 -> 325 us, fp32 mode 392 -> 380.  Vector instructions now issue 67 % of a SIMD's time, matrix ones about a third.
+// machine: bf16 382 -> 326 us, fp32 mode 405 -> 379.  Vector instructions now issue 68 % of a SIMD's time, matrix ones about a third.
 // Errors against 64 bits, T16 to T1024, slow to strong decays, largest, before -> now: y 2.4 -> 1.7e-7, sT 1.6 -> 1.0e-7, sa 2.3 -> 1.7e-7.
 template <bool F32, bool KEEP>
 __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c p) {
@@ -409,9 +409,9 @@ __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c p) {
 // What bounds it: issue, and waits for LDS and at barriers.  B8 T1024 C4096, one call: 762 us with fp32 matrix instructions (962 a
 // chunk, 57 % of a SIMD's time in which it could issue no vector instruction), 676 with split products.  Of that, causal tiles
 // and the inverse moved from phase 1, where everybody waited for wave 0, into the phase 3 before: 727 -> 676.  Both forms in alternation
-// on one machine: bf16 711 -> 622 us, vector instructions issuing 62 % of a SIMD's time.  The fp32 mode lost, 795 -> 820 (on another
-// machine 796 -> 826): its 24 rows a chunk leave from registers, 64 bytes at a time, and it splits v and dy as well; forward and
-// backward together 1186 -> 1171 there, 1189 -> 1191 on the other.
+// on one machine: bf16 720 -> 623 us, vector instructions issuing 63 % of a SIMD's time; fp32 mode 800 -> 766, 53 %: its 24 rows a chunk
+// leave from registers, 64 bytes at a time, and it splits v and dy as well.  (With 26 spilled registers, addresses for the most part, it
+// took 826: see lane_again.)
 // Errors against 64 bits, T16 to T1024, slow to strong decays, largest, before -> now: ds0 1.8 -> 1.0e-7, dr 1.9 -> 1.3e-7, dk 2.1 ->
 // 1.3e-7, dv 2.2 -> 1.7e-7, da 3.0 -> 2.2e-7, db 3.2 -> 2.1e-7; dw 3.2 -> 2.4e-6 at T1024 and usual decays, 7.3 -> 6.9e-6 at decays near
 // e^-0.6, where 1 - sig has few digits.

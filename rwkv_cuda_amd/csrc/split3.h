@@ -42,7 +42,7 @@ DEVINL uint32_t round2(float a, float b) {
 }
 // The pair with an infinity replaced by the largest bf16 of its sign, in all of 16-bit integers: what is beyond 0x7f7f on the positive
 // side, on the negative one what is beyond 0xff7f as unsigned numbers.  Two instructions a pair: B8 T1024 C4096, backward, fp32 mode
-// 802 -> 826 us, bf16 613 -> 638; forward 376 -> 382 and 319 -> 327.  (Values held to that bound before they are rounded cost the
+// 802 -> 826 us, bf16 613 -> 638 (in a form with a few spills); forward 376 -> 382 and 319 -> 327.  (Values held to that bound before they are rounded cost the
 // backward registers: 796 -> 904 and 601 -> 641.  Looking for such values first and branching: 842 and 624.)  Not as inline assembly: a
 // matrix instruction has to stay two wait states behind a vector instruction that writes its operand, and the compiler, which sees
 // to that, does not look into assembly.
