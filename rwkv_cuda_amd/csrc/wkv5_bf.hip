@@ -28,9 +28,9 @@
 // l = -4.5, 0.70 at -8.6, where they took 1.7 to 3.8 ms).
 //
 // What bounds it (B8 T4096 C4096: one workgroup per CU).  Forward 0.43 ms for 2.1 GB, half of them the saved states: HBM (5.0 TB/s;
-// 0.82 ms as four heads of 64).  Backward 1.05 ms: the D waves, some 1600 vector and 170 matrix instructions a chunk, and their
-// waits for the saved state (2.95 ms as two sweeps over four heads of 64, whose fp32 terms went through memory).  Both together
-// 6.56 -> 1.47 ms where a channel's decay was strong, 3.83 -> 1.48 where none was.
+// 0.82 ms as four heads of 64).  Backward 0.98 ms, 3.3 GB: memory and issue, which its two barriers a chunk do not let overlap
+// entirely (2.95 ms as two sweeps over four heads of 64, whose fp32 terms went through memory).  Both together 6.56 -> 1.48 ms where a
+// channel's decay was strong, 3.83 -> 1.44 where none was.
 #include <stddef.h>
 
 #include "wkv6_fused.h"
@@ -38,7 +38,7 @@
 namespace rwkv {
 namespace {
 
-constexpr int NTH = 512;             // waves 0..3 hold states, 4..7 load and prepare
+constexpr int NTH = 512;             // forward: waves 0..3 hold states, 4..7 load and prepare
 constexpr float LAM_MID = -4.5f;     // strongest log decay for one reference (one per half: W_STEPS_BF16)
 constexpr f32x4 ZERO4 = {0.f, 0.f, 0.f, 0.f};
 
@@ -62,9 +62,9 @@ template <int HN> struct G {
     // forward: three slots of planes R' hi, lo, K' hi, lo, V and sum r u k; two sets of tile parts
     static constexpr uint32_t FRH = 0, FRL = PLANE, FKH = 2 * PLANE, FKL = 3 * PLANE, FV = 4 * PLANE, FRUK = 5 * PLANE, FSLOT = FRUK + 4 * L;
     static constexpr uint32_t FPART = BASE + 3 * FSLOT, FTOTAL = FPART + 2 * PARTS * PART;
-    // backward: two slots of planes r, k, v, gy and two scalars a token; the gradient state hi, lo [j][i]; one set of tile parts
+    // backward: two slots of planes r, k, v, gy and two scalars a token; the gradient state hi, lo [j][i]; one set of parts of tile A; tile B in three forms
     static constexpr uint32_t R = 0, K = PLANE, V = 2 * PLANE, GY = 3 * PLANE, VG = 4 * PLANE, RUK = VG + 4 * L, SLOT = RUK + 4 * L;
-    static constexpr uint32_t DSH = BASE + 2 * SLOT, DSL = DSH + HN * ROW, BPART = DSL + HN * ROW, BTOTAL = BPART + PARTS * PART;
+    static constexpr uint32_t DSH = BASE + 2 * SLOT, DSL = DSH + HN * ROW, BPART = DSL + HN * ROW, BTILE = BPART + PARTS * PART, BTOTAL = BTILE + 3 * PART;
 };
 static_assert(G<128>::FTOTAL <= 160 * 1024 && G<128>::BTOTAL <= 160 * 1024, "LDS of one CU");
 
@@ -167,32 +167,33 @@ template <bool LANE_SNK> DEVINL bool causal(int z, int l16, int row) {
     const int a = 16 * Quad<LANE_SNK>::ROWT[z] + row, b = 16 * Quad<LANE_SNK>::LANET[z] + l16;
     return LANE_SNK ? a < b : b < a;
 }
-// the part, masked, with `diag` (of the lane's token in the lane tile) on its diagonal, to LDS
-template <bool LANE_SNK> DEVINL void put_part(lds_t out, const f32x4 (&q)[3], const float (&diag)[2], int lane) {
+// a quadrant of the part, masked, with `diag` (of the lane's token) on its diagonal, to LDS
+template <bool LANE_SNK, int z> DEVINL void put_quad(lds_t out, const f32x4& q, float diag, int lane) {
     const int l16 = lane & 15, g = lane >> 4;
+    f32x4 x;
 #pragma unroll
-    for (int z = 0; z < 3; ++z) {
-        f32x4 x;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            x[v] = causal<LANE_SNK>(z, l16, 4 * g + v) ? q[z][v] : 0.f;
-            if (Quad<LANE_SNK>::ROWT[z] == Quad<LANE_SNK>::LANET[z]) x[v] = l16 == 4 * g + v ? diag[Quad<LANE_SNK>::LANET[z]] : x[v];
-        }
-        lds_st<f32x4>(out + 1024 * z + 16 * lane, x);
+    for (int v = 0; v < 4; ++v) {
+        x[v] = causal<LANE_SNK>(z, l16, 4 * g + v) ? q[v] : 0.f;
+        if (Quad<LANE_SNK>::ROWT[z] == Quad<LANE_SNK>::LANET[z]) x[v] = l16 == 4 * g + v ? diag : x[v];
     }
+    lds_st<f32x4>(out + 1024 * z + 16 * lane, x);
 }
 // the parts added up and split: operands of the two lane tiles (slots: the row tokens in accumulator order)
-template <bool LANE_SNK, int PARTS, uint32_t PART> DEVINL void take_parts(lds_t in, int lane, Op2 (&a)[2]) {
-    f32x4 s[3];
+template <int PARTS, uint32_t PART> DEVINL f32x4 sum_parts(lds_t in, int z, int lane) {
+    f32x4 s = lds_ld<f32x4>(in + 1024 * z + 16 * lane);
 #pragma unroll
-    for (int z = 0; z < 3; ++z) {
-        s[z] = lds_ld<f32x4>(in + 1024 * z + 16 * lane);
-#pragma unroll
-        for (int i = 1; i < PARTS; ++i) s[z] += lds_ld<f32x4>(in + i * PART + 1024 * z + 16 * lane);
-    }
-    // lane is the sink: sources of tile 0 for both lane tiles, of tile 1 for the second; lane is the source: the other way round
-    if constexpr (LANE_SNK) { a[0] = split8(s[0], ZERO4); a[1] = split8(s[1], s[2]); }
-    else { a[0] = split8(s[0], s[1]); a[1] = split8(ZERO4, s[2]); }
+    for (int i = 1; i < PARTS; ++i) s += lds_ld<f32x4>(in + i * PART + 1024 * z + 16 * lane);
+    return s;
+}
+// lane is the sink (forward): sources of tile 0 for both lane tiles, of tile 1 for the second
+template <int PARTS, uint32_t PART> DEVINL void take_parts(lds_t in, int lane, Op2 (&a)[2]) {
+    a[0] = split8(sum_parts<PARTS, PART>(in, 0, lane), ZERO4);
+    a[1] = split8(sum_parts<PARTS, PART>(in, 1, lane), sum_parts<PARTS, PART>(in, 2, lane));
+}
+// lane is the source (backward): the other way round; one lane tile
+template <int PARTS, uint32_t PART, int Z> DEVINL Op2 take_lane_tile(lds_t in, int lane) {
+    if constexpr (Z == 0) return split8(sum_parts<PARTS, PART>(in, 0, lane), sum_parts<PARTS, PART>(in, 1, lane));
+    else return split8(ZERO4, sum_parts<PARTS, PART>(in, 2, lane));
 }
 // powers for a tile part, channel ch0 + e: of token 16 z + l16, x as the sink, y as the source; they are those of the token in its
 // half and serve both.  cx, cy: as sink of the second and source of the first half of a pair across them.
@@ -205,15 +206,14 @@ DEVINL void tile_powers(TilePowers& t, lds_t lam, int l16) {
         t.cx[e] = wpow(l, l16); t.cy[e] = wpow(l, 15 - l16);
     }
 }
-// tile part from raw rows (operands of the two token tiles)
-template <bool LANE_SNK> DEVINL void raw_part(const bf16x8 (&r)[2], const bf16x8 (&k)[2], const TilePowers& t, f32x4 (&q)[3]) {
-    using Q = Quad<LANE_SNK>;
+// tile part from raw rows (operands of the two token tiles), lane = sink
+DEVINL void raw_part(const bf16x8 (&r)[2], const bf16x8 (&k)[2], const TilePowers& t, f32x4 (&q)[3]) {
+    using Q = Quad<true>;
 #pragma unroll
     for (int z = 0; z < 3; ++z) {
         const bool across = Q::ROWT[z] != Q::LANET[z];
-        const int snk = LANE_SNK ? Q::LANET[z] : Q::ROWT[z], src = LANE_SNK ? Q::ROWT[z] : Q::LANET[z];
-        const Op2 x = scaled(r[snk], across ? t.cx : t.px), y = scaled(k[src], across ? t.cy : t.py);
-        q[z] = LANE_SNK ? mm3(y, x, ZERO4) : mm3(x, y, ZERO4);
+        const Op2 x = scaled(r[Q::LANET[z]], across ? t.cx : t.px), y = scaled(k[Q::ROWT[z]], across ? t.cy : t.py);
+        q[z] = mm3(y, x, ZERO4);
     }
 }
 
@@ -286,7 +286,7 @@ template <int HN, bool RAW> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) vo[ct] = ld_tra<A::ROW>(xt + A::FV + 32 * (CT * q + ct));
         Op2 at[2];
-        take_parts<true, A::PARTS, A::PART>(sb + A::FPART + (c & 1) * (A::PARTS * A::PART), lane, at);
+        take_parts<A::PARTS, A::PART>(sb + A::FPART + (c & 1) * (A::PARTS * A::PART), lane, at);
         const rows_t o = rows_of(out + static_cast<size_t>(c) * L * C, T - c * L, C);
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
@@ -379,7 +379,7 @@ template <int HN, bool RAW> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int 
                 const int o = 2 * ((16 * z + l16) * C + 32 * q + 8 * g);
                 r[z] = op4(load16(rr, o)); k[z] = op4(load16(kk, o));
             }
-            raw_part<true>(r, k, tpw, qd);
+            raw_part(r, k, tpw, qd);
         } else {
             Op2 xo[2], yo[2];
 #pragma unroll
@@ -392,7 +392,8 @@ template <int HN, bool RAW> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int 
             for (int z = 0; z < 3; ++z) qd[z] = mm3(yo[Quad<true>::ROWT[z]], xo[Quad<true>::LANET[z]], ZERO4);
         }
         const float diag[2] = {q == 0 ? lds_f(s + A::FRUK + 4 * l16) : 0.f, q == 0 ? lds_f(s + A::FRUK + 4 * (16 + l16)) : 0.f};
-        put_part<true>(sb + A::FPART + ((c & 1) * A::PARTS + q) * A::PART, qd, diag, lane);
+        const lds_t out = sb + A::FPART + ((c & 1) * A::PARTS + q) * A::PART;
+        put_quad<true, 0>(out, qd[0], diag[0], lane); put_quad<true, 1>(out, qd[1], 0.f, lane); put_quad<true, 2>(out, qd[2], diag[1], lane);
     };
     fetch(0, x[0]); fetch(1, x[1]);
     put(0, x[0]); fetch(2, x[0]);
@@ -435,347 +436,387 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_fwd(const ArgsW p) {
 }
 
 // ---------------------------------------------------------------------------------------------------- backward
-// One reverse sweep, two barriers a chunk, two roles of four waves:
-//   D, waves 0..3 (key channels j): the gradient state dS[ct][ib][v] = D[i = 16 ib + 4 g + v][j = own], the B operand of contractions
-//      over the value channel: gk in the first half of a chunk; gr, the gradient state's update and the decay gradient in the second.
-//      The saved state passes through in tiles (an odd chunk's is one update away from the saved one, made on the way).  The tile B is
-//      made by each of these waves in both orientations: its operands are the rows that the state products read anyway, and an
-//      accumulator with the summed tokens in its registers is an operand as it stands.
-//   E, waves 4..7 (value channels i): first half: the loads, the rows of the next chunk to LDS, this chunk's tile A in parts; second
-//      half: gv, for which the D waves left their gradient state in LDS (hi, lo) in the first.
+// One reverse sweep, two barriers a chunk, two roles of HN / 16 waves each (head size 128: all sixteen of a CU):
+//   D (16 key channels j): the gradient state dS[ib][v] = D[i = 16 ib + 4 g + v][j = own], the B operand of contractions over the
+//      value channel: gk in the first half of a chunk; gr, the gradient state's update and the decay gradient in the second.
+//      The saved state passes through in tiles (an odd chunk's is one update away from the saved one, made on the way).
+//   E (32 value channels i of 16 tokens): first half: the loads, the rows of the next chunk to LDS, this chunk's tile A in parts (a
+//      wave makes the quadrants within the halves or the one across, of 32 channels); second half: gv, for which the D waves left
+//      their gradient state in LDS (hi, lo) in the first, and the next chunk's tile B as the operands that the D waves take: B and
+//      its weighted form with lane = source, its transpose with lane = sink.
+// Twice four waves, of 32 key channels each and with the tile B made by each of the D waves, took 1042 us (B8 T4096 C4096 N128) where
+// these take 981 (heads of 64: the same).  Without its memory operations the kernel takes 753 us, and its 3.3 GB about 660 at a copy's rate.
 template <bool LANE_SNK> DEVINL void mask(f32x4 (&b)[3], int l16, int g) {
 #pragma unroll
     for (int z = 0; z < 3; ++z)
 #pragma unroll
         for (int v = 0; v < 4; ++v) b[z][v] = causal<LANE_SNK>(z, l16, 4 * g + v) ? b[z][v] : 0.f;
 }
+// The tile B as operands of its lane tiles, 3 KB a form.  The lane tile that meets both halves of the other side takes 16 bytes a lane
+// and term; the other one has zeros on one side (HIGH: in its low slots), the two terms share 16 bytes.
+template <bool LANE_SNK> DEVINL void put_tile(lds_t o, const f32x4 (&t)[3], int lane) {
+    const Op2 f = LANE_SNK ? split8(t[1], t[2]) : split8(t[0], t[1]);
+    const f32x4& s = LANE_SNK ? t[0] : t[2];
+    const HL a = hilo2k(s[0], s[1]), b = hilo2k(s[2], s[3]);
+    o += 16 * lane;
+    lds_st<bf16x8>(o, f.h); lds_st<bf16x8>(o + 1024, f.l);
+    lds_st<u32x4>(o + 2048, u32x4{a.h, b.h, a.l, b.l});
+}
+template <bool HIGH> DEVINL Op2 half_op(lds_t o) {
+    const u32x4 x = lds_ld<u32x4>(o + 2048);
+    return HIGH ? Op2{as_op(0u, 0u, x[0], x[1]), as_op(0u, 0u, x[2], x[3])} : Op2{as_op(x[0], x[1], 0u, 0u), as_op(x[2], x[3], 0u, 0u)};
+}
+DEVINL Op2 full_op(lds_t o) { return {ld_op(o), ld_op(o + 1024)}; }
+
+// The lane's number, worked out where it is used.  (What is derived from threadIdx is kept in registers across the chunk loop, and where
+// those do not last, in scratch: a reload waits for all loads under way.)
+DEVINL uint32_t lane_now() {
+    uint32_t all = ~0u;
+    asm volatile("" : "+s"(all));
+    return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
+}
 
 template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, int h, int b, size_t base, int nch) {
     using A = G<HN>;
-    constexpr int CT = A::CT, KS = A::KS, NI = A::NB16;
+    constexpr int KS = A::KS, NI = A::NB16;
     const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
     // Powers of a set of eight slots, token 16 a + 4 g + b: a base per lane times o^b times o^{16 a} (or the reverse); the eight would
     // take the registers that the states need.  Bases: cb of o^{t-m}, kb of o^{m-1-t}, m the middle of the token's half.
-    float l[CT], u[CT], o1[CT], o2[CT], o3[CT], o8[CT], o16[CT], o32[CT], cb[CT], kb[CT];
-    f32x4 dS[CT][NI];
-    float gw[CT], gP[CT], gu[CT];
+    const float l = lds_f(sb + A::LAM + 4 * (16 * q + l16));
+    const float o1 = wpow(l, 1), o2 = wpow(l, 2), o3 = wpow(l, 3), o8 = wpow(l, 8), o16 = wpow(l, 16), o32 = wpow(l, 32);
+    const float cb = wpow(l, 4 * g - 8), kb = wpow(l, 4 - 4 * g);
+    f32x4 dS[NI];
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        const int j = 16 * (CT * q + ct) + l16;
-        l[ct] = lds_f(sb + A::LAM + 4 * j); u[ct] = lds_f(sb + A::U + 4 * j);
-        o1[ct] = wpow(l[ct], 1); o2[ct] = wpow(l[ct], 2); o3[ct] = wpow(l[ct], 3); o8[ct] = wpow(l[ct], 8); o16[ct] = wpow(l[ct], 16); o32[ct] = wpow(l[ct], 32);
-        cb[ct] = wpow(l[ct], 4 * g - 8);
-        kb[ct] = wpow(l[ct], 4 - 4 * g);
-#pragma unroll
-        for (int ib = 0; ib < NI; ++ib) dS[ct][ib] = ZERO4;
-        gw[ct] = gP[ct] = gu[ct] = 0.f;
-    }
+    for (int ib = 0; ib < NI; ++ib) dS[ib] = ZERO4;
+    float gw = 0.f, gP = 0.f, gu = 0.f;
     // (hidden: hoisted out of the loop the powers and token numbers would take registers all the same)
     auto hide = [](float x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); return x; };
-    auto up = [&](int ct, float base, bool span, float (&f)[8]) __attribute__((always_inline)) {
+    auto up = [&](float base, bool span, float (&f)[8]) __attribute__((always_inline)) {
         base = hide(base);
-        f[0] = base; f[1] = base * o1[ct]; f[2] = base * o2[ct]; f[3] = base * o3[ct];
+        f[0] = base; f[1] = base * o1; f[2] = base * o2; f[3] = base * o3;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f[4 + e] = span ? f[e] * o16[ct] : f[e];
+        for (int e = 0; e < 4; ++e) f[4 + e] = span ? f[e] * o16 : f[e];
     };
-    auto down = [&](int ct, float base, bool span, float (&f)[8]) __attribute__((always_inline)) {
+    auto down = [&](float base, bool span, float (&f)[8]) __attribute__((always_inline)) {
         base = hide(base);
-        f[4] = base * o3[ct]; f[5] = base * o2[ct]; f[6] = base * o1[ct]; f[7] = base;
+        f[4] = base * o3; f[5] = base * o2; f[6] = base * o1; f[7] = base;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] = span ? f[4 + e] * o16[ct] : f[4 + e];
+        for (int e = 0; e < 4; ++e) f[e] = span ? f[4 + e] * o16 : f[4 + e];
     };
-    auto to_ref = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { up(ct, cb[ct], false, f); };                                    // o^{t-m}
-    auto from_ref = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { down(ct, kb[ct], false, f); };                                // o^{m-1-t}
-    auto from_start = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { up(ct, cb[ct] * o8[ct], true, f); };            // o^t
-    auto to_end = [&](int ct, float (&f)[8]) __attribute__((always_inline)) { down(ct, kb[ct] * o8[ct], true, f); };            // o^{31-t}
+    auto to_ref = [&](float (&f)[8]) __attribute__((always_inline)) { up(cb, false, f); };                    // o^{t-m}
+    auto from_ref = [&](float (&f)[8]) __attribute__((always_inline)) { down(kb, false, f); };                // o^{m-1-t}
+    auto from_start = [&](float (&f)[8]) __attribute__((always_inline)) { up(hide(cb) * o8, true, f); };            // o^t
+    auto to_end = [&](float (&f)[8]) __attribute__((always_inline)) { down(hide(kb) * o8, true, f); };              // o^{31-t}
+    auto stage = [] __attribute__((always_inline)) () { __builtin_amdgcn_sched_barrier(0); };      // (or operands are asked for so early that the registers do not hold them)
     // The operands that a tile's lane tiles 0 and 1 are applied to, referred to the middle of the lane's half whichever half a slot's
     // token lies in.  f: the powers of the token in its own half.  Only the far pair (sinks of the second half for a source of the
     // first, or sources of the first for a sink of the second) takes o^16; the slots on the wrong side of the lane tile meet zeros.
-    auto tile_operands = [&](int ct, bool sinks, const bf16x8& x, const float (&f)[8], Op2 (&o)[2]) __attribute__((always_inline)) {
+    auto tile_operands = [&](bool sinks, const bf16x8& x, const float (&f)[8], Op2 (&o)[2]) __attribute__((always_inline)) {
         float fx[8], ff[4];
         unpack(x, fx);
 #pragma unroll
         for (int e = 0; e < 8; ++e) fx[e] *= f[e];
         o[0] = o[1] = split8(fx);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ff[e] = (sinks ? fx[4 + e] : fx[e]) * o8[ct] * o8[ct];      // (o^16 may underflow where this does not)
+        for (int e = 0; e < 4; ++e) ff[e] = (sinks ? fx[4 + e] : fx[e]) * o8 * o8;      // (o^16 may underflow where this does not)
         const HL a = hilo2k(ff[0], ff[1]), b = hilo2k(ff[2], ff[3]);
         Op2& w = o[sinks ? 0 : 1];
         const uint4 h = __builtin_bit_cast(uint4, w.h), lo = __builtin_bit_cast(uint4, w.l);
         w = sinks ? Op2{as_op(h.x, h.y, a.h, b.h), as_op(lo.x, lo.y, a.l, b.l)} : Op2{as_op(a.h, b.h, h.z, h.w), as_op(a.l, b.l, lo.z, lo.w)};
     };
-    const float t0 = static_cast<float>(4 * g);
-    const int to = tile_offset(l16, g, C);
     const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * (nch / 2) * HN * HN;
-    const uint32_t so = (16 * CT * q + l16) * HN + 4 * g;         // (a scalar base and one lane offset)
-    auto fetch_state = [&](int c, int ks, f32x4 (&s)[CT][2]) __attribute__((always_inline)) {
-        const float* const d = sv + static_cast<size_t>(c >> 1) * HN * HN + 32 * ks;
+    auto fetch_state = [&](int c, int ks, uint32_t so, f32x4 (&s)[2]) __attribute__((always_inline)) {      // (a scalar base and one lane offset)
+        const char* const d = reinterpret_cast<const char*>(sv + static_cast<size_t>(c >> 1) * HN * HN + 32 * ks);
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
+        for (int z = 0; z < 2; ++z) s[z] = *reinterpret_cast<const f32x4*>(d + 64 * z + so);
+    };
+    // the lane's addresses, anew in each half of a chunk
+    struct Lane { lds_t row, tra, tile; uint32_t state; int out; float t; };
+    auto lane_of = [&]() __attribute__((always_inline)) {
+        const uint32_t me = lane_now(), n = me & 15, gg = me >> 4;
+        return Lane{n * A::ROW + 8 * gg, (4 * gg + (n >> 2)) * A::ROW + 8 * (n & 3), 16 * me, ((16 * q + n) * HN + 4 * gg) * 4,
+                    tile_offset(static_cast<int>(n), static_cast<int>(gg), C), static_cast<float>(4 * gg)};
+    };
+    // second half of a chunk: gr, update
+    auto second = [&](auto odd_, const int c, const f32x4 (&part)[2], f32x4 (&Sn)[2][2]) __attribute__((always_inline)) {
+        constexpr bool ODD = decltype(odd_)::value;
+        const lds_t sx = sb + A::BASE + (ODD ? A::SLOT : 0);
+        const Lane at = lane_of();
+        const lds_t xr = at.row + sx, xu = at.tra + sx, xt = xu + 32 * q, qt = at.tra + sb + A::BASE + (ODD ? 0 : A::SLOT);
+        const rows_t gr_ = rows_of(p.gr + base + static_cast<size_t>(c) * L * C + 16 * q, T - c * L, C);
+        Op2 rs, kp;
+        {
+            float f[8];
+            from_start(f);
+            rs = scaled(ld_tra<A::ROW>(xt + A::R), f);
+            stage();
+            if constexpr (ODD) {
+                to_end(f);
+                kp = scaled(ld_tra<A::ROW>(qt + A::K + 32 * q), f);
+            }
+        }
+        f32x4 X[2] = {ZERO4, ZERO4};
 #pragma unroll
-            for (int z = 0; z < 2; ++z) s[ct][z] = *reinterpret_cast<const f32x4*>(d + 16 * ct * HN + 16 * z + so);
+        for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const bf16x8 gt = ld_tra<A::ROW>(xu + A::GY + 64 * ks + 32 * z);
+                bf16x8 vt;
+                if constexpr (ODD) vt = ld_tra<A::ROW>(qt + A::V + 64 * ks + 32 * z);
+                f32x4& s = Sn[ks & 1][z];
+                f32x4& d = dS[2 * ks + z];
+                if constexpr (ODD) s = mfma(vt, kp.l, mfma(vt, kp.h, s * o32));
+                gP += (s[0] * d[0] + s[1] * d[1]) + (s[2] * d[2] + s[3] * d[3]);
+                d = mfma(gt, rs.l, mfma(gt, rs.h, d * o32));
+                stage();
+            }
+            const Op2 s = split8(Sn[ks & 1][0], Sn[ks & 1][1]);
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const bf16x8 ga = ld_acc(xr + A::GY + 16 * z * A::ROW + 64 * ks);
+                X[z] = mfma(ga, s.l, mfma(ga, s.h, X[z]));
+            }
+            if (ks + 2 < KS) fetch_state(c, ks + 2, at.state, Sn[ks & 1]);
+            stage();
+        }
+        stage();
+        {
+            const uint4 r4 = __builtin_bit_cast(uint4, ld_tra<A::ROW>(xt + A::R));
+            float r[8], ps[8];
+            unpack8(r4, r);
+            from_start(ps);
+            const float th = at.t;
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                f32x4 o;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int e = 4 * z + v;
+                    const float x = X[z][v] * ps[e];
+                    gw = fmaf(r[e] * (th + static_cast<float>(16 * z + v)), x, gw);
+                    o[v] = x + part[z][v];
+                }
+                store_tile(gr_, at.out + 32 * z * C, C, static_cast<int>(at.tile >> 4), o);
+            }
+        }
     };
     auto chunk = [&](auto odd_, const int c) __attribute__((always_inline)) {
         constexpr bool ODD = decltype(odd_)::value;
         const lds_t sx = sb + A::BASE + (ODD ? A::SLOT : 0);
-        lds_t xr = sx + l16 * A::ROW + 8 * g, xt = sx + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3), xs = sx + 16 * g;
-        lds_t ho = sb + A::DSH + (16 * CT * q + l16) * A::ROW + 8 * g;
-        opaque(xr); opaque(xt); opaque(xs); opaque(ho);
-        const size_t co = base + static_cast<size_t>(c) * L * C + 16 * CT * q;
-        const rows_t gk_ = rows_of(p.gk + co, T - c * L, C), gr_ = rows_of(p.gr + co, T - c * L, C);
-        // ---- first half: gk
-        f32x4 Z[2][CT], Bt[3] = {ZERO4, ZERO4, ZERO4}, Ct[3] = {ZERO4, ZERO4, ZERO4};
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) { Z[0][ct] = ZERO4; Z[1][ct] = ZERO4; }
+        const Lane at = lane_of();
+        const lds_t xr = at.row + sx, xt = at.tra + sx + 32 * q, xs = sx + 4 * static_cast<lds_t>(at.t), ho = at.row + sb + A::DSH + 16 * q * A::ROW, tl = at.tile + sb + A::BTILE;
+        const size_t co = base + static_cast<size_t>(c) * L * C + 16 * q;
+        const rows_t gk_ = rows_of(p.gk + co, T - c * L, C);
+        // ---- first half: gk, gr's tile part
+        f32x4 Z[2] = {ZERO4, ZERO4};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            bf16x8 va[2], ga[2];
+            const Op2 s = split8(dS[2 * ks], dS[2 * ks + 1]);
+            const uint4 hi = __builtin_bit_cast(uint4, s.h), lo = __builtin_bit_cast(uint4, s.l);
+            const lds_t o = ho + 64 * ks;
+            lds_st<u32x2>(o, u32x2{hi.x, hi.y}); lds_st<u32x2>(o + 32, u32x2{hi.z, hi.w});
+            lds_st<u32x2>(o + (A::DSL - A::DSH), u32x2{lo.x, lo.y}); lds_st<u32x2>(o + (A::DSL - A::DSH) + 32, u32x2{lo.z, lo.w});
 #pragma unroll
-            for (int z = 0; z < 2; ++z) { va[z] = ld_acc(xr + A::V + 16 * z * A::ROW + 64 * ks); ga[z] = ld_acc(xr + A::GY + 16 * z * A::ROW + 64 * ks); }
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const Op2 s = split8(dS[ct][2 * ks], dS[ct][2 * ks + 1]);
-                const uint4 hi = __builtin_bit_cast(uint4, s.h), lo = __builtin_bit_cast(uint4, s.l);
-                const lds_t o = ho + 16 * ct * A::ROW + 64 * ks;
-                lds_st<u32x2>(o, u32x2{hi.x, hi.y}); lds_st<u32x2>(o + 32, u32x2{hi.z, hi.w});
-                lds_st<u32x2>(o + (A::DSL - A::DSH), u32x2{lo.x, lo.y}); lds_st<u32x2>(o + (A::DSL - A::DSH) + 32, u32x2{lo.z, lo.w});
-#pragma unroll
-                for (int z = 0; z < 2; ++z) Z[z][ct] = mfma(va[z], s.l, mfma(va[z], s.h, Z[z][ct]));
-            }
-#pragma unroll
-            for (int z = 0; z < 3; ++z) {
-                Bt[z] = mfma(ga[Quad<false>::ROWT[z]], va[Quad<false>::LANET[z]], Bt[z]);         // rows: sinks, lane: source
-                Ct[z] = mfma(va[Quad<true>::ROWT[z]], ga[Quad<true>::LANET[z]], Ct[z]);           // rows: sources, lane: sink
+            for (int z = 0; z < 2; ++z) {
+                const bf16x8 va = ld_acc(xr + A::V + 16 * z * A::ROW + 64 * ks);
+                Z[z] = mfma(va, s.l, mfma(va, s.h, Z[z]));
             }
         }
-        mask<false>(Bt, l16, g); mask<true>(Ct, l16, g);
-        f32x4 Lt[3];                                     // the tile weighted with the tokens between, for the decay gradient
+        f32x4 part[2];                                   // gr without the state's part
         {
-            const float lag = hide(t0 - static_cast<float>(l16 + 1));
-#pragma unroll
-            for (int z = 0; z < 3; ++z)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) Lt[z][v] = Bt[z][v] * (lag + static_cast<float>(16 * (Quad<false>::ROWT[z] - Quad<false>::LANET[z]) + v));
-        }
-        const Op2 ba[2] = {split8(Bt[0], Bt[1]), split8(ZERO4, Bt[2])}, la[2] = {split8(Lt[0], Lt[1]), split8(ZERO4, Lt[2])}, ca[2] = {split8(Ct[0], ZERO4), split8(Ct[1], Ct[2])};
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const bf16x8 rT = ld_tra<A::ROW>(xt + A::R + 32 * (CT * q + ct)), kT = ld_tra<A::ROW>(xt + A::K + 32 * (CT * q + ct));
-            const f32x4 vg0 = lds_ld<f32x4>(xs + A::VG), vg1 = lds_ld<f32x4>(xs + A::VG + 64);
-            float r[8], k[8], pe[8], pf[8], pm[8];
-            unpack(rT, r); unpack(kT, k);
+            const bf16x8 rT = ld_tra<A::ROW>(xt + A::R), kT = ld_tra<A::ROW>(xt + A::K);
+            const uint4 r4 = __builtin_bit_cast(uint4, rT), k4 = __builtin_bit_cast(uint4, kT);
+            f32x4 tx[2];
+            {
+                float pm[8];
+                Op2 ko[2];
+                from_ref(pm);
+                tile_operands(false, kT, pm, ko);
+                tx[0] = mm3(half_op<false>(tl + 2 * 3072), ko[0], ZERO4);
+                tx[1] = mm3(full_op(tl + 2 * 3072), ko[1], ZERO4);
+            }
+            const float u = lds_f(sb + A::U + 64 * q + (at.tile >> 2 & 60u));
             Op2 ro[2];
-            to_ref(ct, pm);
-            tile_operands(ct, true, rT, pm, ro);
-            from_ref(ct, pf);
-            to_end(ct, pe);
-            const float th = hide(t0);
+            {
+                float pm[8];
+                to_ref(pm);
+                tile_operands(true, rT, pm, ro);
+            }
 #pragma unroll
             for (int z = 0; z < 2; ++z) {
-                const f32x4 tz[2] = {mm3(ba[z], ro[z], ZERO4), mm3(la[z], ro[z], ZERO4)};
+                f32x4 tz, tw;
+                if (z) { tz = mm3(half_op<true>(tl), ro[z], ZERO4); tw = mm3(half_op<true>(tl + 3072), ro[z], ZERO4); }
+                else { tz = mm3(full_op(tl), ro[z], ZERO4); tw = mm3(full_op(tl + 3072), ro[z], ZERO4); }
+                const f32x4 vg4 = lds_ld<f32x4>(xs + A::VG + 64 * z);
+                const uint32_t rw[2] = {z ? r4.z : r4.x, z ? r4.w : r4.y}, kw[2] = {z ? k4.z : k4.x, z ? k4.w : k4.y};
+                const float th = at.t + static_cast<float>(16 * z), ba = hide(kb), bc = hide(cb);
+                const float pf[4] = {ba * o3, ba * o2, ba * o1, ba}, pc[4] = {bc, bc * o1, bc * o2, bc * o3};
                 f32x4 o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const int e = 4 * z + v;
-                    const float zs = Z[z][ct][v] * pe[e], ti = tz[0][v] * pf[e], vg = z ? vg1[v] : vg0[v], t = th + static_cast<float>(16 * z + v);
-                    gw[ct] = fmaf(k[e], (31.f - t) * zs + tz[1][v] * pf[e], gw[ct]);
-                    const float rv = r[e] * vg;
-                    gu[ct] = fmaf(rv, k[e], gu[ct]);
-                    o[v] = fmaf(rv, u[ct], zs + ti);
+                    const float r = v & 1 ? bf_hi(rw[v >> 1]) : bf_lo(rw[v >> 1]), k = v & 1 ? bf_hi(kw[v >> 1]) : bf_lo(kw[v >> 1]);
+                    float zs = Z[z][v] * (pf[v] * o8);
+                    if (z == 0) zs *= o16;
+                    const float vg = vg4[v], t = th + static_cast<float>(v), rv = r * vg;
+                    gw = fmaf(k, (31.f - t) * zs + tw[v] * pf[v], gw);
+                    gu = fmaf(rv, k, gu);
+                    o[v] = fmaf(rv, u, fmaf(tz[v], pf[v], zs));
+                    part[z][v] = fmaf(k * vg, u, tx[z][v] * pc[v]);
                 }
-                store_tile(gk_, to + 32 * z * C + 32 * ct, C, l16, o);
+                store_tile(gk_, at.out + 32 * z * C, C, static_cast<int>(at.tile >> 4), o);
             }
         }
-        f32x4 Sn[2][CT][2];
-        fetch_state(c, 0, Sn[0]);
-        fetch_state(c, 1, Sn[1]);
+        f32x4 Sn[2][2];
+        fetch_state(c, 0, at.state, Sn[0]);
+        fetch_state(c, 1, at.state, Sn[1]);
         __syncthreads();                                 // the rows of the chunk before are there, the gradient state is handed over
-        // ---- second half: gr, update
-        const lds_t qt = sb + A::BASE + (ODD ? 0 : A::SLOT) + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3);
-        Op2 rs[CT], kp[CT];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            float f[8];
-            from_start(ct, f);
-            rs[ct] = scaled(ld_tra<A::ROW>(xt + A::R + 32 * (CT * q + ct)), f);
-            if constexpr (ODD) {
-                to_end(ct, f);
-                kp[ct] = scaled(ld_tra<A::ROW>(qt + A::K + 32 * (CT * q + ct)), f);
-            }
-        }
-        f32x4 X[2][CT];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) { X[0][ct] = ZERO4; X[1][ct] = ZERO4; }
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            bf16x8 ga[2];
-#pragma unroll
-            for (int z = 0; z < 2; ++z) {
-                const bf16x8 gt = ld_tra<A::ROW>(xt + A::GY + 64 * ks + 32 * z);
-                bf16x8 vt;
-                if constexpr (ODD) vt = ld_tra<A::ROW>(qt + A::V + 64 * ks + 32 * z);
-                ga[z] = ld_acc(xr + A::GY + 16 * z * A::ROW + 64 * ks);
-#pragma unroll
-                for (int ct = 0; ct < CT; ++ct) {
-                    f32x4& s = Sn[ks & 1][ct][z];
-                    f32x4& d = dS[ct][2 * ks + z];
-                    if constexpr (ODD) s = mfma(vt, kp[ct].l, mfma(vt, kp[ct].h, s * o32[ct]));
-                    gP[ct] += (s[0] * d[0] + s[1] * d[1]) + (s[2] * d[2] + s[3] * d[3]);
-                    d = mfma(gt, rs[ct].l, mfma(gt, rs[ct].h, d * o32[ct]));
-                }
-            }
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const Op2 s = split8(Sn[ks & 1][ct][0], Sn[ks & 1][ct][1]);
-#pragma unroll
-                for (int z = 0; z < 2; ++z) X[z][ct] = mfma(ga[z], s.l, mfma(ga[z], s.h, X[z][ct]));
-            }
-            if (ks + 2 < KS) fetch_state(c, ks + 2, Sn[ks & 1]);
-        }
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const bf16x8 rT = ld_tra<A::ROW>(xt + A::R + 32 * (CT * q + ct)), kT = ld_tra<A::ROW>(xt + A::K + 32 * (CT * q + ct));
-            const f32x4 vg0 = lds_ld<f32x4>(xs + A::VG), vg1 = lds_ld<f32x4>(xs + A::VG + 64);
-            float r[8], k[8], ps[8], pf[8], pm[8];
-            unpack(rT, r); unpack(kT, k);
-            Op2 ko[2];
-            from_ref(ct, pm);
-            tile_operands(ct, false, kT, pm, ko);
-            to_ref(ct, pf);
-            from_start(ct, ps);
-            const float th = hide(t0);
-#pragma unroll
-            for (int z = 0; z < 2; ++z) {
-                const f32x4 tx = mm3(ca[z], ko[z], ZERO4);
-                f32x4 o;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int e = 4 * z + v;
-                    const float x = X[z][ct][v] * ps[e], ti = tx[v] * pf[e], vg = z ? vg1[v] : vg0[v], t = th + static_cast<float>(16 * z + v);
-                    gw[ct] = fmaf(r[e] * t, x, gw[ct]);
-                    o[v] = fmaf(k[e] * vg, u[ct], x + ti);
-                }
-                store_tile(gr_, to + 32 * z * C + 32 * ct, C, l16, o);
-            }
-        }
+        second(odd_, c, part, Sn);
         __syncthreads();
     };
     __syncthreads();                                     // the top chunk is there
+    __syncthreads();                                     // and its tile B
     for (int c = nch - 1; c >= 0; c -= 2) {
         chunk(std::true_type{}, c);
         chunk(std::false_type{}, c - 1);
     }
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        const int c = h * HN + 16 * (CT * q + ct) + l16;
-        const float sw = allreduce_rows(fmaf(32.f * o32[ct], gP[ct], gw[ct])), su = allreduce_rows(gu[ct]);
-        if (g == 0) {
-            p.gw[static_cast<size_t>(b) * C + c] = f2bf(l[ct] * sw);
-            p.gu[static_cast<size_t>(b) * C + c] = f2bf(su);
-        }
+    const int c = h * HN + 16 * q + l16;
+    const float sw = allreduce_rows(fmaf(32.f * o32, gP, gw)), su = allreduce_rows(gu);
+    if (g == 0) {
+        p.gw[static_cast<size_t>(b) * C + c] = f2bf(l * sw);
+        p.gu[static_cast<size_t>(b) * C + c] = f2bf(su);
     }
 }
 
 template <int HN> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, size_t base, int nch) {
     using A = G<HN>;
-    constexpr int CT = A::CT, KS = A::KS, NP = A::PASSES;
-    const int q = __builtin_amdgcn_readfirstlane(te >> 6), lane = te & 63, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
-    const int row0 = te / A::PIECES, c8 = (te % A::PIECES) * 8, to = tile_offset(l16, g, C);
-    float cke[2][KS][8];                                 // o^{31-t} of token 16 tt + l16, channel 32 ks + 8 g + e
+    constexpr int KS = A::KS, PARTS = A::PARTS;
+    const int w = __builtin_amdgcn_readfirstlane(te >> 6), lane = te & 63, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    const int row0 = te / A::PIECES, c8 = (te % A::PIECES) * 8;
+    // gv: value channels 32 wq .. + 31, tokens 16 wz .. + 15; tile A: channels 32 part .., the quadrant across the halves or the others
+    const int wq = w >> 1, wz = w & 1, part = w % PARTS;
+    const bool across = w >= PARTS;
+    const int form = PARTS > 2 ? w - PARTS : (w == 0 ? 1 : (w == 1 ? -1 : 2 * (w - 2)));       // of tile B: 0 as it is, 1 weighted, 2 transposed
+    float cke[KS][8];                                    // o^{31-t} of token 16 wz + l16, channel 32 ks + 8 g + e
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) cke[ks][e] = wpow(lds_f(sb + A::LAM + 4 * (32 * ks + 8 * g + e)), 31 - 16 * wz - l16);
+    float px[8], py[8];                                  // tile A: as sink and as source, see TilePowers
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const float l = lds_f(sb + A::LAM + 4 * (32 * ks + 8 * g + e));
-            cke[0][ks][e] = wpow(l, 31 - l16); cke[1][ks][e] = wpow(l, 15 - l16);
-        }
+        const float l = lds_f(sb + A::LAM + 4 * (32 * part + 8 * g + e));
+        px[e] = wpow(l, across ? l16 : l16 - 8); py[e] = wpow(l, across ? 15 - l16 : 7 - l16);
     }
-    TilePowers tp;
-    tile_powers(tp, sb + A::LAM + 4 * (32 * (q % A::PARTS) + 8 * g), l16);
-    auto fetch = [&](const int c, uint4 (&d)[4][NP]) __attribute__((always_inline)) {
+    auto fetch = [&](const int c, uint4 (&d)[4]) __attribute__((always_inline)) {
         const int cc = max(c, 0);
         const size_t o = base + static_cast<size_t>(cc) * L * C;
-        const int left = T - cc * L;
+        const int left = T - cc * L, lo = 2 * (row0 * C + c8);
         const rows_t r = rows_of(p.r + o, left, C), k = rows_of(p.k + o, left, C), v = rows_of(p.v + o, left, C), gy = rows_of(p.gy + o, left, C);
-#pragma unroll
-        for (int z = 0; z < NP; ++z) {
-            const int lo = 2 * ((row0 + z * A::ROWS) * C + c8);
-            d[0][z] = load16(r, lo); d[1][z] = load16(k, lo); d[2][z] = load16(v, lo); d[3][z] = load16(gy, lo);
-        }
+        d[0] = load16(r, lo); d[1] = load16(k, lo); d[2] = load16(v, lo); d[3] = load16(gy, lo);
     };
-    auto put = [&](const int sl, const uint4 (&d)[4][NP]) __attribute__((always_inline)) {
+    auto put = [&](const int sl, const uint4 (&d)[4]) __attribute__((always_inline)) {
         const lds_t s = sb + A::BASE + sl * A::SLOT;
         const f32x4 u[2] = {lds_ld<f32x4>(sb + A::U + 4 * c8), lds_ld<f32x4>(sb + A::U + 4 * c8 + 16)};      // (registers for these across the loop would spill others)
+        const lds_t o = s + row0 * A::ROW + 2 * c8;
 #pragma unroll
-        for (int z = 0; z < NP; ++z) {
-            const int t = row0 + z * A::ROWS;
-            const lds_t o = s + t * A::ROW + 2 * c8;
+        for (int i = 0; i < 4; ++i) lds_st<bf16x8>(o + i * A::PLANE, op4(d[i]));
+        float r[8], k[8], v[8], gy[8], a = 0.f, b = 0.f;
+        unpack8(d[0], r); unpack8(d[1], k); unpack8(d[2], v); unpack8(d[3], gy);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) lds_st<bf16x8>(o + i * A::PLANE, op4(d[i][z]));
-            float r[8], k[8], v[8], gy[8], a = 0.f, b = 0.f;
-            unpack8(d[0][z], r); unpack8(d[1][z], k); unpack8(d[2][z], v); unpack8(d[3][z], gy);
+        for (int e = 0; e < 8; ++e) { a = fmaf(r[e] * u[e >> 2][e & 3], k[e], a); b = fmaf(v[e], gy[e], b); }
+        a = lanes_sum<A::PIECES>(a); b = lanes_sum<A::PIECES>(b);
+        if (c8 == 0) { lds_st<float>(s + A::RUK + 4 * row0, a); lds_st<float>(s + A::VG + 4 * row0, b); }
+    };
+    // the three forms of tile B of the chunk in a slot, one a wave, by those that have less to do for tile A before others
+    auto tile_b = [&](const int sl) __attribute__((always_inline)) {
+        if (form < 0 || form > 2) return;
+        const int lane = static_cast<int>(lane_now()), l16 = lane & 15, g = lane >> 4;
+        lds_t xr = sb + A::BASE + sl * A::SLOT + l16 * A::ROW + 16 * g;
+        opaque(xr);
+        const lds_t out = sb + A::BTILE;
+        const bool transposed = form == 2;
+        const lds_t rows = xr + (transposed ? A::V : A::GY), cols = xr + (transposed ? A::GY : A::V);
+        const lds_t row1 = rows + (transposed ? 0 : 16 * A::ROW), col1 = cols + (transposed ? 16 * A::ROW : 0);       // (the quadrant across the halves)
+        f32x4 t[3] = {ZERO4, ZERO4, ZERO4};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) { a = fmaf(r[e] * u[e >> 2][e & 3], k[e], a); b = fmaf(v[e], gy[e], b); }
-            a = lanes_sum<A::PIECES>(a); b = lanes_sum<A::PIECES>(b);
-            if (c8 == 0) { lds_st<float>(s + A::RUK + 4 * t, a); lds_st<float>(s + A::VG + 4 * t, b); }
+        for (int ks = 0; ks < KS; ++ks) {
+            t[0] = mfma(ld_op(rows + 64 * ks), ld_op(cols + 64 * ks), t[0]);
+            t[1] = mfma(ld_op(row1 + 64 * ks), ld_op(col1 + 64 * ks), t[1]);
+            t[2] = mfma(ld_op(rows + 16 * A::ROW + 64 * ks), ld_op(cols + 16 * A::ROW + 64 * ks), t[2]);
+        }
+        if (transposed) {
+            mask<true>(t, l16, g);
+            put_tile<true>(out + 2 * 3072, t, lane);
+            return;
+        }
+        mask<false>(t, l16, g);
+        if (form == 0) put_tile<false>(out, t, lane);
+        else {                                           // weighted with the tokens between, for the decay gradient
+            const float lag = static_cast<float>(4 * g - (l16 + 1));
+#pragma unroll
+            for (int z = 0; z < 3; ++z)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) t[z][v] *= lag + static_cast<float>(16 * (Quad<false>::ROWT[z] - Quad<false>::LANET[z]) + v);
+            put_tile<false>(out + 3072, t, lane);
         }
     };
-    uint4 ring[2][4][NP];
-    {
-        uint4 top[4][NP];
-        fetch(nch - 1, top);
-        fetch(nch - 2, ring[0]);                         // chunk c rides in ring[c & 1]
-        fetch(nch - 3, ring[1]);
-        put(1, top);
-    }
+    uint4 next[4];                                       // a chunk ahead of its way to LDS
+    fetch(nch - 1, next);
+    put(1, next);
+    fetch(nch - 2, next);
     auto chunk = [&](auto odd_, const int c) __attribute__((always_inline)) {
         constexpr bool ODD = decltype(odd_)::value;
         constexpr int PREV = ODD ? 0 : 1;
         const lds_t sx = sb + A::BASE + (ODD ? A::SLOT : 0);
         // ---- first half
-        if (q < A::PARTS) {
-            lds_t o = sx + l16 * A::ROW + 64 * q + 16 * g;
+        {
+            const int lane = static_cast<int>(lane_now()), l16 = lane & 15, g = lane >> 4;
+            lds_t o = sx + l16 * A::ROW + 64 * part + 16 * g;
             opaque(o);
-            const bf16x8 r[2] = {ld_op(o + A::R), ld_op(o + A::R + 16 * A::ROW)}, k[2] = {ld_op(o + A::K), ld_op(o + A::K + 16 * A::ROW)};
-            f32x4 qd[3];
-            raw_part<false>(r, k, tp, qd);
-            const float diag[2] = {q == 0 ? lds_f(sx + A::RUK + 4 * l16) : 0.f, q == 0 ? lds_f(sx + A::RUK + 4 * (16 + l16)) : 0.f};
-            put_part<false>(sb + A::BPART + q * A::PART, qd, diag, lane);
+            const lds_t out = sb + A::BPART + part * A::PART;
+            if (across) {
+                const Op2 x = scaled(ld_op(o + A::R + 16 * A::ROW), px), y = scaled(ld_op(o + A::K), py);
+                put_quad<false, 1>(out, mm3(x, y, ZERO4), 0.f, lane);
+            } else {
+#pragma unroll
+                for (int z = 0; z < 2; ++z) {
+                    const Op2 x = scaled(ld_op(o + A::R + 16 * z * A::ROW), px), y = scaled(ld_op(o + A::K + 16 * z * A::ROW), py);
+                    const float diag = part == 0 ? lds_f(sx + A::RUK + 4 * (16 * z + l16)) : 0.f;
+                    if (z == 0) put_quad<false, 0>(out, mm3(x, y, ZERO4), diag, lane);
+                    else put_quad<false, 2>(out, mm3(x, y, ZERO4), diag, lane);
+                }
+            }
         }
-        put(PREV, ring[PREV]);                           // (chunk 0: rows that nobody reads)
-        fetch(c - 3, ring[PREV]);
+        put(PREV, next);                                 // (chunk 0: rows that nobody reads)
+        fetch(c - 2, next);
         __syncthreads();
         // ---- second half: gv
-        lds_t xo = sx + l16 * A::ROW + 16 * g, ht = sb + A::DSH + (8 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3) + 32 * CT * q;
-        lds_t xt = sx + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3) + 32 * CT * q;
+        const int lane = static_cast<int>(lane_now()), l16 = lane & 15, g = lane >> 4, to = tile_offset(l16, g, C);
+        lds_t xo = sx + (16 * wz + l16) * A::ROW + 16 * g, ht = sb + A::DSH + (8 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3) + 64 * wq;
+        lds_t xt = sx + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3) + 64 * wq;
         opaque(xo); opaque(ht); opaque(xt);
-        f32x4 O[2][CT];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) { O[0][ct] = ZERO4; O[1][ct] = ZERO4; }
+        f32x4 O[2] = {ZERO4, ZERO4};
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            const Op2 ke[2] = {scaled(ld_op(xo + A::K + 64 * ks), cke[0][ks]), scaled(ld_op(xo + A::K + 16 * A::ROW + 64 * ks), cke[1][ks])};
+            const Op2 ke = scaled(ld_op(xo + A::K + 64 * ks), cke[ks]);
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
+            for (int ct = 0; ct < 2; ++ct) {
                 const Op2 s = {ld_tr(ht + 32 * ks * A::ROW + 32 * ct, A::ROW), ld_tr(ht + (A::DSL - A::DSH) + 32 * ks * A::ROW + 32 * ct, A::ROW)};
-#pragma unroll
-                for (int z = 0; z < 2; ++z) O[z][ct] = mm3(ke[z], s, O[z][ct]);
+                O[ct] = mm3(ke, s, O[ct]);
             }
         }
-        Op2 at[2];
-        take_parts<false, A::PARTS, A::PART>(sb + A::BPART, lane, at);
-        const rows_t out = rows_of(p.gv + base + static_cast<size_t>(c) * L * C + 16 * CT * q, T - c * L, C);
+        const Op2 at = wz ? take_lane_tile<PARTS, A::PART, 1>(sb + A::BPART, lane) : take_lane_tile<PARTS, A::PART, 0>(sb + A::BPART, lane);
+        const rows_t out = rows_of(p.gv + base + static_cast<size_t>(c) * L * C + 32 * wq, T - c * L, C);
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
+        for (int ct = 0; ct < 2; ++ct) {
             const bf16x8 go = ld_tra<A::ROW>(xt + A::GY + 32 * ct);
-#pragma unroll
-            for (int z = 0; z < 2; ++z) {
-                const f32x4 o = mfma(at[z].l, go, mfma(at[z].h, go, O[z][ct]));
-                store_tile(out, to + 32 * z * C + 32 * ct, C, l16, o);
-            }
+            store_tile(out, to + 32 * wz * C + 32 * ct, C, l16, mfma(at.l, go, mfma(at.h, go, O[ct])));
         }
+        tile_b(PREV);
         __syncthreads();
     };
+    __syncthreads();
+    tile_b(1);
     __syncthreads();
     for (int c = nch - 1; c >= 0; c -= 2) {
         chunk(std::true_type{}, c);
@@ -784,7 +825,7 @@ template <int HN> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, size_t ba
 }
 
 template <int HN>
-__global__ __launch_bounds__(NTH, 2) void wkv5b_bwd(const ArgsW p) {
+__global__ __launch_bounds__(8 * HN, HN / 32) void wkv5b_bwd(const ArgsW p) {
     const lds_t sb = lds_of(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = 2 * ((p.T + 2 * L - 1) / (2 * L));      // whole pairs (a last chunk without tokens adds zeros)
@@ -792,16 +833,16 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_bwd(const ArgsW p) {
     if ((HN == 64 && !strong_layer(p.w, p.C, tid & 63)) || steps_head<false, HN>(p.w, nullptr, h * HN)) return;
     head_setup<HN>(p, sb, h, b, tid);
     __syncthreads();
-    if (w < 4) role_d<HN>(p, sb, w, tid & 63, h, b, base, nch);
-    else role_e<HN>(p, sb, tid - 256, base, nch);
+    if (w < HN / 16) role_d<HN>(p, sb, w, tid & 63, h, b, base, nch);
+    else role_e<HN>(p, sb, tid - 4 * HN, base, nch);
 }
 
-template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, uint32_t lds) {
+template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, int threads, uint32_t lds) {
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); e != hipSuccess) {
         g_last_hip_error = static_cast<int>(e);
         return RWKV_ERR_LAUNCH;
     }
-    hipLaunchKernelGGL(kernel, dim3(B * p.H), dim3(NTH), lds, st, p);
+    hipLaunchKernelGGL(kernel, dim3(B * p.H), dim3(threads), lds, st, p);
     return launch_status();
 }
 
@@ -815,14 +856,14 @@ int launch_wkv5b_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t*
                      const uint16_t* u, uint16_t* y, float* decay, float* saved) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.decay = decay; p.saved = saved;
-    return C == H * 64 ? launch(wkv5b_fwd<64>, st, B, p, G<64>::FTOTAL) : launch(wkv5b_fwd<128>, st, B, p, G<128>::FTOTAL);
+    return C == H * 64 ? launch(wkv5b_fwd<64>, st, B, p, NTH, G<64>::FTOTAL) : launch(wkv5b_fwd<128>, st, B, p, NTH, G<128>::FTOTAL);
 }
 int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
                      const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu, const float* saved) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv; p.gw = gw; p.gu = gu;
     p.saved = const_cast<float*>(saved);
-    return C == H * 64 ? launch(wkv5b_bwd<64>, st, B, p, G<64>::BTOTAL) : launch(wkv5b_bwd<128>, st, B, p, G<128>::BTOTAL);
+    return C == H * 64 ? launch(wkv5b_bwd<64>, st, B, p, 512, G<64>::BTOTAL) : launch(wkv5b_bwd<128>, st, B, p, 1024, G<128>::BTOTAL);
 }
 
 }  // namespace rwkv
