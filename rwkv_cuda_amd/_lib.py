@@ -165,10 +165,14 @@ SIGNATURES = {
     "rwkv_wkv5a_backward_ex": (_I, [_P, _I, _I, _I, _I] + [_P] * 17 + [_U]),
     "rwkv_wkv5f32s_saved_bytes": (_Z, [_I, _I, _I, _I]),
     "rwkv_wkv5f32s_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 6 + [_P, _Z]),
+    "rwkv_wkv5f32s_forward_workspace_bytes": (_Z, [_I, _I, _I, _I]),
+    "rwkv_wkv5f32s_forward_ws": (_I, [_P, _I, _I, _I, _I] + [_P] * 6 + [_P, _Z, _P, _Z]),
     "rwkv_wkv5f32s_backward_workspace_bytes": (_Z, [_I, _I, _I, _I]),
     "rwkv_wkv5f32s_backward": (_I, [_P, _I, _I, _I, _I] + [_P] * 11 + [_P, _Z, _P, _Z]),
     "rwkv_wkv5as_saved_bytes": (_Z, [_I, _I, _I, _I]),
     "rwkv_wkv5as_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 8 + [_P, _Z]),
+    "rwkv_wkv5as_forward_workspace_bytes": (_Z, [_I, _I, _I, _I]),
+    "rwkv_wkv5as_forward_ws": (_I, [_P, _I, _I, _I, _I] + [_P] * 8 + [_P, _Z, _P, _Z]),
     "rwkv_wkv5as_backward_workspace_bytes": (_Z, [_I, _I, _I, _I]),
     "rwkv_wkv5as_backward": (_I, [_P, _I, _I, _I, _I] + [_P] * 15 + [_P, _Z, _P, _Z]),
     "rwkv_wkv6_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 6),

@@ -160,7 +160,9 @@ struct Wkv5F32 : Function<Wkv5F32> {
         if (chunked) {
             const size_t n = grad ? rwkv_wkv5f32s_saved_bytes(d.B, d.T, d.C, d.H) : 0;
             const Tensor saved = grad ? bytes(r, n) : Tensor();
-            ok(rwkv_wkv5f32s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(saved), n));
+            const size_t nw = rwkv_wkv5f32s_forward_workspace_bytes(d.B, d.T, d.C, d.H);
+            const Tensor ws = nw > 0 ? bytes(r, nw) : Tensor();
+            ok(rwkv_wkv5f32s_forward_ws(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(saved), n, P(ws), nw));
             if (grad) ctx->save_for_backward({r, k, v, w, u, saved});
         } else {
             const Tensor ew = w.exp().neg_(), eew = ew.exp();
@@ -213,7 +215,9 @@ struct Wkv5A : Function<Wkv5A> {
         if (chunked) {
             const size_t n = grad ? rwkv_wkv5as_saved_bytes(d.B, d.T, d.C, d.H) : 0;
             const Tensor saved = grad ? bytes(r, n) : Tensor();
-            ok(rwkv_wkv5as_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w1), P(u1), P(w2), P(u2), P(y), P(saved), n));
+            const size_t nw = rwkv_wkv5as_forward_workspace_bytes(d.B, d.T, d.C, d.H);
+            const Tensor ws = nw > 0 ? bytes(r, nw) : Tensor();
+            ok(rwkv_wkv5as_forward_ws(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w1), P(u1), P(w2), P(u2), P(y), P(saved), n, P(ws), nw));
             if (grad) ctx->save_for_backward({r, k, v, w1, u1, w2, u2, saved});
         } else {
             const Tensor ew1 = w1.exp().neg_(), eew1 = ew1.exp(), ew2 = w2.exp().neg_(), eew2 = ew2.exp();

@@ -213,12 +213,12 @@ int launch_wkv5_bwd_b_split(hipStream_t st, int cross, int B, int T, int C, int 
                             const uint16_t* v, const float* ew, const uint16_t* u, const uint16_t* gy, float* gk32, float* gv32,
                             float* gw32, const float* rdr);
 // wkv56.hip: the heads of an fp32 wkv5 (wkv5a: w2, u2 not null) layer of 64-channel heads that the chunked kernels leave out; gw, gu,
-// gw2, gu2: per-batch rows [B][C]
+// gw2, gu2: per-batch rows [B][C]; flags (may be null): a word per (batch, head) that says so instead of the decays and marks
 int launch_wkv5f32_steps_fwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
-                             const float* u, const float* w2, const float* u2, float* y);
+                             const float* u, const float* w2, const float* u2, float* y, const int* flags = nullptr);
 int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
                              const float* u, const float* w2, const float* u2, const float* gy, float* gr, float* gk, float* gv,
-                             float* gw, float* gu, float* gw2, float* gu2);
+                             float* gw, float* gu, float* gw2, float* gu2, const int* flags = nullptr);
 
 // wkv5_bf.hip: wkv5, bf16, heads of 128 or 64 channels, whole heads; w raw.  Size 64: only layers with a
 // strong decay (strong_layer), the others belong to the one-sweep kernels above and the launch returns at once.

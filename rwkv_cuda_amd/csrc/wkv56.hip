@@ -834,9 +834,10 @@ __global__ __launch_bounds__((RowGeom<NP, PARTS>::NTHREADS)) void wkv_rows(const
 // bf16, heads of 64, in a layer without a strong decay: the heads that a one-sweep kernel has given up (its flag words, of the
 // forward and in the backward of both directions: such a forward has left no states).
 // fp32: also the heads whose inputs are not all finite, which the chunked kernels mark by a NaN in the first element of each output
-// (wkv5_f32.hip); out: the one that this workgroup would write.
+// (wkv5_f32.hip); out: the one that this workgroup would write.  With sequences cut into blocks of time a word per head says which.
 template <int NP, bool F32, bool TWO> DEVINL bool steps_for(const Args& a, const uint16_t* out) {
     if constexpr (F32) {
+        if (a.flags != nullptr) return a.flags[blockIdx.x] != 0;
         const size_t first = static_cast<size_t>(blockIdx.x / a.H) * a.T * a.C + static_cast<size_t>(blockIdx.x % a.H) * NP;
         const float x = reinterpret_cast<const float*>(out)[first];
         __syncthreads();                                 // all waves have it before one of them writes
@@ -1054,8 +1055,9 @@ uint16_t* out_elems(float* p) { return reinterpret_cast<uint16_t*>(p); }
 }  // namespace
 
 int launch_wkv5f32_steps_fwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
-                             const float* u, const float* w2, const float* u2, float* y) {
+                             const float* u, const float* w2, const float* u2, float* y, const int* flags) {
     Args a{};
+    a.flags = flags;
     a.T = T; a.C = H * N; a.H = H; a.r = as_elems(r); a.k = as_elems(k); a.v = as_elems(v); a.w = w; a.u = as_elems(u); a.w2 = w2;
     a.u2 = as_elems(u2); a.y = out_elems(y);
     const auto kernel = w2 != nullptr ? wkv5_steps_fwd<true, true> : wkv5_steps_fwd<true, false>;
@@ -1085,8 +1087,9 @@ int launch_wkv5_steps_bwd(hipStream_t st, int B, int T, int C, int H, const uint
 }  // namespace
 int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r, const float* k, const float* v, const float* w,
                              const float* u, const float* w2, const float* u2, const float* gy, float* gr, float* gk, float* gv,
-                             float* gw, float* gu, float* gw2, float* gu2) {
+                             float* gw, float* gu, float* gw2, float* gu2, const int* flags) {
     Args a{};
+    a.flags = flags;
     a.T = T; a.C = H * N; a.H = H; a.r = as_elems(r); a.k = as_elems(k); a.v = as_elems(v); a.w = w; a.u = as_elems(u); a.w2 = w2;
     a.u2 = as_elems(u2); a.gy = as_elems(gy); a.gr = out_elems(gr); a.gk = out_elems(gk); a.gv = out_elems(gv); a.gw = out_elems(gw);
     a.gu = out_elems(gu); a.gw2 = out_elems(gw2); a.gu2 = out_elems(gu2);

@@ -75,7 +75,31 @@ struct ArgsC {
     float *y, *gr, *gk, *gv;
     float *gw, *gu, *gw2, *gu2;                         // per-batch rows [B][C]
     float* saved;                                       // [B*H][segments][i][j]
+    // sequences cut into blocks of time (NB > 1): blocks of `per` segments, a workgroup each; what each block leaves of a state that
+    // entered it empty, [B*H][NB - 1][64][64] (the last block's is not needed, in the backward the first's); heads for the step kernels
+    int B, NB, per;
+    float* local;
+    int* flags;
 };
+
+// The workgroup's head and its part of the sequence: chunks first .. first + chunks - 1, tokens that are left from there on.
+template <bool TWO> struct Part {
+    int h, b, n, first, chunks, left;
+    size_t bh, base;
+};
+template <bool TWO> DEVINL Part<TWO> part_of(const ArgsC& p) {
+    Part<TWO> x;
+    const int BH = p.B * p.H, nch = (p.T + L - 1) / L;
+    // (divisions are done in vector registers)
+    x.n = __builtin_amdgcn_readfirstlane(p.NB > 1 ? static_cast<int>(blockIdx.x) / BH : 0);
+    x.bh = blockIdx.x - x.n * BH;
+    x.b = __builtin_amdgcn_readfirstlane(static_cast<int>(x.bh) / p.H); x.h = static_cast<int>(x.bh) - x.b * p.H;
+    x.first = x.n * p.per * SEG<TWO>;
+    x.chunks = p.NB > 1 ? min(p.per * SEG<TWO>, nch - x.first) : nch;
+    x.left = p.T - x.first * L;
+    x.base = (static_cast<size_t>(x.b) * p.T + static_cast<size_t>(x.first) * L) * p.C + static_cast<size_t>(x.h) * N;
+    return x;
+}
 
 // e^{lam n} for a small integer n, exact to fp32 rounding: the product and the base-2 exponent carry their rounding errors along
 DEVINL float wpow(float lam, float n) {
@@ -97,7 +121,14 @@ DEVINL float row_sum(float x) {
     return x;
 }
 
-struct Head { float lam[N], lam2[N], u[N], u2[N], dec[N], dec2[N]; };
+// The lane's number, worked out where it is used: what is derived from threadIdx is kept in registers, or spilled, across a loop.
+DEVINL uint32_t lane_now() {
+    uint32_t all = ~0u;
+    asm volatile("" : "+s"(all));
+    return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
+}
+
+struct Head { float lam[N], lam2[N], u[N], u2[N], dec[N], dec2[N], blk[N], blk2[N]; };      // decays of a chunk, of a block of time
 
 // whether any element is no number, or infinite
 DEVINL bool not_finite(const f32x4& a, const f32x4& b, const f32x4& c, const f32x4& d = ZERO4) {
@@ -106,7 +137,7 @@ DEVINL bool not_finite(const f32x4& a, const f32x4& b, const f32x4& c, const f32
     for (int e = 0; e < 4; ++e) s = fmaf(a[e], 0.f, fmaf(b[e], 0.f, fmaf(c[e], 0.f, fmaf(d[e], 0.f, s))));
     return s != 0.f;
 }
-// the mark, by the lane that has written this element before
+// the mark, by the lane that has written this element before; in blocks of time a word of the head's own, as other workgroups write that
 DEVINL void mark(float* first) { *first = __builtin_nanf(""); }
 
 // the head's parameters into LDS (by the first wave); every wave finds out for itself whether a decay is strong
@@ -119,6 +150,8 @@ template <bool TWO> DEVINL bool head_setup(Head& hd, const ArgsC& p, int h, int 
     if (tid < N) {
         hd.lam[lane] = l1; hd.dec[lane] = wpow(l1, L); hd.u[lane] = p.u[c];
         hd.lam2[lane] = l2; hd.dec2[lane] = wpow(l2, L); hd.u2[lane] = TWO ? p.u2[c] : 0.f;
+        const float len = static_cast<float>(p.per * SEG<TWO> * L);
+        hd.blk[lane] = wpow(l1, len); hd.blk2[lane] = wpow(l2, len);
     }
     return __builtin_amdgcn_readfirstlane(mn < LAM_STRONG ? 1 : 0) != 0;
 }
@@ -165,6 +198,112 @@ DEVINL void store_rows(float* out, int lo, int C, int left, bool whole, const f3
     }
 }
 
+// where the states of the part's segments are
+template <bool TWO> DEVINL float* saved_state(const ArgsC& p, const Part<TWO>& x) {
+    const size_t nch = (p.T + L - 1) / L, nseg = (nch + SEG<TWO> - 1) / SEG<TWO>;
+    return p.saved + (x.bh * nseg + x.first / SEG<TWO>) * N * N;
+}
+
+// step(the lane's sixteen elements of a block's state) for n blocks' states, `next` floats apart; four are under way at once
+template <class F> DEVINL void add_up(const float* x, int next, int n, const F& step) {
+    f32x4 y[4][4];
+    int m = 0;
+    for (; m + 4 <= n; m += 4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i, x += next)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) y[i][t] = ld4(x + 16 * t);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) step(y[i]);
+    }
+#pragma unroll 1
+    for (; m < n; ++m, x += next) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) y[0][t] = ld4(x + 16 * t);
+        step(y[0]);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------- blocks of time, first pass
+// What a block leaves of an empty state: sum over its tokens of v_t k_t^T with the decay that is left to the block's end, or (REV) from
+// the end backwards what the gradient state takes up, gy_t r_t^T.  Both are E[outer][inner] = sum_t Y_t[outer] X_t[inner] o^{15 - t} in
+// chunks whose tokens are counted in the direction of travel; forward X = k, Y = v, backward X = gy, Y = r, so that a lane holds the
+// element order of the state in the kernels that follow.  A workgroup makes 16 of the 64 outer channels, its waves a quarter of the
+// block each, added up at the end.  Operands come from memory as the matrix instruction takes them.
+template <bool TWO, bool REV>
+__global__ __launch_bounds__(256) void wkv5c_local(const ArgsC p) {
+    __shared__ f32x4 part[4][4][64];
+    const int tid = threadIdx.x, lane = tid & 63, z = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
+    const int q = blockIdx.x & 3, BH = p.B * p.H, m = (blockIdx.x >> 2) / BH, bh = (blockIdx.x >> 2) - m * BH, b = bh / p.H, h = bh - b * p.H, C = p.C;
+    const bool steps = steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, h * N);
+    if (m == 0 && q == 0 && tid == 0) p.flags[bh] = steps;
+    if (steps) return;
+    const float* const wx = REV ? (TWO ? p.w2 : nullptr) : p.w;
+    const float* const wy = REV ? p.w : (TWO ? p.w2 : nullptr);
+    const int n = REV ? m + 1 : m, nch = (p.T + L - 1) / L, first = n * p.per * SEG<TWO>, chunks = min(p.per * SEG<TWO>, nch - first), per = (chunks + 3) / 4;
+    auto log_decay = [&](const float* w, int c) __attribute__((always_inline)) { return w != nullptr ? -expf(w[h * N + c]) : 0.f; };
+    const int own = 16 * q + l16;
+    const float ly = log_decay(wy, own), dy = wpow(ly, L);
+    float px[4][4], py[4];                               // token 4 s + g, inner channel 16 t + l16
+    F4 dx[4];                                            // o^16 of inner channel 16 t + 4 g + v
+    float lx[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const float l = log_decay(wx, 16 * t + l16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            px[t][e] = wpow(l, static_cast<float>(15 - 4 * e - g));
+            lx[t][e] = log_decay(wx, 16 * t + 4 * g + e);
+            dx[t][e] = wpow(lx[t][e], L) * dy;
+        }
+        py[t] = wpow(ly, static_cast<float>(15 - 4 * t - g));
+    }
+    const float* const X = (REV ? p.gy : p.k) + static_cast<size_t>(b) * p.T * C + h * N;
+    const float* const Y = (REV ? p.r : p.v) + static_cast<size_t>(b) * p.T * C + h * N;
+    const int c0 = min(z * per, chunks), c1 = min(c0 + per, chunks);        // counted in the direction of travel
+    struct Rows { float x[4][4], y[4]; };
+    auto fetch = [&](const int i, Rows& d) __attribute__((always_inline)) {
+        const int c = first + (REV ? chunks - 1 - min(i, chunks - 1) : min(i, chunks - 1));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = c * L + (REV ? 15 - 4 * e - g : 4 * e + g);
+            const size_t o = static_cast<size_t>(min(t, p.T - 1)) * C;
+            const bool in = t < p.T;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { const float x = X[o + 16 * k + l16]; d.x[k][e] = in ? x : 0.f; }
+            const float y = Y[o + own];
+            d.y[e] = in ? y : 0.f;
+        }
+    };
+    f32x4 acc[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
+    Rows now, next;
+    fetch(c0, now);
+    for (int i = c0; i < c1; ++i) {
+        fetch(i + 1, next);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4 a = acc[t] * dx[t];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a = mm(now.x[t][e] * px[t][e], now.y[e] * py[e], a);
+            acc[t] = a;
+        }
+        now = next;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) part[z][t][lane] = acc[t];
+    __syncthreads();
+    f32x4 s = part[0][z][lane];                          // inner channels 16 z + 4 g + v
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+        const float len = static_cast<float>(L * (min((i + 1) * per, chunks) - min(i * per, chunks)));
+        f32x4 e;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) e[v] = wpow(z == 0 ? lx[0][v] : (z == 1 ? lx[1][v] : (z == 2 ? lx[2][v] : lx[3][v])), len) * wpow(ly, len);
+        s = s * e + part[i][z][lane];
+    }
+    st4(p.local + (static_cast<size_t>(bh) * (p.NB - 1) + m) * N * N + own * N + 16 * z + 4 * g, s);
+}
+
 // ---------------------------------------------------------------------------------------------------- forward
 // Waves 0..3 (value channels 16 q + l16): St[jt][v] = S[i = 16 q + l16][j = 16 jt + 4 g + v], as it stands the B operand of a
 // contraction over j.  Waves 4..7 load: chunk c + 2 into LDS while chunk c is worked on (three slots, one barrier a chunk),
@@ -182,9 +321,21 @@ struct SmemF {
 constexpr int FDEPTH = 4;
 
 template <bool TWO, bool STRONG>
-DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base, int nch) {
-    const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, const Part<TWO>& part) {
+    const int l16 = lane & 15, g = lane >> 4, T = part.left, C = p.C, nch = part.chunks;
+    const size_t base = part.base;
     const int own = 16 * q + l16;
+    f32x4 St[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
+    if (part.n > 0) {                                    // the state that enters the block, from what the blocks before leave
+        const float* x = p.local + part.bh * (p.NB - 1) * N * N + own * N + 4 * g;
+        const float e2 = TWO ? S.hd.blk2[own] : 1.f;
+        auto step = [&](const f32x4 (&y)[4]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int jt = 0; jt < 4; ++jt) St[jt] = St[jt] * (ld4(&S.hd.blk[16 * jt + 4 * g]) * e2) + y[jt];
+        };
+        add_up(x, N * N, part.n, step);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     // powers: A operands over j (r o1^t, token t = l16; k o1^{15-t}, token 4 g + v), the tile's, the value side's
     F4 crs[4], cke[4], ctx, cty, ct4;
     {
@@ -205,10 +356,10 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base,
         }
     }
     F4 c2s = {}, c2m = {}, c2k = {}, c2e = {};
-    float u2 = 0.f, d2 = 1.f, w24 = 1.f;
+    float u2 = 0.f;
     if constexpr (TWO) {
         const float l = S.hd.lam2[own];
-        u2 = S.hd.u2[own]; d2 = S.hd.dec2[own]; w24 = wpow(l, 4.f);
+        u2 = S.hd.u2[own];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int t = 4 * g + v, m = ref<STRONG>(t);
@@ -230,9 +381,7 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base,
 #pragma unroll
         for (int v = 0; v < 4; ++v) out[4 * g + v][l16] = l16 < 4 * g + v ? acc[v] : 0.f;
     };
-    const int nseg = (nch + SEG<TWO> - 1) / SEG<TWO>;
-    float* const sv = p.saved != nullptr ? p.saved + static_cast<size_t>(blockIdx.x) * nseg * N * N + own * N + 4 * g : nullptr;
-    f32x4 St[4] = {ZERO4, ZERO4, ZERO4, ZERO4};
+    float* const sv = p.saved != nullptr ? saved_state<TWO>(p, part) : nullptr;
     __syncthreads();                                     // chunks 0 and 1 are there
     tile(S.slot[0], S.part[0][q]);
     __syncthreads();
@@ -242,10 +391,11 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base,
         const SlotF& X = S.slot[sl];
         sl = sl == 2 ? 0 : sl + 1;
         if (c + 1 < nch) tile(S.slot[sl], S.part[(c + 1) & 1][q]);
-        if (sv != nullptr && c > 0 && c % SEG<TWO> == 0) {
-            float* d = sv + static_cast<size_t>(c / SEG<TWO>) * N * N;
+        if (sv != nullptr && (c > 0 || part.n > 0) && c % SEG<TWO> == 0) {
+            char* d = reinterpret_cast<char*>(sv + static_cast<size_t>(c / SEG<TWO>) * N * N);
+            const uint32_t me = lane_now(), so = ((16 * q + (me & 15)) * N + 4 * (me >> 4)) * 4;
 #pragma unroll
-            for (int jt = 0; jt < 4; ++jt) st4(d + 16 * jt, St[jt]);
+            for (int jt = 0; jt < 4; ++jt) st4(reinterpret_cast<float*>(d + 64 * jt + so), St[jt]);
         }
         f32x4 y2[2] = {ZERO4, ZERO4};
 #pragma unroll
@@ -262,7 +412,7 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base,
         const f32x4 ruk = ld4(&X.ruk[4 * g]);
         f32x4 y = y2[0] + y2[1];
         if constexpr (TWO) {
-            const f32x4 ap = apply<STRONG>(at, vop * c2k, l16 >= 8 && g < 2, w24);
+            const f32x4 ap = apply<STRONG>(at, vop * c2k, l16 >= 8 && g < 2, STRONG ? wpow(S.hd.lam2[own], 4.f) : 1.f);      // (anew: a register less across the loop)
             y = y * c2s + ap * c2m + vop * (ruk + u2 * ld4(&X.rk[4 * g]));
         } else {
             y += vop * ruk;
@@ -272,6 +422,7 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base,
         float* const out = p.y + base + static_cast<size_t>(c) * L * C;
         store_rows(out, lo, C, T - c * L - 4 * g, c * L + L <= T, y);
         const f32x4 ve = TWO ? vop * c2e : vop;
+        const float d2 = TWO ? S.hd.dec2[own] : 1.f;     // (likewise)
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
             f32x4 acc = St[jt] * ld4(&S.hd.dec[16 * jt + 4 * g]);
@@ -282,16 +433,16 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, size_t base,
         }
         __syncthreads();
     }
-    if (q == 0 && lane == 0 && S.marked) mark(p.y + base);
+    if (q == 0 && lane == 0 && S.marked) { if (p.NB > 1) p.flags[part.bh] = 1; else mark(p.y + base); }
 }
 
 template <bool TWO>
 __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
     __shared__ SmemF S;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = w & 3;
-    const int h = blockIdx.x % p.H, b = blockIdx.x / p.H, T = p.T, C = p.C;
-    const int nch = (T + L - 1) / L;
-    const size_t base = static_cast<size_t>(b) * T * C + static_cast<size_t>(h) * N;
+    const Part<TWO> part = part_of<TWO>(p);
+    const int h = part.h, T = part.left, C = p.C, nch = part.chunks;
+    const size_t base = part.base;
     if (steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, h * N)) return;
     const bool strong = head_setup<TWO>(S.hd, p, h, tid);
     if (tid == 0) S.marked = 0;
@@ -339,8 +490,8 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC p) {
         }
         return;
     }
-    if (strong) fwd_products<TWO, true>(S, p, q, lane, base, nch);
-    else fwd_products<TWO, false>(S, p, q, lane, base, nch);
+    if (strong) fwd_products<TWO, true>(S, p, q, lane, part);
+    else fwd_products<TWO, false>(S, p, q, lane, part);
 }
 
 // ---------------------------------------------------------------------------------------------------- backward
@@ -442,14 +593,16 @@ DEVINL void store_chunk(float* p, size_t base, int c, int g, int own, int C, int
 }
 
 template <bool TWO, bool STRONG>
-DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b, size_t base, int nch) {
+DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, const Part<TWO>& part) {
     constexpr int G = SEG<TWO>;
     using A = At<TWO>;
-    const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = p.T;
+    const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = part.left, nch = part.chunks;
+    const size_t base = part.base;
+    const bool later = part.n > 0;                       // a state enters the first segment
     const uint32_t orow = l16 * ROWB + 16 * g, ocol = 4 * g * ROWB + 4 * own, oall = 4 * g * ROWB + 4 * l16;      // [l16][4 g ..], [4 g + v][own], [4 g + v][l16]
     const uint32_t otr = l16 * TROWB + 16 * g, otc = 4 * g * TROWB + 4 * l16;
     const int nseg = (nch + G - 1) / G;
-    const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * nseg * N * N + 4 * g * N + own;
+    const float* const sv = saved_state<TWO>(p, part) + 4 * g * N + own;
     const float l1 = S.hd.lam[own], u1 = S.hd.u[own], d1 = S.hd.dec[own], w4 = wpow(l1, 4.f);
     F4 cs, ce, cm, ck, tf, tr15, lag;                    // o1^t, o1^{15-t}, o1^{t-m}, o1^{m-1-t}, t, 15 - t for t = 4 g + v; t' - 1 - t for t' = l16
 #pragma unroll
@@ -469,7 +622,7 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
 #pragma unroll
         for (int ib = 0; ib < 4; ++ib)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) Sn[ib][v] = s > 0 ? d[(16 * ib + v) * N] : 0.f;      // the sequence starts from nothing
+            for (int v = 0; v < 4; ++v) Sn[ib][v] = s > 0 || later ? d[(16 * ib + v) * N] : 0.f;      // the sequence starts from nothing
     };
     auto decay = [&](const int ib) __attribute__((always_inline)) {
         if constexpr (TWO) return lds4(hide(16 * g) + A::DEC2 + 64 * ib) * d1;
@@ -537,6 +690,15 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
         if constexpr (TWO) rows(c - 1);                  // (earlier, under the products above, the registers do not reach for this)
     };
     fetch_state(nseg - 1);
+    if (part.n + 1 < p.NB) {                             // the gradient of the state that leaves the block, from what the blocks after take up
+        const float* x = p.local + (part.bh * (p.NB - 1) + p.NB - 2) * N * N + own * N + 4 * g;
+        const float e1 = S.hd.blk[own];
+        auto step = [&](const f32x4 (&y)[4]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib) dS[ib] = dS[ib] * (TWO ? ld4(&S.hd.blk2[16 * ib + 4 * g]) * e1 : f32x4{e1, e1, e1, e1}) + y[ib];
+        };
+        add_up(x, -N * N, p.NB - 1 - part.n, step);
+    }
     hand_over(A::ds(nch - 1) + ocol, dS);
     __syncthreads();                                     // the top chunks are there
     rows(nch - 1);
@@ -578,18 +740,19 @@ DEVINL void role_d(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
     __syncthreads();
     gw = allreduce_rows(gw); gu = allreduce_rows(gu);
     if (g == 0) {
-        const size_t o = static_cast<size_t>(b) * C + h * N + own;
+        const size_t o = (static_cast<size_t>(part.n) * p.B + part.b) * C + part.h * N + own;
         p.gw[o] = l1 * gw;
         p.gu[o] = gu;
     }
-    if (q == 0 && lane == 0 && S.marked) { mark(p.gr + base); mark(p.gk + base); }
+    if (q == 0 && lane == 0 && S.marked) { if (p.NB > 1) p.flags[part.bh] = 1; else { mark(p.gr + base); mark(p.gk + base); } }
 }
 
 template <bool TWO, bool STRONG>
-DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b, size_t base, int nch) {
+DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, const Part<TWO>& part) {
     constexpr int G = SEG<TWO>;
     using A = At<TWO>;
-    const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = p.T;
+    const int l16 = lane & 15, g = lane >> 4, own = 16 * q + l16, C = p.C, T = part.left, nch = part.chunks;
+    const size_t base = part.base;
     const uint32_t orow = l16 * ROWB + 16 * g, ocol = 4 * g * ROWB + 4 * own;                // [l16][4 g ..], [4 g + v][own]
     const uint32_t otr = l16 * TROWB + 16 * g, otc = 4 * g * TROWB + 4 * l16, odt = own * ROWB + 16 * g;
     const int te = 64 * q + lane, row = te >> 4, c4 = (te & 15) * 4;
@@ -711,11 +874,11 @@ DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
         }
     }
     __syncthreads();
-    if (q == 0 && lane == 0 && S.marked) mark(p.gv + base);
+    if (q == 0 && lane == 0 && S.marked && p.NB == 1) mark(p.gv + base);
     if constexpr (TWO) {
         gw2 = allreduce_rows(gw2); gu2 = allreduce_rows(gu2);
         if (g == 0) {
-            const size_t o = static_cast<size_t>(b) * C + h * N + own;
+            const size_t o = (static_cast<size_t>(part.n) * p.B + part.b) * C + part.h * N + own;
 #pragma unroll
             for (int z = 0; z < 4; ++z) gw2 += S.red[z][own];
             p.gw2[o] = l2 * gw2;
@@ -725,35 +888,68 @@ DEVINL void role_e(SmemB<TWO>& S, const ArgsC& p, int q, int lane, int h, int b,
 }
 
 template <bool TWO, bool STRONG>
-DEVINL void bwd_roles(SmemB<TWO>& S, const ArgsC& p, int w, int lane, int h, int b, size_t base, int nch) {
+DEVINL void bwd_roles(SmemB<TWO>& S, const ArgsC& p, int w, int lane, const Part<TWO>& part) {
     const int q = w & 3;
-    if (w < 4) role_d<TWO, STRONG>(S, p, q, lane, h, b, base, nch);
-    else role_e<TWO, STRONG>(S, p, q, lane, h, b, base, nch);
+    if (w < 4) role_d<TWO, STRONG>(S, p, q, lane, part);
+    else role_e<TWO, STRONG>(S, p, q, lane, part);
 }
 
 template <bool TWO>
 __global__ __launch_bounds__(NTB, 2) void wkv5c_bwd(const ArgsC p) {
     SmemB<TWO>& S = *reinterpret_cast<SmemB<TWO>*>(smem_raw);
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = blockIdx.x % p.H, b = blockIdx.x / p.H;
-    const int nch = (p.T + L - 1) / L;
-    const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * N;
-    if (steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, h * N)) return;
-    const bool strong = head_setup<TWO>(S.hd, p, h, tid);
+    const Part<TWO> part = part_of<TWO>(p);
+    if (steps_head<true, N>(p.w, TWO ? p.w2 : nullptr, part.h * N)) return;
+    const bool strong = head_setup<TWO>(S.hd, p, part.h, tid);
     if (tid == 0) S.marked = 0;
     __syncthreads();
-    if (strong) bwd_roles<TWO, true>(S, p, w, lane, h, b, base, nch);
-    else bwd_roles<TWO, false>(S, p, w, lane, h, b, base, nch);
+    if (strong) bwd_roles<TWO, true>(S, p, w, lane, part);
+    else bwd_roles<TWO, false>(S, p, w, lane, part);
 }
 
-// out[c] = sum over the batch of rows of up to four [B][C] arrays that lie behind each other
-__global__ __launch_bounds__(256) void rows_sum(int B, int C, const float* __restrict__ rows, float* o0, float* o1, float* o2, float* o3) {
+// out[c] = sum over blocks and batch of the rows of up to four [NB][B][C] arrays that lie behind each other.  A head that the step kernels
+// have done has its sum in the first of its blocks' rows.
+__global__ __launch_bounds__(256) void rows_sum(int B, int C, int NB, const int* __restrict__ flags, const float* __restrict__ rows, float* o0, float* o1, float* o2, float* o3) {
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
-    const float* x = rows + static_cast<size_t>(blockIdx.y) * B * C + c;
+    const float* x = rows + static_cast<size_t>(blockIdx.y) * NB * B * C + c;
     float s = 0.f;
-    for (int b = 0; b < B; ++b) s += x[static_cast<size_t>(b) * C];
+    for (int b = 0; b < B; ++b) {
+        const int blocks = NB > 1 && flags[b * (C / N) + c / N] == 0 ? NB : 1;
+        float t = 0.f;
+        for (int n = 0; n < blocks; ++n) t += x[(static_cast<size_t>(n) * B + b) * C];
+        s += t;
+    }
     (blockIdx.y == 0 ? o0 : (blockIdx.y == 1 ? o1 : (blockIdx.y == 2 ? o2 : o3)))[c] = s;
+}
+
+// Blocks of time: as many as there is room for on the card at a time (two workgroups a CU in the forward, one in the backward), of
+// BLOCK_SEGS segments at least; 1: whole sequences.  per: segments a block.  Where the line lies, B H sequences, us as they are whole / in
+// blocks: wkv5 forward 8 of T400 41 / 26, of T4096 355 / 62; 64 of T400 42 / 36, of T4096 360 / 146; 128 of T400 43 / 45, of T800 76 / 75, of
+// T4096 358 / 246; 192 (two blocks) of T800 78 / 85, of T4096 360 / 349.  Forward + backward of T4096: 8 sequences 1015 / 129, 32
+// 1022 / 232, 128 1056 / 691; wkv5a 1252 / 160, 1276 / 267, 1301 / 789.  Below some 300 tokens the launch in front takes what the blocks save.
+constexpr int BLOCK_SEGS = 2, SLOTS_FWD = 512, SLOTS_BWD = 256;
+template <bool TWO> int time_blocks(int B, int T, int H, bool bwd, int* per) {
+    const long long bh = static_cast<long long>(B) * H;
+    const int nch = static_cast<int>((static_cast<long long>(T) + L - 1) / L), nseg = (nch + SEG<TWO> - 1) / SEG<TWO>;
+    *per = nseg;
+    const long long want = (bwd ? SLOTS_BWD : SLOTS_FWD) / bh;
+    if (want < (bwd ? 2 : 4) || nch < 16 + bh / 4) return 1;
+    const int least = static_cast<int>((nseg + want - 1) / want);
+    *per = least > BLOCK_SEGS ? least : BLOCK_SEGS;
+    return (nseg + *per - 1) / *per;
+}
+// bytes of the blocks' states and of the heads' words
+size_t blocks_bytes(int B, int H, int NB) {
+    const size_t bh = static_cast<size_t>(B) * H;
+    return NB > 1 ? bh * (NB - 1) * N * N * sizeof(float) + (bh * sizeof(int) + 15) / 16 * 16 : 0;
+}
+template <bool TWO> void set_blocks(ArgsC& p, int B, int NB, int per, void* ws) {
+    p.B = B; p.NB = NB; p.per = per;
+    if (NB > 1) {
+        p.local = static_cast<float*>(ws);
+        p.flags = reinterpret_cast<int*>(p.local + static_cast<size_t>(B) * p.H * (NB - 1) * N * N);
+    }
 }
 
 template <bool TWO> size_t saved_bytes(int B, int T, int C, int H) {
@@ -767,19 +963,47 @@ int check(int B, int T, int C, int H) {
     return RWKV_OK;
 }
 
-template <bool TWO> int start_fwd(void* stream, int B, const ArgsC& p) {
-    hipLaunchKernelGGL(wkv5c_fwd<TWO>, dim3(B * p.H), dim3(NT), 0, static_cast<hipStream_t>(stream), p);
-    return launch_wkv5f32_steps_fwd(static_cast<hipStream_t>(stream), B, p.T, p.H, p.r, p.k, p.v, p.w, p.u, p.w2, p.u2, p.y);
+template <bool TWO> size_t fwd_ws_bytes(int B, int T, int C, int H) {
+    int per;
+    return check(B, T, C, H) == RWKV_OK ? blocks_bytes(B, H, time_blocks<TWO>(B, T, H, false, &per)) : 0;
 }
-template <bool TWO> int start_bwd(void* stream, int B, const ArgsC& p, float* rows, float* gw, float* gu, float* gw2, float* gu2) {
+// per-block and per-batch rows of the parameters' gradients, then what the blocks take
+template <bool TWO> size_t bwd_rows_bytes(int B, int C, int NB) { return ((TWO ? 4 : 2) * static_cast<size_t>(NB) * B * C * sizeof(float) + 15) / 16 * 16; }
+template <bool TWO> size_t bwd_ws_bytes(int B, int T, int C, int H) {
+    if (check(B, T, C, H) != RWKV_OK) return 0;
+    int per;
+    const int NB = time_blocks<TWO>(B, T, H, true, &per);
+    return bwd_rows_bytes<TWO>(B, C, NB) + blocks_bytes(B, H, NB);
+}
+template <bool TWO> int start_fwd(void* stream, int B, ArgsC& p, void* ws, size_t ws_bytes) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    int per = 0, NB = 1;
+    if (ws != nullptr) {
+        if (ws_bytes < fwd_ws_bytes<TWO>(B, p.T, p.C, p.H) || !aligned16(ws)) return RWKV_ERR_WORKSPACE;
+        NB = time_blocks<TWO>(B, p.T, p.H, false, &per);
+    }
+    set_blocks<TWO>(p, B, NB, per, ws);
+    if (NB > 1) hipLaunchKernelGGL((wkv5c_local<TWO, false>), dim3(B * p.H * (NB - 1) * 4), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(wkv5c_fwd<TWO>, dim3(B * p.H * NB), dim3(NT), 0, st, p);
+    return launch_wkv5f32_steps_fwd(st, B, p.T, p.H, p.r, p.k, p.v, p.w, p.u, p.w2, p.u2, p.y, p.flags);
+}
+template <bool TWO> int start_bwd(void* stream, int B, ArgsC& p, void* ws, float* gw, float* gu, float* gw2, float* gu2) {
     static_assert(sizeof(SmemB<TWO>) <= 160 * 1024, "the backward's LDS must fit one CU");
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(wkv5c_bwd<TWO>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        static_cast<int>(sizeof(SmemB<TWO>)));
     if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(wkv5c_bwd<TWO>, dim3(B * p.H), dim3(NTB), sizeof(SmemB<TWO>), st, p);
-    if (int e = launch_wkv5f32_steps_bwd(st, B, p.T, p.H, p.r, p.k, p.v, p.w, p.u, p.w2, p.u2, p.gy, p.gr, p.gk, p.gv, p.gw, p.gu, p.gw2, p.gu2)) return e;
-    hipLaunchKernelGGL(rows_sum, dim3((p.C + 255) / 256, TWO ? 4 : 2), dim3(256), 0, st, B, p.C, rows, gw, gu, gw2, gu2);
+    int per;
+    const int NB = time_blocks<TWO>(B, p.T, p.H, true, &per);
+    const size_t m = static_cast<size_t>(NB) * B * p.C;
+    float* const rows = static_cast<float*>(ws);
+    p.gw = rows; p.gu = rows + m;
+    if constexpr (TWO) { p.gw2 = rows + 2 * m; p.gu2 = rows + 3 * m; }
+    set_blocks<TWO>(p, B, NB, per, static_cast<char*>(ws) + bwd_rows_bytes<TWO>(B, p.C, NB));
+    if (NB > 1) hipLaunchKernelGGL((wkv5c_local<TWO, true>), dim3(B * p.H * (NB - 1) * 4), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(wkv5c_bwd<TWO>, dim3(B * p.H * NB), dim3(NTB), sizeof(SmemB<TWO>), st, p);
+    if (int e = launch_wkv5f32_steps_bwd(st, B, p.T, p.H, p.r, p.k, p.v, p.w, p.u, p.w2, p.u2, p.gy, p.gr, p.gk, p.gv, p.gw, p.gu, p.gw2, p.gu2, p.flags)) return e;
+    hipLaunchKernelGGL(rows_sum, dim3((p.C + 255) / 256, TWO ? 4 : 2), dim3(256), 0, st, B, p.C, NB, p.flags, rows, gw, gu, gw2, gu2);
     return launch_status();
 }
 
@@ -792,22 +1016,24 @@ extern "C" {
 
 size_t rwkv_wkv5f32s_saved_bytes(int B, int T, int C, int H) { return saved_bytes<false>(B, T, C, H); }
 size_t rwkv_wkv5as_saved_bytes(int B, int T, int C, int H) { return saved_bytes<true>(B, T, C, H); }
-size_t rwkv_wkv5f32s_backward_workspace_bytes(int B, int T, int C, int H) {
-    return check(B, T, C, H) == RWKV_OK ? 2 * static_cast<size_t>(B) * C * sizeof(float) : 0;
-}
-size_t rwkv_wkv5as_backward_workspace_bytes(int B, int T, int C, int H) {
-    return check(B, T, C, H) == RWKV_OK ? 4 * static_cast<size_t>(B) * C * sizeof(float) : 0;
-}
+size_t rwkv_wkv5f32s_forward_workspace_bytes(int B, int T, int C, int H) { return fwd_ws_bytes<false>(B, T, C, H); }
+size_t rwkv_wkv5as_forward_workspace_bytes(int B, int T, int C, int H) { return fwd_ws_bytes<true>(B, T, C, H); }
+size_t rwkv_wkv5f32s_backward_workspace_bytes(int B, int T, int C, int H) { return bwd_ws_bytes<false>(B, T, C, H); }
+size_t rwkv_wkv5as_backward_workspace_bytes(int B, int T, int C, int H) { return bwd_ws_bytes<true>(B, T, C, H); }
 
-int rwkv_wkv5f32s_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w,
-                          const float* u, float* y, void* saved, size_t bytes) {
+int rwkv_wkv5f32s_forward_ws(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w,
+                             const float* u, float* y, void* saved, size_t bytes, void* workspace, size_t workspace_bytes) {
     if (int e = check(B, T, C, H)) return e;
     if (int e = check_ptrs({r, k, v, u, y})) return e;
     if (int e = check_ptrs({w}, false)) return e;
     if (saved != nullptr && (bytes < saved_bytes<false>(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.saved = static_cast<float*>(saved);
-    return start_fwd<false>(stream, B, p);
+    return start_fwd<false>(stream, B, p, workspace, workspace_bytes);
+}
+int rwkv_wkv5f32s_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w,
+                          const float* u, float* y, void* saved, size_t bytes) {
+    return rwkv_wkv5f32s_forward_ws(stream, B, T, C, H, r, k, v, w, u, y, saved, bytes, nullptr, 0);
 }
 
 int rwkv_wkv5f32s_backward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w,
@@ -817,17 +1043,16 @@ int rwkv_wkv5f32s_backward(void* stream, int B, int T, int C, int H, const float
     if (int e = check_ptrs({r, k, v, u, gy, gr, gk, gv, gw, gu})) return e;
     if (int e = check_ptrs({w}, false)) return e;
     if (saved == nullptr || bytes < saved_bytes<false>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
-    if (workspace == nullptr || workspace_bytes < rwkv_wkv5f32s_backward_workspace_bytes(B, T, C, H)) return RWKV_ERR_WORKSPACE;
-    float* rows = static_cast<float*>(workspace);
-    const size_t m = static_cast<size_t>(B) * C;
+    if (workspace == nullptr || workspace_bytes < bwd_ws_bytes<false>(B, T, C, H)) return RWKV_ERR_WORKSPACE;
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv;
-    p.gw = rows; p.gu = rows + m; p.saved = static_cast<float*>(const_cast<void*>(saved));
-    return start_bwd<false>(stream, B, p, rows, gw, gu, nullptr, nullptr);
+    p.saved = static_cast<float*>(const_cast<void*>(saved));
+    return start_bwd<false>(stream, B, p, workspace, gw, gu, nullptr, nullptr);
 }
 
-int rwkv_wkv5as_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
-                        const float* u1, const float* w2, const float* u2, float* y, void* saved, size_t bytes) {
+int rwkv_wkv5as_forward_ws(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
+                           const float* u1, const float* w2, const float* u2, float* y, void* saved, size_t bytes, void* workspace,
+                           size_t workspace_bytes) {
     if (int e = check(B, T, C, H)) return e;
     if (int e = check_ptrs({r, k, v, u1, u2, y})) return e;
     if (int e = check_ptrs({w1, w2}, false)) return e;
@@ -835,7 +1060,11 @@ int rwkv_wkv5as_forward(void* stream, int B, int T, int C, int H, const float* r
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w1; p.u = u1; p.w2 = w2; p.u2 = u2; p.y = y;
     p.saved = static_cast<float*>(saved);
-    return start_fwd<true>(stream, B, p);
+    return start_fwd<true>(stream, B, p, workspace, workspace_bytes);
+}
+int rwkv_wkv5as_forward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
+                        const float* u1, const float* w2, const float* u2, float* y, void* saved, size_t bytes) {
+    return rwkv_wkv5as_forward_ws(stream, B, T, C, H, r, k, v, w1, u1, w2, u2, y, saved, bytes, nullptr, 0);
 }
 
 int rwkv_wkv5as_backward(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
@@ -846,14 +1075,11 @@ int rwkv_wkv5as_backward(void* stream, int B, int T, int C, int H, const float* 
     if (int e = check_ptrs({r, k, v, u1, u2, gy, gr, gk, gv, gw1, gu1, gw2, gu2})) return e;
     if (int e = check_ptrs({w1, w2}, false)) return e;
     if (saved == nullptr || bytes < saved_bytes<true>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
-    if (workspace == nullptr || workspace_bytes < rwkv_wkv5as_backward_workspace_bytes(B, T, C, H)) return RWKV_ERR_WORKSPACE;
-    float* rows = static_cast<float*>(workspace);
-    const size_t m = static_cast<size_t>(B) * C;
+    if (workspace == nullptr || workspace_bytes < bwd_ws_bytes<true>(B, T, C, H)) return RWKV_ERR_WORKSPACE;
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w1; p.u = u1; p.w2 = w2; p.u2 = u2; p.gy = gy;
-    p.gr = gr; p.gk = gk; p.gv = gv; p.gw = rows; p.gu = rows + m; p.gw2 = rows + 2 * m; p.gu2 = rows + 3 * m;
-    p.saved = static_cast<float*>(const_cast<void*>(saved));
-    return start_bwd<true>(stream, B, p, rows, gw1, gu1, gw2, gu2);
+    p.gr = gr; p.gk = gk; p.gv = gv; p.saved = static_cast<float*>(const_cast<void*>(saved));
+    return start_bwd<true>(stream, B, p, workspace, gw1, gu1, gw2, gu2);
 }
 
 }  // extern "C"
