@@ -470,6 +470,19 @@ int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float*
                        const void* r, const void* w, const void* k, const void* v, const void* a, const void* b,
                        void* y, float* sT);
 
+/* Forward and backward of all three ops in both modes with a workspace (rwkv7_workspace_bytes; 0: none is needed): few sequences (B H
+ * <= 256, in the backward <= 128) that are long enough are cut into blocks of time that are worked on side by side.  Without one whole
+ * sequences are walked through, as by the other entry points, and results are theirs bit for bit; in blocks they differ by rounding.
+ * s and sa are of one kind either way.  s0, sT, ds0, dsT may be NULL, and s with sa where no backward follows; `backward`: 0 or 1. */
+size_t rwkv7_workspace_bytes(int B, int T, int H, int backward);
+int rwkv7_forward_ws(void* stream, int B, int T, int H, int fp32, const float* s0,
+                     const void* r, const void* w, const void* k, const void* v, const void* a, const void* b,
+                     void* y, float* sT, float* s, float* sa, void* workspace, size_t workspace_bytes);
+int rwkv7_backward_ws(void* stream, int B, int T, int H, int fp32,
+                      const void* r, const void* w, const void* k, const void* v, const void* a, const void* b,
+                      const void* dy, const float* dsT, const float* s, const float* sa, float* ds0,
+                      void* dr, void* dw, void* dk, void* dv, void* da, void* db, void* workspace, size_t workspace_bytes);
+
 /* The two siblings of the state-passing op, served by the same kernels:
  *   rwkv7_state_*  : initial state s0 and its gradient ds0, no final state.  Replaces cuda_forward /
  *                    cuda_backward of rwkv7_fast_fused/cuda/rwkv7_state_clampw.cpp:10,17.

@@ -47,7 +47,7 @@ HIPCC_FLAGS = [
 # prefetch and its use (and a forward variant that spilled eleven registers gave wrong results): none may spill.
 SPILL_LIMIT = {"wkv6_bwd_fused": 0, "wkv6_fwd_fused": 0, "wkv6_fwd_ws": 0, "wkv6_bwd_a_ws": 0, "wkv6_bwd_b_wsILi0E": 3, "wkv6_bwd_b_wsILi1E": 1, "wkv6_bwd_b_wsILi2E": 1,
                "wkv_rows": 0, "wkv5_steps": 0, "wkv5b_fwd": 0, "wkv5b_bwd": 0, "wkv5c_fwd": 0, "wkv5c_bwdILb0E": 6, "wkv5c_bwdILb1E": 9, "wkv4_fwd_reg": 0, "wkv4_bwd_reg": 0, "timex_conv_h2": 0, "timex_gw_sum_h2": 0,
-               "timex_conv_any": 0, "timex_gw_any": 2, "rwkv7c_fwd": 0, "rwkv7c_bwd": 0}
+               "timex_conv_any": 0, "timex_gw_any": 2, "rwkv7c_fwd": 0, "rwkv7c_bwd": 0, "rwkv7c_local": 0, "rwkv7c_scan": 0}
 
 _lib = None
 
@@ -197,6 +197,9 @@ SIGNATURES = {
     "rwkv7_state_backward": (_I, [_P, _I, _I, _I] + [_P] * 16),
     "rwkv7_forward": (_I, [_P, _I, _I, _I] + [_P] * 9),
     "rwkv7_backward": (_I, [_P, _I, _I, _I] + [_P] * 15),
+    "rwkv7_workspace_bytes": (_Z, [_I, _I, _I, _I]),
+    "rwkv7_forward_ws": (_I, [_P, _I, _I, _I, _I] + [_P] * 11 + [_P, _Z]),
+    "rwkv7_backward_ws": (_I, [_P, _I, _I, _I, _I] + [_P] * 17 + [_P, _Z]),
     "rwkv7_forward_only": (_I, [_P, _I, _I, _I, _I] + [_P] * 9),
     "rwkv7_statepassing_forward_f32": (_I, [_P, _I, _I, _I] + [_P] * 11),
     "rwkv7_statepassing_backward_f32": (_I, [_P, _I, _I, _I] + [_P] * 17),

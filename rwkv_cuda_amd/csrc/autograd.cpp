@@ -406,14 +406,19 @@ variable_list rwkv7_run(AutogradContext* ctx, const Tensor& s0, const Tensor& r,
     Tensor y = flat || passing ? at::empty({B, T, H * HEAD}, r.options()) : at::empty({B, T, H, HEAD}, r.options());
     Tensor sT = passing ? at::empty({B, H, HEAD, HEAD}, f32) : Tensor();
     void* st = stream_of(r);
-    if (!grad && !(flags & RWKV_FLAG_SWEEPS)) {
+    const bool sweeps = flags & RWKV_FLAG_SWEEPS;
+    const size_t n = sweeps ? 0 : rwkv7_workspace_bytes(b_, t_, h_, 0);
+    const Tensor ws = n > 0 ? bytes(r, n) : Tensor();
+    if (!grad && !sweeps) {
         // no backward can follow: nothing is kept for one
-        ok(rwkv7_forward_only(st, b_, t_, h_, dt == F32, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT)));
+        ok(rwkv7_forward_ws(st, b_, t_, h_, dt == F32, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), nullptr, nullptr, P(ws), n));
         if (passing) return {y, sT};
         return {y};
     }
     Tensor s = at::empty({B, H, T / CHUNK7, HEAD, HEAD}, f32), sa = at::empty({B, T, H, HEAD}, f32);
-    if (dt == BF)
+    if (!sweeps)
+        ok(rwkv7_forward_ws(st, b_, t_, h_, dt == F32, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), P(ws), n));
+    else if (dt == BF)
         ok(rwkv7_statepassing_forward_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)));
     else
         ok(rwkv7_statepassing_forward_f32_ex(st, b_, t_, h_, P(s0), P(r), P(w), P(k), P(v), P(a), P(b), P(y), P(sT), P(s), P(sa), static_cast<unsigned>(flags)));
@@ -432,7 +437,12 @@ variable_list rwkv7_grads(AutogradContext* ctx, const Tensor& dy_, const Tensor&
     Tensor ds0 = state ? at::empty({B, H, HEAD, HEAD}, r.options().dtype(F32)) : Tensor(), d[6];
     for (int i = 0; i < 6; ++i) d[i] = at::empty(x[i].sizes(), r.options());       // (each input may have come in either shape)
     void* st = stream_of(r);
-    if (r.scalar_type() == BF)
+    if (!(get(ctx, "flags") & RWKV_FLAG_SWEEPS)) {
+        const size_t n = rwkv7_workspace_bytes(B, T, H, 1);
+        const Tensor ws = n > 0 ? bytes(r, n) : Tensor();
+        ok(rwkv7_backward_ws(st, B, T, H, r.scalar_type() == F32, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]),
+                             P(d[2]), P(d[3]), P(d[4]), P(d[5]), P(ws), n));
+    } else if (r.scalar_type() == BF)
         ok(rwkv7_statepassing_backward_ex(st, B, T, H, P(r), P(w), P(k), P(v), P(a), P(b), P(dy), P(dsT), P(s), P(sa), P(ds0), P(d[0]), P(d[1]), P(d[2]),
                                           P(d[3]), P(d[4]), P(d[5]), static_cast<unsigned>(get(ctx, "flags"))));
     else

@@ -232,11 +232,13 @@ int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t*
                      const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu,
                      const float* saved);
 
-// rwkv7_chunk.hip: chunked rwkv7 kernels (r..b, y, dy, dr..db are bf16 or, with f32, float); s0, sT, dsT, ds0 may be null
+// rwkv7_chunk.hip: chunked rwkv7 kernels (r..b, y, dy, dr..db are bf16 or, with f32, float); s0, sT, dsT, ds0 may be null.  ws (may be
+// null: whole sequences): rwkv7c_workspace_bytes, 16-byte aligned, for few sequences in blocks of time
+size_t rwkv7c_workspace_bytes(int B, int T, int H, bool bwd);
 int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0, const void* r, const void* w, const void* k,
-                 const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa);
+                 const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa, void* ws = nullptr);
 int launch7c_bwd(hipStream_t st, bool f32, int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
                  const void* a, const void* b, const void* dy, const float* dsT, const float* s, const float* sa,
-                 float* ds0, void* dr, void* dw, void* dk, void* dv, void* da, void* db);
+                 float* ds0, void* dr, void* dw, void* dk, void* dv, void* da, void* db, void* ws = nullptr);
 
 }  // namespace rwkv

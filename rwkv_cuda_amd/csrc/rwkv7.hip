@@ -471,6 +471,29 @@ int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float*
     return launch7c_fwd(static_cast<hipStream_t>(stream), fp32 != 0, B, T, H, s0, r, w, k, v, a, b, y, sT, nullptr, nullptr);
 }
 
+// All three ops in both modes, chunked kernels, with a workspace for few sequences.
+size_t rwkv7_workspace_bytes(int B, int T, int H, int backward) { return check7(B, T, H) == RWKV_OK ? rwkv7c_workspace_bytes(B, T, H, backward != 0) : 0; }
+
+int rwkv7_forward_ws(void* stream, int B, int T, int H, int fp32, const float* s0, const void* r, const void* w, const void* k,
+                     const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa, void* workspace, size_t workspace_bytes) {
+    if (int e = check7(B, T, H)) return e;
+    if (int e = check_ptrs({r, w, k, v, a, b, y})) return e;
+    if ((s == nullptr) != (sa == nullptr)) return RWKV_ERR_NULL;
+    if (!aligned16(s0) || !aligned16(sT) || !aligned16(s) || !aligned16(sa)) return RWKV_ERR_ALIGN;
+    if (workspace != nullptr && (workspace_bytes < rwkv7_workspace_bytes(B, T, H, 0) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+    return launch7c_fwd(static_cast<hipStream_t>(stream), fp32 != 0, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa, workspace);
+}
+
+int rwkv7_backward_ws(void* stream, int B, int T, int H, int fp32, const void* r, const void* w, const void* k, const void* v,
+                      const void* a, const void* b, const void* dy, const float* dsT, const float* s, const float* sa, float* ds0,
+                      void* dr, void* dw, void* dk, void* dv, void* da, void* db, void* workspace, size_t workspace_bytes) {
+    if (int e = check7(B, T, H)) return e;
+    if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, dr, dw, dk, dv, da, db})) return e;
+    if (!aligned16(dsT) || !aligned16(ds0)) return RWKV_ERR_ALIGN;
+    if (workspace != nullptr && (workspace_bytes < rwkv7_workspace_bytes(B, T, H, 1) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+    return launch7c_bwd(static_cast<hipStream_t>(stream), fp32 != 0, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db, workspace);
+}
+
 // ---- fp32 I/O: what the reference builds from the same sources with -D_FP32_ (rwkv7_cuda_benchmark.py:102-126 and the
 // same lines of its _state and _state_passing siblings).  The chunked kernels, whose arithmetic is fp32 in either mode: only
 // loads and stores differ.

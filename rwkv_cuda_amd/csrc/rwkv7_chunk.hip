@@ -68,7 +68,24 @@ struct Args7c {
     float *sT, *ds0;
     float* s;     // [B,H,T/16][i][j]: state entering each chunk
     float* sa;    // [B,T,H,N]: U
+    // sequences cut into NB > 1 blocks of `per` chunks, a workgroup each (blockIdx.z); per head: what each block makes of a state (local:
+    // E and M of the blocks but the last in the direction of travel), the states entering the blocks but the first (enter), whether the
+    // head is done as a whole (flags)
+    int NB, per;
+    float *local, *enter;
+    int* flags;
 };
+
+// The chunks of the workgroup's block; false: another workgroup does them.
+struct Part7 { int n, first, chunks; };
+DEVINL bool part_of(const Args7c& p, size_t bh, Part7& x) {
+    const int nch = p.T / CL;
+    x = {0, 0, nch};
+    if (p.NB == 1) return true;
+    if (__builtin_amdgcn_readfirstlane(p.flags[bh]) != 0) return blockIdx.z == 0;
+    x.n = blockIdx.z; x.first = x.n * p.per; x.chunks = min(p.per, nch - x.first);
+    return true;
+}
 
 // element base + o as it comes from memory, and its value
 // (a scalar base and one 32-bit byte offset a lane)
@@ -301,14 +318,15 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
     }
 }
 
-template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb, const Args7c& p, int q, int tid, size_t bh, size_t tok0, int nch, int h) {
+// s0, sT, slots: of this head and block
+template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb, const Args7c& p, const float* s0, float* sT, float* slots, int q, int tid, size_t tok0, int nch, int h) {
     const int lane = tid & 63, l16 = lane & 15, g = lane >> 4, H = p.H;
     const int i_own = 16 * q + l16;
     // state, transposed tiles: St[jt][v] = S[i_own][16 jt + 4 g + v]
     f32x4 St[4];
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
-        St[jt] = p.s0 != nullptr ? ld4(p.s0 + bh * N * N + static_cast<size_t>(i_own) * N + 16 * jt + 4 * g) : ZERO4;
+        St[jt] = s0 != nullptr ? ld4(s0 + static_cast<size_t>(i_own) * N + 16 * jt + 4 * g) : ZERO4;
     // y and sa = U (fp32) of chunk c as whole rows
     auto store_rows = [&](const int c) __attribute__((always_inline)) {
         const int t = tid >> 4, i4 = (tid & 15) * 4;
@@ -339,7 +357,7 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
         if (c > 0) store_rows(c - 1);
         // the state entering the chunk, for the backward
         if constexpr (KEEP) {
-            float* slot = p.s + (bh * nch + c) * N * N + static_cast<size_t>(i_own) * N + 4 * g;
+            float* slot = slots + static_cast<size_t>(c) * N * N + static_cast<size_t>(i_own) * N + 4 * g;
 #pragma unroll
             for (int jt = 0; jt < 4; ++jt) st4(slot + 16 * jt, St[jt]);
         }
@@ -367,8 +385,8 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
         __syncthreads();
     }
     store_rows(nch - 1);
-    if (p.sT != nullptr) {
-        float* dst = p.sT + bh * N * N + static_cast<size_t>(i_own) * N + 4 * g;
+    if (sT != nullptr) {
+        float* dst = sT + static_cast<size_t>(i_own) * N + 4 * g;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) st4(dst + 16 * jt, St[jt]);
     }
@@ -387,11 +405,217 @@ __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c p) {
     const lds_t sb = lds_of(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x, b = blockIdx.y;
-    const int nch = p.T / CL;
     const size_t bh = static_cast<size_t>(b) * p.H + h;
-    const size_t tok0 = static_cast<size_t>(b) * p.T;                 // first token row of this batch
-    if (w < 4) fwd_role_s<F32, KEEP>(S, sb, p, w, tid, bh, tok0, nch, h);
-    else fwd_role_p<F32>(S, sb, p, w - 4, tid & 63, tok0, nch, h);
+    Part7 x;
+    if (!part_of(p, bh, x)) return;
+    const size_t tok0 = static_cast<size_t>(b) * p.T + x.first * CL;  // first token row of this block
+    if (w < 4) {
+        const int all = p.T / CL;
+        const float* const s0 = x.n > 0 ? p.enter + (bh * (p.NB - 1) + x.n - 1) * N * N : (p.s0 != nullptr ? p.s0 + bh * N * N : nullptr);
+        float* const sT = p.sT != nullptr && x.first + x.chunks == all ? p.sT + bh * N * N : nullptr;
+        fwd_role_s<F32, KEEP>(S, sb, p, s0, sT, KEEP ? p.s + (bh * all + x.first) * N * N : nullptr, w, tid, tok0, x.chunks, h);
+    } else fwd_role_p<F32>(S, sb, p, w - 4, tid & 63, tok0, x.chunks, h);
+}
+
+// ---------------------------------------------------------------------------------------------------- blocks of time
+// Few sequences: the heads' sequences in blocks, a workgroup each, in three launches.  A block takes the state S to S M + E, row by row:
+// E is what it makes of an empty state, M of the identity without its own v; backwards the gradient state D becomes D M^T + F.  Both are
+// one recurrence,  W = P1 S^T + T1 V, U = M0 W, S = S dec + U^T P2 + V^T P3,  per chunk:
+//     forward   P1 = a e^{c_t}            T1 = AK     M0 = (I - AB)^{-1}  P2 = b e^{c_L - c_{s+1}}  P3 = k e^{c_L - c_{s+1}}  V = v
+//     backward  P1 = b e^{c_L - c_{s+1}}  T1 = RB^T   M0 = (I - AB)^{-T}  P2 = a e^{c_t}            P3 = r e^{c_{t+1}}        V = dy
+// which rwkv7c_local walks through (the roles of the forward without its outputs; a workgroup for E and one for M, which has no V).
+// rwkv7c_scan takes the blocks in turn, 16 rows of a head a workgroup, on the fp32 matrix instructions.  M may overflow where the state
+// itself is small (a, b that make it grow): a head with a scanned state that is not finite is walked through as a whole by the workgroup
+// of its first block, as are heads with inputs that are no number.
+struct SmemL {
+    float Ap[CL][PS], Bp[CL][PS], Xp[CL][PS];
+    float AB[CL][TS];
+    float part[4][N];
+    float dec[2][N];
+};
+constexpr uint32_t L_S = (sizeof(SmemL) + 31) / 32 * 32, L_KB = L_S + PLANE3, L_V = L_KB + 2 * PAIR3;
+template <bool F32> constexpr uint32_t L_MA = L_V + (F32 ? PLANE3 : TERM);
+template <bool F32> constexpr uint32_t L_TOTAL = L_MA<F32> + TPAIR3;
+static_assert(L_TOTAL<true> <= 80 * 1024, "two workgroups a CU");
+
+template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb, const Args7c& p, bool unit, int q, int lane, size_t tok0, int nch, int h) {
+    const int l16 = lane & 15, g = lane >> 4, H = p.H;
+    uint32_t nx[5][4];
+    auto fetch = [&](int c) __attribute__((always_inline)) {
+        c = c < nch ? c : nch - 1;
+        const size_t base = ((tok0 + static_cast<size_t>(REV ? nch - 1 - c : c) * CL) * H + h) * N;
+        uint32_t lo = lane;
+        asm volatile("" : "+v"(lo));
+        const uint16_t* const src[5] = {p.w, REV ? p.r : p.k, REV ? p.dy : p.v, p.a, p.b};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int k = 0; k < 5; ++k) nx[k][e] = ld_raw<F32>(src[k], base, static_cast<uint32_t>((4 * q + e) * H) * N + lo);
+    };
+    float lam[4], xx[4], aa[4], bb[4];
+    uint32_t vb[4];
+    auto convert = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            lam[e] = W_SCALE * sigmoid_fast(widen<F32>(nx[0][e]));
+            xx[e] = widen<F32>(nx[1][e]);
+            vb[e] = unit ? 0u : nx[2][e];
+            aa[e] = widen<F32>(nx[3][e]); bb[e] = widen<F32>(nx[4][e]);
+        }
+        S.part[q][lane] = (lam[0] + lam[1]) + (lam[2] + lam[3]);
+    };
+    auto planes = [&](const int slot) __attribute__((always_inline)) {
+        float cm, cl;
+        const Factors f = chunk_factors(lam, S.part, q, lane, cm, cl);
+        f32x4 as, be, xs;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 4 * q + e;
+            S.Ap[t][lane] = aa[e] * f.ea[e];
+            S.Bp[t][lane] = bb[e] * f.eb[e];
+            S.Xp[t][lane] = xx[e] * (REV ? f.er[e] : f.eb[e]);
+            as[e] = aa[e] * f.es[e];
+            be[e] = bb[e] * f.ee[e];
+            xs[e] = xx[e] * (REV ? f.es[e] * __expf(lam[e]) : f.ee[e]);
+        }
+        const lds_t o = sb + piece(lane, q);
+        // (no factor is above 1: what comes from bf16 inputs stays within bf16's range)
+        put3(o + L_S, split3<!F32>(REV ? be : as));
+        put_pair<TERM2>(sb + L_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(xs), split3<!F32>(REV ? as : be));
+        if constexpr (F32) put3(o + L_V, split3(f32x4{widen<F32>(vb[0]), widen<F32>(vb[1]), widen<F32>(vb[2]), widen<F32>(vb[3])}));
+        else lds_st<u32x2>(o + L_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
+        if (q == 0) S.dec[slot][lane] = exp_acc(cl);
+    };
+    fetch(0);
+    convert();
+    fetch(1);
+    __syncthreads();
+    planes(0);
+    __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+        if (q < 2) {
+            f32x4 x;
+            if (q == 0) {
+                const f32x4 t = causal_acc<false>(S.Ap, S.Bp, true, l16, g);
+                float m[CL];
+                // (this wave wrote AB itself: LDS keeps a wave's accesses in order)
+                if constexpr (REV) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) S.AB[4 * g + v][l16] = t[v];
+                    inverse_cols(S.AB, l16, m);
+                } else {
+                    st4(&S.AB[l16][4 * g], t);
+                    inverse_rows(S.AB, l16, m);
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) x[v] = by_group(g, m[v], m[4 + v], m[8 + v], m[12 + v]);
+            } else if constexpr (REV) x = causal_acc<false>(S.Xp, S.Bp, false, l16, g);
+            else x = causal_acc<true>(S.Ap, S.Xp, true, l16, g);
+            put_half<TTERM2>(sb + piece2(l16, g) + L_MA<F32> + (q == 0 ? 0 : 8), split3(x));
+        }
+        convert();
+        fetch(c + 2);
+        __syncthreads();
+        planes((c + 1) & 1);
+        __syncthreads();
+    }
+}
+template <bool F32> DEVINL void local_role_s(SmemL& S, const lds_t sb, float* out, bool unit, int q, int lane, int nch) {
+    const int l16 = lane & 15, g = lane >> 4, i_own = 16 * q + l16;
+    f32x4 St[4];                                         // S[i_own][16 jt + 4 g + v]
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) St[jt][v] = unit && i_own == 16 * jt + 4 * g + v ? 1.f : 0.f;
+    const Tr tr = tr_bases(sb, l16, g);
+    const lds_t pp = sb + piece2(l16, g), vp = sb + L_V + piece(i_own, g);
+    __syncthreads();
+    __syncthreads();
+    for (int c = 0; c < nch; ++c) {
+        const auto vop = [&]() __attribute__((always_inline)) { if constexpr (F32) return get3(vp); else return lds_ld<u32x2>(vp); }();
+        Sum2 W = SUM0;
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) add32(W, get3_tr(L_S, tr, hb), join(split3(St[2 * hb]), split3(St[2 * hb + 1])));
+        here(W);
+        __syncthreads();
+        add16(W, get_half<TTERM2>(pp + L_MA<F32> + 8), vop);
+        Sum2 Us = SUM0;
+        add16(Us, get_half<TTERM2>(pp + L_MA<F32>), split3(total(W)));
+        const Op3 vu = join(as3(vop), split3(total(Us)));
+        const lds_t kb = pp + L_KB + (c & 1) * PAIR3;
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) {
+            Sum2 x = SUM0;
+            add32(x, get_pair<TERM2>(kb + 1024 * jt), vu);
+            St[jt] = St[jt] * ld4(&S.dec[c & 1][16 * jt + 4 * g]) + total(x);
+        }
+        __syncthreads();
+    }
+    float* const dst = out + static_cast<size_t>(i_own) * N + 4 * g;
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) st4(dst + 16 * jt, St[jt]);
+}
+template <bool F32, bool REV>
+__global__ __launch_bounds__(NTF, 4) void rwkv7c_local(const Args7c p) {
+    extern __shared__ __align__(32) unsigned char smem_raw[];
+    SmemL& S = *reinterpret_cast<SmemL*>(smem_raw);
+    const lds_t sb = lds_of(smem_raw);
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = blockIdx.x, b = blockIdx.y, m = blockIdx.z >> 1, n = REV ? p.NB - 1 - m : m;
+    const bool unit = blockIdx.z & 1;
+    const size_t bh = static_cast<size_t>(b) * p.H + h;
+    if (blockIdx.z == 0 && tid == 0) p.flags[bh] = 0;
+    const int chunks = min(p.per, p.T / CL - n * p.per);
+    const size_t tok0 = static_cast<size_t>(b) * p.T + static_cast<size_t>(n) * p.per * CL;
+    if (w < 4) local_role_s<F32>(S, sb, p.local + ((bh * (p.NB - 1) + m) * 2 + unit) * N * N, unit, w, tid & 63, chunks);
+    else local_role_p<F32, REV>(S, sb, p, unit, w - 4, tid & 63, tok0, chunks, h);
+}
+// X_0 = s0 (backward: dsT), X_{m+1} = X_m M_m + E_m: a chain of NB - 1 small products; the next block's matrices are under way.
+template <bool REV>
+__global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
+    __shared__ float X[2][16][PS];
+    const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
+    const int rows = blockIdx.x & 3, h = blockIdx.x >> 2;
+    const size_t bh = static_cast<size_t>(blockIdx.y) * p.H + h;
+    const float* const init = REV ? p.dsT : p.s0;
+    const uint32_t o = (16 * rows + 4 * g) * N + 16 * q + l16;       // element [4 g][16 q + l16] of these rows
+    f32x4 x = ZERO4;
+    if (init != nullptr)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[v] = init[bh * N * N + o + v * N];
+    const float* at = p.local + bh * (p.NB - 1) * 2 * N * N;
+    float* to = p.enter + bh * (p.NB - 1) * N * N + o;
+    struct Block { float m[4][4]; f32x4 e; };
+    auto fetch = [&](Block& d) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d.m[s][e] = at[N * N + (16 * s + 4 * g + e) * N + 16 * q + l16];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) d.e[v] = at[o + v * N];
+    };
+    Block now, next;
+    fetch(now);
+    float bad = 0.f;
+    for (int m = 0; m + 1 < p.NB; ++m, to += N * N) {
+        if (m + 2 < p.NB) at += 2 * N * N;
+        fetch(next);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) X[m & 1][4 * g + v][16 * q + l16] = x[v];
+        __syncthreads();
+        f32x4 acc[2] = {now.e, ZERO4};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const f32x4 a = ld4(&X[m & 1][l16][16 * s + 4 * g]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[s & 1] = mm(a[e], now.m[s][e], acc[s & 1]);
+        }
+        x = acc[0] + acc[1];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) { to[v * N] = x[v]; bad = fmaf(x[v], 0.f, bad); }
+        now = next;
+    }
+    if (bad != 0.f) p.flags[bh] = 1;                     // (0, or no number)
 }
 
 // ---------------------------------------------------------------------------------------------------- backward
@@ -650,13 +874,13 @@ template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const lds_t sb, const
     if constexpr (!F32) bwd_store_rows(S, (nch - 1) & 1, p, tok0, tp, H, h);
 }
 
-template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
+template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const Args7c& p, const float* dsT, float* ds0, int tid, int w, int nch, size_t tok0, int H, int h) {
     const int lane = tid & 63, q = w & 3, l16 = lane & 15, g = lane >> 4;
     const int own = 16 * q + l16;                    // value channel i of this lane's column
     f32x4 dS[4];                                     // dS[i = own][j = 16 jt + 4 g + v]
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
-        dS[jt] = p.dsT != nullptr ? ld4(p.dsT + bh * N * N + static_cast<size_t>(own) * N + 16 * jt + 4 * g) : ZERO4;
+        dS[jt] = dsT != nullptr ? ld4(dsT + static_cast<size_t>(own) * N + 16 * jt + 4 * g) : ZERO4;
     using L = LB<F32>;
     const LaneB one = lane_bases(sb + L::ONE, l16, g, own);
     const Tr base_tr = tr_bases(sb, l16, g);
@@ -737,8 +961,8 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
         __syncthreads();
     }
     __syncthreads();
-    if (p.ds0 != nullptr) {
-        float* dst = p.ds0 + bh * N * N + static_cast<size_t>(own) * N + 4 * g;
+    if (ds0 != nullptr) {
+        float* dst = ds0 + static_cast<size_t>(own) * N + 4 * g;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) st4(dst + 16 * jt, dS[jt]);
     }
@@ -751,7 +975,7 @@ DEVINL uint32_t lane_again() {
     asm volatile("" : "+s"(all));
     return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
 }
-template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t bh, int nch, size_t tok0, int H, int h) {
+template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const Args7c& p, const float* dsT, const float* slots, int tid, int w, int nch, size_t tok0, int H, int h) {
     const int lane = tid & 63, q = w & 3, l16 = lane & 15, g = lane >> 4;
     const int own = 16 * q + l16;                    // key channel j of this lane's column
     using L = LB<F32>;
@@ -762,9 +986,9 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     for (int ib = 0; ib < 4; ++ib)
 #pragma unroll
         for (int v = 0; v < 4; ++v)
-            dS[ib][v] = p.dsT != nullptr ? p.dsT[bh * N * N + static_cast<size_t>(16 * ib + 4 * g + v) * N + own] : 0.f;
+            dS[ib][v] = dsT != nullptr ? dsT[static_cast<size_t>(16 * ib + 4 * g + v) * N + own] : 0.f;
     auto fetch_state = [&](int c) __attribute__((always_inline)) {
-        const float* slot = p.s + (bh * nch + c) * N * N;
+        const float* slot = slots + static_cast<size_t>(c) * N * N;
         const uint32_t me = lane_again();
         const uint32_t o = ((me >> 4) * (4 * N) + 16 * q + (me & 15)) * 4u;
         const char* const at = reinterpret_cast<const char*>(slot);
@@ -844,7 +1068,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         const LaneB two = moved(one, L::TWO + (i & 1) * L::SLOT - L::ONE);
         // ---------------------------------------------------------------- phase 1: finish the previous visit's chunk
         if (i > 0) finish(planes_of(i - 1), tok0 + static_cast<size_t>(c + 1) * CL);
-        else if (p.dsT != nullptr) {
+        else if (dsT != nullptr) {
             // P at the end of the call: sum_i dsT o S_T with S_T = S0 dec + U^T (B' d2) + V^T (K' d2) of the last chunk
             const float decj = chan(O, 2);
             const Op3 bdk = join(get3(one.own + L::BD), get3(one.own + L::KD));
@@ -927,52 +1151,94 @@ __global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c p) {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x, b = blockIdx.y;
     const size_t bh = static_cast<size_t>(b) * p.H + h;
-    const size_t tok0 = static_cast<size_t>(b) * p.T;
-    const int nch = p.T / CL;
+    Part7 x;
+    if (!part_of(p, bh, x)) return;
+    const size_t tok0 = static_cast<size_t>(b) * p.T + x.first * CL;
+    const int nch = x.chunks, all = p.T / CL;
     const lds_t sb = lds_of(smem_raw);
-    if (w < 4) bwd_role_a(S, sb, p, tid, w, bh, nch, tok0, p.H, h);
-    else if (w < 8) bwd_role_b(S, sb, p, tid, w, bh, nch, tok0, p.H, h);
-    else bwd_role_p(S, sb, p, tid, w, tok0, nch, p.H, h);
+    if (w >= 8) { bwd_role_p(S, sb, p, tid, w, tok0, nch, p.H, h); return; }
+    const float* const dsT = x.first + nch < all ? p.enter + (bh * (p.NB - 1) + p.NB - 2 - x.n) * N * N : (p.dsT != nullptr ? p.dsT + bh * N * N : nullptr);
+    if (w < 4) bwd_role_a(S, sb, p, dsT, p.ds0 != nullptr && x.n == 0 ? p.ds0 + bh * N * N : nullptr, tid, w, nch, tok0, p.H, h);
+    else bwd_role_b(S, sb, p, dsT, p.s + (bh * all + x.first) * N * N, tid, w, nch, tok0, p.H, h);
 }
 
 const uint16_t* el(const void* p) { return static_cast<const uint16_t*>(p); }
 uint16_t* el(void* p) { return static_cast<uint16_t*>(p); }
 
-template <bool F32, bool KEEP> int start_fwd(hipStream_t st, int B, int H, const Args7c& p) {
+// Blocks of time: as many as there is room for on the card at a time (two workgroups a CU in the forward, one in the backward), of
+// BLOCK_CHUNKS chunks at least; 1: whole sequences.  per: chunks a block.  The first pass does the work of a forward without its outputs
+// twice, which pays where a whole sequence leaves most of the card idle.  Where the line lies, B H sequences, us whole / in blocks, bf16
+// forward: 8 of T256 48 / 35, of T4096 709 / 112; 64 of T256 49 / 46, of T4096 719 / 378; 128 of T256 50 / 65, of T1024 183 / 178, of T4096
+// 720 / 645; 192 (two blocks) of T4096 721 / 1000.  Forward + backward of T4096: 8 sequences 1796 / 215, 32 1818 / 491, 128 1817 / 1573;
+// fp32 mode 1899 / 226, 2024 / 550, 2099 / 1785.  128 of T256, backward alone: 78 / 74.
+constexpr int BLOCK_CHUNKS = 4, SLOTS_FWD = 512, SLOTS_BWD = 256;
+int time_blocks(int B, int T, int H, bool bwd, int* per) {
+    const long long bh = static_cast<long long>(B) * H, want = (bwd ? SLOTS_BWD : SLOTS_FWD) / bh;
+    const int nch = T / CL;
+    *per = nch;
+    if (want < (bwd ? 2 : 4) || nch < 4 * BLOCK_CHUNKS || (!bwd && nch * 256LL < bh * bh)) return 1;
+    const int least = static_cast<int>((nch + want - 1) / want);
+    *per = least > BLOCK_CHUNKS ? least : BLOCK_CHUNKS;
+    return (nch + *per - 1) / *per;
+}
+size_t blocks_bytes(size_t bh, int NB) { return NB > 1 ? bh * (NB - 1) * 3 * N * N * sizeof(float) + (bh * sizeof(int) + 15) / 16 * 16 : 0; }
+// the kernels that bring the states to the blocks' borders, where there are blocks
+template <bool F32, bool REV> int cut(hipStream_t st, int B, Args7c& p, void* ws) {
+    p.NB = 1;
+    if (ws == nullptr) return RWKV_OK;
+    p.NB = time_blocks(B, p.T, p.H, REV, &p.per);
+    if (p.NB == 1) return RWKV_OK;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_local<F32, REV>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       static_cast<int>(L_TOTAL<F32>));
+    if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
+    const size_t n = static_cast<size_t>(B) * p.H * (p.NB - 1) * N * N;
+    p.local = static_cast<float*>(ws); p.enter = p.local + 2 * n; p.flags = reinterpret_cast<int*>(p.enter + n);
+    rwkv7c_local<F32, REV><<<dim3(p.H, B, 2 * (p.NB - 1)), dim3(NTF), L_TOTAL<F32>, st>>>(p);
+    rwkv7c_scan<REV><<<dim3(4 * p.H, B), dim3(256), 0, st>>>(p);
+    return launch_status();
+}
+
+template <bool F32, bool KEEP> int start_fwd(hipStream_t st, int B, Args7c& p, void* ws) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_fwd<F32, KEEP>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        static_cast<int>(F_TOTAL<F32>));
     if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
-    rwkv7c_fwd<F32, KEEP><<<dim3(H, B), dim3(NTF), F_TOTAL<F32>, st>>>(p);
+    if (int e = cut<F32, false>(st, B, p, ws)) return e;
+    rwkv7c_fwd<F32, KEEP><<<dim3(p.H, B, p.NB), dim3(NTF), F_TOTAL<F32>, st>>>(p);
     return launch_status();
 }
-template <bool F32> int start_bwd(hipStream_t st, int B, int H, const Args7c& p) {
+template <bool F32> int start_bwd(hipStream_t st, int B, Args7c& p, void* ws) {
     static_assert(LB<F32>::BYTES <= 160 * 1024, "the backward's LDS must fit one CU");
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_bwd<F32>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        static_cast<int>(LB<F32>::BYTES));
     if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
-    hipLaunchKernelGGL(rwkv7c_bwd<F32>, dim3(H, B), dim3(NTB), LB<F32>::BYTES, st, p);
+    if (int e = cut<F32, true>(st, B, p, ws)) return e;
+    hipLaunchKernelGGL(rwkv7c_bwd<F32>, dim3(p.H, B, p.NB), dim3(NTB), LB<F32>::BYTES, st, p);
     return launch_status();
 }
 
 }  // namespace
 
+size_t rwkv7c_workspace_bytes(int B, int T, int H, bool bwd) {
+    int per;
+    return blocks_bytes(static_cast<size_t>(B) * H, time_blocks(B, T, H, bwd, &per));
+}
 int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0, const void* r, const void* w, const void* k,
-                 const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa) {
+                 const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa, void* ws) {
     Args7c p{};
     p.T = T; p.H = H; p.s0 = s0; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b); p.y = el(y);
     p.sT = sT; p.s = s; p.sa = sa;
-    if (s != nullptr) return f32 ? start_fwd<true, true>(st, B, H, p) : start_fwd<false, true>(st, B, H, p);
-    return f32 ? start_fwd<true, false>(st, B, H, p) : start_fwd<false, false>(st, B, H, p);
+    if (s != nullptr) return f32 ? start_fwd<true, true>(st, B, p, ws) : start_fwd<false, true>(st, B, p, ws);
+    return f32 ? start_fwd<true, false>(st, B, p, ws) : start_fwd<false, false>(st, B, p, ws);
 }
 
 int launch7c_bwd(hipStream_t st, bool f32, int B, int T, int H, const void* r, const void* w, const void* k, const void* v,
                  const void* a, const void* b, const void* dy, const float* dsT, const float* s, const float* sa,
-                 float* ds0, void* dr, void* dw, void* dk, void* dv, void* da, void* db) {
+                 float* ds0, void* dr, void* dw, void* dk, void* dv, void* da, void* db, void* ws) {
     Args7c p{};
     p.T = T; p.H = H; p.r = el(r); p.w = el(w); p.k = el(k); p.v = el(v); p.a = el(a); p.b = el(b); p.dy = el(dy); p.dsT = dsT;
     p.s = const_cast<float*>(s); p.sa = const_cast<float*>(sa); p.ds0 = ds0;
     p.dr = el(dr); p.dw = el(dw); p.dk = el(dk); p.dv = el(dv); p.da = el(da); p.db = el(db);
-    return f32 ? start_bwd<true>(st, B, H, p) : start_bwd<false>(st, B, H, p);
+    return f32 ? start_bwd<true>(st, B, p, ws) : start_bwd<false>(st, B, p, ws);
 }
 
 }  // namespace rwkv

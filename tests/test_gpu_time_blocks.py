@@ -2,14 +2,19 @@
 oracle where a cut can go wrong: a last block of one token, of one chunk, of one segment between saved states and one off, blocks of
 two segments and of more, and many blocks.
 
-Tolerance, fp32: 1e-5 relative to the largest element and to the RMS, the bar of these operators' other tests; a block's state is a sum
-in another order, of the same products."""
+Tolerances.  wkv5, wkv5a fp32: 1e-5 relative to the largest element and to the RMS, the bar of these operators' other tests; a block's
+state is a sum in another order, of the same products.  rwkv7: fp32 results 4e-7 (some four to eight roundings of 2^-24 a result, as
+without blocks; a state at a border is one more product over 64 channels), dw 3e-7 a chunk adding up as a random walk, bf16 results the
+rounding of the output."""
+import math
+
 import pytest
 import torch
 
 from oracle import err_ratio, max_rel_to_peak
 from oracle import wkv5a as A
 from oracle import wkv56 as O
+from rwkv_cuda_amd import rwkv7_fast_fused as R
 from rwkv_cuda_amd import wkv5, wkv5a
 from rwkv_cuda_amd._call import call
 from _gpu_util import DEV, garbage
@@ -82,3 +87,80 @@ def test_fp32_inputs_that_are_not_finite_are_the_step_kernels(lib, bad):
         for h in (0, 2):
             assert torch.equal(a[..., 64 * h:64 * h + 64], b[..., 64 * h:64 * h + 64])
     assert bool(torch.isfinite(got[2][0, 391:]).all()) and bool(torch.isfinite(got[4].view(H, 64)[0]).all())
+
+
+def _rwkv7(B, T, H, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    n = lambda *s: torch.randn(*s, generator=g)
+    kk = torch.nn.functional.normalize(n(B, T, H, 64), dim=-1)
+    x = [n(B, T, H, 64) * 0.5, n(B, T, H, 64) + 0.5, n(B, T, H, 64) * 0.5, n(B, T, H, 64) * 0.5, -kk, kk * torch.sigmoid(n(B, T, H, 64))]
+    return n(B, H, 64, 64) * 0.1, [t.to(dtype).view(B, T, H * 64) for t in x], n(B, T, H * 64).to(dtype), n(B, H, 64, 64) * 0.1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("variant", ["passing", "state", "none"])
+@pytest.mark.parametrize("B,T,H", [(1, 256, 2), (2, 272, 1), (1, 33 * 16, 3), (1, 19 * 16, 70)])      # (the last: nothing cut in the forward)
+def test_rwkv7(lib, variant, dtype, B, T, H):
+    assert lib.rwkv7_workspace_bytes(B, T, H, 1) > 0, "not in blocks"
+    print(f"\nrwkv7 {variant} B={B} T={T} H={H} {dtype}", flush=True)
+    s0, x, dy, dsT = _rwkv7(B, T, H, dtype, 5 * T + H)
+    ins = ([] if variant == "none" else [s0]) + x
+    dev = [t.to(DEV).requires_grad_(True) for t in ins]
+    op = {"passing": R.RWKV7_STATE_PASSING_CLAMPW_CUDA, "state": R.RWKV7_STATE_CLAMPW_CUDA, "none": R.RWKV7_CLAMPW_CUDA}[variant]
+    out = list(op(*dev)) if variant == "passing" else [op(*dev)]
+    up = [dy, dsT] if variant == "passing" else [dy]
+    got = [z.detach() for z in out] + list(torch.autograd.grad(out, dev, [z.to(DEV) for z in up]))
+    with torch.no_grad():                                   # the forward that keeps nothing is cut in the same way
+        again = op(*dev)
+    assert torch.equal(again[0] if variant == "passing" else again, got[0])
+    p = [t.double().to(DEV).requires_grad_(True) for t in ins]          # (the step form in 64 bits, on the GPU for its speed)
+    S = p[0] if variant != "none" else torch.zeros(B, H, 64, 64, dtype=torch.float64, device=DEV)
+    r, w, k, v, a, b = (t.view(B, T, H, 64) for t in p[-6:])
+    d, ys = torch.exp(-math.exp(-0.5) * torch.sigmoid(w)), []
+    for t in range(T):
+        sa = (S * a[:, t, :, None, :]).sum(-1)
+        S = S * d[:, t, :, None, :] + sa[..., None] * b[:, t, :, None, :] + v[:, t, :, :, None] * k[:, t, :, None, :]
+        ys.append((S * r[:, t, :, None, :]).sum(-1))
+    outs = [torch.stack(ys, 1).view(B, T, H * 64)] + ([S] if variant == "passing" else [])
+    want = [z.detach() for z in outs] + list(torch.autograd.grad(outs, p, [z.double().to(DEV) for z in up]))
+    names = ["y"] + (["sT"] if variant == "passing" else []) + (["ds0"] if variant != "none" else []) + ["dr", "dw", "dk", "dv", "da", "db"]
+    for name, e, g in zip(names, want, got):
+        q = float((g.double().view_as(e) - e).norm() / e.norm())
+        print(f"  {name}: {q:.2e}", flush=True)
+        assert q <= (2.0 ** -8 if g.dtype == torch.bfloat16 else 6e-7 * (T / 16) ** 0.5 if name == "dw" else 4e-7), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("which", ["a", "k"])
+def test_rwkv7_heads_that_blocks_cannot_carry_are_done_as_a_whole(lib, which, dtype):
+    """A NaN among the inputs, and a transition that overflows over a block where the state itself is zero: the bits of a call without a
+    workspace, forward and backward, and other heads are not touched.  (k does not enter the gradient state: the backward of that head
+    is not done as a whole, and has no more results that are no number than one that is.)"""
+    B, T, H = 1, 512, 3
+    s0, x, dy, _ = _rwkv7(B, T, H, dtype, 3)
+    head = lambda t, h: t[..., 64 * h:64 * h + 64]
+    s0[:, 0] = 0
+    head(x[3], 0).zero_()                                   # v
+    head(x[4], 0).mul_(-3)                                  # a b^T: a growth of about 4.5 a step
+    head(x[5], 0).mul_(3)
+    head(dy, 0).zero_()
+    head(x[4 if which == "a" else 2], 1)[0, 300, 7] = math.nan
+    s0, dy, x = s0.to(DEV), dy.to(DEV), [t.to(DEV) for t in x]
+    f32 = int(dtype == torch.float32)
+    new = lambda *s, dt=torch.float32: garbage(s, dt)
+    res = []
+    for cut in (False, True):
+        n = [lib.rwkv7_workspace_bytes(B, T, H, i) if cut else 0 for i in (0, 1)]
+        ws = [garbage((m,), torch.uint8) if cut else None for m in n]
+        y, sT, s, sa, ds0 = new(B, T, H * 64, dt=dtype), new(B, H, 64, 64), new(B, H, T // 16, 64, 64), new(B, T, H, 64), new(B, H, 64, 64)
+        d = [new(B, T, H * 64, dt=dtype) for _ in range(6)]
+        call("rwkv7_forward_ws", y.device, B, T, H, f32, s0, *x, y, sT, s, sa, ws[0], n[0])
+        call("rwkv7_backward_ws", y.device, B, T, H, f32, *x, dy, None, s, sa, ds0, *d, ws[1], n[1])
+        res.append([y, *d, sT.transpose(1, 2).reshape(B, 64, H * 64), ds0.transpose(1, 2).reshape(B, 64, H * 64)])
+    for z, (whole, blocks) in enumerate(zip(*res)):
+        assert torch.equal(head(whole, 0), head(blocks, 0)), z
+        if which == "a" or z in (0, 7):
+            assert torch.equal(head(whole, 1).nan_to_num(7.0), head(blocks, 1).nan_to_num(7.0)), z
+        assert not bool((head(whole, 1).isfinite() & ~head(blocks, 1).isfinite()).any()), z
+        assert bool(head(blocks, 2).isfinite().all()) and not torch.equal(head(blocks, 2), garbage((1,), dtype).expand_as(head(blocks, 2)))
+    assert bool((head(res[1][0], 0) == 0).all())
