@@ -46,7 +46,7 @@ HIPCC_FLAGS = [
 # The one-sweep kernels let the compiler count their waits: a spill inside their loops would put scratch traffic between a
 # prefetch and its use (and a forward variant that spilled eleven registers gave wrong results): none may spill.
 SPILL_LIMIT = {"wkv6_bwd_fused": 0, "wkv6_fwd_fused": 0, "wkv6_fwd_ws": 0, "wkv6_bwd_a_ws": 0, "wkv6_bwd_b_wsILi0E": 3, "wkv6_bwd_b_wsILi1E": 1, "wkv6_bwd_b_wsILi2E": 1,
-               "wkv_rows": 0, "wkv5_steps": 0, "wkv5b_fwd": 0, "wkv5b_bwd": 0, "wkv5c_fwd": 0, "wkv5c_bwdILb0E": 6, "wkv5c_bwdILb1E": 9, "wkv4_fwd_reg": 0, "wkv4_bwd_reg": 0, "timex_conv_h2": 0, "timex_gw_sum_h2": 0,
+               "wkv_rows": 0, "wkv5_steps": 0, "wkv5b_fwd": 0, "wkv5b_bwd": 0, "wkv5b_local": 0, "wkv5c_fwd": 0, "wkv5c_bwdILb0E": 6, "wkv5c_bwdILb1E": 9, "wkv4_fwd_reg": 0, "wkv4_bwd_reg": 0, "timex_conv_h2": 0, "timex_gw_sum_h2": 0,
                "timex_conv_any": 0, "timex_gw_any": 2, "rwkv7c_fwd": 0, "rwkv7c_bwd": 0, "rwkv7c_local": 0, "rwkv7c_scan": 0}
 
 _lib = None
@@ -155,6 +155,8 @@ SIGNATURES = {
     "rwkv_wkv6f_backward_saved": (_I, [_P, _I, _I, _I, _I] + [_P] * 13 + [_P, _Z, _P, _Z, _U]),
     "rwkv_wkv5s_saved_bytes": (_Z, [_I, _I, _I, _I]),
     "rwkv_wkv5s_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 7 + [_P, _Z, _U]),
+    "rwkv_wkv5s_blocks_workspace_bytes": (_Z, [_I, _I, _I, _I, _I]),
+    "rwkv_wkv5s_forward_ws": (_I, [_P, _I, _I, _I, _I] + [_P] * 7 + [_P, _Z, _P, _Z, _U]),
     "rwkv_wkv5s_backward_workspace_bytes": (_Z, [_I, _I, _I, _I]),
     "rwkv_wkv5s_backward": (_I, [_P, _I, _I, _I, _I] + [_P] * 12 + [_P, _Z, _P, _Z, _U]),
     "rwkv_wkv5f32_forward": (_I, [_P, _I, _I, _I, _I] + [_P] * 6),

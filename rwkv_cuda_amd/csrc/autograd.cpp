@@ -273,7 +273,9 @@ struct Wkv5Bf16 : Function<Wkv5Bf16> {
             // (at 128 only if a backward can follow)
             const bool keep = grad || !whole;
             const Tensor saved = keep ? bytes(r, n) : Tensor();
-            ok(rwkv_wkv5s_forward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(saved), keep ? n : 0, flags));
+            const size_t nw = rwkv_wkv5s_blocks_workspace_bytes(d.B, d.T, d.C, d.H, 0);
+            const Tensor ws = nw > 0 ? bytes(r, nw) : Tensor();
+            ok(rwkv_wkv5s_forward_ws(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(u), P(y), P(decay), P(saved), keep ? n : 0, P(ws), nw, flags));
             if (keep) ctx->save_for_backward({r, k, v, decay, u, w, saved});
         } else {
             // heads of 128 channels with options run as four heads of 64 whose fp32 terms need scratch; every other size needs none
@@ -296,8 +298,9 @@ struct Wkv5Bf16 : Function<Wkv5Bf16> {
         Tensor gw = at::empty({d.H, d.C / d.H}, o), gu = at::empty({d.H, d.C / d.H}, o);       // summed over the batch by the library (:86-87)
         if (s.size() > 5) {
             const Tensor &w = s[5], &saved = s[6];
-            // (at head size 128 without options the per-batch rows of gw and gu are all)
-            const size_t n = d.C == d.H * MAX_HEAD ? 4 * static_cast<size_t>(d.B) * d.C : rwkv_wkv5s_backward_workspace_bytes(d.B, d.T, d.C, d.H);
+            // (at head size 128 without options the per-batch rows of gw and gu are all, and what blocks of time take)
+            const size_t nb = rwkv_wkv5s_blocks_workspace_bytes(d.B, d.T, d.C, d.H, 1);
+            const size_t n = nb > 0 ? nb : d.C == d.H * MAX_HEAD ? 4 * static_cast<size_t>(d.B) * d.C : rwkv_wkv5s_backward_workspace_bytes(d.B, d.T, d.C, d.H);
             Tensor ws = bytes(r, n);
             ok(rwkv_wkv5s_backward(stream_of(r), d.B, d.T, d.C, d.H, P(r), P(k), P(v), P(w), P(decay), P(u), P(gy), P(gr), P(gk), P(gv), P(gw), P(gu),
                                    P(saved), saved.numel(), P(ws), n, flags));

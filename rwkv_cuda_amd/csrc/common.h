@@ -225,12 +225,14 @@ int launch_wkv5f32_steps_bwd(hipStream_t st, int B, int T, int H, const float* r
 // Heads that run step by step (steps_head) are left out.  saved (may be null in the forward):
 // the states for the backward; gw, gu: per-batch rows [B][C].
 constexpr int WKV5B_MAX_C = 1 << 24;           // byte offsets within 32 rows are 32-bit
+// ws (may be null: whole sequences): wkv5b_blocks_bytes, 16-byte aligned, for few sequences in blocks of time (heads of 128)
 size_t wkv5b_saved_bytes(int B, int T, int C, int H);
+size_t wkv5b_blocks_bytes(int B, int T, int C, int H, bool bwd);
 int launch_wkv5b_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
-                     const uint16_t* u, uint16_t* y, float* decay, float* saved);
+                     const uint16_t* u, uint16_t* y, float* decay, float* saved, void* ws = nullptr);
 int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
                      const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu,
-                     const float* saved);
+                     const float* saved, void* ws = nullptr);
 
 // rwkv7_chunk.hip: chunked rwkv7 kernels (r..b, y, dy, dr..db are bf16 or, with f32, float); s0, sT, dsT, ds0 may be null.  ws (may be
 // null: whole sequences): rwkv7c_workspace_bytes, 16-byte aligned, for few sequences in blocks of time

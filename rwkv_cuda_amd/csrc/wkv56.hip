@@ -1496,9 +1496,21 @@ size_t rwkv_wkv5s_saved_bytes(int B, int T, int C, int H) {
     return n == 0 || C > WKV5B_MAX_C ? 0 : (n < wkv5b_saved_bytes(B, T, C, H) ? wkv5b_saved_bytes(B, T, C, H) : n);
 }
 
+size_t rwkv_wkv5s_blocks_workspace_bytes(int B, int T, int C, int H, int backward) {
+    if (check_dims(B, T, C, H) != RWKV_OK || !whole_head_ok(C, H, 0u)) return 0;
+    const size_t n = wkv5b_blocks_bytes(B, T, C, H, backward != 0);
+    return n == 0 ? 0 : n + (backward != 0 ? whole_head_ws_bytes(B, C) : 0);
+}
+
 int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16* r, const rwkv_bf16* k, const rwkv_bf16* v,
                        const rwkv_bf16* w_raw, const rwkv_bf16* u, rwkv_bf16* y, float* decay, void* saved, size_t saved_bytes,
                        unsigned flags) {
+    return rwkv_wkv5s_forward_ws(stream, B, T, C, H, r, k, v, w_raw, u, y, decay, saved, saved_bytes, nullptr, 0, flags);
+}
+
+int rwkv_wkv5s_forward_ws(void* stream, int B, int T, int C, int H, const rwkv_bf16* r, const rwkv_bf16* k, const rwkv_bf16* v,
+                          const rwkv_bf16* w_raw, const rwkv_bf16* u, rwkv_bf16* y, float* decay, void* saved, size_t saved_bytes,
+                          void* workspace, size_t workspace_bytes, unsigned flags) {
     if (int e = check_dims(B, T, C, H)) return e;
     if (int e = check_ptrs({r, k, v, w_raw, u, y, decay}, C == H * N)) return e;
     const hipStream_t st = static_cast<hipStream_t>(stream);
@@ -1506,7 +1518,8 @@ int rwkv_wkv5s_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         const int e = check_ptrs({r, k, v, w_raw, u, y, decay});
         if (e == RWKV_OK) {
             if (saved != nullptr && (saved_bytes < wkv5b_saved_bytes(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
-            if (int e2 = launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved))) return e2;
+            if (workspace != nullptr && (workspace_bytes < wkv5b_blocks_bytes(B, T, C, H, false) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+            if (int e2 = launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved), flags & RWKV_FLAG_WHOLE ? nullptr : workspace)) return e2;
             return launch_wkv5_steps_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, nullptr);
         }
         if (saved != nullptr) return e;
@@ -1556,7 +1569,10 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
         if (workspace == nullptr || workspace_bytes < whole_head_ws_bytes(B, C) || !aligned16(workspace)) return RWKV_ERR_WORKSPACE;
         uint16_t* pw = static_cast<uint16_t*>(workspace);                                 // per-batch gw, then per-batch gu
         uint16_t* pu = pw + whole_head_ws_bytes(B, C) / 4;
-        if (int e = launch_wkv5b_bwd(static_cast<hipStream_t>(stream), B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved))) return e;
+        // few sequences in blocks of time where the workspace is large enough for it
+        const size_t blocks = flags & RWKV_FLAG_WHOLE ? 0 : wkv5b_blocks_bytes(B, T, C, H, true);
+        void* const ws = blocks > 0 && workspace_bytes >= whole_head_ws_bytes(B, C) + blocks ? static_cast<char*>(workspace) + whole_head_ws_bytes(B, C) : nullptr;
+        if (int e = launch_wkv5b_bwd(static_cast<hipStream_t>(stream), B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, static_cast<const float*>(saved), ws)) return e;
         if (int e = launch_wkv5_steps_bwd(static_cast<hipStream_t>(stream), B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, pw, pu, nullptr, nullptr)) return e;
         hipLaunchKernelGGL(bf16_batch_sum, dim3((C + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), B, C, pw, gw, pu, gu);
         return launch_status();

@@ -48,7 +48,37 @@ struct ArgsW {
     uint16_t *y, *gr, *gk, *gv, *gw, *gu;        // gw, gu: per-batch rows [B][C]
     float* decay;                                // [e^l | l], 2 C floats (forward)
     float* saved;                                // [B*H][ceil(chunks / 2)][j][i]: the state entering every even chunk
+    // sequences cut into blocks of time (NB > 1): blocks of `per` pairs of chunks, a workgroup each; what each block leaves of a state that
+    // entered it empty, [B*H][NB - 1][HN][HN] (the last block's is not needed, in the backward the first's); gw, gu in fp32 [NB][B][C]
+    int B, NB, per;
+    float *local, *gw32, *gu32;
 };
+
+// The workgroup's head and its part of the sequence: chunks first .. first + chunks - 1, tokens that are left from there on.
+struct Part {
+    int h, b, n, first, chunks, left;
+    size_t bh, base;
+};
+// pairs: an odd number of chunks is rounded up
+DEVINL Part part_of(const ArgsW& p, int hn, bool pairs) {
+    Part x;
+    const int BH = p.B * p.H;
+    int nch = (p.T + L - 1) / L;
+    if (pairs) nch += nch & 1;
+    // (divisions are done in vector registers)
+    x.n = __builtin_amdgcn_readfirstlane(p.NB > 1 ? static_cast<int>(blockIdx.x) / BH : 0);
+    x.bh = blockIdx.x - x.n * BH;
+    x.b = __builtin_amdgcn_readfirstlane(static_cast<int>(x.bh) / p.H); x.h = static_cast<int>(x.bh) - x.b * p.H;
+    x.first = x.n * 2 * p.per;
+    x.chunks = p.NB > 1 ? min(2 * p.per, nch - x.first) : nch;
+    x.left = p.T - x.first * L;
+    x.base = (static_cast<size_t>(x.b) * p.T + static_cast<size_t>(x.first) * L) * p.C + static_cast<size_t>(x.h) * hn;
+    return x;
+}
+// where the states of the part's pairs of chunks are
+template <int HN> DEVINL float* saved_state(const ArgsW& p, const Part& x) {
+    return p.saved + (x.bh * ((p.T + 2 * L - 1) / (2 * L)) + x.first / 2) * HN * HN;
+}
 
 extern __shared__ __align__(16) unsigned char smem_raw[];
 
@@ -57,7 +87,7 @@ template <int HN> struct G {
     static constexpr int CT = HN / 64, KS = HN / 32, NB16 = HN / 16, PARTS = HN / 32;
     static constexpr int PIECES = HN / 8, ROWS = 256 / PIECES, PASSES = L / ROWS;
     static constexpr uint32_t ROW = 2 * HN + 16, PLANE = L * ROW;
-    static constexpr uint32_t LAM = 0, U = 4 * HN, BASE = 8 * HN;
+    static constexpr uint32_t LAM = 0, U = 4 * HN, BLK = 8 * HN, BASE = 12 * HN;      // BLK: decay of a block of time
     static constexpr uint32_t PART = 3 * 1024;                                   // the three quadrants of a tile, fp32, as the lanes hold them
     // forward: three slots of planes R' hi, lo, K' hi, lo, V and sum r u k; two sets of tile parts
     static constexpr uint32_t FRH = 0, FRL = PLANE, FKH = 2 * PLANE, FKL = 3 * PLANE, FV = 4 * PLANE, FRUK = 5 * PLANE, FSLOT = FRUK + 4 * L;
@@ -117,18 +147,19 @@ template <uint32_t ROW> DEVINL bf16x8 ld_tra(const lds_t a) {
 DEVINL int slot_token(int g, int e) { return 16 * (e >> 2) + 4 * g + (e & 3); }
 
 // The head's parameters into LDS (by the first wave); every wave finds out for itself what its strongest log decay is.
-template <int HN> DEVINL float head_setup(const ArgsW& p, lds_t sb, int h, int b, int tid) {
+template <int HN> DEVINL float head_setup(const ArgsW& p, lds_t sb, const Part& part, int tid) {
     const int lane = tid & 63;
     float mn = 0.f;
 #pragma unroll
     for (int z = 0; z < HN / 64; ++z) {
-        const int n = 64 * z + lane, c = h * HN + n;
+        const int n = 64 * z + lane, c = part.h * HN + n;
         const float l = -expf(bf2f(p.w[c]));
         mn = fminf(mn, l);
         if (tid < 64) {
             lds_st<float>(sb + G<HN>::LAM + 4 * n, l);
             lds_st<float>(sb + G<HN>::U + 4 * n, bf2f(p.u[c]));
-            if (p.decay != nullptr && b == 0) { p.decay[c] = expf(l); p.decay[p.C + c] = l; }
+            lds_st<float>(sb + G<HN>::BLK + 4 * n, wpow(l, 2 * L * p.per));
+            if (p.decay != nullptr && part.b == 0 && part.n == 0) { p.decay[c] = expf(l); p.decay[p.C + c] = l; }
         }
     }
 #pragma unroll
@@ -217,16 +248,104 @@ DEVINL void raw_part(const bf16x8 (&r)[2], const bf16x8 (&k)[2], const TilePower
     }
 }
 
+// ---------------------------------------------------------------------------------------------------- blocks of time, first pass
+// What a block leaves of an empty state: sum over its tokens of v_t k_t^T with the decay that is left to the block's end, stored as [i][j]
+// for the forward, or (REV) from the end backwards what the gradient state takes up, gy_t r_t^T, stored as [j][i] for the D waves.  A wave
+// makes 32 key channels, whose operand takes the powers (hi + lo); the other side is exact.
+template <int HN, bool REV>
+__global__ __launch_bounds__(256) void wkv5b_local(const ArgsW p) {
+    using A = G<HN>;
+    constexpr int NT = A::NB16, NP = A::PASSES, CT = A::CT;
+    __shared__ __align__(16) unsigned char rows[4 * A::PLANE];           // two sets of key and value rows
+    const lds_t sb = lds_of(rows);
+    const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4, C = p.C;
+    const int BH = p.B * p.H, m = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / BH), bh = blockIdx.x - m * BH;
+    const int b = __builtin_amdgcn_readfirstlane(bh / p.H), h = bh - b * p.H, n = REV ? m + 1 : m;
+    if (steps_head<false, HN>(p.w, nullptr, h * HN)) return;
+    const int first = n * 2 * p.per, chunks = min(2 * p.per, (p.T + L - 1) / L - first);
+    const size_t base = (static_cast<size_t>(b) * p.T + static_cast<size_t>(first) * L) * C + static_cast<size_t>(h) * HN;
+    const int left = p.T - first * L, row0 = tid / A::PIECES, c8 = (tid % A::PIECES) * 8;
+    const uint16_t* const key = (REV ? p.r : p.k) + base;
+    const uint16_t* const val = (REV ? p.gy : p.v) + base;
+    float pw[CT][8], dec[CT][4];
+    auto log_decay = [&](int j) __attribute__((always_inline)) { return -expf(bf2f(p.w[h * HN + j])); };
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int j0 = 16 * (CT * q + ct);
+        const float l = log_decay(j0 + l16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pw[ct][e] = wpow(l, REV ? slot_token(g, e) : 31 - slot_token(g, e));
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dec[ct][v] = REV ? wpow(l, L) : wpow(log_decay(j0 + 4 * g + v), L);
+    }
+    uint4 x[2][NP];
+    auto fetch = [&](const int i) __attribute__((always_inline)) {       // i-th chunk in the direction of travel
+        const int c = REV ? max(chunks - 1 - i, 0) : min(i, chunks - 1);
+        const rows_t kr = rows_of(key + static_cast<size_t>(c) * L * C, left - c * L, C), vr = rows_of(val + static_cast<size_t>(c) * L * C, left - c * L, C);
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+            const int lo = 2 * ((row0 + z * A::ROWS) * C + c8);
+            x[0][z] = load16(kr, lo); x[1][z] = load16(vr, lo);
+        }
+    };
+    auto put = [&](const int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int z = 0; z < NP; ++z) {
+            const lds_t o = sb + set * 2 * A::PLANE + (row0 + z * A::ROWS) * A::ROW + 2 * c8;
+            lds_st<bf16x8>(o, op4(x[0][z])); lds_st<bf16x8>(o + A::PLANE, op4(x[1][z]));
+        }
+    };
+    f32x4 acc[CT][NT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int e = 0; e < NT; ++e) acc[ct][e] = ZERO4;
+    fetch(0);
+    put(0);
+    fetch(1);
+    __syncthreads();
+    for (int i = 0; i < chunks; ++i) {
+        lds_t o = sb + (i & 1) * 2 * A::PLANE + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3);
+        opaque(o);
+        Op2 k[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) k[ct] = scaled(ld_tra<A::ROW>(o + 32 * (CT * q + ct)), pw[ct]);
+#pragma unroll
+        for (int e = 0; e < NT; ++e) {
+            const bf16x8 v = ld_tra<A::ROW>(o + A::PLANE + 32 * e);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                f32x4 s = acc[ct][e];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) s[t] *= dec[ct][t];
+                acc[ct][e] = REV ? mfma(v, k[ct].l, mfma(v, k[ct].h, s)) : mfma(k[ct].l, v, mfma(k[ct].h, v, s));
+            }
+        }
+        put((i + 1) & 1);
+        fetch(i + 2);
+        __syncthreads();
+    }
+    float* const out = p.local + (static_cast<size_t>(bh) * (p.NB - 1) + m) * HN * HN;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int e = 0; e < NT; ++e) {
+            const int j0 = 16 * (CT * q + ct), i0 = 16 * e;
+            *reinterpret_cast<f32x4*>(out + (REV ? (j0 + l16) * HN + i0 + 4 * g : (i0 + l16) * HN + j0 + 4 * g)) = acc[ct][e];
+        }
+}
+
 // ---------------------------------------------------------------------------------------------------- forward
 // Waves 0..3 hold St[ct][jt][v] = S[j = 16 jt + 4 g + v][i = own], as it stands the B operand of a contraction over j.  Waves 4..7
 // load (two chunks ahead of the planes, the planes two chunks ahead of their use) and make the next chunk's tile in parts of 32
 // key channels.  One barrier a chunk.
 // Planes: R' = r o^{t-16}, K' = k o^{15-t} (they serve the tile, the state times o^16 on its way in and out of the update); RAW, for
 // strong decays: r o^t, k o^{31-t}, and the tile is made from the raw rows (read once more, from L2).
-template <int HN, bool RAW> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int q, int lane, size_t base, int nch) {
+template <int HN, bool RAW> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int q, int lane, const Part& part) {
     using A = G<HN>;
     constexpr int CT = A::CT, KS = A::KS, NJ = A::NB16;
-    const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    const int l16 = lane & 15, g = lane >> 4, T = part.left, C = p.C, nch = part.chunks;
+    const size_t base = part.base;
     float dd[NJ][4];                                     // o^16; RAW: o^32
 #pragma unroll
     for (int jt = 0; jt < NJ; ++jt)
@@ -237,8 +356,18 @@ template <int HN, bool RAW> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int
     for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
         for (int jt = 0; jt < NJ; ++jt) St[ct][jt] = ZERO4;
-    const int nseg = (nch + 1) / 2;
-    float* const sv = p.saved != nullptr ? p.saved + static_cast<size_t>(blockIdx.x) * nseg * HN * HN + 16 * CT * q + l16 + 4 * g * HN : nullptr;
+    if (part.n > 0) {                                    // the state that enters the block, from what the blocks before leave
+        const float* x = p.local + part.bh * (p.NB - 1) * HN * HN + (16 * CT * q + l16) * HN + 4 * g;
+#pragma unroll 2
+        for (int m = 0; m < part.n; ++m, x += HN * HN)
+#pragma unroll
+            for (int jt = 0; jt < NJ; ++jt) {
+                const f32x4 d = lds_ld<f32x4>(sb + A::BLK + 4 * (16 * jt + 4 * g));
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) St[ct][jt] = St[ct][jt] * d + *reinterpret_cast<const f32x4*>(x + 16 * ct * HN + 16 * jt);
+            }
+    }
+    float* const sv = p.saved != nullptr ? saved_state<HN>(p, part) + 16 * CT * q + l16 + 4 * g * HN : nullptr;
     uint16_t* const out = p.y + base + 16 * CT * q;
     const int to = tile_offset(l16, g, C);
     const lds_t orow = sb + A::BASE + l16 * A::ROW + 8 * g, otr = sb + A::BASE + (4 * g + (l16 >> 2)) * A::ROW + 8 * (l16 & 3);
@@ -317,10 +446,11 @@ template <int HN, bool RAW> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int
     }
 }
 
-template <int HN, bool RAW> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int tp, size_t base, int nch) {
+template <int HN, bool RAW> DEVINL void fwd_loads(const ArgsW& p, lds_t sb, int tp, const Part& part) {
     using A = G<HN>;
     constexpr int NP = A::PASSES;
-    const int lane = tp & 63, q = tp >> 6, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    const int lane = tp & 63, q = tp >> 6, l16 = lane & 15, g = lane >> 4, T = part.left, C = p.C, nch = part.chunks;
+    const size_t base = part.base;
     const int row0 = tp / A::PIECES, c8 = (tp % A::PIECES) * 8;
     float u[8], pr[NP][8], pk[NP][8];
 #pragma unroll
@@ -420,18 +550,17 @@ template <int HN>
 __global__ __launch_bounds__(NTH, 2) void wkv5b_fwd(const ArgsW p) {
     const lds_t sb = lds_of(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = (p.T + L - 1) / L;
-    const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
+    const Part part = part_of(p, HN, false);
     if (HN == 64 && !strong_layer(p.w, p.C, tid & 63)) return;      // the one-sweep kernels of wkv6 have done this layer
-    const float lmin = head_setup<HN>(p, sb, h, b, tid);            // (the decays of every head go to p.decay)
-    if (steps_head<false, HN>(p.w, nullptr, h * HN)) return;
+    const float lmin = head_setup<HN>(p, sb, part, tid);            // (the decays of every head go to p.decay)
+    if (steps_head<false, HN>(p.w, nullptr, part.h * HN)) return;
     __syncthreads();
     if (w < 4) {
-        if (lmin < LAM_MID) fwd_states<HN, true>(p, sb, w, tid & 63, base, nch);
-        else fwd_states<HN, false>(p, sb, w, tid & 63, base, nch);
+        if (lmin < LAM_MID) fwd_states<HN, true>(p, sb, w, tid & 63, part);
+        else fwd_states<HN, false>(p, sb, w, tid & 63, part);
     } else {
-        if (lmin < LAM_MID) fwd_loads<HN, true>(p, sb, tid - 256, base, nch);
-        else fwd_loads<HN, false>(p, sb, tid - 256, base, nch);
+        if (lmin < LAM_MID) fwd_loads<HN, true>(p, sb, tid - 256, part);
+        else fwd_loads<HN, false>(p, sb, tid - 256, part);
     }
 }
 
@@ -476,10 +605,11 @@ DEVINL uint32_t lane_now() {
     return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u));
 }
 
-template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, int h, int b, size_t base, int nch) {
+template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, const Part& part) {
     using A = G<HN>;
     constexpr int KS = A::KS, NI = A::NB16;
-    const int l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    const int l16 = lane & 15, g = lane >> 4, T = part.left, C = p.C, nch = part.chunks;
+    const size_t base = part.base;
     // Powers of a set of eight slots, token 16 a + 4 g + b: a base per lane times o^b times o^{16 a} (or the reverse); the eight would
     // take the registers that the states need.  Bases: cb of o^{t-m}, kb of o^{m-1-t}, m the middle of the token's half.
     const float l = lds_f(sb + A::LAM + 4 * (16 * q + l16));
@@ -488,6 +618,14 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
     f32x4 dS[NI];
 #pragma unroll
     for (int ib = 0; ib < NI; ++ib) dS[ib] = ZERO4;
+    if (part.n + 1 < p.NB) {                             // the gradient of the state that leaves the block, from what the blocks after take up
+        const float* x = p.local + (part.bh * (p.NB - 1) + p.NB - 2) * HN * HN + (16 * q + l16) * HN + 4 * g;
+        const float d = lds_f(sb + A::BLK + 4 * (16 * q + l16));
+#pragma unroll 1
+        for (int m = p.NB - 1; m > part.n; --m, x -= HN * HN)
+#pragma unroll
+            for (int ib = 0; ib < NI; ++ib) dS[ib] = dS[ib] * d + *reinterpret_cast<const f32x4*>(x + 16 * ib);
+    }
     float gw = 0.f, gP = 0.f, gu = 0.f;
     // (hidden: hoisted out of the loop the powers and token numbers would take registers all the same)
     auto hide = [](float x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); return x; };
@@ -524,7 +662,7 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
         const uint4 h = __builtin_bit_cast(uint4, w.h), lo = __builtin_bit_cast(uint4, w.l);
         w = sinks ? Op2{as_op(h.x, h.y, a.h, b.h), as_op(lo.x, lo.y, a.l, b.l)} : Op2{as_op(a.h, b.h, h.z, h.w), as_op(a.l, b.l, lo.z, lo.w)};
     };
-    const float* const sv = p.saved + static_cast<size_t>(blockIdx.x) * (nch / 2) * HN * HN;
+    const float* const sv = saved_state<HN>(p, part);
     auto fetch_state = [&](int c, int ks, uint32_t so, f32x4 (&s)[2]) __attribute__((always_inline)) {      // (a scalar base and one lane offset)
         const char* const d = reinterpret_cast<const char*>(sv + static_cast<size_t>(c >> 1) * HN * HN + 32 * ks);
 #pragma unroll
@@ -679,18 +817,19 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
         chunk(std::true_type{}, c);
         chunk(std::false_type{}, c - 1);
     }
-    const int c = h * HN + 16 * q + l16;
+    const size_t o = (static_cast<size_t>(part.n) * p.B + part.b) * C + part.h * HN + 16 * q + l16;
     const float sw = allreduce_rows(fmaf(32.f * o32, gP, gw)), su = allreduce_rows(gu);
     if (g == 0) {
-        p.gw[static_cast<size_t>(b) * C + c] = f2bf(l * sw);
-        p.gu[static_cast<size_t>(b) * C + c] = f2bf(su);
+        if (p.NB > 1) { p.gw32[o] = l * sw; p.gu32[o] = su; }
+        else { p.gw[o] = f2bf(l * sw); p.gu[o] = f2bf(su); }
     }
 }
 
-template <int HN> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, size_t base, int nch) {
+template <int HN> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, const Part& part_) {
     using A = G<HN>;
     constexpr int KS = A::KS, PARTS = A::PARTS;
-    const int w = __builtin_amdgcn_readfirstlane(te >> 6), lane = te & 63, l16 = lane & 15, g = lane >> 4, T = p.T, C = p.C;
+    const int w = __builtin_amdgcn_readfirstlane(te >> 6), lane = te & 63, l16 = lane & 15, g = lane >> 4, T = part_.left, C = p.C, nch = part_.chunks;
+    const size_t base = part_.base;
     const int row0 = te / A::PIECES, c8 = (te % A::PIECES) * 8;
     // gv: value channels 32 wq .. + 31, tokens 16 wz .. + 15; tile A: channels 32 part .., the quadrant across the halves or the others
     const int wq = w >> 1, wz = w & 1, part = w % PARTS;
@@ -828,13 +967,22 @@ template <int HN>
 __global__ __launch_bounds__(8 * HN, HN / 32) void wkv5b_bwd(const ArgsW p) {
     const lds_t sb = lds_of(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b = __builtin_amdgcn_readfirstlane(blockIdx.x / p.H), h = blockIdx.x - b * p.H, nch = 2 * ((p.T + 2 * L - 1) / (2 * L));      // whole pairs (a last chunk without tokens adds zeros)
-    const size_t base = static_cast<size_t>(b) * p.T * p.C + static_cast<size_t>(h) * HN;
-    if ((HN == 64 && !strong_layer(p.w, p.C, tid & 63)) || steps_head<false, HN>(p.w, nullptr, h * HN)) return;
-    head_setup<HN>(p, sb, h, b, tid);
+    const Part part = part_of(p, HN, true);              // (a last chunk without tokens adds zeros)
+    if ((HN == 64 && !strong_layer(p.w, p.C, tid & 63)) || steps_head<false, HN>(p.w, nullptr, part.h * HN)) return;
+    head_setup<HN>(p, sb, part, tid);
     __syncthreads();
-    if (w < HN / 16) role_d<HN>(p, sb, w, tid & 63, h, b, base, nch);
-    else role_e<HN>(p, sb, tid - 4 * HN, base, nch);
+    if (w < HN / 16) role_d<HN>(p, sb, w, tid & 63, part);
+    else role_e<HN>(p, sb, tid - 4 * HN, part);
+}
+
+// gw, gu of a batch row from its blocks, rounded once
+__global__ __launch_bounds__(256) void block_rows(int NB, size_t n, const float* __restrict__ w32, const float* __restrict__ u32, uint16_t* gw, uint16_t* gu) {
+    const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float* const x = (blockIdx.y == 0 ? w32 : u32) + i;
+    float s = 0.f;
+    for (int m = 0; m < NB; ++m) s += x[m * n];
+    (blockIdx.y == 0 ? gw : gu)[i] = f2bf(s);
 }
 
 template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, int threads, uint32_t lds) {
@@ -842,8 +990,32 @@ template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, 
         g_last_hip_error = static_cast<int>(e);
         return RWKV_ERR_LAUNCH;
     }
-    hipLaunchKernelGGL(kernel, dim3(B * p.H), dim3(threads), lds, st, p);
+    hipLaunchKernelGGL(kernel, dim3(B * p.H * p.NB), dim3(threads), lds, st, p);
     return launch_status();
+}
+
+// Blocks of time, heads of 128 channels: as many as give every CU a workgroup (the kernels' LDS leaves room for one), of BLOCK_PAIRS pairs of
+// chunks at least; 1: whole sequences.  per: pairs a block.  Where the line lies, B H sequences, us whole / in blocks: forward 8 of T400 34 / 30,
+// of T4096 255 / 99; 64 of T400 34 / 34, of T4096 261 / 130; 128 of T400 36 / 43, of T800 60 / 61, of T2000 135 / 122; forward + backward 8 of
+// T400 135 / 102, of T4096 1093 / 209; 32 of T4096 1174 / 257; 128 of T400 146 / 125, of T4096 1269 / 836.
+constexpr int BLOCK_PAIRS = 2, SLOTS = 256;
+int time_blocks(int B, int T, int H, bool bwd, int* per) {
+    const long long bh = static_cast<long long>(B) * H, want = SLOTS / bh;
+    const int pairs = static_cast<int>((static_cast<long long>(T) + 2 * L - 1) / (2 * L));
+    *per = pairs;
+    if (want < 2 || pairs < 3 * BLOCK_PAIRS || (!bwd && pairs * 8 < bh)) return 1;
+    const int least = static_cast<int>((pairs + want - 1) / want);
+    *per = least > BLOCK_PAIRS ? least : BLOCK_PAIRS;
+    return (pairs + *per - 1) / *per;
+}
+size_t round16(size_t x) { return (x + 15) & ~static_cast<size_t>(15); }
+void set_blocks(ArgsW& p, int B, bool bwd, void* ws) {
+    p.B = B; p.NB = 1; p.per = 0;
+    if (ws == nullptr) return;
+    p.NB = time_blocks(B, p.T, p.H, bwd, &p.per);
+    p.local = static_cast<float*>(ws);
+    p.gw32 = p.local + static_cast<size_t>(B) * p.H * (p.NB - 1) * 128 * 128;
+    p.gu32 = p.gw32 + static_cast<size_t>(p.NB) * B * p.C;
 }
 
 }  // namespace
@@ -852,18 +1024,33 @@ size_t wkv5b_saved_bytes(int B, int T, int C, int H) {
     const size_t nch = (static_cast<size_t>(T) + L - 1) / L, n = C / H;
     return static_cast<size_t>(B) * H * ((nch + 1) / 2) * n * n * sizeof(float);
 }
+size_t wkv5b_blocks_bytes(int B, int T, int C, int H, bool bwd) {
+    int per;
+    const int NB = C == H * 128 ? time_blocks(B, T, H, bwd, &per) : 1;
+    if (NB == 1) return 0;
+    return static_cast<size_t>(B) * H * (NB - 1) * 128 * 128 * sizeof(float) + (bwd ? round16(2 * static_cast<size_t>(NB) * B * C * sizeof(float)) : 0);
+}
 int launch_wkv5b_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
-                     const uint16_t* u, uint16_t* y, float* decay, float* saved) {
+                     const uint16_t* u, uint16_t* y, float* decay, float* saved, void* ws) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.decay = decay; p.saved = saved;
+    set_blocks(p, B, false, ws);
+    if (p.NB > 1) hipLaunchKernelGGL((wkv5b_local<128, false>), dim3(B * H * (p.NB - 1)), dim3(256), 0, st, p);
     return C == H * 64 ? launch(wkv5b_fwd<64>, st, B, p, NTH, G<64>::FTOTAL) : launch(wkv5b_fwd<128>, st, B, p, NTH, G<128>::FTOTAL);
 }
 int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
-                     const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu, const float* saved) {
+                     const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu, const float* saved, void* ws) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv; p.gw = gw; p.gu = gu;
     p.saved = const_cast<float*>(saved);
-    return C == H * 64 ? launch(wkv5b_bwd<64>, st, B, p, 512, G<64>::BTOTAL) : launch(wkv5b_bwd<128>, st, B, p, 1024, G<128>::BTOTAL);
+    set_blocks(p, B, true, ws);
+    if (p.NB > 1) hipLaunchKernelGGL((wkv5b_local<128, true>), dim3(B * H * (p.NB - 1)), dim3(256), 0, st, p);
+    if (int e = C == H * 64 ? launch(wkv5b_bwd<64>, st, B, p, 512, G<64>::BTOTAL) : launch(wkv5b_bwd<128>, st, B, p, 1024, G<128>::BTOTAL)) return e;
+    if (p.NB > 1) {
+        const size_t n = static_cast<size_t>(B) * C;
+        hipLaunchKernelGGL(block_rows, dim3(static_cast<unsigned>((n + 255) / 256), 2), dim3(256), 0, st, p.NB, n, p.gw32, p.gu32, gw, gu);
+    }
+    return launch_status();
 }
 
 }  // namespace rwkv

@@ -5,7 +5,7 @@ two segments and of more, and many blocks.
 Tolerances.  wkv5, wkv5a fp32: 1e-5 relative to the largest element and to the RMS, the bar of these operators' other tests; a block's
 state is a sum in another order, of the same products.  rwkv7: fp32 results 4e-7 (some four to eight roundings of 2^-24 a result, as
 without blocks; a state at a border is one more product over 64 channels), dw 3e-7 a chunk adding up as a random walk, bf16 results the
-rounding of the output."""
+rounding of the output.  wkv5 bf16: the bar of the other bf16 kernels, no further from fp64 than fp32 arithmetic with rounded outputs."""
 import math
 
 import pytest
@@ -15,9 +15,9 @@ from oracle import err_ratio, max_rel_to_peak
 from oracle import wkv5a as A
 from oracle import wkv56 as O
 from rwkv_cuda_amd import rwkv7_fast_fused as R
-from rwkv_cuda_amd import wkv5, wkv5a
+from rwkv_cuda_amd import synth, wkv5, wkv5_bf16, wkv5a
 from rwkv_cuda_amd._call import call
-from _gpu_util import DEV, garbage
+from _gpu_util import DEV, assert_no_worse, garbage
 
 pytestmark = pytest.mark.gpu
 
@@ -164,3 +164,24 @@ def test_rwkv7_heads_that_blocks_cannot_carry_are_done_as_a_whole(lib, which, dt
         assert not bool((head(whole, 1).isfinite() & ~head(blocks, 1).isfinite()).any()), z
         assert bool(head(blocks, 2).isfinite().all()) and not torch.equal(head(blocks, 2), garbage((1,), dtype).expand_as(head(blocks, 2)))
     assert bool((head(res[1][0], 0) == 0).all())
+
+
+@pytest.mark.parametrize("B,H,T", [(1, 2, 321), (1, 1, 384), (2, 1, 385), (1, 3, 449), (1, 9, 700)])
+@pytest.mark.parametrize("decays", ["usual", "fast", "mixed"])             # one reference a chunk; up to one per half chunk; some heads step by step
+def test_wkv5_bf16_heads_of_128(lib, decays, B, H, T):
+    C = H * 128
+    assert lib.rwkv_wkv5s_blocks_workspace_bytes(B, T, C, H, 0) > 0 and lib.rwkv_wkv5s_blocks_workspace_bytes(B, T, C, H, 1) > 0, "not in blocks"
+    print(f"\nwkv5 N=128 B={B} H={H} T={T} {decays}", flush=True)
+    r, k, v, w, u, gy = synth.wkv5_inputs(B, T, C, H, seed=T)
+    if decays != "usual":
+        lo, hi = {"fast": (-1.0, 2.18), "mixed": (-6.0, 2.3)}[decays]
+        w = (torch.rand(w.shape, generator=torch.Generator().manual_seed(5)) * (hi - lo) + lo).to(w.dtype)
+    ref = O.wkv5_grads(B, T, C, H, r, k, v, w, u, gy)
+    emu = O.emulate_wkv5_bf16(B, T, C, H, r, k, v, w, u, gy)
+    t = [x.to(DEV).requires_grad_(True) for x in (r, k, v, w, u)]
+    y = wkv5_bf16.RUN_CUDA(B, T, C, H, *t)
+    y.backward(gy.to(DEV))
+    with torch.no_grad():                                   # a forward that keeps no states is cut in the same way
+        assert torch.equal(wkv5_bf16.RUN_CUDA(B, T, C, H, *t), y)
+    for name, a, e, g in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, [y] + [x.grad for x in t]):
+        assert_no_worse(name, a, e.reshape(a.shape), g.reshape(a.shape))
