@@ -18,7 +18,7 @@ _INCLUDE = os.path.join(_ROOT, "include")
 LIB_PATH = os.path.join(_HERE, "librwkv_hip.so")
 HASH_PATH = LIB_PATH + ".srchash"        # digest of the sources the library was built from (content, not mtime)
 
-SOURCES = ["abi.hip", "wkv56.hip", "wkv6_fwd.hip", "wkv6_bwd_a.hip", "wkv6_bwd_b.hip", "wkv6_fwd_f.hip", "wkv6_bwd_f.hip", "wkv4.hip", "timex.hip", "wkv5_f32.hip", "wkv5_bf.hip", "rwkv7.hip", "rwkv7_chunk.hip"]
+SOURCES = ["abi.hip", "wkv56.hip", "wkv6_fwd.hip", "wkv6_bwd_a.hip", "wkv6_bwd_b.hip", "wkv6_fwd_f.hip", "wkv6_bwd_f.hip", "wkv6_local.hip", "wkv4.hip", "timex.hip", "wkv5_f32.hip", "wkv5_bf.hip", "rwkv7.hip", "rwkv7_chunk.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -45,7 +45,7 @@ HIPCC_FLAGS = [
 # rwkv7c_bwd: a reload in the chunk loop waits for the state that the same wave has asked for, so none.
 # The one-sweep kernels let the compiler count their waits: a spill inside their loops would put scratch traffic between a
 # prefetch and its use (and a forward variant that spilled eleven registers gave wrong results): none may spill.
-SPILL_LIMIT = {"wkv6_bwd_fused": 0, "wkv6_fwd_fused": 0, "wkv6_fwd_ws": 0, "wkv6_bwd_a_ws": 0, "wkv6_bwd_b_wsILi0E": 3, "wkv6_bwd_b_wsILi1E": 1, "wkv6_bwd_b_wsILi2E": 1,
+SPILL_LIMIT = {"wkv6_local": 0, "wkv6_bwd_fused": 0, "wkv6_fwd_fused": 0, "wkv6_fwd_ws": 0, "wkv6_bwd_a_ws": 0, "wkv6_bwd_b_wsILi0E": 3, "wkv6_bwd_b_wsILi1E": 1, "wkv6_bwd_b_wsILi2E": 1,
                "wkv_rows": 0, "wkv5_steps": 0, "wkv5b_fwd": 0, "wkv5b_bwd": 0, "wkv5b_local": 0, "wkv5c_fwd": 0, "wkv5c_bwdILb0E": 6, "wkv5c_bwdILb1E": 9, "wkv4_fwd_reg": 0, "wkv4_bwd_reg": 0, "timex_conv_h2": 0, "timex_gw_sum_h2": 0,
                "timex_conv_any": 0, "timex_gw_any": 2, "rwkv7c_fwd": 0, "rwkv7c_bwd": 0, "rwkv7c_local": 0, "rwkv7c_scan": 0}
 

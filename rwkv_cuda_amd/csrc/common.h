@@ -177,11 +177,18 @@ int launch_wkv6_fwd_chunk(hipStream_t st, int wmode, int B, int T, int C, int H,
 // wkv6_fwd_f.hip: the forward that goes with wkv6_bwd_f.hip (raw bf16 decay, head size 64): y and the state entering
 // every second chunk; flags [B*H][8] names the (batch, head) pairs that have to be redone by the kernel above
 // NB > 1: the sequences in NB blocks of TB tokens, one workgroup per (batch, head, block): local states, a scan, the outputs
-// (blk_state, s32: [B*H*NB][64][64] floats each, blk_decay: [B*H*NB][64]; flags cleared by the caller)
+// (blk_state, s32: [B*H*NB][64][64] floats each, blk_decay: [B*H*NB][64])
 int launch_wkv6_fwd_fused(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v,
                           const uint16_t* w, const uint16_t* u, const uint16_t* s0, uint16_t* y, char* saved, int* flags,
                           int NB = 1, int TB = 0, float* blk_state = nullptr, float* blk_decay = nullptr, float* s32 = nullptr,
                           float* decay_out = nullptr);
+// wkv6_local.hip: the first of these, for either direction (backward: key = r, val = gy); flags are cleared
+int launch_wkv6_local(hipStream_t st, bool reverse, bool head_decay, int B, int T, int C, int H, int NB, int TB, const uint16_t* key, const uint16_t* val,
+                      const uint16_t* w, float* state, float* decay, int* flags);
+// As many blocks as this at most: what enters a block is added up by the kernel that starts from there, while its loads are under way.  B1 H32
+// T3001, 8 blocks, forward + backward 109.5 us with wkv6_scan between (4.3 us each way), 106.3 without; B1 H8 T2000, 16 blocks, forward
+// 30.7 and 30.1; a step of the sum takes about 0.7 us.
+constexpr int SCAN_BLOCKS = 16;
 int launch_wkv6_scan_reverse(hipStream_t st, int BH, int NB, const float* local, const float* logdec, float* out);
 int launch_wkv6_bwd_a_chunk(hipStream_t st, int wmode, int B, int T, int C, int H, const uint16_t* r,
                             const uint16_t* k, const uint16_t* v, const void* w, const uint16_t* u,

@@ -978,14 +978,6 @@ __global__ __launch_bounds__(256) void bf16_batch_sum(int B, int C, const uint16
 }
 
 size_t round16(size_t x) { return (x + 15) & ~static_cast<size_t>(15); }
-// a fill kernel rather than hipMemsetAsync, which a caller's graph capture replays unreliably
-__global__ void zero_words_kernel(int* p, size_t n) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-void zero_words(hipStream_t st, int* p, size_t n) {
-    hipLaunchKernelGGL(zero_words_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, p, n);
-}
 
 // ---- wkv5 with heads of 128 channels on the matrix-core kernels: every head as four heads of 64, two launches per kernel,
 //      each leaving one fp32 term of every output element (see ArgsB in wkv6_chunk.h); the terms are added here
@@ -1423,7 +1415,6 @@ int rwkv_wkv6f_forward(void* stream, int B, int T, int C, int H, const rwkv_bf16
         float* local = reinterpret_cast<float*>(sb + saved_states_bytes(B, T, H) + nflag);
         float* s32 = local + nq * 64 * 64;
         float* logdec = s32 + nq * 64 * 64;
-        zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w, u, s, y, static_cast<char*>(saved), flg, NB, TB, local, logdec, s32)) return e;
     } else if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w, u, s, y, static_cast<char*>(saved), flg)) return e;
     return launch_wkv6_fwd_chunk(st, W_RAW, B, T, C, H, r, k, v, w, u, s, y, static_cast<char*>(saved), flg);
@@ -1467,7 +1458,6 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H, const rw
         float* ds32 = local + nq * 64 * 64;
         float* logdec = ds32 + nq * 64 * 64;
         gu32 = logdec + nq * 64;
-        zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w, u, gy, gr, gk, gv, gw, pu, gs, static_cast<const char*>(saved), flg,
                                           NB, TB, local, logdec, ds32, gu32)) return e;
     } else if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w, u, gy, gr, gk, gv, gw, pu, gs, static_cast<const char*>(saved), flg)) return e;
@@ -1540,7 +1530,6 @@ int rwkv_wkv5s_forward_ws(void* stream, int B, int T, int C, int H, const rwkv_b
         float* local = reinterpret_cast<float*>(sb + saved_states_bytes(B, T, H) + nflag);
         float* s32 = local + nq * 64 * 64;
         float* logdec = s32 + nq * 64 * 64;
-        zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, NB, TB, local, logdec, s32, decay)) return e;
     } else if (int e = launch_wkv6_fwd_fused(st, B, T, C, H, r, k, v, w_raw, u, nullptr, y, static_cast<char*>(saved), flg, 1, 0, nullptr, nullptr, nullptr, decay)) return e;
     // the heads that run step by step (before wkv5_bf.hip, whose states may lie where the flag words are), then a strong layer
@@ -1598,7 +1587,6 @@ int rwkv_wkv5s_backward(void* stream, int B, int T, int C, int H, const rwkv_bf1
         float* logdec = ds32 + nq * 64 * 64;
         float* gu32 = logdec + nq * 64;
         float* gw32 = gu32 + static_cast<size_t>(NB) * B * C;
-        zero_words(st, flg, static_cast<size_t>(B) * H * 8);
         if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, nullptr, pu, nullptr, static_cast<const char*>(saved), flg,
                                           NB, TB, local, logdec, ds32, gu32, pw, gw32)) return e;
     } else if (int e = launch_wkv6_bwd_fused(st, B, T, C, H, r, k, v, w_raw, u, gy, gr, gk, gv, nullptr, pu, nullptr, static_cast<const char*>(saved), flg,

@@ -47,7 +47,6 @@ constexpr int DEPTH = 2;           // chunks that the prep waves load ahead (fou
 constexpr int KEPT = 3;            // iterations between the preparation of a chunk and its finishing
 constexpr int TRIP = 6;            // iterations per trip of the prep loop: a multiple of both, so that the registers of the
                                    // loads in flight and of what is kept for the finishing have fixed names (no copies)
-template <bool LOCAL> constexpr int trip = LOCAL ? DEPTH : TRIP;      // (LOCAL: nothing is finished)
 constexpr int TQ = 20;             // causal tiles [t][s], 32 bf16 and 16 bytes of padding: 80 B (16-byte reads of 16 rows hit all banks once)
 
 struct alignas(16) SlotG {
@@ -85,14 +84,12 @@ struct ArgsG {
     uint16_t *gr, *gk, *gv, *gw, *gu, *gs;
     const char* saved;             // [B*H][ceil(n/2)] saved states (SAVED_STATE_B bytes each): the forward state entering every even chunk
     int* flags;                    // [B*H][8]
-    // Sequences cut into NB blocks of TB tokens (a multiple of 64), one workgroup per (batch, head, block), see
-    // wkv6_fwd_f.hip.  LOCAL = true leaves in blk_ds the gradient state that a block builds from nothing, going down from
-    // its end, and in blk_decay the log2 of its total decay; wkv6_scan (reverse) turns these into the gradient state
-    // that enters every block from above (ds32); LOCAL = false then starts each block from there.
-    int NB, TB;
+    // Sequences cut into NB blocks of TB tokens (a multiple of 64), one workgroup per (batch, head, block): wkv6_local leaves the gradient
+    // state that every block builds from nothing, going down from its end, and the log2 of its total decay; what enters a block from
+    // above is added up here or, with more than SCAN_BLOCKS, by wkv6_scan (ds32, reverse).
+    int NB, TB, blk;
     const float* ds32;             // [B*H][NB][64][64], [value][key], or null
-    float* blk_ds;                 // [B*H][NB][64][64]
-    float* blk_decay;              // [B*H][NB][64]
+    const float *local, *logdec;   // [B*H][NB][64][64], [B*H][NB][64], or null
     float* gu32;                   // NB > 1: gu of this (batch, head, block) in fp32 (the blocks are added before rounding)
     bool first, above;             // this is block 0; there is a block above this one
     // wkv5: w is one raw decay per channel, [H][64], and its gradient is summed over the tokens: a row per batch row in
@@ -136,7 +133,7 @@ DEVINL void expand_saved(const SavedRaw& q, f32x4 (&x)[4]) {
 
 // ---------------------------------------------------------------------------------------------------- P waves
 // wave w (0..7): channels 8w..8w+7; lane = 16 * (channel pair) + token: a thread has two channels of tokens tp and tp + 16
-template <int WMODE, bool LOCAL>
+template <int WMODE>
 DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, const size_t base, const int h, const size_t bh, const int n, const int nit) {
     // jq, tp (and hl, rw below) are redefined behind an empty asm in every iteration, see role_sd
     int jq = lane >> 4, tp = lane & 15;
@@ -166,9 +163,7 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
     // (HD: the r waves keep their second load, of the head's decay row at every token - a cache hit - so that all prep waves
     //  run the same loads and the waits count the same; the decay itself is read once, below)
     const char* __restrict__ pB = reinterpret_cast<const char*>(lower ? (HD ? static_cast<const uint16_t*>(a.w) + h * N : static_cast<const uint16_t*>(a.w) + base) : a.v + base);   // w | v
-    // LOCAL: a gradient state takes no k and no v (as in wkv6_fwd_f.hip: one row of them that hits the cache, and no K').  B1 T3001 C2048:
-    // 27.1 -> 22.9 us, 19.3 with two iterations past the last chunk instead of up to eight.
-    const uint32_t amask = (LOCAL && !lower) ? 127u : ~0u, bmask = (lower ? HD : LOCAL) ? 127u : ~0u;
+    const uint32_t bmask = lower && HD ? 127u : ~0u;
     const char* __restrict__ pC = reinterpret_cast<const char*>(a.gy + base);
     const uint32_t row_b = 2u * static_cast<uint32_t>(a.C);                                     // bytes from a token to the next
     uint32_t offA = (8 * (w & 3) + (lane >> 3)) * row_b + 16 * (lane & 7);                      // rows 8 (w & 3) .. +7
@@ -184,7 +179,7 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
     auto fetch = [&](const int c, Raw& x) __attribute__((always_inline)) {
         const uint32_t cb = static_cast<uint32_t>(c * L) * row_b;
         const uint32_t o = min(cb + offA, lastA), og = min(cb + offG, lastA);
-        x.a = *reinterpret_cast<const u32x4*>(pA + (o & amask));
+        x.a = *reinterpret_cast<const u32x4*>(pA + o);
         x.b = *reinterpret_cast<const u32x4*>(pB + (o & bmask));
         x.c = *reinterpret_cast<const u32x4*>(pC + og);    // (both halves of the wave ask for the same four rows)
     };
@@ -206,7 +201,6 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
     struct Held { uint32_t r[2], k[2]; float ea[2][2], eb[2][2], lf[2][2]; };
     Held hq[3] = {};
     bool any_exact = false, met_ok = true;
-    float logdec[2] = {0.f, 0.f};          // LOCAL: log2 of the decay over the whole block
     float carry[2] = {0.f, 0.f}, gu_acc[2] = {0.f, 0.f}, gw_acc[2] = {0.f, 0.f};
     // HD: the factors of every whole chunk are the same: the sums along time are products, the exponentials are taken once
     float lamc[2] = {0.f, 0.f}, eac[2][2] = {}, ebc[2][2] = {}, dc[2] = {0.f, 0.f}, lfc[2] = {0.f, 0.f};
@@ -251,7 +245,6 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
 #pragma unroll
                 for (int z = 0; z < 2; ++z) { ea[e][z] = eac[e][z]; eb[e][z] = ebc[e][z]; }
             a0 = dc[0]; a1 = dc[1]; b0 = dc[0]; b1 = dc[1];
-            if constexpr (LOCAL) { logdec[0] += 32.f * lamc[0]; logdec[1] += 32.f * lamc[1]; }
         } else {
             float cc[2][2];
 #pragma unroll
@@ -269,7 +262,6 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
                 cc[1][z] = p1 - lam[1][z];
                 l1[z] = bc<0>(s0);
                 l2[z] = bc<15>(p1);
-                if constexpr (LOCAL) logdec[z] += l1[z] + l2[z];
             }
             {
                 const bool bad = (-l1[0] > RANGE_LIMIT * LOG2E) || (-l2[0] > RANGE_LIMIT * LOG2E) || (-l1[1] > RANGE_LIMIT * LOG2E) || (-l2[1] > RANGE_LIMIT * LOG2E);
@@ -304,8 +296,7 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
 #pragma unroll
         for (int e = 0; e < 2; ++e) { lds_st<uint32_t>(so + O_RPH + e * 16 * ROW_B + b_tp, r0[e].h); lds_st<uint32_t>(so + O_RPL + e * 16 * ROW_B + b_tp, r0[e].l); }
 #pragma unroll
-        for (int e = 0; e < (LOCAL ? 0 : 2); ++e) { lds_st<uint32_t>(so + O_KPH + e * 16 * ROW_B + b_tp, k0[e].h); lds_st<uint32_t>(so + O_KPL + e * 16 * ROW_B + b_tp, k0[e].l); }
-        if constexpr (LOCAL) return;
+        for (int e = 0; e < 2; ++e) { lds_st<uint32_t>(so + O_KPH + e * 16 * ROW_B + b_tp, k0[e].h); lds_st<uint32_t>(so + O_KPL + e * 16 * ROW_B + b_tp, k0[e].l); }
         allreduce2_rows(ruk[0], ruk[1]);                       // sums over the four channel pairs of this wave
         if (jq == 0) { lds_st<float>(so + O_RUK + w * (4 * L) + b_l, ruk[0]); lds_st<float>(so + O_RUK + w * (4 * L) + 64 + b_l, ruk[1]); }
     };
@@ -376,7 +367,6 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
     // covers everything).  Below chunk 0 the rows that are staged all count as dead, in the planes of a slot that nobody reads any
     // more (c < 0: the slot of chunk c + 3, whose products were done in the iteration before), and nothing is prepared (which neither
     // loads nor touches the ring).
-    constexpr int TRIP = trip<LOCAL>;
     for (int it0 = 0; it0 < nit; it0 += TRIP)
         static_for<TRIP>([&](auto Z) {
             constexpr int z = decltype(Z)::value % DEPTH, zk = decltype(Z)::value % KEPT;
@@ -384,62 +374,52 @@ DEVINL void role_prep(SmemG& S, const ArgsG& a, const int lane, const int w, con
             const int cp = n - 1 - it;
             asm volatile("" : "+v"(jq), "+v"(tp), "+v"(rq), "+v"(pc), "+v"(rg), "+v"(offA), "+v"(offG));
             opaque(b_row); opaque(b_rowg); opaque(b_tp); opaque(b_ch); opaque(b_l); opaque(b_x);
-            const bool fin = !LOCAL && it >= 3 && cp + 3 >= 0;      // chunk cp + 3 is finished in this iteration
+            const bool fin = it >= 3 && cp + 3 >= 0;      // chunk cp + 3 is finished in this iteration
             if ((cut && it == 0) || cp < 0) stage_in(cp, ring[z], part); else stage_in(cp, ring[z], full);
             meet_signal(&S.met[0], lane);
             __builtin_amdgcn_sched_barrier(0);
             fetch(cp >= DEPTH ? cp - DEPTH : 0, ring[z]);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (!LOCAL) {
-                if (it == 3 && a.above) {
-                    // P at the end of the block, from the gradient state that enters from above and the saved state there
-                    const f32x2 p2 = lds_ld<f32x2>(sb + PEX0 + ((n >> 1) & 1) * (4 * N) + b_ch);
-                    carry[0] = p2.x; carry[1] = p2.y;
-                }
-                if (fin) { if (cut && it == 3) finish(cp + 3, hq[zk], part); else finish(cp + 3, hq[zk], full); }
-                meet_signal(&S.met[1], lane);
+            if (it == 3 && a.above) {
+                // P at the end of the block, from the gradient state that enters from above and the saved state there
+                const f32x2 p2 = lds_ld<f32x2>(sb + PEX0 + ((n >> 1) & 1) * (4 * N) + b_ch);
+                carry[0] = p2.x; carry[1] = p2.y;
             }
+            if (fin) { if (cut && it == 3) finish(cp + 3, hq[zk], part); else finish(cp + 3, hq[zk], full); }
+            meet_signal(&S.met[1], lane);
             __builtin_amdgcn_sched_barrier(0);
             met_ok = meet_wait(&S.met[0], 8u * (it + 1)) && met_ok;        // all rows of chunk cp are staged
             if (cut && it == 0) prep(cp, hq[zk], part); else if (cp >= 0) prep(cp, hq[zk], full);
             __syncthreads();
         });
     // (a meeting that never completed, which the counting excludes, would leave this head to the two-sweep kernels)
-    // (with several blocks per head the words are cleared by the caller and only ever set)
+    // (with several blocks per head the words are cleared before, by wkv6_local, and only ever set)
     // (S.met[3]: a meeting of the E waves that never completed; written before the last barrier)
     const bool flag = any_exact || !met_ok || S.met[3] != 0;
     if (lane == 0 && (a.NB == 1 || flag)) a.flags[bh * 8 + w] = flag ? 1 : 0;
-    if constexpr (LOCAL) {
-        if (tp == 0) *reinterpret_cast<float2*>(a.blk_decay + ch0) = make_float2(logdec[0], logdec[1]);
-    } else {
-        // gu of this batch row (and block): sum over the tokens (lanes of a row)
+    // gu of this batch row (and block): sum over the tokens (lanes of a row)
 #pragma unroll
-        for (int z = 0; z < 2; ++z) gu_acc[z] = row_sum_to_last(gu_acc[z]);
+    for (int z = 0; z < 2; ++z) gu_acc[z] = row_sum_to_last(gu_acc[z]);
+    if (tp == 15) {
+        if (a.gu32 != nullptr) *reinterpret_cast<float2*>(a.gu32 + ch0) = make_float2(gu_acc[0], gu_acc[1]);
+        else *reinterpret_cast<uint32_t*>(a.gu + ch0) = pack_bf2(gu_acc[0], gu_acc[1]);
+    }
+    if (HD) {
+#pragma unroll
+        for (int z = 0; z < 2; ++z) gw_acc[z] = row_sum_to_last(gw_acc[z]);
         if (tp == 15) {
-            if (a.gu32 != nullptr) *reinterpret_cast<float2*>(a.gu32 + ch0) = make_float2(gu_acc[0], gu_acc[1]);
-            else *reinterpret_cast<uint32_t*>(a.gu + ch0) = pack_bf2(gu_acc[0], gu_acc[1]);
-        }
-        if (HD) {
-#pragma unroll
-            for (int z = 0; z < 2; ++z) gw_acc[z] = row_sum_to_last(gw_acc[z]);
-            if (tp == 15) {
-                if (a.gw32 != nullptr) *reinterpret_cast<float2*>(a.gw32 + ch0) = make_float2(gw_acc[0], gw_acc[1]);
-                else *reinterpret_cast<uint32_t*>(a.gwp + ch0) = pack_bf2(gw_acc[0], gw_acc[1]);
-            }
+            if (a.gw32 != nullptr) *reinterpret_cast<float2*>(a.gw32 + ch0) = make_float2(gw_acc[0], gw_acc[1]);
+            else *reinterpret_cast<uint32_t*>(a.gwp + ch0) = pack_bf2(gw_acc[0], gw_acc[1]);
         }
     }
 }
 
 // ---------------------------------------------------------------------------------------------------- SD waves
-template <int WMODE, bool LOCAL>
+template <int WMODE>
 DEVINL void role_sd(SmemG& S, const ArgsG& a, const int lane, const int w, const size_t bh, const int n, const int nit) {
     const int g = lane >> 4, l16 = lane & 15, j = 16 * w + l16;
     const int nseg = (n + 1) / 2;
     const char* __restrict__ sv = a.saved;                                      // the saved states of this block
-    if constexpr (LOCAL) {                 // only the E waves have work
-        for (int it = 0; it < nit; ++it) __syncthreads();
-        return;
-    }
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
     const lds_t sb = lds_of(&S);
     // per-lane address parts
@@ -566,8 +546,19 @@ DEVINL void role_sd(SmemG& S, const ArgsG& a, const int lane, const int w, const
         }
     };
 
-    if (a.ds32 != nullptr) {
-        load_state(a.ds32, b_sv, D);       // the gradient state that enters the block from above
+    if (a.ds32 != nullptr || a.local != nullptr) {
+        // the gradient state that enters the block from above
+        if (a.ds32 != nullptr) load_state(a.ds32, b_sv, D);
+        else
+            for (int m = a.NB - 1; m > a.blk; --m) {
+                f32x4 y[4];
+                load_state(a.local + m * (N * N), b_sv, y);
+                const float e = exp2_fast(a.logdec[m * N + j]);
+#pragma unroll
+                for (int tl = 0; tl < 4; ++tl)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) D[tl][v] = fmaf(D[tl][v], e, y[tl][v]);
+            }
         if (a.above) {
             // P there, with the forward state at the end of the block (the first saved state of the block above)
             fetch_saved(sv + static_cast<size_t>(n >> 1) * SAVED_STATE_B, w, b_q, Sq);
@@ -611,7 +602,7 @@ DEVINL void role_sd(SmemG& S, const ArgsG& a, const int lane, const int w, const
 }
 
 // ---------------------------------------------------------------------------------------------------- E waves
-template <int WMODE, bool LOCAL>
+template <int WMODE>
 DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const size_t base, const int n, const int nit) {
     constexpr bool HD = WMODE == W_HEAD;
     const int g = lane >> 4, l16 = lane & 15;
@@ -638,9 +629,20 @@ DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const 
     bool met_ok = true;
     f32x4 E[4] = {zero4, zero4, zero4, zero4};     // dS[i = 16w + l16][j = 16 tile + 4g + v]
     const uint32_t b_e = (16 * w + l16) * N + 4 * g;                            // that element of a [value][key] state
-    if (!LOCAL && a.ds32 != nullptr) {
+    if (a.ds32 != nullptr) {
 #pragma unroll
         for (int tl = 0; tl < 4; ++tl) E[tl] = *reinterpret_cast<const f32x4*>(a.ds32 + b_e + 16 * tl);
+    } else if (a.local != nullptr) {
+        for (int m = a.NB - 1; m > a.blk; --m) {
+            const float* y = a.local + m * (N * N) + b_e;
+            const float* d = a.logdec + m * N + 4 * g;
+#pragma unroll
+            for (int tl = 0; tl < 4; ++tl) {
+                const f32x4 e = *reinterpret_cast<const f32x4*>(d + 16 * tl), z = *reinterpret_cast<const f32x4*>(y + 16 * tl);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) E[tl][v] = fmaf(E[tl][v], exp2_fast(e[v]), z[v]);
+            }
+        }
     }
 
     // causal tiles of chunk c, quadrants (t, s) = (0,0) (1,0) (1,1); accumulator rows are s, lanes t.  A = tril(K' R'^T) with
@@ -731,10 +733,9 @@ DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const 
                 de[q] = lds_ld<float>(so + O_DEC + 64 * q + b_g);
                 d1[q] = lds_ld<float>(so + O_D1 + 64 * q + b_g);
             }
-            // (LOCAL: only the gradient state is wanted, everything that serves gv is left out)
             bf16x8 kh[2][2], kl[2][2];
 #pragma unroll
-            for (int tt = 0; tt < (LOCAL ? 0 : 2); ++tt)
+            for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
                 for (int ks = 0; ks < 2; ++ks) {
                     kh[tt][ks] = ld_acc(so + O_KPH + tt * 16 * ROW_B + 64 * ks + b_acc);
@@ -744,7 +745,7 @@ DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const 
             // ------------------------------------------------------------ gv^T[i][s] = (dS d2) K'^T + GY^T A
             bf16x8 dh[2], dl[2];
 #pragma unroll
-            for (int ks = 0; ks < (LOCAL ? 0 : 2); ++ks) {
+            for (int ks = 0; ks < 2; ++ks) {
                 float p[4], q[4];
                 static_for<4>([&](auto V) {
                     constexpr int v = decltype(V)::value;
@@ -760,11 +761,11 @@ DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const 
             const bf16x8 gyo = ld_tr(so + O_GY + 32 * w + b_tr, ROW_B);        // lane = value channel 16w + l16, K = tokens
             bf16x8 ah[2], al[2];
 #pragma unroll
-            for (int tt = 0; tt < (LOCAL ? 0 : 2); ++tt) { ah[tt] = ld_tr(to + T_AH + 32 * tt + b_trt, TROW_B); al[tt] = ld_tr(to + T_AL + 32 * tt + b_trt, TROW_B); }
+            for (int tt = 0; tt < 2; ++tt) { ah[tt] = ld_tr(to + T_AH + 32 * tt + b_trt, TROW_B); al[tt] = ld_tr(to + T_AL + 32 * tt + b_trt, TROW_B); }
             __builtin_amdgcn_sched_barrier(0);
             f32x4 G[2] = {zero4, zero4};
 #pragma unroll
-            for (int ks = 0; ks < (LOCAL ? 0 : 2); ++ks)
+            for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
                 for (int tt = 0; tt < 2; ++tt) {
                     G[tt] = mfma(dh[ks], kh[tt][ks], G[tt]);
@@ -778,7 +779,7 @@ DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const 
             for (int tl = 0; tl < 4; ++tl) { rh[tl] = ld_tr(so + O_RPH + 32 * tl + b_tr, ROW_B); rl[tl] = ld_tr(so + O_RPL + 32 * tl + b_tr, ROW_B); }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int tt = 0; tt < (LOCAL ? 0 : 2); ++tt) {
+            for (int tt = 0; tt < 2; ++tt) {
                 G[tt] = mfma(gyo, ah[tt], G[tt]);
                 G[tt] = mfma(gyo, al[tt], G[tt]);
             }
@@ -792,7 +793,7 @@ DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const 
             // gv: lane = token, four consecutive value channels in registers (the rows of the last chunk were taken out of
             // `out` before the barrier)
 #pragma unroll
-            for (int tt = 0; tt < (LOCAL ? 0 : 2); ++tt)
+            for (int tt = 0; tt < 2; ++tt)
                 lds_st<u32x2>(sb + OUT0 + 3 * PLANE_B + tt * 16 * ROW_B + 32 * w + b_acc, u32x2{pack_bf2(G[tt][0], G[tt][1]), pack_bf2(G[tt][2], G[tt][3])});
             // ------------------------------------------------------------ dS^T <- dS^T dec + d1 R'^T GY
 #pragma unroll
@@ -806,37 +807,29 @@ DEVINL void role_e(SmemG& S, const ArgsG& a, const int lane, const int w, const 
                 });
         }
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!LOCAL) {
-            // gv of chunk c, when all four E waves have written their channels
-            meet_signal(&S.met[2], lane);
-            met_ok = meet_wait(&S.met[2], 4u * (it + 1)) && met_ok;
-            const u32x4 o = lds_ld<u32x4>(sb + OUT0 + 3 * PLANE_B + b_row);
-            if (it >= 2 && c >= 0 && c * L + 8 * w + (lane >> 3) < T) *reinterpret_cast<u32x4*>(pgv + (static_cast<uint32_t>(c * L) * row_b + offA)) = o;
-        }
+        // gv of chunk c, when all four E waves have written their channels
+        meet_signal(&S.met[2], lane);
+        met_ok = meet_wait(&S.met[2], 4u * (it + 1)) && met_ok;
+        const u32x4 o = lds_ld<u32x4>(sb + OUT0 + 3 * PLANE_B + b_row);
+        if (it >= 2 && c >= 0 && c * L + 8 * w + (lane >> 3) < T) *reinterpret_cast<u32x4*>(pgv + (static_cast<uint32_t>(c * L) * row_b + offA)) = o;
         __builtin_amdgcn_sched_barrier(0);
-        if (!LOCAL && it >= 1 && c - 1 >= 0) tiles(c - 1);
+        if (it >= 1 && c - 1 >= 0) tiles(c - 1);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!LOCAL) {
-            // gr, gk, gw of chunk c + 1, when all eight prep waves have finished their columns
-            met_ok = meet_wait(&S.met[1], 8u * (it + 1)) && met_ok;
-            const u32x4 o0 = lds_ld<u32x4>(sb + OUT0 + b_row), o1 = lds_ld<u32x4>(sb + OUT0 + PLANE_B + b_row), o2 = lds_ld<u32x4>(sb + OUT0 + 2 * PLANE_B + b_row);
-            if (it >= 3 && c + 1 >= 0 && (c + 1) * L + 8 * w + (lane >> 3) < T) {
-                const uint32_t ob = static_cast<uint32_t>((c + 1) * L) * row_b + offA;
-                *reinterpret_cast<u32x4*>(pgr + ob) = o0;
-                *reinterpret_cast<u32x4*>(pgk + ob) = o1;
-                if (!HD) *reinterpret_cast<u32x4*>(pgw + ob) = o2;
-            }
+        // gr, gk, gw of chunk c + 1, when all eight prep waves have finished their columns
+        met_ok = meet_wait(&S.met[1], 8u * (it + 1)) && met_ok;
+        const u32x4 o0 = lds_ld<u32x4>(sb + OUT0 + b_row), o1 = lds_ld<u32x4>(sb + OUT0 + PLANE_B + b_row), o2 = lds_ld<u32x4>(sb + OUT0 + 2 * PLANE_B + b_row);
+        if (it >= 3 && c + 1 >= 0 && (c + 1) * L + 8 * w + (lane >> 3) < T) {
+            const uint32_t ob = static_cast<uint32_t>((c + 1) * L) * row_b + offA;
+            *reinterpret_cast<u32x4*>(pgr + ob) = o0;
+            *reinterpret_cast<u32x4*>(pgk + ob) = o1;
+            if (!HD) *reinterpret_cast<u32x4*>(pgw + ob) = o2;
         }
         if (!met_ok && lane == 0) S.met[3] = 1;        // (the prep waves read it after the last barrier and flag the head)
         __syncthreads();
     }
-    if constexpr (LOCAL) {
-#pragma unroll
-        for (int tl = 0; tl < 4; ++tl) *reinterpret_cast<f32x4*>(a.blk_ds + b_e + 16 * tl) = E[tl];
-    }
 }
 
-template <int WMODE, bool LOCAL>
+template <int WMODE>
 __global__ __launch_bounds__(NTG) void wkv6_bwd_fused(const ArgsG arg) {
     __shared__ SmemG S;
     const int tid = threadIdx.x;
@@ -860,7 +853,7 @@ __global__ __launch_bounds__(NTG) void wkv6_bwd_fused(const ArgsG arg) {
     a.first = blk == 0;
     a.above = blk + 1 < arg.NB;
     if (arg.ds32 != nullptr) a.ds32 = arg.ds32 + bq * (N * N);
-    if (arg.blk_ds != nullptr) { a.blk_ds = arg.blk_ds + bq * (N * N); a.blk_decay = arg.blk_decay + bq * N; }
+    if (arg.local != nullptr) { a.local = arg.local + bh * arg.NB * (N * N); a.logdec = arg.logdec + bh * arg.NB * N; a.blk = blk; }
     // gu: a row per batch row [B][C], or per block and batch row [NB][B][C] in fp32
     if (arg.gu32 != nullptr) a.gu32 = arg.gu32 + ((static_cast<size_t>(blk) * (gridDim.x / (arg.NB * arg.H)) + b) * arg.H + h) * N;
     else a.gu = arg.gu + bh * N;
@@ -872,16 +865,16 @@ __global__ __launch_bounds__(NTG) void wkv6_bwd_fused(const ArgsG arg) {
     if (tid < 4) S.met[tid] = 0;
     __syncthreads();
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, w = wid & 3;
-    const int nit = (n + (LOCAL ? 2 : 3) + trip<LOCAL> - 1) / trip<LOCAL> * trip<LOCAL>;      // iterations of the pipeline: n + 3 (nothing to finish: n + 2), in whole trips of the prep loop
-    if (wid < 8) role_prep<WMODE, LOCAL>(S, a, lane, wid, base, h, bh, n, nit);
-    else if (wid < 12) role_sd<WMODE, LOCAL>(S, a, lane, w, bh, n, nit);
+    const int nit = (n + 3 + TRIP - 1) / TRIP * TRIP;               // iterations of the pipeline: n + 3, in whole trips of the prep loop
+    if (wid < 8) role_prep<WMODE>(S, a, lane, wid, base, h, bh, n, nit);
+    else if (wid < 12) role_sd<WMODE>(S, a, lane, w, bh, n, nit);
     else {
         // The dS waves carry the recurrence and issue little; left at the default priority they are the youngest waves of
         // their SIMDs, get the issue slots that the others leave, and the whole workgroup waits for them at every barrier
         // (measured: 5 % of their time at the barrier against 22..37 % for the others).  Ahead of the others they cost those
         // almost nothing.  (Raising the X/Z waves as well starves the prep waves: slower.)
         __builtin_amdgcn_s_setprio(2);
-        role_e<WMODE, LOCAL>(S, a, lane, w, base, n, nit);
+        role_e<WMODE>(S, a, lane, w, base, n, nit);
     }
 }
 
@@ -906,18 +899,20 @@ int launch_wkv6_bwd_fused(hipStream_t st, int B, int T, int C, int H, const uint
     a.NB = 1; a.TB = T;
     const bool hd = a.head_decay;
     if (NB <= 1) {
-        if (hd) hipLaunchKernelGGL((wkv6_bwd_fused<W_HEAD, false>), dim3(B * H), dim3(NTG), 0, st, a);
-        else hipLaunchKernelGGL((wkv6_bwd_fused<W_RAW, false>), dim3(B * H), dim3(NTG), 0, st, a);
+        if (hd) hipLaunchKernelGGL((wkv6_bwd_fused<W_HEAD>), dim3(B * H), dim3(NTG), 0, st, a);
+        else hipLaunchKernelGGL((wkv6_bwd_fused<W_RAW>), dim3(B * H), dim3(NTG), 0, st, a);
         return launch_status();
     }
-    a.NB = NB; a.TB = TB; a.blk_ds = blk_ds; a.blk_decay = blk_decay;
-    if (hd) hipLaunchKernelGGL((wkv6_bwd_fused<W_HEAD, true>), dim3(B * H * NB), dim3(NTG), 0, st, a);
-    else hipLaunchKernelGGL((wkv6_bwd_fused<W_RAW, true>), dim3(B * H * NB), dim3(NTG), 0, st, a);
-    if (int e = launch_wkv6_scan_reverse(st, B * H, NB, blk_ds, blk_decay, ds32)) return e;
-    a.blk_ds = nullptr; a.blk_decay = nullptr; a.ds32 = ds32; a.gu32 = gu32;
+    a.NB = NB; a.TB = TB;
+    if (int e = launch_wkv6_local(st, true, hd, B, T, C, H, NB, TB, r, gy, w, blk_ds, blk_decay, flags)) return e;
+    if (NB > SCAN_BLOCKS) {
+        if (int e = launch_wkv6_scan_reverse(st, B * H, NB, blk_ds, blk_decay, ds32)) return e;
+        a.ds32 = ds32;
+    } else { a.local = blk_ds; a.logdec = blk_decay; }
+    a.gu32 = gu32;
     if (gwp != nullptr) a.gw32 = gw32;
-    if (hd) hipLaunchKernelGGL((wkv6_bwd_fused<W_HEAD, false>), dim3(B * H * NB), dim3(NTG), 0, st, a);
-    else hipLaunchKernelGGL((wkv6_bwd_fused<W_RAW, false>), dim3(B * H * NB), dim3(NTG), 0, st, a);
+    if (hd) hipLaunchKernelGGL((wkv6_bwd_fused<W_HEAD>), dim3(B * H * NB), dim3(NTG), 0, st, a);
+    else hipLaunchKernelGGL((wkv6_bwd_fused<W_RAW>), dim3(B * H * NB), dim3(NTG), 0, st, a);
     if (hd) {
         const size_t n = static_cast<size_t>(B) * C;
         hipLaunchKernelGGL(block_sums, dim3(static_cast<unsigned>((n + 255) / 256), 2), dim3(256), 0, st, NB, n, gu32, gu, gw32, gwp);

@@ -60,20 +60,19 @@ struct ArgsQ {
     char* saved;                   // [B*H][ceil(n/2)] saved states (SAVED_STATE_B bytes each): the state entering every even chunk
     int* flags;                    // [B*H][8]
     // Sequences cut into NB blocks of TB tokens (a multiple of 64), one workgroup per (batch, head, block), for shapes with
-    // fewer (batch, head) pairs than the chip has CUs.  Three launches: LOCAL = true leaves in blk_state the state that a
-    // block builds from nothing and in blk_decay the log2 of its total decay per key channel; wkv6_scan turns these into
-    // the state entering every block (s32); LOCAL = false then starts each block from there.  NB = 1: one launch, TB = T.
-    int NB, TB;
+    // fewer (batch, head) pairs than the chip has CUs.  wkv6_local leaves the state that every block builds from nothing and the log2 of its
+    // total decay per key channel; the state waves add up what enters their block or, with more than SCAN_BLOCKS, wkv6_scan has (s32).
+    // NB = 1: one launch, TB = T.
+    int NB, TB, blk;
     const float* s32;              // [B*H][NB][64][64] or null
-    float* blk_state;              // [B*H][NB][64][64]
-    float* blk_decay;              // [B*H][NB][64]
+    const float *local, *logdec;   // [B*H][NB][64][64], [B*H][NB][64], or null
     bool head_decay;               // wkv5: w is one raw decay per channel, [H][64], the same at every token
     float* decay_out;              // wkv5: [2][C] fp32, exp(-exp(w)) and -exp(w), left for the two-sweep kernels and the backward
     bool first_row;                // this workgroup has batch row 0 (and block 0): it writes decay_out
 };
 
 // ---------------------------------------------------------------------------------------------------- P waves
-template <bool LOCAL, bool HD>
+template <bool HD>
 DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, const size_t base, const int h, const size_t bh, const int n, const int nit) {
     int jq = lane >> 4, tp = lane & 15;                 // arithmetic: channel pair, token (and token + 16)
     // Global memory is touched in whole 128-byte rows: eight lanes per row, eight rows per wave and instruction (waves
@@ -93,9 +92,6 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
     //  row at every token - a cache hit - so that all prep waves run the same loads and the waits count the same)
     const char* __restrict__ pB = reinterpret_cast<const char*>(lower ? (HD ? a.w + h * N : a.w + base) : a.v + base);   // w | v
     const uint32_t bmask = (HD && lower) ? 127u : ~0u;
-    // LOCAL: a state takes no r.  Its rows are not read (the loads stay, of one row that hits the cache, for the same reason), R' is not made
-    // and neither is the diagonal of A.  B1 T3001 C2048: 24.5 -> 20.8 us, 18.9 with nothing prepared past the end.
-    const uint32_t amask = (LOCAL && lower) ? 127u : ~0u;
     const uint32_t row_b = 2u * static_cast<uint32_t>(a.C);                                     // bytes from a token to the next
     uint32_t offA = (8 * (w & 3) + (lane >> 3)) * row_b + 16 * (lane & 7);                      // rows 8 (w & 3) .. +7
     const uint32_t lastA = static_cast<uint32_t>(a.T - 1) * row_b + 16 * (lane & 7);
@@ -116,7 +112,7 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
     Raw ring[DEPTH];                       // DEPTH chunks ahead
     auto fetch = [&](const int c, Raw& x) __attribute__((always_inline)) {
         const uint32_t o = min(static_cast<uint32_t>(c * L) * row_b + offA, lastA);
-        x.a = *reinterpret_cast<const u32x4*>(pA + (o & amask));
+        x.a = *reinterpret_cast<const u32x4*>(pA + o);
         x.b = *reinterpret_cast<const u32x4*>(pB + (o & bmask));
     };
     // the rows of chunk c into the slot: r, k, w where the R' hi, K' hi, R' lo planes will be (staging), v in place
@@ -130,7 +126,6 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
         meet_signal(&S.met[0], lane);
     };
     bool any_exact = false, met_ok = true;
-    float logdec[2] = {0.f, 0.f};          // LOCAL: log2 of the decay over the whole block
     // HD (wkv5): the decay of a channel is the same at every token, and so are the factors of every whole chunk: the sums
     // along time are products, the exponentials are taken once
     float lamc[2] = {0.f, 0.f}, eac[2][2] = {}, ebc[2][2] = {}, dc[2] = {0.f, 0.f};
@@ -146,7 +141,7 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
         }
         const bool bad = (-16.f * lamc[0] > RANGE_LIMIT * LOG2E) || (-16.f * lamc[1] > RANGE_LIMIT * LOG2E);
         any_exact = __ballot(bad) != 0ull;
-        if (!LOCAL && a.first_row && tp == 0) {
+        if (a.first_row && tp == 0) {
             // the wrapper-side transform of wkv5_bf16/run.py:63-64, for whoever needs the decay in that form afterwards
             const float e0 = -expf(bf_lo(x)), e1 = -expf(bf_hi(x));
             *reinterpret_cast<float2*>(a.decay_out + h * N + ch0) = make_float2(expf(e0), expf(e1));
@@ -176,7 +171,6 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
 #pragma unroll
                 for (int z = 0; z < 2; ++z) { ea[e][z] = eac[e][z]; eb[e][z] = ebc[e][z]; }
             a0 = dc[0]; a1 = dc[1]; b0 = dc[0]; b1 = dc[1];
-            if constexpr (LOCAL) { logdec[0] += 32.f * lamc[0]; logdec[1] += 32.f * lamc[1]; }
         } else {
             float cc[2][2];
 #pragma unroll
@@ -194,7 +188,6 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
                 cc[1][z] = p1 - lam[1][z];
                 l1[z] = bc<0>(s0);
                 l2[z] = bc<15>(p1);
-                if constexpr (LOCAL) logdec[z] += l1[z] + l2[z];
             }
             {
                 const bool bad = (-l1[0] > RANGE_LIMIT * LOG2E) || (-l2[0] > RANGE_LIMIT * LOG2E) || (-l1[1] > RANGE_LIMIT * LOG2E) || (-l2[1] > RANGE_LIMIT * LOG2E);
@@ -222,10 +215,9 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
         }
         // (the stores side by side, with no load between them: the compiler then pairs them, two planes or two rows an instruction)
 #pragma unroll
-        for (int e = 0; e < (LOCAL ? 0 : 2); ++e) { lds_st<uint32_t>(so + O_RPH + e * 16 * ROW_B + b_tp, r0[e].h); lds_st<uint32_t>(so + O_RPL + e * 16 * ROW_B + b_tp, r0[e].l); }
+        for (int e = 0; e < 2; ++e) { lds_st<uint32_t>(so + O_RPH + e * 16 * ROW_B + b_tp, r0[e].h); lds_st<uint32_t>(so + O_RPL + e * 16 * ROW_B + b_tp, r0[e].l); }
 #pragma unroll
         for (int e = 0; e < 2; ++e) { lds_st<uint32_t>(so + O_KPH + e * 16 * ROW_B + b_tp, k0[e].h); lds_st<uint32_t>(so + O_KPL + e * 16 * ROW_B + b_tp, k0[e].l); }
-        if constexpr (LOCAL) return;
         allreduce2_rows(ruk[0], ruk[1]);                       // sums over the four channel pairs of this wave
         if (jq == 0) { lds_st<float>(so + O_RUK + w * (4 * L) + b_l, ruk[0]); lds_st<float>(so + O_RUK + w * (4 * L) + 64 + b_l, ruk[1]); }
     };
@@ -263,23 +255,19 @@ DEVINL void role_prep(SmemQ& S, const ArgsQ& a, const int lane, const int w, con
             __builtin_amdgcn_sched_barrier(0);
             fetch(it + DEPTH < n ? it + DEPTH : n - 1, ring[z]);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (!LOCAL) store_y(it >= 3 ? it - 3 : 0, it >= 3);
+            store_y(it >= 3 ? it - 3 : 0, it >= 3);
             __builtin_amdgcn_sched_barrier(0);
             met_ok = meet_wait(&S.met[0], 8u * (it + 1)) && met_ok;      // all eight waves have staged their rows of chunk it
             if (it < n - 1) prep(it, full); else if (it < n) prep(it, part);
             __syncthreads();
         });
     // (a meeting that never completed, which the counting excludes, would leave the results of this head to the other kernel)
-    // (with several blocks per head the words are cleared by the caller and only ever set)
+    // (with several blocks per head the words are cleared before, by wkv6_local, and only ever set)
     const bool flag = any_exact || !met_ok;
     if (lane == 0 && (a.NB == 1 || flag)) a.flags[bh * 8 + w] = flag ? 1 : 0;
-    if constexpr (LOCAL) {
-        if (tp == 0) *reinterpret_cast<float2*>(a.blk_decay + ch0) = make_float2(logdec[0], logdec[1]);
-    }
 }
 
 // ---------------------------------------------------------------------------------------------------- S waves
-template <bool LOCAL>
 DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, const size_t bh, const int n, const int nit) {
     const int g = lane >> 4, l16 = lane & 15, i = 16 * w + l16;
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
@@ -291,10 +279,10 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
     const uint32_t b_sv = i * N + 4 * g;                                        // [value channel i][key channel 4 g] of a state
     lds_t b_ss = (i * SS + 4 * g) * 4;                                          // the same in the LDS copy
     f32x4 St[4];                           // S[i = 16w + l16][j = 16 tile + 4g + v]
-    if (!LOCAL && a.s32 != nullptr) {
+    if (a.s32 != nullptr) {
 #pragma unroll
         for (int tl = 0; tl < 4; ++tl) St[tl] = *reinterpret_cast<const f32x4*>(a.s32 + b_sv + 16 * tl);
-    } else if (!LOCAL && a.s0 != nullptr) {
+    } else if (a.s0 != nullptr) {
 #pragma unroll
         for (int tl = 0; tl < 4; ++tl) {
             const uint2 x = *reinterpret_cast<const uint2*>(a.s0 + bh * (N * N) + b_sv + 16 * tl);
@@ -303,6 +291,18 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
     } else {
 #pragma unroll
         for (int tl = 0; tl < 4; ++tl) St[tl] = zero4;
+    }
+    if (a.local != nullptr) {
+        const float* y = a.local + b_sv;
+        const float* d = a.logdec + 4 * g;
+#pragma unroll 2
+        for (int m = 0; m < a.blk; ++m, y += N * N, d += N)
+#pragma unroll
+            for (int tl = 0; tl < 4; ++tl) {
+                const f32x4 e = *reinterpret_cast<const f32x4*>(d + 16 * tl), z = *reinterpret_cast<const f32x4*>(y + 16 * tl);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) St[tl][v] = fmaf(St[tl][v], exp2_fast(e[v]), z[v]);
+            }
     }
     __syncthreads();                       // iterations 0 and 1: nothing prepared yet
     __syncthreads();
@@ -325,15 +325,13 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
         const lds_t so = uniform_base(sb + SLOT0 + (c % 3) * SLOT_B);
 #pragma unroll
         for (int q = 0; q < 4; ++q) dq[q] = lds_ld<float>(so + O_D1 + 64 * q + b_g);
-        if constexpr (!LOCAL) {
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    rh[tt][ks] = ld_acc(so + O_RPH + tt * 16 * ROW_B + 64 * ks + b_acc);
-                    rl[tt][ks] = ld_acc(so + O_RPL + tt * 16 * ROW_B + 64 * ks + b_acc);
-                }
-        }
+            for (int ks = 0; ks < 2; ++ks) {
+                rh[tt][ks] = ld_acc(so + O_RPH + tt * 16 * ROW_B + 64 * ks + b_acc);
+                rl[tt][ks] = ld_acc(so + O_RPL + tt * 16 * ROW_B + 64 * ks + b_acc);
+            }
     };
     ahead(0);
     ahead_late(0);
@@ -341,7 +339,7 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
     for (int c = 0; c < n; ++c) {
         opaque(b_acc); opaque(b_tr); opaque(b_natt); opaque(b_g); opaque(b_ss);
         const lds_t so = uniform_base(sb + SLOT0 + (c % 3) * SLOT_B), to = uniform_base(sb + TILE0 + (c & 1) * TILE_B);
-        if (!LOCAL && !(c & 1)) {
+        if (!(c & 1)) {
             // The state entering an even chunk goes to LDS and from there, in the next iteration, to global memory through
             // a wave that has nothing else to do: every workgroup writes its 16 KB at about the same moment, the memory
             // system takes a while to accept such a burst, and a state wave that waited for that would hold up the chunk.
@@ -351,16 +349,15 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
         // ------------------------------------------------------------ batch 1: d1, R' (natural rows), v and the A tile
         // per-channel factors: a lane holds the one of channel 16 tile + 4 g + (l16 & 3), a 4-byte read that all rows of
         // four lanes share; the products below take lane v of the 16-lane row inside the multiply (row_newbcast)
-        // (LOCAL: only the state is wanted, everything that serves y is left out)
         // (the A tile by rows: it arrives while the state is scaled and split)
         bf16x8 ah[2], al[2];
 #pragma unroll
-        for (int tt = 0; tt < (LOCAL ? 0 : 2); ++tt) { ah[tt] = ld_op(to + T_AH + tt * 16 * TROW_B + b_natt); al[tt] = ld_op(to + T_AL + tt * 16 * TROW_B + b_natt); }
+        for (int tt = 0; tt < 2; ++tt) { ah[tt] = ld_op(to + T_AH + tt * 16 * TROW_B + b_natt); al[tt] = ld_op(to + T_AL + tt * 16 * TROW_B + b_natt); }
         __builtin_amdgcn_sched_barrier(0);
         // ------------------------------------------------------------ y^T[i][t] = (S d1) R'^T + V^T A^T
         bf16x8 sh[2], sl[2];
 #pragma unroll
-        for (int ks = 0; ks < (LOCAL ? 0 : 2); ++ks) {
+        for (int ks = 0; ks < 2; ++ks) {
             float p[4], q[4];
             static_for<4>([&](auto V) {
                 constexpr int v = decltype(V)::value;
@@ -374,7 +371,7 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
         __builtin_amdgcn_sched_barrier(0);
         f32x4 Y[2] = {zero4, zero4};
 #pragma unroll
-        for (int ks = 0; ks < (LOCAL ? 0 : 2); ++ks)
+        for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt) {
                 Y[tt] = mfma(sh[ks], rh[tt][ks], Y[tt]);
@@ -388,7 +385,7 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
         for (int tl = 0; tl < 4; ++tl) { kh[tl] = ld_tr(so + O_KPH + 32 * tl + b_tr, ROW_B); kl[tl] = ld_tr(so + O_KPL + 32 * tl + b_tr, ROW_B); }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int tt = 0; tt < (LOCAL ? 0 : 2); ++tt) {
+        for (int tt = 0; tt < 2; ++tt) {
             Y[tt] = mfma(vop, ah[tt], Y[tt]);
             Y[tt] = mfma(vop, al[tt], Y[tt]);
         }
@@ -403,7 +400,7 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
         __builtin_amdgcn_sched_barrier(0);
         // y: lane = token, four consecutive value channels in registers
 #pragma unroll
-        for (int tt = 0; tt < (LOCAL ? 0 : 2); ++tt)
+        for (int tt = 0; tt < 2; ++tt)
             lds_st<u32x2>(sb + YB0 + (c & 1) * PLANE_B + tt * 16 * ROW_B + 32 * w + b_acc, u32x2{pack_bf2(Y[tt][0], Y[tt][1]), pack_bf2(Y[tt][2], Y[tt][3])});
         // ------------------------------------------------------------ S^T <- S^T dec + d2 K'^T V
 #pragma unroll
@@ -420,14 +417,9 @@ DEVINL void role_state(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
         __syncthreads();
     }
     for (int it = n + 2; it < nit; ++it) __syncthreads();      // the P waves store the last y
-    if constexpr (LOCAL) {
-#pragma unroll
-        for (int tl = 0; tl < 4; ++tl) *reinterpret_cast<f32x4*>(a.blk_state + b_sv + 16 * tl) = St[tl];
-    }
 }
 
 // ---------------------------------------------------------------------------------------------------- T waves
-template <bool LOCAL>
 DEVINL void role_tiles(SmemQ& S, const ArgsQ& a, const int lane, const int w, const size_t bh, const int n, const int nit) {
     const int g = lane >> 4, l16 = lane & 15;
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
@@ -446,7 +438,7 @@ DEVINL void role_tiles(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
 #pragma unroll 1
     for (int c = 0; c < nit - 1; ++c) {    // iteration c + 1
         opaque(b_nat); opaque(b_tw); opaque(b_l); opaque(b_sr);
-        if (!LOCAL && w == 3 && c >= 2 && c - 2 < n && !(c & 1)) {
+        if (w == 3 && c >= 2 && c - 2 < n && !(c & 1)) {
             char* dst = sv + static_cast<size_t>((c - 2) >> 1) * SAVED_STATE_B;
 #pragma unroll
             for (int wq = 0; wq < 4; ++wq) {
@@ -469,7 +461,7 @@ DEVINL void role_tiles(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
                 *reinterpret_cast<u32x4*>(dst + SAVED_LO_B + wq * 1024) = lo;
             }
         }
-        if (!LOCAL && c < n && w < 3) {
+        if (c < n && w < 3) {
             const lds_t so = uniform_base(sb + SLOT0 + (c % 3) * SLOT_B), to = uniform_base(sb + TILE0 + (c & 1) * TILE_B);
             // (in accumulator order, two 8-byte pieces: any order of the channels serves a contraction over them, and these
             //  reads run at the LDS's rate where 16-byte reads of rows take 1.6 x as long)
@@ -511,7 +503,7 @@ DEVINL void role_tiles(SmemQ& S, const ArgsQ& a, const int lane, const int w, co
     }
 }
 
-template <bool LOCAL, bool HD>
+template <bool HD>
 __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
     __shared__ SmemQ S;
     const int tid = threadIdx.x;
@@ -538,7 +530,7 @@ __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
     const int nseg = ((arg.T + L - 1) / L + 1) / 2;                 // saved states of a whole sequence
     a.saved = arg.saved + (bh * nseg + t0 / (2 * L)) * SAVED_STATE_B;
     if (arg.s32 != nullptr) a.s32 = arg.s32 + bq * (N * N);
-    if (arg.blk_state != nullptr) { a.blk_state = arg.blk_state + bq * (N * N); a.blk_decay = arg.blk_decay + bq * N; }
+    if (arg.local != nullptr) { a.local = arg.local + bh * arg.NB * (N * N); a.logdec = arg.logdec + bh * arg.NB * N; a.blk = blk; }
     a.first_row = b == 0 && blk == 0;
     const int n = (a.T + L - 1) / L;
     // the quadrant t < 16 <= s of the tiles is never written and must read as zero
@@ -546,14 +538,14 @@ __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
     if (tid == 0) S.met[0] = 0;
     __syncthreads();
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, w = wid & 3;
-    const int nit = (n + (LOCAL ? 1 : 2) + DEPTH) & ~(DEPTH - 1);        // iterations of the pipeline: n + 3 (no y to store: n + 2), in whole trips of the prep loop
-    if (wid < 8) role_prep<LOCAL, HD>(S, a, lane, wid, base, h, bh, n, nit);
-    else if (wid < 12) role_state<LOCAL>(S, a, lane, w, bh, n, nit);
-    else role_tiles<LOCAL>(S, a, lane, w, bh, n, nit);
+    const int nit = (n + 2 + DEPTH) & ~(DEPTH - 1);                     // iterations of the pipeline: n + 3, in whole trips of the prep loop
+    if (wid < 8) role_prep<HD>(S, a, lane, wid, base, h, bh, n, nit);
+    else if (wid < 12) role_state(S, a, lane, w, bh, n, nit);
+    else role_tiles(S, a, lane, w, bh, n, nit);
 }
 
-// States entering the blocks from the local results, four key channels of one value channel per thread, a quarter of a (batch,
-// head) per workgroup of 256.  Forward (reverse = 0): S = s0; out[blk] = S; S <- S 2^logdec[blk] + local[blk].
+// More than SCAN_BLOCKS blocks: the states entering them from the local results, four key channels of one value channel per thread, a quarter of
+// a (batch, head) per workgroup of 256.  Forward (reverse = 0): S = s0; out[blk] = S; S <- S 2^logdec[blk] + local[blk].
 // Reverse: the same from the last block down, from zero: what enters a block from above.
 // It is there for few (batch, head) pairs, so what bounds it is latency: 16 bytes a lane, side by side, and the reads of SCAN_AHEAD
 // blocks, of which none depends on another, in flight together.  B1 H32, 8 blocks: 5.1 us (launch, one round of reads, the stores); with sixteen channels a thread (a quarter
@@ -600,17 +592,18 @@ int launch_wkv6_fwd_fused(hipStream_t st, int B, int T, int C, int H, const uint
     a.T = T; a.C = C; a.H = H; a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.s0 = s0; a.y = y; a.saved = saved; a.flags = flags;
     a.NB = 1; a.TB = T;
     if (NB <= 1) {
-        if (head_decay) hipLaunchKernelGGL((wkv6_fwd_fused<false, true>), dim3(B * H), dim3(NTQ), 0, st, a);
-        else hipLaunchKernelGGL((wkv6_fwd_fused<false, false>), dim3(B * H), dim3(NTQ), 0, st, a);
+        if (head_decay) hipLaunchKernelGGL((wkv6_fwd_fused<true>), dim3(B * H), dim3(NTQ), 0, st, a);
+        else hipLaunchKernelGGL((wkv6_fwd_fused<false>), dim3(B * H), dim3(NTQ), 0, st, a);
         return launch_status();
     }
-    a.NB = NB; a.TB = TB; a.blk_state = blk_state; a.blk_decay = blk_decay;
-    if (head_decay) hipLaunchKernelGGL((wkv6_fwd_fused<true, true>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
-    else hipLaunchKernelGGL((wkv6_fwd_fused<true, false>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
-    hipLaunchKernelGGL(wkv6_scan, dim3(B * H * SCAN_WG), dim3(256), 0, st, blk_state, blk_decay, s0, s32, NB, 0);
-    a.blk_state = nullptr; a.blk_decay = nullptr; a.s32 = s32;
-    if (head_decay) hipLaunchKernelGGL((wkv6_fwd_fused<false, true>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
-    else hipLaunchKernelGGL((wkv6_fwd_fused<false, false>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
+    a.NB = NB; a.TB = TB;
+    if (int e = launch_wkv6_local(st, false, head_decay, B, T, C, H, NB, TB, k, v, w, blk_state, blk_decay, flags)) return e;
+    if (NB > SCAN_BLOCKS) {
+        hipLaunchKernelGGL(wkv6_scan, dim3(B * H * SCAN_WG), dim3(256), 0, st, blk_state, blk_decay, s0, s32, NB, 0);
+        a.s32 = s32;
+    } else { a.local = blk_state; a.logdec = blk_decay; }
+    if (head_decay) hipLaunchKernelGGL((wkv6_fwd_fused<true>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
+    else hipLaunchKernelGGL((wkv6_fwd_fused<false>), dim3(B * H * NB), dim3(NTQ), 0, st, a);
     return launch_status();
 }
 

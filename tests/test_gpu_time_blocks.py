@@ -15,7 +15,7 @@ from oracle import err_ratio, max_rel_to_peak
 from oracle import wkv5a as A
 from oracle import wkv56 as O
 from rwkv_cuda_amd import rwkv7_fast_fused as R
-from rwkv_cuda_amd import synth, wkv5, wkv5_bf16, wkv5a
+from rwkv_cuda_amd import synth, wkv5, wkv5_bf16, wkv5a, wkv6_state
 from rwkv_cuda_amd._call import call
 from _gpu_util import DEV, assert_no_worse, garbage
 
@@ -185,3 +185,21 @@ def test_wkv5_bf16_heads_of_128(lib, decays, B, H, T):
         assert torch.equal(wkv5_bf16.RUN_CUDA(B, T, C, H, *t), y)
     for name, a, e, g in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, [y] + [x.grad for x in t]):
         assert_no_worse(name, a, e.reshape(a.shape), g.reshape(a.shape))
+
+
+@pytest.mark.parametrize("H,T", [(3, 257), (3, 1100), (3, 2300), (64, 1025), (100, 641), (100, 1300)])       # 2, 9, 18 (a scan of its own), 4, 2, 2 blocks of 128 .. 704 tokens
+def test_wkv6_state_blocks_of_every_length(lib, H, T):
+    """The first pass takes a block's tokens up to 256 at a time, 32 or more a part; three heads of the layer against the oracle."""
+    B, C, heads = 1, H * 64, [0, H // 2, H - 1]
+    r, k, v, w, u, gy, s0 = synth.wkv6_inputs(B, T, C, H, seed=T + H, state=True)
+    t = [x.to(DEV).requires_grad_(True) for x in (r, k, v, w, u, s0)]
+    y = wkv6_state.RUN_CUDA(B, T, C, H, *t)
+    got = [y] + list(torch.autograd.grad(y, t, gy.to(DEV)))
+    some = lambda x: x.reshape(B, T, H, 64)[:, :, heads].reshape(B, T, 3 * 64).contiguous() if x.dim() == 3 and x.shape[1] == T else x.reshape(-1, H, *x.shape[-2:])[:, heads] if x.dim() == 4 else x.reshape(H, 64)[heads]
+    a = [some(x) for x in (r, k, v, w, u)]
+    s1 = some(s0)
+    ref = O.wkv6_grads(B, T, 192, 3, *a, some(gy), s0=s1)
+    emu = O.emulate_wkv6_bf16(B, T, 192, 3, *a, some(gy), s0=s1)
+    print(f"\nwkv6_state H={H} T={T}", flush=True)
+    for name, e, m, g in zip(["y", "gr", "gk", "gv", "gw", "gu", "gs"], ref, emu, got):
+        assert_no_worse(name, e, m.reshape(e.shape), some(g.detach()).cpu().reshape(e.shape))
