@@ -76,6 +76,12 @@ struct Args7c {
     int* flags;
 };
 
+// Whole sequences (CUT = false) have an instance of their kernels of their own: with the choice left to run time what belongs to the
+// blocks costs them scalar work and the backward 4 registers (B8 4 x T1024 C4096 3.87 -> 3.83 ms).
+template <bool CUT> DEVINL Args7c only_whole(Args7c p) {
+    if constexpr (!CUT) p.NB = 1;
+    return p;
+}
 // The chunks of the workgroup's block; false: another workgroup does them.
 struct Part7 { int n, first, chunks; };
 DEVINL bool part_of(const Args7c& p, size_t bh, Part7& x) {
@@ -398,8 +404,9 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
 // (96 a wave and chunk) held the vector unit for half of the time.  The first of these forms and this one in alternation on one
 // machine: bf16 382 -> 326 us, fp32 mode 405 -> 379.  Vector instructions now issue 68 % of a SIMD's time, matrix ones about a third.
 // Errors against 64 bits, T16 to T1024, slow to strong decays, largest, before -> now: y 2.4 -> 1.7e-7, sT 1.6 -> 1.0e-7, sa 2.3 -> 1.7e-7.
-template <bool F32, bool KEEP>
-__global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c p) {
+template <bool F32, bool KEEP, bool CUT>
+__global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c args) {
+    const Args7c p = only_whole<CUT>(args);
     extern __shared__ __align__(32) unsigned char smem_raw[];
     SmemCF& S = *reinterpret_cast<SmemCF*>(smem_raw);
     const lds_t sb = lds_of(smem_raw);
@@ -1144,8 +1151,9 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     __syncthreads();
 }
 
-template <bool F32>
-__global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c p) {
+template <bool F32, bool CUT>
+__global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c args) {
+    const Args7c p = only_whole<CUT>(args);
     extern __shared__ __align__(32) unsigned char smem_raw[];
     SmemCB<F32>& S = *reinterpret_cast<SmemCB<F32>*>(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1198,21 +1206,22 @@ template <bool F32, bool REV> int cut(hipStream_t st, int B, Args7c& p, void* ws
     return launch_status();
 }
 
+hipError_t raise_lds(void (*kernel)(Args7c), size_t bytes) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+}
 template <bool F32, bool KEEP> int start_fwd(hipStream_t st, int B, Args7c& p, void* ws) {
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_fwd<F32, KEEP>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       static_cast<int>(F_TOTAL<F32>));
-    if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
+    static const hipError_t attr[2] = {raise_lds(rwkv7c_fwd<F32, KEEP, false>, F_TOTAL<F32>), raise_lds(rwkv7c_fwd<F32, KEEP, true>, F_TOTAL<F32>)};
+    for (const hipError_t e : attr) if (e != hipSuccess) { g_last_hip_error = static_cast<int>(e); return RWKV_ERR_LAUNCH; }
     if (int e = cut<F32, false>(st, B, p, ws)) return e;
-    rwkv7c_fwd<F32, KEEP><<<dim3(p.H, B, p.NB), dim3(NTF), F_TOTAL<F32>, st>>>(p);
+    hipLaunchKernelGGL((p.NB > 1 ? rwkv7c_fwd<F32, KEEP, true> : rwkv7c_fwd<F32, KEEP, false>), dim3(p.H, B, p.NB), dim3(NTF), F_TOTAL<F32>, st, p);
     return launch_status();
 }
 template <bool F32> int start_bwd(hipStream_t st, int B, Args7c& p, void* ws) {
     static_assert(LB<F32>::BYTES <= 160 * 1024, "the backward's LDS must fit one CU");
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_bwd<F32>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                       static_cast<int>(LB<F32>::BYTES));
-    if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
+    static const hipError_t attr[2] = {raise_lds(rwkv7c_bwd<F32, false>, LB<F32>::BYTES), raise_lds(rwkv7c_bwd<F32, true>, LB<F32>::BYTES)};
+    for (const hipError_t e : attr) if (e != hipSuccess) { g_last_hip_error = static_cast<int>(e); return RWKV_ERR_LAUNCH; }
     if (int e = cut<F32, true>(st, B, p, ws)) return e;
-    hipLaunchKernelGGL(rwkv7c_bwd<F32>, dim3(p.H, B, p.NB), dim3(NTB), LB<F32>::BYTES, st, p);
+    hipLaunchKernelGGL((p.NB > 1 ? rwkv7c_bwd<F32, true> : rwkv7c_bwd<F32, false>), dim3(p.H, B, p.NB), dim3(NTB), LB<F32>::BYTES, st, p);
     return launch_status();
 }
 
