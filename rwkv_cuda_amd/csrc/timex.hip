@@ -9,6 +9,8 @@
 // of 32 steps and full batches, timex_conv_any / timex_gw_any (three bf16 terms) for every other length and batch size.
 // timex_gw (vector units) makes the per-batch gw of the reference's signature: one workgroup per (b,c) row; a thread owns 4
 // consecutive lags d.
+#include <algorithm>
+
 #include "common.h"
 
 namespace rwkv {
@@ -579,12 +581,12 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // with fp32's exponents.  The five small products have accumulators of their own: the sum of the large ones, whose roundings are
 // what is left of an error, rounds once an instruction.  Nothing is scaled, so an element's accuracy does not depend on its
 // neighbours: short rows, rows that grow late and batches of unequal rows come out as from an fp32 loop, which two fp16 terms
-// under a common power of two (half the products, 58 and 101 us where these take 95 and 111) do not give.  A unit with an element that is no number, infinite or beyond
+// under a common power of two (half the products, 58 and 101 us where these took 95 and 111) do not give.  A unit with an element that is no number, infinite or beyond
 // bf16's largest is done by such a loop (a matrix product would carry it to earlier steps: zero times infinity).
 // Rows lie in LDS as blocks of 32 + 8 terms (80 bytes: 16-byte reads of neighbouring columns fall on different banks if a
 // row has an odd number of blocks), 512 threads, 128 registers, and up to T = 2900 (gradient) and 3360 at most 80 KB: two
 // workgroups share a CU, one converts its rows while the other multiplies; longer rows take a CU each.  B13 C384 T1500:
-// 95 us a convolution, 111 us the kernel gradient, relative errors 1.8e-7 and 1.0e-7; the fp32 loops on the vector units that
+// 77 us a convolution (92 with a wave per column tile, units of 4, 4, 4 and 1 rows), 111 us the kernel gradient, relative errors 1.8e-7 and 1.0e-7; the fp32 loops on the vector units that
 // these replace took 315 / 286 and, with the sum over the batch, 243 us, with 5.6e-7.
 constexpr int BLK = 40;                // elements of a block in LDS, 32 of them data
 constexpr int LDS_ANY = 80 * 1024;     // two workgroups per CU
@@ -607,6 +609,27 @@ inline AnyGeom any_geom(int T, int bg, int span) {        // span: how many bloc
     q.pitch = q.nt + q.zb;
     return q;
 }
+// What the eight waves of a workgroup of timex_conv_any do.  A pair of column tiles, neighbours in the order of decreasing work, needs
+// its longer tile's block lags once for both (they share the Toeplitz operand); its lags are cut into runs of about equal work, a
+// wave each, as many as it takes for the eight waves to be done at about the same time.  Wave w: lags d0 .. d1 - 1 of pair `pair`
+// (NO_PAIR: nothing to do).  The pair's lowest wave adds the others' sums to its own and stores the tiles.
+// (A tile of 1500 steps has up to 47 lags and there are six tiles of four rows: one wave a tile, or two short tiles, left two waves without
+// work and the others waiting for the one with 47: B13 C384 T1500 92 us a convolution, 77 so.)
+constexpr int NO_PAIR = 255;
+struct ConvPlan {
+    AnyGeom q;
+    uint8_t pair[TXW];
+    uint8_t d0[TXW], d1[TXW];
+};
+static_assert(T_ANY / 32 < 255, "a block lag is a byte");
+struct ConvPlans { ConvPlan p[2]; };   // for units of ceil(B / groups) and of floor(B / groups) rows
+__host__ __device__ inline int tile_lags(const AnyGeom& q, bool mirror, int tile) {
+    const int ncol = q.nt * q.bg, last = 32 * tile + 31 < ncol ? 32 * tile + 31 : ncol - 1;
+    return mirror ? q.nt - 32 * tile / q.bg : last / q.bg + 1;
+}
+// tile number `rank` in the order of decreasing work; none: -1
+__host__ __device__ inline int tile_of(int ntile, bool mirror, int rank) { return rank < ntile ? (mirror ? rank : ntile - 1 - rank) : -1; }
+constexpr size_t SUM_SLOT = 2 * 32 * 32;      // floats of a wave's two tiles
 inline size_t conv_any_lds(const AnyGeom& q) { return (NPL * q.plane() + 2 * NPL * static_cast<size_t>(h2_line_len(32 * q.nt))) * 2 + 16; }
 inline size_t gw_any_lds(const AnyGeom& q) { return 2 * NPL * q.plane() * 2 + static_cast<size_t>(q.nt) * 256 + 16; }
 
@@ -688,14 +711,16 @@ DEVINL void zero_blocks(uint16_t* rp, const AnyGeom& q) {
 
 template <bool MIRROR>
 __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict__ w, const float* __restrict__ in, float* __restrict__ out,
-                                                         float eps, int B, int C, int T, int ng, const AnyGeom q) {
+                                                         float eps, int B, int C, int T, int ng, const ConvPlans plans) {
     extern __shared__ __align__(16) float lds[];
+    const int c = blockIdx.x / ng, grp = blockIdx.x - c * ng, fewer = B / ng, b0 = grp * fewer + min(grp, B % ng);
+    const ConvPlan& plan = plans.p[grp < B % ng || B % ng == 0 ? 0 : 1];
+    const AnyGeom& q = plan.q;
     const int Tp = 32 * q.nt, xl = h2_line_len(Tp), plane = static_cast<int>(q.plane());
     uint16_t* rp = reinterpret_cast<uint16_t*>(lds);                    // [NPL][plane]
     uint16_t* al = rp + NPL * plane;                                    // [NPL planes][2 copies][xl]
     int* red = reinterpret_cast<int*>(al + 2 * NPL * xl);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, kh = lane >> 5;
-    const int c = blockIdx.x / ng, b0 = (blockIdx.x - c * ng) * q.bg;
     {
         Stager<CONV_PIECES> st;
         st.fetch(in, q, c, b0, B, C, T);
@@ -714,7 +739,6 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
         if (any_thread(beyond, red)) {
             for (int i = tid; i < q.bg * T; i += TXT) {
                 const int b = i / T, t = i - b * T;
-                if (b0 + b >= B) break;
                 const size_t row = (static_cast<size_t>(b0 + b) * C + c) * T;
                 const float *x = in + row, *wl = w + static_cast<size_t>(c) * T + T - 1;       // wl[-lag]
                 float acc = 0.f;
@@ -738,16 +762,14 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
         }
         __syncthreads();
     }
-    // Column tiles in the order of decreasing work go to the waves back and forth: ranks wv and 15 - wv, at most two a wave, the
-    // shorter one along with the longer one (they share the Toeplitz operand) as far as it goes.
+    const int pair = plan.pair[wv], d0 = plan.d0[wv], d1 = plan.d1[wv];
     const int ncol = q.nt * q.bg, ntile = (ncol + 31) >> 5;
     int tile[2], nd[2];
     const uint16_t* bp[2];
 #pragma unroll
     for (int z = 0; z < 2; ++z) {
-        const int rank = z == 0 ? wv : 2 * TXW - 1 - wv;
-        tile[z] = MIRROR ? rank : ntile - 1 - rank;
-        nd[z] = rank < ntile ? (MIRROR ? q.nt - 32 * tile[z] / q.bg : min(32 * tile[z] + 31, ncol - 1) / q.bg + 1) : 0;
+        tile[z] = pair == NO_PAIR ? -1 : tile_of(ntile, MIRROR, 2 * pair + z);
+        nd[z] = tile[z] < 0 ? 0 : tile_lags(q, MIRROR, tile[z]);
         const int col = min(32 * max(tile[z], 0) + ln, ncol - 1), a = col / q.bg, b = col - a * q.bg;
         bp[z] = rp + (q.zb + b * q.pitch + a) * BLK + 8 * kh;
     }
@@ -758,9 +780,9 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
     for (int z = 0; z < 2; ++z)
 #pragma unroll
         for (int v = 0; v < 16; ++v) { acc[z][v] = 0.f; low[z][v] = 0.f; }
-    auto run = [&](auto NTL, const int d0, const int d1) __attribute__((always_inline)) {
+    auto run = [&](auto NTL, const int from, const int to) __attribute__((always_inline)) {
         constexpr int NT_ = decltype(NTL)::value;
-        for (int d = d0; d < d1; ++d) {
+        for (int d = from; d < to; ++d) {
             const int o = MIRROR ? d : -d;
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
@@ -785,12 +807,38 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
             }
         }
     };
-    run(std::integral_constant<int, 2>{}, 0, nd[1]);
-    run(std::integral_constant<int, 1>{}, nd[1], nd[0]);
+    run(std::integral_constant<int, 2>{}, d0, min(d1, nd[1]));
+    run(std::integral_constant<int, 1>{}, max(d0, nd[1]), d1);
+    // the sums of a pair's other waves, through the LDS that the rows no longer need
+    bool owner = pair != NO_PAIR;
+    for (int x = 0; x < wv; ++x) owner &= plan.pair[x] != pair;
+    float4* const slot = reinterpret_cast<float4*>(lds);
+    constexpr int SLOT4 = SUM_SLOT / 4;
+    __syncthreads();
+    if (pair != NO_PAIR && !owner) {
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+#pragma unroll
+            for (int v4 = 0; v4 < 4; ++v4)
+                slot[wv * SLOT4 + (4 * z + v4) * 64 + lane] = make_float4(acc[z][4 * v4] + low[z][4 * v4], acc[z][4 * v4 + 1] + low[z][4 * v4 + 1],
+                                                                         acc[z][4 * v4 + 2] + low[z][4 * v4 + 2], acc[z][4 * v4 + 3] + low[z][4 * v4 + 3]);
+    }
+    __syncthreads();
+    if (!owner) return;
+    for (int x = wv + 1; x < TXW; ++x) {
+        if (plan.pair[x] != pair) continue;
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+#pragma unroll
+            for (int v4 = 0; v4 < 4; ++v4) {
+                const float4 y = slot[x * SLOT4 + (4 * z + v4) * 64 + lane];
+                acc[z][4 * v4] += y.x; acc[z][4 * v4 + 1] += y.y; acc[z][4 * v4 + 2] += y.z; acc[z][4 * v4 + 3] += y.w;
+            }
+    }
 #pragma unroll
     for (int z = 0; z < 2; ++z) {
         const int col = 32 * tile[z] + ln, a = col / q.bg, b = col - a * q.bg;
-        if (nd[z] > 0 && col < ncol && b0 + b < B) {
+        if (tile[z] >= 0 && col < ncol) {
             float* o = out + (static_cast<size_t>(b0 + b) * C + c) * T;
 #pragma unroll
             for (int v4 = 0; v4 < 4; ++v4) {
@@ -938,22 +986,69 @@ __global__ __launch_bounds__(256) void timex_add_parts(const float4* __restrict_
     out[i] = a;
 }
 
-// Batch rows of a unit.  Convolution: what finishes first by a count of matrix clocks (96 per column tile and block lag on a
-// CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (two a wave) and 80 KB
-// (a single row may have more).
-AnyGeom conv_any_geom(int B, int C, int T) {
-    AnyGeom best{};
-    double cost = 1e300;
-    for (int bg = 1; bg <= B && bg <= 32; ++bg) {
-        const AnyGeom q = any_geom(T, bg, 31);
-        const int ncol = q.nt * bg, ntile = (ncol + 31) / 32;
-        if (ntile > 2 * TXW || conv_any_lds(q) > LDS_ANY || 8 * ncol > CONV_PIECES * TXT) { if (bg > 1) break; }
-        long long pairs = 0;
-        for (int t = 0; t < ntile; ++t) pairs += (32 * t + 31 < ncol ? 32 * t + 31 : ncol - 1) / bg + 1;
-        const long long units = static_cast<long long>(C) * ((B + bg - 1) / bg);
-        const double x = static_cast<double>((units + 2 * NCU - 1) / (2 * NCU)) * (96.0 * pairs + 0.15 * bg * T + 3000.0);
-        if (x < cost) { cost = x; best = q; }
+// The waves' shares: runs of a pair's lags are added where the longest run is, until there are eight, then the longest four runs go to the
+// four SIMDs (a wave w runs on SIMD w mod 4) and the others to the least loaded ones.
+void plan_waves(ConvPlan& p, bool mirror) {
+    const int ntile = (p.q.nt * p.q.bg + 31) / 32, npair = (ntile + 1) / 2;
+    int lags[TXW][2] = {}, runs[TXW] = {}, work[TXW] = {};
+    for (int m = 0; m < npair; ++m) {
+        for (int z = 0; z < 2; ++z) {
+            const int t = tile_of(ntile, mirror, 2 * m + z);
+            lags[m][z] = t < 0 ? 0 : tile_lags(p.q, mirror, t);
+        }
+        work[m] = lags[m][0] + lags[m][1];
+        runs[m] = 1;
     }
+    for (int n = npair; n < TXW; ++n) {
+        int most = -1;
+        for (int m = 0; m < npair; ++m)
+            if (runs[m] < lags[m][0] && (most < 0 || work[m] * runs[most] > work[most] * runs[m])) most = m;
+        if (most < 0) break;
+        ++runs[most];
+    }
+    struct Run { int pair, d0, d1, work; } run[TXW];
+    int n = 0;
+    for (int m = 0; m < npair; ++m) {
+        const auto lag_at = [&](int x) { return x < 2 * lags[m][1] ? (x + 1) / 2 : x - lags[m][1]; };      // after x steps of the pair
+        for (int k = 0; k < runs[m]; ++k) {
+            const int d0 = lag_at(work[m] * k / runs[m]), d1 = k + 1 == runs[m] ? lags[m][0] : lag_at(work[m] * (k + 1) / runs[m]);
+            if (d1 > d0) run[n++] = {m, d0, d1, (d1 - d0) + (d0 < lags[m][1] ? (d1 < lags[m][1] ? d1 : lags[m][1]) - d0 : 0)};
+        }
+    }
+    std::sort(run, run + n, [](const Run& a, const Run& b) { return a.work > b.work; });
+    for (int w = 0; w < TXW; ++w) p.pair[w] = NO_PAIR, p.d0[w] = p.d1[w] = 0;
+    for (int i = 0; i < n; ++i) {
+        const int w = i < 4 ? i : 11 - i;
+        p.pair[w] = static_cast<uint8_t>(run[i].pair);
+        p.d0[w] = static_cast<uint8_t>(run[i].d0); p.d1[w] = static_cast<uint8_t>(run[i].d1);
+    }
+}
+size_t conv_plan_lds(const ConvPlans& x) { return std::max({conv_any_lds(x.p[0].q), conv_any_lds(x.p[1].q), TXW * SUM_SLOT * sizeof(float)}); }
+// Batch rows of a unit, dealt evenly to `ng` units a channel.  What finishes first by a count of matrix clocks (96 per column tile and
+// block lag on a CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (a pair a wave) and
+// 80 KB (a single row may have more).
+ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
+    ConvPlans best{};
+    double cost = 1e300;
+    for (int most = 1; most <= B && most <= 32; ++most) {
+        const int groups = (B + most - 1) / most, rows[2] = {(B + groups - 1) / groups, B / groups};
+        if (rows[0] != most) continue;
+        ConvPlans x{};
+        double unit = 0;
+        for (int z = 0; z < 2; ++z) {
+            x.p[z].q = any_geom(T, rows[z], 31);
+            const int ntile = (x.p[z].q.nt * rows[z] + 31) / 32;
+            if (ntile > 2 * TXW) { unit = -1; break; }
+            const int share = z == 1 ? groups - B % groups : B % groups;
+            long long steps = 0;
+            for (int t = 0; t < ntile; ++t) steps += tile_lags(x.p[z].q, mirror, t);
+            unit += (96.0 * steps + 0.15 * rows[z] * T + 3000.0) * share / groups;
+        }
+        if (unit < 0 || conv_plan_lds(x) > LDS_ANY || 8 * x.p[0].q.nt * rows[0] > CONV_PIECES * TXT) { if (most > 1) break; }
+        const double c = static_cast<double>((static_cast<long long>(C) * groups + 2 * NCU - 1) / (2 * NCU)) * unit;
+        if (c < cost) { cost = c; best = x; *ng = groups; }
+    }
+    for (ConvPlan& p : best.p) plan_waves(p, mirror);
     return best;
 }
 AnyGeom gw_any_geom(int B, int T) {
@@ -1010,12 +1105,12 @@ template <bool MIRROR> int launch_conv(void* stream, const float* w, const float
         if (int e = raise_lds_limit(kernel, lds)) return e;
         hipLaunchKernelGGL(kernel, dim3(conv_grid(B, C)), dim3(TXT), lds, st, w, in, out, eps, B, C, T);
     } else {
-        const AnyGeom q = conv_any_geom(B, C, T);
-        const size_t lds = conv_any_lds(q);
-        const int ng = (B + q.bg - 1) / q.bg;
+        int ng;
+        const ConvPlans plans = conv_any_plans(B, C, T, MIRROR, &ng);
+        const size_t lds = conv_plan_lds(plans);
         if (static_cast<long long>(C) * ng > 0x7fffffffLL) return RWKV_ERR_SHAPE;
         if (int e = raise_lds_limit(timex_conv_any<MIRROR>, lds)) return e;
-        hipLaunchKernelGGL(timex_conv_any<MIRROR>, dim3(C * ng), dim3(TXT), lds, st, w, in, out, eps, B, C, T, ng, q);
+        hipLaunchKernelGGL(timex_conv_any<MIRROR>, dim3(C * ng), dim3(TXT), lds, st, w, in, out, eps, B, C, T, ng, plans);
     }
     return RWKV_OK;
 }

@@ -35,7 +35,8 @@ def test_shapes(lib, B, T):
     _check(B, 3, T, *synth.timex_inputs(B, 3, T, seed=B + T))
 
 
-@pytest.mark.parametrize("B,C,T", [(7, 5, 96), (16, 2, 772), (31, 2, 68), (32, 3, 100), (33, 2, 36), (64, 1, 1500), (70, 2, 4), (3, 600, 52)])
+@pytest.mark.parametrize("B,C,T", [(7, 5, 96), (16, 2, 772), (31, 2, 68), (32, 3, 100), (33, 2, 36), (64, 1, 1500), (70, 2, 4), (3, 600, 52),
+                                   (13, 40, 500), (33, 40, 500), (13, 200, 100), (7, 40, 1500)])   # the last four: units of unequal numbers of rows
 def test_more_batches(lib, B, C, T):
     print(f"\ntimex any B={B} C={C} T={T}", flush=True)
     _check(B, C, T, *synth.timex_inputs(B, C, T, seed=B + C + T))
