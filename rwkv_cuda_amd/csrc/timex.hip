@@ -6,7 +6,7 @@
 //   gw[b,c,T-1-d] =   sum_{u}    g[b,c,u+d] k[b,c,u]         (per batch; the wrapper sums over b)
 //
 // Two families on the matrix cores at fp32 accuracy: timex_conv_h2 / timex_gw_sum_h2 (two fp16 terms per operand) for whole tiles
-// of 32 steps and full batches, timex_conv_any / timex_gw_any (three bf16 terms) for every other length and batch size.
+// of 32 steps and full batches, timex_conv_any / timex_gw_any, timex_gw_short (three bf16 terms) for every other length and batch size.
 // timex_gw (vector units) makes the per-batch gw of the reference's signature: one workgroup per (b,c) row; a thread owns 4
 // consecutive lags d.
 #include <algorithm>
@@ -572,10 +572,12 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // b), numbered a Bg + b in a unit of Bg batch rows of one channel, and 32 consecutive columns are a tile of one matrix
 // instruction.  Two rows of 1500 steps fill three column tiles, where a tile of 32 batch rows would be empty but for two.
 // A tile's columns differ in a by at most 31 / Bg: d runs to the largest a, and blocks before a row's start (mirror: after its
-// end) read as zeros, of which every row has zb behind it.  The kernel gradient is the same contraction turned round:
-//     gw[lag 32 d + i - j] = sum over the diagonals of M_d[i][j] = sum_columns g[32 a + i] k[32 (a - d) + j],
-// K slots are columns, sixteen an instruction, g and k operands by transposing LDS reads whose lanes point at blocks of their
-// own.
+// end) read as zeros, of which every row has zb behind it.  The kernel gradient takes 256 lags a tile, d = i' + 8 j + 128 h with (i', h) the
+// rows and j the columns of one 16 x 16 instruction, and time as its contraction:
+//     M[(i', h)][j] = sum_t g[t + i' + 128 h] k[t - 8 j],
+// a Hankel operand (the windows of g) and one whose columns begin 8 steps apart, so that every element is a tap: nothing is summed over
+// diagonals, and the sums of all rows that a workgroup does stay in registers.  (Lag tiles of 32, columns (block, row) as above, whose
+// sub-diagonals are summed after every few instructions, are timex_gw_short.)
 // Operands are THREE bf16 terms, x = h + m + l (each the nearest of what is left: all 24 bits of x), and a product is
 //     x y = h h' + h m' + m h' + m m' + h l' + l h'            (the terms left out are below 2^-24 of the product, 2^-26 rms)
 // with fp32's exponents.  The five small products have accumulators of their own: the sum of the large ones, whose roundings are
@@ -584,21 +586,31 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // under a common power of two (half the products, 58 and 101 us where these took 95 and 111) do not give.  A unit with an element that is no number, infinite or beyond
 // bf16's largest is done by such a loop (a matrix product would carry it to earlier steps: zero times infinity).
 // Rows lie in LDS as blocks of 32 + 8 terms (80 bytes: 16-byte reads of neighbouring columns fall on different banks if a
-// row has an odd number of blocks), 512 threads, 128 registers, and up to T = 2900 (gradient) and 3360 at most 80 KB: two
+// row has an odd number of blocks), 512 threads, 128 registers, and up to T = 3360 (gradient: always) at most 80 KB: two
 // workgroups share a CU, one converts its rows while the other multiplies; longer rows take a CU each.  B13 C384 T1500:
-// 77 us a convolution (92 with a wave per column tile, units of 4, 4, 4 and 1 rows), 111 us the kernel gradient, relative errors 1.8e-7 and 1.0e-7; the fp32 loops on the vector units that
-// these replace took 315 / 286 and, with the sum over the batch, 243 us, with 5.6e-7.
+// 77 us a convolution (92 with a wave per column tile and units of 4, 4, 4 and 1 rows; matrix pipes busy 70 % of the time that a CU has
+// work), 77 us the kernel gradient (107 as lag tiles of 32), relative errors 1.8e-7 and 1.0e-7; the fp32 loops on the vector units
+// that these replace took 315 / 286 and, with the sum over the batch, 243 us, with 5.6e-7.
 constexpr int BLK = 40;                // elements of a block in LDS, 32 of them data
 constexpr int LDS_ANY = 80 * 1024;     // two workgroups per CU
 constexpr int PZ = 32;                 // zeros in front of the forward line (lags beyond the last tap, of rows past T)
-constexpr int CONV_PIECES = 8, GW_PIECES = 4;   // 16-byte pieces a thread stages (per tensor): Bg nt 8 / 512 at most
+constexpr int CONV_PIECES = 8, GW_PIECES = 3;   // 16-byte pieces a thread stages (per tensor): Bg nt 8 / 512 at most
 constexpr int NPL = 3;                 // planes: terms of an operand
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 // the six products of two operands, the small ones first
 constexpr int TERM_A[6] = {2, 0, 1, 1, 0, 0}, TERM_B[6] = {0, 2, 1, 0, 1, 0};
 
+// Division by sizes of a launch, a multiplication and a shift: a real one is 30 vector instructions in kernels whose waves issue some 800.
+// Exact for a column (at most 512) over rows (at most 32) and a zero block's number (at most 32 33) over the zero blocks of a row (at most 32):
+// x (d - 1) < 2^16; and for a piece (at most 512) over the pieces of a row (at most 1024).
+__host__ __device__ inline uint32_t inv16(int d) { return (65536u + d - 1) / d; }
+__host__ __device__ inline uint32_t inv_per(int d) { return ((1u << 20) + d - 1) / d; }
+__host__ __device__ inline int over16(int x, uint32_t inv) { return static_cast<int>(static_cast<uint32_t>(x) * inv >> 16); }
+__host__ __device__ inline int over_per(int x, uint32_t inv) { return static_cast<int>(static_cast<uint32_t>(x) * inv >> 20); }
 struct AnyGeom {
     int nt, bg, zb, pitch;             // blocks of a row, rows of a unit, zero blocks behind a row, nt + zb (odd)
+    uint32_t bg_inv, zb_inv, per_inv;
     __host__ __device__ size_t plane() const { return static_cast<size_t>(zb + bg * pitch) * BLK; }     // elements
 };
 inline AnyGeom any_geom(int T, int bg, int span) {        // span: how many blocks the columns of one operand may differ by
@@ -607,6 +619,7 @@ inline AnyGeom any_geom(int T, int bg, int span) {        // span: how many bloc
     q.zb = (span + bg - 1) / bg;
     q.zb += (q.nt + q.zb + 1) & 1;
     q.pitch = q.nt + q.zb;
+    q.bg_inv = inv16(bg); q.zb_inv = inv16(q.zb); q.per_inv = inv_per(8 * q.nt);
     return q;
 }
 // What the eight waves of a workgroup of timex_conv_any do.  A pair of column tiles, neighbours in the order of decreasing work, needs
@@ -618,20 +631,46 @@ inline AnyGeom any_geom(int T, int bg, int span) {        // span: how many bloc
 constexpr int NO_PAIR = 255;
 struct ConvPlan {
     AnyGeom q;
-    uint8_t pair[TXW];
-    uint8_t d0[TXW], d1[TXW];
+    int shared;                        // whether a pair has more than one wave
+    uint64_t pair, d0, d1;             // a byte a wave: read once, where bytes read one by one are a trip to memory each
+    __host__ __device__ static int of(uint64_t x, int w) { return static_cast<int>(x >> (8 * w) & 255); }
 };
+static_assert(TXW == 8, "a word holds a byte a wave");
 static_assert(T_ANY / 32 < 255, "a block lag is a byte");
 struct ConvPlans { ConvPlan p[2]; };   // for units of ceil(B / groups) and of floor(B / groups) rows
 __host__ __device__ inline int tile_lags(const AnyGeom& q, bool mirror, int tile) {
     const int ncol = q.nt * q.bg, last = 32 * tile + 31 < ncol ? 32 * tile + 31 : ncol - 1;
-    return mirror ? q.nt - 32 * tile / q.bg : last / q.bg + 1;
+    return mirror ? q.nt - over16(32 * tile, q.bg_inv) : over16(last, q.bg_inv) + 1;
 }
 // tile number `rank` in the order of decreasing work; none: -1
 __host__ __device__ inline int tile_of(int ntile, bool mirror, int rank) { return rank < ntile ? (mirror ? rank : ntile - 1 - rank) : -1; }
 constexpr size_t SUM_SLOT = 2 * 32 * 32;      // floats of a wave's two tiles
 inline size_t conv_any_lds(const AnyGeom& q) { return (NPL * q.plane() + 2 * NPL * static_cast<size_t>(h2_line_len(32 * q.nt))) * 2 + 16; }
-inline size_t gw_any_lds(const AnyGeom& q) { return 2 * NPL * q.plane() * 2 + static_cast<size_t>(q.nt) * 256 + 16; }
+
+// The kernel gradient.  In LDS g lies in blocks of 128 steps and the GW_OVER - 128 after them (a window of eight steps is read within one
+// block), a zero block behind, which is also what lies in front of k.  A window that begins at an odd step is the same five dwords as
+// the one before it, shifted in registers (a second copy of g, shifted by one step, is half as many rows in LDS and four more writes a
+// piece and term: B32 C1000 T36 18.9 us, 16.2 so).  A read of half a wave takes eight or nine dwords each from two blocks in a row, which are 8 banks
+// apart (at the same bank such reads took twice as long, and they were as many cycles of LDS as those of k).
+constexpr int GW_OVER = 144;
+constexpr int GW_TILES = 8;            // lag tiles of a wave, 256 lags each
+constexpr int GW_WAVES = 6;            // of more than eight tiles (T > 2048): the waves that take the first eight, which have about three times the work
+struct GwGeom {
+    int nt, bg, k, plane;              // elements from a plane's start to k, to the next plane
+    uint32_t per_inv;
+    __host__ __device__ int bytes() const { return bg * NPL * plane * 2 + 16; }
+};
+inline GwGeom gw_geom(int T, int bg) {
+    GwGeom q;
+    q.nt = (T + 31) / 32; q.bg = bg;
+    q.k = GW_OVER * ((q.nt + 3) / 4 + 1);
+    q.plane = q.k + 32 * q.nt;
+    q.per_inv = inv_per(8 * q.nt);
+    return q;
+}
+inline size_t gw_any_lds(const GwGeom& q, int T) {
+    return std::max(static_cast<size_t>(q.bytes()), TXW * sizeof(float) * 256 * std::min((T + 255) / 256, GW_TILES));
+}
 
 // an element that three bf16 terms do not carry: its nearest bf16 is not finite
 DEVINL bool beyond_terms(float x) { return (__float_as_uint(x) & 0x7fffffffu) >= 0x7f7f8000u; }
@@ -660,20 +699,27 @@ DEVINL int own_thread() {
     asm volatile("" : "+v"(t));
     return t;
 }
-// rows b0 .. of channel c as 16-byte pieces: piece idx = tid + 512 i <-> (row, four steps)
+// Rows as 16-byte pieces, `per` a row: the thread's pieces tid + 512 i of `rows` rows are each(i, row, first step).
+template <int NP, class F> DEVINL void for_pieces(int rows, int per, uint32_t per_inv, const F& each) {
+    const int me = own_thread(), dr = over_per(TXT, per_inv), dt = 4 * (TXT - dr * per);
+    int rr = over_per(me, per_inv), t = 4 * (me - rr * per);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        if (TXT * i >= rows * per) break;
+        each(i, rr, t);
+        rr += dr; t += dt;
+        if (t >= 4 * per) { t -= 4 * per; ++rr; }
+    }
+}
+// rows b0 .. b0 + q.bg - 1 of channel c
 template <int NP> struct Stager {
     float4 x[NP];
     DEVINL void fetch(const float* __restrict__ in, const AnyGeom& q, int c, int b0, int B, int C, int T) {
-        const int per = 8 * q.nt, total = q.bg * per, tid = own_thread();
 #pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            const int idx = tid + TXT * i;
-            if (idx < total) {
-                const int b = idx / per, t = 4 * (idx - b * per);
-                if (b0 + b < B && t < T) x[i] = *reinterpret_cast<const float4*>(in + (static_cast<size_t>(b0 + b) * C + c) * T + t);
-            }
-        }
+        for (int i = 0; i < NP; ++i) x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for_pieces<NP>(q.bg, 8 * q.nt, q.per_inv, [&](int i, int rr, int t) __attribute__((always_inline)) {
+            if (rr < q.bg && b0 + rr < B && t < T) x[i] = *reinterpret_cast<const float4*>(in + (static_cast<size_t>(b0 + rr) * C + c) * T + t);
+        });
     }
     DEVINL bool beyond() const {
         bool on = false;
@@ -682,27 +728,29 @@ template <int NP> struct Stager {
         return on;
     }
     DEVINL void store(uint16_t* rp, const AnyGeom& q) const {
-        const int per = 8 * q.nt, total = q.bg * per, tid = own_thread();
-        const size_t pl = q.plane();
+        const int pl = static_cast<int>(q.plane());
+        for_pieces<NP>(q.bg, 8 * q.nt, q.per_inv, [&](int i, int rr, int t) __attribute__((always_inline)) {
+            if (rr >= q.bg) return;
+            uint16_t* d = rp + (q.zb + rr * q.pitch + (t >> 5)) * BLK + (t & 31);
+            const B3x4 y = split3x4(x[i]);
 #pragma unroll
-        for (int i = 0; i < NP; ++i) {
-            const int idx = tid + TXT * i;
-            if (idx < total) {
-                const int b = idx / per, r = idx - b * per;
-                uint16_t* d = rp + (q.zb + b * q.pitch + (r >> 3)) * BLK + 4 * (r & 7);
-                const B3x4 y = split3x4(x[i]);
-#pragma unroll
-                for (int p = 0; p < NPL; ++p) *reinterpret_cast<uint2*>(d + p * pl) = y.p[p];
-            }
-        }
+            for (int p = 0; p < NPL; ++p) *reinterpret_cast<uint2*>(d + p * pl) = y.p[p];
+        });
     }
 };
+// four elements at place `at` of a line (a multiple of 4) and one place further down in its second copy (nothing before its start)
+DEVINL void put_line4(uint16_t* line, uint16_t* copy, int at, const uint2& y) {
+    *reinterpret_cast<uint2*>(line + at) = y;
+    if (at > 0) copy[at - 1] = static_cast<uint16_t>(y.x);
+    *reinterpret_cast<uint32_t*>(copy + at) = (y.x >> 16) | (y.y << 16);
+    copy[at + 2] = static_cast<uint16_t>(y.y >> 16);
+}
 // the blocks in front of the first row and behind every row
 DEVINL void zero_blocks(uint16_t* rp, const AnyGeom& q) {
     const int n = q.zb * (q.bg + 1) * (BLK / 8);
     const size_t pl = q.plane();
     for (int i = threadIdx.x; i < n; i += TXT) {
-        const int blk = i / (BLK / 8), e = i - blk * (BLK / 8), row = blk / q.zb, z = blk - row * q.zb;      // row 0: the front
+        const int blk = i / (BLK / 8), e = i - blk * (BLK / 8), row = over16(blk, q.zb_inv), z = blk - row * q.zb;      // row 0: the front
         uint16_t* d = rp + (row * q.pitch + z) * BLK + 8 * e;
 #pragma unroll
         for (int p = 0; p < NPL; ++p) *reinterpret_cast<uint4*>(d + p * pl) = make_uint4(0, 0, 0, 0);
@@ -724,17 +772,18 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
     {
         Stager<CONV_PIECES> st;
         st.fetch(in, q, c, b0, B, C, T);
-        float wr[T_ANY / TXT];
-        bool beyond = st.beyond();
+        float4 wr[T_ANY / (4 * TXT)];
 #pragma unroll
-        for (int z = 0; z < T_ANY / TXT; ++z) {
-            const int tau = z * TXT + tid;
-            wr[z] = tau < T ? w[static_cast<size_t>(c) * T + tau] : 0.f;
-            beyond |= beyond_terms(wr[z]);
+        for (int z = 0; z < T_ANY / (4 * TXT); ++z) {
+            const int tau = 4 * (z * TXT + tid);
+            wr[z] = tau < T ? *reinterpret_cast<const float4*>(w + static_cast<size_t>(c) * T + tau) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
-        for (int i = tid; i < NPL * xl; i += TXT) reinterpret_cast<uint32_t*>(al)[i] = 0;
+        for (int i = tid; i < NPL * xl / 4; i += TXT) reinterpret_cast<uint4*>(al)[i] = make_uint4(0, 0, 0, 0);
         zero_blocks(rp, q);
         if (tid == 0) *red = 0;
+        bool beyond = st.beyond();
+#pragma unroll
+        for (int z = 0; z < T_ANY / (4 * TXT); ++z) beyond |= beyond_terms(wr[z]);
         __syncthreads();
         if (any_thread(beyond, red)) {
             for (int i = tid; i < q.bg * T; i += TXT) {
@@ -749,20 +798,31 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
             return;
         }
         st.store(rp, q);
-        // tap tau (lag T-1-tau) sits at line position PZ + tau (forward) or 31 + lag (mirror); the rest is zero
+        // tap tau (lag T-1-tau) sits at line position PZ + tau (forward) or 31 + lag (mirror); the rest is zero.  Four taps a thread: mirrored
+        // they lie the other way round, an odd place up in the line and an even one in its second copy
 #pragma unroll
-        for (int z = 0; z < T_ANY / TXT; ++z) {
-            const int tau = z * TXT + tid;
+        for (int z = 0; z < T_ANY / (4 * TXT); ++z) {
+            const int tau = 4 * (z * TXT + tid);
             if (tau < T) {
-                const B3x4 a = split3x4(make_float4(wr[z], 0.f, 0.f, 0.f));
-                const int pos = MIRROR ? 31 + (T - 1 - tau) : PZ + tau;
+                const B3x4 a = split3x4(MIRROR ? make_float4(wr[z].w, wr[z].z, wr[z].y, wr[z].x) : wr[z]);
 #pragma unroll
-                for (int p = 0; p < NPL; ++p) { al[(2 * p) * xl + pos] = static_cast<uint16_t>(a.p[p].x); al[(2 * p + 1) * xl + pos - 1] = static_cast<uint16_t>(a.p[p].x); }
+                for (int p = 0; p < NPL; ++p) {
+                    uint16_t *line = al + 2 * p * xl, *copy = line + xl;
+                    if constexpr (MIRROR) {
+                        line += 28 + T - 4 - tau; copy += 28 + T - 4 - tau;          // (the lowest of the four at line[3], copy[2])
+                        line[3] = static_cast<uint16_t>(a.p[p].x);
+                        *reinterpret_cast<uint32_t*>(line + 4) = (a.p[p].x >> 16) | (a.p[p].y << 16);
+                        line[6] = static_cast<uint16_t>(a.p[p].y >> 16);
+                        *reinterpret_cast<uint32_t*>(copy + 2) = a.p[p].x;
+                        *reinterpret_cast<uint32_t*>(copy + 4) = a.p[p].y;
+                    } else put_line4(line, copy, PZ + tau, a.p[p]);
+                }
             }
         }
         __syncthreads();
     }
-    const int pair = plan.pair[wv], d0 = plan.d0[wv], d1 = plan.d1[wv];
+    const uint64_t pairs = plan.pair;
+    const int pair = ConvPlan::of(pairs, wv), d0 = ConvPlan::of(plan.d0, wv), d1 = ConvPlan::of(plan.d1, wv);
     const int ncol = q.nt * q.bg, ntile = (ncol + 31) >> 5;
     int tile[2], nd[2];
     const uint16_t* bp[2];
@@ -770,7 +830,7 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
     for (int z = 0; z < 2; ++z) {
         tile[z] = pair == NO_PAIR ? -1 : tile_of(ntile, MIRROR, 2 * pair + z);
         nd[z] = tile[z] < 0 ? 0 : tile_lags(q, MIRROR, tile[z]);
-        const int col = min(32 * max(tile[z], 0) + ln, ncol - 1), a = col / q.bg, b = col - a * q.bg;
+        const int col = min(32 * max(tile[z], 0) + ln, ncol - 1), a = over16(col, q.bg_inv), b = col - a * q.bg;
         bp[z] = rp + (q.zb + b * q.pitch + a) * BLK + 8 * kh;
     }
     const int start = (MIRROR ? 31 - ln : PZ + T - 1 - ln) + 8 * kh;    // forward: line[start - 32 d + j], mirror: line[start + 32 d + j]
@@ -811,22 +871,24 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
     run(std::integral_constant<int, 1>{}, max(d0, nd[1]), d1);
     // the sums of a pair's other waves, through the LDS that the rows no longer need
     bool owner = pair != NO_PAIR;
-    for (int x = 0; x < wv; ++x) owner &= plan.pair[x] != pair;
+    for (int x = 0; x < wv; ++x) owner &= ConvPlan::of(pairs, x) != pair;
     float4* const slot = reinterpret_cast<float4*>(lds);
     constexpr int SLOT4 = SUM_SLOT / 4;
-    __syncthreads();
-    if (pair != NO_PAIR && !owner) {
+    if (plan.shared) {
+        __syncthreads();
+        if (pair != NO_PAIR && !owner) {
 #pragma unroll
-        for (int z = 0; z < 2; ++z)
+            for (int z = 0; z < 2; ++z)
 #pragma unroll
-            for (int v4 = 0; v4 < 4; ++v4)
-                slot[wv * SLOT4 + (4 * z + v4) * 64 + lane] = make_float4(acc[z][4 * v4] + low[z][4 * v4], acc[z][4 * v4 + 1] + low[z][4 * v4 + 1],
-                                                                         acc[z][4 * v4 + 2] + low[z][4 * v4 + 2], acc[z][4 * v4 + 3] + low[z][4 * v4 + 3]);
+                for (int v4 = 0; v4 < 4; ++v4)
+                    slot[wv * SLOT4 + (4 * z + v4) * 64 + lane] = make_float4(acc[z][4 * v4] + low[z][4 * v4], acc[z][4 * v4 + 1] + low[z][4 * v4 + 1],
+                                                                             acc[z][4 * v4 + 2] + low[z][4 * v4 + 2], acc[z][4 * v4 + 3] + low[z][4 * v4 + 3]);
+        }
+        __syncthreads();
     }
-    __syncthreads();
     if (!owner) return;
     for (int x = wv + 1; x < TXW; ++x) {
-        if (plan.pair[x] != pair) continue;
+        if (ConvPlan::of(pairs, x) != pair) continue;
 #pragma unroll
         for (int z = 0; z < 2; ++z)
 #pragma unroll
@@ -837,7 +899,7 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
     }
 #pragma unroll
     for (int z = 0; z < 2; ++z) {
-        const int col = 32 * tile[z] + ln, a = col / q.bg, b = col - a * q.bg;
+        const int col = 32 * tile[z] + ln, a = over16(col, q.bg_inv), b = col - a * q.bg;
         if (tile[z] >= 0 && col < ncol) {
             float* o = out + (static_cast<size_t>(b0 + b) * C + c) * T;
 #pragma unroll
@@ -867,8 +929,9 @@ DEVINL void add_diagonals(float* diag, const f32x16& acc, int d, int ln, int kh)
     else if (ln >= 1) diag[64 * d + ln - 1] += neg;
 }
 
-// one workgroup: channel c = blockIdx.x, batch groups blockIdx.y, blockIdx.y + gridDim.y, ...; out[blockIdx.y][c][T]
-__global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__ k, const float* __restrict__ g, float* __restrict__ out,
+// The kernel gradient of short rows (T <= GW_SHORT), where a tile of 256 lags is mostly empty: lag tiles of 32, M_d of columns (block, row) as in
+// the convolution.  One workgroup: channel c = blockIdx.x, batch groups blockIdx.y, blockIdx.y + gridDim.y, ...; out[blockIdx.y][c][T]
+__global__ __launch_bounds__(TXT, 4) void timex_gw_short(const float* __restrict__ k, const float* __restrict__ g, float* __restrict__ out,
                                                        int B, int C, int T, int ng, const AnyGeom q) {
     extern __shared__ __align__(16) float lds[];
     const int plane = static_cast<int>(q.plane());
@@ -925,7 +988,7 @@ __global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__
             uint32_t at[2];
 #pragma unroll
             for (int z = 0; z < 2; ++z) {
-                const int col = 16 * s + 8 * kh + (l16 >> 2) + 4 * z, a = col / q.bg;
+                const int col = 16 * s + 8 * kh + (l16 >> 2) + 4 * z, a = over16(col, q.bg_inv);
                 bb[z] = col - a * q.bg;
                 at[z] = lds0 + 2u * static_cast<uint32_t>((q.zb + bb[z] * q.pitch + a) * BLK + 16 * (ln >> 4) + 4 * (l16 & 3));
             }
@@ -974,6 +1037,137 @@ __global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__
         o[x] = diag[64 * d + 31 + e] + (d + 1 < q.nt ? diag[64 * (d + 1) + e - 1] : 0.f);
     }
 }
+// one workgroup: channel c = blockIdx.x, the batch rows of part blockIdx.y of gridDim.y, at most q.bg at a time; out[blockIdx.y][c][T]
+__global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__ k, const float* __restrict__ g, float* __restrict__ out,
+                                                       int B, int C, int T, const GwGeom q) {
+    extern __shared__ __align__(16) float lds[];
+    uint16_t* gp = reinterpret_cast<uint16_t*>(lds);            // [bg][NPL][plane]
+    int* red = reinterpret_cast<int*>(gp + q.bg * NPL * q.plane);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, kg = lane >> 4;
+    const int c = blockIdx.x, np = gridDim.y, fewer = B / np, more = B % np, part = blockIdx.y;
+    const int first = part * fewer + min(part, more), last = first + fewer + (part < more ? 1 : 0);
+    const int bg = (last - first + (last - first + q.bg - 1) / q.bg - 1) / ((last - first + q.bg - 1) / q.bg);      // rows at a time, dealt evenly
+    float* const o = out + (static_cast<size_t>(part) * C + c) * T;
+    // nothing writes to the zeros around the rows again
+    for (int i = tid; i < bg * NPL * q.plane / 8; i += TXT) reinterpret_cast<uint4*>(lds)[i] = make_uint4(0, 0, 0, 0);
+    constexpr int NP = GW_PIECES;
+    const int per = 8 * q.nt;
+    float4 xg[NP], xk[NP];
+    auto fetch = [&](const int b0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) xg[i] = xk[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for_pieces<NP>(bg, per, q.per_inv, [&](int i, int rr, int t) __attribute__((always_inline)) {
+            if (rr < bg && b0 + rr < last && t < T) {
+                const size_t at = (static_cast<size_t>(b0 + rr) * C + c) * T + t;
+                xg[i] = *reinterpret_cast<const float4*>(g + at);
+                xk[i] = *reinterpret_cast<const float4*>(k + at);
+            }
+        });
+    };
+    fetch(first);
+    if (tid == 0) *red = 0;
+    // what this wave adds up: lag tiles q0 .. q0 + nq - 1, every nw-th of the steps that they have
+    const int all = (T + 255) >> 8;
+    const bool wide = all > GW_TILES, second = wide && wv >= GW_WAVES;
+    const int q0 = second ? GW_TILES : 0, nq = min(all - q0, GW_TILES), nw = wide ? (second ? TXW - GW_WAVES : GW_WAVES) : TXW;
+    const int steps = q.nt - 8 * q0;
+    f32x4 acc[GW_TILES], low[GW_TILES];          // as in timex_conv_any
+#pragma unroll
+    for (int z = 0; z < GW_TILES; ++z)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[z][v] = low[z][v] = 0.f;
+    // g[t + (i & 7) + 128 (i >> 3)], K slots t = 8 kg ..; k[t - 8 j]
+    const uint32_t* const ga = reinterpret_cast<const uint32_t*>(gp) + (((l16 & 7) + GW_OVER * (l16 >> 3) + 8 * kg) >> 1) + GW_OVER * q0;
+    const uint32_t odd = 16 * (l16 & 1);
+    const uint16_t* const ka = gp + q.k + 8 * kg - 8 * l16;
+    bool fell = false;
+    for (int b0 = first; b0 < last; b0 += bg) {
+        bool beyond = false;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) beyond |= beyond_terms(xg[i]) | beyond_terms(xk[i]);
+        __syncthreads();               // everybody is done with the group before
+        const bool loop = any_thread(beyond, red);
+        if (loop) {
+            for (int lag = tid; lag < T; lag += TXT) {
+                float a = fell ? o[T - 1 - lag] : 0.f;
+                for (int b = b0; b < last && b < b0 + bg; ++b) {
+                    const size_t row = (static_cast<size_t>(b) * C + c) * T;
+                    for (int u = 0; u + lag < T; ++u) a = fmaf(g[row + u + lag], k[row + u], a);
+                }
+                o[T - 1 - lag] = a;    // (read again by this thread alone)
+            }
+            fell = true;
+        } else {
+            for_pieces<NP>(bg, per, q.per_inv, [&](int i, int rr, int t) __attribute__((always_inline)) {
+                if (rr >= bg) return;
+                const B3x4 yg = split3x4(xg[i]), yk = split3x4(xk[i]);
+                uint16_t* d = gp + rr * NPL * q.plane + GW_OVER * (t >> 7);
+                uint16_t* dk = gp + rr * NPL * q.plane + q.k + t;
+                const int r = t & 127;
+                const bool twice = r < GW_OVER - 128 && t >= 128;
+                static_assert(GW_OVER == 128 + 16, "");
+#pragma unroll
+                for (int p = 0; p < NPL; ++p, d += q.plane, dk += q.plane) {
+                    *reinterpret_cast<uint2*>(d + r) = yg.p[p];
+                    if (twice) *reinterpret_cast<uint2*>(d + r - 16) = yg.p[p];        // at the end of the block before
+                    *reinterpret_cast<uint2*>(dk) = yk.p[p];
+                }
+            });
+        }
+        if (b0 + bg < last) fetch(b0 + bg);
+        __syncthreads();
+        if (tid == 0) *red = 0;
+        if (loop || steps <= 0) continue;
+        const int rows = min(bg, last - b0);
+        int s = second ? wv - GW_WAVES : wv, row = 0;
+        for (; s >= steps; s -= steps) ++row;
+        while (row < rows) {
+            const uint32_t* a4 = ga + (row * NPL * q.plane >> 1) + (GW_OVER / 2) * (s >> 2) + 16 * (s & 3);
+            const uint16_t* b8 = ka + row * NPL * q.plane + 32 * s;
+            const int on = min(nq, (s >> 3) + 1);
+            bf16x8 fa[NPL];
+#pragma unroll
+            for (int p = 0; p < NPL; ++p, a4 += q.plane >> 1) {
+                uint32_t x[5];
+#pragma unroll
+                for (int e = 0; e < 5; ++e) x[e] = a4[e];
+                fa[p] = __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_alignbit(x[1], x[0], odd), __builtin_amdgcn_alignbit(x[2], x[1], odd),
+                                                              __builtin_amdgcn_alignbit(x[3], x[2], odd), __builtin_amdgcn_alignbit(x[4], x[3], odd)));
+            }
+#pragma unroll
+            for (int z = 0; z < GW_TILES; ++z)
+                if (z < on) {
+                    bf16x8 fb[NPL];
+#pragma unroll
+                    for (int p = 0; p < NPL; ++p) fb[p] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(b8 + p * q.plane - 256 * z));
+#pragma unroll
+                    for (int term = 0; term < 6; ++term) {
+                        f32x4& sum = term == 5 ? acc[z] : low[z];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[TERM_A[term]], fb[TERM_B[term]], sum, 0, 0, 0);
+                    }
+                }
+            for (s += nw; s >= steps; s -= steps) ++row;
+        }
+    }
+    // the waves' sums, in their order, through the LDS that the rows no longer need
+    __syncthreads();
+    f32x4* const slot = reinterpret_cast<f32x4*>(lds);
+    const int slots = min(all, GW_TILES);
+#pragma unroll
+    for (int z = 0; z < GW_TILES; ++z)
+        if (z < nq) slot[(wv * slots + z) * 64 + lane] = acc[z] + low[z];
+    __syncthreads();
+    for (int lag = tid; lag < T; lag += TXT) {
+        const int r = lag & 255, i = (r & 7) + 8 * (r >> 7), z = lag >> 8;
+        const bool up = z >= GW_TILES;
+        const int w0 = up ? GW_WAVES : 0, w1 = wide && !up ? GW_WAVES : TXW;
+        const float* x = lds + (w0 * slots + (up ? z - GW_TILES : z)) * 256 + (16 * (i >> 2) + ((r >> 3) & 15)) * 4 + (i & 3);
+        float sum = fell ? o[T - 1 - lag] : 0.f;
+        for (int w = w0; w < w1; ++w, x += 256 * slots) sum += *x;
+        o[T - 1 - lag] = sum;
+    }
+}
 // out[x] = sum of n parts that lie `size` floats apart, four elements a thread
 __global__ __launch_bounds__(256) void timex_add_parts(const float4* __restrict__ part, float4* __restrict__ out, size_t size4, int n) {
     const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -986,8 +1180,10 @@ __global__ __launch_bounds__(256) void timex_add_parts(const float4* __restrict_
     out[i] = a;
 }
 
-// The waves' shares: runs of a pair's lags are added where the longest run is, until there are eight, then the longest four runs go to the
+// The waves' shares: runs of a pair's lags are added where the longest run is, until there are eight or a run would have less than RUN_MIN
+// steps (of a tile and a lag; so many take about what it takes to add two waves' sums), then the longest four runs go to the
 // four SIMDs (a wave w runs on SIMD w mod 4) and the others to the least loaded ones.
+constexpr int RUN_MIN = 4;
 void plan_waves(ConvPlan& p, bool mirror) {
     const int ntile = (p.q.nt * p.q.bg + 31) / 32, npair = (ntile + 1) / 2;
     int lags[TXW][2] = {}, runs[TXW] = {}, work[TXW] = {};
@@ -1002,7 +1198,7 @@ void plan_waves(ConvPlan& p, bool mirror) {
     for (int n = npair; n < TXW; ++n) {
         int most = -1;
         for (int m = 0; m < npair; ++m)
-            if (runs[m] < lags[m][0] && (most < 0 || work[m] * runs[most] > work[most] * runs[m])) most = m;
+            if (work[m] >= RUN_MIN * (runs[m] + 1) && (most < 0 || work[m] * runs[most] > work[most] * runs[m])) most = m;
         if (most < 0) break;
         ++runs[most];
     }
@@ -1016,14 +1212,19 @@ void plan_waves(ConvPlan& p, bool mirror) {
         }
     }
     std::sort(run, run + n, [](const Run& a, const Run& b) { return a.work > b.work; });
-    for (int w = 0; w < TXW; ++w) p.pair[w] = NO_PAIR, p.d0[w] = p.d1[w] = 0;
+    p.shared = n > npair;
+    p.pair = ~uint64_t{0};
+    p.d0 = p.d1 = 0;
     for (int i = 0; i < n; ++i) {
-        const int w = i < 4 ? i : 11 - i;
-        p.pair[w] = static_cast<uint8_t>(run[i].pair);
-        p.d0[w] = static_cast<uint8_t>(run[i].d0); p.d1[w] = static_cast<uint8_t>(run[i].d1);
+        const int at = 8 * (i < 4 ? i : 11 - i);
+        p.pair ^= static_cast<uint64_t>(NO_PAIR ^ run[i].pair) << at;
+        p.d0 |= static_cast<uint64_t>(run[i].d0) << at;
+        p.d1 |= static_cast<uint64_t>(run[i].d1) << at;
     }
 }
-size_t conv_plan_lds(const ConvPlans& x) { return std::max({conv_any_lds(x.p[0].q), conv_any_lds(x.p[1].q), TXW * SUM_SLOT * sizeof(float)}); }
+size_t conv_plan_lds(const ConvPlans& x) {
+    return std::max({conv_any_lds(x.p[0].q), conv_any_lds(x.p[1].q), x.p[0].shared || x.p[1].shared ? TXW * SUM_SLOT * sizeof(float) : 0});
+}
 // Batch rows of a unit, dealt evenly to `ng` units a channel.  What finishes first by a count of matrix clocks (96 per column tile and
 // block lag on a CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (a pair a wave) and
 // 80 KB (a single row may have more).
@@ -1051,19 +1252,46 @@ ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
     for (ConvPlan& p : best.p) plan_waves(p, mirror);
     return best;
 }
-AnyGeom gw_any_geom(int B, int T) {
+// Up to here the kernel gradient takes lag tiles of 32 (timex_gw_short).  Lag tiles of 32 / of 256, the kernel alone: B32 C1000 T36 12.7 / 16.2 us,
+// B20 C700 T260 27.6 / 27.7 (forward + backward 59.9 / 62.1), B30 C200 T516 29.6 / 27.3, B13 C384 T1500 107 / 77.
+constexpr int GW_SHORT = 384;
+inline size_t gw_short_lds(const AnyGeom& q) { return 2 * NPL * q.plane() * 2 + static_cast<size_t>(q.nt) * 256 + 16; }
+AnyGeom gw_short_geom(int B, int T) {
     AnyGeom best = any_geom(T, 1, 15);
     for (int bg = 2; bg <= B && bg <= 32; ++bg) {
         const AnyGeom q = any_geom(T, bg, 15);
-        if (gw_any_lds(q) > LDS_ANY || 8 * q.nt * bg > GW_PIECES * TXT) break;
+        if (gw_short_lds(q) > LDS_ANY || 8 * q.nt * bg > GW_PIECES * TXT) break;
         best = q;
     }
     return best;
 }
-// batch groups that work side by side (their sums are added by a second kernel): as many as it takes for two workgroups per CU
-int gw_any_parts(int B, int C, const AnyGeom& q) {
-    const int ng = (B + q.bg - 1) / q.bg, want = (2 * NCU + C - 1) / C;
-    return ng < want ? ng : want;
+// as many rows at a time as leave room for two workgroups per CU
+GwGeom gw_any_geom(int B, int T) {
+    GwGeom best = gw_geom(T, 1);
+    for (int bg = 2; bg <= B && bg <= 32; ++bg) {
+        const GwGeom q = gw_geom(T, bg);
+        if (gw_any_lds(q, T) > LDS_ANY || 8 * q.nt * bg > GW_PIECES * TXT) break;
+        best = q;
+    }
+    return best;
+}
+// Parts of the batch that work side by side (their sums are added by a second kernel): what finishes first by a count of clocks, in rounds of
+// two workgroups per CU: 48 a row, step and lag tile, 3 a row and step of time for its conversion, a fixed cost a workgroup and that of the second kernel.
+int gw_any_parts(int B, int C, int T) {
+    if (T <= GW_SHORT) {               // (groups of rows side by side, as many as it takes for two workgroups per CU)
+        const int bg = gw_short_geom(B, T).bg, ng = (B + bg - 1) / bg, want = (2 * NCU + C - 1) / C;
+        return ng < want ? ng : want;
+    }
+    const int nt = (T + 31) / 32;
+    long long row = 3LL * T;
+    for (int s = 0; s < nt; s += 8) row += 48LL * (nt - s);
+    int best = 1;
+    long long cost = -1;
+    for (int p = 1; p <= B && (p == 1 || static_cast<long long>(C) * p <= 8 * NCU); ++p) {
+        const long long x = (static_cast<long long>(C) * p + 2 * NCU - 1) / (2 * NCU) * (12000 + row * B / p) + (p > 1 ? 10000 : 0);
+        if (cost < 0 || x < cost) { cost = x; best = p; }
+    }
+    return best;
 }
 
 constexpr int T_MAX = 4096;
@@ -1151,7 +1379,7 @@ int rwkv_timex_backward_sum(void* stream, const float* w, const float* k, const 
 
 size_t rwkv_timex_backward_ws_bytes(int B, int C, int T) {
     if (check_tx(B, C, T) != RWKV_OK || (T % 32 == 0 && T <= T_MFMA_MAX)) return 0;
-    const int parts = gw_any_parts(B, C, gw_any_geom(B, T));
+    const int parts = gw_any_parts(B, C, T);
     return parts <= 1 ? 0 : static_cast<size_t>(parts) * C * T * sizeof(float);
 }
 
@@ -1160,14 +1388,22 @@ int rwkv_timex_backward_ws(void* stream, const float* w, const float* k, const f
     if (int e = check_tx(B, C, T)) return e;
     if (T % 32 == 0 && T <= T_MFMA_MAX) return rwkv_timex_backward_sum(stream, w, k, gwk, gw_sum, gk, B, C, T);
     if (int e = check_ptrs({w, k, gwk, gw_sum, gk})) return e;
-    const AnyGeom q = gw_any_geom(B, T);
-    const int ng = (B + q.bg - 1) / q.bg, parts = gw_any_parts(B, C, q);
+    const int parts = gw_any_parts(B, C, T);
     if (parts > 1 && (workspace == nullptr || workspace_bytes < rwkv_timex_backward_ws_bytes(B, C, T) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
     if (int e = launch_conv<true>(stream, w, gwk, gk, 0.0f, B, C, T)) return e;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const size_t lds = gw_any_lds(q);
-    if (int e = raise_lds_limit(timex_gw_any, lds)) return e;
-    hipLaunchKernelGGL(timex_gw_any, dim3(C, parts), dim3(TXT), lds, st, k, gwk, parts > 1 ? static_cast<float*>(workspace) : gw_sum, B, C, T, ng, q);
+    float* const to = parts > 1 ? static_cast<float*>(workspace) : gw_sum;
+    if (T <= GW_SHORT) {
+        const AnyGeom q = gw_short_geom(B, T);
+        const size_t lds = gw_short_lds(q);
+        if (int e = raise_lds_limit(timex_gw_short, lds)) return e;
+        hipLaunchKernelGGL(timex_gw_short, dim3(C, parts), dim3(TXT), lds, st, k, gwk, to, B, C, T, (B + q.bg - 1) / q.bg, q);
+    } else {
+        const GwGeom q = gw_any_geom(B, T);
+        const size_t lds = gw_any_lds(q, T);
+        if (int e = raise_lds_limit(timex_gw_any, lds)) return e;
+        hipLaunchKernelGGL(timex_gw_any, dim3(C, parts), dim3(TXT), lds, st, k, gwk, to, B, C, T, q);
+    }
     if (parts > 1) {
         const size_t n4 = static_cast<size_t>(C) * T / 4;
         hipLaunchKernelGGL(timex_add_parts, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, st,

@@ -1,9 +1,9 @@
-"""GPU: depthwise_conv1d at the lengths and batch sizes that are not whole tiles (timex_conv_any, timex_gw_any), against the fp64
+"""GPU: depthwise_conv1d at the lengths and batch sizes that are not whole tiles (timex_conv_any, timex_gw_any, timex_gw_short), against the fp64
 oracle: one block of steps, a block and a piece, odd numbers of blocks, the longest sequence, batches of one row up to more than
 one unit, batch groups that are summed by a second kernel and ones that are not.
 
 Tolerance: the fp32 ops' bar of 1e-5, and element by element the bound of an fp32 loop: n products leave at most n 2^-24 of the
-sum of their magnitudes.  An operand keeps its 24 bits, a product loses less than 2^-23, and a matrix instruction adds sixteen products
+sum of their magnitudes.  An operand keeps its 24 bits, a product loses less than 2^-23, and a matrix instruction adds up to 32 products
 at a time in six parts: fewer roundings than the loop has."""
 import pytest
 import torch
@@ -28,7 +28,7 @@ def _check(B, C, T, w, k, g, eps=0.25):
         assert e <= 1e-5 and m <= 1e-5, name
 
 
-@pytest.mark.parametrize("T", [4, 8, 28, 32, 36, 60, 100, 516, 1000, 1028, 1056, 1500, 2048, 4092, 4096])
+@pytest.mark.parametrize("T", [4, 8, 28, 32, 36, 60, 100, 384, 388, 516, 1000, 1028, 1056, 1500, 2048, 2052, 4092, 4096])
 @pytest.mark.parametrize("B", [1, 2, 5, 13])
 def test_shapes(lib, B, T):
     print(f"\ntimex any B={B} T={T}", flush=True)
