@@ -77,7 +77,7 @@ struct Args7c {
 };
 
 // Whole sequences (CUT = false) have an instance of their kernels of their own: with the choice left to run time what belongs to the
-// blocks costs them scalar work and the backward 4 registers (B8 4 x T1024 C4096 3.87 -> 3.83 ms).
+// blocks costs them scalar work (B8 4 x T1024 C4096 3.87 -> 3.83 ms).
 template <bool CUT> DEVINL Args7c only_whole(Args7c p) {
     if constexpr (!CUT) p.NB = 1;
     return p;
