@@ -586,8 +586,8 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // under a common power of two (half the products, 58 and 101 us where these took 95 and 111) do not give.  A unit with an element that is no number, infinite or beyond
 // bf16's largest is done by such a loop (a matrix product would carry it to earlier steps: zero times infinity).
 // Rows lie in LDS as blocks of 32 + 8 terms (80 bytes: 16-byte reads of neighbouring columns fall on different banks if a
-// row has an odd number of blocks), 512 threads, 128 registers, and up to T = 3360 (gradient: always) at most 80 KB: two
-// workgroups share a CU, one converts its rows while the other multiplies; longer rows take a CU each.  B13 C384 T1500:
+// row has an odd number of blocks), 512 threads, 128 registers, and at most 80 KB: two
+// workgroups share a CU, one converts its rows while the other multiplies.  B13 C384 T1500:
 // 77 us a convolution (92 with a wave per column tile and units of 4, 4, 4 and 1 rows; matrix pipes busy 70 % of the time that a CU has
 // work), 77 us the kernel gradient (107 as lag tiles of 32), relative errors 1.8e-7 and 1.0e-7; the fp32 loops on the vector units
 // that these replace took 315 / 286 and, with the sum over the batch, 243 us, with 5.6e-7.
@@ -637,7 +637,10 @@ struct ConvPlan {
 };
 static_assert(TXW == 8, "a word holds a byte a wave");
 static_assert(T_ANY / 32 < 255, "a block lag is a byte");
-struct ConvPlans { ConvPlan p[2]; };   // for units of ceil(B / groups) and of floor(B / groups) rows
+// copies: of the taps' line.  With the second one, shifted by one, an odd window begins at a whole dword as an even one does; with one it is
+// five dwords, shifted in registers, which makes room for a second workgroup on a CU beyond T = 3360: B1 C1024 T4096 forward + backward 297 us
+// with two copies, 265 with one; T1500 with two 212, with one 216.
+struct ConvPlans { ConvPlan p[2]; int copies; };   // p: for units of ceil(B / groups) and of floor(B / groups) rows
 __host__ __device__ inline int tile_lags(const AnyGeom& q, bool mirror, int tile) {
     const int ncol = q.nt * q.bg, last = 32 * tile + 31 < ncol ? 32 * tile + 31 : ncol - 1;
     return mirror ? q.nt - over16(32 * tile, q.bg_inv) : over16(last, q.bg_inv) + 1;
@@ -645,7 +648,7 @@ __host__ __device__ inline int tile_lags(const AnyGeom& q, bool mirror, int tile
 // tile number `rank` in the order of decreasing work; none: -1
 __host__ __device__ inline int tile_of(int ntile, bool mirror, int rank) { return rank < ntile ? (mirror ? rank : ntile - 1 - rank) : -1; }
 constexpr size_t SUM_SLOT = 2 * 32 * 32;      // floats of a wave's two tiles
-inline size_t conv_any_lds(const AnyGeom& q) { return (NPL * q.plane() + 2 * NPL * static_cast<size_t>(h2_line_len(32 * q.nt))) * 2 + 16; }
+inline size_t conv_any_lds(const AnyGeom& q, int copies) { return (NPL * q.plane() + copies * NPL * static_cast<size_t>(h2_line_len(32 * q.nt))) * 2 + 16; }
 
 // The kernel gradient.  In LDS g lies in blocks of 128 steps and the GW_OVER - 128 after them (a window of eight steps is read within one
 // block), a zero block behind, which is also what lies in front of k.  A window that begins at an odd step is the same five dwords as
@@ -745,6 +748,14 @@ DEVINL void put_line4(uint16_t* line, uint16_t* copy, int at, const uint2& y) {
     *reinterpret_cast<uint32_t*>(copy + at) = (y.x >> 16) | (y.y << 16);
     copy[at + 2] = static_cast<uint16_t>(y.y >> 16);
 }
+// eight elements from the first (shift = 0) or second (16) of the dwords at x
+DEVINL bf16x8 window8(const uint32_t* x, uint32_t shift) {
+    uint32_t d[5];
+#pragma unroll
+    for (int e = 0; e < 5; ++e) d[e] = x[e];
+    return __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_alignbit(d[1], d[0], shift), __builtin_amdgcn_alignbit(d[2], d[1], shift),
+                                                 __builtin_amdgcn_alignbit(d[3], d[2], shift), __builtin_amdgcn_alignbit(d[4], d[3], shift)));
+}
 // the blocks in front of the first row and behind every row
 DEVINL void zero_blocks(uint16_t* rp, const AnyGeom& q) {
     const int n = q.zb * (q.bg + 1) * (BLK / 8);
@@ -757,7 +768,7 @@ DEVINL void zero_blocks(uint16_t* rp, const AnyGeom& q) {
     }
 }
 
-template <bool MIRROR>
+template <bool MIRROR, int COPIES>
 __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict__ w, const float* __restrict__ in, float* __restrict__ out,
                                                          float eps, int B, int C, int T, int ng, const ConvPlans plans) {
     extern __shared__ __align__(16) float lds[];
@@ -766,8 +777,8 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
     const AnyGeom& q = plan.q;
     const int Tp = 32 * q.nt, xl = h2_line_len(Tp), plane = static_cast<int>(q.plane());
     uint16_t* rp = reinterpret_cast<uint16_t*>(lds);                    // [NPL][plane]
-    uint16_t* al = rp + NPL * plane;                                    // [NPL planes][2 copies][xl]
-    int* red = reinterpret_cast<int*>(al + 2 * NPL * xl);
+    uint16_t* al = rp + NPL * plane;                                    // [NPL planes][COPIES][xl]
+    int* red = reinterpret_cast<int*>(al + COPIES * NPL * xl);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, kh = lane >> 5;
     {
         Stager<CONV_PIECES> st;
@@ -778,7 +789,7 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
             const int tau = 4 * (z * TXT + tid);
             wr[z] = tau < T ? *reinterpret_cast<const float4*>(w + static_cast<size_t>(c) * T + tau) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
-        for (int i = tid; i < NPL * xl / 4; i += TXT) reinterpret_cast<uint4*>(al)[i] = make_uint4(0, 0, 0, 0);
+        for (int i = tid; i < COPIES * NPL * xl / 8; i += TXT) reinterpret_cast<uint4*>(al)[i] = make_uint4(0, 0, 0, 0);
         zero_blocks(rp, q);
         if (tid == 0) *red = 0;
         bool beyond = st.beyond();
@@ -807,15 +818,18 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
                 const B3x4 a = split3x4(MIRROR ? make_float4(wr[z].w, wr[z].z, wr[z].y, wr[z].x) : wr[z]);
 #pragma unroll
                 for (int p = 0; p < NPL; ++p) {
-                    uint16_t *line = al + 2 * p * xl, *copy = line + xl;
+                    uint16_t *line = al + COPIES * p * xl, *copy = line + xl;
                     if constexpr (MIRROR) {
                         line += 28 + T - 4 - tau; copy += 28 + T - 4 - tau;          // (the lowest of the four at line[3], copy[2])
                         line[3] = static_cast<uint16_t>(a.p[p].x);
                         *reinterpret_cast<uint32_t*>(line + 4) = (a.p[p].x >> 16) | (a.p[p].y << 16);
                         line[6] = static_cast<uint16_t>(a.p[p].y >> 16);
-                        *reinterpret_cast<uint32_t*>(copy + 2) = a.p[p].x;
-                        *reinterpret_cast<uint32_t*>(copy + 4) = a.p[p].y;
-                    } else put_line4(line, copy, PZ + tau, a.p[p]);
+                        if constexpr (COPIES == 2) {
+                            *reinterpret_cast<uint32_t*>(copy + 2) = a.p[p].x;
+                            *reinterpret_cast<uint32_t*>(copy + 4) = a.p[p].y;
+                        }
+                    } else if constexpr (COPIES == 2) put_line4(line, copy, PZ + tau, a.p[p]);
+                    else *reinterpret_cast<uint2*>(line + PZ + tau) = a.p[p];
                 }
             }
         }
@@ -834,7 +848,8 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
         bp[z] = rp + (q.zb + b * q.pitch + a) * BLK + 8 * kh;
     }
     const int start = (MIRROR ? 31 - ln : PZ + T - 1 - ln) + 8 * kh;    // forward: line[start - 32 d + j], mirror: line[start + 32 d + j]
-    const uint32_t* ap = reinterpret_cast<const uint32_t*>(al + (start & 1) * xl) + (start >> 1);
+    const uint32_t* ap = reinterpret_cast<const uint32_t*>(al + (COPIES == 2 ? start & 1 : 0) * xl) + (start >> 1);
+    const uint32_t odd = 16 * (start & 1);
     f32x16 acc[2], low[2];          // the products of the first terms, which are what rounds; the other five
 #pragma unroll
     for (int z = 0; z < 2; ++z)
@@ -849,8 +864,9 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
                 bf16x8 fa[NPL], fb[NT_][NPL];
 #pragma unroll
                 for (int p = 0; p < NPL; ++p) {
-                    const uint32_t* a4 = ap + 16 * o + 8 * ks + p * xl;          // a plane is 2 xl elements = xl dwords
-                    fa[p] = __builtin_bit_cast(bf16x8, make_uint4(a4[0], a4[1], a4[2], a4[3]));
+                    const uint32_t* a4 = ap + 16 * o + 8 * ks + p * (COPIES * xl >> 1);
+                    if constexpr (COPIES == 2) fa[p] = __builtin_bit_cast(bf16x8, make_uint4(a4[0], a4[1], a4[2], a4[3]));
+                    else fa[p] = window8(a4, odd);
                 }
 #pragma unroll
                 for (int z = 0; z < NT_; ++z)
@@ -1129,11 +1145,7 @@ __global__ __launch_bounds__(TXT, 4) void timex_gw_any(const float* __restrict__
             bf16x8 fa[NPL];
 #pragma unroll
             for (int p = 0; p < NPL; ++p, a4 += q.plane >> 1) {
-                uint32_t x[5];
-#pragma unroll
-                for (int e = 0; e < 5; ++e) x[e] = a4[e];
-                fa[p] = __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_alignbit(x[1], x[0], odd), __builtin_amdgcn_alignbit(x[2], x[1], odd),
-                                                              __builtin_amdgcn_alignbit(x[3], x[2], odd), __builtin_amdgcn_alignbit(x[4], x[3], odd)));
+                fa[p] = window8(a4, odd);
             }
 #pragma unroll
             for (int z = 0; z < GW_TILES; ++z)
@@ -1223,11 +1235,11 @@ void plan_waves(ConvPlan& p, bool mirror) {
     }
 }
 size_t conv_plan_lds(const ConvPlans& x) {
-    return std::max({conv_any_lds(x.p[0].q), conv_any_lds(x.p[1].q), x.p[0].shared || x.p[1].shared ? TXW * SUM_SLOT * sizeof(float) : 0});
+    return std::max({conv_any_lds(x.p[0].q, x.copies), conv_any_lds(x.p[1].q, x.copies), x.p[0].shared || x.p[1].shared ? TXW * SUM_SLOT * sizeof(float) : 0});
 }
 // Batch rows of a unit, dealt evenly to `ng` units a channel.  What finishes first by a count of matrix clocks (96 per column tile and
 // block lag on a CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (a pair a wave) and
-// 80 KB (a single row may have more).
+// 80 KB.
 ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
     ConvPlans best{};
     double cost = 1e300;
@@ -1245,6 +1257,7 @@ ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
             for (int t = 0; t < ntile; ++t) steps += tile_lags(x.p[z].q, mirror, t);
             unit += (96.0 * steps + 0.15 * rows[z] * T + 3000.0) * share / groups;
         }
+        x.copies = most == 1 && conv_any_lds(x.p[0].q, 2) > LDS_ANY ? 1 : 2;
         if (unit < 0 || conv_plan_lds(x) > LDS_ANY || 8 * x.p[0].q.nt * rows[0] > CONV_PIECES * TXT) { if (most > 1) break; }
         const double c = static_cast<double>((static_cast<long long>(C) * groups + 2 * NCU - 1) / (2 * NCU)) * unit;
         if (c < cost) { cost = c; best = x; *ng = groups; }
@@ -1337,8 +1350,9 @@ template <bool MIRROR> int launch_conv(void* stream, const float* w, const float
         const ConvPlans plans = conv_any_plans(B, C, T, MIRROR, &ng);
         const size_t lds = conv_plan_lds(plans);
         if (static_cast<long long>(C) * ng > 0x7fffffffLL) return RWKV_ERR_SHAPE;
-        if (int e = raise_lds_limit(timex_conv_any<MIRROR>, lds)) return e;
-        hipLaunchKernelGGL(timex_conv_any<MIRROR>, dim3(C * ng), dim3(TXT), lds, st, w, in, out, eps, B, C, T, ng, plans);
+        const auto kernel = plans.copies == 2 ? timex_conv_any<MIRROR, 2> : timex_conv_any<MIRROR, 1>;
+        if (int e = raise_lds_limit(kernel, lds)) return e;
+        hipLaunchKernelGGL(kernel, dim3(C * ng), dim3(TXT), lds, st, w, in, out, eps, B, C, T, ng, plans);
     }
     return RWKV_OK;
 }
