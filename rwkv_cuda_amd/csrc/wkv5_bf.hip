@@ -129,12 +129,20 @@ DEVINL Op2 split8(const float (&x)[8]) {
 DEVINL Op2 split8(const f32x4& x, const f32x4& y) { const float f[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]}; return split8(f); }
 DEVINL f32x4 mm3(const Op2& a, const Op2& b, f32x4 c) { return mfma(a.l, b.h, mfma(a.h, b.l, mfma(a.h, b.h, c))); }
 DEVINL void unpack(const bf16x8& x, float (&f)[8]) { unpack8(__builtin_bit_cast(uint4, x), f); }
+// hi and lo of the products a p and b q; the remainders are those of the exact products.  (Written as a product and its split, they are that
+// where the compiler finds both in one basic block, and of the rounded product elsewhere.)
+DEVINL HL hilo2p(float a, float p, float b, float q) {
+    HL r;
+    r.h = cvt2(a * p, b * q);
+    asm("" : "+v"(r.h));
+    r.l = cvt2(fmaf(a, p, -__uint_as_float(r.h << 16)), fmaf(b, q, -__uint_as_float(r.h & 0xffff0000u)));
+    return r;
+}
 DEVINL Op2 scaled(const bf16x8& x, const float (&p)[8]) {
     float f[8];
     unpack(x, f);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] *= p[e];
-    return split8(f);
+    const HL a = hilo2p(f[0], p[0], f[1], p[1]), b = hilo2p(f[2], p[2], f[3], p[3]), c = hilo2p(f[4], p[4], f[5], p[5]), d = hilo2p(f[6], p[6], f[7], p[7]);
+    return {as_op(a.h, b.h, c.h, d.h), as_op(a.l, b.l, c.l, d.l)};
 }
 // Operand with the 32 rows (tokens) of a plane along K in accumulator order: slot (g, e) <-> row 16 (e >> 2) + 4 g + (e & 3), lane
 // <-> column.  a: element [4 g + (l16 >> 2)][col + 4 (l16 & 3)].
@@ -574,7 +582,9 @@ __global__ __launch_bounds__(NTH, 2) void wkv5b_fwd(const ArgsW p) {
 //      their gradient state in LDS (hi, lo) in the first, and the next chunk's tile B as the operands that the D waves take: B and
 //      its weighted form with lane = source, its transpose with lane = sink.
 // Twice four waves, of 32 key channels each and with the tile B made by each of the D waves, took 1042 us (B8 T4096 C4096 N128) where
-// these take 981 (heads of 64: the same).  Without its memory operations the kernel takes 753 us, and its 3.3 GB about 660 at a copy's rate.
+// these take 986 (heads of 64: the same), with the same bits: every sum has that kernel's order, so gr's tile part is kept over the barrier and
+// its bonus term added after the state's (the other way round 981 us).  Without its memory operations the kernel takes 753 us, and its 3.3 GB
+// about 660 at a copy's rate.
 template <bool LANE_SNK> DEVINL void mask(f32x4 (&b)[3], int l16, int g) {
 #pragma unroll
     for (int z = 0; z < 3; ++z)
@@ -582,14 +592,18 @@ template <bool LANE_SNK> DEVINL void mask(f32x4 (&b)[3], int l16, int g) {
         for (int v = 0; v < 4; ++v) b[z][v] = causal<LANE_SNK>(z, l16, 4 * g + v) ? b[z][v] : 0.f;
 }
 // The tile B as operands of its lane tiles, 3 KB a form.  The lane tile that meets both halves of the other side takes 16 bytes a lane
-// and term; the other one has zeros on one side (HIGH: in its low slots), the two terms share 16 bytes.
-template <bool LANE_SNK> DEVINL void put_tile(lds_t o, const f32x4 (&t)[3], int lane) {
-    const Op2 f = LANE_SNK ? split8(t[1], t[2]) : split8(t[0], t[1]);
-    const f32x4& s = LANE_SNK ? t[0] : t[2];
-    const HL a = hilo2k(s[0], s[1]), b = hilo2k(s[2], s[3]);
+// and term; the other one has zeros on one side (HIGH: in its low slots), the two terms share 16 bytes.  LAGS: every element times
+// the tokens between, lag + 16 (row tile - lane tile) + v.
+template <bool LANE_SNK, bool LAGS> DEVINL void put_tile(lds_t o, const f32x4 (&t)[3], int lane, float lag = 0.f) {
+    const auto two = [&](int z, int v) __attribute__((always_inline)) {
+        const float m = lag + static_cast<float>(16 * (Quad<LANE_SNK>::ROWT[z] - Quad<LANE_SNK>::LANET[z]) + v);
+        return LAGS ? hilo2p(t[z][v], m, t[z][v + 1], m + 1.f) : hilo2k(t[z][v], t[z][v + 1]);
+    };
+    constexpr int full = LANE_SNK ? 1 : 0, half = LANE_SNK ? 0 : 2;
+    const HL a = two(full, 0), b = two(full, 2), c = two(full + 1, 0), d = two(full + 1, 2), e = two(half, 0), f = two(half, 2);
     o += 16 * lane;
-    lds_st<bf16x8>(o, f.h); lds_st<bf16x8>(o + 1024, f.l);
-    lds_st<u32x4>(o + 2048, u32x4{a.h, b.h, a.l, b.l});
+    lds_st<bf16x8>(o, as_op(a.h, b.h, c.h, d.h)); lds_st<bf16x8>(o + 1024, as_op(a.l, b.l, c.l, d.l));
+    lds_st<u32x4>(o + 2048, u32x4{e.h, f.h, e.l, f.l});
 }
 template <bool HIGH> DEVINL Op2 half_op(lds_t o) {
     const u32x4 x = lds_ld<u32x4>(o + 2048);
@@ -676,11 +690,11 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
                     tile_offset(static_cast<int>(n), static_cast<int>(gg), C), static_cast<float>(4 * gg)};
     };
     // second half of a chunk: gr, update
-    auto second = [&](auto odd_, const int c, const f32x4 (&part)[2], f32x4 (&Sn)[2][2]) __attribute__((always_inline)) {
+    auto second = [&](auto odd_, const int c, const f32x4 (&tx)[2], f32x4 (&Sn)[2][2]) __attribute__((always_inline)) {
         constexpr bool ODD = decltype(odd_)::value;
         const lds_t sx = sb + A::BASE + (ODD ? A::SLOT : 0);
         const Lane at = lane_of();
-        const lds_t xr = at.row + sx, xu = at.tra + sx, xt = xu + 32 * q, qt = at.tra + sb + A::BASE + (ODD ? 0 : A::SLOT);
+        const lds_t xr = at.row + sx, xu = at.tra + sx, xt = xu + 32 * q, qt = at.tra + sb + A::BASE + (ODD ? 0 : A::SLOT), xs = sx + 4 * static_cast<lds_t>(at.t);
         const rows_t gr_ = rows_of(p.gr + base + static_cast<size_t>(c) * L * C + 16 * q, T - c * L, C);
         Op2 rs, kp;
         {
@@ -719,22 +733,25 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
         }
         stage();
         {
-            const uint4 r4 = __builtin_bit_cast(uint4, ld_tra<A::ROW>(xt + A::R));
-            float r[8], ps[8];
-            unpack8(r4, r);
-            from_start(ps);
-            const float th = at.t;
+            const uint4 r4 = __builtin_bit_cast(uint4, ld_tra<A::ROW>(xt + A::R)), k4 = __builtin_bit_cast(uint4, ld_tra<A::ROW>(xt + A::K));
+            const float u = lds_f(sb + A::U + 64 * q + (at.tile >> 2 & 60u));
+            const float bc = hide(cb), bs = bc * o8;
+            const float pc[4] = {bc, bc * o1, bc * o2, bc * o3}, ps[4] = {bs, bs * o1, bs * o2, bs * o3};
 #pragma unroll
             for (int z = 0; z < 2; ++z) {
+                const f32x4 vg4 = lds_ld<f32x4>(xs + A::VG + 64 * z);
+                const uint32_t rw[2] = {z ? r4.z : r4.x, z ? r4.w : r4.y}, kw[2] = {z ? k4.z : k4.x, z ? k4.w : k4.y};
+                const float th = at.t + static_cast<float>(16 * z);
                 f32x4 o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const int e = 4 * z + v;
-                    const float x = X[z][v] * ps[e];
-                    gw = fmaf(r[e] * (th + static_cast<float>(16 * z + v)), x, gw);
-                    o[v] = x + part[z][v];
+                    const float r = v & 1 ? bf_hi(rw[v >> 1]) : bf_lo(rw[v >> 1]), k = v & 1 ? bf_hi(kw[v >> 1]) : bf_lo(kw[v >> 1]);
+                    const float x = X[z][v] * (z ? ps[v] * o16 : ps[v]);
+                    gw = fmaf(r * (th + static_cast<float>(v)), x, gw);
+                    o[v] = fmaf(k * vg4[v], u, fmaf(tx[z][v], pc[v], x));
                 }
                 store_tile(gr_, at.out + 32 * z * C, C, static_cast<int>(at.tile >> 4), o);
+                stage();
             }
         }
     };
@@ -760,19 +777,10 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
                 Z[z] = mfma(va, s.l, mfma(va, s.h, Z[z]));
             }
         }
-        f32x4 part[2];                                   // gr without the state's part
+        f32x4 tx[2];                                     // gr's tile part
         {
             const bf16x8 rT = ld_tra<A::ROW>(xt + A::R), kT = ld_tra<A::ROW>(xt + A::K);
             const uint4 r4 = __builtin_bit_cast(uint4, rT), k4 = __builtin_bit_cast(uint4, kT);
-            f32x4 tx[2];
-            {
-                float pm[8];
-                Op2 ko[2];
-                from_ref(pm);
-                tile_operands(false, kT, pm, ko);
-                tx[0] = mm3(half_op<false>(tl + 2 * 3072), ko[0], ZERO4);
-                tx[1] = mm3(full_op(tl + 2 * 3072), ko[1], ZERO4);
-            }
             const float u = lds_f(sb + A::U + 64 * q + (at.tile >> 2 & 60u));
             Op2 ro[2];
             {
@@ -787,28 +795,33 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
                 else { tz = mm3(full_op(tl), ro[z], ZERO4); tw = mm3(full_op(tl + 3072), ro[z], ZERO4); }
                 const f32x4 vg4 = lds_ld<f32x4>(xs + A::VG + 64 * z);
                 const uint32_t rw[2] = {z ? r4.z : r4.x, z ? r4.w : r4.y}, kw[2] = {z ? k4.z : k4.x, z ? k4.w : k4.y};
-                const float th = at.t + static_cast<float>(16 * z), ba = hide(kb), bc = hide(cb);
-                const float pf[4] = {ba * o3, ba * o2, ba * o1, ba}, pc[4] = {bc, bc * o1, bc * o2, bc * o3};
+                const float th = at.t + static_cast<float>(16 * z), ba = hide(kb), be = ba * o8;
+                const float pf[4] = {ba * o3, ba * o2, ba * o1, ba}, pe[4] = {be * o3, be * o2, be * o1, be};
                 f32x4 o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const float r = v & 1 ? bf_hi(rw[v >> 1]) : bf_lo(rw[v >> 1]), k = v & 1 ? bf_hi(kw[v >> 1]) : bf_lo(kw[v >> 1]);
-                    float zs = Z[z][v] * (pf[v] * o8);
-                    if (z == 0) zs *= o16;
-                    const float vg = vg4[v], t = th + static_cast<float>(v), rv = r * vg;
-                    gw = fmaf(k, (31.f - t) * zs + tw[v] * pf[v], gw);
+                    const float zs = Z[z][v] * (z == 0 ? pe[v] * o16 : pe[v]), t = th + static_cast<float>(v), rv = r * vg4[v];
+                    gw = fmaf(k, fmaf(zs, 31.f - t, tw[v] * pf[v]), gw);
                     gu = fmaf(rv, k, gu);
                     o[v] = fmaf(rv, u, fmaf(tz[v], pf[v], zs));
-                    part[z][v] = fmaf(k * vg, u, tx[z][v] * pc[v]);
                 }
                 store_tile(gk_, at.out + 32 * z * C, C, static_cast<int>(at.tile >> 4), o);
+            }
+            {
+                float pm[8];
+                Op2 ko[2];
+                from_ref(pm);
+                tile_operands(false, kT, pm, ko);
+                tx[0] = mm3(half_op<false>(tl + 2 * 3072), ko[0], ZERO4);
+                tx[1] = mm3(full_op(tl + 2 * 3072), ko[1], ZERO4);
             }
         }
         f32x4 Sn[2][2];
         fetch_state(c, 0, at.state, Sn[0]);
         fetch_state(c, 1, at.state, Sn[1]);
         __syncthreads();                                 // the rows of the chunk before are there, the gradient state is handed over
-        second(odd_, c, part, Sn);
+        second(odd_, c, tx, Sn);
         __syncthreads();
     };
     __syncthreads();                                     // the top chunk is there
@@ -870,34 +883,29 @@ template <int HN> DEVINL void role_e(const ArgsW& p, lds_t sb, int te, const Par
     auto tile_b = [&](const int sl) __attribute__((always_inline)) {
         if (form < 0 || form > 2) return;
         const int lane = static_cast<int>(lane_now()), l16 = lane & 15, g = lane >> 4;
-        lds_t xr = sb + A::BASE + sl * A::SLOT + l16 * A::ROW + 16 * g;
+        lds_t xr = sb + A::BASE + sl * A::SLOT + l16 * A::ROW + 8 * g;
         opaque(xr);
         const lds_t out = sb + A::BTILE;
-        const bool transposed = form == 2;
-        const lds_t rows = xr + (transposed ? A::V : A::GY), cols = xr + (transposed ? A::GY : A::V);
-        const lds_t row1 = rows + (transposed ? 0 : 16 * A::ROW), col1 = cols + (transposed ? 16 * A::ROW : 0);       // (the quadrant across the halves)
         f32x4 t[3] = {ZERO4, ZERO4, ZERO4};
+        const auto products = [&](auto transposed_, const lds_t rows, const lds_t cols) __attribute__((always_inline)) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            t[0] = mfma(ld_op(rows + 64 * ks), ld_op(cols + 64 * ks), t[0]);
-            t[1] = mfma(ld_op(row1 + 64 * ks), ld_op(col1 + 64 * ks), t[1]);
-            t[2] = mfma(ld_op(rows + 16 * A::ROW + 64 * ks), ld_op(cols + 16 * A::ROW + 64 * ks), t[2]);
-        }
-        if (transposed) {
+            for (int ks = 0; ks < KS; ++ks) {
+                const bf16x8 a[2] = {ld_acc(rows + 64 * ks), ld_acc(rows + 16 * A::ROW + 64 * ks)}, b[2] = {ld_acc(cols + 64 * ks), ld_acc(cols + 16 * A::ROW + 64 * ks)};
+                using Q = Quad<decltype(transposed_)::value>;
+#pragma unroll
+                for (int z = 0; z < 3; ++z) t[z] = mfma(a[Q::ROWT[z]], b[Q::LANET[z]], t[z]);
+            }
+        };
+        if (form == 2) {
+            products(std::true_type{}, xr + A::V, xr + A::GY);
             mask<true>(t, l16, g);
-            put_tile<true>(out + 2 * 3072, t, lane);
+            put_tile<true, false>(out + 2 * 3072, t, lane);
             return;
         }
+        products(std::false_type{}, xr + A::GY, xr + A::V);
         mask<false>(t, l16, g);
-        if (form == 0) put_tile<false>(out, t, lane);
-        else {                                           // weighted with the tokens between, for the decay gradient
-            const float lag = static_cast<float>(4 * g - (l16 + 1));
-#pragma unroll
-            for (int z = 0; z < 3; ++z)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) t[z][v] *= lag + static_cast<float>(16 * (Quad<false>::ROWT[z] - Quad<false>::LANET[z]) + v);
-            put_tile<false>(out + 3072, t, lane);
-        }
+        if (form == 0) put_tile<false, false>(out, t, lane);
+        else put_tile<false, true>(out + 3072, t, lane, static_cast<float>(4 * g - (l16 + 1)));       // for the decay gradient
     };
     uint4 next[4];                                       // a chunk ahead of its way to LDS
     fetch(nch - 1, next);

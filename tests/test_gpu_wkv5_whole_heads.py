@@ -2,6 +2,8 @@
 oracle where it can go wrong: one token, whole chunks (32 tokens) and pairs of them (a saved state each) and one off, and decays
 of every strength: slow ones, some beyond what one reference token per chunk carries ("fast": up to the limit of one per half a
 chunk), and ones beyond that, whose heads run step by step ("mixed", "strong": nearly all heads).  The bar is that of the other bf16 kernels: no further from fp64 than fp32 arithmetic with rounded outputs."""
+import hashlib
+
 import pytest
 import torch
 
@@ -86,3 +88,26 @@ def test_wkv5_around_the_thresholds(lib, head, w1):
     emu = O.emulate_wkv5_bf16(B, T, C, H, r, k, v, w, u, gy)
     for name, a, e, g in zip(["y", "gr", "gk", "gv", "gw", "gu"], ref, emu, _run(B, T, C, H, r, k, v, w, u, gy)):
         assert_no_worse(name, a, e.reshape(a.shape), g.reshape(a.shape))
+
+
+# B, T, heads, head size, range of the raw decays -> the bits of y, gr, gk, gv, gw, gu (heads of 64: layers with a strong decay)
+BITS = {
+    (2, 300, 16, 128, -1.5, 0.5): "9e5d287c9604 c816c03755cf 9aefa4db7628 bbe91d845816 b423a4898c9d 278fcac95b29",
+    (3, 97, 20, 128, -1, 2.18): "287d8d19bd15 28c8d598c883 d8aeacb94e1d feaffe1c6659 36b35110b6e8 5905df063a65",
+    (4, 200, 24, 64, -2, 2.18): "bf0a6042268c a01564a7c684 7e1cda288c1c 3031bdeb0626 2e686ef0c88a b31c2582b0ee",
+}
+
+
+@pytest.mark.parametrize("case", BITS, ids=str)
+def test_the_order_of_the_sums_is_fixed(lib, case):
+    """Whole sequences have given these bits since the kernels were first written, whatever the split of the work among waves: every sum in its
+    order, the products of a split pair unrounded before their remainder is taken.  Inputs are multiples of 1/128 from integers, the same
+    on every machine."""
+    B, T, H, head, lo, hi = case
+    g = torch.Generator().manual_seed(T)
+    draw = lambda a, b, *s: (torch.randint(int(a * 128), int(b * 128) + 1, s, generator=g) / 128).to(torch.bfloat16)
+    C = H * head
+    r, k, v, gy = (draw(-1, 1, B, T, C) for _ in range(4))
+    got = _run(B, T, C, H, r, k, v, draw(lo, hi, H, head), draw(-0.5, 0.5, H, head), gy)
+    digest = lambda x: hashlib.sha256(x.detach().cpu().contiguous().view(torch.uint8).numpy().tobytes()).hexdigest()[:12]
+    assert [digest(x) for x in got] == BITS[case].split()
