@@ -998,13 +998,15 @@ template <bool TWO> int start_fwd(void* stream, int B, ArgsC& p, void* ws, size_
 hipError_t raise_lds(void (*kernel)(ArgsC), size_t bytes) {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
 }
-template <bool TWO> int start_bwd(void* stream, int B, ArgsC& p, void* ws, float* gw, float* gu, float* gw2, float* gu2) {
+// (a workspace that holds the rows of whole sequences and no more, which is all that it takes without blocks, is for whole sequences)
+template <bool TWO> int start_bwd(void* stream, int B, ArgsC& p, void* ws, size_t ws_bytes, float* gw, float* gu, float* gw2, float* gu2) {
+    if (ws == nullptr || ws_bytes < bwd_rows_bytes<TWO>(B, p.C, 1)) return RWKV_ERR_WORKSPACE;
     static_assert(sizeof(SmemB<TWO>) <= 160 * 1024, "the backward's LDS must fit one CU");
     static const hipError_t attr[2] = {raise_lds(wkv5c_bwd<TWO, false>, sizeof(SmemB<TWO>)), raise_lds(wkv5c_bwd<TWO, true>, sizeof(SmemB<TWO>))};
     for (const hipError_t e : attr) if (e != hipSuccess) { g_last_hip_error = static_cast<int>(e); return RWKV_ERR_LAUNCH; }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    int per;
-    const int NB = time_blocks<TWO>(B, p.T, p.H, true, &per);
+    int per = 0;
+    const int NB = ws_bytes < bwd_ws_bytes<TWO>(B, p.T, p.C, p.H) ? 1 : time_blocks<TWO>(B, p.T, p.H, true, &per);
     const size_t m = static_cast<size_t>(NB) * B * p.C;
     float* const rows = static_cast<float*>(ws);
     p.gw = rows; p.gu = rows + m;
@@ -1053,11 +1055,10 @@ int rwkv_wkv5f32s_backward(void* stream, int B, int T, int C, int H, const float
     if (int e = check_ptrs({r, k, v, u, gy, gr, gk, gv, gw, gu})) return e;
     if (int e = check_ptrs({w}, false)) return e;
     if (saved == nullptr || bytes < saved_bytes<false>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
-    if (workspace == nullptr || workspace_bytes < bwd_ws_bytes<false>(B, T, C, H)) return RWKV_ERR_WORKSPACE;
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv;
     p.saved = static_cast<float*>(const_cast<void*>(saved));
-    return start_bwd<false>(stream, B, p, workspace, gw, gu, nullptr, nullptr);
+    return start_bwd<false>(stream, B, p, workspace, workspace_bytes, gw, gu, nullptr, nullptr);
 }
 
 int rwkv_wkv5as_forward_ws(void* stream, int B, int T, int C, int H, const float* r, const float* k, const float* v, const float* w1,
@@ -1085,11 +1086,10 @@ int rwkv_wkv5as_backward(void* stream, int B, int T, int C, int H, const float* 
     if (int e = check_ptrs({r, k, v, u1, u2, gy, gr, gk, gv, gw1, gu1, gw2, gu2})) return e;
     if (int e = check_ptrs({w1, w2}, false)) return e;
     if (saved == nullptr || bytes < saved_bytes<true>(B, T, C, H) || !aligned16(saved)) return RWKV_ERR_WORKSPACE;
-    if (workspace == nullptr || workspace_bytes < bwd_ws_bytes<true>(B, T, C, H)) return RWKV_ERR_WORKSPACE;
     ArgsC p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w1; p.u = u1; p.w2 = w2; p.u2 = u2; p.gy = gy;
     p.gr = gr; p.gk = gk; p.gv = gv; p.saved = static_cast<float*>(const_cast<void*>(saved));
-    return start_bwd<true>(stream, B, p, workspace, gw1, gu1, gw2, gu2);
+    return start_bwd<true>(stream, B, p, workspace, workspace_bytes, gw1, gu1, gw2, gu2);
 }
 
 }  // extern "C"

@@ -89,6 +89,36 @@ def test_fp32_inputs_that_are_not_finite_are_the_step_kernels(lib, bad):
     assert bool(torch.isfinite(got[2][0, 391:]).all()) and bool(torch.isfinite(got[4].view(H, 64)[0]).all())
 
 
+def _f32_backward(lib, two, B, T, H, at):
+    """Both directions of wkv5 or wkv5a by the C entry points; at(bytes of the rows, bytes of everything) -> (address, bytes) of the backward's workspace."""
+    C, name = H * 64, "as" if two else "f32s"
+    (r, k, v), par, gy = _f32_inputs(B, T, H, 17 + T)
+    par = par if two else [x.view(C) for x in par[:2]]
+    ref = (A.grads if two else O.wkv5_grads)(B, T, C, H, r, k, v, *par, gy)
+    r, k, v, gy, *par = (x.to(DEV) for x in (r, k, v, gy, *par))
+    n = getattr(lib, f"rwkv_wkv5{name}_saved_bytes")(B, T, C, H)
+    saved, y, gr, gk, gv = garbage((n,), torch.uint8), *(garbage((B, T, C), torch.float32) for _ in range(4))
+    gpar = [garbage((C,), torch.float32) for _ in par]
+    call(f"rwkv_wkv5{name}_forward", y.device, B, T, C, H, r, k, v, *par, y, saved, n)
+    address, m = at(4 * len(par) * B * C, getattr(lib, f"rwkv_wkv5{name}_backward_workspace_bytes")(B, T, C, H))
+    call(f"rwkv_wkv5{name}_backward", y.device, B, T, C, H, r, k, v, *par, gy, gr, gk, gv, *gpar, saved, n, address, m)
+    _check(["y", "gr", "gk", "gv", "gw1", "gu1", "gw2", "gu2"], ref, [y, gr, gk, gv, *gpar])
+
+
+@pytest.mark.parametrize("two", [False, True])
+def test_fp32_backward_with_a_workspace_for_the_rows_only(lib, two):
+    """What the backward took before there were blocks of time: whole sequences are walked through, and nothing behind the rows is written."""
+    buffer = torch.full((1 << 16,), 7.5, device=DEV)
+
+    def at(rows, everything):
+        assert rows < everything and rows % 4 == 0, "not in blocks"
+        at.rows = rows
+        return buffer.data_ptr(), rows
+
+    _f32_backward(lib, two, 2, 400, 2, at)
+    assert bool((buffer[at.rows // 4:] == 7.5).all())
+
+
 def _rwkv7(B, T, H, dtype, seed):
     g = torch.Generator().manual_seed(seed)
     n = lambda *s: torch.randn(*s, generator=g)
