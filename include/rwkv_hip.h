@@ -263,8 +263,8 @@ int rwkv_wkv5a_backward_ex(void* stream, int B, int T, int C, int H,
  *   without a backward: 16 KB per head and 48 (wkv5a: 32) tokens, 721 MB (1.07 GB) at B8 T4096 C4096.  `workspace`
  *   (*_backward_workspace_bytes): per-batch rows of the parameter gradients and, for few sequences (B H <= 128 and at least 16 + B H / 4
  *   chunks of 16 tokens), what it takes to cut them into blocks of time that are worked on side by side; one that holds the rows only, 2
- *   (wkv5a: 4) B C floats, will do: whole sequences are walked through.  The forward cuts them with a workspace (*_forward_ws,
- *   *_forward_workspace_bytes; 0: none is needed).  The raw decays (w, w1, w2) may have any alignment.
+ *   (wkv5a: 4) B C floats, or that is not 16-byte aligned will do: whole sequences are walked through.  The forward cuts them with a
+ *   workspace (*_forward_ws, *_forward_workspace_bytes; 0: none is needed).  The raw decays (w, w1, w2) may have any alignment.
  *   Heads with a decay below e^-17 a step, a decay that is no number, or an input that is not finite run step by step.
  * ------------------------------------------------------------------------------------- */
 size_t rwkv_wkv5f32s_saved_bytes(int B, int T, int C, int H);

@@ -998,7 +998,8 @@ template <bool TWO> int start_fwd(void* stream, int B, ArgsC& p, void* ws, size_
 hipError_t raise_lds(void (*kernel)(ArgsC), size_t bytes) {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
 }
-// (a workspace that holds the rows of whole sequences and no more, which is all that it takes without blocks, is for whole sequences)
+// (a workspace that holds the rows of whole sequences and no more, or that the blocks' 16-byte accesses do not fit, is for whole sequences: they
+// take single floats)
 template <bool TWO> int start_bwd(void* stream, int B, ArgsC& p, void* ws, size_t ws_bytes, float* gw, float* gu, float* gw2, float* gu2) {
     if (ws == nullptr || ws_bytes < bwd_rows_bytes<TWO>(B, p.C, 1)) return RWKV_ERR_WORKSPACE;
     static_assert(sizeof(SmemB<TWO>) <= 160 * 1024, "the backward's LDS must fit one CU");
@@ -1006,7 +1007,7 @@ template <bool TWO> int start_bwd(void* stream, int B, ArgsC& p, void* ws, size_
     for (const hipError_t e : attr) if (e != hipSuccess) { g_last_hip_error = static_cast<int>(e); return RWKV_ERR_LAUNCH; }
     hipStream_t st = static_cast<hipStream_t>(stream);
     int per = 0;
-    const int NB = ws_bytes < bwd_ws_bytes<TWO>(B, p.T, p.C, p.H) ? 1 : time_blocks<TWO>(B, p.T, p.H, true, &per);
+    const int NB = ws_bytes < bwd_ws_bytes<TWO>(B, p.T, p.C, p.H) || !aligned16(ws) ? 1 : time_blocks<TWO>(B, p.T, p.H, true, &per);
     const size_t m = static_cast<size_t>(NB) * B * p.C;
     float* const rows = static_cast<float*>(ws);
     p.gw = rows; p.gu = rows + m;

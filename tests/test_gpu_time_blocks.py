@@ -119,6 +119,21 @@ def test_fp32_backward_with_a_workspace_for_the_rows_only(lib, two):
     assert bool((buffer[at.rows // 4:] == 7.5).all())
 
 
+@pytest.mark.parametrize("two", [False, True])
+def test_fp32_backward_with_a_workspace_at_any_float(lib, two):
+    """The blocks' states are stored and loaded 16 bytes at a time, the rows as single floats: a workspace of any alignment is taken as it
+    was before there were blocks, for whole sequences (nothing behind the rows is written)."""
+    buffer = torch.full((1 << 18,), 7.5, device=DEV)
+
+    def at(rows, everything):
+        assert rows < everything <= 4 * buffer.numel() - 4, "not in blocks"
+        at.rows = rows
+        return buffer.data_ptr() + 4, everything
+
+    _f32_backward(lib, two, 2, 400, 2, at)
+    assert float(buffer[0]) == 7.5 and bool((buffer[1 + at.rows // 4:] == 7.5).all())
+
+
 def _rwkv7(B, T, H, dtype, seed):
     g = torch.Generator().manual_seed(seed)
     n = lambda *s: torch.randn(*s, generator=g)
