@@ -151,8 +151,9 @@ int rwkv_timex_backward(void* stream, const float* w, const float* k, const floa
 int rwkv_timex_backward_sum(void* stream, const float* w, const float* k, const float* gwk,
                             float* gw_sum, float* gk, int B, int C, int T);
 /* The same for every shape the op takes (T % 4 == 0, T <= 4096, any B): `workspace` holds the kernel gradients of batch groups
- * that are worked on side by side, rwkv_timex_backward_ws_bytes() bytes (0 for many shapes: then NULL will do).  The order of
- * every fp32 sum is fixed here too. */
+ * that are worked on side by side, rwkv_timex_backward_ws_bytes() bytes (0 for many shapes: then NULL will do).  With room for
+ * fewer it takes fewer, as long as they fill the card (C >= 512: with NULL, too).  The order of every fp32 sum is fixed here too,
+ * for a shape and a number of groups. */
 size_t rwkv_timex_backward_ws_bytes(int B, int C, int T);
 int rwkv_timex_backward_ws(void* stream, const float* w, const float* k, const float* gwk,
                            float* gw_sum, float* gk, int B, int C, int T, void* workspace, size_t workspace_bytes);

@@ -1288,13 +1288,16 @@ GwGeom gw_any_geom(int B, int T) {
     }
     return best;
 }
+// Batch groups side by side (gw_short_geom's, whichever kernel takes them), as many as it takes for two workgroups per CU: those of timex_gw_short, and
+// the least that a workspace for timex_gw_any has to hold.
+int gw_group_parts(int B, int C, int T) {
+    const int bg = gw_short_geom(B, T).bg, ng = (B + bg - 1) / bg, want = (2 * NCU + C - 1) / C;
+    return ng < want ? ng : want;
+}
 // Parts of the batch that work side by side (their sums are added by a second kernel): what finishes first by a count of clocks, in rounds of
 // two workgroups per CU: 48 a row, step and lag tile, 3 a row and step of time for its conversion, a fixed cost a workgroup and that of the second kernel.
 int gw_any_parts(int B, int C, int T) {
-    if (T <= GW_SHORT) {               // (groups of rows side by side, as many as it takes for two workgroups per CU)
-        const int bg = gw_short_geom(B, T).bg, ng = (B + bg - 1) / bg, want = (2 * NCU + C - 1) / C;
-        return ng < want ? ng : want;
-    }
+    if (T <= GW_SHORT) return gw_group_parts(B, C, T);
     const int nt = (T + 31) / 32;
     long long row = 3LL * T;
     for (int s = 0; s < nt; s += 8) row += 48LL * (nt - s);
@@ -1402,8 +1405,11 @@ int rwkv_timex_backward_ws(void* stream, const float* w, const float* k, const f
     if (int e = check_tx(B, C, T)) return e;
     if (T % 32 == 0 && T <= T_MFMA_MAX) return rwkv_timex_backward_sum(stream, w, k, gwk, gw_sum, gk, B, C, T);
     if (int e = check_ptrs({w, k, gwk, gw_sum, gk})) return e;
-    const int parts = gw_any_parts(B, C, T);
-    if (parts > 1 && (workspace == nullptr || workspace_bytes < rwkv_timex_backward_ws_bytes(B, C, T) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+    // as many parts as there is room for (none in the workspace: one, in gw_sum itself), but the batch groups that fill the CUs at least
+    const int most = gw_any_parts(B, C, T), groups = gw_group_parts(B, C, T), least = groups < most ? groups : most;
+    const size_t room = workspace != nullptr && aligned16(workspace) ? workspace_bytes / (static_cast<size_t>(C) * T * sizeof(float)) : 0;
+    if (least > 1 && room < static_cast<size_t>(least)) return RWKV_ERR_WORKSPACE;
+    const int parts = room >= static_cast<size_t>(most) ? most : (room > 1 ? static_cast<int>(room) : 1);
     if (int e = launch_conv<true>(stream, w, gwk, gk, 0.0f, B, C, T)) return e;
     hipStream_t st = static_cast<hipStream_t>(stream);
     float* const to = parts > 1 ? static_cast<float*>(workspace) : gw_sum;

@@ -11,6 +11,7 @@ import torch
 from oracle import err_ratio, max_rel_to_peak
 from oracle import timex as OT
 from rwkv_cuda_amd import depthwise_conv1d, synth
+from rwkv_cuda_amd._call import call
 from _gpu_util import DEV
 
 pytestmark = pytest.mark.gpu
@@ -43,7 +44,6 @@ def test_more_batches(lib, B, C, T):
 
 
 def test_reference_signature_gives_per_batch_kernel_gradients(lib):
-    from rwkv_cuda_amd._call import call
     B, C, T = 3, 4, 76
     w, k, g = synth.timex_inputs(B, C, T, seed=9)
     d = [x.to(DEV) for x in (w, k, g)]
@@ -51,6 +51,40 @@ def test_reference_signature_gives_per_batch_kernel_gradients(lib):
     call("rwkv_timex_backward", d[0].device, *d, gw, gk, B, C, T)
     ref_gw, ref_gk = OT.grads_closed_form(*(x.double() for x in (w, k, g)), B, C, T)
     assert max_rel_to_peak(ref_gw, gw.double().cpu()) <= 1e-5 and max_rel_to_peak(ref_gk, gk.double().cpu()) <= 1e-5
+
+
+def _some_channels(B, C, T, seed, some):
+    """w, k, g on the GPU, and out, gw, gk of a few channels in 64 bits."""
+    w, k, g = synth.timex_inputs(B, C, T, seed=seed)
+    return [x.to(DEV) for x in (w, k, g)], OT.grads(w[some], k[:, some], g[:, some], B, len(some), T)
+
+
+def _backward_ws(w, k, g, B, C, T, ws, n):
+    gw, gk = torch.full((C, T), 1e9, device=DEV), torch.full((B, C, T), 1e9, device=DEV)
+    call("rwkv_timex_backward_ws", w.device, w, k, g, gw, gk, B, C, T, ws, n)
+    return gw, gk
+
+
+@pytest.mark.parametrize("B,C,T,parts", [(24, 600, 388, 0), (32, 768, 1500, 0), (13, 384, 1500, 2), (13, 64, 1500, 7)])
+def test_a_workspace_for_fewer_groups(lib, B, C, T, parts):
+    """What was enough when every lag tile had 32 lags (none at all for 512 channels and more) still is."""
+    part = 4 * C * T
+    assert lib.rwkv_timex_backward_ws_bytes(B, C, T) > max(parts, 1) * part
+    some = [0, C // 2, C - 1]
+    d, (_, gw, gk) = _some_channels(B, C, T, B + T, some)
+    ws = torch.full((parts * C * T + 1024,), 7.5, device=DEV)
+    got = _backward_ws(*d, B, C, T, ws if parts else None, parts * part)
+    assert max_rel_to_peak(gw, got[0][some].double().cpu()) <= 1e-5 and max_rel_to_peak(gk, got[1][:, some].double().cpu()) <= 1e-5
+    assert bool((ws[parts * C * T:] == 7.5).all())
+
+
+@pytest.mark.parametrize("B,C,T,parts", [(13, 384, 1500, 2), (13, 64, 1500, 7), (30, 200, 300, 2)])
+def test_a_workspace_for_too_few_groups_is_refused(lib, B, C, T, parts):
+    d = [x.to(DEV) for x in synth.timex_inputs(B, C, T, seed=1)]
+    ws = torch.empty(parts * C * T, device=DEV)
+    for w, n in ((ws, 4 * parts * C * T - 4), (None, 0), (ws.data_ptr() + 4, 4 * parts * C * T)):
+        with pytest.raises(RuntimeError):
+            _backward_ws(*d, B, C, T, w, n)
 
 
 def test_rows_of_very_different_size(lib):
