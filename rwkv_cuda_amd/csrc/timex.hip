@@ -640,7 +640,7 @@ static_assert(T_ANY / 32 < 255, "a block lag is a byte");
 // copies: of the taps' line.  With the second one, shifted by one, an odd window begins at a whole dword as an even one does; with one it is
 // five dwords, shifted in registers, which makes room for a second workgroup on a CU beyond T = 3360: B1 C1024 T4096 forward + backward 297 us
 // with two copies, 265 with one; T1500 with two 212, with one 216.
-struct ConvPlans { ConvPlan p[2]; int copies; };   // p: for units of ceil(B / groups) and of floor(B / groups) rows
+struct ConvPlans { ConvPlan p[2]; int copies, pairs; };   // p: for units of ceil(B / groups) and of floor(B / groups) rows; pairs: which kernel
 __host__ __device__ inline int tile_lags(const AnyGeom& q, bool mirror, int tile) {
     const int ncol = q.nt * q.bg, last = 32 * tile + 31 < ncol ? 32 * tile + 31 : ncol - 1;
     return mirror ? q.nt - over16(32 * tile, q.bg_inv) : over16(last, q.bg_inv) + 1;
@@ -768,7 +768,8 @@ DEVINL void zero_blocks(uint16_t* rp, const AnyGeom& q) {
     }
 }
 
-template <bool MIRROR, int COPIES>
+// PAIRS: as the plan says; without, every tile has a wave of its own, the longest four on the four SIMDs
+template <bool MIRROR, int COPIES, bool PAIRS>
 __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict__ w, const float* __restrict__ in, float* __restrict__ out,
                                                          float eps, int B, int C, int T, int ng, const ConvPlans plans) {
     extern __shared__ __align__(16) float lds[];
@@ -835,24 +836,26 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
         }
         __syncthreads();
     }
-    const uint64_t pairs = plan.pair;
-    const int pair = ConvPlan::of(pairs, wv), d0 = ConvPlan::of(plan.d0, wv), d1 = ConvPlan::of(plan.d1, wv);
+    constexpr int TILES = PAIRS ? 2 : 1;
+    const uint64_t pairs = PAIRS ? plan.pair : 0;
+    const int pair = PAIRS ? ConvPlan::of(pairs, wv) : (wv < 4 ? wv : 11 - wv);
     const int ncol = q.nt * q.bg, ntile = (ncol + 31) >> 5;
-    int tile[2], nd[2];
-    const uint16_t* bp[2];
+    int tile[TILES], nd[TILES];
+    const uint16_t* bp[TILES];
 #pragma unroll
-    for (int z = 0; z < 2; ++z) {
-        tile[z] = pair == NO_PAIR ? -1 : tile_of(ntile, MIRROR, 2 * pair + z);
+    for (int z = 0; z < TILES; ++z) {
+        tile[z] = PAIRS && pair == NO_PAIR ? -1 : tile_of(ntile, MIRROR, TILES * pair + z);
         nd[z] = tile[z] < 0 ? 0 : tile_lags(q, MIRROR, tile[z]);
         const int col = min(32 * max(tile[z], 0) + ln, ncol - 1), a = over16(col, q.bg_inv), b = col - a * q.bg;
         bp[z] = rp + (q.zb + b * q.pitch + a) * BLK + 8 * kh;
     }
+    const int d0 = PAIRS ? ConvPlan::of(plan.d0, wv) : 0, d1 = PAIRS ? ConvPlan::of(plan.d1, wv) : nd[0];
     const int start = (MIRROR ? 31 - ln : PZ + T - 1 - ln) + 8 * kh;    // forward: line[start - 32 d + j], mirror: line[start + 32 d + j]
     const uint32_t* ap = reinterpret_cast<const uint32_t*>(al + (COPIES == 2 ? start & 1 : 0) * xl) + (start >> 1);
     const uint32_t odd = 16 * (start & 1);
-    f32x16 acc[2], low[2];          // the products of the first terms, which are what rounds; the other five
+    f32x16 acc[TILES], low[TILES];  // the products of the first terms, which are what rounds; the other five
 #pragma unroll
-    for (int z = 0; z < 2; ++z)
+    for (int z = 0; z < TILES; ++z)
 #pragma unroll
         for (int v = 0; v < 16; ++v) { acc[z][v] = 0.f; low[z][v] = 0.f; }
     auto run = [&](auto NTL, const int from, const int to) __attribute__((always_inline)) {
@@ -883,38 +886,42 @@ __global__ __launch_bounds__(TXT, 4) void timex_conv_any(const float* __restrict
             }
         }
     };
-    run(std::integral_constant<int, 2>{}, d0, min(d1, nd[1]));
-    run(std::integral_constant<int, 1>{}, max(d0, nd[1]), d1);
-    // the sums of a pair's other waves, through the LDS that the rows no longer need
-    bool owner = pair != NO_PAIR;
-    for (int x = 0; x < wv; ++x) owner &= ConvPlan::of(pairs, x) != pair;
-    float4* const slot = reinterpret_cast<float4*>(lds);
-    constexpr int SLOT4 = SUM_SLOT / 4;
-    if (plan.shared) {
-        __syncthreads();
-        if (pair != NO_PAIR && !owner) {
+    if constexpr (PAIRS) {
+        run(std::integral_constant<int, 2>{}, d0, min(d1, nd[1]));
+        run(std::integral_constant<int, 1>{}, max(d0, nd[1]), d1);
+        // the sums of a pair's other waves, through the LDS that the rows no longer need
+        bool owner = pair != NO_PAIR;
+        for (int x = 0; x < wv; ++x) owner &= ConvPlan::of(pairs, x) != pair;
+        float4* const slot = reinterpret_cast<float4*>(lds);
+        constexpr int SLOT4 = SUM_SLOT / 4;
+        if (plan.shared) {
+            __syncthreads();
+            if (pair != NO_PAIR && !owner) {
+#pragma unroll
+                for (int z = 0; z < 2; ++z)
+#pragma unroll
+                    for (int v4 = 0; v4 < 4; ++v4)
+                        slot[wv * SLOT4 + (4 * z + v4) * 64 + lane] = make_float4(acc[z][4 * v4] + low[z][4 * v4], acc[z][4 * v4 + 1] + low[z][4 * v4 + 1],
+                                                                                 acc[z][4 * v4 + 2] + low[z][4 * v4 + 2], acc[z][4 * v4 + 3] + low[z][4 * v4 + 3]);
+            }
+            __syncthreads();
+        }
+        if (!owner) return;
+        for (int x = wv + 1; x < TXW; ++x) {
+            if (ConvPlan::of(pairs, x) != pair) continue;
 #pragma unroll
             for (int z = 0; z < 2; ++z)
 #pragma unroll
-                for (int v4 = 0; v4 < 4; ++v4)
-                    slot[wv * SLOT4 + (4 * z + v4) * 64 + lane] = make_float4(acc[z][4 * v4] + low[z][4 * v4], acc[z][4 * v4 + 1] + low[z][4 * v4 + 1],
-                                                                             acc[z][4 * v4 + 2] + low[z][4 * v4 + 2], acc[z][4 * v4 + 3] + low[z][4 * v4 + 3]);
+                for (int v4 = 0; v4 < 4; ++v4) {
+                    const float4 y = slot[x * SLOT4 + (4 * z + v4) * 64 + lane];
+                    acc[z][4 * v4] += y.x; acc[z][4 * v4 + 1] += y.y; acc[z][4 * v4 + 2] += y.z; acc[z][4 * v4 + 3] += y.w;
+                }
         }
-        __syncthreads();
-    }
-    if (!owner) return;
-    for (int x = wv + 1; x < TXW; ++x) {
-        if (ConvPlan::of(pairs, x) != pair) continue;
-#pragma unroll
-        for (int z = 0; z < 2; ++z)
-#pragma unroll
-            for (int v4 = 0; v4 < 4; ++v4) {
-                const float4 y = slot[x * SLOT4 + (4 * z + v4) * 64 + lane];
-                acc[z][4 * v4] += y.x; acc[z][4 * v4 + 1] += y.y; acc[z][4 * v4 + 2] += y.z; acc[z][4 * v4 + 3] += y.w;
-            }
+    } else {
+        run(std::integral_constant<int, 1>{}, d0, d1);
     }
 #pragma unroll
-    for (int z = 0; z < 2; ++z) {
+    for (int z = 0; z < TILES; ++z) {
         const int col = 32 * tile[z] + ln, a = over16(col, q.bg_inv), b = col - a * q.bg;
         if (tile[z] >= 0 && col < ncol) {
             float* o = out + (static_cast<size_t>(b0 + b) * C + c) * T;
@@ -1196,7 +1203,8 @@ __global__ __launch_bounds__(256) void timex_add_parts(const float4* __restrict_
 // steps (of a tile and a lag; so many take about what it takes to add two waves' sums), then the longest four runs go to the
 // four SIMDs (a wave w runs on SIMD w mod 4) and the others to the least loaded ones.
 constexpr int RUN_MIN = 4;
-void plan_waves(ConvPlan& p, bool mirror) {
+// returns how many more steps the longest tile has than the longest run, 0 at least; large: more tiles than waves
+int plan_waves(ConvPlan& p, bool mirror) {
     const int ntile = (p.q.nt * p.q.bg + 31) / 32, npair = (ntile + 1) / 2;
     int lags[TXW][2] = {}, runs[TXW] = {}, work[TXW] = {};
     for (int m = 0; m < npair; ++m) {
@@ -1233,10 +1241,17 @@ void plan_waves(ConvPlan& p, bool mirror) {
         p.d0 |= static_cast<uint64_t>(run[i].d0) << at;
         p.d1 |= static_cast<uint64_t>(run[i].d1) << at;
     }
+    return ntile > TXW ? 1 << 20 : std::max(0, tile_lags(p.q, mirror, tile_of(ntile, mirror, 0)) - run[0].work);
 }
 size_t conv_plan_lds(const ConvPlans& x) {
     return std::max({conv_any_lds(x.p[0].q, x.copies), conv_any_lds(x.p[1].q, x.copies), x.p[0].shared || x.p[1].shared ? TXW * SUM_SLOT * sizeof(float) : 0});
 }
+// A wave a tile is what short rows take (up to some 300 to 500 steps), where the longest tile has no more than so many steps over the longest run: an
+// instance without sums through LDS, without the plan's bytes and with the accumulators of one tile, in half the registers, so that four
+// workgroups share a CU.  Fewer steps where a CU has one workgroup at most, which waits for its longest wave.  A convolution, us, as runs / a
+// wave a tile: B16 C768 T132 11.3 / 8.3, B32 C1000 T60 10.8 / 7.9, B3 C768 T452 14.1 / 11.5; B6 C768 T772 (more than 11 steps) 25.0 / 26.5; few
+// workgroups: B1 C64 T260 (4 steps) 5.5 / 6.4.
+constexpr int TILE_STEPS = 11, TILE_STEPS_FEW = 3;
 // Batch rows of a unit, dealt evenly to `ng` units a channel.  What finishes first by a count of matrix clocks (96 per column tile and
 // block lag on a CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (a pair a wave) and
 // 80 KB.
@@ -1262,7 +1277,10 @@ ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
         const double c = static_cast<double>((static_cast<long long>(C) * groups + 2 * NCU - 1) / (2 * NCU)) * unit;
         if (c < cost) { cost = c; best = x; *ng = groups; }
     }
-    for (ConvPlan& p : best.p) plan_waves(p, mirror);
+    int longer = 0;
+    for (ConvPlan& p : best.p) longer = std::max(longer, plan_waves(p, mirror));
+    best.pairs = best.copies != 2 || longer > (static_cast<long long>(C) * *ng > 2 * NCU ? TILE_STEPS : TILE_STEPS_FEW);
+    if (!best.pairs) best.p[0].shared = best.p[1].shared = 0;
     return best;
 }
 // Up to here the kernel gradient takes lag tiles of 32 (timex_gw_short).  Lag tiles of 32 / of 256, the kernel alone: B32 C1000 T36 12.7 / 16.2 us,
@@ -1353,7 +1371,7 @@ template <bool MIRROR> int launch_conv(void* stream, const float* w, const float
         const ConvPlans plans = conv_any_plans(B, C, T, MIRROR, &ng);
         const size_t lds = conv_plan_lds(plans);
         if (static_cast<long long>(C) * ng > 0x7fffffffLL) return RWKV_ERR_SHAPE;
-        const auto kernel = plans.copies == 2 ? timex_conv_any<MIRROR, 2> : timex_conv_any<MIRROR, 1>;
+        const auto kernel = !plans.pairs ? timex_conv_any<MIRROR, 2, false> : (plans.copies == 2 ? timex_conv_any<MIRROR, 2, true> : timex_conv_any<MIRROR, 1, true>);
         if (int e = raise_lds_limit(kernel, lds)) return e;
         hipLaunchKernelGGL(kernel, dim3(C * ng), dim3(TXT), lds, st, w, in, out, eps, B, C, T, ng, plans);
     }

@@ -59,6 +59,18 @@ def _some_channels(B, C, T, seed, some):
     return [x.to(DEV) for x in (w, k, g)], OT.grads(w[some], k[:, some], g[:, some], B, len(some), T)
 
 
+@pytest.mark.parametrize("B,C,T", [(32, 520, 36), (16, 520, 132), (13, 1030, 68), (9, 520, 292), (3, 768, 388), (16, 520, 500), (5, 540, 452), (24, 600, 484)])
+def test_many_short_rows(lib, B, C, T):
+    """More workgroups than the card takes at a time, a wave a column tile (one tile to eight; units of unequal numbers of rows)."""
+    some = [0, C // 2, C - 1]
+    (w, k, g), ref = _some_channels(B, C, T, B + T, some)
+    w, k = w.requires_grad_(True), k.requires_grad_(True)
+    x = depthwise_conv1d.RUN_CUDA(w, k, B, C, T, 0.0)
+    gw, gk = torch.autograd.grad(x, (w, k), g)
+    for name, a, got in zip(("x", "gw", "gk"), ref, (x[:, some], gw[some], gk[:, some])):
+        assert max_rel_to_peak(a, got.detach().double().cpu()) <= 1e-5, name
+
+
 def _backward_ws(w, k, g, B, C, T, ws, n):
     gw, gk = torch.full((C, T), 1e9, device=DEV), torch.full((B, C, T), 1e9, device=DEV)
     call("rwkv_timex_backward_ws", w.device, w, k, g, gw, gk, B, C, T, ws, n)
