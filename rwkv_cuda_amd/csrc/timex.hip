@@ -592,7 +592,7 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // work), 77 us the kernel gradient (107 as lag tiles of 32), relative errors 1.8e-7 and 1.0e-7; the fp32 loops on the vector units
 // that these replace took 315 / 286 and, with the sum over the batch, 243 us, with 5.6e-7.
 constexpr int BLK = 40;                // elements of a block in LDS, 32 of them data
-constexpr int LDS_ANY = 80 * 1024;     // two workgroups per CU
+constexpr int LDS_CU = 160 * 1024, LDS_ANY = LDS_CU / 2;     // two workgroups per CU
 constexpr int PZ = 32;                 // zeros in front of the forward line (lags beyond the last tap, of rows past T)
 constexpr int CONV_PIECES = 8, GW_PIECES = 3;   // 16-byte pieces a thread stages (per tensor): Bg nt 8 / 512 at most
 constexpr int NPL = 3;                 // planes: terms of an operand
@@ -1246,15 +1246,18 @@ int plan_waves(ConvPlan& p, bool mirror) {
 size_t conv_plan_lds(const ConvPlans& x) {
     return std::max({conv_any_lds(x.p[0].q, x.copies), conv_any_lds(x.p[1].q, x.copies), x.p[0].shared || x.p[1].shared ? TXW * SUM_SLOT * sizeof(float) : 0});
 }
-// A wave a tile is what short rows take (up to some 300 to 500 steps), where the longest tile has no more than so many steps over the longest run: an
-// instance without sums through LDS, without the plan's bytes and with the accumulators of one tile, in half the registers, so that four
-// workgroups share a CU.  Fewer steps where a CU has one workgroup at most, which waits for its longest wave.  A convolution, us, as runs / a
-// wave a tile: B16 C768 T132 11.3 / 8.3, B32 C1000 T60 10.8 / 7.9, B3 C768 T452 14.1 / 11.5; B6 C768 T772 (more than 11 steps) 25.0 / 26.5; few
-// workgroups: B1 C64 T260 (4 steps) 5.5 / 6.4.
-constexpr int TILE_STEPS = 11, TILE_STEPS_FEW = 3;
+// A wave a tile is what short rows take, up to SHORT_ROWS steps, where the longest tile has no more than so many steps over the longest run: an
+// instance without sums through LDS, without the plan's bytes and with the accumulators of one tile, in half the registers, so that three or four
+// workgroups share a CU; fewer steps where the rows' LDS has room for two only, and where a CU has one workgroup at most, which waits for its
+// longest wave.  A convolution, us, as runs / a wave a tile: B16 C768 T132 11.3 / 8.3, B32 C1000 T60 10.8 / 7.9, B3 C768 T452 14.1 / 11.5, B4 C1000 T484
+// (12 steps) 17.0 / 13.2, B3 C640 T644 (17) 14.9 / 12.5; two by LDS: B10 C640 T580 (8) 21.7 / 22.7; few workgroups: B1 C64 T260 (4) 5.5 / 6.4.
+constexpr int TILE_STEPS = 16, TILE_STEPS_FULL = 5, TILE_STEPS_FEW = 3;
+constexpr int SHORT_ROWS = 672;        // (B13 C300 T772 25.2 / 26.6)
 // Batch rows of a unit, dealt evenly to `ng` units a channel.  What finishes first by a count of matrix clocks (96 per column tile and
 // block lag on a CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (a pair a wave) and
-// 80 KB.
+// 80 KB.  Units of two sizes count by their mean, but in the last round, up to SHORT_ROWS steps, by the larger: B3 C200 T516 as 2 + 1 rows, one round,
+// 9.9 us, as 1 + 1 + 1, two rounds of half the time, 8.5; B5 C768 T516 21.2 / 17.1.  Longer rows' units take turns of their own: B19 C400 T1060
+// 61 us by the mean, 71 so.
 ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
     ConvPlans best{};
     double cost = 1e300;
@@ -1262,7 +1265,7 @@ ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
         const int groups = (B + most - 1) / most, rows[2] = {(B + groups - 1) / groups, B / groups};
         if (rows[0] != most) continue;
         ConvPlans x{};
-        double unit = 0;
+        double unit = 0, largest = 0;
         for (int z = 0; z < 2; ++z) {
             x.p[z].q = any_geom(T, rows[z], 31);
             const int ntile = (x.p[z].q.nt * rows[z] + 31) / 32;
@@ -1270,16 +1273,19 @@ ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
             const int share = z == 1 ? groups - B % groups : B % groups;
             long long steps = 0;
             for (int t = 0; t < ntile; ++t) steps += tile_lags(x.p[z].q, mirror, t);
-            unit += (96.0 * steps + 0.15 * rows[z] * T + 3000.0) * share / groups;
+            const double one = 96.0 * steps + 0.15 * rows[z] * T + 3000.0;
+            if (z == 0) largest = one;
+            unit += one * share / groups;
         }
         x.copies = most == 1 && conv_any_lds(x.p[0].q, 2) > LDS_ANY ? 1 : 2;
         if (unit < 0 || conv_plan_lds(x) > LDS_ANY || 8 * x.p[0].q.nt * rows[0] > CONV_PIECES * TXT) { if (most > 1) break; }
-        const double c = static_cast<double>((static_cast<long long>(C) * groups + 2 * NCU - 1) / (2 * NCU)) * unit;
+        const double c = static_cast<double>((static_cast<long long>(C) * groups - 1) / (2 * NCU)) * unit + (T <= SHORT_ROWS ? largest : unit);
         if (c < cost) { cost = c; best = x; *ng = groups; }
     }
     int longer = 0;
     for (ConvPlan& p : best.p) longer = std::max(longer, plan_waves(p, mirror));
-    best.pairs = best.copies != 2 || longer > (static_cast<long long>(C) * *ng > 2 * NCU ? TILE_STEPS : TILE_STEPS_FEW);
+    const bool room = 3 * std::max(conv_any_lds(best.p[0].q, best.copies), conv_any_lds(best.p[1].q, best.copies)) <= LDS_CU;
+    best.pairs = T > SHORT_ROWS || longer > (static_cast<long long>(C) * *ng <= 2 * NCU ? TILE_STEPS_FEW : (room ? TILE_STEPS : TILE_STEPS_FULL));
     if (!best.pairs) best.p[0].shared = best.p[1].shared = 0;
     return best;
 }
