@@ -952,7 +952,7 @@ DEVINL void add_diagonals(float* diag, const f32x16& acc, int d, int ln, int kh)
     else if (ln >= 1) diag[64 * d + ln - 1] += neg;
 }
 
-// The kernel gradient of short rows (T <= GW_SHORT), where a tile of 256 lags is mostly empty: lag tiles of 32, M_d of columns (block, row) as in
+// The kernel gradient of short rows, where a tile of 256 lags is mostly empty (gw_plan): lag tiles of 32, M_d of columns (block, row) as in
 // the convolution.  One workgroup: channel c = blockIdx.x, batch groups blockIdx.y, blockIdx.y + gridDim.y, ...; out[blockIdx.y][c][T]
 __global__ __launch_bounds__(TXT, 4) void timex_gw_short(const float* __restrict__ k, const float* __restrict__ g, float* __restrict__ out,
                                                        int B, int C, int T, int ng, const AnyGeom q) {
@@ -1289,9 +1289,6 @@ ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
     if (!best.pairs) best.p[0].shared = best.p[1].shared = 0;
     return best;
 }
-// Up to here the kernel gradient takes lag tiles of 32 (timex_gw_short).  Lag tiles of 32 / of 256, the kernel alone: B32 C1000 T36 12.7 / 16.2 us,
-// B20 C700 T260 27.6 / 27.7 (forward + backward 59.9 / 62.1), B30 C200 T516 29.6 / 27.3, B13 C384 T1500 107 / 77.
-constexpr int GW_SHORT = 384;
 inline size_t gw_short_lds(const AnyGeom& q) { return 2 * NPL * q.plane() * 2 + static_cast<size_t>(q.nt) * 256 + 16; }
 AnyGeom gw_short_geom(int B, int T) {
     AnyGeom best = any_geom(T, 1, 15);
@@ -1312,24 +1309,55 @@ GwGeom gw_any_geom(int B, int T) {
     }
     return best;
 }
-// Batch groups side by side (gw_short_geom's, whichever kernel takes them), as many as it takes for two workgroups per CU: those of timex_gw_short, and
-// the least that a workspace for timex_gw_any has to hold.
+// What the kernel gradient does: lag tiles of 32 (timex_gw_short) or of 256, and how many parts of the batch side by side (their sums are added
+// by a second kernel).
+struct GwPlan { bool narrow; int parts; };
+// Batch groups of timex_gw_short side by side: as many as it takes for two workgroups per CU.
 int gw_group_parts(int B, int C, int T) {
     const int bg = gw_short_geom(B, T).bg, ng = (B + bg - 1) / bg, want = (2 * NCU + C - 1) / C;
     return ng < want ? ng : want;
 }
-// Parts of the batch that work side by side (their sums are added by a second kernel): what finishes first by a count of clocks, in rounds of
-// two workgroups per CU: 48 a row, step and lag tile, 3 a row and step of time for its conversion, a fixed cost a workgroup and that of the second kernel.
-int gw_any_parts(int B, int C, int T) {
-    if (T <= GW_SHORT) return gw_group_parts(B, C, T);
+int gw_most_parts(int B, int C) { return std::max(1, std::min(B, 8 * NCU / C)); }
+// Parts for timex_gw_any by a count of clocks, in rounds of two workgroups per CU: 48 a row, step and lag tile, 3 a row and step of time for its
+// conversion, a fixed cost a workgroup and that of the second kernel.
+int gw_clock_parts(int B, int C, int T) {
     const int nt = (T + 31) / 32;
     long long row = 3LL * T;
     for (int s = 0; s < nt; s += 8) row += 48LL * (nt - s);
     int best = 1;
     long long cost = -1;
-    for (int p = 1; p <= B && (p == 1 || static_cast<long long>(C) * p <= 8 * NCU); ++p) {
+    for (int p = 1; p <= gw_most_parts(B, C); ++p) {
         const long long x = (static_cast<long long>(C) * p + 2 * NCU - 1) / (2 * NCU) * (12000 + row * B / p) + (p > 1 ? 10000 : 0);
         if (cost < 0 || x < cost) { cost = x; best = p; }
+    }
+    return best;
+}
+// Up to GW_SHORT steps lag tiles of 32, a tile of 256 being mostly empty: the kernel alone, 32 / 256, B32 C1000 T36 12.7 / 16.2 us, B20 C700 T260 27.6 /
+// 27.7.  Up to GW_MIDDLE what takes less by the formulas below, us fitted to 5400 timings of both with one to sixteen parts (B2 to B32, C64 to
+// C1000, T388 to T708; they are off by 4 % rms): timex_gw_short's whole groups of rows, of which one or two fit a small batch, and its fewer
+// workgroups against timex_gw_any's parts.  Backward, 32 / 256 with the formula's parts / with those by clocks: B24 C300 T484 46.3 / 48.0 / 52.2 us, B8
+// C200 T484 17.7 / 19.2 / 20.2, B20 C1000 T388 74.0 / 79.6 / 80.1, B12 C768 T452 53.5 / 48.3 / 48.1.  Up to GW_FITTED, where the timings end, the parts
+// are the formula's, too (B6 C200 T644 23.0 -> 21.7); beyond, by clocks (B7 C300 T1500 74 us, 81 by the formula).
+constexpr int GW_SHORT = 384, GW_MIDDLE = 512, GW_FITTED = 708;
+GwPlan gw_plan(int B, int C, int T) {
+    const int groups = gw_group_parts(B, C, T);
+    if (T <= GW_SHORT) return {true, groups};
+    if (T > GW_FITTED) return {false, gw_clock_parts(B, C, T)};
+    const auto over = [](long long x, long long d) { return static_cast<double>((x + d - 1) / d); };
+    const int nt = (T + 31) / 32, bg = gw_any_geom(B, T).bg;
+    double steps = 0, cost = 1e300;
+    for (int s = 0; s < nt; s += 8) steps += nt - s;
+    GwPlan best{false, 1};
+    for (int p = 1; p <= gw_most_parts(B, C); ++p) {
+        const long long w = static_cast<long long>(C) * p, rows = (B + p - 1) / p;
+        const double x = 1.41 * over(w, 2 * NCU) * over(rows, bg) + rows * steps * (0.0141 * over(w, NCU) + 0.011 * over(w, 2 * NCU)) + (p > 1 ? 1.13 + 5.2e-6 * w * T : 0.0);
+        if (x < cost) { cost = x; best.parts = p; }
+    }
+    if (T <= GW_MIDDLE) {
+        const int rows = gw_short_geom(B, T).bg;
+        const long long w = static_cast<long long>(C) * groups;
+        const double per = over(over(B, rows), groups);
+        if (over(w, 2 * NCU) * (0.55 + 1.61 * per) + 0.00144 * over(w, NCU) * per * rows * nt * nt + (groups > 1 ? 0.95 : 0.0) < cost) return {true, groups};
     }
     return best;
 }
@@ -1420,7 +1448,7 @@ int rwkv_timex_backward_sum(void* stream, const float* w, const float* k, const 
 
 size_t rwkv_timex_backward_ws_bytes(int B, int C, int T) {
     if (check_tx(B, C, T) != RWKV_OK || (T % 32 == 0 && T <= T_MFMA_MAX)) return 0;
-    const int parts = gw_any_parts(B, C, T);
+    const int parts = gw_plan(B, C, T).parts;
     return parts <= 1 ? 0 : static_cast<size_t>(parts) * C * T * sizeof(float);
 }
 
@@ -1429,15 +1457,18 @@ int rwkv_timex_backward_ws(void* stream, const float* w, const float* k, const f
     if (int e = check_tx(B, C, T)) return e;
     if (T % 32 == 0 && T <= T_MFMA_MAX) return rwkv_timex_backward_sum(stream, w, k, gwk, gw_sum, gk, B, C, T);
     if (int e = check_ptrs({w, k, gwk, gw_sum, gk})) return e;
-    // as many parts as there is room for (none in the workspace: one, in gw_sum itself), but the batch groups that fill the CUs at least
-    const int most = gw_any_parts(B, C, T), groups = gw_group_parts(B, C, T), least = groups < most ? groups : most;
+    // a workspace with room for fewer parts is for timex_gw_any, which takes any number of them (without room: one, in gw_sum itself); too few to
+    // fill the card, as all rules for their number have it, are refused
+    GwPlan plan = gw_plan(B, C, T);
+    const int groups = gw_group_parts(B, C, T), least = T <= GW_SHORT ? groups : std::min({plan.parts, groups, gw_clock_parts(B, C, T)});
     const size_t room = workspace != nullptr && aligned16(workspace) ? workspace_bytes / (static_cast<size_t>(C) * T * sizeof(float)) : 0;
     if (least > 1 && room < static_cast<size_t>(least)) return RWKV_ERR_WORKSPACE;
-    const int parts = room >= static_cast<size_t>(most) ? most : (room > 1 ? static_cast<int>(room) : 1);
+    if (plan.parts > 1 && room < static_cast<size_t>(plan.parts)) plan = {false, room > 1 ? static_cast<int>(room) : 1};
+    const int parts = plan.parts;
     if (int e = launch_conv<true>(stream, w, gwk, gk, 0.0f, B, C, T)) return e;
     hipStream_t st = static_cast<hipStream_t>(stream);
     float* const to = parts > 1 ? static_cast<float*>(workspace) : gw_sum;
-    if (T <= GW_SHORT) {
+    if (plan.narrow) {
         const AnyGeom q = gw_short_geom(B, T);
         const size_t lds = gw_short_lds(q);
         if (int e = raise_lds_limit(timex_gw_short, lds)) return e;

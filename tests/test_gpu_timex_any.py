@@ -71,6 +71,16 @@ def test_many_short_rows(lib, B, C, T):
         assert max_rel_to_peak(a, got.detach().double().cpu()) <= 1e-5, name
 
 
+@pytest.mark.parametrize("B,C,T", [(24, 300, 508), (27, 300, 452), (12, 768, 452), (32, 64, 512 + 4), (6, 200, 644), (16, 64, 708), (16, 64, 712)])
+def test_kernel_gradients_of_middle_lengths(lib, B, C, T):
+    """Lag tiles of 32 or of 256, and as many parts of the batch, as take less time: either side of the lengths where the rule changes."""
+    some = [0, C // 2, C - 1]
+    (w, k, g), ref = _some_channels(B, C, T, B + T, some)
+    n = lib.rwkv_timex_backward_ws_bytes(B, C, T)
+    gw, gk = _backward_ws(w, k, g, B, C, T, torch.empty(max(n, 16), dtype=torch.uint8, device=DEV), n)
+    assert max_rel_to_peak(ref[1], gw[some].double().cpu()) <= 1e-5 and max_rel_to_peak(ref[2], gk[:, some].double().cpu()) <= 1e-5
+
+
 def _backward_ws(w, k, g, B, C, T, ws, n):
     gw, gk = torch.full((C, T), 1e9, device=DEV), torch.full((B, C, T), 1e9, device=DEV)
     call("rwkv_timex_backward_ws", w.device, w, k, g, gw, gk, B, C, T, ws, n)
