@@ -326,7 +326,7 @@ struct SmemF {
 };
 constexpr int FDEPTH = 4;
 
-template <bool TWO, bool STRONG>
+template <bool TWO, bool STRONG, bool CUT>
 DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, const Part<TWO>& part) {
     const int l16 = lane & 15, g = lane >> 4, T = part.left, C = p.C, nch = part.chunks;
     const size_t base = part.base;
@@ -362,10 +362,11 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, const Part<T
         }
     }
     F4 c2s = {}, c2m = {}, c2k = {}, c2e = {};
-    float u2 = 0.f;
+    float u2 = 0.f, d2 = 1.f, w24 = 1.f;
     if constexpr (TWO) {
         const float l = S.hd.lam2[own];
         u2 = S.hd.u2[own];
+        if constexpr (!CUT) { d2 = S.hd.dec2[own]; w24 = wpow(l, 4.f); }       // (with blocks of time anew in every chunk: the registers do not reach)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int t = 4 * g + v, m = ref<STRONG>(t);
@@ -418,7 +419,7 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, const Part<T
         const f32x4 ruk = ld4(&X.ruk[4 * g]);
         f32x4 y = y2[0] + y2[1];
         if constexpr (TWO) {
-            const f32x4 ap = apply<STRONG>(at, vop * c2k, l16 >= 8 && g < 2, STRONG ? wpow(S.hd.lam2[own], 4.f) : 1.f);      // (anew: a register less across the loop)
+            const f32x4 ap = apply<STRONG>(at, vop * c2k, l16 >= 8 && g < 2, STRONG && CUT ? wpow(S.hd.lam2[own], 4.f) : w24);
             y = y * c2s + ap * c2m + vop * (ruk + u2 * ld4(&X.rk[4 * g]));
         } else {
             y += vop * ruk;
@@ -428,7 +429,7 @@ DEVINL void fwd_products(SmemF& S, const ArgsC& p, int q, int lane, const Part<T
         float* const out = p.y + base + static_cast<size_t>(c) * L * C;
         store_rows(out, lo, C, T - c * L - 4 * g, c * L + L <= T, y);
         const f32x4 ve = TWO ? vop * c2e : vop;
-        const float d2 = TWO ? S.hd.dec2[own] : 1.f;     // (likewise)
+        if constexpr (TWO && CUT) d2 = S.hd.dec2[own];
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
             f32x4 acc = St[jt] * ld4(&S.hd.dec[16 * jt + 4 * g]);
@@ -497,8 +498,8 @@ __global__ __launch_bounds__(NT, 4) void wkv5c_fwd(const ArgsC args) {
         }
         return;
     }
-    if (strong) fwd_products<TWO, true>(S, p, q, lane, part);
-    else fwd_products<TWO, false>(S, p, q, lane, part);
+    if (strong) fwd_products<TWO, true, CUT>(S, p, q, lane, part);
+    else fwd_products<TWO, false, CUT>(S, p, q, lane, part);
 }
 
 // ---------------------------------------------------------------------------------------------------- backward
