@@ -109,6 +109,76 @@ def test_a_workspace_for_too_few_groups_is_refused(lib, B, C, T, parts):
             _backward_ws(*d, B, C, T, w, n)
 
 
+def _rows_at_a_time(B, T, narrow):
+    """How many batch rows a workgroup of the kernel gradient has in LDS at a time (gw_short_geom, gw_any_geom of timex.hip)."""
+    nt, best = (T + 31) // 32, 1
+    for bg in range(2, min(B, 32) + 1):
+        if narrow:                      # three planes each of g and k in blocks of 40 elements, zero blocks between the rows, and the diagonals' sums
+            zb = -(-15 // bg)
+            zb += (nt + zb + 1) & 1
+            size = 2 * 3 * (zb + bg * (nt + zb)) * 40 * 2 + 256 * nt + 16
+        else:                           # three planes of g in blocks of 144 and of k; the eight waves' sums
+            size = max(bg * 3 * (144 * ((nt + 3) // 4 + 1) + 32 * nt) * 2 + 16, 8 * 1024 * min(-(-T // 256), 8))
+        if size > 80 * 1024 or 8 * nt * bg > 3 * 512:
+            break
+        best = bg
+    return best
+
+
+# B, T -> groups of rows that one workgroup takes one after the other, where the whole batch is its part (512 channels and more, no workspace)
+GROUPS = {(13, 1500): 4, (9, 1500): 3, (13, 712): 2, (16, 1000): 4, (5, 2052): 3, (7, 4092): 7, (31, 516): 4, (33, 260): 3, (40, 384): 4, (64, 68): 2}
+
+
+def _one_part(lib, B, T, monkey=None):
+    """w, k, g of 512 channels, of which the rows of 0, 200 and 511 may be changed by `monkey`, and both sides' gradients of these."""
+    C, some = 512, [0, 200, 511]
+    at_a_time = _rows_at_a_time(B, T, T <= 384)
+    assert -(-B // at_a_time) == GROUPS[B, T]
+    w, k, g = synth.timex_inputs(B, C, T, seed=B + T)
+    if monkey is not None:
+        monkey(k, g)
+    ref = OT.grads(w[some], k[:, some], g[:, some], B, 3, T)
+    w, k, g = (x.to(DEV) for x in (w, k, g))
+    gw, gk = _backward_ws(w, k, g, B, C, T, None, 0)
+    return ref[1], gw[some].double().cpu(), ref[2], gk[:, some].double().cpu(), at_a_time
+
+
+@pytest.mark.parametrize("B,T", list(GROUPS))
+def test_groups_of_rows_one_after_the_other(lib, B, T):
+    """Sums that are kept over groups, the next group's rows loaded under the products, a last group of fewer rows."""
+    gw, got_gw, gk, got_gk, _ = _one_part(lib, B, T)
+    assert max_rel_to_peak(gw, got_gw) <= 1e-5 and max_rel_to_peak(gk, got_gk) <= 1e-5
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3.4e38])
+@pytest.mark.parametrize("where", ["first", "middle", "first and last"])
+@pytest.mark.parametrize("B,T", [(13, 1500), (9, 1500), (33, 260)])
+def test_groups_with_an_element_that_terms_do_not_carry(lib, B, T, where, bad):
+    """A group that is done by the fp32 loop before, between or after groups on the matrix cores: their sums add up, and lags that the
+    element does not act on are finite.  3.4e38 is a number that three bf16 terms do not carry: nothing is lost."""
+    rows = {"first": [1], "middle": [B // 2], "first and last": [0, B - 1]}[where]
+    t0 = T - T // 3
+
+    def put(k, g):
+        g.clamp_(-0.9 / len(rows), 0.9 / len(rows))         # (the products add up to no more than fp32's largest)
+        for i, b in enumerate(rows):
+            k[b, 0, t0 + 2 * i] = bad
+
+    gw, got, _, _, bg = _one_part(lib, B, T, put)
+    groups = -(-B // bg)
+    even = bg if T <= 384 else -(-B // groups)
+    assert len({b // even for b in rows}) == len(rows) and (where != "middle" or 0 < rows[0] // even < groups - 1)
+    lag = torch.arange(T - 1, -1, -1)
+    hit = lag <= T - 1 - t0                                 # of channel 0
+    if bad != 3.4e38:
+        assert torch.equal(~torch.isfinite(got[0]), hit)
+        assert max_rel_to_peak(gw[0][~hit], got[0][~hit]) <= 1e-5
+    else:
+        for z in (hit, ~hit):
+            assert max_rel_to_peak(gw[0][z], got[0][z]) <= 1e-5
+    assert max_rel_to_peak(gw[1:], got[1:]) <= 1e-5
+
+
 def test_rows_of_very_different_size(lib):
     """The rows of a unit do not meet."""
     B, C, T = 6, 2, 500
