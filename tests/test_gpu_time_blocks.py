@@ -77,7 +77,7 @@ def test_fp32_inputs_that_are_not_finite_are_the_step_kernels(lib, bad):
     assert torch.equal(whole[..., 64:128].nan_to_num(7.0), blocks[..., 64:128].nan_to_num(7.0))
     assert torch.equal(blocks[..., :64], clean[..., :64]) and torch.equal(blocks[..., 128:], clean[..., 128:])
     assert bool(torch.isfinite(blocks[0, :390]).all()) and not bool(torch.isfinite(blocks[0, 390, 64:128]).all()) and bool(torch.isfinite(clean).all())
-    # and backwards: the gradients of the other heads are untouched, those of this one are the step kernels'
+    # and backwards: the gradients of the other heads are untouched (those of this one: the test below)
     t = [z.clone().requires_grad_(True) for z in (r, k, v, w.view(C), u.view(C))]
     good = torch.autograd.grad(wkv5.RUN_CUDA(B, T, C, H, *t), t, gy)
     with torch.no_grad():
@@ -87,6 +87,48 @@ def test_fp32_inputs_that_are_not_finite_are_the_step_kernels(lib, bad):
         for h in (0, 2):
             assert torch.equal(a[..., 64 * h:64 * h + 64], b[..., 64 * h:64 * h + 64])
     assert bool(torch.isfinite(got[2][0, 391:]).all()) and bool(torch.isfinite(got[4].view(H, 64)[0]).all())
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("which", ["r", "k", "v", "gy"])
+@pytest.mark.parametrize("t", [5, 200, 391])                # in the first, a middle and the last block
+@pytest.mark.parametrize("two", [False, True])
+def test_fp32_head_with_an_input_that_is_not_finite(lib, two, t, which, bad):
+    """wkv5, wkv5a, both directions: whatever block such an input is in, the head's outputs and gradients, those of its parameters among them, are
+    the bits of a call without blocks, where the step kernels do the head; the other heads' are those of a call without that input."""
+    B, H, T, name = 2, 3, 400, "as" if two else "f32s"
+    C = H * 64
+    x, par, gy = _f32_inputs(B, T, H, 11 + t)
+    par = par if two else [z.view(C) for z in par[:2]]
+    clean = [z.to(DEV) for z in (*x, gy)]
+    par = [z.to(DEV) for z in par]
+    spoilt = [z.clone() for z in clean]
+    spoilt[["r", "k", "v", "gy"].index(which)][1, t, 64 + 7] = bad
+    size = lambda what: getattr(lib, f"rwkv_wkv5{name}_{what}_bytes")(B, T, C, H)
+
+    def run(ins, blocks):
+        r, k, v, gy = ins
+        saved, y, gr, gk, gv = garbage((size("saved"),), torch.uint8), *(garbage((B, T, C), torch.float32) for _ in range(4))
+        gpar = [garbage((C,), torch.float32) for _ in par]
+        n, m = (size("forward_workspace"), size("backward_workspace")) if blocks else (0, 4 * len(par) * B * C)
+        assert not blocks or n > 0 and m > 4 * len(par) * B * C, "not in blocks"
+        call(f"rwkv_wkv5{name}_forward_ws", y.device, B, T, C, H, r, k, v, *par, y, saved, saved.numel(), garbage((n,), torch.uint8) if n else None, n)
+        call(f"rwkv_wkv5{name}_backward", y.device, B, T, C, H, r, k, v, *par, gy, gr, gk, gv, *gpar, saved, saved.numel(), garbage((m,), torch.uint8), m)
+        return [z.view(B, T, H, 64) for z in (y, gr, gk, gv)], [z.view(H, 64) for z in gpar]
+
+    (a, pa), (b, pb), (c, pc) = run(spoilt, False), run(spoilt, True), run(clean, True)
+    same = lambda p, q: torch.equal(p.nan_to_num(7.0, 8.0, 9.0), q.nan_to_num(7.0, 8.0, 9.0))
+    for i, (whole, blocks, good) in enumerate(zip(a, b, c)):
+        hit = i > 0 or which != "gy"                        # (gy is none of the forward's inputs: that head is in blocks there)
+        assert same(whole[1, :, 1], blocks[1, :, 1]) if hit else torch.equal(good[1, :, 1], blocks[1, :, 1]), i
+        assert torch.equal(blocks[0], good[0]) and torch.equal(blocks[1, :, [0, 2]], good[1, :, [0, 2]]), i
+    assert not all(bool(z[1, :, 1].isfinite().all()) for z in b)
+    # the parameters' gradients: head 1's of batch row 1 from the step kernels in either call, of row 0 from blocks in one of them
+    for i, (whole, blocks, good) in enumerate(zip(pa, pb, pc)):
+        assert torch.equal(blocks[[0, 2]], good[[0, 2]]), i
+        assert torch.equal(whole[1].isfinite(), blocks[1].isfinite()), i
+        ok = whole[1].isfinite()
+        assert float((whole[1][ok] - blocks[1][ok]).abs().max() if bool(ok.any()) else 0.0) <= 1e-5 * float(good[1].abs().max()) + 1e-5 * float(whole[1][ok].abs().max() if bool(ok.any()) else 0.0), i
 
 
 def _f32_backward(lib, two, B, T, H, at):
