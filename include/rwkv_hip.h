@@ -83,9 +83,9 @@ int rwkv_hbm_probe(void* stream, int mode, const void* src, void* dst, size_t by
 #define RWKV_PASS_GK 4u
 #define RWKV_PASS_ALL 7u
 #define RWKV_FLAG_SWEEPS 0x100u
-/*   RWKV_FLAG_WHOLE  : rwkv_wkv6f_forward / rwkv_wkv6f_backward_saved keep one workgroup per (batch, head) also where
- *                      B H is below the number of CUs (by default such shapes run as several blocks per sequence joined
- *                      by a scan).  Forward and backward of one step must agree on it. */
+/*   RWKV_FLAG_WHOLE  : rwkv_wkv6f_forward / rwkv_wkv6f_backward_saved and rwkv_wkv5s_* keep one workgroup per (batch, head) also
+ *                      where B H is below the number of CUs (by default such shapes run as several blocks of time per
+ *                      sequence).  Forward and backward of one step must agree on it. */
 #define RWKV_FLAG_WHOLE 0x200u
 
 /* ---------------------------------------------------------------------------------------
@@ -480,9 +480,10 @@ int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float*
                        void* y, float* sT);
 
 /* Forward and backward of all three ops in both modes with a workspace (rwkv7_workspace_bytes; 0: none is needed): few sequences (B H
- * <= 256, in the backward <= 128) that are long enough are cut into blocks of time that are worked on side by side.  Without one whole
- * sequences are walked through, as by the other entry points, and results are theirs bit for bit; in blocks they differ by rounding.
- * s and sa are of one kind either way.  s0, sT, ds0, dsT may be NULL, and s with sa where no backward follows; `backward`: 0 or 1. */
+ * <= 128) of 256 tokens and more (in the forward also of (B H)^2 / 16 and more) are cut into blocks of time that are worked on side by
+ * side.  Without one whole sequences are walked through, as by the other entry points, and results are theirs bit for bit; in blocks they
+ * differ by rounding.  s and sa are of one kind either way.  s0, sT, ds0, dsT may be NULL, and s with sa where no backward follows;
+ * `backward`: 0 or 1. */
 size_t rwkv7_workspace_bytes(int B, int T, int H, int backward);
 int rwkv7_forward_ws(void* stream, int B, int T, int H, int fp32, const float* s0,
                      const void* r, const void* w, const void* k, const void* v, const void* a, const void* b,

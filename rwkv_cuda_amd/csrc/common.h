@@ -136,8 +136,8 @@ template <bool F32, int HN> DEVINL bool steps_head(const void* w, const void* w2
 // bf16, heads of 64: whether any channel of the layer decays faster than the mid-point factors of the one-sweep kernels
 // (wkv6_fwd_f.hip, wkv6_bwd_f.hip) carry (16 tokens by more than e^-60: w > 1.32; the threshold is the bfloat16 below), or is no
 // number.  One such channel moves the whole layer to wkv5_bf.hip: redoing the one head after the others would cost the time of the
-// longest sequence once more (B8 T4096 C2048, forward + backward: 0.54 ms in one sweep; there 0.60 ms with a channel at w = 1.5 and
-// 0.70 at 2.15; 3.1 ms with the one head step by step, as a head beyond W_STEPS_BF16 still is).  Every wave looks at every channel (C is a multiple of 64), so
+// longest sequence once more (B8 T4096 C2048, forward + backward: 0.54 ms in one sweep; there 0.69 ms with a channel at w = 1.5 or
+// 2.15; 3.1 ms with the one head step by step, as a head beyond W_STEPS_BF16 still is).  Every wave looks at every channel (C is a multiple of 64), so
 // all come to the same answer.
 DEVINL bool strong_decay(const float w) { return !(w <= 1.3125f); }
 DEVINL bool strong_layer(const uint16_t* w, const int C, const int lane) {

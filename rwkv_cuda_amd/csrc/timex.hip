@@ -578,6 +578,7 @@ __global__ __launch_bounds__(TXT) void timex_gw_sum_h2(const float* __restrict__
 // a Hankel operand (the windows of g) and one whose columns begin 8 steps apart, so that every element is a tap: nothing is summed over
 // diagonals, and the sums of all rows that a workgroup does stay in registers.  (Lag tiles of 32, columns (block, row) as above, whose
 // sub-diagonals are summed after every few instructions, are timex_gw_short.)
+// Which of the two a shape takes: gw_plan.
 // Operands are THREE bf16 terms, x = h + m + l (each the nearest of what is left: all 24 bits of x), and a product is
 //     x y = h h' + h m' + m h' + m m' + h l' + l h'            (the terms left out are below 2^-24 of the product, 2^-26 rms)
 // with fp32's exponents.  The five small products have accumulators of their own: the sum of the large ones, whose roundings are
@@ -1201,7 +1202,7 @@ __global__ __launch_bounds__(256) void timex_add_parts(const float4* __restrict_
 
 // The waves' shares: runs of a pair's lags are added where the longest run is, until there are eight or a run would have less than RUN_MIN
 // steps (of a tile and a lag; so many take about what it takes to add two waves' sums), then the longest four runs go to the
-// four SIMDs (a wave w runs on SIMD w mod 4) and the others to the least loaded ones.
+// four SIMDs (a wave w runs on SIMD w mod 4) and the others to the least loaded ones.  The plans of a call take 0.15 to 1.0 us of host time.
 constexpr int RUN_MIN = 4;
 // returns how many more steps the longest tile has than the longest run, 0 at least; large: more tiles than waves
 int plan_waves(ConvPlan& p, bool mirror) {

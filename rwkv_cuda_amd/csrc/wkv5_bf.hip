@@ -24,13 +24,13 @@
 // loops spill hundreds of registers, and decays below e^-17 are out of reach all the same.
 // Handing every head with a strong decay (|l| > 3.7) to step-by-step kernels, as the kernels before did, made one such channel in
 // 4096 cost more than everything else: B8 T4096 C4096 N128, forward + backward, 3.8 ms without one, 6.6 to 11.3 ms with.  That is
-// why layers of 64-channel heads come here as well once they have such a channel (B8 T4096 C2048: 0.60 ms with a channel at
-// l = -4.5, 0.70 at -8.6, where they took 1.7 to 3.8 ms).
+// why layers of 64-channel heads come here as well once they have such a channel (B8 T4096 C2048: 0.69 ms with a channel at
+// l = -4.5 or -8.6, where they took 1.7 to 3.8 ms).
 //
 // What bounds it (B8 T4096 C4096: one workgroup per CU).  Forward 0.43 ms for 2.1 GB, half of them the saved states: HBM (5.0 TB/s;
 // 0.82 ms as four heads of 64).  Backward 0.98 ms, 3.3 GB: memory and issue, which its two barriers a chunk do not let overlap
 // entirely (2.95 ms as two sweeps over four heads of 64, whose fp32 terms went through memory).  Both together 6.56 -> 1.48 ms where a
-// channel's decay was strong, 3.83 -> 1.44 where none was.
+// channel's decay was strong, 3.83 -> 1.43 where none was.
 #include <stddef.h>
 
 #include "wkv6_fused.h"
@@ -1005,7 +1005,7 @@ template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, 
 // Blocks of time, heads of 128 channels: as many as give every CU a workgroup (the kernels' LDS leaves room for one), of BLOCK_PAIRS pairs of
 // chunks at least; 1: whole sequences.  per: pairs a block.  Where the line lies, B H sequences, us whole / in blocks: forward 8 of T400 34 / 30,
 // of T4096 255 / 99; 64 of T400 34 / 34, of T4096 261 / 130; 128 of T400 36 / 43, of T800 60 / 61, of T2000 135 / 122; forward + backward 8 of
-// T400 135 / 102, of T4096 1093 / 209; 32 of T4096 1174 / 257; 128 of T400 146 / 125, of T4096 1269 / 836.
+// T400 129 / 77, of T4096 1059 / 191; 32 of T4096 1095 / 251; 64 of T4096 1112 / 428; 128 of T400 136 / 116, of T4096 1153 / 821.
 constexpr int BLOCK_PAIRS = 2, SLOTS = 256;
 int time_blocks(int B, int T, int H, bool bwd, int* per) {
     const long long bh = static_cast<long long>(B) * H, want = SLOTS / bh;

@@ -34,7 +34,7 @@
 //
 // What bounds it.  Forward: HBM (B8 T4096 C4096: 2.9 GB in 0.61 ms; the sequential kernel took 1.3).  Backward: the fp32 matrix
 // instruction, which occupies a SIMD's vector ALU for 32 clocks (99 of them per SIMD and chunk and some 230 vector
-// instructions fill two thirds of its 1.42 ms; the three sequential sweeps took 4.1).  wkv5a: 0.67 + 1.90 ms, 6.2 before.
+// instructions fill two thirds of its 1.42 ms; the three sequential sweeps took 4.1).  wkv5a: 0.67 + 1.85 ms, 6.2 before.
 #include <stddef.h>
 
 #include "common.h"

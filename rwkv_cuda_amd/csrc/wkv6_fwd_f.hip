@@ -548,8 +548,9 @@ __global__ __launch_bounds__(NTQ) void wkv6_fwd_fused(const ArgsQ arg) {
 // a (batch, head) per workgroup of 256.  Forward (reverse = 0): S = s0; out[blk] = S; S <- S 2^logdec[blk] + local[blk].
 // Reverse: the same from the last block down, from zero: what enters a block from above.
 // It is there for few (batch, head) pairs, so what bounds it is latency: 16 bytes a lane, side by side, and the reads of SCAN_AHEAD
-// blocks, of which none depends on another, in flight together.  B1 H32, 8 blocks: 5.1 us (launch, one round of reads, the stores); with sixteen channels a thread (a quarter
-// of the workgroups, 64 bytes between lanes) and the reads of one block at a time 11.
+// blocks, of which none depends on another, in flight together.  B1 H8 T4096, 32 blocks of 128 tokens: 8.2 us (launch, four rounds of reads, the
+// stores).  At 8 blocks, which no longer come here, 5.1 us for 32 heads; with sixteen channels a thread (a quarter of the workgroups, 64 bytes between
+// lanes) and the reads of one block at a time 11.
 constexpr int SCAN_AHEAD = 8, SCAN_WG = N * N / (4 * 256);
 __global__ __launch_bounds__(256) void wkv6_scan(const float* __restrict__ local, const float* __restrict__ logdec, const uint16_t* __restrict__ s0,
                                                  float* __restrict__ out, const int NB, const int reverse) {

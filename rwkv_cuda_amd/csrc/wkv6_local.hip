@@ -1,5 +1,6 @@
 // wkv6 / wkv6_state (raw bf16 decay) and wkv5 (one decay per channel), head size 64, sequences cut into blocks of time: what a block
-// makes of a state that enters it empty, and the log2 of its decay per key channel, for wkv6_scan (wkv6_fwd_f.hip) to chain.
+// makes of a state that enters it empty, and the log2 of its decay per key channel.  Up to SCAN_BLOCKS blocks are chained by the kernels that start
+// from them (wkv6_fwd_f.hip, wkv6_bwd_f.hip), more by wkv6_scan (wkv6_fwd_f.hip).
 //     forward   E[i][j] = sum_t v_t[i] k_t[j] 2^{sum of the decays after t}          backward  sum_t gy_t[i] r_t[j] 2^{sum of the decays before t}
 // Nothing but this sum comes out of a block, so it is no chain of chunks: the tokens' exponents are direct sums of log decays (never above
 // zero: nothing overflows, and whatever a decay is it needs no second path), and E is one product over up to SUP tokens at a time.
