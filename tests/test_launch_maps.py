@@ -1,4 +1,4 @@
-"""CPU: two index maps that decide which workgroup computes what, checked as maps (bijections, exact covers) with the
+"""CPU: three index maps that decide which workgroup computes what, checked as maps (bijections, exact covers) with the
 expressions taken from the sources.
 
 * wkv4: workgroups are renumbered so that the two that share every 128-byte line run on the same XCD (csrc/wkv4.hip,
@@ -6,7 +6,9 @@ expressions taken from the sources.
 * wkv5 at head size 128: every head runs as four heads of 64 in two launches; workgroup h of a launch takes its value
   channels from block h and its key channels from block h ^ cross (csrc/wkv6_fwd.hip and the two sweeps).  Every block
   (value half, key half) of every head must be computed exactly once, and every output block must receive exactly one
-  term from each launch."""
+  term from each launch.
+* depthwise_conv1d of any shape: a unit is a channel and a group of batch rows (csrc/timex.hip, timex_conv_any).  Every channel's
+  rows must be covered once, and groups of unequal size must not end up on some of the eight XCDs only."""
 import os
 import re
 
@@ -55,3 +57,25 @@ def test_split_heads_cover_every_block_once():
                 by_value = sorted(c for (hd, i, j), (c,) in ((k, tuple(v)) for k, v in blocks.items()) if hd == head and i == half)
                 by_key = sorted(c for (hd, i, j), (c,) in ((k, tuple(v)) for k, v in blocks.items()) if hd == head and j == half)
                 assert by_value == [0, 1] and by_key == [0, 1]
+
+
+def test_conv_units_cover_every_row_once_and_spread_over_the_xcds():
+    src = open(os.path.join(CSRC, "timex.hip")).read()
+    m = re.search(r"void timex_conv_any\([^;]*;.*?const int ([^;]*b0 = .+?);", src, re.S)
+    assert m
+    parts = [p.split("=") for p in re.split(r",\s*(?=\w+ =)", m.group(1))]
+    assert sorted(name.strip() for name, _ in parts) == ["b0", "c", "fewer", "grp"]
+    code = [(name.strip(), compile(expr.replace("blockIdx.x", "block").replace("/", "//").strip(), "timex.hip", "eval")) for name, expr in parts]
+    for B, C, ng in [(1, 5, 1), (7, 12, 2), (10, 768, 4), (3, 768, 2), (5, 200, 3), (19, 96, 6), (13, 41, 8), (32, 7, 32)]:
+        rows, xcd = set(), [0] * 8
+        for block in range(C * ng):
+            env = {"block": block, "B": B, "C": C, "ng": ng, "min": min}
+            for name, expr in code:
+                env[name] = eval(expr, {}, env)
+            n = env["fewer"] + (env["grp"] < B % ng)
+            for b in range(env["b0"], env["b0"] + n):
+                assert 0 <= env["c"] < C and 0 <= b < B and (env["c"], b) not in rows
+                rows.add((env["c"], b))
+            xcd[block % 8] += n
+        assert len(rows) == B * C
+        assert max(xcd) - min(xcd) <= ng * -(-B // ng), (B, C, ng, xcd)      # a unit of each group at most
