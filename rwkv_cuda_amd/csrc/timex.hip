@@ -1258,9 +1258,9 @@ constexpr int TILE_STEPS = 16, TILE_STEPS_FULL = 5, TILE_STEPS_FEW = 3;
 constexpr int SHORT_ROWS = 672;        // (B13 C300 T772 25.2 / 26.6)
 // Batch rows of a unit, dealt evenly to `ng` units a channel.  What finishes first by a count of matrix clocks (96 per column tile and
 // block lag on a CU's four SIMDs), conversion and a fixed cost, in rounds of two workgroups per CU; at most 16 tiles (a pair a wave) and
-// 80 KB.  Units of two sizes count by their mean, but in the last round, up to SHORT_ROWS steps, by the larger: B3 C200 T516 as 2 + 1 rows, one round,
-// 9.9 us, as 1 + 1 + 1, two rounds of half the time, 8.5; B5 C768 T516 21.2 / 17.1.  Longer rows' units take turns of their own: B19 C400 T1060
-// 61 us by the mean, 71 so.
+// 80 KB.  Units of two sizes count by their mean, but in the last round by the larger: B3 C200 T644 as 2 + 1 rows, one round, 9.2 us, as
+// 1 + 1 + 1, two rounds of half the time, 8.1; B9 C200 T196 7.0 / 5.9.  A last round after others that leaves every CU one workgroup at most, which
+// then runs nearly twice as fast, counts three quarters: B3 C768 T1500 as 3 rows, 1.5 rounds, 36.0 us, as 2 + 1, three, 44.6; B19 C640 T772 50.7 / 56.6.
 ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
     ConvPlans best{};
     double cost = 1e300;
@@ -1282,7 +1282,8 @@ ConvPlans conv_any_plans(int B, int C, int T, bool mirror, int* ng) {
         }
         x.copies = most == 1 && conv_any_lds(x.p[0].q, 2) > LDS_ANY ? 1 : 2;
         if (unit < 0 || conv_plan_lds(x) > LDS_ANY || 8 * x.p[0].q.nt * rows[0] > CONV_PIECES * TXT) { if (most > 1) break; }
-        const double c = static_cast<double>((static_cast<long long>(C) * groups - 1) / (2 * NCU)) * unit + (T <= SHORT_ROWS ? largest : unit);
+        const long long units = static_cast<long long>(C) * groups, full = (units - 1) / (2 * NCU);
+        const double c = full * unit + (full > 0 && units - full * 2 * NCU <= NCU ? 0.75 : 1.0) * largest;
         if (c < cost) { cost = c; best = x; *ng = groups; }
     }
     int longer = 0;

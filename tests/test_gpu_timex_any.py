@@ -71,6 +71,18 @@ def test_many_short_rows(lib, B, C, T):
         assert max_rel_to_peak(a, got.detach().double().cpu()) <= 1e-5, name
 
 
+@pytest.mark.parametrize("B,C,T", [(3, 700, 1500), (3, 384, 1500), (10, 330, 1300), (19, 350, 772), (13, 320, 644)])
+def test_last_rounds_of_few_units(lib, B, C, T):
+    """Units chosen with a last round that leaves CUs one workgroup (the second: not), of one size and of two."""
+    some = [0, C // 2, C - 1]
+    (w, k, g), ref = _some_channels(B, C, T, B + T, some)
+    w, k = w.requires_grad_(True), k.requires_grad_(True)
+    x = depthwise_conv1d.RUN_CUDA(w, k, B, C, T, 0.0)
+    gw, gk = torch.autograd.grad(x, (w, k), g)
+    for name, a, got in zip(("x", "gw", "gk"), ref, (x[:, some], gw[some], gk[:, some])):
+        assert max_rel_to_peak(a, got.detach().double().cpu()) <= 1e-5, name
+
+
 @pytest.mark.parametrize("B,C,T", [(24, 300, 508), (27, 300, 452), (12, 768, 452), (32, 64, 512 + 4), (6, 200, 644), (16, 64, 708), (16, 64, 712)])
 def test_kernel_gradients_of_middle_lengths(lib, B, C, T):
     """Lag tiles of 32 or of 256, and as many parts of the batch, as take less time: either side of the lengths where the rule changes."""
