@@ -195,6 +195,56 @@ DEVINL float sigmoid_fast(float x) {
     return 0.25f * fmaf(fmaf(-fminf(d, 3.40282346638528859812e38f), y, 1.f), y, y);
 }
 
+// The factors of the four tokens (4 q + e) of a channel held by a thread, from their decays in units of log 2 (part: the waves' sums of
+// them).  All four inputs are referred to one border of the chunk, forwards its end, backwards its start, so that each is split once and
+// serves both the causal tiles and the state: x[e] = e^{c_L - c_t} (e^{c_t}), t = 4 q + e, e = 0 .. 4, carry to or from the border what
+// is added to the state that is handed on, y[e] = HOLD / x[e] meet the state that came in, which has the chunk's whole decay on it
+// beforehand.  An exponent is one sum and no difference, so what is near the border, the largest part of the new state, has the smallest
+// errors; and a tile's factors x[s + 1] / x[t] are each other's reciprocals for neighbours, whatever the exponents' roundings.  HOLD: or
+// e^9.7 would take inputs out of range that e^4.9 (referred to the chunk's middle) did not.
+constexpr float HOLD = 0.0078125f, UNHOLD = 128.f;
+template <bool END> DEVINL void growth(const float (&lam)[4], const float (*part)[N], int q, int j, float (&x)[5], float (&y)[5]) {
+    float out = 0.f;                                   // between the thread's tokens and the border
+    const int n = END ? 3 - q : q, d = END ? -1 : 1, b = END ? 3 : 0;
+    if (n > 0) out = part[b][j];
+    if (n > 1) out += part[b + d][j];
+    if (n > 2) out += part[b + 2 * d][j];
+    float sum = 0.f;
+#pragma unroll
+    for (int z = 0; z < 5; ++z) {
+        const int e = END ? 4 - z : z;
+        if (z > 0) sum += lam[END ? e : e - 1];
+        x[e] = __builtin_amdgcn_exp2f(z > 0 ? sum + out : out);
+        y[e] = __builtin_amdgcn_rcpf(x[e]) * HOLD;
+    }
+}
+// decay of a step in units of log 2: W_SCALE log2(e) sigmoid(x).  The product of the two constants falls between two fp32 numbers, of which
+// the nearest is 3e-8 off, in every step the same way; the quotient of these two is 3e-13 off.
+DEVINL float log2_decay(float x) {
+    constexpr float C = 0x1.fee3f2p-3f, M = -0x1.bf0c86p-3f;
+    const float d = fmaf(__builtin_amdgcn_exp2f(x * -1.44269504088896340736f), C, C);
+    const float y = __builtin_amdgcn_rcpf(d);
+    return M * fmaf(fmaf(-fminf(d, 3.40282346638528859812e38f), y, 1.f), y, y);
+}
+
+// HOLD tile[t][s] = sum_c a_t e^{c_t} b_s e^{-c_{s+1}} over 64 channels, masked to s < t (strict) or s <= t: register v <-> t = 4 g + v, lane <-> s,
+// or (ROWS) register v <-> s = 4 g + v, lane <-> t.  ta: the plane of the t side, sp: of the s side, one of a pair.
+template <bool ROWS> DEVINL f32x4 causal_tile(const Tr& ta, lds_t sp, bool strict, int l16, int g) {
+    Sum2 sum = SUM0;
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+        const Op3 x = get3_tr(0, ta, hb), y = get3_tr_pair(0, sp, hb);
+        if constexpr (ROWS) add32(sum, y, x); else add32(sum, x, y);
+    }
+    f32x4 acc = total(sum);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int t = ROWS ? l16 : 4 * g + v, s = ROWS ? 4 * g + v : l16;
+        acc[v] = (strict ? s < t : s <= t) ? acc[v] : 0.f;
+    }
+    return acc;
+}
+
 // tile[t][s] = sum_c X[t][c] Y[s][c] over 64 channels, masked to s < t (strict) or s <= t: register v <-> t = 4 g + v, lane <-> s, or
 // (ROWS) register v <-> s = 4 g + v, lane <-> t
 template <bool ROWS> DEVINL f32x4 causal_acc(const float (*X)[PS], const float (*Y)[PS], bool strict, int l16, int g) {
@@ -224,13 +274,12 @@ template <bool ROWS> DEVINL f32x4 causal_acc(const float (*X)[PS], const float (
 // The P waves make the tiles on the fp32 matrix instructions, all other products are split ones (split3.h).
 constexpr int NTF = 8 * 64;        // waves 0..3 role S, 4..7 role P
 struct SmemCF {
-    float Ap[CL][PS], Rp[CL][PS], Bp[CL][PS], Kp[CL][PS];      // referred to the middle of the chunk: the tiles
     float Yo[CL][PS], Uo[CL][PS];
     float ABt[CL][TS];
     float part[4][N];
     float dec[2][N];
 };
-// three-term planes and tiles behind it: a e^{c_t}, r e^{c_{t+1}}, k and b carried to the end of the chunk (e^{c_L - c_{s+1}}), v (one term
+// three-term planes and tiles behind it: a HOLD e^{c_t - c_L}, r HOLD e^{c_{t+1} - c_L}, k and b times e^{c_L - c_{s+1}}, v (one term
 // where it is bf16), AK, RB, RK, (I - AB)^{-1}
 constexpr uint32_t F_AS = (sizeof(SmemCF) + 31) / 32 * 32, F_RS = F_AS + PLANE3, F_KB = F_RS + PLANE3, F_V = F_KB + 2 * PAIR3;
 template <bool F32> constexpr uint32_t F_MA = F_V + (F32 ? PLANE3 : TERM);      // (I - AB)^{-1} and AK
@@ -258,7 +307,7 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
     auto convert = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            lam[e] = W_SCALE * sigmoid_fast(widen<F32>(nx[0][e]));
+            lam[e] = log2_decay(widen<F32>(nx[0][e]));
             // (a value of its own: the product could join an addition in one of the two copies of this code and not in the other, and a
             // sequence cut into calls would no longer give the same bits)
             asm volatile("" : "+v"(lam[e]));
@@ -269,29 +318,26 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
         S.part[q][lane] = (lam[0] + lam[1]) + (lam[2] + lam[3]);
     };
     auto planes = [&](const int slot) __attribute__((always_inline)) {
-        float cm, cl;
-        const Factors f = chunk_factors(lam, S.part, q, lane, cm, cl);
-        f32x4 as, rs, ke, be;
+        float x[5], y[5];
+        growth<true>(lam, S.part, q, lane, x, y);
+        f32x4 as, rs, ks, bs;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int t = 4 * q + e;
-            S.Ap[t][lane] = aa[e] * f.ea[e];
-            S.Rp[t][lane] = rr[e] * f.er[e];
-            S.Bp[t][lane] = bb[e] * f.eb[e];
-            S.Kp[t][lane] = kk[e] * f.eb[e];
-            as[e] = aa[e] * f.es[e];
-            rs[e] = rr[e] * (f.es[e] * __expf(lam[e]));
-            ke[e] = kk[e] * f.ee[e];
-            be[e] = bb[e] * f.ee[e];
+            as[e] = aa[e] * y[e];
+            rs[e] = rr[e] * y[e + 1];
+            ks[e] = kk[e] * x[e + 1];
+            bs[e] = bb[e] * x[e + 1];
         }
         const lds_t o = sb + piece(lane, q);
-        // (no factor is above 1: what comes from bf16 inputs stays within bf16's range)
-        put3(o + F_AS, split3<!F32>(as)); put3(o + F_RS, split3<!F32>(rs));
-        put_pair<TERM2>(sb + F_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(ke), split3<!F32>(be));
+        put3(o + F_AS, split3(as)); put3(o + F_RS, split3(rs));
+        // (x is not above 1: what comes from bf16 inputs stays within bf16's range)
+        put_pair<TERM2>(sb + F_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(ks), split3<!F32>(bs));
         if constexpr (F32) put3(o + F_V, split3(f32x4{vv[0], vv[1], vv[2], vv[3]}));
         else lds_st<u32x2>(o + F_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
-        if (q == 0) S.dec[slot][lane] = exp_acc(cl);
+        if (q == 0) S.dec[slot][lane] = x[0];
     };
+    const Tr ta = tr_bases(sb + (q < 2 ? F_AS : F_RS), l16, g);
+    const lds_t sp = tr_pair(sb + F_KB + ((q & 1) ? 0 : 8), l16, g);
     fetch(0);
     convert();
     fetch(1);
@@ -301,17 +347,16 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
     for (int c = 0; c < nch; ++c) {
         // ---------------------------------------------------------------- phase X
         {
-            const float (*X)[PS] = q < 2 ? S.Ap : S.Rp;
-            const float (*Y)[PS] = (q & 1) ? S.Kp : S.Bp;
             f32x4 x;
+            const lds_t slot = sp + (c & 1) * PAIR3;
             if (q == 0) {
-                st4(&S.ABt[l16][4 * g], causal_acc<false>(X, Y, true, l16, g));
+                st4(&S.ABt[l16][4 * g], causal_tile<false>(ta, slot, true, l16, g) * UNHOLD);
                 // this wave wrote AB itself (LDS keeps a wave's accesses in order): the inverse once, for all four S waves
                 float m[CL];
                 inverse_rows(S.ABt, l16, m);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) x[v] = by_group(g, m[v], m[4 + v], m[8 + v], m[12 + v]);
-            } else x = causal_acc<true>(X, Y, q == 1, l16, g);
+            } else x = causal_tile<true>(ta, slot, q == 1, l16, g);
             // (one store with a selected address, as in the backward)
             put_half<TTERM2>(sb + piece2(l16, g) + (q == 0 ? F_MA<F32> : (q == 1 ? F_MA<F32> + 8 : (q == 2 ? F_RKB<F32> + 8 : F_RKB<F32>))), split3(x));
         }
@@ -352,10 +397,12 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
     for (int c = 0; c < nch; ++c) {
         // ---------------------------------------------------------------- phase X: what needs no tile
         const auto vop = load_v();                   // V[s = 4 g + v][i_own]
-        Sum2 W = SUM0, Y = SUM0;
+        const float* const dec = &S.dec[c & 1][4 * g];
+        Sum2 W = SUM0, Y = SUM0;                     // HOLD W, HOLD Y
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
-            const Op3 st = join(split3(St[2 * hb]), split3(St[2 * hb + 1]));
+            // (decayed for these products only: in the update a fused multiplication and addition rounds the state once)
+            const Op3 st = join(split3(St[2 * hb] * ld4(dec + 32 * hb)), split3(St[2 * hb + 1] * ld4(dec + 32 * hb + 16)));
             add32(W, get3_tr(F_AS, tr, hb), st);
             add32(Y, get3_tr(F_RS, tr, hb), st);
         }
@@ -371,11 +418,11 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
         // ---------------------------------------------------------------- phase Y
         add16(W, get_half<TTERM2>(pp + F_MA<F32> + 8), vop);
         Sum2 Us = SUM0;
-        add16(Us, get_half<TTERM2>(pp + F_MA<F32>), split3(total(W)));
+        add16(Us, get_half<TTERM2>(pp + F_MA<F32>), split3(total(W) * UNHOLD));
         const f32x4 U = total(Us);
         const Op3 vu = join(as3(vop), split3(U));        // V and U share the instructions of what follows
         add32(Y, get_pair<TTERM2>(pp + F_RKB<F32>), vu);
-        const f32x4 y = total(Y);
+        const f32x4 y = total(Y) * UNHOLD;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             S.Yo[4 * g + v][i_own] = y[v];
@@ -386,7 +433,7 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
         for (int jt = 0; jt < 4; ++jt) {
             Sum2 x = SUM0;
             add32(x, get_pair<TERM2>(kb + 1024 * jt), vu);
-            St[jt] = St[jt] * ld4(&S.dec[c & 1][16 * jt + 4 * g]) + total(x);
+            St[jt] = St[jt] * ld4(dec + 16 * jt) + total(x);
         }
         __syncthreads();
     }

@@ -131,6 +131,16 @@ DEVINL Op3 get3_tr(uint32_t plane, const Tr& o, int hb) { return {ld_tr16(o, pla
 // contraction over the columns takes them.
 constexpr uint32_t TERM2 = 2 * TERM, PAIR3 = 3 * TERM2, TTERM2 = 1024, TPAIR3 = 3 * TTERM2;
 DEVINL lds_t piece2(int ch, int tg) { return static_cast<lds_t>(ch * 64 + 16 * (tg ^ ((ch >> 2) & 3))); }      // of a tile: row, column / 4
+// One of the two planes over channels, as get3_tr: the plane's pieces are every other eight bytes.  The channels' turns repeat every 16, so
+// one address serves both blocks.
+DEVINL lds_t tr_pair(lds_t base, int l16, int g) { return base + piece2(4 * g + (l16 >> 2), l16 & 3); }
+DEVINL bf16x8 ld_tr16_pair(lds_t o, uint32_t plane, int hb) {
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    typedef v4s __attribute__((address_space(3))) * ptr;
+    const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + plane + 2048 * hb)), y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + plane + 2048 * hb + 1024));
+    return op2(__builtin_bit_cast(u32x2, x), __builtin_bit_cast(u32x2, y));
+}
+DEVINL Op3 get3_tr_pair(uint32_t plane, lds_t o, int hb) { return {ld_tr16_pair(o, plane, hb), ld_tr16_pair(o, plane + TERM2, hb), ld_tr16_pair(o, plane + 2 * TERM2, hb)}; }
 template <uint32_t STRIDE> DEVINL void put_pair(lds_t a, const B3& x, const B3& y) {
     lds_st<u32x4>(a, u32x4{x.h[0], x.h[1], y.h[0], y.h[1]});
     lds_st<u32x4>(a + STRIDE, u32x4{x.m[0], x.m[1], y.m[0], y.m[1]});
