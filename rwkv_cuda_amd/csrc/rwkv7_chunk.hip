@@ -102,8 +102,18 @@ template <bool F32> DEVINL uint32_t ld_raw(const uint16_t* p, size_t base, uint3
 }
 template <bool F32> DEVINL float widen(uint32_t x) { return F32 ? __uint_as_float(x) : bf2f(static_cast<uint16_t>(x)); }
 
-// the value a lane group g takes from four candidates (register index that depends on the lane group)
-DEVINL float by_group(int g, float x0, float x1, float x2, float x3) { return g == 0 ? x0 : (g == 1 ? x1 : (g == 2 ? x2 : x3)); }
+// the four values x[4 g + v] of lane group g (behind an empty asm: the compiler would make branches of the choice, with the sums in them)
+DEVINL f32x4 by_group(int g, float (&x)[CL]) {
+#pragma unroll
+    for (int i = 0; i < CL; ++i) asm volatile("" : "+v"(x[i]));
+    f32x4 r;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const float lo = g & 1 ? x[4 + v] : x[v], hi = g & 1 ? x[12 + v] : x[8 + v];
+        r[v] = g & 2 ? hi : lo;
+    }
+    return r;
+}
 
 // Rows of M = (I - AB)^{-1}: lane (l16 = r) gets m[s] = M[r][s] from the column recurrence M[r][s] = [r == s] + sum_{t>s} M[r][t] AB[t][s].
 // ABt[s][t] = AB[t][s] is read with wave-uniform addresses (LDS broadcast).
@@ -195,45 +205,57 @@ DEVINL float sigmoid_fast(float x) {
     return 0.25f * fmaf(fmaf(-fminf(d, 3.40282346638528859812e38f), y, 1.f), y, y);
 }
 
-// The factors of the four tokens (4 q + e) of a channel held by a thread, from their decays in units of log 2 (part: the waves' sums of
-// them).  All four inputs are referred to one border of the chunk, forwards its end, backwards its start, so that each is split once and
+// Decay of a step in two parts, in units of log 2 a multiple of 2^-19 below 1, of which sums over a chunk (below 14) are exact, and in those
+// of e the rest, below 2^-20: with the sum of the first parts rounded to fp32 an exponential is off by up to 3e-7.
+struct Decay { float hi, lo; };
+constexpr float LN2 = 0.69314718055994530942f;
+DEVINL Decay add(const Decay& a, const Decay& b) { return {a.hi + b.hi, a.lo + b.lo}; }
+DEVINL float grow(const Decay& d) { const float e = __builtin_amdgcn_exp2f(d.hi); return fmaf(e, d.lo, e); }
+// W_SCALE log2(e) sigmoid(x), from the sigmoid
+DEVINL Decay decay_of_sig(float sig) {
+    constexpr double C = -0.6065306597 * 1.44269504088896340736;
+    constexpr float HI = static_cast<float>(C), LO = static_cast<float>(C - static_cast<double>(HI));
+    const float hi = fmaf(sig, HI, 24.f) - 24.f;                   // (24: whose last place is 2^-19)
+    return {hi, LN2 * fmaf(sig, LO, fmaf(sig, HI, -hi))};
+}
+// The factors of the four tokens (4 q + e) of a channel held by a thread, from their decays (part: the waves' sums of them).  All four
+// inputs are referred to one border of the chunk, forwards its end, backwards its start, so that each is split once and
 // serves both the causal tiles and the state: x[e] = e^{c_L - c_t} (e^{c_t}), t = 4 q + e, e = 0 .. 4, carry to or from the border what
 // is added to the state that is handed on, y[e] = HOLD / x[e] meet the state that came in, which has the chunk's whole decay on it
-// beforehand.  An exponent is one sum and no difference, so what is near the border, the largest part of the new state, has the smallest
-// errors; and a tile's factors x[s + 1] / x[t] are each other's reciprocals for neighbours, whatever the exponents' roundings.  HOLD: or
-// e^9.7 would take inputs out of range that e^4.9 (referred to the chunk's middle) did not.
+// beforehand.  HOLD: or e^9.7 would take inputs out of range that e^4.9 (referred to the chunk's middle) did not.
 constexpr float HOLD = 0.0078125f, UNHOLD = 128.f;
-template <bool END> DEVINL void growth(const float (&lam)[4], const float (*part)[N], int q, int j, float (&x)[5], float (&y)[5]) {
-    float out = 0.f;                                   // between the thread's tokens and the border
+DEVINL float held_inverse(float x) { return __builtin_amdgcn_rcpf(x) * HOLD; }
+template <bool END> DEVINL void growth(const Decay (&lam)[4], const Decay (*part)[N], int q, int j, float (&x)[5], float (&y)[5]) {
+    Decay at = {0.f, 0.f};                             // between the thread's tokens and the border
     const int n = END ? 3 - q : q, d = END ? -1 : 1, b = END ? 3 : 0;
-    if (n > 0) out = part[b][j];
-    if (n > 1) out += part[b + d][j];
-    if (n > 2) out += part[b + 2 * d][j];
-    float sum = 0.f;
+    if (n > 0) at = part[b][j];
+    if (n > 1) at = add(at, part[b + d][j]);
+    if (n > 2) at = add(at, part[b + 2 * d][j]);
 #pragma unroll
     for (int z = 0; z < 5; ++z) {
         const int e = END ? 4 - z : z;
-        if (z > 0) sum += lam[END ? e : e - 1];
-        x[e] = __builtin_amdgcn_exp2f(z > 0 ? sum + out : out);
-        y[e] = __builtin_amdgcn_rcpf(x[e]) * HOLD;
+        if (z > 0) at = add(at, lam[END ? e : e - 1]);
+        x[e] = grow(at);
+        y[e] = held_inverse(x[e]);
     }
 }
-// decay of a step in units of log 2: W_SCALE log2(e) sigmoid(x).  The product of the two constants falls between two fp32 numbers, of which
-// the nearest is 3e-8 off, in every step the same way; the quotient of these two is 3e-13 off.
-DEVINL float log2_decay(float x) {
+DEVINL Decay sum4(const Decay (&l)[4]) { return add(add(l[0], l[1]), add(l[2], l[3])); }
+// the same from x, in a backward-less chain: c / (1 + e^-x) with the quotient of the two constants 3e-13 from the product
+DEVINL Decay decay_of(float x) {
     constexpr float C = 0x1.fee3f2p-3f, M = -0x1.bf0c86p-3f;
     const float d = fmaf(__builtin_amdgcn_exp2f(x * -1.44269504088896340736f), C, C);
-    const float y = __builtin_amdgcn_rcpf(d);
-    return M * fmaf(fmaf(-fminf(d, 3.40282346638528859812e38f), y, 1.f), y, y);
+    const float y = __builtin_amdgcn_rcpf(d), s = fmaf(fmaf(-fminf(d, 3.40282346638528859812e38f), y, 1.f), y, y);
+    const float hi = fmaf(s, M, 24.f) - 24.f;
+    return {hi, LN2 * fmaf(s, M, -hi)};
 }
 
 // HOLD tile[t][s] = sum_c a_t e^{c_t} b_s e^{-c_{s+1}} over 64 channels, masked to s < t (strict) or s <= t: register v <-> t = 4 g + v, lane <-> s,
-// or (ROWS) register v <-> s = 4 g + v, lane <-> t.  ta: the plane of the t side, sp: of the s side, one of a pair.
-template <bool ROWS> DEVINL f32x4 causal_tile(const Tr& ta, lds_t sp, bool strict, int l16, int g) {
+// or (ROWS) register v <-> s = 4 g + v, lane <-> t.  ta, sb: operand of 32 channels of the t side, of the s side.
+template <bool ROWS, class TA, class SB> DEVINL f32x4 causal_tile(TA ta, SB sb, bool strict, int l16, int g) {
     Sum2 sum = SUM0;
 #pragma unroll
     for (int hb = 0; hb < 2; ++hb) {
-        const Op3 x = get3_tr(0, ta, hb), y = get3_tr_pair(0, sp, hb);
+        const Op3 x = ta(hb), y = sb(hb);
         if constexpr (ROWS) add32(sum, y, x); else add32(sum, x, y);
     }
     f32x4 acc = total(sum);
@@ -276,7 +298,7 @@ constexpr int NTF = 8 * 64;        // waves 0..3 role S, 4..7 role P
 struct SmemCF {
     float Yo[CL][PS], Uo[CL][PS];
     float ABt[CL][TS];
-    float part[4][N];
+    Decay part[4][N];
     float dec[2][N];
 };
 // three-term planes and tiles behind it: a HOLD e^{c_t - c_L}, r HOLD e^{c_{t+1} - c_L}, k and b times e^{c_L - c_{s+1}}, v (one term
@@ -301,21 +323,22 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
 #pragma unroll
             for (int k = 0; k < 6; ++k) nx[k][e] = ld_raw<F32>(src[k], base, static_cast<uint32_t>((4 * q + e) * H) * N + lo);
     };
-    float lam[4], rr[4], kk[4], aa[4], bb[4];
+    Decay lam[4];
+    float rr[4], kk[4], aa[4], bb[4];
     [[maybe_unused]] float vv[4];
     [[maybe_unused]] uint32_t vb[4];
     auto convert = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            lam[e] = log2_decay(widen<F32>(nx[0][e]));
+            lam[e] = decay_of(widen<F32>(nx[0][e]));
             // (a value of its own: the product could join an addition in one of the two copies of this code and not in the other, and a
             // sequence cut into calls would no longer give the same bits)
-            asm volatile("" : "+v"(lam[e]));
+            asm volatile("" : "+v"(lam[e].hi), "+v"(lam[e].lo));
             rr[e] = widen<F32>(nx[1][e]); kk[e] = widen<F32>(nx[2][e]);
             if constexpr (F32) vv[e] = widen<F32>(nx[3][e]); else vb[e] = nx[3][e];
             aa[e] = widen<F32>(nx[4][e]); bb[e] = widen<F32>(nx[5][e]);
         }
-        S.part[q][lane] = (lam[0] + lam[1]) + (lam[2] + lam[3]);
+        S.part[q][lane] = sum4(lam);
     };
     auto planes = [&](const int slot) __attribute__((always_inline)) {
         float x[5], y[5];
@@ -348,15 +371,15 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
         // ---------------------------------------------------------------- phase X
         {
             f32x4 x;
-            const lds_t slot = sp + (c & 1) * PAIR3;
+            auto top = [&](int hb) __attribute__((always_inline)) { return get3_tr(0, ta, hb); };
+            auto sop = [&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, sp + (c & 1) * PAIR3, hb); };
             if (q == 0) {
-                st4(&S.ABt[l16][4 * g], causal_tile<false>(ta, slot, true, l16, g) * UNHOLD);
+                st4(&S.ABt[l16][4 * g], causal_tile<false>(top, sop, true, l16, g) * UNHOLD);
                 // this wave wrote AB itself (LDS keeps a wave's accesses in order): the inverse once, for all four S waves
                 float m[CL];
                 inverse_rows(S.ABt, l16, m);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) x[v] = by_group(g, m[v], m[4 + v], m[8 + v], m[12 + v]);
-            } else x = causal_tile<true>(ta, slot, q == 1, l16, g);
+                x = by_group(g, m);
+            } else x = causal_tile<true>(top, sop, q == 1, l16, g);
             // (one store with a selected address, as in the backward)
             put_half<TTERM2>(sb + piece2(l16, g) + (q == 0 ? F_MA<F32> : (q == 1 ? F_MA<F32> + 8 : (q == 2 ? F_RKB<F32> + 8 : F_RKB<F32>))), split3(x));
         }
@@ -561,8 +584,7 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
                     st4(&S.AB[l16][4 * g], t);
                     inverse_rows(S.AB, l16, m);
                 }
-#pragma unroll
-                for (int v = 0; v < 4; ++v) x[v] = by_group(g, m[v], m[4 + v], m[8 + v], m[12 + v]);
+                x = by_group(g, m);
             } else if constexpr (REV) x = causal_acc<false>(S.Xp, S.Bp, false, l16, g);
             else x = causal_acc<true>(S.Ap, S.Xp, true, l16, g);
             put_half<TTERM2>(sb + piece2(l16, g) + L_MA<F32> + (q == 0 ? 0 : 8), split3(x));
@@ -695,46 +717,40 @@ __global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
 // e^-0.6, where 1 - sig has few digits.
 constexpr int NTB = 12 * 64;       // waves 0..3 role A, 4..7 role B, 8..11 role P
 
-// Everything that is a function of one chunk's inputs alone; two copies (but for the planes that only phase 1 reads): the P waves fill
-// one while the A and B waves work on the other.
-struct PlanesB {
-    float Ap[CL][PS], Rp[CL][PS], Bp[CL][PS], Kp[CL][PS];   // referred to the middle of the chunk (tiles, dA' .. dK')
-    float EA[CL][PS], ER[CL][PS], DWF[CL][PS];               // e^{c_t - c_m}, e^{c_{t+1} - c_m}, W_SCALE sig (1 - sig)
-    float d1[N], d2[N], dec[N];
-};
-static_assert(offsetof(PlanesB, Rp) == 4 * CL * PS && offsetof(PlanesB, d1) == 7 * 4 * CL * PS && offsetof(PlanesB, dec) == offsetof(PlanesB, d1) + 8 * N, "role B's addresses");
 constexpr int PK = 72;            // row stride (bf16 elements) of a parked output
 // fp32 outputs are not parked (twice the bytes would not fit the CU's LDS): the waves that finish them store them from
 // registers, 64 bytes of four rows per instruction.
 template <bool F32>
 struct SmemCB {
-    PlanesB pl[2];
-    float part[4][N];
+    Decay part[4][N];
+    float dec[2][N];
     float AB[CL][TS];
-    uint16_t park[F32 ? 1 : 5][F32 ? 1 : CL][PK];                                // da, dr, db, dk, dw of the chunk that role B finished last, [token][channel]
-    uint16_t parkv[F32 ? 1 : 2][F32 ? 1 : CL][PK];                               // dv, which is ready one visit earlier than the other five
+    uint16_t park[F32 ? 1 : 5][F32 ? 1 : CL][F32 ? 1 : PK];                                // da, dr, db, dk, dw of the chunk that role B finished last, [token][channel]
+    uint16_t parkv[F32 ? 1 : 2][F32 ? 1 : CL][F32 ? 1 : PK];                               // dv, which is ready one visit earlier than the other five
 };
-// three-term planes and tiles behind it.  Two copies: r e^{c_{t+1}} and a e^{c_t} (RA, the state-gradient update), U, v and dy (one term
-// each where they are bf16).  One: b, k times e^{c_L - c_{s+1}} (dU, dV), dW, and the tiles, each as the lanes of its products hold
-// it: the transposes of (I - AB)^{-1} and RB (MB), RK and AK (RKA); by rows (over s) dAB and dAK for dA', dRB and dRK for dR'; by columns (over t)
-// dAB and dRB for dB', dAK and dRK for dK'.
+// Planes and tiles behind it.  Two copies, of which the P waves fill one while the A and B waves work on the other: a e^{c_t} and
+// r e^{c_{t+1}} (AR), b and k times HOLD e^{-c_{s+1}} (BK), U, v and dy (one term each where they are bf16) in three terms; fp32, 16 bytes of
+// four tokens as the pairs lie: e^{c_{t+1}} (ES), W_SCALE sig (1 - sig) (DWF); inputs a, r, b, k as they are (RAW).  One: dW, and the
+// tiles, each as the lanes of its products hold it: the transposes of (I - AB)^{-1} and RB (MB), AK and RK (AKR); by rows (over s) dAB and
+// dAK for dA', dRB and dRK for dR'; by columns (over t) dAB and dRB for dB', dAK and dRK for dK'.
 template <bool F32> struct LB {
     static constexpr uint32_t TWO = (sizeof(SmemCB<F32>) + 31) / 32 * 32, EX = F32 ? PLANE3 : TERM;      // from TWO on
-    static constexpr uint32_t RA = 0, U = PAIR3, V = U + PLANE3, DY = V + EX, SLOT = DY + EX;
+    static constexpr uint32_t AR = 0, BK = PAIR3, U = 2 * PAIR3, V = U + PLANE3, DY = V + EX, ES = DY + EX, DWF = ES + 4 * CL * N, RAW = DWF + 4 * CL * N,
+                              RAWB = F32 ? 4 * CL * N : TERM, SLOT = RAW + 4 * RAWB;
     static constexpr uint32_t ONE = TWO + 2 * SLOT;                                                         // from ONE on
-    static constexpr uint32_t BD = 0, KD = PLANE3, DW = 2 * PLANE3, MB = 3 * PLANE3, RKA = MB + TPAIR3;
-    static constexpr uint32_t A_ROWS = RKA + TPAIR3, R_ROWS = A_ROWS + TPAIR3, B_COLS = R_ROWS + TPAIR3, K_COLS = B_COLS + TPAIR3, BYTES = ONE + K_COLS + TPAIR3;
+    static constexpr uint32_t DW = 0, MB = PLANE3, AKR = MB + TPAIR3;
+    static constexpr uint32_t A_ROWS = AKR + TPAIR3, R_ROWS = A_ROWS + TPAIR3, B_COLS = R_ROWS + TPAIR3, K_COLS = B_COLS + TPAIR3, BYTES = ONE + K_COLS + TPAIR3;
 };
 // A lane's addresses in one of the two regions
-struct LaneB { Tr tr; lds_t rows[2], own, pair, own_pair; };
+struct LaneB { Tr tr; lds_t own, pair, own_pair; };
 DEVINL LaneB lane_bases(lds_t base, int l16, int g, int own) {
-    LaneB b{tr_bases(base, l16, g), {base + piece(l16, g), base + (piece(l16, g) ^ 16u)}, base + piece(own, g), base + piece2(l16, g), base + piece2(own, g)};
-    opaque(b.tr.a); opaque(b.tr.b); opaque(b.rows[0]); opaque(b.rows[1]); opaque(b.own); opaque(b.pair); opaque(b.own_pair);
+    LaneB b{tr_bases(base, l16, g), base + piece(own, g), base + piece2(l16, g), base + piece2(own, g)};
+    opaque(b.tr.a); opaque(b.tr.b); opaque(b.own); opaque(b.pair); opaque(b.own_pair);
     return b;
 }
 // The same lane's addresses in another region, d bytes on (modulo 2^32): an addition each, where bases of its own would be spilled
 DEVINL LaneB moved(const LaneB& b, lds_t d) {
-    return {{b.tr.a + d, b.tr.b + d}, {b.rows[0] + d, b.rows[1] + d}, b.own + d, b.pair + d, b.own_pair + d};
+    return {{b.tr.a + d, b.tr.b + d}, b.own + d, b.pair + d, b.own_pair + d};
 }
 // v, dy: four tokens of a channel, and over channels
 template <bool F32> DEVINL auto exact_piece(lds_t a) { if constexpr (F32) return get3(a); else return lds_ld<u32x2>(a); }
@@ -774,12 +790,12 @@ DEVINL f32x4 causal_split(const Tr& o, lds_t a, bool a3, lds_t b, bool b3, bool 
 //          phase 1                          | phase 2                                   | phase 3
 //   A:     state parts of dU, dV of (i)      | dU, dW, dV, state update of (i)           | dAB, dAK of (i), both ways; tile, M of (i + 1)
 //   B:     other tile parts, rest of (i - 1) | dY S0, U dS, V dS, dRB, dRK of (i)        | dW S0, state update, dr of (i)
-//   P:     decay sums, U, v, dy (i + 1)      | fp32 planes (i + 1)                       | other three-term planes (i + 1)
+//   P:     decay sums, U, v, dy (i + 1)      | AR, BK, ES (i + 1)                        | RAW, DWF (i + 1)
 // (the rows of visit i - 1 leave in phase 3, through the two A waves that have no tile there)
 
 // ---- role P: elementwise preparation (lane = channel, tokens 4 wp + e) one visit ahead, and the row-wise output stores
 struct Prep7 { uint32_t nx[7][4]; float nsa[4]; };
-template <bool F32> struct Conv7 { float sg[4], uu[4]; uint32_t pk[6][F32 ? 4 : 2]; };   // sigmoid(w), sa, and r k v a b dy: fp32, or bf16 pairs (tokens 2 z, 2 z + 1)
+template <bool F32> struct Conv7 { float sg[4], uu[4]; Decay lam[4]; uint32_t pk[6][F32 ? 4 : 2]; };   // sigmoid(w), sa, and r k v a b dy: fp32, or bf16 pairs (tokens 2 z, 2 z + 1)
 template <bool F32> DEVINL void bwd_fetch(const Args7c& p, Prep7& x, size_t row0, int wp, int lane, int H, int h) {
     // wave-uniform base (scalar registers) plus a 32-bit lane offset: no 64-bit address per tensor and token in vector registers
     // (the lane part is hidden from the optimiser: it would otherwise turn every tensor-and-token address into a 64-bit
@@ -798,9 +814,13 @@ template <bool F32> DEVINL void bwd_fetch(const Args7c& p, Prep7& x, size_t row0
 }
 // first half of the preparation: the decay of each token, this wave's decay sum; the other inputs are kept packed so that the
 // registers of x are free for the next fetch
-template <bool F32> DEVINL void bwd_convert(float (*part)[N], const Prep7& x, Conv7<F32>& y, int wp, int lane) {
+template <bool F32> DEVINL void bwd_convert(Decay (*part)[N], const Prep7& x, Conv7<F32>& y, int wp, int lane) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) { y.sg[e] = sigmoid_fast(widen<F32>(x.nx[0][e])); y.uu[e] = x.nsa[e]; }
+    for (int e = 0; e < 4; ++e) {
+        y.sg[e] = sigmoid_fast(widen<F32>(x.nx[0][e]));
+        y.lam[e] = decay_of_sig(y.sg[e]);
+        y.uu[e] = x.nsa[e];
+    }
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
         if constexpr (F32) {
@@ -811,9 +831,9 @@ template <bool F32> DEVINL void bwd_convert(float (*part)[N], const Prep7& x, Co
             for (int z = 0; z < 2; ++z) y.pk[k][z] = x.nx[k + 1][2 * z] | (x.nx[k + 1][2 * z + 1] << 16);
         }
     }
-    part[wp][lane] = W_SCALE * ((y.sg[0] + y.sg[1]) + (y.sg[2] + y.sg[3]));
+    part[wp][lane] = sum4(y.lam);
 }
-// second half (after a barrier), in two parts, each with the factors that it needs: the fp32 planes; three-term planes
+// second half (after a barrier), in two parts: what the factors enter; the rest
 template <bool F32> struct In7 {
     const Conv7<F32>& y;
     DEVINL float operator()(int k, int e) const {
@@ -821,43 +841,43 @@ template <bool F32> struct In7 {
         else return (e & 1) ? bf_hi(y.pk[k][e >> 1]) : bf_lo(y.pk[k][e >> 1]);
     }
 };
-template <bool F32> DEVINL void bwd_planes(PlanesB& O, const float (*part)[N], const Conv7<F32>& y, int wp, int lane) {
-    float cm, cl;
-    const float lam[4] = {W_SCALE * y.sg[0], W_SCALE * y.sg[1], W_SCALE * y.sg[2], W_SCALE * y.sg[3]};
-    const Factors f = chunk_factors(lam, part, wp, lane, cm, cl);
-    const In7<F32> in{y};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int t = 4 * wp + e;
-        O.Ap[t][lane] = in(3, e) * f.ea[e];
-        O.Rp[t][lane] = in(0, e) * f.er[e];
-        O.Bp[t][lane] = in(4, e) * f.eb[e];
-        O.Kp[t][lane] = in(1, e) * f.eb[e];
-        O.EA[t][lane] = f.ea[e];
-        O.ER[t][lane] = f.er[e];
-        O.DWF[t][lane] = W_SCALE * y.sg[e] * (1.f - y.sg[e]);
-    }
-    if (wp == 0) { O.d1[lane] = exp_acc(cm); O.d2[lane] = exp_acc(cl - cm); O.dec[lane] = exp_acc(cl); }
-}
-// sb: LDS base, slot: offset of the chunk's copy
-template <bool F32> DEVINL void bwd_planes3(const lds_t sb, const lds_t slot, const float (*part)[N], const Conv7<F32>& y, int wp, int lane) {
+// sb: LDS base, slot: offset of the chunk's copy, dec: of the chunk
+template <bool F32> DEVINL f32x4 bwd_planes(const lds_t sb, const lds_t slot, float* dec, const Decay (*part)[N], const Conv7<F32>& y, int wp, int lane) {
     using O = LB<F32>;
-    float cm, cl;
-    const float lam[4] = {W_SCALE * y.sg[0], W_SCALE * y.sg[1], W_SCALE * y.sg[2], W_SCALE * y.sg[3]};
-    const Factors f = chunk_factors(lam, part, wp, lane, cm, cl);
+    float x[5], i[5];
+    growth<false>(y.lam, part, wp, lane, x, i);
     const In7<F32> in{y};
-    f32x4 as, rs, bd, kd;
+    f32x4 as, rs, bs, ks;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        as[e] = in(3, e) * f.es[e];
-        rs[e] = in(0, e) * (f.es[e] * __expf(lam[e]));
-        bd[e] = in(4, e) * f.ee[e];
-        kd[e] = in(1, e) * f.ee[e];
+        as[e] = in(3, e) * x[e];
+        rs[e] = in(0, e) * x[e + 1];
+        bs[e] = in(4, e) * i[e + 1];
+        ks[e] = in(1, e) * i[e + 1];
     }
-    const lds_t o = sb + O::ONE + piece(lane, wp);
-    // (no factor is above 1: what comes from bf16 inputs stays within bf16's range)
-    put_pair<TERM2>(sb + O::TWO + slot + O::RA + piece2(lane, wp), split3<!F32>(rs), split3<!F32>(as));
-    put3(o + O::BD, split3<!F32>(bd)); put3(o + O::KD, split3<!F32>(kd));
+    // (rounded products: a remainder fused with one would put into the planes what role B's factors do not hold)
+    asm volatile("" : "+v"(as), "+v"(rs), "+v"(bs), "+v"(ks));
+    const lds_t o = sb + O::TWO + slot + piece2(lane, wp);
+    // (x is not above 1: what comes from bf16 inputs stays within bf16's range)
+    put_pair<TERM2>(o + O::AR, split3<!F32>(as), split3<!F32>(rs));
+    put_pair<TERM2>(o + O::BK, split3(bs), split3(ks));
+    if (wp == 3) dec[lane] = x[4];
+    return {x[1], x[2], x[3], x[4]};
+}
+template <bool F32> DEVINL void bwd_planes_rest(const lds_t sb, const lds_t slot, const f32x4& es, const Conv7<F32>& y, int wp, int lane) {
+    using O = LB<F32>;
+    const lds_t o = sb + O::TWO + slot;
+    lds_st<f32x4>(o + O::ES + piece2(lane, wp), es);
+    f32x4 f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f[e] = W_SCALE * y.sg[e] * (1.f - y.sg[e]);
+    lds_st<f32x4>(o + O::DWF + piece2(lane, wp), f);
+    const int k[4] = {3, 0, 4, 1};                       // a, r, b, k
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+        if constexpr (F32) lds_st<u32x4>(o + O::RAW + z * O::RAWB + piece2(lane, wp), u32x4{y.pk[k[z]][0], y.pk[k[z]][1], y.pk[k[z]][2], y.pk[k[z]][3]});
+        else lds_st<u32x2>(o + O::RAW + z * O::RAWB + piece(lane, wp), u32x2{y.pk[k[z]][0], y.pk[k[z]][1]});
+    }
 }
 // U, v and dy, which no factor enters
 template <bool F32> DEVINL void bwd_planes_raw(const lds_t sb, const lds_t slot, const Conv7<F32>& y, int wp, int lane) {
@@ -891,41 +911,75 @@ DEVINL void store_f32(uint16_t* dst, size_t first, uint32_t o, float x) {
     *reinterpret_cast<float*>(reinterpret_cast<char*>(dst) + first * 4 + o * 4u) = x;
 }
 template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const lds_t sb, const Args7c& p, int tid, int w, size_t tok0, int nch, int H, int h) {
-    const int lane = tid & 63, wp = w - 8, tp = tid - 8 * 64;
+    const int lane = tid & 63, wp = w - 8;
     // Raw rows are asked for two visits before they are converted (one visit, of which only two phases lie between the
     // request and the use, is less than the memory system takes under load: the A and B waves then waited for the P waves
     // at two of the three barriers of every visit).  Two register sets take turns; the chunk index is clamped instead of
     // the request being skipped, so that every visit issues the same loads and the waits count the same.
     Prep7 x[2];
     Conv7<F32> y;
+    const int l16 = lane & 15, g = lane >> 4;
+    using L = LB<F32>;
+    const lds_t tp = tr_pair(sb, l16, g);
+    // a causal tile of a visit
+    auto tile = [&](const int visit) __attribute__((always_inline)) {
+        const lds_t at = tp + L::TWO + (visit & 1) * L::SLOT;
+        return causal_tile<false>([&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, at + (wp < 2 ? L::AR : L::AR + 8), hb); },
+                                  [&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, at + (wp & 1 ? L::BK + 8 : L::BK), hb); }, wp < 2, l16, g);
+    };
+    // its place, of AB the inverse's
+    auto put_tile = [&](const f32x4& acc) __attribute__((always_inline)) {
+        f32x4 x = acc;
+        if (wp == 0) {                           // this wave wrote AB itself: LDS keeps a wave's accesses in order
+#pragma unroll
+            for (int v = 0; v < 4; ++v) S.AB[4 * g + v][l16] = acc[v] * UNHOLD;
+            float m[CL];
+            inverse_cols(S.AB, l16, m);
+                x = by_group(g, m);
+        }
+        // (one store with a selected address: with one in each of the branches the compiler merged them and left the address undefined
+        // on one way there)
+        put_half<TTERM2>(sb + L::ONE + piece2(l16, g) + (wp == 0 ? L::MB : (wp == 1 ? L::AKR : (wp == 2 ? L::MB + 8 : L::AKR + 8))), split3(x));
+    };
     auto row_of = [&](int visit) { const int c = nch - 1 - visit; return tok0 + static_cast<size_t>(c > 0 ? c : 0) * CL; };
     bwd_fetch<F32>(p, x[0], row_of(0), wp, lane, H, h);
     bwd_fetch<F32>(p, x[1], row_of(1), wp, lane, H, h);
     bwd_convert(S.part, x[0], y, wp, lane);           // visit 0, before the loop
     bwd_fetch<F32>(p, x[0], row_of(2), wp, lane, H, h);
     __syncthreads();
-    bwd_planes<F32>(S.pl[0], S.part, y, wp, lane);
-    bwd_planes3<F32>(sb, 0, S.part, y, wp, lane);
+    bwd_planes_rest<F32>(sb, 0, bwd_planes<F32>(sb, 0, S.dec[0], S.part, y, wp, lane), y, wp, lane);
     bwd_planes_raw<F32>(sb, 0, y, wp, lane);
     __syncthreads();
+    put_tile(tile(0));
+    if (nch > 1) bwd_convert(S.part, x[1], y, wp, lane);
+    bwd_fetch<F32>(p, x[1], row_of(3), wp, lane, H, h);
+    __syncthreads();
     auto visit = [&](const int i, auto Z) __attribute__((always_inline)) {     // visit i is chunk nch - 1 - i
-        constexpr int z = decltype(Z)::value;        // the set that holds visit i + 1
+        constexpr int z = decltype(Z)::value;        // the set that holds visit i + 2
         const bool next = i + 1 < nch;
-        if (next) bwd_convert(S.part, x[z], y, wp, lane);
-        bwd_fetch<F32>(p, x[z], row_of(i + 3), wp, lane, H, h);
-        if (next) bwd_planes_raw<F32>(sb, ((i + 1) & 1) * LB<F32>::SLOT, y, wp, lane);
+        const lds_t slot = ((i + 1) & 1) * L::SLOT;
+        f32x4 es = ZERO4, t = ZERO4;
+        if (next) {
+            es = bwd_planes<F32>(sb, slot, S.dec[(i + 1) & 1], S.part, y, wp, lane);
+            bwd_planes_raw<F32>(sb, slot, y, wp, lane);
+        }
         __syncthreads();
-        if (next) bwd_planes<F32>(S.pl[(i + 1) & 1], S.part, y, wp, lane);
+        if (next) {
+            t = tile(i + 1);
+            bwd_planes_rest<F32>(sb, slot, es, y, wp, lane);
+        }
         __syncthreads();
-        if (next) bwd_planes3<F32>(sb, ((i + 1) & 1) * LB<F32>::SLOT, S.part, y, wp, lane);
+        if (next) put_tile(t);
+        if (i + 2 < nch) bwd_convert(S.part, x[z], y, wp, lane);
+        bwd_fetch<F32>(p, x[z], row_of(i + 4), wp, lane, H, h);
         __syncthreads();
     };
     for (int i = 0; i < nch; i += 2) {
-        visit(i, std::integral_constant<int, 1>{});
-        if (i + 1 < nch) visit(i + 1, std::integral_constant<int, 0>{});
+        visit(i, std::integral_constant<int, 0>{});
+        if (i + 1 < nch) visit(i + 1, std::integral_constant<int, 1>{});
     }
     __syncthreads();                                 // role B finishes the last chunk
-    if constexpr (!F32) bwd_store_rows(S, (nch - 1) & 1, p, tok0, tp, H, h);
+    if constexpr (!F32) bwd_store_rows(S, (nch - 1) & 1, p, tok0, tid - 8 * 64, H, h);
 }
 
 template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const Args7c& p, const float* dsT, float* ds0, int tid, int w, int nch, size_t tok0, int H, int h) {
@@ -938,49 +992,46 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
     using L = LB<F32>;
     const LaneB one = lane_bases(sb + L::ONE, l16, g, own);
     const Tr base_tr = tr_bases(sb, l16, g);
-    // a causal tile of a visit, and M
-    auto tiles = [&](const PlanesB& O) __attribute__((always_inline)) {
-        const f32x4 acc = causal_acc<false>(q < 2 ? O.Ap : O.Rp, (q & 1) ? O.Kp : O.Bp, q < 2, l16, g);
-        f32x4 x = acc;
-        if (q == 0) {                            // this wave wrote AB itself: LDS keeps a wave's accesses in order
-#pragma unroll
-            for (int v = 0; v < 4; ++v) S.AB[4 * g + v][l16] = acc[v];
-            float m[CL];
-            inverse_cols(S.AB, l16, m);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) x[v] = by_group(g, m[v], m[4 + v], m[8 + v], m[12 + v]);
-        }
-        // (one store with a selected address: with one in each of the branches the compiler merged them and left the address undefined
-        // on one way there)
-        put_half<TTERM2>(one.pair + (q == 0 ? L::MB : (q == 1 ? L::RKA + 8 : (q == 2 ? L::MB + 8 : L::RKA))), split3(x));
-    };
+    const lds_t tp = tr_pair(sb, l16, g);
     __syncthreads();
     __syncthreads();
-    tiles(S.pl[0]);
+    __syncthreads();
     for (int i = 0; i < nch; ++i) {
-        const PlanesB& O = S.pl[i & 1];
         const LaneB two = moved(one, L::TWO + (i & 1) * L::SLOT - L::ONE);
+        const float* const dec = &S.dec[i & 1][4 * g];
         // ---------------------------------------------------------------- phase 1: the parts of dU, dV that need no tile
-        Sum2 dUs = SUM0, dVs = SUM0;
+        Sum2 dUs = SUM0, dVs = SUM0;                     // HOLD dU, HOLD dV
+        const lds_t bk = tp + L::TWO + (i & 1) * L::SLOT + L::BK;
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
-            const Op3 st = join(split3(dS[2 * hb]), split3(dS[2 * hb + 1]));
-            add32(dUs, get3_tr(L::BD, one.tr, hb), st);
-            add32(dVs, get3_tr(L::KD, one.tr, hb), st);
+            // (decayed for these products only: in the update a fused multiplication and addition rounds the state once)
+            const Op3 st = join(split3(dS[2 * hb] * ld4(dec + 32 * hb)), split3(dS[2 * hb + 1] * ld4(dec + 32 * hb + 16)));
+            add32(dUs, get3_tr_pair(0, bk, hb), st);
+            add32(dVs, get3_tr_pair(8, bk, hb), st);
         }
         here(dUs); here(dVs);
+        // dRB (q even), dRK, by rows and by columns; their places are free after the barrier
+        const bool byrow = q < 2;
+        const lds_t uv = L::TWO + (i & 1) * L::SLOT + (q & 1 ? L::V : L::U);
+        const bool uv3 = F32 || (q & 1) == 0;
+        f32x4 dr;
+        {
+            const lds_t y = L::TWO + (i & 1) * L::SLOT + L::DY;
+            dr = causal_split(base_tr, byrow ? uv : y, byrow ? uv3 : F32, byrow ? y : uv, byrow ? F32 : uv3, byrow, false, l16, g);
+            asm volatile("" : "+v"(dr));
+        }
         __syncthreads();
         // ---------------------------------------------------------------- phase 2: dU, dW = M^T dU, dV, the gradient state
         {
             const auto dyop = exact_piece<F32>(two.own + L::DY);             // dY[tau = 4 g + v][i]
             add16(dUs, get_half<TTERM2>(one.pair + L::MB + 8), dyop);
             Sum2 dWs = SUM0;
-            add16(dWs, get_half<TTERM2>(one.pair + L::MB), split3(total(dUs)));
+            add16(dWs, get_half<TTERM2>(one.pair + L::MB), split3(total(dUs) * UNHOLD));
             const B3 dW = split3(total(dWs));
             put3(one.own + L::DW, dW);
-            const Op3 yw = join(as3(dyop), dW);          // dY and dW share the instructions of what follows
-            add32(dVs, get_pair<TTERM2>(one.pair + L::RKA), yw);
-            const f32x4 dV = total(dVs);
+            const Op3 wy = join(dW, as3(dyop));          // dW and dY share the instructions of what follows
+            add32(dVs, get_pair<TTERM2>(one.pair + L::AKR), wy);
+            const f32x4 dV = total(dVs) * UNHOLD;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 if constexpr (F32) store_f32(p.dv, ((tok0 + static_cast<size_t>(nch - 1 - i) * CL) * H + h) * N, static_cast<uint32_t>((4 * g + v) * H) * N + own, dV[v]);
@@ -989,28 +1040,22 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
 #pragma unroll
             for (int jt = 0; jt < 4; ++jt) {
                 Sum2 x = SUM0;
-                add32(x, get_pair<TERM2>(two.pair + L::RA + 1024 * jt), yw);
-                dS[jt] = dS[jt] * ld4(&O.dec[16 * jt + 4 * g]) + total(x);
+                add32(x, get_pair<TERM2>(two.pair + L::AR + 1024 * jt), wy);
+                dS[jt] = dS[jt] * ld4(dec + 16 * jt) + total(x);
             }
+            put_half<TTERM2>(one.pair + (q == 0 ? L::R_ROWS : (q == 1 ? L::R_ROWS + 8 : (q == 2 ? L::B_COLS + 8 : L::K_COLS + 8))), split3(dr));
         }
         __syncthreads();
         // ---------------------------------------------------------------- phase 3: dAB (q even), dAK (they need dW), by rows and by columns
         {
-            const lds_t w = L::ONE + L::DW, o = L::TWO + (i & 1) * L::SLOT + (q & 1 ? L::V : L::U);
-            const bool o3 = F32 || (q & 1) == 0, byrow = q < 2;
-            const f32x4 t = causal_split(base_tr, byrow ? o : w, byrow ? o3 : true, byrow ? w : o, byrow ? true : o3, byrow, true, l16, g);
+            const lds_t w = L::ONE + L::DW;
+            const f32x4 t = causal_split(base_tr, byrow ? uv : w, byrow ? uv3 : true, byrow ? w : uv, byrow ? true : uv3, byrow, true, l16, g);
             put_half<TTERM2>(one.pair + (q == 0 ? L::A_ROWS : (q == 1 ? L::A_ROWS + 8 : (q == 2 ? L::B_COLS : L::K_COLS))), split3(t));
         }
-        if (i + 1 < nch) tiles(S.pl[(i + 1) & 1]);
+        // These waves carry the finished rows of the visit before to global memory (parked by the B waves in phase 1, dv by this role one
+        // visit earlier; both stay as they are until the next visit).
         if constexpr (!F32) {
-          if (q >= 2 && i > 0) {
-            // Two waves carry the finished rows of the visit before to global memory (parked by the
-            // B waves in phase 1, dv by this role one visit earlier; both stay as they are until the next visit): the P
-            // waves, for which this was a third of a phase that everybody waits for, keep to loads.
-            const int tp = tid - 2 * 64;
-            bwd_store_rows(S, (i - 1) & 1, p, tok0 + static_cast<size_t>(nch - i) * CL, tp, H, h);
-            bwd_store_rows(S, (i - 1) & 1, p, tok0 + static_cast<size_t>(nch - i) * CL, tp + 128, H, h);
-          }
+            if (i > 0) bwd_store_rows(S, (i - 1) & 1, p, tok0 + static_cast<size_t>(nch - i) * CL, tid, H, h);
         }
         __syncthreads();
     }
@@ -1051,16 +1096,18 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
 #pragma unroll
             for (int v = 0; v < 4; ++v) S0b[ib][v] = *reinterpret_cast<const float*>(at + (16 * ib + v) * N * 4 + o);
     };
-    // fp32 planes of a visit, element [4 g + v][own] of plane k; d1, d2, dec of the own channel; parked outputs
-    lds_t fl = sb + static_cast<uint32_t>(4 * g * PS + own) * 4, cl = sb + 7 * 4 * CL * PS + 4 * own;
-    [[maybe_unused]] lds_t park = sb + static_cast<uint32_t>(offsetof(SmemCB<F32>, park)) + static_cast<uint32_t>(4 * g * PK + own) * 2;
-    opaque(fl); opaque(cl); opaque(park);
-    auto planes_of = [&](int visit) __attribute__((always_inline)) { return static_cast<lds_t>((visit & 1) * sizeof(PlanesB)); };
-    auto plane = [&](lds_t O, int k, int v) __attribute__((always_inline)) { return lds_ld<float>(fl + O + 4 * PS * (CL * k + v)); };
-    auto chan = [&](lds_t O, int k) __attribute__((always_inline)) { return lds_ld<float>(cl + O + 4 * N * k); };
+    [[maybe_unused]] lds_t park = sb + static_cast<uint32_t>(offsetof(SmemCB<F32>, park)) + static_cast<uint32_t>(4 * g * PK + own) * 2;      // parked outputs
+    opaque(park);
+    // (addresses worked out where they are used: kept in registers, others go to scratch)
+    auto decay_of = [&](int visit) __attribute__((always_inline)) {
+        return lds_ld<float>(sb + static_cast<uint32_t>(offsetof(SmemCB<F32>, dec)) + 64 * q + (visit & 1) * 4 * N + 4 * (lane_again() & 15));
+    };
+    // piece of channel l16; of channel 16 ib + l16, 512 ib on, it is turned by two groups where ib is odd
+    auto rows = [&]() __attribute__((always_inline)) { const uint32_t me = lane_again(); return piece(me & 15, me >> 4); };
+    auto copy_of = [&](int visit) __attribute__((always_inline)) { return static_cast<lds_t>(L::TWO + (visit & 1) * L::SLOT); };
     float Pj = 0.f;                                  // P at the end of the chunk that is finished next
     f32x4 xA = ZERO4, xB = ZERO4, xK = ZERO4, dRp = ZERO4;    // state parts of dA', dB', dK', and dR', carried into the next visit's phase 1
-    Op3 bk;                                          // and B', K' as an operand
+    Op3 ar, bk;                                      // and the planes of the own channel, whose places the P waves fill anew there
     // a contraction over 16 with a pair of tiles (one after the other: the registers do not hold the operands of all of them)
     auto tile2 = [&](uint32_t pair, const Op3& b) __attribute__((always_inline)) {
         Sum2 s = SUM0;
@@ -1068,8 +1115,8 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         __builtin_amdgcn_sched_barrier(0);
         return total(s);
     };
-    // tile parts, scaling, decay gradient of the chunk whose planes are O and whose first row is row0; results parked as bf16
-    auto finish = [&](const lds_t O, const size_t row0) __attribute__((always_inline)) {
+    // tile parts, scaling, decay gradient of the chunk of a visit, whose first row is row0; results parked as bf16
+    auto finish = [&](const int visit, const size_t row0) __attribute__((always_inline)) {
         const uint32_t me = lane_again();
         [[maybe_unused]] const uint32_t lo = (me >> 4) * static_cast<uint32_t>(4 * H * N) + 16 * q + (me & 15);
         [[maybe_unused]] const size_t first = (row0 * H + h) * N;
@@ -1077,34 +1124,42 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             if constexpr (F32) store_f32(dst, first, lo + static_cast<uint32_t>(v * H) * N, x);
             else lds_st<uint16_t>(park + 2 * PK * (CL * k + v), f2bf(x));
         };
-        const float d1j = chan(O, 0), d2j = chan(O, 1);
-        f32x4 bp, kp, ap, rp;                        // planes at [s or t = 4 g + v][j]
-#pragma unroll
-        for (int v = 0; v < 4; ++v) { bp[v] = plane(O, 2, v); kp[v] = plane(O, 3, v); ap[v] = plane(O, 0, v); rp[v] = plane(O, 1, v); }
+        const lds_t two = one.own_pair - L::ONE + copy_of(visit);
         const f32x4 tA = tile2(L::A_ROWS, bk);
-        const Op3 ar = join(split3(ap), split3(rp));
         const f32x4 tB = tile2(L::B_COLS, ar), tK = tile2(L::K_COLS, ar);
-        float del[4], ada[4], dwf[4];
+        const f32x4 es = lds_ld<f32x4>(two + L::ES), dwf = lds_ld<f32x4>(two + L::DWF);
+        // e^{c_t} of the token before the lane's four (of the first four it is 1)
+        float ea = lds_ld<float>(sb + copy_of(visit) + L::ES + 12 + piece2(16 * q + (me & 15), me > 15 ? (me >> 4) - 1 : 0));
+        if (me < 16) ea = 1.f;
+        std::conditional_t<F32, f32x4, u32x2> raw[4];
+#pragma unroll
+        for (int z = 0; z < 4; ++z) {
+            if constexpr (F32) raw[z] = lds_ld<f32x4>(two + L::RAW + z * L::RAWB);
+            else raw[z] = lds_ld<u32x2>(one.own - L::ONE + copy_of(visit) + L::RAW + z * L::RAWB);
+        }
+        auto input = [&](const int z, const int v) __attribute__((always_inline)) {
+            if constexpr (F32) return raw[z][v];
+            else return v & 1 ? bf_hi(raw[z][v >> 1]) : bf_lo(raw[z][v >> 1]);
+        };
+        float del[4], ada[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const float dAp = fmaf(d1j, xA[v], tA[v]);
-            const float dBp = fmaf(d2j, xB[v], tB[v]), dKp = fmaf(d2j, xK[v], tK[v]);
-            const float ea = plane(O, 4, v), er = plane(O, 5, v);
-            float eb = __builtin_amdgcn_rcpf(er);                               // (er is between e^-4.9 and e^4.9)
-            eb = fmaf(fmaf(-er, eb, 1.f), eb, eb);
+            const float dAp = fmaf(UNHOLD, tA[v], xA[v]), dBp = tB[v] + xB[v], dKp = tK[v] + xK[v];
+            const float er = es[v], hb = held_inverse(er), eb = hb * UNHOLD;
             put(0, p.da, v, dAp * ea);
             put(1, p.dr, v, dRp[v] * er);
             put(2, p.db, v, dBp * eb);
             put(3, p.dk, v, dKp * eb);
-            ada[v] = ap[v] * dAp;
-            del[v] = fmaf(rp[v], dRp[v], -fmaf(bp[v], dBp, kp[v] * dKp));      // r dr - b db - k dk
-            dwf[v] = plane(O, 6, v);
+            // a da;  r dr - b db - k dk, of the values that the tiles' planes hold: what of one is in another cancels in the sums below
+            ada[v] = (input(0, v) * ea) * dAp;
+            del[v] = fmaf(input(1, v) * er, dRp[v], -UNHOLD * fmaf(input(2, v) * hb, dBp, (input(3, v) * hb) * dKp));
+            ea = er;
         }
         // G_t = P_{t+1} + del_t,  P_t = G_t + a da:  suffix sums over t = 4 g + v, later lane groups first
         const float tot = (del[0] + ada[0]) + (del[1] + ada[1]) + (del[2] + ada[2]) + (del[3] + ada[3]);
         auto of_lane = [](uint32_t l, float x) __attribute__((always_inline)) { return __int_as_float(__builtin_amdgcn_ds_bpermute(static_cast<int>(4 * l), __float_as_int(x))); };
         const float t1 = of_lane(me + 16, tot), t2 = of_lane(me + 32, tot), t3 = of_lane(me + 48, tot);
-        float Pn = Pj + (g < 3 ? t1 : 0.f) + (g < 2 ? t2 : 0.f) + (g < 1 ? t3 : 0.f);     // P after this lane's last token
+        float Pn = Pj + (me < 48 ? t1 : 0.f) + (me < 32 ? t2 : 0.f) + (me < 16 ? t3 : 0.f);     // P after this lane's last token
 #pragma unroll
         for (int v = 3; v >= 0; --v) {
             const float G = Pn + del[v];
@@ -1116,25 +1171,26 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     fetch_state(nch - 1);
     __syncthreads();
     __syncthreads();
+    __syncthreads();
     for (int i = 0; i < nch; ++i) {
         const int c = nch - 1 - i;
-        const lds_t O = planes_of(i);
-        const LaneB two = moved(one, L::TWO + (i & 1) * L::SLOT - L::ONE);
+        const LaneB two = moved(one, copy_of(i) - L::ONE);
         // ---------------------------------------------------------------- phase 1: finish the previous visit's chunk
-        if (i > 0) finish(planes_of(i - 1), tok0 + static_cast<size_t>(c + 1) * CL);
+        if (i > 0) finish(i - 1, tok0 + static_cast<size_t>(c + 1) * CL);
         else if (dsT != nullptr) {
-            // P at the end of the call: sum_i dsT o S_T with S_T = S0 dec + U^T (B' d2) + V^T (K' d2) of the last chunk
-            const float decj = chan(O, 2);
-            const Op3 bdk = join(get3(one.own + L::BD), get3(one.own + L::KD));
+            // P at the end of the call: sum_i dsT o S_T with S_T = (S0 + U^T (b e^{-c_{s+1}}) + V^T (k e^{-c_{s+1}})) dec of the last chunk
+            const float decj = decay_of(i);
+            const Op3 bk = get_pair<TERM2>(two.own_pair + L::BK);
+            const lds_t row = rows();
             float pp = 0.f;
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) {
-                const lds_t o = two.rows[ib & 1] + 512 * ib;
+                const lds_t o = sb + copy_of(i) + (row ^ (ib & 1 ? 16u : 0u)) + 512 * ib;
                 Sum2 x = SUM0;
-                add32(x, join(get3(o + L::U), as3(exact_piece<F32>(o + L::V))), bdk);
+                add32(x, join(get3(o + L::U), as3(exact_piece<F32>(o + L::V))), bk);
                 const f32x4 acc = total(x);
 #pragma unroll
-                for (int v = 0; v < 4; ++v) pp = fmaf(dS[ib][v], fmaf(S0b[ib][v], decj, acc[v]), pp);
+                for (int v = 0; v < 4; ++v) pp = fmaf(dS[ib][v], fmaf(acc[v], UNHOLD, S0b[ib][v]) * decj, pp);
             }
             pp += __shfl_xor(pp, 16, 64);
             pp += __shfl_xor(pp, 32, 64);
@@ -1149,52 +1205,45 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         f32x4 xR;
         {
             Sum2 pr = SUM0, pb = SUM0, pk = SUM0;
+            const float decj = decay_of(i);
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb) {
                 s0[hb] = join(split3(S0b[2 * hb]), split3(S0b[2 * hb + 1]));
-                const Op3 ds = join(split3(dS[2 * hb]), split3(dS[2 * hb + 1]));
+                const Op3 ds = join(split3(dS[2 * hb] * decj), split3(dS[2 * hb + 1] * decj));
                 add32(pr, ya(hb), s0[hb]);
                 add32(pb, ua(hb), ds);
                 add32(pk, va(hb), ds);
             }
             xR = total(pr); xB = total(pb); xK = total(pk);
         }
-        {
-            const lds_t copy = L::TWO + (i & 1) * L::SLOT, y = copy + L::DY, o = copy + (q & 1 ? L::V : L::U);
-            const bool o3 = F32 || (q & 1) == 0, byrow = q < 2;
-            const f32x4 t = causal_split(base_tr, byrow ? o : y, byrow ? o3 : F32, byrow ? y : o, byrow ? F32 : o3, byrow, false, l16, g);
-            put_half<TTERM2>(one.pair + (q == 0 ? L::R_ROWS : (q == 1 ? L::R_ROWS + 8 : (q == 2 ? L::B_COLS + 8 : L::K_COLS + 8))), split3(t));
-        }
         __syncthreads();
         // ---------------------------------------------------------------- phase 3: dW S0; the gradient state
         {
-            const float decj = chan(O, 2);
-            const Op3 ra = get_pair<TERM2>(two.own_pair + L::RA);
+            const float decj = decay_of(i);
+            ar = get_pair<TERM2>(two.own_pair + L::AR);
             Sum2 pa = SUM0;
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb) add32(pa, get3_tr(L::DW, one.tr, hb), s0[hb]);
             xA = total(pa);
+            const lds_t row = rows();
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) {
                 Sum2 x = SUM0;
-                add32(x, join(as3(exact_piece<F32>(two.rows[ib & 1] + 512 * ib + L::DY)), get3(one.rows[ib & 1] + 512 * ib + L::DW)), ra);
+                const lds_t o = (row ^ (ib & 1 ? 16u : 0u)) + 512 * ib;
+                add32(x, join(get3(sb + L::ONE + o + L::DW), as3(exact_piece<F32>(sb + copy_of(i) + o + L::DY))), ar);
                 dS[ib] = dS[ib] * decj + total(x);
             }
-            // dR' needs no tile of this phase; B', K' stay for dA'
-            f32x4 bp, kp;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) { bp[v] = plane(O, 2, v); kp[v] = plane(O, 3, v); }
-            bk = join(split3(bp), split3(kp));
+            // dR' needs no tile of this phase
+            bk = get_pair<TERM2>(two.own_pair + L::BK);
             const f32x4 tR = tile2(L::R_ROWS, bk);
-            const float d1j = chan(O, 0);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) dRp[v] = fmaf(d1j, xR[v], tR[v]);
+            for (int v = 0; v < 4; ++v) dRp[v] = fmaf(UNHOLD, tR[v], xR[v]);
             if (c > 0) fetch_state(c - 1);
         }
         __syncthreads();
     }
     opaque(one.pair);                                // (or the tiles' addresses are kept from before the loop, in scratch)
-    finish(planes_of(nch - 1), tok0);
+    finish(nch - 1, tok0);
     __syncthreads();
 }
 
@@ -1211,9 +1260,11 @@ __global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c args) {
     const size_t tok0 = static_cast<size_t>(b) * p.T + x.first * CL;
     const int nch = x.chunks, all = p.T / CL;
     const lds_t sb = lds_of(smem_raw);
-    if (w >= 8) { bwd_role_p(S, sb, p, tid, w, tok0, nch, p.H, h); return; }
+    // (thread numbers anew: role B has no register to hold one across its loop for the code of the others, which lies behind)
+    const auto again = [&]() __attribute__((always_inline)) { return 64 * w + static_cast<int>(lane_again()); };
+    if (w >= 8) { bwd_role_p(S, sb, p, again(), w, tok0, nch, p.H, h); return; }
     const float* const dsT = x.first + nch < all ? p.enter + (bh * (p.NB - 1) + p.NB - 2 - x.n) * N * N : (p.dsT != nullptr ? p.dsT + bh * N * N : nullptr);
-    if (w < 4) bwd_role_a(S, sb, p, dsT, p.ds0 != nullptr && x.n == 0 ? p.ds0 + bh * N * N : nullptr, tid, w, nch, tok0, p.H, h);
+    if (w < 4) bwd_role_a(S, sb, p, dsT, p.ds0 != nullptr && x.n == 0 ? p.ds0 + bh * N * N : nullptr, again(), w, nch, tok0, p.H, h);
     else bwd_role_b(S, sb, p, dsT, p.s + (bh * all + x.first) * N * N, tid, w, nch, tok0, p.H, h);
 }
 
