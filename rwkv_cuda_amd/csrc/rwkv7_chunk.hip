@@ -728,17 +728,26 @@ struct SmemCB {
     uint16_t park[F32 ? 1 : 5][F32 ? 1 : CL][F32 ? 1 : PK];                                // da, dr, db, dk, dw of the chunk that role B finished last, [token][channel]
     uint16_t parkv[F32 ? 1 : 2][F32 ? 1 : CL][F32 ? 1 : PK];                               // dv, which is ready one visit earlier than the other five
 };
+// A 64 x 64 matrix in bf16 terms, [i][j]: pieces of four j, turned by the row so that the writing lanes (16 rows by four pieces) and the
+// transposing reads (8 rows of four pieces) meet every bank once.  i: of the first 16 rows, the others 2048 bytes on each
+constexpr uint32_t DTERM = 64 * 128;
+DEVINL lds_t square(int i, int piece) { return static_cast<lds_t>(128 * i + 8 * (piece ^ (4 * ((i >> 1) & 3)) ^ (2 * ((i >> 3) & 1)))); }
+DEVINL bf16x8 tr16_square(lds_t o, int hb) {       // rows 32 hb + 16 (e >> 2) + 4 g + (e & 3) of a column
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    typedef v4s __attribute__((address_space(3))) * ptr;
+    const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + 4096 * hb)), y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + 4096 * hb + 2048));
+    return op2(__builtin_bit_cast(u32x2, x), __builtin_bit_cast(u32x2, y));
+}
 // Planes and tiles behind it.  Two copies, of which the P waves fill one while the A and B waves work on the other: a e^{c_t} and
 // r e^{c_{t+1}} (AR), b and k times HOLD e^{-c_{s+1}} (BK), U, v and dy (one term each where they are bf16) in three terms; fp32, 16 bytes of
-// four tokens as the pairs lie: e^{c_{t+1}} (ES), W_SCALE sig (1 - sig) (DWF); inputs a, r, b, k as they are (RAW).  One: dW, and the
+// four tokens as the pairs lie: e^{c_{t+1}} (ES), W_SCALE sig (1 - sig) (DWF).  One: dS with the chunk's decay on it, in three terms (DS), dW, and the
 // tiles, each as the lanes of its products hold it: the transposes of (I - AB)^{-1} and RB (MB), AK and RK (AKR); by rows (over s) dAB and
 // dAK for dA', dRB and dRK for dR'; by columns (over t) dAB and dRB for dB', dAK and dRK for dK'.
 template <bool F32> struct LB {
     static constexpr uint32_t TWO = (sizeof(SmemCB<F32>) + 31) / 32 * 32, EX = F32 ? PLANE3 : TERM;      // from TWO on
-    static constexpr uint32_t AR = 0, BK = PAIR3, U = 2 * PAIR3, V = U + PLANE3, DY = V + EX, ES = DY + EX, DWF = ES + 4 * CL * N, RAW = DWF + 4 * CL * N,
-                              RAWB = F32 ? 4 * CL * N : TERM, SLOT = RAW + 4 * RAWB;
-    static constexpr uint32_t ONE = TWO + 2 * SLOT;                                                         // from ONE on
-    static constexpr uint32_t DW = 0, MB = PLANE3, AKR = MB + TPAIR3;
+    static constexpr uint32_t AR = 0, BK = PAIR3, U = 2 * PAIR3, V = U + PLANE3, DY = V + EX, ES = DY + EX, DWF = ES + 4 * CL * N, SLOT = DWF + 4 * CL * N;
+    static constexpr uint32_t ONE = (TWO + 2 * SLOT + 127) / 128 * 128;                                     // from ONE on
+    static constexpr uint32_t DS = 0, DW = 3 * DTERM, MB = DW + PLANE3, AKR = MB + TPAIR3;
     static constexpr uint32_t A_ROWS = AKR + TPAIR3, R_ROWS = A_ROWS + TPAIR3, B_COLS = R_ROWS + TPAIR3, K_COLS = B_COLS + TPAIR3, BYTES = ONE + K_COLS + TPAIR3;
 };
 // A lane's addresses in one of the two regions
@@ -872,12 +881,6 @@ template <bool F32> DEVINL void bwd_planes_rest(const lds_t sb, const lds_t slot
 #pragma unroll
     for (int e = 0; e < 4; ++e) f[e] = W_SCALE * y.sg[e] * (1.f - y.sg[e]);
     lds_st<f32x4>(o + O::DWF + piece2(lane, wp), f);
-    const int k[4] = {3, 0, 4, 1};                       // a, r, b, k
-#pragma unroll
-    for (int z = 0; z < 4; ++z) {
-        if constexpr (F32) lds_st<u32x4>(o + O::RAW + z * O::RAWB + piece2(lane, wp), u32x4{y.pk[k[z]][0], y.pk[k[z]][1], y.pk[k[z]][2], y.pk[k[z]][3]});
-        else lds_st<u32x2>(o + O::RAW + z * O::RAWB + piece(lane, wp), u32x2{y.pk[k[z]][0], y.pk[k[z]][1]});
-    }
 }
 // U, v and dy, which no factor enters
 template <bool F32> DEVINL void bwd_planes_raw(const lds_t sb, const lds_t slot, const Conv7<F32>& y, int wp, int lane) {
@@ -968,9 +971,9 @@ template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const lds_t sb, const
             t = tile(i + 1);
             bwd_planes_rest<F32>(sb, slot, es, y, wp, lane);
         }
+        if (i + 2 < nch) bwd_convert(S.part, x[z], y, wp, lane);
         __syncthreads();
         if (next) put_tile(t);
-        if (i + 2 < nch) bwd_convert(S.part, x[z], y, wp, lane);
         bwd_fetch<F32>(p, x[z], row_of(i + 4), wp, lane, H, h);
         __syncthreads();
     };
@@ -993,8 +996,24 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
     const LaneB one = lane_bases(sb + L::ONE, l16, g, own);
     const Tr base_tr = tr_bases(sb, l16, g);
     const lds_t tp = tr_pair(sb, l16, g);
+    const lds_t sq = sb + L::ONE + L::DS + square(own, g);
+    auto put_square = [&](int jt, const B3& x) __attribute__((always_inline)) {
+        const lds_t o = sq ^ (32u * jt);             // (128-byte rows, and the piece's upper bits are turned by exclusive or)
+        lds_st<u32x2>(o, x.h); lds_st<u32x2>(o + DTERM, x.m); lds_st<u32x2>(o + 2 * DTERM, x.l);
+    };
+    // dRB (q odd), dRK, by rows and by columns, of a visit, made in the one before.  (With U, the longer ones where v is one term, on the odd
+    // waves: the inverse runs beside wave 0.)
+    const bool byrow = q < 2, uv3 = F32 || (q & 1) != 0;
+    auto uv_of = [&](int visit) __attribute__((always_inline)) { return L::TWO + (visit & 1) * L::SLOT + (q & 1 ? L::U : L::V); };
+    auto dr_tile = [&](int visit) __attribute__((always_inline)) {
+        const lds_t y = L::TWO + (visit & 1) * L::SLOT + L::DY, uv = uv_of(visit);
+        f32x4 t = causal_split(base_tr, byrow ? uv : y, byrow ? uv3 : F32, byrow ? y : uv, byrow ? F32 : uv3, byrow, false, l16, g);
+        asm volatile("" : "+v"(t));
+        return t;
+    };
     __syncthreads();
     __syncthreads();
+    f32x4 dr = dr_tile(0);
     __syncthreads();
     for (int i = 0; i < nch; ++i) {
         const LaneB two = moved(one, L::TWO + (i & 1) * L::SLOT - L::ONE);
@@ -1005,21 +1024,13 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
             // (decayed for these products only: in the update a fused multiplication and addition rounds the state once)
-            const Op3 st = join(split3(dS[2 * hb] * ld4(dec + 32 * hb)), split3(dS[2 * hb + 1] * ld4(dec + 32 * hb + 16)));
+            const B3 s0 = split3(dS[2 * hb] * ld4(dec + 32 * hb)), s1 = split3(dS[2 * hb + 1] * ld4(dec + 32 * hb + 16));
+            put_square(2 * hb, s0); put_square(2 * hb + 1, s1);      // for role B
+            const Op3 st = join(s0, s1);
             add32(dUs, get3_tr_pair(0, bk, hb), st);
             add32(dVs, get3_tr_pair(8, bk, hb), st);
         }
         here(dUs); here(dVs);
-        // dRB (q even), dRK, by rows and by columns; their places are free after the barrier
-        const bool byrow = q < 2;
-        const lds_t uv = L::TWO + (i & 1) * L::SLOT + (q & 1 ? L::V : L::U);
-        const bool uv3 = F32 || (q & 1) == 0;
-        f32x4 dr;
-        {
-            const lds_t y = L::TWO + (i & 1) * L::SLOT + L::DY;
-            dr = causal_split(base_tr, byrow ? uv : y, byrow ? uv3 : F32, byrow ? y : uv, byrow ? F32 : uv3, byrow, false, l16, g);
-            asm volatile("" : "+v"(dr));
-        }
         __syncthreads();
         // ---------------------------------------------------------------- phase 2: dU, dW = M^T dU, dV, the gradient state
         {
@@ -1043,15 +1054,16 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
                 add32(x, get_pair<TERM2>(two.pair + L::AR + 1024 * jt), wy);
                 dS[jt] = dS[jt] * ld4(dec + 16 * jt) + total(x);
             }
-            put_half<TTERM2>(one.pair + (q == 0 ? L::R_ROWS : (q == 1 ? L::R_ROWS + 8 : (q == 2 ? L::B_COLS + 8 : L::K_COLS + 8))), split3(dr));
+            put_half<TTERM2>(one.pair + (q == 1 ? L::R_ROWS : (q == 0 ? L::R_ROWS + 8 : (q == 3 ? L::B_COLS + 8 : L::K_COLS + 8))), split3(dr));
         }
         __syncthreads();
-        // ---------------------------------------------------------------- phase 3: dAB (q even), dAK (they need dW), by rows and by columns
+        // ---------------------------------------------------------------- phase 3: dAB (q odd), dAK (they need dW), by rows and by columns
         {
-            const lds_t w = L::ONE + L::DW;
+            const lds_t w = L::ONE + L::DW, uv = uv_of(i);
             const f32x4 t = causal_split(base_tr, byrow ? uv : w, byrow ? uv3 : true, byrow ? w : uv, byrow ? true : uv3, byrow, true, l16, g);
-            put_half<TTERM2>(one.pair + (q == 0 ? L::A_ROWS : (q == 1 ? L::A_ROWS + 8 : (q == 2 ? L::B_COLS : L::K_COLS))), split3(t));
+            put_half<TTERM2>(one.pair + (q == 1 ? L::A_ROWS : (q == 0 ? L::A_ROWS + 8 : (q == 3 ? L::B_COLS : L::K_COLS))), split3(t));
         }
+        if (i + 1 < nch) dr = dr_tile(i + 1);
         // These waves carry the finished rows of the visit before to global memory (parked by the B waves in phase 1, dv by this role one
         // visit earlier; both stay as they are until the next visit).
         if constexpr (!F32) {
@@ -1080,12 +1092,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     using L = LB<F32>;
     LaneB one = lane_bases(sb + L::ONE, l16, g, own);
     const Tr base_tr = tr_bases(sb, l16, g);
-    f32x4 dS[4], S0b[4];                             // dS, S0 at [i = 16 ib + 4 g + v][j = own]
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            dS[ib][v] = dsT != nullptr ? dsT[static_cast<size_t>(16 * ib + 4 * g + v) * N + own] : 0.f;
+    f32x4 S0b[4];                                    // S0 at [i = 16 ib + 4 g + v][j = own]
     auto fetch_state = [&](int c) __attribute__((always_inline)) {
         const float* slot = slots + static_cast<size_t>(c) * N * N;
         const uint32_t me = lane_again();
@@ -1107,13 +1114,29 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     auto copy_of = [&](int visit) __attribute__((always_inline)) { return static_cast<lds_t>(L::TWO + (visit & 1) * L::SLOT); };
     float Pj = 0.f;                                  // P at the end of the chunk that is finished next
     f32x4 xA = ZERO4, xB = ZERO4, xK = ZERO4, dRp = ZERO4;    // state parts of dA', dB', dK', and dR', carried into the next visit's phase 1
-    Op3 ar, bk;                                      // and the planes of the own channel, whose places the P waves fill anew there
+    // and of the planes of the own channel, whose places the P waves fill anew there, operands and values; e^{c_{t+1}}, before the first
+    // of the four tokens e^{c_t}, HOLD e^{-c_{t+1}}
+    Op3 ar, bk;
+    f32x4 va, vr, vb, vk, er, eb;
+    float ea0 = 1.f;
     // a contraction over 16 with a pair of tiles (one after the other: the registers do not hold the operands of all of them)
     auto tile2 = [&](uint32_t pair, const Op3& b) __attribute__((always_inline)) {
         Sum2 s = SUM0;
         add32(s, get_pair<TTERM2>(one.pair + pair), b);
         __builtin_amdgcn_sched_barrier(0);
         return total(s);
+    };
+    // the values that a side of an operand holds.  (Those, and not inputs times factors, go into the sums for the decay gradient: what of
+    // one product is in another cancels there.)
+    auto value = [&](const Op3& o, const int side) __attribute__((always_inline)) {
+        f32x4 x;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const uint32_t h = __builtin_bit_cast(u32x4, o.h)[2 * side + w], m = __builtin_bit_cast(u32x4, o.m)[2 * side + w], l = __builtin_bit_cast(u32x4, o.l)[2 * side + w];
+            x[2 * w] = bf_lo(h) + (bf_lo(m) + bf_lo(l));
+            x[2 * w + 1] = bf_hi(h) + (bf_hi(m) + bf_hi(l));
+        }
+        return x;
     };
     // tile parts, scaling, decay gradient of the chunk of a visit, whose first row is row0; results parked as bf16
     auto finish = [&](const int visit, const size_t row0) __attribute__((always_inline)) {
@@ -1124,36 +1147,19 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             if constexpr (F32) store_f32(dst, first, lo + static_cast<uint32_t>(v * H) * N, x);
             else lds_st<uint16_t>(park + 2 * PK * (CL * k + v), f2bf(x));
         };
-        const lds_t two = one.own_pair - L::ONE + copy_of(visit);
         const f32x4 tA = tile2(L::A_ROWS, bk);
         const f32x4 tB = tile2(L::B_COLS, ar), tK = tile2(L::K_COLS, ar);
-        const f32x4 es = lds_ld<f32x4>(two + L::ES), dwf = lds_ld<f32x4>(two + L::DWF);
-        // e^{c_t} of the token before the lane's four (of the first four it is 1)
-        float ea = lds_ld<float>(sb + copy_of(visit) + L::ES + 12 + piece2(16 * q + (me & 15), me > 15 ? (me >> 4) - 1 : 0));
-        if (me < 16) ea = 1.f;
-        std::conditional_t<F32, f32x4, u32x2> raw[4];
-#pragma unroll
-        for (int z = 0; z < 4; ++z) {
-            if constexpr (F32) raw[z] = lds_ld<f32x4>(two + L::RAW + z * L::RAWB);
-            else raw[z] = lds_ld<u32x2>(one.own - L::ONE + copy_of(visit) + L::RAW + z * L::RAWB);
-        }
-        auto input = [&](const int z, const int v) __attribute__((always_inline)) {
-            if constexpr (F32) return raw[z][v];
-            else return v & 1 ? bf_hi(raw[z][v >> 1]) : bf_lo(raw[z][v >> 1]);
-        };
+        const f32x4 dwf = lds_ld<f32x4>(one.own_pair - L::ONE + copy_of(visit) + L::DWF);
         float del[4], ada[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const float dAp = fmaf(UNHOLD, tA[v], xA[v]), dBp = tB[v] + xB[v], dKp = tK[v] + xK[v];
-            const float er = es[v], hb = held_inverse(er), eb = hb * UNHOLD;
-            put(0, p.da, v, dAp * ea);
-            put(1, p.dr, v, dRp[v] * er);
-            put(2, p.db, v, dBp * eb);
-            put(3, p.dk, v, dKp * eb);
-            // a da;  r dr - b db - k dk, of the values that the tiles' planes hold: what of one is in another cancels in the sums below
-            ada[v] = (input(0, v) * ea) * dAp;
-            del[v] = fmaf(input(1, v) * er, dRp[v], -UNHOLD * fmaf(input(2, v) * hb, dBp, (input(3, v) * hb) * dKp));
-            ea = er;
+            put(0, p.da, v, dAp * (v == 0 ? ea0 : er[v - 1]));
+            put(1, p.dr, v, dRp[v] * er[v]);
+            put(2, p.db, v, dBp * (eb[v] * UNHOLD));
+            put(3, p.dk, v, dKp * (eb[v] * UNHOLD));
+            ada[v] = va[v] * dAp;
+            del[v] = fmaf(vr[v], dRp[v], -UNHOLD * fmaf(vb[v], dBp, vk[v] * dKp));      // r dr - b db - k dk
         }
         // G_t = P_{t+1} + del_t,  P_t = G_t + a da:  suffix sums over t = 4 g + v, later lane groups first
         const float tot = (del[0] + ada[0]) + (del[1] + ada[1]) + (del[2] + ada[2]) + (del[3] + ada[3]);
@@ -1190,7 +1196,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
                 add32(x, join(get3(o + L::U), as3(exact_piece<F32>(o + L::V))), bk);
                 const f32x4 acc = total(x);
 #pragma unroll
-                for (int v = 0; v < 4; ++v) pp = fmaf(dS[ib][v], fmaf(acc[v], UNHOLD, S0b[ib][v]) * decj, pp);
+                for (int v = 0; v < 4; ++v) pp = fmaf(dsT[(16 * ib + 4 * g + v) * N + own], fmaf(acc[v], UNHOLD, S0b[ib][v]) * decj, pp);
             }
             pp += __shfl_xor(pp, 16, 64);
             pp += __shfl_xor(pp, 32, 64);
@@ -1198,43 +1204,42 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         }
         __syncthreads();
         // ---------------------------------------------------------------- phase 2: dY S0, U dS, V dS; dRB (q even), dRK, by rows and by columns
-        auto ya = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::DY, two.tr, hb); };
-        auto ua = [&](int hb) __attribute__((always_inline)) { return get3_tr(L::U, two.tr, hb); };
-        auto va = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::V, two.tr, hb); };
+        auto dy_of = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::DY, two.tr, hb); };
+        auto u_of = [&](int hb) __attribute__((always_inline)) { return get3_tr(L::U, two.tr, hb); };
+        auto v_of = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::V, two.tr, hb); };
         Op3 s0[2];
         f32x4 xR;
+        ar = get_pair<TERM2>(two.own_pair + L::AR); bk = get_pair<TERM2>(two.own_pair + L::BK);
+        va = value(ar, 0); vr = value(ar, 1); vb = value(bk, 0); vk = value(bk, 1);
+        asm volatile("" : "+v"(va), "+v"(vr), "+v"(vb), "+v"(vk));            // (here, or the compiler takes all this to where it is used)
         {
             Sum2 pr = SUM0, pb = SUM0, pk = SUM0;
-            const float decj = decay_of(i);
+            const lds_t sq = sb + L::ONE + L::DS + square(4 * g + (l16 >> 2), 4 * q + (l16 & 3));
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb) {
                 s0[hb] = join(split3(S0b[2 * hb]), split3(S0b[2 * hb + 1]));
-                const Op3 ds = join(split3(dS[2 * hb] * decj), split3(dS[2 * hb + 1] * decj));
-                add32(pr, ya(hb), s0[hb]);
-                add32(pb, ua(hb), ds);
-                add32(pk, va(hb), ds);
+                const Op3 ds = {tr16_square(sq, hb), tr16_square(sq + DTERM, hb), tr16_square(sq + 2 * DTERM, hb)};      // dS dec, of role A
+                add32(pr, dy_of(hb), s0[hb]);
+                add32(pb, u_of(hb), ds);
+                add32(pk, v_of(hb), ds);
             }
             xR = total(pr); xB = total(pb); xK = total(pk);
         }
         __syncthreads();
         // ---------------------------------------------------------------- phase 3: dW S0; the gradient state
         {
-            const float decj = decay_of(i);
-            ar = get_pair<TERM2>(two.own_pair + L::AR);
+            er = lds_ld<f32x4>(two.own_pair + L::ES);
+            const uint32_t me = lane_again();
+            ea0 = lds_ld<float>(sb + copy_of(i) + L::ES + 12 + piece2(16 * q + (me & 15), me > 15 ? (me >> 4) - 1 : 0));
+            if (me < 16) ea0 = 1.f;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) eb[v] = held_inverse(er[v]);                    // (er is between e^-9.8 and 1)
+            asm volatile("" : "+v"(er), "+v"(eb), "+v"(ea0));
             Sum2 pa = SUM0;
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb) add32(pa, get3_tr(L::DW, one.tr, hb), s0[hb]);
             xA = total(pa);
-            const lds_t row = rows();
-#pragma unroll
-            for (int ib = 0; ib < 4; ++ib) {
-                Sum2 x = SUM0;
-                const lds_t o = (row ^ (ib & 1 ? 16u : 0u)) + 512 * ib;
-                add32(x, join(get3(sb + L::ONE + o + L::DW), as3(exact_piece<F32>(sb + copy_of(i) + o + L::DY))), ar);
-                dS[ib] = dS[ib] * decj + total(x);
-            }
             // dR' needs no tile of this phase
-            bk = get_pair<TERM2>(two.own_pair + L::BK);
             const f32x4 tR = tile2(L::R_ROWS, bk);
 #pragma unroll
             for (int v = 0; v < 4; ++v) dRp[v] = fmaf(UNHOLD, tR[v], xR[v]);
@@ -1250,7 +1255,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
 template <bool F32, bool CUT>
 __global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c args) {
     const Args7c p = only_whole<CUT>(args);
-    extern __shared__ __align__(32) unsigned char smem_raw[];
+    extern __shared__ __align__(128) unsigned char smem_raw[];
     SmemCB<F32>& S = *reinterpret_cast<SmemCB<F32>*>(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.x, b = blockIdx.y;
