@@ -2,37 +2,34 @@
 //
 // Step form (rwkv7_fast_fused/cuda/rwkv7_statepassing_clampw.cu:20-187), one head, S[i][j] (i value, j key):
 //     sa_t = S_t a_t;   S_{t+1} = S_t diag(w_t) + sa_t b_t^T + v_t k_t^T;   y_t = S_{t+1} r_t;   w_t = exp(W_SCALE sigmoid(w_raw_t))
-// A chunk of L = 16 steps (the reference's CHUNK_LEN), local t = 0..15, S0 the state entering it.  With lam_t = log w_t,
-// c_t = sum_{z<t} lam_z and the chunk's middle m = 8 as the reference point (the clamp bounds |c_t - c_m| by 0.607 * 8, so
-// no factor exceeds e^4.9 and nothing needs a fallback):
-//     A'_t = a_t e^{c_t - c_m}    R'_t = r_t e^{c_{t+1} - c_m}    B'_s = b_s e^{c_m - c_{s+1}}    K'_s = k_s e^{c_m - c_{s+1}}
-//     d1 = e^{c_m}   d2 = e^{c_L - c_m}   dec = e^{c_L}
-//     AB = tril_-(A' B'^T)  AK = tril_-(A' K'^T)  RB = tril(R' B'^T)  RK = tril(R' K'^T)                 [16 x 16]
-//     U  = (I - AB)^{-1} ((A' d1) S0^T + AK V)         rows of U are sa_t (the tensor `sa` of the interface)
-//     Y  = (R' d1) S0^T + RB U + RK V
-//     S_L = S0 diag(dec) + U^T (B' d2) + V^T (K' d2)
-// (the state update takes B' d2 = b e^{c_L - c_{s+1}} and K' d2 from one exponential each: a factor's relative error is the
-// absolute error of its exponent, and referred to the chunk's end the newest, largest contributions have the smallest
-// exponents; through the middle every term would carry two factors of e^{+-4.9} -- 3e-7 on the fp32 state instead of 5e-8.)
-// Backward of a chunk from dY and dS_L (the gradient w.r.t. S_L through everything after the chunk):
-//     dU  = RB^T dY + (B' d2) dS_L^T          dW = (I - AB)^{-T} dU
+// A chunk of L = 16 steps (the reference's CHUNK_LEN), local t = 0..15, S0 the state entering it, lam_t = log w_t, c_t = sum_{z<t} lam_z.
+// Everything is referred to one border of the chunk, e^{+-9.8} at most, so nothing needs a fallback.  Forward, to the chunk's end, with
+// x_t = e^{c_L - c_t}, dec = x_0 = e^{c_L}:
+//     A_t = a_t / x_t    R_t = r_t / x_{t+1}    B_s = b_s x_{s+1}    K_s = k_s x_{s+1}    D0 = S0 diag(dec)
+//     AB = tril_-(A B^T)  AK = tril_-(A K^T)  RB = tril(R B^T)  RK = tril(R K^T)                         [16 x 16]
+//     U  = (I - AB)^{-1} (A D0^T + AK V)               rows of U are sa_t (the tensor `sa` of the interface)
+//     Y  = R D0^T + RB U + RK V
+//     S_L = D0 + U^T B + V^T K
+// So each input is multiplied and split once: A and R meet the state and make the tiles, B and K make the tiles and the new state.  What
+// is near the end, the largest part of that, has the smallest exponents.  (Referred to the middle for the tiles, to the start for A and R and to
+// the end for B and K, which is as accurate, the four inputs were eight planes.)
+// Backward of a chunk from dY and dS_L (the gradient w.r.t. S_L through everything after the chunk), referred to the chunk's start, with
+// x_t = e^{c_t}, dec = x_L, A_t = a_t x_t, R_t = r_t x_{t+1}, B_s = b_s / x_{s+1}, K_s = k_s / x_{s+1}, E = dS_L diag(dec) (the tiles are the same):
+//     dU  = RB^T dY + B E^T                   dW = (I - AB)^{-T} dU
 //     dAB = tril_-(dW U^T)  dAK = tril_-(dW V^T)  dRB = tril(dY U^T)  dRK = tril(dY V^T)
-//     dV  = AK^T dW + RK^T dY + (K' d2) dS_L^T
-//     dS0 = dS_L diag(dec) + d1 (dY^T R' + dW^T A')
-//     dA' = dAB B' + dAK K' + d1 (dW S0)      dR' = dRB B' + dRK K' + d1 (dY S0)
-//     dB' = dAB^T A' + dRB^T R' + d2 (U dS_L)  dK' = dAK^T A' + dRK^T R' + d2 (V dS_L)
-//     da = dA' e^{c_t - c_m}, dr = dR' e^{c_{t+1} - c_m}, db = dB' e^{c_m - c_{t+1}}, dk likewise
+//     dV  = AK^T dW + RK^T dY + K E^T
+//     dS0 = E + dY^T R + dW^T A
+//     dA = dAB B + dAK K + dW S0              dR = dRB B + dRK K + dY S0
+//     dB = dAB^T A + dRB^T R + U E            dK = dAK^T A + dRK^T R + V E
+//     da = dA x_t, dr = dR x_{t+1}, db = dB / x_{t+1}, dk = dK / x_{t+1}
 //     decay: with P_t = sum_i dS_t o S_t per key channel,  G_t = P_{t+1} + r dr - b db - k dk,  P_t = G_t + a da,
 //            dw_raw = G W_SCALE sig (1 - sig);  P at the end of the call = sum_i dsT o S_T.
+// What is divided by x is held by 2^-7 (HOLD below).
 // Every product takes all 24 bits of its operands, so the fp32 outputs sT, ds0 and the saved sa keep the accuracy class of the
 // reference's fp32 recurrence; the bf16 outputs are rounded once at the store.  The fp32 mode is therefore the same kernel with fp32
-// loads and stores.  Products are split ones (split3.h) but for the tiles AB, AK, RB, RK in both directions, which are fp32 matrix
-// instructions, 16 a wave and chunk.  Each of A', R', B', K' enters two of them.  Split operands were not built: the wave that makes a
-// tile would split both of its sides, 176 vector instructions beside 12 matrix ones, or read them from LDS split, and the backward,
-// whose B waves split those planes for products of their own, has 1 KB of LDS left where two copies of them take 14 KB more.
+// loads and stores.  Products are split ones (split3.h); the few of the scan over blocks are fp32 matrix instructions.
 //
-// One workgroup per (batch, head).  A 16x16x4 fp32 matrix instruction takes A[row = lane & 15][k = lane >> 4],
-// B[k = lane >> 4][col = lane & 15] and leaves D[row = 4 (lane >> 4) + v][col = lane & 15] in register v.  The state is
+// One workgroup per (batch, head).  A 16x16 matrix instruction leaves D[row = 4 (lane >> 4) + v][col = lane & 15] in register v.  The state is
 // kept TRANSPOSED in accumulator registers, S^T tile jt of wave q: register v of lane (l16, g) = S[i = 16 q + l16][j = 16 jt + 4 g + v].
 // K slots may be assigned to channels (or tokens) in any order as long as both operands agree, so accumulator registers, split, are the
 // B operand of the next product: two state tiles of a contraction over 32 channels, U, W, dU, dW of one over 16 tokens.  Nothing is
@@ -151,51 +148,6 @@ DEVINL void inverse_cols(const float (*AB)[TS], int c, float (&m)[CL]) {
     }
 }
 
-// e^x to fp32 accuracy for |x| of a few units: the hardware exponential takes x log2(e), whose rounding alone costs |x| 6e-8;
-// the product is carried as a rounded part plus its error, and the error enters to first order.
-DEVINL float exp_acc(float x) {
-    constexpr float L2E_HI = 1.44269502162933349609f, L2E_LO = 1.92596299112661746e-8f, LN2 = 0.69314718055994530942f;
-    const float t = x * L2E_HI;
-    const float e = fmaf(x, L2E_HI, -t) + x * L2E_LO;
-    const float y = __builtin_amdgcn_exp2f(t);
-    return fmaf(y, e * LN2, y);
-}
-
-// In-chunk factors of the four tokens (4 q + e) of channel j held by a thread, from lam and the per-wave sums in part[][].
-// Every exponent is formed as a direct sum of the lam between the token and its reference point (never as a difference of
-// two long cumulative sums), so its absolute error -- the factor's relative error -- scales with the exponent itself.
-struct Factors { float ea[4], er[4], eb[4], es[4], ee[4]; };   // e^{c_t - c_m}, e^{c_{t+1} - c_m}, e^{c_m - c_{t+1}}, e^{c_t}, e^{c_L - c_{t+1}}
-DEVINL Factors chunk_factors(const float (&lam)[4], const float (*part)[N], int q, int j, float& cm_out, float& cl_out) {
-    const float p0 = part[0][j], p1 = part[1][j], p2 = part[2][j], p3 = part[3][j];
-    const float cm = p0 + p1, cl = (p0 + p1) + (p2 + p3);
-    const float before = q == 0 ? 0.f : (q == 1 ? p0 : (q == 2 ? cm : cm + p2));        // c_t of the wave's first token
-    const float after = q == 3 ? 0.f : (q == 2 ? p3 : (q == 1 ? p2 + p3 : p1 + (p2 + p3)));   // c_L - c of the token after the wave's last
-    // lam between the wave's tokens and the middle: first half, the tokens after the wave up to the middle; second half, those from the middle up to the wave
-    const float gap = q == 0 ? p1 : (q == 3 ? p2 : 0.f);
-    float pre[5], suf[5];                      // pre[e] = sum of lam[0..e-1], suf[e] = sum of lam[e..3]
-    pre[0] = 0.f; suf[4] = 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) pre[e + 1] = pre[e] + lam[e];
-#pragma unroll
-    for (int e = 3; e >= 0; --e) suf[e] = suf[e + 1] + lam[e];
-    Factors f = {};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {                  // (a caller pays for the factors that it takes)
-        // c_t - c_m and c_{t+1} - c_m
-        const float xt = q < 2 ? -(suf[e] + gap) : gap + pre[e];
-        const float xn = q < 2 ? -(suf[e + 1] + gap) : gap + pre[e + 1];
-        // the middle-referenced factors always come in pairs whose exponents cancel only partly, so the extra digits of
-        // exp_acc would be lost anyway; the start- and end-referenced ones carry the fp32 states and keep them
-        f.ea[e] = __expf(xt);
-        f.er[e] = __expf(xn);
-        f.eb[e] = __expf(-xn);
-        f.es[e] = exp_acc(before + pre[e]);
-        f.ee[e] = exp_acc(suf[e + 1] + after);
-    }
-    cm_out = cm; cl_out = cl;
-    return f;
-}
-
 // (a Newton step behind the hardware reciprocal instead of a full division, a sixth of the vector instructions that turn inputs into
 // planes.  A quarter of the denominator, since the reciprocal flushes what is below 2^-126; an overflown exponential leaves zero, and
 // so no decay gradient, where the step by itself would make a NaN; a NaN passes by y)
@@ -267,33 +219,14 @@ template <bool ROWS, class TA, class SB> DEVINL f32x4 causal_tile(TA ta, SB sb, 
     return acc;
 }
 
-// tile[t][s] = sum_c X[t][c] Y[s][c] over 64 channels, masked to s < t (strict) or s <= t: register v <-> t = 4 g + v, lane <-> s, or
-// (ROWS) register v <-> s = 4 g + v, lane <-> t
-template <bool ROWS> DEVINL f32x4 causal_acc(const float (*X)[PS], const float (*Y)[PS], bool strict, int l16, int g) {
-    f32x4 part[2] = {ZERO4, ZERO4};               // two independent chains
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-        const f32x4 xa = ld4(&X[l16][16 * cb + 4 * g]), yb = ld4(&Y[l16][16 * cb + 4 * g]);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) part[cb & 1] = ROWS ? mm(yb[v], xa[v], part[cb & 1]) : mm(xa[v], yb[v], part[cb & 1]);
-    }
-    f32x4 acc = part[0] + part[1];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int t = ROWS ? l16 : 4 * g + v, s = ROWS ? 4 * g + v : l16;
-        acc[v] = (strict ? s < t : s <= t) ? acc[v] : 0.f;
-    }
-    return acc;
-}
 // ---------------------------------------------------------------------------------------------------- forward
 // One workgroup of eight waves per (batch, head), two of them on a CU, two roles with their own loops and two barriers a chunk:
 //          phase X                                                   | phase Y
-//   S:     (a e^{c_t}) S0^T, (r e^{c_{t+1}}) S0^T; rows of the chunk  | AK V, U, RK V + RB U, the state
-//          before and the state entering to memory                    |
+//   S:     A D0^T, R D0^T; rows of the chunk before and the state     | AK V, U, RK V + RB U, the state
+//          entering to memory                                         |
 //   P:     causal tiles and the inverse of this chunk; decay sums of  | factors, planes of the next chunk
 //          the next                                                   |
-// A plane that one phase writes and the other reads needs no second copy (k, b carried to the chunk's end and dec, which S reads while P writes, do).
-// The P waves make the tiles on the fp32 matrix instructions, all other products are split ones (split3.h).
+// A plane that one phase writes and the other reads needs no second copy (B, K and dec, which S reads while P writes, do).
 constexpr int NTF = 8 * 64;        // waves 0..3 role S, 4..7 role P
 struct SmemCF {
     float Yo[CL][PS], Uo[CL][PS];
@@ -301,8 +234,7 @@ struct SmemCF {
     Decay part[4][N];
     float dec[2][N];
 };
-// three-term planes and tiles behind it: a HOLD e^{c_t - c_L}, r HOLD e^{c_{t+1} - c_L}, k and b times e^{c_L - c_{s+1}}, v (one term
-// where it is bf16), AK, RB, RK, (I - AB)^{-1}
+// three-term planes and tiles behind it: HOLD A, HOLD R, K and B, v (one term where it is bf16), AK, RB, RK, (I - AB)^{-1}
 constexpr uint32_t F_AS = (sizeof(SmemCF) + 31) / 32 * 32, F_RS = F_AS + PLANE3, F_KB = F_RS + PLANE3, F_V = F_KB + 2 * PAIR3;
 template <bool F32> constexpr uint32_t F_MA = F_V + (F32 ? PLANE3 : TERM);      // (I - AB)^{-1} and AK
 template <bool F32> constexpr uint32_t F_RKB = F_MA<F32> + TPAIR3;                // RK and RB
@@ -469,11 +401,13 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
 }
 
 // KEEP: `s` and `sa` are written for a backward, 20 bytes per element beside the 14 of a bf16 forward's inputs and output.
-// What bounds it: issue.  B8 T1024 C4096, one call: 398 us with every product on the fp32 matrix instructions, in four waves that did
-// everything in turn between four barriers; 390 in two roles of four waves; 335 with split products, since the fp32 instructions
-// (96 a wave and chunk) held the vector unit for half of the time.  The first of these forms and this one in alternation on one
-// machine: bf16 382 -> 326 us, fp32 mode 405 -> 379.  Vector instructions now issue 68 % of a SIMD's time, matrix ones about a third.
-// Errors against 64 bits, T16 to T1024, slow to strong decays, largest, before -> now: y 2.4 -> 1.7e-7, sT 1.6 -> 1.0e-7, sa 2.3 -> 1.7e-7.
+// What bounds it: issue and, with KEEP, the writes (half of the states, and it takes 310 us instead of 332; fp32 mode 324 of 372).
+// B8 T1024 C4096, one call, bf16: 398 us with every product on the fp32 matrix instructions, in four waves that did
+// everything in turn between four barriers; 390 in two roles of four waves; 335 with split products but for the tiles, whose 16 fp32
+// instructions a P wave held the vector unit for 512 cycles and took four more planes, twice the exponentials.  That form and this one in
+// alternation on one machine: bf16 355 -> 331 us, 268 -> 241 without KEEP; fp32 mode 386 -> 368, 306 -> 280.
+// Not kept: a ninth wave for the inverse (one workgroup a CU then: 502 us); rows asked for two chunks ahead (bf16 without KEEP 242 -> 253).
+// Errors against 64 bits, T1024, usual decays / strong ones, before -> now, 1e-7: y 1.39 -> 0.81 / 1.47 -> 0.78, sT 0.61 -> 0.58 / 0.61 -> 0.57.
 template <bool F32, bool KEEP, bool CUT>
 __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c args) {
     const Args7c p = only_whole<CUT>(args);
@@ -500,14 +434,14 @@ __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c args) {
 // one recurrence,  W = P1 S^T + T1 V, U = M0 W, S = S dec + U^T P2 + V^T P3,  per chunk:
 //     forward   P1 = a e^{c_t}            T1 = AK     M0 = (I - AB)^{-1}  P2 = b e^{c_L - c_{s+1}}  P3 = k e^{c_L - c_{s+1}}  V = v
 //     backward  P1 = b e^{c_L - c_{s+1}}  T1 = RB^T   M0 = (I - AB)^{-T}  P2 = a e^{c_t}            P3 = r e^{c_{t+1}}        V = dy
+// (P1 S^T as in the kernels proper, P1 e^{-c_L} and S with the chunk's decay on it),
 // which rwkv7c_local walks through (the roles of the forward without its outputs; a workgroup for E and one for M, which has no V).
 // rwkv7c_scan takes the blocks in turn, 16 rows of a head a workgroup, on the fp32 matrix instructions.  M may overflow where the state
 // itself is small (a, b that make it grow): a head with a scanned state that is not finite is walked through as a whole by the workgroup
 // of its first block, as are heads with inputs that are no number.
 struct SmemL {
-    float Ap[CL][PS], Bp[CL][PS], Xp[CL][PS];
     float AB[CL][TS];
-    float part[4][N];
+    Decay part[4][N];
     float dec[2][N];
 };
 constexpr uint32_t L_S = (sizeof(SmemL) + 31) / 32 * 32, L_KB = L_S + PLANE3, L_V = L_KB + 2 * PAIR3;
@@ -529,40 +463,39 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
 #pragma unroll
             for (int k = 0; k < 5; ++k) nx[k][e] = ld_raw<F32>(src[k], base, static_cast<uint32_t>((4 * q + e) * H) * N + lo);
     };
-    float lam[4], xx[4], aa[4], bb[4];
+    Decay lam[4];
+    float xx[4], aa[4], bb[4];
     uint32_t vb[4];
     auto convert = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            lam[e] = W_SCALE * sigmoid_fast(widen<F32>(nx[0][e]));
+            lam[e] = decay_of(widen<F32>(nx[0][e]));
             xx[e] = widen<F32>(nx[1][e]);
             vb[e] = unit ? 0u : nx[2][e];
             aa[e] = widen<F32>(nx[3][e]); bb[e] = widen<F32>(nx[4][e]);
         }
-        S.part[q][lane] = (lam[0] + lam[1]) + (lam[2] + lam[3]);
+        S.part[q][lane] = sum4(lam);
     };
     auto planes = [&](const int slot) __attribute__((always_inline)) {
-        float cm, cl;
-        const Factors f = chunk_factors(lam, S.part, q, lane, cm, cl);
-        f32x4 as, be, xs;
+        float x[5], y[5];
+        growth<!REV>(lam, S.part, q, lane, x, y);
+        f32x4 p1, p2, p3;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int t = 4 * q + e;
-            S.Ap[t][lane] = aa[e] * f.ea[e];
-            S.Bp[t][lane] = bb[e] * f.eb[e];
-            S.Xp[t][lane] = xx[e] * (REV ? f.er[e] : f.eb[e]);
-            as[e] = aa[e] * f.es[e];
-            be[e] = bb[e] * f.ee[e];
-            xs[e] = xx[e] * (REV ? f.es[e] * __expf(lam[e]) : f.ee[e]);
+            p1[e] = REV ? bb[e] * y[e + 1] : aa[e] * y[e];
+            p2[e] = REV ? aa[e] * x[e] : bb[e] * x[e + 1];
+            p3[e] = xx[e] * x[e + 1];
         }
         const lds_t o = sb + piece(lane, q);
-        // (no factor is above 1: what comes from bf16 inputs stays within bf16's range)
-        put3(o + L_S, split3<!F32>(REV ? be : as));
-        put_pair<TERM2>(sb + L_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(xs), split3<!F32>(REV ? as : be));
+        put3(o + L_S, split3(p1));
+        // (x is not above 1: what comes from bf16 inputs stays within bf16's range)
+        put_pair<TERM2>(sb + L_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(p3), split3<!F32>(p2));
         if constexpr (F32) put3(o + L_V, split3(f32x4{widen<F32>(vb[0]), widen<F32>(vb[1]), widen<F32>(vb[2]), widen<F32>(vb[3])}));
         else lds_st<u32x2>(o + L_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
-        if (q == 0) S.dec[slot][lane] = exp_acc(cl);
+        if (q == (REV ? 3 : 0)) S.dec[slot][lane] = x[REV ? 4 : 0];
     };
+    const Tr sp = tr_bases(sb + L_S, l16, g);
+    const lds_t pp = tr_pair(sb + L_KB + (q == 0 ? 8 : 0), l16, g);
     fetch(0);
     convert();
     fetch(1);
@@ -571,9 +504,13 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
     __syncthreads();
     for (int c = 0; c < nch; ++c) {
         if (q < 2) {
+            auto one = [&](int hb) __attribute__((always_inline)) { return get3_tr(0, sp, hb); };
+            auto pair = [&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, pp + (c & 1) * PAIR3, hb); };
             f32x4 x;
             if (q == 0) {
-                const f32x4 t = causal_acc<false>(S.Ap, S.Bp, true, l16, g);
+                f32x4 t;
+                if constexpr (REV) t = causal_tile<false>(pair, one, true, l16, g) * UNHOLD;
+                else t = causal_tile<false>(one, pair, true, l16, g) * UNHOLD;
                 float m[CL];
                 // (this wave wrote AB itself: LDS keeps a wave's accesses in order)
                 if constexpr (REV) {
@@ -585,8 +522,8 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
                     inverse_rows(S.AB, l16, m);
                 }
                 x = by_group(g, m);
-            } else if constexpr (REV) x = causal_acc<false>(S.Xp, S.Bp, false, l16, g);
-            else x = causal_acc<true>(S.Ap, S.Xp, true, l16, g);
+            } else if constexpr (REV) x = causal_tile<false>(pair, one, false, l16, g);
+            else x = causal_tile<true>(one, pair, true, l16, g);
             put_half<TTERM2>(sb + piece2(l16, g) + L_MA<F32> + (q == 0 ? 0 : 8), split3(x));
         }
         convert();
@@ -609,21 +546,23 @@ template <bool F32> DEVINL void local_role_s(SmemL& S, const lds_t sb, float* ou
     __syncthreads();
     for (int c = 0; c < nch; ++c) {
         const auto vop = [&]() __attribute__((always_inline)) { if constexpr (F32) return get3(vp); else return lds_ld<u32x2>(vp); }();
-        Sum2 W = SUM0;
+        const float* const dec = &S.dec[c & 1][4 * g];
+        Sum2 W = SUM0;                                   // HOLD W
 #pragma unroll
-        for (int hb = 0; hb < 2; ++hb) add32(W, get3_tr(L_S, tr, hb), join(split3(St[2 * hb]), split3(St[2 * hb + 1])));
+        for (int hb = 0; hb < 2; ++hb)
+            add32(W, get3_tr(L_S, tr, hb), join(split3(St[2 * hb] * ld4(dec + 32 * hb)), split3(St[2 * hb + 1] * ld4(dec + 32 * hb + 16))));
         here(W);
         __syncthreads();
         add16(W, get_half<TTERM2>(pp + L_MA<F32> + 8), vop);
         Sum2 Us = SUM0;
-        add16(Us, get_half<TTERM2>(pp + L_MA<F32>), split3(total(W)));
+        add16(Us, get_half<TTERM2>(pp + L_MA<F32>), split3(total(W) * UNHOLD));
         const Op3 vu = join(as3(vop), split3(total(Us)));
         const lds_t kb = pp + L_KB + (c & 1) * PAIR3;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
             Sum2 x = SUM0;
             add32(x, get_pair<TERM2>(kb + 1024 * jt), vu);
-            St[jt] = St[jt] * ld4(&S.dec[c & 1][16 * jt + 4 * g]) + total(x);
+            St[jt] = St[jt] * ld4(dec + 16 * jt) + total(x);
         }
         __syncthreads();
     }
@@ -696,25 +635,21 @@ __global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
 
 // ---------------------------------------------------------------------------------------------------- backward
 // One workgroup of twelve waves per (batch, head), three roles with their own loops; wave w: q = w & 3.
-//   waves 0..3 ("A", value-channel tile q): dSa[jt][v] = dS[i = 16 q + l16][j = 16 jt + 4 g + v]   (rows j, columns i): the B operand
-//                of the contractions over the key channel, (B' d2) dS^T and (K' d2) dS^T; they make the causal tiles, dU, the
-//                triangular solve, dW, dV and ds0.
-//   waves 4..7 ("B", key-channel tile q):   dSb[ib][v] = dS[i = 16 ib + 4 g + v][j = 16 q + l16]   (rows i, columns j): the B operand
-//                of the contractions over the value channel, U dS and V dS, next to S0 of the chunk loaded from `s` in the same
-//                layout (dW S0, dY S0); they make dA', dR', dB', dK' (register v <-> token 4 g + v, lane <-> key channel), scale
-//                them, scan the decay gradient and park the results; they run one phase behind the A waves.
-//   waves 8..11 ("P"): fetch the seven input rows and `sa` two chunks ahead, convert them and build the operand planes
-//                (double-buffered).  The finished gradient rows leave LDS-staged, as whole rows, through A waves 2 and 3.
-// The gradient state is therefore kept twice (both copies get the same update).
-// What bounds it: issue, and waits for LDS and at barriers.  B8 T1024 C4096, one call: 762 us with fp32 matrix instructions (962 a
-// chunk, 57 % of a SIMD's time in which it could issue no vector instruction), 676 with split products.  Of that, causal tiles
-// and the inverse moved from phase 1, where everybody waited for wave 0, into the phase 3 before: 727 -> 676.  Both forms in alternation
-// on one machine: bf16 720 -> 623 us, vector instructions issuing 63 % of a SIMD's time; fp32 mode 800 -> 766, 53 %: its 24 rows a chunk
-// leave from registers, 64 bytes at a time, and it splits v and dy as well.  (With 26 spilled registers, addresses for the most part, it
-// took 826: see lane_again.)
-// Errors against 64 bits, T16 to T1024, slow to strong decays, largest, before -> now: ds0 1.8 -> 1.0e-7, dr 1.9 -> 1.3e-7, dk 2.1 ->
-// 1.3e-7, dv 2.2 -> 1.7e-7, da 3.0 -> 2.2e-7, db 3.2 -> 2.1e-7; dw 3.2 -> 2.4e-6 at T1024 and usual decays, 7.3 -> 6.9e-6 at decays near
-// e^-0.6, where 1 - sig has few digits.
+//   waves 0..3 ("A", value-channel tile q): the gradient state, dS[jt][v] = dS[i = 16 q + l16][j = 16 jt + 4 g + v]   (rows j, columns i): the
+//                B operand of the contractions over the key channel, B E^T and K E^T; dU, dW, dV, ds0, and the tiles dAB, dAK, dRB, dRK.
+//   waves 4..7 ("B", key-channel tile q): the contractions over the value channel: U E and V E, with the split E of role A through LDS,
+//                and dW S0, dY S0, with S0 of the chunk from `s`; they make dA, dR, dB, dK (register v <-> token 4 g + v, lane <-> key
+//                channel), scale them, scan the decay gradient and park the results; they run one phase behind the A waves.
+//   waves 8..11 ("P"): fetch the seven input rows and `sa` two chunks ahead, convert them, build the operand planes
+//                (double-buffered), the causal tiles and the inverse.  The finished gradient rows leave LDS-staged, as whole rows, through the A waves.
+// What bounds it: issue.  Over the three phases a SIMD issues 4300 to 4900 cycles of vector and 2900 of matrix instructions, which overlap by
+// a fifth, of some 9000.  B8 T1024 C4096, one call, bf16 mode / fp32 mode, us: 762 / . with fp32 matrix instructions; 626 / 765 with split
+// products but for the tiles, 11800 cycles a chunk, 5200 of them phase 3, where wave 0 of role A made a tile, an fp32 one and the inverse;
+// 606 / 708 with inputs split once, the tiles with the P waves a phase earlier and what role B waited for with role A; 588 / 642 with one
+// gradient state instead of two and the values that finish a chunk worked out in the phases before, in which role B waited.  First and last
+// form in alternation on one machine.
+// Errors against 64 bits, T1024, usual decays, before -> now, 1e-7: ds0 0.81 -> 0.78, dr 1.12 -> 0.92, dk 1.19 -> 0.94, dv 1.43 -> 0.94,
+// da 1.89 -> 1.37, db 1.85 -> 1.31, dw 6.6 -> 5.4; decays near e^-0.6, where 1 - sig has few digits, dw 57 -> 57, the others 0.88 .. 2.07 -> 0.83 .. 1.36.
 constexpr int NTB = 12 * 64;       // waves 0..3 role A, 4..7 role B, 8..11 role P
 
 constexpr int PK = 72;            // row stride (bf16 elements) of a parked output
@@ -742,7 +677,7 @@ DEVINL bf16x8 tr16_square(lds_t o, int hb) {       // rows 32 hb + 16 (e >> 2) +
 // r e^{c_{t+1}} (AR), b and k times HOLD e^{-c_{s+1}} (BK), U, v and dy (one term each where they are bf16) in three terms; fp32, 16 bytes of
 // four tokens as the pairs lie: e^{c_{t+1}} (ES), W_SCALE sig (1 - sig) (DWF).  One: dS with the chunk's decay on it, in three terms (DS), dW, and the
 // tiles, each as the lanes of its products hold it: the transposes of (I - AB)^{-1} and RB (MB), AK and RK (AKR); by rows (over s) dAB and
-// dAK for dA', dRB and dRK for dR'; by columns (over t) dAB and dRB for dB', dAK and dRK for dK'.
+// dAK for dA, dRB and dRK for dR; by columns (over t) dAB and dRB for dB, dAK and dRK for dK.
 template <bool F32> struct LB {
     static constexpr uint32_t TWO = (sizeof(SmemCB<F32>) + 31) / 32 * 32, EX = F32 ? PLANE3 : TERM;      // from TWO on
     static constexpr uint32_t AR = 0, BK = PAIR3, U = 2 * PAIR3, V = U + PLANE3, DY = V + EX, ES = DY + EX, DWF = ES + 4 * CL * N, SLOT = DWF + 4 * CL * N;
@@ -1091,7 +1026,6 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     const int own = 16 * q + l16;                    // key channel j of this lane's column
     using L = LB<F32>;
     LaneB one = lane_bases(sb + L::ONE, l16, g, own);
-    const Tr base_tr = tr_bases(sb, l16, g);
     f32x4 S0b[4];                                    // S0 at [i = 16 ib + 4 g + v][j = own]
     auto fetch_state = [&](int c) __attribute__((always_inline)) {
         const float* slot = slots + static_cast<size_t>(c) * N * N;
@@ -1113,7 +1047,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
     auto rows = [&]() __attribute__((always_inline)) { const uint32_t me = lane_again(); return piece(me & 15, me >> 4); };
     auto copy_of = [&](int visit) __attribute__((always_inline)) { return static_cast<lds_t>(L::TWO + (visit & 1) * L::SLOT); };
     float Pj = 0.f;                                  // P at the end of the chunk that is finished next
-    f32x4 xA = ZERO4, xB = ZERO4, xK = ZERO4, dRp = ZERO4;    // state parts of dA', dB', dK', and dR', carried into the next visit's phase 1
+    f32x4 xA = ZERO4, xB = ZERO4, xK = ZERO4, dRp = ZERO4;    // state parts of dA, dB, dK, and dR, carried into the next visit's phase 1
     // and of the planes of the own channel, whose places the P waves fill anew there, operands and values; e^{c_{t+1}}, before the first
     // of the four tokens e^{c_t}, HOLD e^{-c_{t+1}}
     Op3 ar, bk;
@@ -1239,7 +1173,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb) add32(pa, get3_tr(L::DW, one.tr, hb), s0[hb]);
             xA = total(pa);
-            // dR' needs no tile of this phase
+            // dR needs no tile of this phase
             const f32x4 tR = tile2(L::R_ROWS, bk);
 #pragma unroll
             for (int v = 0; v < 4; ++v) dRp[v] = fmaf(UNHOLD, tR[v], xR[v]);

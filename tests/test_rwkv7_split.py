@@ -92,3 +92,42 @@ def test_no_instruction_is_inline_assembly(name):
         text = re.sub(r"//[^\n]*", "", f.read())
     bodies = re.findall(r"\basm\b(?:\s+volatile)?\s*\(\s*\"([^\"]*)\"", text)
     assert bodies and all(b == "" for b in bodies), bodies
+
+
+def decay_parts(sig):
+    """decay_of_sig of csrc/rwkv7_chunk.hip, fused operations in fp64 and rounded (HI, LO: the two constants)."""
+    f = np.float32
+    C = -0.6065306597 * 1.4426950408889634
+    HI = f(C)
+    LO = f(C - float(HI))
+    fma = lambda a, b, c: (a.astype(np.float64) * np.float64(b) + c).astype(f)
+    hi = fma(sig, HI, 24.0) - f(24)
+    return hi, (f(0.69314718055994530942) * fma(sig, LO, fma(sig, HI, -hi.astype(np.float64)).astype(np.float64))).astype(f)
+
+
+def test_decays_of_a_chunk_add_up_exactly():
+    """Sums of the first parts over 16 steps are exact in any order, the second parts stay below 2^-20, and e to the sum of both is off by
+    the exponential's rounding and a few of 2^-40: 1e-7 where a sum of fp32 decays is off by 4e-7."""
+    rng = np.random.default_rng(3)
+    sig = np.concatenate([rng.uniform(0, 1, (4000, 16)), 1 / (1 + np.exp(rng.uniform(0, 12, (4000, 16)))), np.ones((1, 16)), np.zeros((1, 16))]).astype(np.float32)
+    hi, lo = decay_parts(sig)
+    assert np.all(np.abs(lo) <= 2.0 ** -20)
+    for order in (slice(None), slice(None, None, -1)):
+        run = np.cumsum(hi[:, order], axis=1, dtype=np.float32)
+        assert np.array_equal(run.astype(np.float64), np.cumsum(hi[:, order].astype(np.float64), axis=1))
+    total = lo[:, 0].copy()
+    for t in range(1, 16):
+        total += lo[:, t]
+    got = np.exp2(hi.astype(np.float64).sum(1)).astype(np.float32)
+    got = (got.astype(np.float64) * total + got).astype(np.float32).astype(np.float64)
+    want = np.exp(-0.6065306597 * sig.astype(np.float64).sum(1))
+    assert np.max(np.abs(got / want - 1)) <= 2 * 2.0 ** -24 + 2.0 ** -32
+
+
+def test_constants_of_the_decay():
+    """The quotient of the two constants of decay_of is W_SCALE log2(e) to 1e-12, where the nearest fp32 number is 3e-8 off."""
+    with open(os.path.join(CSRC, "rwkv7_chunk.hip")) as f:
+        m = re.search(r"constexpr float C = (0x[0-9a-f.p+-]+)f, M = (-0x[0-9a-f.p+-]+)f;", f.read())
+    C, M = (float.fromhex(z) for z in m.groups())
+    assert float(np.float32(C)) == C and float(np.float32(M)) == M
+    assert abs(M / C / (-0.6065306597 * 1.4426950408889634) - 1) < 1e-12
