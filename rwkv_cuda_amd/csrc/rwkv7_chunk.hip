@@ -235,7 +235,7 @@ struct SmemCF {
     float dec[2][N];
 };
 // three-term planes and tiles behind it: HOLD A, HOLD R, K and B, v (one term where it is bf16), AK, RB, RK, (I - AB)^{-1}
-constexpr uint32_t F_AS = (sizeof(SmemCF) + 31) / 32 * 32, F_RS = F_AS + PLANE3, F_KB = F_RS + PLANE3, F_V = F_KB + 2 * PAIR3;
+constexpr uint32_t F_AS = (sizeof(SmemCF) + 31) / 32 * 32, F_RS = F_AS + PLANE3, F_KB = F_RS + PLANE3, F_V = F_KB + 2 * TWIN3;
 template <bool F32> constexpr uint32_t F_MA = F_V + (F32 ? PLANE3 : TERM);      // (I - AB)^{-1} and AK
 template <bool F32> constexpr uint32_t F_RKB = F_MA<F32> + TPAIR3;                // RK and RB
 template <bool F32> constexpr uint32_t F_TOTAL = F_RKB<F32> + TPAIR3;
@@ -286,13 +286,13 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
         const lds_t o = sb + piece(lane, q);
         put3(o + F_AS, split3(as)); put3(o + F_RS, split3(rs));
         // (x is not above 1: what comes from bf16 inputs stays within bf16's range)
-        put_pair<TERM2>(sb + F_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(ks), split3<!F32>(bs));
+        put_twin(sb + F_KB + slot * TWIN3 + twin(lane, q), split3<!F32>(ks), split3<!F32>(bs));
         if constexpr (F32) put3(o + F_V, split3(f32x4{vv[0], vv[1], vv[2], vv[3]}));
         else lds_st<u32x2>(o + F_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
         if (q == 0) S.dec[slot][lane] = x[0];
     };
     const Tr ta = tr_bases(sb + (q < 2 ? F_AS : F_RS), l16, g);
-    const lds_t sp = tr_pair(sb + F_KB + ((q & 1) ? 0 : 8), l16, g);
+    const lds_t sp = tr_twin(sb + F_KB + ((q & 1) ? 0 : 32), l16, g);
     fetch(0);
     convert();
     fetch(1);
@@ -304,7 +304,7 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
         {
             f32x4 x;
             auto top = [&](int hb) __attribute__((always_inline)) { return get3_tr(0, ta, hb); };
-            auto sop = [&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, sp + (c & 1) * PAIR3, hb); };
+            auto sop = [&](int hb) __attribute__((always_inline)) { return get3_tr_twin(0, sp + (c & 1) * TWIN3, hb); };
             if (q == 0) {
                 st4(&S.ABt[l16][4 * g], causal_tile<false>(top, sop, true, l16, g) * UNHOLD);
                 // this wave wrote AB itself (LDS keeps a wave's accesses in order): the inverse once, for all four S waves
@@ -343,7 +343,7 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
         if constexpr (KEEP) st4(p.sa + o, ld4(&S.Uo[t][i4]));
     };
     const Tr tr = tr_bases(sb, l16, g);
-    const lds_t pp = sb + piece2(l16, g), vp = sb + F_V + piece(i_own, g);
+    const lds_t pp = sb + piece2(l16, g), vp = sb + F_V + piece(i_own, g), kbs = sb + F_KB + twin(l16, g);
     auto load_v = [&]() __attribute__((always_inline)) {
         if constexpr (F32) return get3(vp); else return lds_ld<u32x2>(vp);
     };
@@ -383,11 +383,11 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
             S.Yo[4 * g + v][i_own] = y[v];
             if constexpr (KEEP) S.Uo[4 * g + v][i_own] = U[v];
         }
-        const lds_t kb = pp + F_KB + (c & 1) * PAIR3;
+        const lds_t kb = kbs + (c & 1) * TWIN3;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
             Sum2 x = SUM0;
-            add32(x, get_pair<TERM2>(kb + 1024 * jt), vu);
+            add32(x, get_twin(kb + TWIN_ROWS * jt), vu);
             St[jt] = St[jt] * ld4(dec + 16 * jt) + total(x);
         }
         __syncthreads();
@@ -444,7 +444,7 @@ struct SmemL {
     Decay part[4][N];
     float dec[2][N];
 };
-constexpr uint32_t L_S = (sizeof(SmemL) + 31) / 32 * 32, L_KB = L_S + PLANE3, L_V = L_KB + 2 * PAIR3;
+constexpr uint32_t L_S = (sizeof(SmemL) + 31) / 32 * 32, L_KB = L_S + PLANE3, L_V = L_KB + 2 * TWIN3;
 template <bool F32> constexpr uint32_t L_MA = L_V + (F32 ? PLANE3 : TERM);
 template <bool F32> constexpr uint32_t L_TOTAL = L_MA<F32> + TPAIR3;
 static_assert(L_TOTAL<true> <= 80 * 1024, "two workgroups a CU");
@@ -489,13 +489,13 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
         const lds_t o = sb + piece(lane, q);
         put3(o + L_S, split3(p1));
         // (x is not above 1: what comes from bf16 inputs stays within bf16's range)
-        put_pair<TERM2>(sb + L_KB + slot * PAIR3 + piece2(lane, q), split3<!F32>(p3), split3<!F32>(p2));
+        put_twin(sb + L_KB + slot * TWIN3 + twin(lane, q), split3<!F32>(p3), split3<!F32>(p2));
         if constexpr (F32) put3(o + L_V, split3(f32x4{widen<F32>(vb[0]), widen<F32>(vb[1]), widen<F32>(vb[2]), widen<F32>(vb[3])}));
         else lds_st<u32x2>(o + L_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
         if (q == (REV ? 3 : 0)) S.dec[slot][lane] = x[REV ? 4 : 0];
     };
     const Tr sp = tr_bases(sb + L_S, l16, g);
-    const lds_t pp = tr_pair(sb + L_KB + (q == 0 ? 8 : 0), l16, g);
+    const lds_t pp = tr_twin(sb + L_KB + (q == 0 ? 32 : 0), l16, g);
     fetch(0);
     convert();
     fetch(1);
@@ -505,7 +505,7 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
     for (int c = 0; c < nch; ++c) {
         if (q < 2) {
             auto one = [&](int hb) __attribute__((always_inline)) { return get3_tr(0, sp, hb); };
-            auto pair = [&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, pp + (c & 1) * PAIR3, hb); };
+            auto pair = [&](int hb) __attribute__((always_inline)) { return get3_tr_twin(0, pp + (c & 1) * TWIN3, hb); };
             f32x4 x;
             if (q == 0) {
                 f32x4 t;
@@ -541,7 +541,7 @@ template <bool F32> DEVINL void local_role_s(SmemL& S, const lds_t sb, float* ou
 #pragma unroll
         for (int v = 0; v < 4; ++v) St[jt][v] = unit && i_own == 16 * jt + 4 * g + v ? 1.f : 0.f;
     const Tr tr = tr_bases(sb, l16, g);
-    const lds_t pp = sb + piece2(l16, g), vp = sb + L_V + piece(i_own, g);
+    const lds_t pp = sb + piece2(l16, g), vp = sb + L_V + piece(i_own, g), kbs = sb + L_KB + twin(l16, g);
     __syncthreads();
     __syncthreads();
     for (int c = 0; c < nch; ++c) {
@@ -557,11 +557,11 @@ template <bool F32> DEVINL void local_role_s(SmemL& S, const lds_t sb, float* ou
         Sum2 Us = SUM0;
         add16(Us, get_half<TTERM2>(pp + L_MA<F32>), split3(total(W) * UNHOLD));
         const Op3 vu = join(as3(vop), split3(total(Us)));
-        const lds_t kb = pp + L_KB + (c & 1) * PAIR3;
+        const lds_t kb = kbs + (c & 1) * TWIN3;
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
             Sum2 x = SUM0;
-            add32(x, get_pair<TERM2>(kb + 1024 * jt), vu);
+            add32(x, get_twin(kb + TWIN_ROWS * jt), vu);
             St[jt] = St[jt] * ld4(dec + 16 * jt) + total(x);
         }
         __syncthreads();
@@ -680,21 +680,21 @@ DEVINL bf16x8 tr16_square(lds_t o, int hb) {       // rows 32 hb + 16 (e >> 2) +
 // dAK for dA, dRB and dRK for dR; by columns (over t) dAB and dRB for dB, dAK and dRK for dK.
 template <bool F32> struct LB {
     static constexpr uint32_t TWO = (sizeof(SmemCB<F32>) + 31) / 32 * 32, EX = F32 ? PLANE3 : TERM;      // from TWO on
-    static constexpr uint32_t AR = 0, BK = PAIR3, U = 2 * PAIR3, V = U + PLANE3, DY = V + EX, ES = DY + EX, DWF = ES + 4 * CL * N, SLOT = DWF + 4 * CL * N;
+    static constexpr uint32_t AR = 0, BK = TWIN3, U = 2 * TWIN3, V = U + PLANE3, DY = V + EX, ES = DY + EX, DWF = ES + 4 * CL * N, SLOT = DWF + 4 * CL * N;
     static constexpr uint32_t ONE = (TWO + 2 * SLOT + 127) / 128 * 128;                                     // from ONE on
     static constexpr uint32_t DS = 0, DW = 3 * DTERM, MB = DW + PLANE3, AKR = MB + TPAIR3;
     static constexpr uint32_t A_ROWS = AKR + TPAIR3, R_ROWS = A_ROWS + TPAIR3, B_COLS = R_ROWS + TPAIR3, K_COLS = B_COLS + TPAIR3, BYTES = ONE + K_COLS + TPAIR3;
 };
 // A lane's addresses in one of the two regions
-struct LaneB { Tr tr; lds_t own, pair, own_pair; };
+struct LaneB { Tr tr; lds_t own, pair, twin, own_twin; };
 DEVINL LaneB lane_bases(lds_t base, int l16, int g, int own) {
-    LaneB b{tr_bases(base, l16, g), base + piece(own, g), base + piece2(l16, g), base + piece2(own, g)};
-    opaque(b.tr.a); opaque(b.tr.b); opaque(b.own); opaque(b.pair); opaque(b.own_pair);
+    LaneB b{tr_bases(base, l16, g), base + piece(own, g), base + piece2(l16, g), base + rwkv::twin(l16, g), base + rwkv::twin(own, g)};
+    opaque(b.tr.a); opaque(b.tr.b); opaque(b.own); opaque(b.pair); opaque(b.twin); opaque(b.own_twin);
     return b;
 }
 // The same lane's addresses in another region, d bytes on (modulo 2^32): an addition each, where bases of its own would be spilled
 DEVINL LaneB moved(const LaneB& b, lds_t d) {
-    return {{b.tr.a + d, b.tr.b + d}, b.own + d, b.pair + d, b.own_pair + d};
+    return {{b.tr.a + d, b.tr.b + d}, b.own + d, b.pair + d, b.twin + d, b.own_twin + d};
 }
 // v, dy: four tokens of a channel, and over channels
 template <bool F32> DEVINL auto exact_piece(lds_t a) { if constexpr (F32) return get3(a); else return lds_ld<u32x2>(a); }
@@ -801,10 +801,10 @@ template <bool F32> DEVINL f32x4 bwd_planes(const lds_t sb, const lds_t slot, fl
     }
     // (rounded products: a remainder fused with one would put into the planes what role B's factors do not hold)
     asm volatile("" : "+v"(as), "+v"(rs), "+v"(bs), "+v"(ks));
-    const lds_t o = sb + O::TWO + slot + piece2(lane, wp);
+    const lds_t o = sb + O::TWO + slot + twin(lane, wp);
     // (x is not above 1: what comes from bf16 inputs stays within bf16's range)
-    put_pair<TERM2>(o + O::AR, split3<!F32>(as), split3<!F32>(rs));
-    put_pair<TERM2>(o + O::BK, split3(bs), split3(ks));
+    put_twin(o + O::AR, split3<!F32>(as), split3<!F32>(rs));
+    put_twin(o + O::BK, split3(bs), split3(ks));
     if (wp == 3) dec[lane] = x[4];
     return {x[1], x[2], x[3], x[4]};
 }
@@ -858,12 +858,12 @@ template <bool F32> DEVINL void bwd_role_p(SmemCB<F32>& S, const lds_t sb, const
     Conv7<F32> y;
     const int l16 = lane & 15, g = lane >> 4;
     using L = LB<F32>;
-    const lds_t tp = tr_pair(sb, l16, g);
+    const lds_t tp = tr_twin(sb, l16, g);
     // a causal tile of a visit
     auto tile = [&](const int visit) __attribute__((always_inline)) {
         const lds_t at = tp + L::TWO + (visit & 1) * L::SLOT;
-        return causal_tile<false>([&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, at + (wp < 2 ? L::AR : L::AR + 8), hb); },
-                                  [&](int hb) __attribute__((always_inline)) { return get3_tr_pair(0, at + (wp & 1 ? L::BK + 8 : L::BK), hb); }, wp < 2, l16, g);
+        return causal_tile<false>([&](int hb) __attribute__((always_inline)) { return get3_tr_twin(0, at + (wp < 2 ? L::AR : L::AR + 32), hb); },
+                                  [&](int hb) __attribute__((always_inline)) { return get3_tr_twin(0, at + (wp & 1 ? L::BK + 32 : L::BK), hb); }, wp < 2, l16, g);
     };
     // its place, of AB the inverse's
     auto put_tile = [&](const f32x4& acc) __attribute__((always_inline)) {
@@ -930,7 +930,7 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
     using L = LB<F32>;
     const LaneB one = lane_bases(sb + L::ONE, l16, g, own);
     const Tr base_tr = tr_bases(sb, l16, g);
-    const lds_t tp = tr_pair(sb, l16, g);
+    const lds_t tp = tr_twin(sb, l16, g);
     const lds_t sq = sb + L::ONE + L::DS + square(own, g);
     auto put_square = [&](int jt, const B3& x) __attribute__((always_inline)) {
         const lds_t o = sq ^ (32u * jt);             // (128-byte rows, and the piece's upper bits are turned by exclusive or)
@@ -962,8 +962,8 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
             const B3 s0 = split3(dS[2 * hb] * ld4(dec + 32 * hb)), s1 = split3(dS[2 * hb + 1] * ld4(dec + 32 * hb + 16));
             put_square(2 * hb, s0); put_square(2 * hb + 1, s1);      // for role B
             const Op3 st = join(s0, s1);
-            add32(dUs, get3_tr_pair(0, bk, hb), st);
-            add32(dVs, get3_tr_pair(8, bk, hb), st);
+            add32(dUs, get3_tr_twin(0, bk, hb), st);
+            add32(dVs, get3_tr_twin(32, bk, hb), st);
         }
         here(dUs); here(dVs);
         __syncthreads();
@@ -986,7 +986,7 @@ template <bool F32> DEVINL void bwd_role_a(SmemCB<F32>& S, const lds_t sb, const
 #pragma unroll
             for (int jt = 0; jt < 4; ++jt) {
                 Sum2 x = SUM0;
-                add32(x, get_pair<TERM2>(two.pair + L::AR + 1024 * jt), wy);
+                add32(x, get_twin(two.twin + L::AR + TWIN_ROWS * jt), wy);
                 dS[jt] = dS[jt] * ld4(dec + 16 * jt) + total(x);
             }
             put_half<TTERM2>(one.pair + (q == 1 ? L::R_ROWS : (q == 0 ? L::R_ROWS + 8 : (q == 3 ? L::B_COLS + 8 : L::K_COLS + 8))), split3(dr));
@@ -1083,7 +1083,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         };
         const f32x4 tA = tile2(L::A_ROWS, bk);
         const f32x4 tB = tile2(L::B_COLS, ar), tK = tile2(L::K_COLS, ar);
-        const f32x4 dwf = lds_ld<f32x4>(one.own_pair - L::ONE + copy_of(visit) + L::DWF);
+        const f32x4 dwf = lds_ld<f32x4>(sb + copy_of(visit) + L::DWF + piece2(16 * q + (me & 15), me >> 4));
         float del[4], ada[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -1120,7 +1120,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         else if (dsT != nullptr) {
             // P at the end of the call: sum_i dsT o S_T with S_T = (S0 + U^T (b e^{-c_{s+1}}) + V^T (k e^{-c_{s+1}})) dec of the last chunk
             const float decj = decay_of(i);
-            const Op3 bk = get_pair<TERM2>(two.own_pair + L::BK);
+            const Op3 bk = get_twin(two.own_twin + L::BK);
             const lds_t row = rows();
             float pp = 0.f;
 #pragma unroll
@@ -1143,7 +1143,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         auto v_of = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::V, two.tr, hb); };
         Op3 s0[2];
         f32x4 xR;
-        ar = get_pair<TERM2>(two.own_pair + L::AR); bk = get_pair<TERM2>(two.own_pair + L::BK);
+        ar = get_twin(two.own_twin + L::AR); bk = get_twin(two.own_twin + L::BK);
         va = value(ar, 0); vr = value(ar, 1); vb = value(bk, 0); vk = value(bk, 1);
         asm volatile("" : "+v"(va), "+v"(vr), "+v"(vb), "+v"(vk));            // (here, or the compiler takes all this to where it is used)
         {
@@ -1162,8 +1162,8 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
         __syncthreads();
         // ---------------------------------------------------------------- phase 3: dW S0; the gradient state
         {
-            er = lds_ld<f32x4>(two.own_pair + L::ES);
             const uint32_t me = lane_again();
+            er = lds_ld<f32x4>(sb + copy_of(i) + L::ES + piece2(16 * q + (me & 15), me >> 4));
             ea0 = lds_ld<float>(sb + copy_of(i) + L::ES + 12 + piece2(16 * q + (me & 15), me > 15 ? (me >> 4) - 1 : 0));
             if (me < 16) ea0 = 1.f;
 #pragma unroll

@@ -126,26 +126,36 @@ DEVINL bf16x8 ld_tr16(const Tr& o, uint32_t plane, int hb) {
 }
 DEVINL Op3 get3_tr(uint32_t plane, const Tr& o, int hb) { return {ld_tr16(o, plane, hb), ld_tr16(o, plane + TERM, hb), ld_tr16(o, plane + 2 * TERM, hb)}; }
 
-// Two planes (x, y) or tiles whose products share instructions, interleaved by pieces: 16 bytes are a side of one instruction.  (Held apart,
-// each would be read by itself and its halves moved together.)  Of a tile a lane holds row l16, columns 4 g + 0..3, as a side of a
-// contraction over the columns takes them.
-constexpr uint32_t TERM2 = 2 * TERM, PAIR3 = 3 * TERM2, TTERM2 = 1024, TPAIR3 = 3 * TTERM2;
-DEVINL lds_t piece2(int ch, int tg) { return static_cast<lds_t>(ch * 64 + 16 * (tg ^ ((ch >> 2) & 3))); }      // of a tile: row, column / 4
-// One of the two planes over channels, as get3_tr: the plane's pieces are every other eight bytes.  The channels' turns repeat every 16, so
-// one address serves both blocks.
-DEVINL lds_t tr_pair(lds_t base, int l16, int g) { return base + piece2(4 * g + (l16 >> 2), l16 & 3); }
-DEVINL bf16x8 ld_tr16_pair(lds_t o, uint32_t plane, int hb) {
+// Two planes (x, y) whose products share instructions, which are also read over channels one by one: a channel's row is 32 bytes of x
+// and 32 of y, 32 bytes more behind every four channels, and its pieces are turned by the channel's number, bits reversed.  So the pieces
+// that half a wave reads or writes meet every bank once: of four channels by four groups, two groups (transposing), of sixteen by two
+// (rows), of 32 channels (P waves).  (x and y in turn, 16 bytes a piece: one instruction reads both, but the transposing reads use half of
+// the banks: in rwkv7c_bwd 38 % of the LDS's active time were conflicts, 23 % so, and the time goes from 599 to 591 us.)
+constexpr uint32_t TWIN = 64 * 64 + 16 * 32, TWIN3 = 3 * TWIN, TWIN_ROWS = 1152;      // a term; 16 channels on
+DEVINL lds_t twin(int ch, int tg) { return static_cast<lds_t>(64 * ch + 32 * (ch >> 2) + 8 * (tg ^ ((ch & 1) << 1 | (ch >> 1 & 1)))); }
+DEVINL void put_twin(lds_t a, const B3& x, const B3& y) {
+    lds_st<u32x2>(a, x.h); lds_st<u32x2>(a + 32, y.h);
+    lds_st<u32x2>(a + TWIN, x.m); lds_st<u32x2>(a + TWIN + 32, y.m);
+    lds_st<u32x2>(a + 2 * TWIN, x.l); lds_st<u32x2>(a + 2 * TWIN + 32, y.l);
+}
+DEVINL Op3 get_twin(lds_t a) {
+    return {op2(lds_ld<u32x2>(a), lds_ld<u32x2>(a + 32)), op2(lds_ld<u32x2>(a + TWIN), lds_ld<u32x2>(a + TWIN + 32)), op2(lds_ld<u32x2>(a + 2 * TWIN), lds_ld<u32x2>(a + 2 * TWIN + 32))};
+}
+// one of the two over channels, as get3_tr (y: 32 bytes on)
+DEVINL lds_t tr_twin(lds_t base, int l16, int g) { return base + twin(4 * g + (l16 >> 2), l16 & 3); }
+DEVINL bf16x8 ld_tr16_twin(lds_t o, uint32_t plane, int hb) {
     typedef short v4s __attribute__((ext_vector_type(4)));
     typedef v4s __attribute__((address_space(3))) * ptr;
-    const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + plane + 2048 * hb)), y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + plane + 2048 * hb + 1024));
+    const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + plane + 2 * TWIN_ROWS * hb)), y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(o + plane + 2 * TWIN_ROWS * hb + TWIN_ROWS));
     return op2(__builtin_bit_cast(u32x2, x), __builtin_bit_cast(u32x2, y));
 }
-DEVINL Op3 get3_tr_pair(uint32_t plane, lds_t o, int hb) { return {ld_tr16_pair(o, plane, hb), ld_tr16_pair(o, plane + TERM2, hb), ld_tr16_pair(o, plane + 2 * TERM2, hb)}; }
-template <uint32_t STRIDE> DEVINL void put_pair(lds_t a, const B3& x, const B3& y) {
-    lds_st<u32x4>(a, u32x4{x.h[0], x.h[1], y.h[0], y.h[1]});
-    lds_st<u32x4>(a + STRIDE, u32x4{x.m[0], x.m[1], y.m[0], y.m[1]});
-    lds_st<u32x4>(a + 2 * STRIDE, u32x4{x.l[0], x.l[1], y.l[0], y.l[1]});
-}
+DEVINL Op3 get3_tr_twin(uint32_t plane, lds_t o, int hb) { return {ld_tr16_twin(o, plane, hb), ld_tr16_twin(o, plane + TWIN, hb), ld_tr16_twin(o, plane + 2 * TWIN, hb)}; }
+
+// Two tiles whose products share instructions, interleaved by pieces: 16 bytes are a side of one instruction.  (Held apart,
+// each would be read by itself and its halves moved together.)  Of a tile a lane holds row l16, columns 4 g + 0..3, as a side of a
+// contraction over the columns takes them.
+constexpr uint32_t TTERM2 = 1024, TPAIR3 = 3 * TTERM2;
+DEVINL lds_t piece2(int row, int piece) { return static_cast<lds_t>(row * 64 + 16 * (piece ^ ((row >> 2) & 3))); }      // (a channel's 16 bytes of four tokens lie so as well)
 template <uint32_t STRIDE> DEVINL void put_half(lds_t a, const B3& x) { lds_st<u32x2>(a, x.h); lds_st<u32x2>(a + STRIDE, x.m); lds_st<u32x2>(a + 2 * STRIDE, x.l); }
 template <uint32_t STRIDE> DEVINL B3 get_half(lds_t a) { return {lds_ld<u32x2>(a), lds_ld<u32x2>(a + STRIDE), lds_ld<u32x2>(a + 2 * STRIDE)}; }
 template <uint32_t STRIDE> DEVINL Op3 get_pair(lds_t a) {
