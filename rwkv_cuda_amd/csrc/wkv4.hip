@@ -404,11 +404,14 @@ __global__ __launch_bounds__(NTS) void wkv4_bwd_seg(int T, int C, int S, const f
 // instead of one dependent load per step and sweep, and the backward needs no workspace.  The arithmetic and its order
 // are those of wkv4_fwd_seg / wkv4_bwd_seg, so the results are the same bit for bit.
 //   CHR channels x NSEG segments per workgroup; SM = the most steps a segment may have (8 with 16 channels, 16 with 8).
-// Workgroups are handed to the chip's 8 XCDs in turn, each with an L2 of its own, and a workgroup's 16 channels are half of
-// a 128-byte line: numbered as launched, the two workgroups that share every line would sit on different XCDs and each
-// L2 would fetch the whole line.  Workgroup x of XCD d takes piece d * (n / 8) + x instead, so neighbours share an L2.
+// Workgroups are handed to the chip's 8 XCDs in turn, each with an L2 of its own, and a workgroup's 8 or 16 channels are a
+// quarter or half of a 128-byte line: numbered as launched, the workgroups that share a line would sit on different XCDs and
+// each L2 would fetch the whole line.  XCD d takes n / 8 adjacent pieces instead (the first n % 8 of them one more), so
+// neighbours share an L2.  Forward / backward, us, numbered as launched -> so: B29 T1000 C700 135 -> 50 / 231 ->
+// 160, B13 T900 C1000 69 -> 32 / 122 -> 82, B2 T4000 C2500 114 -> 84 / 370 -> 335.
 DEVINL int paired_workgroup(int launched, int n) {
-    return n % 16 == 0 ? (launched % 8) * (n / 8) + launched / 8 : launched;
+    return n % 8 == 0 ? (launched % 8) * (n / 8) + launched / 8
+                      : (launched % 8) * (n / 8) + min(launched % 8, n % 8) + launched / 8;
 }
 
 template <bool RAW, int CHR, int SM>

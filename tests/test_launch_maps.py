@@ -39,6 +39,19 @@ def test_wkv4_paired_workgroups_are_a_permutation():
             assert all(inv[q] % 8 == inv[q + 1] % 8 for q in range(0, n, 2))
 
 
+def test_wkv4_neighbours_share_an_xcd_for_any_number_of_workgroups():
+    src = open(os.path.join(CSRC, "wkv4.hip")).read()
+    cond, rest = re.search(r"DEVINL int paired_workgroup\(int launched, int n\) \{\s*return (.+?);\s*\}", src, re.S).group(1).split("?")
+    yes, no = (e.replace("/", "//").strip() for e in rest.split(":"))
+    for n in [1, 7, 8, 9, 15, 16, 17, 23, 24, 25, 98, 686, 1625, 2552]:
+        xcd = {}
+        for launched in range(n):
+            env = {"launched": launched, "n": n, "min": min}
+            xcd[eval(yes if eval(cond.strip(), {}, env) else no, {}, env)] = launched % 8
+        assert sorted(xcd) == list(range(n))
+        assert [xcd[q] for q in range(n)] == sorted(xcd.values())      # one run of adjacent pieces an XCD
+
+
 def test_split_heads_cover_every_block_once():
     for f in ("wkv6_fwd.hip", "wkv6_bwd_a.hip", "wkv6_bwd_b.hip"):
         src = open(os.path.join(CSRC, f)).read()
