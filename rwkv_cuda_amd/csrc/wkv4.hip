@@ -398,12 +398,20 @@ __global__ __launch_bounds__(NTS) void wkv4_bwd_seg(int T, int C, int S, const f
 }
 
 // ---------------------------------------------------------------------------------------- time-parallel, inputs in registers
-// Up to NSEG * 16 = 1024 steps (the reference's own limit, wkv/run.py:149,153) a segment is at most 16 steps long,
+// Up to 1024 steps (the reference's own limit, wkv/run.py:149,153) a segment is at most 16 steps long,
 // and a lane can hold its segment's k, v, gy and, in the backward, what the ascending sweep hands to the descending one
 // (y_t, 1/den_t, zexp_t) in registers: every input is fetched once, all loads of a segment are in flight together
-// instead of one dependent load per step and sweep, and the backward needs no workspace.  The arithmetic and its order
-// are those of wkv4_fwd_seg / wkv4_bwd_seg, so the results are the same bit for bit.
-//   CHR channels x NSEG segments per workgroup; SM = the most steps a segment may have (8 with 16 channels, 16 with 8).
+// instead of one dependent load per step and sweep, and the backward needs no workspace.  The arithmetic is that of
+// wkv4_fwd_seg / wkv4_bwd_seg.
+//   CHR channels x SEG segments per workgroup; SM = the most steps a segment may have.
+// A round of the scan costs a lane about what two steps do, so a sequence is cut into as few segments as the registers allow, and
+// what a workgroup of 512 then has left goes to channels: 8 steps a segment up to 256 steps (69 registers in the backward,
+// three workgroups a CU), 16 beyond (122, two).  us, 64 segments whatever the length, 16 channels up to 512 steps -> so, forward /
+// backward with the 4 us of wkv4_batch_sum: B64 T64 C2048 57 -> 20 / 203 -> 55; B128 T128 C1024 68 -> 33 / 264 -> 98; B64 T256 C1024
+// 47 -> 36 / 182 -> 103; B64 T512 C768 75 -> 69 / 222 -> 168; B32 T400 C1000 36 -> 31 / 121 -> 84.  Half of that in the backward
+// is the workgroup's size: one of 1024 lanes has a CU for itself there (the same segments with 8 channels: B64 T512 C768 222 -> 174).
+// Not kept: 513 to 1024 steps in 128 segments of 8 (B32 T768 C768 backward 155 -> 198), 16 steps a segment up to 256 (103 -> 97, but
+// the smallest calls 6.2 -> 7.0).
 // Workgroups are handed to the chip's 8 XCDs in turn, each with an L2 of its own, and a workgroup's 8 or 16 channels are a
 // quarter or half of a 128-byte line: numbered as launched, the workgroups that share a line would sit on different XCDs and
 // each L2 would fetch the whole line.  XCD d takes n / 8 adjacent pieces instead (the first n % 8 of them one more), so
@@ -414,11 +422,11 @@ DEVINL int paired_workgroup(int launched, int n) {
                       : (launched % 8) * (n / 8) + min(launched % 8, n % 8) + launched / 8;
 }
 
-template <bool RAW, int CHR, int SM>
-__global__ __launch_bounds__(CHR * NSEG) void wkv4_fwd_reg(int T, int C, int S, const float* __restrict__ w_,
+template <bool RAW, int CHR, int SM, int SEG>
+__global__ __launch_bounds__(CHR * SEG) void wkv4_fwd_reg(int T, int C, int S, const float* __restrict__ w_,
                                                           const float* __restrict__ u_, const float* __restrict__ k_,
                                                           const float* __restrict__ v_, float* __restrict__ y_) {
-    __shared__ State3 X[2][NSEG][CHR];
+    __shared__ State3 X[2][SEG][CHR];
     const int cl = threadIdx.x % CHR, s = threadIdx.x / CHR;
     const int q = paired_workgroup(blockIdx.x, gridDim.x), nx = (C + CHR - 1) / CHR;
     const int c = (q % nx) * CHR + cl, b = q / nx;
@@ -452,7 +460,7 @@ __global__ __launch_bounds__(CHR * NSEG) void wkv4_fwd_reg(int T, int C, int S, 
     __syncthreads();
     int cur = 0;
 #pragma unroll
-    for (int d = 1; d < NSEG; d *= 2) {
+    for (int d = 1; d < SEG; d *= 2) {
         State3 mine = X[cur][s][cl];
         if (s >= d) {
             State3 older = X[cur][s - d][cl];
@@ -482,13 +490,13 @@ __global__ __launch_bounds__(CHR * NSEG) void wkv4_fwd_reg(int T, int C, int S, 
     }
 }
 
-template <bool RAW, int CHR, int SM>
-__global__ __launch_bounds__(CHR * NSEG) void wkv4_bwd_reg(int T, int C, int S, const float* __restrict__ w_,
+template <bool RAW, int CHR, int SM, int SEG>
+__global__ __launch_bounds__(CHR * SEG, 4) void wkv4_bwd_reg(int T, int C, int S, const float* __restrict__ w_,
                                                           const float* __restrict__ u_, const float* __restrict__ k_,
                                                           const float* __restrict__ v_, const float* __restrict__ gy_,
                                                           float* __restrict__ gw_, float* __restrict__ gu_,
                                                           float* __restrict__ gk_, float* __restrict__ gv_) {
-    __shared__ State5 X[2][NSEG][CHR];
+    __shared__ State5 X[2][SEG][CHR];
     const int cl = threadIdx.x % CHR, s = threadIdx.x / CHR;
     const int q = paired_workgroup(blockIdx.x, gridDim.x), nx = (C + CHR - 1) / CHR;
     const int c = (q % nx) * CHR + cl, b = q / nx;
@@ -532,7 +540,7 @@ __global__ __launch_bounds__(CHR * NSEG) void wkv4_bwd_reg(int T, int C, int S, 
     __syncthreads();
     int cur = 0;
 #pragma unroll
-    for (int d = 1; d < NSEG; d *= 2) {
+    for (int d = 1; d < SEG; d *= 2) {
         State5 mine = X[cur][s][cl];
         if (s >= d) {
             State5 older = X[cur][s - d][cl];
@@ -591,13 +599,13 @@ __global__ __launch_bounds__(CHR * NSEG) void wkv4_bwd_reg(int T, int C, int S, 
             g.o = no;
         }
     }
-    State3 (*G)[NSEG][CHR] = reinterpret_cast<State3 (*)[NSEG][CHR]>(&X[0][0][0]);  // [2][NSEG][CHR], inside X
-    const int rs = NSEG - 1 - s;                   // position in the descending order
+    State3 (*G)[SEG][CHR] = reinterpret_cast<State3 (*)[SEG][CHR]>(&X[0][0][0]);  // [2][SEG][CHR], inside X
+    const int rs = SEG - 1 - s;                   // position in the descending order
     G[0][rs][cl] = g;
     __syncthreads();
     cur = 0;
 #pragma unroll
-    for (int d = 1; d < NSEG; d *= 2) {
+    for (int d = 1; d < SEG; d *= 2) {
         State3 mine = G[cur][rs][cl];
         if (rs >= d) {
             State3 older = G[cur][rs - d][cl];
@@ -633,12 +641,12 @@ __global__ __launch_bounds__(CHR * NSEG) void wkv4_bwd_reg(int T, int C, int S, 
     }
 
     // ---- gw, gu: the segments' sums, added in time order
-    float2* part = reinterpret_cast<float2*>(&X[0][0][0]);                         // [NSEG][CHR]
+    float2* part = reinterpret_cast<float2*>(&X[0][0][0]);                         // [SEG][CHR]
     part[s * CHR + cl] = make_float2(gw, gu);
     __syncthreads();
     if (s == 0 && live) {
         float a = 0.f, bsum = 0.f;
-        for (int z = 0; z < NSEG; ++z) { a += part[z * CHR + cl].x; bsum += part[z * CHR + cl].y; }
+        for (int z = 0; z < SEG; ++z) { a += part[z * CHR + cl].x; bsum += part[z * CHR + cl].y; }
         // the caller's buffers are accumulated into, as the reference does (wkv_cuda_v2.cu:112-113)
         if constexpr (RAW) {                        // per-batch partials in the library's own scratch: plain stores
             gw_[static_cast<size_t>(b) * C + c] = a * w;
@@ -651,12 +659,17 @@ __global__ __launch_bounds__(CHR * NSEG) void wkv4_bwd_reg(int T, int C, int S, 
 }
 
 // ------------------------------------------------------------------------------- longer sequences: blocks of 512 steps
-// Beyond NSEG * 16 steps a workgroup walks over blocks of NSEG * 8 steps and hands the state from block to block: inside
+// Beyond 1024 steps a workgroup walks over blocks of 512 steps and hands the state from block to block: inside
 // a block everything is as in the register kernels, and the state in front of a segment is the block's entering state,
 // aged by the steps in between, combined with the segments of the block before it.  The backward first walks up with
 // the ascending sweep's summaries only (k, v read, nothing written) to learn the state entering every block, keeps those
 // in LDS, then walks down block by block doing both sweeps.  k and v are read twice, gy once, nothing is parked in memory.
-constexpr int BLK_S = 8, BLK_T = NSEG * BLK_S, BLK_CH = 16;
+// CHR, SM, SEG as above.  Forward: 16 channels, 64 segments of 8 steps.  Backward: 16 channels, 32 segments of 16, half the rounds of the
+// scans and two workgroups a CU: us, 64 segments -> so, B28 T1100 C768 306 -> 221, B17 T2000 C768 325 -> 242, B6 T4000 C768 323 -> 240, B2 T4000
+// C2500 335 -> 221 (the forward that way: B12 T4000 C768 156 -> 169, B17 T2000 C768 100 -> 97).
+// Where pieces of 16 channels leave half of the CUs without work, both take 8 channels and 64 segments: B2 T4000 C768 52 -> 44 /
+// 145 -> 116 (backward in 32 segments: 137), B1 T4096 C2048 51 -> 43 / 142 -> 107 (138); with 144 pieces it is 53 -> 56 / 147 -> 143 (140).
+constexpr int BLK_T = 512;
 constexpr int BLK_MAX = 64;            // blocks whose entering states fit in LDS: T <= 32768
 
 DEVINL State3 aged(State3 a, float steps, float w) { a.o += steps * w; return a; }
@@ -667,14 +680,15 @@ DEVINL State5 aged(State5 a, float steps, float w) {
     return a;
 }
 
-template <bool RAW>
-__global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_fwd_blk(int T, int C, const float* __restrict__ w_,
+template <bool RAW, int CHR, int SM, int SEG>
+__global__ __launch_bounds__(CHR * SEG) void wkv4_fwd_blk(int T, int C, const float* __restrict__ w_,
                                                              const float* __restrict__ u_, const float* __restrict__ k_,
                                                              const float* __restrict__ v_, float* __restrict__ y_) {
-    __shared__ State3 X[2][NSEG][BLK_CH];
-    const int cl = threadIdx.x % BLK_CH, s = threadIdx.x / BLK_CH;
-    const int q = paired_workgroup(blockIdx.x, gridDim.x), nx = (C + BLK_CH - 1) / BLK_CH;
-    const int c = (q % nx) * BLK_CH + cl, b = q / nx;
+    static_assert(SM * SEG == BLK_T);
+    __shared__ State3 X[2][SEG][CHR];
+    const int cl = threadIdx.x % CHR, s = threadIdx.x / CHR;
+    const int q = paired_workgroup(blockIdx.x, gridDim.x), nx = (C + CHR - 1) / CHR;
+    const int c = (q % nx) * CHR + cl, b = q / nx;
     const bool live = c < C;
     const int cc = live ? c : C - 1;
     const float u = u_[cc], w = RAW ? -expf(w_[cc]) : w_[cc];        // RAW: the wrapper's w = -exp(w_raw) done here
@@ -682,20 +696,20 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_fwd_blk(int T, int C, cons
     State3 carry = {0.f, 0.f, O_INIT};             // the state entering the block; every lane of a channel holds it
 
     for (int blk = 0; blk < nblk; ++blk) {
-        const int t0 = min(blk * BLK_T + s * BLK_S, T), n = live ? min(t0 + BLK_S, T) - t0 : 0;
+        const int t0 = min(blk * BLK_T + s * SM, T), n = live ? min(t0 + SM, T) - t0 : 0;
         const size_t off = (static_cast<size_t>(b) * T + t0) * C + cc;
         const float* __restrict__ k = k_ + off;
         const float* __restrict__ v = v_ + off;
         float* __restrict__ y = y_ + off;
-        float kk[BLK_S], vv[BLK_S];
+        float kk[SM], vv[SM];
 #pragma unroll
-        for (int j = 0; j < BLK_S; ++j) {
+        for (int j = 0; j < SM; ++j) {
             kk[j] = 0.f; vv[j] = 0.f;
             if (j < n) { kk[j] = k[static_cast<size_t>(j) * C]; vv[j] = v[static_cast<size_t>(j) * C]; }
         }
         State3 x = {0.f, 0.f, O_INIT};
 #pragma unroll
-        for (int j = 0; j < BLK_S; ++j) {
+        for (int j = 0; j < SM; ++j) {
             if (j < n) {
                 const ExpPair e = exp_pair(w + x.o, kk[j]);
                 x.p = e.ea * x.p + e.eb * vv[j];
@@ -707,18 +721,18 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_fwd_blk(int T, int C, cons
         __syncthreads();
         int cur = 0;
 #pragma unroll
-        for (int d = 1; d < NSEG; d *= 2) {
+        for (int d = 1; d < SEG; d *= 2) {
             State3 mine = X[cur][s][cl];
-            if (s >= d) mine = combine(aged(X[cur][s - d][cl], static_cast<float>(d * BLK_S), w), mine);
+            if (s >= d) mine = combine(aged(X[cur][s - d][cl], static_cast<float>(d * SM), w), mine);
             X[cur ^ 1][s][cl] = mine;
             cur ^= 1;
             __syncthreads();
         }
-        x = aged(carry, static_cast<float>(s * BLK_S), w);
+        x = aged(carry, static_cast<float>(s * SM), w);
         if (s > 0) x = combine(x, X[cur][s - 1][cl]);
-        carry = combine(aged(carry, static_cast<float>(BLK_T), w), X[cur][NSEG - 1][cl]);
+        carry = combine(aged(carry, static_cast<float>(BLK_T), w), X[cur][SEG - 1][cl]);
 #pragma unroll
-        for (int j = 0; j < BLK_S; ++j) {
+        for (int j = 0; j < SM; ++j) {
             if (j < n) {
                 ExpPair e = exp_pair(x.o, u + kk[j]);
                 y[static_cast<size_t>(j) * C] = (e.ea * x.p + e.eb * vv[j]) * recip(e.ea * x.q + e.eb);
@@ -732,17 +746,18 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_fwd_blk(int T, int C, cons
     }
 }
 
-template <bool RAW>
-__global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, const float* __restrict__ w_,
+template <bool RAW, int CHR, int SM, int SEG>
+__global__ __launch_bounds__(CHR * SEG, 4) void wkv4_bwd_blk(int T, int C, const float* __restrict__ w_,
                                                              const float* __restrict__ u_, const float* __restrict__ k_,
                                                              const float* __restrict__ v_, const float* __restrict__ gy_,
                                                              float* __restrict__ gw_, float* __restrict__ gu_,
                                                              float* __restrict__ gk_, float* __restrict__ gv_) {
-    __shared__ State5 X[2][NSEG][BLK_CH];
-    __shared__ State5 ENTER[BLK_MAX][BLK_CH];      // the ascending sweep's state entering each block
-    const int cl = threadIdx.x % BLK_CH, s = threadIdx.x / BLK_CH;
-    const int q = paired_workgroup(blockIdx.x, gridDim.x), nx = (C + BLK_CH - 1) / BLK_CH;
-    const int c = (q % nx) * BLK_CH + cl, b = q / nx;
+    static_assert(SM * SEG == BLK_T);
+    __shared__ State5 X[2][SEG][CHR];
+    __shared__ State5 ENTER[BLK_MAX][CHR];      // the ascending sweep's state entering each block
+    const int cl = threadIdx.x % CHR, s = threadIdx.x / CHR;
+    const int q = paired_workgroup(blockIdx.x, gridDim.x), nx = (C + CHR - 1) / CHR;
+    const int c = (q % nx) * CHR + cl, b = q / nx;
     const bool live = c < C;
     const int cc = live ? c : C - 1;
     const float u = u_[cc], w = RAW ? -expf(w_[cc]) : w_[cc];        // RAW: the wrapper's w = -exp(w_raw) done here
@@ -750,10 +765,10 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
     const size_t row = static_cast<size_t>(b) * T;
 
     // the segment alone, from the empty state, then the scan over the block's segments: X[cur] holds the inclusive prefixes
-    auto summaries = [&](const float (&kk)[BLK_S], const float (&vv)[BLK_S], int n) -> int {
+    auto summaries = [&](const float (&kk)[SM], const float (&vv)[SM], int n) -> int {
         State5 x = {0.f, 0.f, 0.f, 0.f, O_INIT};
 #pragma unroll
-        for (int j = 0; j < BLK_S; ++j) {
+        for (int j = 0; j < SM; ++j) {
             if (j < n) {
                 const ExpPair e = exp_pair(w + x.o, kk[j]);
                 x.dp = e.ea * (x.p + x.dp);
@@ -767,9 +782,9 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
         __syncthreads();
         int cur = 0;
 #pragma unroll
-        for (int d = 1; d < NSEG; d *= 2) {
+        for (int d = 1; d < SEG; d *= 2) {
             State5 mine = X[cur][s][cl];
-            if (s >= d) mine = combine(aged(X[cur][s - d][cl], static_cast<float>(d * BLK_S), w), mine);
+            if (s >= d) mine = combine(aged(X[cur][s - d][cl], static_cast<float>(d * SM), w), mine);
             X[cur ^ 1][s][cl] = mine;
             cur ^= 1;
             __syncthreads();
@@ -782,16 +797,16 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
     for (int blk = 0; blk < nblk; ++blk) {
         if (s == 0) ENTER[blk][cl] = carry;
         if (blk == nblk - 1) break;
-        const int t0 = min(blk * BLK_T + s * BLK_S, T), n = live ? min(t0 + BLK_S, T) - t0 : 0;
+        const int t0 = min(blk * BLK_T + s * SM, T), n = live ? min(t0 + SM, T) - t0 : 0;
         const size_t off = (row + t0) * C + cc;
-        float kk[BLK_S], vv[BLK_S];
+        float kk[SM], vv[SM];
 #pragma unroll
-        for (int j = 0; j < BLK_S; ++j) {
+        for (int j = 0; j < SM; ++j) {
             kk[j] = 0.f; vv[j] = 0.f;
             if (j < n) { kk[j] = k_[off + static_cast<size_t>(j) * C]; vv[j] = v_[off + static_cast<size_t>(j) * C]; }
         }
         const int cur = summaries(kk, vv, n);
-        carry = combine(aged(carry, static_cast<float>(BLK_T), w), X[cur][NSEG - 1][cl]);
+        carry = combine(aged(carry, static_cast<float>(BLK_T), w), X[cur][SEG - 1][cl]);
         __syncthreads();                           // X is written again by the next block
     }
     __syncthreads();
@@ -799,15 +814,15 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
     // ---- down: both sweeps of a block, the descending sweep's state handed from block to block
     State3 gcarry = {0.f, 0.f, O_INIT};
     float gw = 0.f, gu = 0.f;
-    const int rs = NSEG - 1 - s;                   // position in the descending order
+    const int rs = SEG - 1 - s;                   // position in the descending order
     for (int blk = nblk - 1; blk >= 0; --blk) {
-        const int t0 = min(blk * BLK_T + s * BLK_S, T), n = live ? min(t0 + BLK_S, T) - t0 : 0;
+        const int t0 = min(blk * BLK_T + s * SM, T), n = live ? min(t0 + SM, T) - t0 : 0;
         const size_t off = (row + t0) * C + cc;
         float* __restrict__ gk = gk_ + off;
         float* __restrict__ gv = gv_ + off;
-        float kk[BLK_S], vv[BLK_S], gg[BLK_S], yy[BLK_S], zz[BLK_S], ze[BLK_S];
+        float kk[SM], vv[SM], gg[SM], yy[SM], zz[SM], ze[SM];
 #pragma unroll
-        for (int j = 0; j < BLK_S; ++j) {
+        for (int j = 0; j < SM; ++j) {
             kk[j] = 0.f; vv[j] = 0.f; gg[j] = 0.f;
             if (j < n) {
                 kk[j] = k_[off + static_cast<size_t>(j) * C]; vv[j] = v_[off + static_cast<size_t>(j) * C];
@@ -815,13 +830,13 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
             }
         }
         int cur = summaries(kk, vv, n);
-        State5 x = aged(ENTER[blk][cl], static_cast<float>(s * BLK_S), w);
+        State5 x = aged(ENTER[blk][cl], static_cast<float>(s * SM), w);
         if (s > 0) x = combine(x, X[cur][s - 1][cl]);
         __syncthreads();                           // X is reused below
 
         // ascending, from the true state
 #pragma unroll
-        for (int j = 0; j < BLK_S; ++j) {
+        for (int j = 0; j < SM; ++j) {
             yy[j] = 0.f; zz[j] = 0.f; ze[j] = 0.f;
             if (j < n) {
                 const float kt = kk[j], vt = vv[j], gt = gg[j];
@@ -845,7 +860,7 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
         // descending: the segment alone (p, q stand for gp, gq)
         State3 g = {0.f, 0.f, O_INIT};
 #pragma unroll
-        for (int j = BLK_S - 1; j >= 0; --j) {
+        for (int j = SM - 1; j >= 0; --j) {
             if (j < n) {
                 const ExpPair e = exp_pair(w + g.o, ze[j] - kk[j] - u);
                 const float Bq = gg[j] * zz[j] * e.eb;
@@ -854,26 +869,26 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
                 g.o = e.no;
             }
         }
-        State3 (*G)[NSEG][BLK_CH] = reinterpret_cast<State3 (*)[NSEG][BLK_CH]>(&X[0][0][0]);    // [2][NSEG][BLK_CH], inside X
+        State3 (*G)[SEG][CHR] = reinterpret_cast<State3 (*)[SEG][CHR]>(&X[0][0][0]);    // [2][SEG][CHR], inside X
         G[0][rs][cl] = g;
         __syncthreads();
         cur = 0;
 #pragma unroll
-        for (int d = 1; d < NSEG; d *= 2) {
+        for (int d = 1; d < SEG; d *= 2) {
             State3 mine = G[cur][rs][cl];
-            if (rs >= d) mine = combine(aged(G[cur][rs - d][cl], static_cast<float>(d * BLK_S), w), mine);
+            if (rs >= d) mine = combine(aged(G[cur][rs - d][cl], static_cast<float>(d * SM), w), mine);
             G[cur ^ 1][rs][cl] = mine;
             cur ^= 1;
             __syncthreads();
         }
-        g = aged(gcarry, static_cast<float>(rs * BLK_S), w);
+        g = aged(gcarry, static_cast<float>(rs * SM), w);
         if (rs > 0) g = combine(g, G[cur][rs - 1][cl]);
-        gcarry = combine(aged(gcarry, static_cast<float>(BLK_T), w), G[cur][NSEG - 1][cl]);
+        gcarry = combine(aged(gcarry, static_cast<float>(BLK_T), w), G[cur][SEG - 1][cl]);
         __syncthreads();                           // X is written again by the next block
 
         // descending, from the true state
 #pragma unroll
-        for (int j = BLK_S - 1; j >= 0; --j) {
+        for (int j = SM - 1; j >= 0; --j) {
             if (j < n) {
                 const float kt = kk[j], vt = vv[j], gt = gg[j];
                 const float y = yy[j], z = zz[j], zexp = ze[j];
@@ -891,12 +906,12 @@ __global__ __launch_bounds__(BLK_CH * NSEG) void wkv4_bwd_blk(int T, int C, cons
     }
 
     // ---- gw, gu: the segments' sums, added in time order
-    float2* part = reinterpret_cast<float2*>(&X[0][0][0]);                         // [NSEG][BLK_CH]
-    part[s * BLK_CH + cl] = make_float2(gw, gu);
+    float2* part = reinterpret_cast<float2*>(&X[0][0][0]);                         // [SEG][CHR]
+    part[s * CHR + cl] = make_float2(gw, gu);
     __syncthreads();
     if (s == 0 && live) {
         float a = 0.f, bsum = 0.f;
-        for (int z = 0; z < NSEG; ++z) { a += part[z * BLK_CH + cl].x; bsum += part[z * BLK_CH + cl].y; }
+        for (int z = 0; z < SEG; ++z) { a += part[z * CHR + cl].x; bsum += part[z * CHR + cl].y; }
         // the caller's buffers are accumulated into, as the reference does (wkv_cuda_v2.cu:112-113)
         if constexpr (RAW) {                        // per-batch partials in the library's own scratch: plain stores
             gw_[static_cast<size_t>(b) * C + c] = a * w;
@@ -929,28 +944,46 @@ __global__ __launch_bounds__(256) void wkv4_batch_sum(int B, int C, const float*
 // Which form runs: one lane per scan beyond the grid's y range, inputs in registers while a segment has at most 16
 // steps, blocks of 512 steps with the state handed on up to 32768 steps, and beyond that the form that parks the ascending
 // sweep's results in memory.
-template <bool RAW, int CHR, int SM, typename... Ptrs>
-void launch4_fwd_reg(hipStream_t st, int B, int T, int C, int S, Ptrs... p) {
-    hipLaunchKernelGGL((wkv4_fwd_reg<RAW, CHR, SM>), dim3(((C + CHR - 1) / CHR) * B), dim3(CHR * NSEG), 0, st, T, C, S, p...);
+template <int CHR> dim3 pieces4(int B, int C) { return dim3(((C + CHR - 1) / CHR) * B); }
+template <bool RAW, int CHR, int SM, int SEG, typename... Ptrs>
+void launch4_fwd_reg(hipStream_t st, int B, int T, int C, Ptrs... p) {
+    hipLaunchKernelGGL((wkv4_fwd_reg<RAW, CHR, SM, SEG>), pieces4<CHR>(B, C), dim3(CHR * SEG), 0, st, T, C, (T + SEG - 1) / SEG, p...);
 }
-template <bool RAW, int CHR, int SM, typename... Ptrs>
-void launch4_bwd_reg(hipStream_t st, int B, int T, int C, int S, Ptrs... p) {
-    hipLaunchKernelGGL((wkv4_bwd_reg<RAW, CHR, SM>), dim3(((C + CHR - 1) / CHR) * B), dim3(CHR * NSEG), 0, st, T, C, S, p...);
+template <bool RAW, int CHR, int SM, int SEG, typename... Ptrs>
+void launch4_bwd_reg(hipStream_t st, int B, int T, int C, Ptrs... p) {
+    hipLaunchKernelGGL((wkv4_bwd_reg<RAW, CHR, SM, SEG>), pieces4<CHR>(B, C), dim3(CHR * SEG), 0, st, T, C, (T + SEG - 1) / SEG, p...);
 }
+template <bool RAW, int CHR, int SM, int SEG, typename... Ptrs>
+void launch4_fwd_blk(hipStream_t st, int B, int T, int C, Ptrs... p) {
+    hipLaunchKernelGGL((wkv4_fwd_blk<RAW, CHR, SM, SEG>), pieces4<CHR>(B, C), dim3(CHR * SEG), 0, st, T, C, p...);
+}
+template <bool RAW, int CHR, int SM, int SEG, typename... Ptrs>
+void launch4_bwd_blk(hipStream_t st, int B, int T, int C, Ptrs... p) {
+    hipLaunchKernelGGL((wkv4_bwd_blk<RAW, CHR, SM, SEG>), pieces4<CHR>(B, C), dim3(CHR * SEG), 0, st, T, C, p...);
+}
+// pieces of 16 channels that leave half of the 256 CUs without work
+bool few_pieces(int B, int C) { return static_cast<long long>(B) * ((C + 15) / 16) <= 128; }
 
 template <bool RAW>
 void launch4_fwd(hipStream_t st, int B, int T, int C, const float* w, const float* u, const float* k, const float* v, float* y) {
-    const int S = (T + NSEG - 1) / NSEG;
     if (B > 65535) {
         const int BC = B * C;
         hipLaunchKernelGGL((wkv4_fwd<RAW>), dim3((BC + NT - 1) / NT), dim3(NT), 0, st, BC, T, C, w, u, k, v, y);
-    } else if (S <= 8) {
-        launch4_fwd_reg<RAW, 16, 8>(st, B, T, C, S, w, u, k, v, y);
-    } else if (S <= 16) {
-        launch4_fwd_reg<RAW, 8, 16>(st, B, T, C, S, w, u, k, v, y);
+    } else if (T <= 64) {
+        launch4_fwd_reg<RAW, 64, 8, 8>(st, B, T, C, w, u, k, v, y);
+    } else if (T <= 128) {
+        launch4_fwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, y);
+    } else if (T <= 256) {
+        launch4_fwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, y);
+    } else if (T <= 512) {
+        launch4_fwd_reg<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, y);
+    } else if (T <= 1024) {
+        launch4_fwd_reg<RAW, 8, 16, 64>(st, B, T, C, w, u, k, v, y);
     } else if (T <= BLK_T * BLK_MAX) {
-        hipLaunchKernelGGL((wkv4_fwd_blk<RAW>), dim3(((C + BLK_CH - 1) / BLK_CH) * B), dim3(BLK_CH * NSEG), 0, st, T, C, w, u, k, v, y);
+        if (few_pieces(B, C)) launch4_fwd_blk<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, y);
+        else launch4_fwd_blk<RAW, 16, 8, 64>(st, B, T, C, w, u, k, v, y);
     } else {
+        const int S = (T + NSEG - 1) / NSEG;
         hipLaunchKernelGGL((wkv4_fwd_seg<RAW>), dim3((C + CH - 1) / CH, B), dim3(NTS), 0, st, T, C, S, w, u, k, v, y);
     }
 }
@@ -958,25 +991,31 @@ void launch4_fwd(hipStream_t st, int B, int T, int C, const float* w, const floa
 template <bool RAW>
 void launch4_bwd(hipStream_t st, int B, int T, int C, const float* w, const float* u, const float* k, const float* v,
                  const float* gy, float* gw, float* gu, float* gk, float* gv, float* ze) {
-    const int S = (T + NSEG - 1) / NSEG;
     if (B > 65535) {
         const int BC = B * C;
         hipLaunchKernelGGL((wkv4_bwd<RAW>), dim3((BC + NT - 1) / NT), dim3(NT), 0, st, BC, T, C, w, u, k, v, gy, gw, gu, gk, gv, ze);
-    } else if (S <= 8) {
-        launch4_bwd_reg<RAW, 16, 8>(st, B, T, C, S, w, u, k, v, gy, gw, gu, gk, gv);
-    } else if (S <= 16) {
-        launch4_bwd_reg<RAW, 8, 16>(st, B, T, C, S, w, u, k, v, gy, gw, gu, gk, gv);
+    } else if (T <= 64) {
+        launch4_bwd_reg<RAW, 64, 8, 8>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+    } else if (T <= 128) {
+        launch4_bwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+    } else if (T <= 256) {
+        launch4_bwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+    } else if (T <= 512) {
+        launch4_bwd_reg<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+    } else if (T <= 1024) {
+        launch4_bwd_reg<RAW, 8, 16, 64>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else if (T <= BLK_T * BLK_MAX) {
-        hipLaunchKernelGGL((wkv4_bwd_blk<RAW>), dim3(((C + BLK_CH - 1) / BLK_CH) * B), dim3(BLK_CH * NSEG), 0, st, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        if (few_pieces(B, C)) launch4_bwd_blk<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        else launch4_bwd_blk<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else {
+        const int S = (T + NSEG - 1) / NSEG;
         hipLaunchKernelGGL((wkv4_bwd_seg<RAW>), dim3((C + CH - 1) / CH, B), dim3(NTS), 0, st, T, C, S, w, u, k, v, gy, gw, gu, gk, gv, ze);
     }
 }
 
 // the forms of launch4_bwd that take the workspace `ze` (the plain kernel and the one for very long sequences)
 bool bwd_uses_workspace(int B, int T) {
-    const int S = (T + NSEG - 1) / NSEG;
-    return B > 65535 || (S > 16 && T > BLK_T * BLK_MAX);
+    return B > 65535 || T > BLK_T * BLK_MAX;
 }
 
 int check4(int B, int T, int C) {
