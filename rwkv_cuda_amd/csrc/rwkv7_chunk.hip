@@ -73,6 +73,7 @@ struct Args7c {
     // E and M of the blocks but the last in the direction of travel), the states entering the blocks but the first (enter), whether the
     // head is done as a whole (flags)
     int NB, per;
+    int at;       // this launch's first head, batch row by batch row (local, enter and flags begin with it)
     float *local, *enter;
     int* flags;
 };
@@ -83,13 +84,19 @@ template <bool CUT> DEVINL Args7c only_whole(Args7c p) {
     if constexpr (!CUT) p.NB = 1;
     return p;
 }
+// head n of the launch
+struct Head7 { size_t bh; int b, h; };
+DEVINL Head7 head_of(const Args7c& p, int n) {
+    const int bh = p.at + n, b = __builtin_amdgcn_readfirstlane(bh / p.H);
+    return {static_cast<size_t>(bh), b, bh - b * p.H};
+}
 // The chunks of the workgroup's block; false: another workgroup does them.
 struct Part7 { int n, first, chunks; };
-DEVINL bool part_of(const Args7c& p, size_t bh, Part7& x) {
+DEVINL bool part_of(const Args7c& p, Part7& x) {
     const int nch = p.T / CL;
     x = {0, 0, nch};
     if (p.NB == 1) return true;
-    if (__builtin_amdgcn_readfirstlane(p.flags[bh]) != 0) return blockIdx.z == 0;
+    if (__builtin_amdgcn_readfirstlane(p.flags[blockIdx.x]) != 0) return blockIdx.z == 0;
     x.n = blockIdx.z; x.first = x.n * p.per; x.chunks = min(p.per, nch - x.first);
     return true;
 }
@@ -419,14 +426,13 @@ __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c args) {
     SmemCF& S = *reinterpret_cast<SmemCF*>(smem_raw);
     const lds_t sb = lds_of(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = blockIdx.x, b = blockIdx.y;
-    const size_t bh = static_cast<size_t>(b) * p.H + h;
+    const auto [bh, b, h] = head_of(p, blockIdx.x);
     Part7 x;
-    if (!part_of(p, bh, x)) return;
+    if (!part_of(p, x)) return;
     const size_t tok0 = static_cast<size_t>(b) * p.T + x.first * CL;  // first token row of this block
     if (w < 4) {
         const int all = p.T / CL;
-        const float* const s0 = x.n > 0 ? p.enter + (bh * (p.NB - 1) + x.n - 1) * N * N : (p.s0 != nullptr ? p.s0 + bh * N * N : nullptr);
+        const float* const s0 = x.n > 0 ? p.enter + (static_cast<size_t>(blockIdx.x) * (p.NB - 1) + x.n - 1) * N * N : (p.s0 != nullptr ? p.s0 + bh * N * N : nullptr);
         float* const sT = p.sT != nullptr && x.first + x.chunks == all ? p.sT + bh * N * N : nullptr;
         fwd_role_s<F32, KEEP>(S, sb, p, s0, sT, KEEP ? p.s + (bh * all + x.first) * N * N : nullptr, w, tid, tok0, x.chunks, h);
     } else fwd_role_p<F32>(S, sb, p, w - 4, tid & 63, tok0, x.chunks, h);
@@ -580,13 +586,13 @@ __global__ __launch_bounds__(NTF, 4) void rwkv7c_local(const Args7c p) {
     SmemL& S = *reinterpret_cast<SmemL*>(smem_raw);
     const lds_t sb = lds_of(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = blockIdx.x, b = blockIdx.y, m = blockIdx.z >> 1, n = REV ? p.NB - 1 - m : m;
+    const int m = blockIdx.z >> 1, n = REV ? p.NB - 1 - m : m;
     const bool unit = blockIdx.z & 1;
-    const size_t bh = static_cast<size_t>(b) * p.H + h;
-    if (blockIdx.z == 0 && tid == 0) p.flags[bh] = 0;
+    const auto [bh, b, h] = head_of(p, blockIdx.x);
+    if (blockIdx.z == 0 && tid == 0) p.flags[blockIdx.x] = 0;
     const int chunks = min(p.per, p.T / CL - n * p.per);
     const size_t tok0 = static_cast<size_t>(b) * p.T + static_cast<size_t>(n) * p.per * CL;
-    if (w < 4) local_role_s<F32>(S, sb, p.local + ((bh * (p.NB - 1) + m) * 2 + unit) * N * N, unit, w, tid & 63, chunks);
+    if (w < 4) local_role_s<F32>(S, sb, p.local + ((static_cast<size_t>(blockIdx.x) * (p.NB - 1) + m) * 2 + unit) * N * N, unit, w, tid & 63, chunks);
     else local_role_p<F32, REV>(S, sb, p, unit, w - 4, tid & 63, tok0, chunks, h);
 }
 // X_0 = s0 (backward: dsT), X_{m+1} = X_m M_m + E_m: a chain of NB - 1 small products; the next block's matrices are under way.
@@ -594,16 +600,16 @@ template <bool REV>
 __global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
     __shared__ float X[2][16][PS];
     const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
-    const int rows = blockIdx.x & 3, h = blockIdx.x >> 2;
-    const size_t bh = static_cast<size_t>(blockIdx.y) * p.H + h;
+    const int rows = blockIdx.x & 3;
+    const size_t head = blockIdx.x >> 2;
     const float* const init = REV ? p.dsT : p.s0;
     const uint32_t o = (16 * rows + 4 * g) * N + 16 * q + l16;       // element [4 g][16 q + l16] of these rows
     f32x4 x = ZERO4;
     if (init != nullptr)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) x[v] = init[bh * N * N + o + v * N];
-    const float* at = p.local + bh * (p.NB - 1) * 2 * N * N;
-    float* to = p.enter + bh * (p.NB - 1) * N * N + o;
+        for (int v = 0; v < 4; ++v) x[v] = init[(p.at + head) * N * N + o + v * N];
+    const float* at = p.local + head * (p.NB - 1) * 2 * N * N;
+    float* to = p.enter + head * (p.NB - 1) * N * N + o;
     struct Block { float m[4][4]; f32x4 e; };
     auto fetch = [&](Block& d) __attribute__((always_inline)) {
 #pragma unroll
@@ -634,7 +640,7 @@ __global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
         for (int v = 0; v < 4; ++v) { to[v * N] = x[v]; bad = fmaf(x[v], 0.f, bad); }
         now = next;
     }
-    if (bad != 0.f) p.flags[bh] = 1;                     // (0, or no number)
+    if (bad != 0.f) p.flags[head] = 1;                     // (0, or no number)
 }
 
 // ---------------------------------------------------------------------------------------------------- backward
@@ -1196,17 +1202,16 @@ __global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c args) {
     extern __shared__ __align__(128) unsigned char smem_raw[];
     SmemCB<F32>& S = *reinterpret_cast<SmemCB<F32>*>(smem_raw);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = blockIdx.x, b = blockIdx.y;
-    const size_t bh = static_cast<size_t>(b) * p.H + h;
+    const auto [bh, b, h] = head_of(p, blockIdx.x);
     Part7 x;
-    if (!part_of(p, bh, x)) return;
+    if (!part_of(p, x)) return;
     const size_t tok0 = static_cast<size_t>(b) * p.T + x.first * CL;
     const int nch = x.chunks, all = p.T / CL;
     const lds_t sb = lds_of(smem_raw);
     // (thread numbers anew: role B has no register to hold one across its loop for the code of the others, which lies behind)
     const auto again = [&]() __attribute__((always_inline)) { return 64 * w + static_cast<int>(lane_again()); };
     if (w >= 8) { bwd_role_p(S, sb, p, again(), w, tok0, nch, p.H, h); return; }
-    const float* const dsT = x.first + nch < all ? p.enter + (bh * (p.NB - 1) + p.NB - 2 - x.n) * N * N : (p.dsT != nullptr ? p.dsT + bh * N * N : nullptr);
+    const float* const dsT = x.first + nch < all ? p.enter + (static_cast<size_t>(blockIdx.x) * (p.NB - 1) + p.NB - 2 - x.n) * N * N : (p.dsT != nullptr ? p.dsT + bh * N * N : nullptr);
     if (w < 4) bwd_role_a(S, sb, p, dsT, p.ds0 != nullptr && x.n == 0 ? p.ds0 + bh * N * N : nullptr, again(), w, nch, tok0, p.H, h);
     else bwd_role_b(S, sb, p, dsT, p.s + (bh * all + x.first) * N * N, tid, w, nch, tok0, p.H, h);
 }
@@ -1221,29 +1226,55 @@ uint16_t* el(void* p) { return static_cast<uint16_t*>(p); }
 // 720 / 645; 192 (two blocks) of T4096 721 / 1000.  Forward + backward of T4096: 8 sequences 1796 / 215, 32 1818 / 491, 128 1817 / 1573;
 // fp32 mode 1899 / 226, 2024 / 550, 2099 / 1785.  128 of T256, backward alone: 78 / 74.
 constexpr int BLOCK_CHUNKS = 4, SLOTS_FWD = 512, SLOTS_BWD = 256;
-int time_blocks(int B, int T, int H, bool bwd, int* per) {
-    const long long bh = static_cast<long long>(B) * H, want = (bwd ? SLOTS_BWD : SLOTS_FWD) / bh;
-    const int nch = T / CL;
+int time_blocks(int heads, int T, bool bwd, int* per) {
+    const int want = (bwd ? SLOTS_BWD : SLOTS_FWD) / heads, nch = T / CL;
     *per = nch;
-    if (want < (bwd ? 2 : 4) || nch < 4 * BLOCK_CHUNKS || (!bwd && nch * 256LL < bh * bh)) return 1;
-    const int least = static_cast<int>((nch + want - 1) / want);
+    if (want < (bwd ? 2 : 4) || nch < 4 * BLOCK_CHUNKS || (!bwd && nch * 256LL < static_cast<long long>(heads) * heads)) return 1;
+    const int least = (nch + want - 1) / want;
     *per = least > BLOCK_CHUNKS ? least : BLOCK_CHUNKS;
     return (nch + *per - 1) / *per;
 }
+// Heads done as whole sequences, then others in NB blocks of `per` chunks.  More heads than CUs leave a last round of few workgroups, as long
+// as the others: the heads beyond a multiple of the CUs are done in blocks where they are so few that this is shorter.  In the
+// forward, where two workgroups of a CU get little more done than one, that is less to gain.  T1024, us whole / split, bf16 and fp32 mode,
+// backward: 264 heads 497 / 316 and 513 / 355, 288 504 / 355 and 525 / 404, 320 532 / 419 and 530 / 459, 352 510 / 470 and 533 / 516, 384 527 / 490 and
+// 541 / 547, 528 753 / 598 and 798 / 678, 576 779 / 681 and 814 / 771; forward: 264 236 / 200 and 274 / 247, 288 249 / 245 and 289 / 292, 320 270 / 295 and
+// 296 / 334, 528 391 / 344 and 464 / 399, 576 401 / 404 and 496 / 481.
+struct Split7 { int whole, rest, NB, per; };
+constexpr int REST_FWD = 16, REST_BWD = 96;
+Split7 split_heads(int B, int T, int H, bool bwd) {
+    if (static_cast<long long>(B) * H > 0x7fffffffLL) return {0, 0, 1, T / CL};      // (no memory holds them)
+    const int all = B * H, rest = all % SLOTS_BWD;
+    Split7 x{all - rest, rest, 1, T / CL};
+    if (rest > 0 && (all < SLOTS_BWD || rest <= (bwd ? REST_BWD : REST_FWD))) x.NB = time_blocks(rest, T, bwd, &x.per);
+    return x.NB > 1 ? x : Split7{all, 0, 1, T / CL};
+}
 size_t blocks_bytes(size_t bh, int NB) { return NB > 1 ? bh * (NB - 1) * 3 * N * N * sizeof(float) + (bh * sizeof(int) + 15) / 16 * 16 : 0; }
-// the kernels that bring the states to the blocks' borders, where there are blocks
-template <bool F32, bool REV> int cut(hipStream_t st, int B, Args7c& p, void* ws) {
-    p.NB = 1;
-    if (ws == nullptr) return RWKV_OK;
-    p.NB = time_blocks(B, p.T, p.H, REV, &p.per);
-    if (p.NB == 1) return RWKV_OK;
+// the kernels that bring the states to the borders of the blocks of the heads from p.at on
+template <bool F32, bool REV> int cut(hipStream_t st, int heads, Args7c& p, void* ws) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(rwkv7c_local<F32, REV>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                                        static_cast<int>(L_TOTAL<F32>));
     if (attr != hipSuccess) { g_last_hip_error = static_cast<int>(attr); return RWKV_ERR_LAUNCH; }
-    const size_t n = static_cast<size_t>(B) * p.H * (p.NB - 1) * N * N;
+    const size_t n = static_cast<size_t>(heads) * (p.NB - 1) * N * N;
     p.local = static_cast<float*>(ws); p.enter = p.local + 2 * n; p.flags = reinterpret_cast<int*>(p.enter + n);
-    rwkv7c_local<F32, REV><<<dim3(p.H, B, 2 * (p.NB - 1)), dim3(NTF), L_TOTAL<F32>, st>>>(p);
-    rwkv7c_scan<REV><<<dim3(4 * p.H, B), dim3(256), 0, st>>>(p);
+    rwkv7c_local<F32, REV><<<dim3(heads, 1, 2 * (p.NB - 1)), dim3(NTF), L_TOTAL<F32>, st>>>(p);
+    rwkv7c_scan<REV><<<dim3(4 * heads), dim3(256), 0, st>>>(p);
+    return launch_status();
+}
+// whole sequences, then those in blocks: a launch each, of the heads from p.at on
+template <bool F32, bool REV, typename Whole, typename Blocks> int in_parts(hipStream_t st, int B, Args7c& p, void* ws, Whole whole, Blocks blocks) {
+    Split7 x = split_heads(B, p.T, p.H, REV);
+    if (x.whole + x.rest == 0) return RWKV_ERR_SHAPE;
+    if (ws == nullptr) x = {B * p.H, 0, 1, p.T / CL};
+    p.NB = 1; p.at = 0;
+    if (x.whole > 0) {
+        whole(p, dim3(x.whole));
+        if (int e = launch_status()) return e;
+    }
+    if (x.rest == 0) return RWKV_OK;
+    p.NB = x.NB; p.per = x.per; p.at = x.whole;
+    if (int e = cut<F32, REV>(st, x.rest, p, ws)) return e;
+    blocks(p, dim3(x.rest, 1, x.NB));
     return launch_status();
 }
 
@@ -1253,24 +1284,24 @@ hipError_t raise_lds(void (*kernel)(Args7c), size_t bytes) {
 template <bool F32, bool KEEP> int start_fwd(hipStream_t st, int B, Args7c& p, void* ws) {
     static const hipError_t attr[2] = {raise_lds(rwkv7c_fwd<F32, KEEP, false>, F_TOTAL<F32>), raise_lds(rwkv7c_fwd<F32, KEEP, true>, F_TOTAL<F32>)};
     for (const hipError_t e : attr) if (e != hipSuccess) { g_last_hip_error = static_cast<int>(e); return RWKV_ERR_LAUNCH; }
-    if (int e = cut<F32, false>(st, B, p, ws)) return e;
-    hipLaunchKernelGGL((p.NB > 1 ? rwkv7c_fwd<F32, KEEP, true> : rwkv7c_fwd<F32, KEEP, false>), dim3(p.H, B, p.NB), dim3(NTF), F_TOTAL<F32>, st, p);
-    return launch_status();
+    return in_parts<F32, false>(st, B, p, ws,
+        [&](const Args7c& q, dim3 grid) { hipLaunchKernelGGL((rwkv7c_fwd<F32, KEEP, false>), grid, dim3(NTF), F_TOTAL<F32>, st, q); },
+        [&](const Args7c& q, dim3 grid) { hipLaunchKernelGGL((rwkv7c_fwd<F32, KEEP, true>), grid, dim3(NTF), F_TOTAL<F32>, st, q); });
 }
 template <bool F32> int start_bwd(hipStream_t st, int B, Args7c& p, void* ws) {
     static_assert(LB<F32>::BYTES <= 160 * 1024, "the backward's LDS must fit one CU");
     static const hipError_t attr[2] = {raise_lds(rwkv7c_bwd<F32, false>, LB<F32>::BYTES), raise_lds(rwkv7c_bwd<F32, true>, LB<F32>::BYTES)};
     for (const hipError_t e : attr) if (e != hipSuccess) { g_last_hip_error = static_cast<int>(e); return RWKV_ERR_LAUNCH; }
-    if (int e = cut<F32, true>(st, B, p, ws)) return e;
-    hipLaunchKernelGGL((p.NB > 1 ? rwkv7c_bwd<F32, true> : rwkv7c_bwd<F32, false>), dim3(p.H, B, p.NB), dim3(NTB), LB<F32>::BYTES, st, p);
-    return launch_status();
+    return in_parts<F32, true>(st, B, p, ws,
+        [&](const Args7c& q, dim3 grid) { hipLaunchKernelGGL((rwkv7c_bwd<F32, false>), grid, dim3(NTB), LB<F32>::BYTES, st, q); },
+        [&](const Args7c& q, dim3 grid) { hipLaunchKernelGGL((rwkv7c_bwd<F32, true>), grid, dim3(NTB), LB<F32>::BYTES, st, q); });
 }
 
 }  // namespace
 
 size_t rwkv7c_workspace_bytes(int B, int T, int H, bool bwd) {
-    int per;
-    return blocks_bytes(static_cast<size_t>(B) * H, time_blocks(B, T, H, bwd, &per));
+    const Split7 x = split_heads(B, T, H, bwd);
+    return blocks_bytes(x.rest, x.NB);
 }
 int launch7c_fwd(hipStream_t st, bool f32, int B, int T, int H, const float* s0, const void* r, const void* w, const void* k,
                  const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa, void* ws) {

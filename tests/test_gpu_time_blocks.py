@@ -218,6 +218,40 @@ def test_rwkv7(lib, variant, dtype, B, T, H):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,forward,backward", [(1, 257, 1, 1), (4, 68, 16, 16), (3, 91, 0, 17), (2, 176, 0, 96), (1, 353, 0, 0), (9, 57, 1, 1)])
+def test_rwkv7_heads_beyond_a_multiple_of_the_cus(lib, B, H, forward, backward, dtype):
+    """forward, backward: how many of the last heads are done in blocks there.  The others have the bits of a call without a workspace, these
+    differ by the rounding of a state that is summed in another order (one more rounding of 2^-24 a block's product, and a bf16 result may
+    fall on the other side)."""
+    T = 256
+    n = [lib.rwkv7_workspace_bytes(B, T, H, i) for i in (0, 1)]
+    assert [m > 0 for m in n] == [forward > 0, backward > 0]
+    s0, x, dy, dsT = _rwkv7(B, T, H, dtype, B + H)
+    s0, dy, dsT, x = s0.to(DEV), dy.to(DEV), dsT.to(DEV), [t.to(DEV) for t in x]
+    f32 = int(dtype == torch.float32)
+    new = lambda *s, dt=torch.float32: garbage(s, dt)
+    rows = lambda t: t.view(B, T, H, 64).transpose(1, 2).reshape(B * H, -1)
+    s, sa = new(B, H, T // 16, 64, 64), new(B, T, H, 64)
+    res = []
+    for cut in (True, False):                               # (the backward of both from the second one's states)
+        ws = [garbage((m,), torch.uint8) if cut and m else None for m in n]
+        y, sT = new(B, T, H * 64, dt=dtype), new(B, H, 64, 64)
+        call("rwkv7_forward_ws", y.device, B, T, H, f32, s0, *x, y, sT, s, sa, ws[0], n[0] if cut else 0)
+        res.append([rows(y), sT.view(B * H, -1), s.view(B * H, -1).clone(), rows(sa).clone()])
+    for i, cut in enumerate((True, False)):
+        ws = garbage((n[1],), torch.uint8) if cut and n[1] else None
+        ds0, d = new(B, H, 64, 64), [new(B, T, H * 64, dt=dtype) for _ in range(6)]
+        call("rwkv7_backward_ws", dy.device, B, T, H, f32, *x, dy, dsT, s, sa, ds0, *d, ws, n[1] if cut else 0)
+        res[i] += [rows(t) for t in d] + [ds0.view(B * H, -1)]
+    for z, (got, whole) in enumerate(zip(*res)):
+        m = B * H - (forward if z < 4 else backward)
+        assert torch.equal(got[:m], whole[:m]), z
+        for a, b in zip(got[m:].double(), whole[m:].double()):
+            q = float((a - b).norm() / b.norm())
+            assert q <= (2.0 ** -8 if got.dtype == torch.bfloat16 else 6e-7 * (T / 16) ** 0.5 if z == 5 else 4e-7), (z, q)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("which", ["a", "k"])
 def test_rwkv7_heads_that_blocks_cannot_carry_are_done_as_a_whole(lib, which, dtype):
     """A NaN among the inputs, and a transition that overflows over a block where the state itself is zero: the bits of a call without a
