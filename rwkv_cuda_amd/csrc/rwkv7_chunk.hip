@@ -1239,14 +1239,15 @@ int time_blocks(int heads, int T, bool bwd, int* per) {
 // forward, where two workgroups of a CU get little more done than one, that is less to gain.  T1024, us whole / split, bf16 and fp32 mode,
 // backward: 264 heads 497 / 316 and 513 / 355, 288 504 / 355 and 525 / 404, 320 532 / 419 and 530 / 459, 352 510 / 470 and 533 / 516, 384 527 / 490 and
 // 541 / 547, 528 753 / 598 and 798 / 678, 576 779 / 681 and 814 / 771; forward: 264 236 / 200 and 274 / 247, 288 249 / 245 and 289 / 292, 320 270 / 295 and
-// 296 / 334, 528 391 / 344 and 464 / 399, 576 401 / 404 and 496 / 481.
+// 296 / 334, 528 391 / 344 and 464 / 399, 576 401 / 404 and 496 / 481.  T256, backward: 264 134 / 105 and 138 / 117, 320 132 / 119 and 144 / 136, 352 136 / 136
+// and 146 / 151; forward: 264 70 / 73 and 66 / 76, 528 97 / 100 and 104 / 121; T512, forward: 264 128 / 113 and 126 / 129.
 struct Split7 { int whole, rest, NB, per; };
-constexpr int REST_FWD = 16, REST_BWD = 96;
+constexpr int REST_FWD = 16, REST_FWD_CHUNKS = 48, REST_BWD = 96;
 Split7 split_heads(int B, int T, int H, bool bwd) {
     if (static_cast<long long>(B) * H > 0x7fffffffLL) return {0, 0, 1, T / CL};      // (no memory holds them)
     const int all = B * H, rest = all % SLOTS_BWD;
     Split7 x{all - rest, rest, 1, T / CL};
-    if (rest > 0 && (all < SLOTS_BWD || rest <= (bwd ? REST_BWD : REST_FWD))) x.NB = time_blocks(rest, T, bwd, &x.per);
+    if (rest > 0 && (all < SLOTS_BWD || (bwd ? rest <= REST_BWD && T / CL * 4 >= rest : rest <= REST_FWD && T / CL >= REST_FWD_CHUNKS))) x.NB = time_blocks(rest, T, bwd, &x.per);
     return x.NB > 1 ? x : Split7{all, 0, 1, T / CL};
 }
 size_t blocks_bytes(size_t bh, int NB) { return NB > 1 ? bh * (NB - 1) * 3 * N * N * sizeof(float) + (bh * sizeof(int) + 15) / 16 * 16 : 0; }

@@ -218,12 +218,12 @@ def test_rwkv7(lib, variant, dtype, B, T, H):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("B,H,forward,backward", [(1, 257, 1, 1), (4, 68, 16, 16), (3, 91, 0, 17), (2, 176, 0, 96), (1, 353, 0, 0), (9, 57, 1, 1)])
-def test_rwkv7_heads_beyond_a_multiple_of_the_cus(lib, B, H, forward, backward, dtype):
+@pytest.mark.parametrize("B,H,T,forward,backward", [(1, 257, 768, 1, 1), (4, 68, 768, 16, 16), (3, 91, 256, 0, 17), (2, 176, 384, 0, 96), (1, 353, 384, 0, 0),
+                                                   (9, 57, 256, 0, 1), (2, 176, 368, 0, 0), (1, 258, 752, 0, 2)])
+def test_rwkv7_heads_beyond_a_multiple_of_the_cus(lib, B, H, T, forward, backward, dtype):
     """forward, backward: how many of the last heads are done in blocks there.  The others have the bits of a call without a workspace, these
     differ by the rounding of a state that is summed in another order (one more rounding of 2^-24 a block's product, and a bf16 result may
     fall on the other side)."""
-    T = 256
     n = [lib.rwkv7_workspace_bytes(B, T, H, i) for i in (0, 1)]
     assert [m > 0 for m in n] == [forward > 0, backward > 0]
     s0, x, dy, dsT = _rwkv7(B, T, H, dtype, B + H)
