@@ -49,25 +49,26 @@ struct ArgsW {
     float* decay;                                // [e^l | l], 2 C floats (forward)
     float* saved;                                // [B*H][ceil(chunks / 2)][j][i]: the state entering every even chunk
     // sequences cut into blocks of time (NB > 1): blocks of `per` pairs of chunks, a workgroup each; what each block leaves of a state that
-    // entered it empty, [B*H][NB - 1][HN][HN] (the last block's is not needed, in the backward the first's); gw, gu in fp32 [NB][B][C]
-    int B, NB, per;
+    // entered it empty, [heads][NB - 1][HN][HN] (the last block's is not needed, in the backward the first's); gw, gu in fp32 [NB][heads][HN].
+    // heads: of this launch, from head `at` on, batch row by batch row
+    int heads, at, NB, per;
     float *local, *gw32, *gu32;
 };
 
 // The workgroup's head and its part of the sequence: chunks first .. first + chunks - 1, tokens that are left from there on.
 struct Part {
-    int h, b, n, first, chunks, left;
+    int h, b, rel, n, first, chunks, left;      // rel: among the launch's heads
     size_t bh, base;
 };
 // pairs: an odd number of chunks is rounded up
 DEVINL Part part_of(const ArgsW& p, int hn, bool pairs) {
     Part x;
-    const int BH = p.B * p.H;
     int nch = (p.T + L - 1) / L;
     if (pairs) nch += nch & 1;
     // (divisions are done in vector registers)
-    x.n = __builtin_amdgcn_readfirstlane(p.NB > 1 ? static_cast<int>(blockIdx.x) / BH : 0);
-    x.bh = blockIdx.x - x.n * BH;
+    x.n = __builtin_amdgcn_readfirstlane(p.NB > 1 ? static_cast<int>(blockIdx.x) / p.heads : 0);
+    x.rel = blockIdx.x - x.n * p.heads;
+    x.bh = p.at + x.rel;
     x.b = __builtin_amdgcn_readfirstlane(static_cast<int>(x.bh) / p.H); x.h = static_cast<int>(x.bh) - x.b * p.H;
     x.first = x.n * 2 * p.per;
     x.chunks = p.NB > 1 ? min(2 * p.per, nch - x.first) : nch;
@@ -267,7 +268,7 @@ __global__ __launch_bounds__(256) void wkv5b_local(const ArgsW p) {
     __shared__ __align__(16) unsigned char rows[4 * A::PLANE];           // two sets of key and value rows
     const lds_t sb = lds_of(rows);
     const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4, C = p.C;
-    const int BH = p.B * p.H, m = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / BH), bh = blockIdx.x - m * BH;
+    const int m = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / p.heads), rel = blockIdx.x - m * p.heads, bh = p.at + rel;
     const int b = __builtin_amdgcn_readfirstlane(bh / p.H), h = bh - b * p.H, n = REV ? m + 1 : m;
     if (steps_head<false, HN>(p.w, nullptr, h * HN)) return;
     const int first = n * 2 * p.per, chunks = min(2 * p.per, (p.T + L - 1) / L - first);
@@ -333,7 +334,7 @@ __global__ __launch_bounds__(256) void wkv5b_local(const ArgsW p) {
         fetch(i + 2);
         __syncthreads();
     }
-    float* const out = p.local + (static_cast<size_t>(bh) * (p.NB - 1) + m) * HN * HN;
+    float* const out = p.local + (static_cast<size_t>(rel) * (p.NB - 1) + m) * HN * HN;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -365,7 +366,7 @@ template <int HN, bool RAW> DEVINL void fwd_states(const ArgsW& p, lds_t sb, int
 #pragma unroll
         for (int jt = 0; jt < NJ; ++jt) St[ct][jt] = ZERO4;
     if (part.n > 0) {                                    // the state that enters the block, from what the blocks before leave
-        const float* x = p.local + part.bh * (p.NB - 1) * HN * HN + (16 * CT * q + l16) * HN + 4 * g;
+        const float* x = p.local + static_cast<size_t>(part.rel) * (p.NB - 1) * HN * HN + (16 * CT * q + l16) * HN + 4 * g;
 #pragma unroll 2
         for (int m = 0; m < part.n; ++m, x += HN * HN)
 #pragma unroll
@@ -638,7 +639,7 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
 #pragma unroll
     for (int ib = 0; ib < NI; ++ib) dS[ib] = ZERO4;
     if (part.n + 1 < p.NB) {                             // the gradient of the state that leaves the block, from what the blocks after take up
-        const float* x = p.local + (part.bh * (p.NB - 1) + p.NB - 2) * HN * HN + (16 * q + l16) * HN + 4 * g;
+        const float* x = p.local + (static_cast<size_t>(part.rel) * (p.NB - 1) + p.NB - 2) * HN * HN + (16 * q + l16) * HN + 4 * g;
         const float d = lds_f(sb + A::BLK + 4 * (16 * q + l16));
 #pragma unroll 1
         for (int m = p.NB - 1; m > part.n; --m, x -= HN * HN)
@@ -835,11 +836,11 @@ template <int HN> DEVINL void role_d(const ArgsW& p, lds_t sb, int q, int lane, 
         chunk(std::true_type{}, c);
         chunk(std::false_type{}, c - 1);
     }
-    const size_t o = (static_cast<size_t>(part.n) * p.B + part.b) * C + part.h * HN + 16 * q + l16;
+    const size_t o = (static_cast<size_t>(part.n) * p.heads + part.rel) * HN + 16 * q + l16;
     const float sw = allreduce_rows(fmaf(32.f * o32, gP, gw)), su = allreduce_rows(gu);
     if (g == 0) {
         if (p.NB > 1) { p.gw32[o] = l * sw; p.gu32[o] = su; }
-        else { p.gw[o] = f2bf(l * sw); p.gu[o] = f2bf(su); }
+        else { p.gw[o] = f2bf(l * sw); p.gu[o] = f2bf(su); }      // (a launch of whole sequences begins with head 0)
     }
 }
 
@@ -998,12 +999,12 @@ __global__ __launch_bounds__(256) void block_rows(int NB, size_t n, const float*
     (blockIdx.y == 0 ? gw : gu)[i] = f2bf(s);
 }
 
-template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, int threads, uint32_t lds) {
+template <class F> int launch(F* kernel, hipStream_t st, const ArgsW& p, int threads, uint32_t lds) {
     if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); e != hipSuccess) {
         g_last_hip_error = static_cast<int>(e);
         return RWKV_ERR_LAUNCH;
     }
-    hipLaunchKernelGGL(kernel, dim3(B * p.H * p.NB), dim3(threads), lds, st, p);
+    hipLaunchKernelGGL(kernel, dim3(p.heads * p.NB), dim3(threads), lds, st, p);
     return launch_status();
 }
 
@@ -1012,23 +1013,46 @@ template <class F> int launch(F* kernel, hipStream_t st, int B, const ArgsW& p, 
 // of T4096 255 / 99; 64 of T400 34 / 34, of T4096 261 / 130; 128 of T400 36 / 43, of T800 60 / 61, of T2000 135 / 122; forward + backward 8 of
 // T400 129 / 77, of T4096 1059 / 191; 32 of T4096 1095 / 251; 64 of T4096 1112 / 428; 128 of T400 136 / 116, of T4096 1153 / 821.
 constexpr int BLOCK_PAIRS = 2, SLOTS = 256;
-int time_blocks(int B, int T, int H, bool bwd, int* per) {
-    const long long bh = static_cast<long long>(B) * H, want = SLOTS / bh;
+int time_blocks(int heads, int T, bool bwd, int* per) {
+    const int want = SLOTS / heads;
     const int pairs = static_cast<int>((static_cast<long long>(T) + 2 * L - 1) / (2 * L));
     *per = pairs;
-    if (want < 2 || pairs < 3 * BLOCK_PAIRS || (!bwd && pairs * 8 < bh)) return 1;
+    if (want < 2 || pairs < 3 * BLOCK_PAIRS || (!bwd && pairs * 8 < heads)) return 1;
     const int least = static_cast<int>((pairs + want - 1) / want);
     *per = least > BLOCK_PAIRS ? least : BLOCK_PAIRS;
     return (pairs + *per - 1) / *per;
 }
 size_t round16(size_t x) { return (x + 15) & ~static_cast<size_t>(15); }
-void set_blocks(ArgsW& p, int B, bool bwd, void* ws) {
-    p.B = B; p.NB = 1; p.per = 0;
-    if (ws == nullptr) return;
-    p.NB = time_blocks(B, p.T, p.H, bwd, &p.per);
+// Heads done as whole sequences, then others in NB blocks of `per` pairs.  The heads beyond a multiple of the CUs would be a last round of few
+// workgroups, as long as the others.  us whole / split, forward, backward: 264 heads of T400 82 / 76, 202 / 157, of T2000 347 / 273, 814 / 539; 288 of T400
+// 76 / 75, 200 / 163, of T2000 360 / 295, 833 / 588; 320 of T800 147 / 152, 357 / 283; 384 of T400 78 / ., 202 / 190, of T2000 390 / 387, 856 / 770; 528 of T800 230 /
+// 218, 520 / 438; 576 of T800 243 / 272, 534 / 480.
+struct SplitW { int whole, rest, NB, per; };
+constexpr int REST_FWD = 32, REST_BWD = 128;
+SplitW split_heads(int B, int T, int H, bool bwd) {
+    if (static_cast<long long>(B) * H > 0x7fffffffLL) return {0, 0, 1, 0};      // (no memory holds them)
+    const int all = B * H, rest = all % SLOTS;
+    SplitW x{all - rest, rest, 1, 0};
+    if (rest > 0 && (all < SLOTS || rest <= (bwd ? REST_BWD : REST_FWD))) x.NB = time_blocks(rest, T, bwd, &x.per);
+    return x.NB > 1 ? x : SplitW{all, 0, 1, 0};
+}
+// whole sequences, then those in blocks (heads of 128): a launch each
+template <bool REV, class F, class W> int in_parts(hipStream_t st, int B, ArgsW& p, void* ws, F* kernel, int threads, uint32_t lds, W after) {
+    SplitW x = split_heads(B, p.T, p.H, REV);
+    if (x.whole + x.rest == 0) return RWKV_ERR_SHAPE;
+    if (ws == nullptr) x = {B * p.H, 0, 1, 0};
+    p.heads = x.whole; p.at = 0; p.NB = 1; p.per = 0;
+    if (x.whole > 0)
+        if (int e = launch(kernel, st, p, threads, lds)) return e;
+    if (x.rest == 0) return RWKV_OK;
+    p.heads = x.rest; p.at = x.whole; p.NB = x.NB; p.per = x.per;
     p.local = static_cast<float*>(ws);
-    p.gw32 = p.local + static_cast<size_t>(B) * p.H * (p.NB - 1) * 128 * 128;
-    p.gu32 = p.gw32 + static_cast<size_t>(p.NB) * B * p.C;
+    p.gw32 = p.local + static_cast<size_t>(x.rest) * (x.NB - 1) * 128 * 128;
+    p.gu32 = p.gw32 + static_cast<size_t>(x.NB) * x.rest * 128;
+    hipLaunchKernelGGL((wkv5b_local<128, REV>), dim3(x.rest * (x.NB - 1)), dim3(256), 0, st, p);
+    if (int e = launch(kernel, st, p, threads, lds)) return e;
+    after();
+    return launch_status();
 }
 
 }  // namespace
@@ -1038,32 +1062,30 @@ size_t wkv5b_saved_bytes(int B, int T, int C, int H) {
     return static_cast<size_t>(B) * H * ((nch + 1) / 2) * n * n * sizeof(float);
 }
 size_t wkv5b_blocks_bytes(int B, int T, int C, int H, bool bwd) {
-    int per;
-    const int NB = C == H * 128 ? time_blocks(B, T, H, bwd, &per) : 1;
-    if (NB == 1) return 0;
-    return static_cast<size_t>(B) * H * (NB - 1) * 128 * 128 * sizeof(float) + (bwd ? round16(2 * static_cast<size_t>(NB) * B * C * sizeof(float)) : 0);
+    if (C != H * 128) return 0;
+    const SplitW x = split_heads(B, T, H, bwd);
+    if (x.NB == 1) return 0;
+    return static_cast<size_t>(x.rest) * (x.NB - 1) * 128 * 128 * sizeof(float) + (bwd ? round16(2 * static_cast<size_t>(x.NB) * x.rest * 128 * sizeof(float)) : 0);
 }
 int launch_wkv5b_fwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
                      const uint16_t* u, uint16_t* y, float* decay, float* saved, void* ws) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.y = y; p.decay = decay; p.saved = saved;
-    set_blocks(p, B, false, ws);
-    if (p.NB > 1) hipLaunchKernelGGL((wkv5b_local<128, false>), dim3(B * H * (p.NB - 1)), dim3(256), 0, st, p);
-    return C == H * 64 ? launch(wkv5b_fwd<64>, st, B, p, NTH, G<64>::FTOTAL) : launch(wkv5b_fwd<128>, st, B, p, NTH, G<128>::FTOTAL);
+    const auto none = []() {};
+    if (C == H * 64) return in_parts<false>(st, B, p, nullptr, wkv5b_fwd<64>, NTH, G<64>::FTOTAL, none);
+    return in_parts<false>(st, B, p, ws, wkv5b_fwd<128>, NTH, G<128>::FTOTAL, none);
 }
 int launch_wkv5b_bwd(hipStream_t st, int B, int T, int C, int H, const uint16_t* r, const uint16_t* k, const uint16_t* v, const uint16_t* w,
                      const uint16_t* u, const uint16_t* gy, uint16_t* gr, uint16_t* gk, uint16_t* gv, uint16_t* gw, uint16_t* gu, const float* saved, void* ws) {
     ArgsW p{};
     p.T = T; p.C = C; p.H = H; p.r = r; p.k = k; p.v = v; p.w = w; p.u = u; p.gy = gy; p.gr = gr; p.gk = gk; p.gv = gv; p.gw = gw; p.gu = gu;
     p.saved = const_cast<float*>(saved);
-    set_blocks(p, B, true, ws);
-    if (p.NB > 1) hipLaunchKernelGGL((wkv5b_local<128, true>), dim3(B * H * (p.NB - 1)), dim3(256), 0, st, p);
-    if (int e = C == H * 64 ? launch(wkv5b_bwd<64>, st, B, p, 512, G<64>::BTOTAL) : launch(wkv5b_bwd<128>, st, B, p, 1024, G<128>::BTOTAL)) return e;
-    if (p.NB > 1) {
-        const size_t n = static_cast<size_t>(B) * C;
-        hipLaunchKernelGGL(block_rows, dim3(static_cast<unsigned>((n + 255) / 256), 2), dim3(256), 0, st, p.NB, n, p.gw32, p.gu32, gw, gu);
-    }
-    return launch_status();
+    const auto rows = [&]() {
+        const size_t n = static_cast<size_t>(p.heads) * 128, o = static_cast<size_t>(p.at) * 128;
+        hipLaunchKernelGGL(block_rows, dim3(static_cast<unsigned>((n + 255) / 256), 2), dim3(256), 0, st, p.NB, n, p.gw32, p.gu32, gw + o, gu + o);
+    };
+    if (C == H * 64) return in_parts<true>(st, B, p, nullptr, wkv5b_bwd<64>, 512, G<64>::BTOTAL, rows);
+    return in_parts<true>(st, B, p, ws, wkv5b_bwd<128>, 1024, G<128>::BTOTAL, rows);
 }
 
 }  // namespace rwkv

@@ -308,6 +308,32 @@ def test_wkv5_bf16_heads_of_128(lib, decays, B, H, T):
         assert_no_worse(name, a, e.reshape(a.shape), g.reshape(a.shape))
 
 
+@pytest.mark.parametrize("B,H,T,forward,backward", [(1, 257, 321, 1, 1), (8, 36, 350, 32, 32), (3, 119, 384, 0, 101), (1, 385, 321, 0, 0)])
+def test_wkv5_heads_of_128_beyond_a_multiple_of_the_cus(lib, B, H, T, forward, backward):
+    """forward, backward: how many of the last heads are done in blocks there.  The others have the bits of a call for whole sequences; these
+    differ by the rounding of bf16, 2^-8 at most an element (gw, gu: of each batch row, and again of their sum)."""
+    C, WHOLE = H * 128, 0x200
+    n = [lib.rwkv_wkv5s_blocks_workspace_bytes(B, T, C, H, i) for i in (0, 1)]
+    assert [m > 0 for m in n] == [forward > 0, backward > 0]
+    r, k, v, w, u, gy = (x.to(DEV) for x in synth.wkv5_inputs(B, T, C, H, seed=H))
+    rows = lambda t: t.view(B, T, H, 128).transpose(1, 2).reshape(B * H, -1)
+    ns, nb = lib.rwkv_wkv5s_saved_bytes(B, T, C, H), max(n[1], lib.rwkv_wkv5s_backward_workspace_bytes(B, T, C, H))
+    saved, decay, res = garbage((ns,), torch.uint8), garbage((2 * C,), torch.float32), []
+    for flags in (0, WHOLE):                                # (the backward of both from the second one's states)
+        y, ws = garbage((B, T, C), torch.bfloat16), garbage((n[0],), torch.uint8) if n[0] and not flags else None
+        call("rwkv_wkv5s_forward_ws", y.device, B, T, C, H, r, k, v, w, u, y, decay, saved, ns, ws, n[0] if ws is not None else 0, flags)
+        res.append([rows(y)])
+    for i, flags in enumerate((0, WHOLE)):
+        g, gw, gu = [garbage((B, T, C), torch.bfloat16) for _ in range(3)], garbage((H, 128), torch.bfloat16), garbage((H, 128), torch.bfloat16)
+        call("rwkv_wkv5s_backward", y.device, B, T, C, H, r, k, v, w, decay, u, gy, *g, gw, gu, saved, ns, garbage((nb,), torch.uint8), nb, flags)
+        res[i] += [rows(t) for t in g] + [gw, gu]
+    for z, (got, whole) in enumerate(zip(*res)):
+        m = (B * H if z < 4 else H) - (forward if z == 0 else backward)
+        assert torch.equal(got[:max(m, 0)], whole[:max(m, 0)]), z
+        for a, b in zip(got[max(m, 0):].double(), whole[max(m, 0):].double()):
+            assert float((a - b).norm() / b.norm()) <= 2.0 ** -8 * (1 if z < 4 else 2), z
+
+
 @pytest.mark.parametrize("H,T", [(3, 257), (3, 1100), (3, 2300), (64, 1025), (100, 641), (100, 1300)])       # 2, 9, 18 (a scan of its own), 4, 2, 2 blocks of 128 .. 704 tokens
 def test_wkv6_state_blocks_of_every_length(lib, H, T):
     """The first pass takes a block's tokens up to 256 at a time, 32 or more a part; three heads of the layer against the oracle."""
