@@ -410,8 +410,8 @@ __global__ __launch_bounds__(NTS) void wkv4_bwd_seg(int T, int C, int S, const f
 // backward with the 4 us of wkv4_batch_sum: B64 T64 C2048 57 -> 20 / 203 -> 55; B128 T128 C1024 68 -> 33 / 264 -> 98; B64 T256 C1024
 // 47 -> 36 / 182 -> 103; B64 T512 C768 75 -> 69 / 222 -> 168; B32 T400 C1000 36 -> 31 / 121 -> 84.  Half of that in the backward
 // is the workgroup's size: one of 1024 lanes has a CU for itself there (the same segments with 8 channels: B64 T512 C768 222 -> 174).
-// Not kept: 513 to 1024 steps in 128 segments of 8 (B32 T768 C768 backward 155 -> 198), 16 steps a segment up to 256 (103 -> 97, but
-// the smallest calls 6.2 -> 7.0).
+// Few pieces of channels take half as many channels and twice the segments (few_pieces).  Not kept: 513 to 1024 steps in 128 segments of 8
+// (B32 T768 C768 backward 155 -> 198), 16 steps a segment up to 256 (103 -> 97, but the smallest calls 6.2 -> 7.0).
 // Workgroups are handed to the chip's 8 XCDs in turn, each with an L2 of its own, and a workgroup's 8 or 16 channels are a
 // quarter or half of a 128-byte line: numbered as launched, the workgroups that share a line would sit on different XCDs and
 // each L2 would fetch the whole line.  XCD d takes n / 8 adjacent pieces instead (the first n % 8 of them one more), so
@@ -667,7 +667,7 @@ __global__ __launch_bounds__(CHR * SEG, 4) void wkv4_bwd_reg(int T, int C, int S
 // CHR, SM, SEG as above.  Forward: 16 channels, 64 segments of 8 steps.  Backward: 16 channels, 32 segments of 16, half the rounds of the
 // scans and two workgroups a CU: us, 64 segments -> so, B28 T1100 C768 306 -> 221, B17 T2000 C768 325 -> 242, B6 T4000 C768 323 -> 240, B2 T4000
 // C2500 335 -> 221 (the forward that way: B12 T4000 C768 156 -> 169, B17 T2000 C768 100 -> 97).
-// Where pieces of 16 channels leave half of the CUs without work, both take 8 channels and 64 segments: B2 T4000 C768 52 -> 44 /
+// Where there are few pieces both take 8 channels and 64 segments: B2 T4000 C768 52 -> 44 /
 // 145 -> 116 (backward in 32 segments: 137), B1 T4096 C2048 51 -> 43 / 142 -> 107 (138); with 144 pieces it is 53 -> 56 / 147 -> 143 (140).
 constexpr int BLK_T = 512;
 constexpr int BLK_MAX = 64;            // blocks whose entering states fit in LDS: T <= 32768
@@ -961,8 +961,10 @@ template <bool RAW, int CHR, int SM, int SEG, typename... Ptrs>
 void launch4_bwd_blk(hipStream_t st, int B, int T, int C, Ptrs... p) {
     hipLaunchKernelGGL((wkv4_bwd_blk<RAW, CHR, SM, SEG>), pieces4<CHR>(B, C), dim3(CHR * SEG), 0, st, T, C, p...);
 }
-// pieces of 16 channels that leave half of the 256 CUs without work
-bool few_pieces(int B, int C) { return static_cast<long long>(B) * ((C + 15) / 16) <= 128; }
+// pieces of CHR channels that leave half of the 256 CUs without work: half the channels and twice the segments then.  Kernel us of the
+// backward, wide / narrow: 48 pieces of T512 13.3 / 11.2, 192 16.2 / 17.6; 48 of T256 9.2 / 8.7, 192 10.2 / 11.9; 16 of T128 9.7 / 7.4, 96 9.6 / 8.2, 288 13.6 /
+// 14.1; 32 of T64 8.2 / 7.1, 256 10.6 / 11.4; forward 48 of T512 6.8 / 5.6, 192 8.5 / 8.8.
+template <int CHR> bool few_pieces(int B, int C) { return static_cast<long long>(B) * ((C + CHR - 1) / CHR) <= 128; }
 
 template <bool RAW>
 void launch4_fwd(hipStream_t st, int B, int T, int C, const float* w, const float* u, const float* k, const float* v, float* y) {
@@ -970,17 +972,21 @@ void launch4_fwd(hipStream_t st, int B, int T, int C, const float* w, const floa
         const int BC = B * C;
         hipLaunchKernelGGL((wkv4_fwd<RAW>), dim3((BC + NT - 1) / NT), dim3(NT), 0, st, BC, T, C, w, u, k, v, y);
     } else if (T <= 64) {
-        launch4_fwd_reg<RAW, 64, 8, 8>(st, B, T, C, w, u, k, v, y);
+        if (few_pieces<64>(B, C)) launch4_fwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, y);
+        else launch4_fwd_reg<RAW, 64, 8, 8>(st, B, T, C, w, u, k, v, y);
     } else if (T <= 128) {
-        launch4_fwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, y);
+        if (few_pieces<32>(B, C)) launch4_fwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, y);
+        else launch4_fwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, y);
     } else if (T <= 256) {
-        launch4_fwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, y);
+        if (few_pieces<16>(B, C)) launch4_fwd_reg<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, y);
+        else launch4_fwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, y);
     } else if (T <= 512) {
-        launch4_fwd_reg<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, y);
+        if (few_pieces<16>(B, C)) launch4_fwd_reg<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, y);
+        else launch4_fwd_reg<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, y);
     } else if (T <= 1024) {
         launch4_fwd_reg<RAW, 8, 16, 64>(st, B, T, C, w, u, k, v, y);
     } else if (T <= BLK_T * BLK_MAX) {
-        if (few_pieces(B, C)) launch4_fwd_blk<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, y);
+        if (few_pieces<16>(B, C)) launch4_fwd_blk<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, y);
         else launch4_fwd_blk<RAW, 16, 8, 64>(st, B, T, C, w, u, k, v, y);
     } else {
         const int S = (T + NSEG - 1) / NSEG;
@@ -995,17 +1001,21 @@ void launch4_bwd(hipStream_t st, int B, int T, int C, const float* w, const floa
         const int BC = B * C;
         hipLaunchKernelGGL((wkv4_bwd<RAW>), dim3((BC + NT - 1) / NT), dim3(NT), 0, st, BC, T, C, w, u, k, v, gy, gw, gu, gk, gv, ze);
     } else if (T <= 64) {
-        launch4_bwd_reg<RAW, 64, 8, 8>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        if (few_pieces<64>(B, C)) launch4_bwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        else launch4_bwd_reg<RAW, 64, 8, 8>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else if (T <= 128) {
-        launch4_bwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        if (few_pieces<32>(B, C)) launch4_bwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        else launch4_bwd_reg<RAW, 32, 8, 16>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else if (T <= 256) {
-        launch4_bwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        if (few_pieces<16>(B, C)) launch4_bwd_reg<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        else launch4_bwd_reg<RAW, 16, 8, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else if (T <= 512) {
-        launch4_bwd_reg<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        if (few_pieces<16>(B, C)) launch4_bwd_reg<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        else launch4_bwd_reg<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else if (T <= 1024) {
         launch4_bwd_reg<RAW, 8, 16, 64>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else if (T <= BLK_T * BLK_MAX) {
-        if (few_pieces(B, C)) launch4_bwd_blk<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
+        if (few_pieces<16>(B, C)) launch4_bwd_blk<RAW, 8, 8, 64>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
         else launch4_bwd_blk<RAW, 16, 16, 32>(st, B, T, C, w, u, k, v, gy, gw, gu, gk, gv);
     } else {
         const int S = (T + NSEG - 1) / NSEG;
