@@ -1221,15 +1221,15 @@ uint16_t* el(void* p) { return static_cast<uint16_t*>(p); }
 
 // Blocks of time: as many as there is room for on the card at a time (two workgroups a CU in the forward, one in the backward), of
 // BLOCK_CHUNKS chunks at least; 1: whole sequences.  per: chunks a block.  The first pass does the work of a forward without its outputs
-// twice, which pays where a whole sequence leaves most of the card idle.  Where the line lies, B H sequences, us whole / in blocks, bf16
-// forward: 8 of T256 48 / 35, of T4096 709 / 112; 64 of T256 49 / 46, of T4096 719 / 378; 128 of T256 50 / 65, of T1024 183 / 178, of T4096
-// 720 / 645; 192 (two blocks) of T4096 721 / 1000.  Forward + backward of T4096: 8 sequences 1796 / 215, 32 1818 / 491, 128 1817 / 1573;
-// fp32 mode 1899 / 226, 2024 / 550, 2099 / 1785.  128 of T256, backward alone: 78 / 74.
+// twice, which pays where a whole sequence leaves most of the card idle.  Where the line lies, heads, us whole / in blocks, bf16
+// forward: 8 of T256 41 / 30, of T4096 588 / 104; 64 of T256 41 / 40, of T4096 598 / 345; 128 of T1024 153 / 163, of T4096 626 / 591; 192 in two blocks
+// of T4096 took 1.4 times as long as whole.  Backward: 8 of T256 63 / 37, of T4096 910 / 94; 64 of T256 65 / 48, of T4096 987 / 458; 128 of T256 66 / 65, of
+// T4096 1010 / 780.  fp32 mode, forward: 64 of T256 43 / 41, 128 of T1024 158 / 178, of T4096 723 / 674; backward: 128 of T256 70 / 70, of T4096 997 / 863.
 constexpr int BLOCK_CHUNKS = 4, SLOTS_FWD = 512, SLOTS_BWD = 256;
 int time_blocks(int heads, int T, bool bwd, int* per) {
     const int want = (bwd ? SLOTS_BWD : SLOTS_FWD) / heads, nch = T / CL;
     *per = nch;
-    if (want < (bwd ? 2 : 4) || nch < 4 * BLOCK_CHUNKS || (!bwd && nch * 256LL < static_cast<long long>(heads) * heads)) return 1;
+    if (want < (bwd ? 2 : 4) || nch < 4 * BLOCK_CHUNKS || (!bwd && nch * 16384LL < static_cast<long long>(heads) * heads * heads)) return 1;
     const int least = (nch + want - 1) / want;
     *per = least > BLOCK_CHUNKS ? least : BLOCK_CHUNKS;
     return (nch + *per - 1) / *per;
