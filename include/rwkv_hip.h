@@ -382,7 +382,8 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H,
  * stands in for every token's decay in the kernels of rwkv_wkv6f_*, and its gradient is added up over the tokens inside
  * the kernel.  Head size 128: one workgroup holds a whole head; the forward may go without `saved` (nothing is kept then),
  * and the backward needs no more workspace than 4 B C bytes (a multiple of 32 above).  With rwkv_wkv5s_blocks_workspace_bytes (0: no use
- * for it) few long sequences (B H <= 128) are cut into blocks of time that are worked on side by side, in the forward by _forward_ws;
+ * for it) few long sequences (B H <= 128, or that many beyond a multiple of 256) are cut into blocks of time that are worked on side by side, in
+ * the forward by _forward_ws;
  * RWKV_FLAG_WHOLE keeps them whole.  Heads with a decay below e^-9 a step, or one that is no number,
  * run step by step, at both sizes.  `saved`: 64 KB (size 64: 16 KB, for any layer) per head and 64 tokens, 1.07 GB at B8 T4096
  * C4096 (268 MB at C2048).  Other head sizes, RWKV_FLAG_SWEEPS / RWKV_PASS_* or (size 64)
@@ -480,8 +481,8 @@ int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float*
                        void* y, float* sT);
 
 /* Forward and backward of all three ops in both modes with a workspace (rwkv7_workspace_bytes; 0: none is needed): few sequences (B H
- * <= 128) of 256 tokens and more (in the forward also of (B H)^2 / 16 and more) are cut into blocks of time that are worked on side by
- * side.  Without one whole sequences are walked through, as by the other entry points, and results are theirs bit for bit; in blocks they
+ * <= 128) of 256 tokens and more (in the forward also of (B H)^3 / 1024 and more) are cut into blocks of time that are worked on side by
+ * side, and so are those beyond a multiple of 256, if they are few (a workspace that is too small for them is not used).  Without one whole sequences are walked through, as by the other entry points, and results are theirs bit for bit; in blocks they
  * differ by rounding.  s and sa are of one kind either way.  s0, sT, ds0, dsT may be NULL, and s with sa where no backward follows;
  * `backward`: 0 or 1. */
 size_t rwkv7_workspace_bytes(int B, int T, int H, int backward);

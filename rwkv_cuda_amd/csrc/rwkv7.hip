@@ -474,13 +474,22 @@ int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float*
 // All three ops in both modes, chunked kernels, with a workspace for few sequences.
 size_t rwkv7_workspace_bytes(int B, int T, int H, int backward) { return check7(B, T, H) == RWKV_OK ? rwkv7c_workspace_bytes(B, T, H, backward != 0) : 0; }
 
+// A workspace that is too small is an error where few sequences are cut; more heads than CUs need none, and go without
+static bool usable7(void*& ws, size_t bytes, int B, int T, int H, bool bwd) {
+    if (ws == nullptr) return true;
+    if (!aligned16(ws)) return false;
+    if (bytes >= rwkv7c_workspace_bytes(B, T, H, bwd)) return true;
+    if (static_cast<long long>(B) * H < 256) return false;
+    ws = nullptr;
+    return true;
+}
 int rwkv7_forward_ws(void* stream, int B, int T, int H, int fp32, const float* s0, const void* r, const void* w, const void* k,
                      const void* v, const void* a, const void* b, void* y, float* sT, float* s, float* sa, void* workspace, size_t workspace_bytes) {
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, y})) return e;
     if ((s == nullptr) != (sa == nullptr)) return RWKV_ERR_NULL;
     if (!aligned16(s0) || !aligned16(sT) || !aligned16(s) || !aligned16(sa)) return RWKV_ERR_ALIGN;
-    if (workspace != nullptr && (workspace_bytes < rwkv7_workspace_bytes(B, T, H, 0) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+    if (!usable7(workspace, workspace_bytes, B, T, H, false)) return RWKV_ERR_WORKSPACE;
     return launch7c_fwd(static_cast<hipStream_t>(stream), fp32 != 0, B, T, H, s0, r, w, k, v, a, b, y, sT, s, sa, workspace);
 }
 
@@ -490,7 +499,7 @@ int rwkv7_backward_ws(void* stream, int B, int T, int H, int fp32, const void* r
     if (int e = check7(B, T, H)) return e;
     if (int e = check_ptrs({r, w, k, v, a, b, dy, s, sa, dr, dw, dk, dv, da, db})) return e;
     if (!aligned16(dsT) || !aligned16(ds0)) return RWKV_ERR_ALIGN;
-    if (workspace != nullptr && (workspace_bytes < rwkv7_workspace_bytes(B, T, H, 1) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+    if (!usable7(workspace, workspace_bytes, B, T, H, true)) return RWKV_ERR_WORKSPACE;
     return launch7c_bwd(static_cast<hipStream_t>(stream), fp32 != 0, B, T, H, r, w, k, v, a, b, dy, dsT, s, sa, ds0, dr, dw, dk, dv, da, db, workspace);
 }
 

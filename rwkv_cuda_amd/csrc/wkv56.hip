@@ -1508,7 +1508,11 @@ int rwkv_wkv5s_forward_ws(void* stream, int B, int T, int C, int H, const rwkv_b
         const int e = check_ptrs({r, k, v, w_raw, u, y, decay});
         if (e == RWKV_OK) {
             if (saved != nullptr && (saved_bytes < wkv5b_saved_bytes(B, T, C, H) || !aligned16(saved))) return RWKV_ERR_WORKSPACE;
-            if (workspace != nullptr && (workspace_bytes < wkv5b_blocks_bytes(B, T, C, H, false) || !aligned16(workspace))) return RWKV_ERR_WORKSPACE;
+            if (workspace != nullptr && !aligned16(workspace)) return RWKV_ERR_WORKSPACE;
+            if (workspace != nullptr && workspace_bytes < wkv5b_blocks_bytes(B, T, C, H, false)) {
+                if (static_cast<long long>(B) * H < 256) return RWKV_ERR_WORKSPACE;
+                workspace = nullptr;                         // (more heads than CUs need none, and go without)
+            }
             if (int e2 = launch_wkv5b_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, decay, static_cast<float*>(saved), flags & RWKV_FLAG_WHOLE ? nullptr : workspace)) return e2;
             return launch_wkv5_steps_fwd(st, B, T, C, H, r, k, v, w_raw, u, y, nullptr);
         }
