@@ -745,7 +745,7 @@ DEVINL f32x4 causal_split(const Tr& o, lds_t a, bool a3, lds_t b, bool b3, bool 
 //   A:     state parts of dU, dV of (i)      | dU, dW, dV, state update of (i)           | dAB, dAK of (i), both ways; tile, M of (i + 1)
 //   B:     other tile parts, rest of (i - 1) | dY S0, U dS, V dS, dRB, dRK of (i)        | dW S0, state update, dr of (i)
 //   P:     decay sums, U, v, dy (i + 1)      | AR, BK, ES (i + 1)                        | RAW, DWF (i + 1)
-// (the rows of visit i - 1 leave in phase 3, through the two A waves that have no tile there)
+// (the rows of visit i - 1 leave through the A waves)
 
 // ---- role P: elementwise preparation (lane = channel, tokens 4 wp + e) one visit ahead, and the row-wise output stores
 struct Prep7 { uint32_t nx[7][4]; float nsa[4]; };
