@@ -173,7 +173,13 @@ DEVINL float sigmoid_fast(float x) {
 struct Decay { float hi, lo; };
 constexpr float LN2 = 0.69314718055994530942f;
 DEVINL Decay add(const Decay& a, const Decay& b) { return {a.hi + b.hi, a.lo + b.lo}; }
-DEVINL float grow(const Decay& d) { const float e = __builtin_amdgcn_exp2f(d.hi); return fmaf(e, d.lo, e); }
+// e to a sum of decays: the hardware's exponential of the nearest exponent; what that leaves is mostly below half a place of the result, so
+// that it is rounded once.  (exp2 of the first part times 1 + lo is rounded twice: at w = -3 to -8 that is 3 % of the errors of what a
+// chunk hands on and of dv, dk.)
+DEVINL float grow(const Decay& d) {
+    const float t = fmaf(d.lo, 1.44269504088896340736f, d.hi), rest = fmaf(LN2, d.hi - t, d.lo), e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e, rest, e);
+}
 // W_SCALE log2(e) sigmoid(x), from the sigmoid
 DEVINL Decay decay_of_sig(float sig) {
     constexpr double C = -0.6065306597 * 1.44269504088896340736;
@@ -186,9 +192,14 @@ DEVINL Decay decay_of_sig(float sig) {
 // serves both the causal tiles and the state: x[e] = e^{c_L - c_t} (e^{c_t}), t = 4 q + e, e = 0 .. 4, carry to or from the border what
 // is added to the state that is handed on, y[e] = HOLD / x[e] meet the state that came in, which has the chunk's whole decay on it
 // beforehand.  HOLD: or e^9.7 would take inputs out of range that e^4.9 (referred to the chunk's middle) did not.
+// (NEAREST: with a Newton step, which the fp32 results of a backward show and bf16 ones do not)
 constexpr float HOLD = 0.0078125f, UNHOLD = 128.f;
-DEVINL float held_inverse(float x) { return __builtin_amdgcn_rcpf(x) * HOLD; }
-template <bool END> DEVINL void growth(const Decay (&lam)[4], const Decay (*part)[N], int q, int j, float (&x)[5], float (&y)[5]) {
+template <bool NEAREST> DEVINL float held_inverse(float x) {
+    float y = __builtin_amdgcn_rcpf(x);
+    if constexpr (NEAREST) y = fmaf(fmaf(-x, y, 1.f), y, y);
+    return y * HOLD;
+}
+template <bool END, bool NEAREST> DEVINL void growth(const Decay (&lam)[4], const Decay (*part)[N], int q, int j, float (&x)[5], float (&y)[5]) {
     Decay at = {0.f, 0.f};                             // between the thread's tokens and the border
     const int n = END ? 3 - q : q, d = END ? -1 : 1, b = END ? 3 : 0;
     if (n > 0) at = part[b][j];
@@ -199,8 +210,19 @@ template <bool END> DEVINL void growth(const Decay (&lam)[4], const Decay (*part
         const int e = END ? 4 - z : z;
         if (z > 0) at = add(at, lam[END ? e : e - 1]);
         x[e] = grow(at);
-        y[e] = held_inverse(x[e]);
+        y[e] = held_inverse<NEAREST>(x[e]);
     }
+}
+// e to the chunk's whole decay, within half a place: the state takes it on in every chunk, and where it decays slowly its error adds up (64
+// chunks of w = -8: sT 1.10e-7 off with the hardware's exponential, 1.25 with its remainder multiplied in, 1.07 so).  A power of two and
+// the series of e^t for |t| < 0.35, to t^7.  (One coefficient behind an empty asm, or it takes a register across the loop.)
+DEVINL float whole_decay(const Decay (*part)[N], int j) {
+    const Decay d = add(add(part[0][j], part[1][j]), add(part[2][j], part[3][j]));
+    const float n = __builtin_rintf(d.hi), t = fmaf(d.hi - n, LN2, d.lo);
+    float p = 1.f / 5040;
+    asm volatile("" : "+v"(p));
+    p = fmaf(t, p, 1.f / 720); p = fmaf(t, p, 1.f / 120); p = fmaf(t, p, 1.f / 24); p = fmaf(t, p, 1.f / 6); p = fmaf(t, p, 0.5f);
+    return __builtin_ldexpf(1.f + fmaf(t * t, p, t), static_cast<int>(fmaxf(n, -16.f)));            // (fmaxf: a NaN is no integer)
 }
 DEVINL Decay sum4(const Decay (&l)[4]) { return add(add(l[0], l[1]), add(l[2], l[3])); }
 // the same from x, in a backward-less chain: c / (1 + e^-x) with the quotient of the two constants 3e-13 from the product
@@ -285,7 +307,7 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
     };
     auto planes = [&](const int slot) __attribute__((always_inline)) {
         float x[5], y[5];
-        growth<true>(lam, S.part, q, lane, x, y);
+        growth<true, false>(lam, S.part, q, lane, x, y);
         f32x4 as, rs, ks, bs;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -300,7 +322,7 @@ template <bool F32> DEVINL void fwd_role_p(SmemCF& S, const lds_t sb, const Args
         put_twin(sb + F_KB + slot * TWIN3 + twin(lane, q), split3<!F32>(ks), split3<!F32>(bs));
         if constexpr (F32) put3(o + F_V, split3(f32x4{vv[0], vv[1], vv[2], vv[3]}));
         else lds_st<u32x2>(o + F_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
-        if (q == 0) S.dec[slot][lane] = x[0];
+        if (q == 0) S.dec[slot][lane] = whole_decay(S.part, lane);
     };
     const Tr ta = tr_bases(sb + (q < 2 ? F_AS : F_RS), l16, g);
     const lds_t sp = tr_twin(sb + F_KB + ((q & 1) ? 0 : 32), l16, g);
@@ -418,7 +440,8 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
 // instructions a P wave held the vector unit for 512 cycles and took four more planes, twice the exponentials.  That form and this one in
 // alternation on one machine: bf16 355 -> 331 us, 268 -> 241 without KEEP; fp32 mode 386 -> 368, 306 -> 280.
 // Not kept: a ninth wave for the inverse (one workgroup a CU then: 502 us); rows asked for two chunks ahead (bf16 without KEEP 242 -> 253).
-// Errors against 64 bits, T1024, usual decays / strong ones, before -> now, 1e-7: y 1.39 -> 0.81 / 1.47 -> 0.78, sT 0.61 -> 0.58 / 0.61 -> 0.57.
+// Errors against 64 bits, T1024, fp32 mode, with the tiles on fp32 instructions -> now, 1e-7, at w = 0.5 +- 1, 2 +- 0.5, -3 +- 0.5, -6 +- 0.5, -8 +- 0.5:
+// y 1.38 -> 0.80, 1.44 -> 0.78, 1.18 -> 0.96, 1.23 -> 1.16, 1.30 -> 1.22; sT 0.61 -> 0.55, 0.61 -> 0.56, 0.75 -> 0.69, 1.00 -> 0.96, 1.10 -> 1.04.
 template <bool F32, bool KEEP, bool CUT>
 __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c args) {
     const Args7c p = only_whole<CUT>(args);
@@ -488,7 +511,7 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
     };
     auto planes = [&](const int slot) __attribute__((always_inline)) {
         float x[5], y[5];
-        growth<!REV>(lam, S.part, q, lane, x, y);
+        growth<!REV, REV && F32>(lam, S.part, q, lane, x, y);
         f32x4 p1, p2, p3;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -502,7 +525,7 @@ template <bool F32, bool REV> DEVINL void local_role_p(SmemL& S, const lds_t sb,
         put_twin(sb + L_KB + slot * TWIN3 + twin(lane, q), split3<!F32>(p3), split3<!F32>(p2));
         if constexpr (F32) put3(o + L_V, split3(f32x4{widen<F32>(vb[0]), widen<F32>(vb[1]), widen<F32>(vb[2]), widen<F32>(vb[3])}));
         else lds_st<u32x2>(o + L_V, u32x2{vb[0] | (vb[1] << 16), vb[2] | (vb[3] << 16)});
-        if (q == (REV ? 3 : 0)) S.dec[slot][lane] = x[REV ? 4 : 0];
+        if (q == 0) S.dec[slot][lane] = whole_decay(S.part, lane);
     };
     const Tr sp = tr_bases(sb + L_S, l16, g);
     const lds_t pp = tr_twin(sb + L_KB + (q == 0 ? 32 : 0), l16, g);
@@ -658,8 +681,15 @@ __global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
 // 606 / 708 with inputs split once, the tiles with the P waves a phase earlier and what role B waited for with role A; 588 / 642 with one
 // gradient state instead of two and the values that finish a chunk worked out in the phases before, in which role B waited.  First and last
 // form in alternation on one machine.
-// Errors against 64 bits, T1024, usual decays, before -> now, 1e-7: ds0 0.81 -> 0.78, dr 1.12 -> 0.92, dk 1.19 -> 0.94, dv 1.43 -> 0.94,
-// da 1.89 -> 1.37, db 1.85 -> 1.31, dw 6.6 -> 5.4; decays near e^-0.6, where 1 - sig has few digits, dw 57 -> 57, the others 0.88 .. 2.07 -> 0.83 .. 1.36.
+// Errors against 64 bits, T1024, fp32 mode, with the tiles on fp32 instructions -> now, 1e-7, at w = 0.5 +- 1, 2 +- 0.5, -3 +- 0.5, -6 +- 0.5, -8 +- 0.5:
+// ds0 0.82 -> 0.76, 0.84 -> 0.80, 0.82 -> 0.75, 1.05 -> 1.02, 1.15 -> 1.09;
+// dr 1.12 -> 0.90, 1.21 -> 0.88, 1.00 -> 0.97, 1.18 -> 1.14, 1.26 -> 1.20;
+// dw 25.78 -> 20.69, 36.07 -> 25.50, 10.08 -> 9.55, 7.16 -> 6.86, 7.07 -> 6.65;
+// dk 1.19 -> 0.93, 1.31 -> 0.91, 1.05 -> 1.03, 1.24 -> 1.22, 1.32 -> 1.27;
+// dv 1.42 -> 0.93, 1.48 -> 0.91, 1.19 -> 1.02, 1.23 -> 1.22, 1.30 -> 1.27;
+// da 1.88 -> 1.35, 2.03 -> 1.33, 1.62 -> 1.46, 1.76 -> 1.71, 1.90 -> 1.78;
+// db 1.85 -> 1.30, 1.99 -> 1.28, 1.60 -> 1.47, 1.76 -> 1.71, 1.88 -> 1.79.
+// (One w for all steps and channels, where a rounding repeats in every chunk: ds0 1.26 -> 1.14 at -4.3, 0.71 -> 0.72 at -1.)
 constexpr int NTB = 12 * 64;       // waves 0..3 role A, 4..7 role B, 8..11 role P
 
 constexpr int PK = 72;            // row stride (bf16 elements) of a parked output
@@ -799,7 +829,7 @@ template <bool F32> struct In7 {
 template <bool F32> DEVINL f32x4 bwd_planes(const lds_t sb, const lds_t slot, float* dec, const Decay (*part)[N], const Conv7<F32>& y, int wp, int lane) {
     using O = LB<F32>;
     float x[5], i[5];
-    growth<false>(y.lam, part, wp, lane, x, i);
+    growth<false, F32>(y.lam, part, wp, lane, x, i);
     const In7<F32> in{y};
     f32x4 as, rs, bs, ks;
 #pragma unroll
@@ -815,7 +845,7 @@ template <bool F32> DEVINL f32x4 bwd_planes(const lds_t sb, const lds_t slot, fl
     // (x is not above 1: what comes from bf16 inputs stays within bf16's range)
     put_twin(o + O::AR, split3<!F32>(as), split3<!F32>(rs));
     put_twin(o + O::BK, split3(bs), split3(ks));
-    if (wp == 3) dec[lane] = x[4];
+    if (wp == 0) dec[lane] = whole_decay(part, lane);
     return {x[1], x[2], x[3], x[4]};
 }
 template <bool F32> DEVINL void bwd_planes_rest(const lds_t sb, const lds_t slot, const f32x4& es, const Conv7<F32>& y, int wp, int lane) {
@@ -1103,13 +1133,13 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             put(2, p.db, v, dBp * (eb[v] * UNHOLD));
             put(3, p.dk, v, dKp * (eb[v] * UNHOLD));
             ada[v] = va[v] * dAp;
-            del[v] = fmaf(vr[v], dRp[v], -UNHOLD * fmaf(vb[v], dBp, vk[v] * dKp));      // r dr - b db - k dk
+            del[v] = fmaf(vr[v], dRp[v], -UNHOLD * fmaf(vk[v], dKp, vb[v] * dBp));      // r dr - b db - k dk
         }
         // G_t = P_{t+1} + del_t,  P_t = G_t + a da:  suffix sums over t = 4 g + v, later lane groups first
-        const float tot = (del[0] + ada[0]) + (del[1] + ada[1]) + (del[2] + ada[2]) + (del[3] + ada[3]);
+        const float tot = ((del[0] + ada[0]) + (del[1] + ada[1])) + ((del[2] + ada[2]) + (del[3] + ada[3]));
         auto of_lane = [](uint32_t l, float x) __attribute__((always_inline)) { return __int_as_float(__builtin_amdgcn_ds_bpermute(static_cast<int>(4 * l), __float_as_int(x))); };
         const float t1 = of_lane(me + 16, tot), t2 = of_lane(me + 32, tot), t3 = of_lane(me + 48, tot);
-        float Pn = Pj + (me < 48 ? t1 : 0.f) + (me < 32 ? t2 : 0.f) + (me < 16 ? t3 : 0.f);     // P after this lane's last token
+        float Pn = Pj + ((me < 48 ? t1 : 0.f) + ((me < 32 ? t2 : 0.f) + (me < 16 ? t3 : 0.f)));     // P after this lane's last token
 #pragma unroll
         for (int v = 3; v >= 0; --v) {
             const float G = Pn + del[v];
@@ -1177,7 +1207,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             ea0 = lds_ld<float>(sb + copy_of(i) + L::ES + 12 + piece2(16 * q + (me & 15), me > 15 ? (me >> 4) - 1 : 0));
             if (me < 16) ea0 = 1.f;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) eb[v] = held_inverse(er[v]);                    // (er is between e^-9.8 and 1)
+            for (int v = 0; v < 4; ++v) eb[v] = held_inverse<F32>(er[v]);                    // (er is between e^-9.8 and 1)
             asm volatile("" : "+v"(er), "+v"(eb), "+v"(ea0));
             Sum2 pa = SUM0;
 #pragma unroll

@@ -376,3 +376,25 @@ def test_where_an_infinity_reaches(lib, dtype, name, value):
         per_head = (lambda z: z) if n in ("sT", "ds0") else (lambda z: z.transpose(1, 2))         # [B, H, ...]
         c, g = per_head(c), per_head(g)
         assert torch.equal(c[1], g[1]) and torch.equal(c[0, 1], g[0, 1]), n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("c", [-8.0, -5.0, -2.0, 2.0])
+def test_rwkv7_the_decay_of_a_chunk_is_within_half_a_place(lib, c, dtype):
+    """One chunk, all other inputs zero, states of ones: sT and ds0 are the chunk's decay as the kernels multiply states by it.  Where it is
+    slow its rounding is what adds up over a sequence.  Bound: half a place of the result, and of the exponent 2^-20 for the steps' sigmoids
+    (argument of up to 14 rounded 3.3e-7, its constant 1.4e-7, exponential, sum, reciprocal and product 4e-7) and for the series."""
+    B, T, H, N = 1, 16, 64, 64
+    g = torch.Generator().manual_seed(int(10 - 10 * c))
+    w = (c + 0.5 * torch.randn(B, T, H, N, generator=g)).to(dtype).to(DEV)
+    zero, one, f32 = torch.zeros_like(w), torch.ones(B, H, N, N, device=DEV), int(dtype == torch.float32)
+    y, sT, s, sa = torch.empty_like(w), torch.empty_like(one), torch.empty_like(one), torch.empty(B, T, H, N, device=DEV)
+    call("rwkv7_forward_ws", y.device, B, T, H, f32, one, zero, w, zero, zero, zero, zero, y, sT, s, sa, None, 0)
+    ds0, d = torch.empty_like(one), [torch.empty_like(w) for _ in range(6)]
+    call("rwkv7_backward_ws", y.device, B, T, H, f32, zero, w, zero, zero, zero, zero, zero, one, s, sa, ds0, *d, None, 0)
+    e = -0.6065306597 * torch.sigmoid(w.double()).sum(1)[:, :, None, :]
+    place = torch.exp2(torch.floor(e / math.log(2)) - 23)
+    for name, x in (("sT", sT), ("ds0", ds0)):
+        off = (x.double() - e.exp()).abs()
+        print(f"  {name}: {float((off / place).max()):.3f} places", flush=True)
+        assert bool((off <= 0.5 * place - e * e.exp() * 2.0 ** -20).all()), name
