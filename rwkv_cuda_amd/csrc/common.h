@@ -51,6 +51,59 @@ template <int J> DEVINL void mul_bc(float& s, float row_vec) {               // 
     asm("v_mul_f32_dpp %0, %1, %0 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
         : "+v"(s) : "v"(row_vec), "n"(J));
 }
+// The sums of a triangular solve by such broadcasts: SOLVE_ROWS m[s] += x[t][lane s] m[t] for t from 15 down and s < t, SOLVE_COLS for t
+// from 0 up and s > t.  x[t] comes from wherever the caller's code left it, so all of it is one statement behind its own wait states:
+// between single ones the compiler could copy an x[t] and, as it does not look into assembly, leave out the wait.
+#define RWKV_BC(t, x, s) "v_fmac_f32_dpp %" #s ", %" #x ", %" #t " row_newbcast:" #s " row_mask:0xf bank_mask:0xf\n\t"
+#define RWKV_DOWN1(t, x) RWKV_BC(t, x, 0)
+#define RWKV_DOWN2(t, x) RWKV_BC(t, x, 1) RWKV_DOWN1(t, x)
+#define RWKV_DOWN3(t, x) RWKV_BC(t, x, 2) RWKV_DOWN2(t, x)
+#define RWKV_DOWN4(t, x) RWKV_BC(t, x, 3) RWKV_DOWN3(t, x)
+#define RWKV_DOWN5(t, x) RWKV_BC(t, x, 4) RWKV_DOWN4(t, x)
+#define RWKV_DOWN6(t, x) RWKV_BC(t, x, 5) RWKV_DOWN5(t, x)
+#define RWKV_DOWN7(t, x) RWKV_BC(t, x, 6) RWKV_DOWN6(t, x)
+#define RWKV_DOWN8(t, x) RWKV_BC(t, x, 7) RWKV_DOWN7(t, x)
+#define RWKV_DOWN9(t, x) RWKV_BC(t, x, 8) RWKV_DOWN8(t, x)
+#define RWKV_DOWN10(t, x) RWKV_BC(t, x, 9) RWKV_DOWN9(t, x)
+#define RWKV_DOWN11(t, x) RWKV_BC(t, x, 10) RWKV_DOWN10(t, x)
+#define RWKV_DOWN12(t, x) RWKV_BC(t, x, 11) RWKV_DOWN11(t, x)
+#define RWKV_DOWN13(t, x) RWKV_BC(t, x, 12) RWKV_DOWN12(t, x)
+#define RWKV_DOWN14(t, x) RWKV_BC(t, x, 13) RWKV_DOWN13(t, x)
+#define RWKV_DOWN15(t, x) RWKV_BC(t, x, 14) RWKV_DOWN14(t, x)
+#define RWKV_UP15(t, x) RWKV_BC(t, x, 15)
+#define RWKV_UP14(t, x) RWKV_BC(t, x, 14) RWKV_UP15(t, x)
+#define RWKV_UP13(t, x) RWKV_BC(t, x, 13) RWKV_UP14(t, x)
+#define RWKV_UP12(t, x) RWKV_BC(t, x, 12) RWKV_UP13(t, x)
+#define RWKV_UP11(t, x) RWKV_BC(t, x, 11) RWKV_UP12(t, x)
+#define RWKV_UP10(t, x) RWKV_BC(t, x, 10) RWKV_UP11(t, x)
+#define RWKV_UP9(t, x) RWKV_BC(t, x, 9) RWKV_UP10(t, x)
+#define RWKV_UP8(t, x) RWKV_BC(t, x, 8) RWKV_UP9(t, x)
+#define RWKV_UP7(t, x) RWKV_BC(t, x, 7) RWKV_UP8(t, x)
+#define RWKV_UP6(t, x) RWKV_BC(t, x, 6) RWKV_UP7(t, x)
+#define RWKV_UP5(t, x) RWKV_BC(t, x, 5) RWKV_UP6(t, x)
+#define RWKV_UP4(t, x) RWKV_BC(t, x, 4) RWKV_UP5(t, x)
+#define RWKV_UP3(t, x) RWKV_BC(t, x, 3) RWKV_UP4(t, x)
+#define RWKV_UP2(t, x) RWKV_BC(t, x, 2) RWKV_UP3(t, x)
+#define RWKV_UP1(t, x) RWKV_BC(t, x, 1) RWKV_UP2(t, x)
+#define RWKV_SOLVE_OPERANDS \
+    : "+&v"(m[0]), "+&v"(m[1]), "+&v"(m[2]), "+&v"(m[3]), "+&v"(m[4]), "+&v"(m[5]), "+&v"(m[6]), "+&v"(m[7]), \
+      "+&v"(m[8]), "+&v"(m[9]), "+&v"(m[10]), "+&v"(m[11]), "+&v"(m[12]), "+&v"(m[13]), "+&v"(m[14]), "+&v"(m[15]) \
+    : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), \
+      "v"(x[8]), "v"(x[9]), "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15])
+template <bool ROWS> DEVINL void solve_bc(float (&m)[16], const float (&x)[16]) {      // operands 0..15 are m, 16..31 x
+    if constexpr (ROWS)
+        asm("s_nop 1\n\t"
+            RWKV_DOWN15(15, 31) RWKV_DOWN14(14, 30) RWKV_DOWN13(13, 29) RWKV_DOWN12(12, 28) RWKV_DOWN11(11, 27)
+            RWKV_DOWN10(10, 26) RWKV_DOWN9(9, 25) RWKV_DOWN8(8, 24) RWKV_DOWN7(7, 23) RWKV_DOWN6(6, 22)
+            RWKV_DOWN5(5, 21) RWKV_DOWN4(4, 20) RWKV_DOWN3(3, 19) RWKV_DOWN2(2, 18) RWKV_DOWN1(1, 17)
+            RWKV_SOLVE_OPERANDS);
+    else
+        asm("s_nop 1\n\t"
+            RWKV_UP1(0, 16) RWKV_UP2(1, 17) RWKV_UP3(2, 18) RWKV_UP4(3, 19) RWKV_UP5(4, 20)
+            RWKV_UP6(5, 21) RWKV_UP7(6, 22) RWKV_UP8(7, 23) RWKV_UP9(8, 24) RWKV_UP10(9, 25)
+            RWKV_UP11(10, 26) RWKV_UP12(11, 27) RWKV_UP13(12, 28) RWKV_UP14(13, 29) RWKV_UP15(14, 30)
+            RWKV_SOLVE_OPERANDS);
+}
 template <int J> DEVINL float bc(float row_vec) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, row_vec),
                                                                 0x150 + J, 0xf, 0xf, true));

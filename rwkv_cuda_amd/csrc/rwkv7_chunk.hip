@@ -127,22 +127,6 @@ DEVINL f32x4 by_group(int g, float (&x)[CL]) {
 // need inside the multiplication, so the tile is read once.  (With every element read from LDS where it was needed, 38 reads in a chain, the
 // wave that makes M took 5100 cycles of the forward's phase and the others 3400: B=8, T=1024, H=64 without a gradient 243 -> 240 us in bf16 and
 // 283 -> 274 in fp32, fp32 backward 642 -> 631; B=1, T=4096, H=32 without a gradient 175 -> 164 and 183 -> 175.)
-template <int t, int s, bool ROWS> DEVINL void inverse_step(float (&m)[CL], const float (&x)[CL]) {
-    if constexpr (ROWS) {            // m[s] += M[r][t] AB[t][s], s < t, t from the end down; x[t] = AB[t][s] in lane s
-        fmac_bc<s>(m[s], x[t], m[t]);
-        if constexpr (s > 0) inverse_step<t, s - 1, ROWS>(m, x);
-    } else {                          // m[s] += AB[s][t] M[t][c], s > t, t from the start up; x[t] = AB[s][t] in lane s
-        fmac_bc<s>(m[s], x[t], m[t]);
-        if constexpr (s + 1 < CL) inverse_step<t, s + 1, ROWS>(m, x);
-    }
-}
-template <int t, bool ROWS> DEVINL void inverse_lines(float (&m)[CL], const float (&x)[CL]) {
-    if constexpr (ROWS) {
-        if constexpr (t > 0) { inverse_step<t, t - 1, true>(m, x); inverse_lines<t - 1, true>(m, x); }
-    } else {
-        if constexpr (t + 1 < CL) { inverse_step<t, t + 1, false>(m, x); inverse_lines<t + 1, false>(m, x); }
-    }
-}
 // ROWS: lane l16 = r gets M[r][0 .. 15] from M[r][s] = [r == s] + sum_{t>s} M[r][t] AB[t][s]; lines holds AB[.][s] as its row s.
 // Otherwise lane l16 = c gets M[0 .. 15][c] from M[t][c] = [t == c] + sum_{s<t} AB[t][s] M[s][c]; lines holds AB itself.
 template <bool ROWS> DEVINL void inverse(const float (*lines)[TS], int l16, float (&m)[CL]) {
@@ -156,7 +140,7 @@ template <bool ROWS> DEVINL void inverse(const float (*lines)[TS], int l16, floa
     asm volatile("" : "+v"(l16));            // (or sixteen comparisons with it live in registers across the caller's loop)
 #pragma unroll
     for (int i = 0; i < CL; ++i) m[i] = l16 == i ? 1.f : 0.f;
-    inverse_lines<ROWS ? CL - 1 : 0, ROWS>(m, x);
+    solve_bc<ROWS>(m, x);
 }
 
 // (a Newton step behind the hardware reciprocal instead of a full division, a sixth of the vector instructions that turn inputs into
