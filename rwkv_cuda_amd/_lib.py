@@ -36,7 +36,8 @@ HIPCC_FLAGS = [
 # build.
 # The row-per-thread kernels for other head sizes (wkv_rows) keep a whole state row in registers; an instantiation that
 # no longer fits gave wrong results on the GPU (fp32 decay-gradient sweep at 128), so none may spill.
-# The wkv4 kernels that hold a segment's inputs in registers exist to avoid memory round trips: a spill defeats them.
+# The wkv4 kernels that hold a segment's inputs in registers exist to avoid memory round trips: a spill of one of them defeats them.  The
+# backward for more than 1024 steps, 16 channels and 16 steps a lane, keeps five other values in scratch (see the kernel): these and no more.
 # The depthwise_conv1d matrix-core kernels hold the next unit's rows in registers across their product loops, which run at
 # the register limit: a spill there is scratch traffic in the innermost loop.
 # wkv5c_bwd runs at the register limit too (256, eight waves a CU) and keeps a few values that a wave needs once a chunk in scratch:
@@ -45,7 +46,8 @@ HIPCC_FLAGS = [
 # The one-sweep kernels let the compiler count their waits: a spill inside their loops would put scratch traffic between a
 # prefetch and its use (and a forward variant that spilled eleven registers gave wrong results): none may spill.
 SPILL_LIMIT = {"wkv6_local": 0, "wkv6_bwd_fused": 0, "wkv6_fwd_fused": 0, "wkv6_fwd_ws": 0, "wkv6_bwd_a_ws": 0, "wkv6_bwd_b_wsILi0E": 3, "wkv6_bwd_b_wsILi1E": 1, "wkv6_bwd_b_wsILi2E": 1,
-               "wkv_rows": 0, "wkv5_steps": 0, "wkv5b_fwd": 0, "wkv5b_bwd": 0, "wkv5b_local": 0, "wkv5c_fwd": 0, "wkv5c_bwdILb0E": 6, "wkv5c_bwdILb1E": 9, "wkv4_fwd_reg": 0, "wkv4_bwd_reg": 0, "timex_conv_h2": 0, "timex_gw_sum_h2": 0,
+               "wkv_rows": 0, "wkv5_steps": 0, "wkv5b_fwd": 0, "wkv5b_bwd": 0, "wkv5b_local": 0, "wkv5c_fwd": 0, "wkv5c_bwdILb0E": 6, "wkv5c_bwdILb1E": 9, "wkv4_fwd_reg": 0, "wkv4_bwd_reg": 0, "wkv4_fwd_blk": 0, "wkv4_bwd_blkILb0ELi8E": 0,
+               "wkv4_bwd_blkILb1ELi8E": 0, "wkv4_bwd_blkILb0ELi16E": 5, "wkv4_bwd_blkILb1ELi16E": 5, "timex_conv_h2": 0, "timex_gw_sum_h2": 0,
                "timex_conv_any": 0, "timex_gw_any": 0, "timex_gw_short": 0, "rwkv7c_fwd": 0, "rwkv7c_bwd": 0, "rwkv7c_local": 0, "rwkv7c_scan": 0}
 
 _lib = None

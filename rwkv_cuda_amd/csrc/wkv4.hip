@@ -669,6 +669,10 @@ __global__ __launch_bounds__(CHR * SEG, 4) void wkv4_bwd_reg(int T, int C, int S
 // C2500 335 -> 221 (the forward that way: B12 T4000 C768 156 -> 169, B17 T2000 C768 100 -> 97).
 // Where there are few pieces both take 8 channels and 64 segments: B2 T4000 C768 52 -> 44 /
 // 145 -> 116 (backward in 32 segments: 137), B1 T4096 C2048 51 -> 43 / 142 -> 107 (138); with 144 pieces it is 53 -> 56 / 147 -> 143 (140).
+// The backward with 16 steps a lane has no register left of the 128 that two workgroups a CU may have, and five values in scratch, none of
+// them an input: a lane writes two and reads three of them once a block of 512 steps.  Without any (the difference that both descending sweeps
+// form worked out twice, gy and 1/den as their product, the step of a row not kept): B28 T1100 C768 211 -> 217, B17 T2000 C768 231 -> 236, B2 T4000 C2500
+// 217 -> 222, B6 T4000 C768 231 -> 226, B1 T32768 C2100 1283 -> 1334, so not so.
 constexpr int BLK_T = 512;
 constexpr int BLK_MAX = 64;            // blocks whose entering states fit in LDS: T <= 32768
 
