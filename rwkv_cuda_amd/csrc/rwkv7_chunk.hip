@@ -38,6 +38,7 @@
 // Private layout of the interface's scratch tensors: `s` slot c holds the state ENTERING chunk c as [i][j] fp32 (the
 // reference stores the state leaving it; the backward here needs the entering one and never inverts a step), `sa` is U.
 #include <stddef.h>
+#include <algorithm>
 
 #include "split3.h"
 
@@ -1276,15 +1277,19 @@ template <bool F32, bool REV> int cut(hipStream_t st, int heads, Args7c& p, void
     rwkv7c_scan<REV><<<dim3(4 * heads), dim3(256), 0, st>>>(p);
     return launch_status();
 }
-// whole sequences, then those in blocks: a launch each, of the heads from p.at on
+// whole sequences, then those in blocks: a launch each, of the heads from p.at on.  More than LAUNCH_HEADS are several: beyond 2^32 work items along
+// x a launch does the remainder only, and reports no error (forward, 16 tokens of 8.4 million heads).
+constexpr int LAUNCH_HEADS = 1 << 22;
+static_assert(static_cast<long long>(LAUNCH_HEADS) * NTB < 1LL << 32 && LAUNCH_HEADS * static_cast<long long>(NTF) < 1LL << 32, "work items of a launch");
 template <bool F32, bool REV, typename Whole, typename Blocks> int in_parts(hipStream_t st, int B, Args7c& p, void* ws, Whole whole, Blocks blocks) {
     Split7 x = split_heads(B, p.T, p.H, REV);
     if (x.whole + x.rest == 0) return RWKV_ERR_SHAPE;
     if (ws == nullptr) x = {B * p.H, 0, 1, p.T / CL};
     p.NB = 1; p.at = 0;
-    if (x.whole > 0) {
-        whole(p, dim3(x.whole));
+    for (; p.at < x.whole; p.at += LAUNCH_HEADS) {
+        whole(p, dim3(std::min(x.whole - p.at, LAUNCH_HEADS)));
         if (int e = launch_status()) return e;
+        if (x.whole - p.at <= LAUNCH_HEADS) break;           // (p.at would go beyond what an int holds)
     }
     if (x.rest == 0) return RWKV_OK;
     p.NB = x.NB; p.per = x.per; p.at = x.whole;

@@ -398,3 +398,21 @@ def test_rwkv7_the_decay_of_a_chunk_is_within_half_a_place(lib, c, dtype):
         off = (x.double() - e.exp()).abs()
         print(f"  {name}: {float((off / place).max()):.3f} places", flush=True)
         assert bool((off <= 0.5 * place - e * e.exp() * 2.0 ** -20).all()), name
+
+
+def test_rwkv7_more_heads_than_one_launch_takes(lib):
+    """8.4 million heads of 16 tokens: 512 work items each are more than the 2^32 that a launch may have along x (beyond, it runs the remainder
+    of 2^32 and reports nothing).  One tensor (17 GB) is all six inputs; the rows at
+    either end and at the border of the launches have the bits of a call of their own."""
+    B, T, H, N = 32768, 16, 257, 64
+    g = torch.Generator().manual_seed(3)
+    x = (torch.randn(1, T, H * N, generator=g) * 0.1).to(torch.bfloat16).to(DEV).repeat(B, 1, 1)
+    rows = [0, 16319, 16320, 16321, 32640, 32641, 32767]      # (2^22 heads: within row 16320)
+    for i in rows:
+        x[i] = (torch.randn(T, H * N, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+    y = torch.empty_like(x)
+    call("rwkv7_forward_ws", y.device, B, T, H, 0, None, x, x, x, x, x, x, y, None, None, None, None, 0)
+    few, want = x[rows].contiguous(), torch.empty(len(rows), T, H * N, dtype=torch.bfloat16, device=DEV)
+    call("rwkv7_forward_ws", y.device, len(rows), T, H, 0, None, few, few, few, few, few, few, want, None, None, None, None, 0)
+    same = [torch.equal(y[i], z) for i, z in zip(rows, want)] + [torch.equal(y[1], y[-3])]
+    assert all(same), same
