@@ -335,6 +335,33 @@ def test_wkv5_heads_of_128_beyond_a_multiple_of_the_cus(lib, B, H, T, forward, b
             assert float((a - b).norm() / b.norm()) <= 2.0 ** -8 * (1 if z < 4 else 2), z
 
 
+@pytest.mark.parametrize("B,H,T,rest", [(1, 257, 321, 1), (8, 36, 350, 32)])
+def test_wkv5_heads_of_128_beyond_a_multiple_of_the_cus_keep_what_their_backward_reads(lib, B, H, T, rest):
+    """`decay` and `saved` of a forward whose last heads are done in blocks: the bits of whole sequences but for the states of those heads, and the
+    gradients from them.  These states differ by roundings of fp32 sums and of bf16 operands, 2^-8 at most; a block's states in the wrong place would be off by their own size."""
+    C, WHOLE = H * 128, 0x200
+    n = [lib.rwkv_wkv5s_blocks_workspace_bytes(B, T, C, H, i) for i in (0, 1)]
+    assert n[0] > 0
+    r, k, v, w, u, gy = (x.to(DEV) for x in synth.wkv5_inputs(B, T, C, H, seed=H))
+    rows = lambda t: t.view(B, T, H, 128).transpose(1, 2).reshape(B * H, -1)
+    ns, nb = lib.rwkv_wkv5s_saved_bytes(B, T, C, H), max(n[1], lib.rwkv_wkv5s_backward_workspace_bytes(B, T, C, H))
+    res = []
+    for flags in (0, WHOLE):
+        y, ws = garbage((B, T, C), torch.bfloat16), garbage((n[0],), torch.uint8) if not flags else None
+        saved, decay = garbage((ns // 4,), torch.float32), garbage((2 * C,), torch.float32)
+        call("rwkv_wkv5s_forward_ws", y.device, B, T, C, H, r, k, v, w, u, y, decay, saved, ns, ws, n[0] if ws is not None else 0, flags)
+        g, gw, gu = [garbage((B, T, C), torch.bfloat16) for _ in range(3)], garbage((H, 128), torch.bfloat16), garbage((H, 128), torch.bfloat16)
+        call("rwkv_wkv5s_backward", y.device, B, T, C, H, r, k, v, w, decay, u, gy, *g, gw, gu, saved, ns, garbage((nb,), torch.uint8), nb, flags)
+        res.append([decay, saved.view(B * H, -1)] + [rows(t) for t in g] + [gw, gu])
+    (decay, saved, *grads), (decay1, saved1, *grads1) = res
+    m = B * H - rest
+    same = [torch.equal(decay, decay1), torch.equal(saved[:m], saved1[:m])]
+    assert all(same), same
+    for z, (got, whole) in enumerate(zip([saved[m:]] + grads, [saved1[m:]] + grads1)):
+        for a, b in zip(got.double(), whole.double()):
+            assert float((a - b).norm() / b.norm()) <= 2.0 ** -8 * (1 if z < 4 else 2), z
+
+
 @pytest.mark.parametrize("H,T", [(3, 257), (3, 1100), (3, 2300), (64, 1025), (100, 641), (100, 1300)])       # 2, 9, 18 (a scan of its own), 4, 2, 2 blocks of 128 .. 704 tokens
 def test_wkv6_state_blocks_of_every_length(lib, H, T):
     """The first pass takes a block's tokens up to 256 at a time, 32 or more a part; three heads of the layer against the oracle."""
