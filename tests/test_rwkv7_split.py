@@ -131,3 +131,56 @@ def test_constants_of_the_decay():
     C, M = (float.fromhex(z) for z in m.groups())
     assert float(np.float32(C)) == C and float(np.float32(M)) == M
     assert abs(M / C / (-0.6065306597 * 1.4426950408889634) - 1) < 1e-12
+
+
+def decay_sources():
+    """The two forms of a step's decay in csrc/rwkv7_chunk.hip, from a sigmoid (backward) and from the input (forward, blocks), with the source's
+    own constants: functions of the input in fp64 that give the two parts, fused operations in fp64 and rounded."""
+    with open(os.path.join(CSRC, "rwkv7_chunk.hip")) as f:
+        text = f.read()
+    f32, fma = np.float32, lambda a, b, c: (a.astype(np.float64) * np.float64(b) + c).astype(np.float32)
+    ln2 = f32(float(re.search(r"constexpr float LN2 = ([\d.]+)f;", text).group(1)))
+    a = text[text.index("DEVINL Decay decay_of_sig(float sig) {"):]
+    a = a[:a.index("\n}")]
+    w, log2e = map(float, re.search(r"constexpr double C = (-[\d.]+) \* ([\d.]+);", a).groups())
+    assert "HI = static_cast<float>(C), LO = static_cast<float>(C - static_cast<double>(HI));" in a
+    off = {float(z) for z in re.search(r"hi = fmaf\(sig, HI, ([\d.]+)f\) - ([\d.]+)f;", a).groups()}
+    assert "return {hi, LN2 * fmaf(sig, LO, fmaf(sig, HI, -hi))};" in a
+    HI = f32(w * log2e)
+    LO = f32(w * log2e - float(HI))
+    b = text[text.index("DEVINL Decay decay_of(float x) {"):]
+    b = b[:b.index("\n}")]
+    C, M = (float.fromhex(z) for z in re.search(r"constexpr float C = (\S+)f, M = (\S+)f;", b).groups())
+    assert "d = fmaf(__builtin_amdgcn_exp2f(x * -1.44269504088896340736f), C, C);" in b and "return {hi, LN2 * fmaf(s, M, -hi)};" in b
+    off |= {float(z) for z in re.search(r"hi = fmaf\(s, M, ([\d.]+)f\) - ([\d.]+)f;", b).groups()}
+    assert len(off) == 1
+    off = off.pop()
+
+    def of_sig(x):
+        sig = (1 / (1 + np.exp(-x))).astype(f32)
+        hi = fma(sig, HI, off) - f32(off)
+        return hi, ln2 * fma(sig, LO, fma(sig, HI, -hi.astype(np.float64)).astype(np.float64))
+
+    def of_input(x):
+        s = (1 / (C * (1 + np.exp(-x)))).astype(f32)
+        hi = fma(s, M, off) - f32(off)
+        return hi, ln2 * fma(s, M, -hi.astype(np.float64))
+
+    return of_sig, of_input
+
+
+def test_both_forms_of_the_decay_add_up_exactly_and_agree():
+    """The backward uses states that the forward has decayed.  Bound of their difference: a sigmoid's rounding of 2^-24 and a product's of 2^-24
+    each, of the sum of 16; second parts to 2^-24 of 2^-20."""
+    rng = np.random.default_rng(4)
+    x = np.concatenate([rng.normal(c, s, (2000, 16)) for c in (-8, -5, -2, 0.5, 3) for s in (0, 1)] + [np.full((1, 16), z) for z in (30.0, 0.0, -80.0)])
+    exact = -0.6065306597 / (1 + np.exp(-x))
+    totals = []
+    for form in decay_sources():
+        hi, lo = form(x)
+        assert np.all(np.abs(lo) <= 2.0 ** -20) and np.all(np.abs(hi) < 1) and np.all(hi * 2.0 ** 19 == np.round(hi * 2.0 ** 19))
+        for order in (slice(None), slice(None, None, -1), rng.permutation(16)):
+            assert np.array_equal(np.cumsum(hi[:, order], axis=1, dtype=np.float32), np.cumsum(hi[:, order].astype(np.float64), axis=1))
+        totals.append(hi.astype(np.float64).sum(1) * np.log(2) + lo.astype(np.float64).sum(1))
+        assert np.all(np.abs(totals[-1] - exact.sum(1)) <= np.abs(exact).sum(1) * 2.0 ** -23 + 16 * 2.0 ** -44)
+    assert np.all(np.abs(totals[0] - totals[1]) <= np.abs(exact).sum(1) * 2.0 ** -22 + 32 * 2.0 ** -44)
