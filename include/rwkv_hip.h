@@ -482,9 +482,11 @@ int rwkv7_forward_only(void* stream, int B, int T, int H, int fp32, const float*
 
 /* Forward and backward of all three ops in both modes with a workspace (rwkv7_workspace_bytes; 0: none is needed): few sequences (B H
  * <= 128) of 256 tokens and more (in the forward also of (B H)^3 / 1024 and more) are cut into blocks of time that are worked on side by
- * side, and so are those beyond a multiple of 256, if they are few (a workspace that is too small for them is not used).  Without one whole sequences are walked through, as by the other entry points, and results are theirs bit for bit; in blocks they
- * differ by rounding.  s and sa are of one kind either way.  s0, sT, ds0, dsT may be NULL, and s with sa where no backward follows;
- * `backward`: 0 or 1. */
+ * side, and so are those beyond a multiple of 256 if they are few (up to 96 in the backward, of 4 B H % 256 tokens and more; up to 16 in the
+ * forward, of 768 and more).  There a workspace that is too small is not used; with B H < 256 it is an error.  Without one whole sequences are walked
+ * through, as by the other entry points, and results are theirs bit for bit; in blocks they differ by rounding, so that a sequence's results
+ * depend on its place in the batch, and calls that pass the state on give one call's bits only without.  s and sa are of one kind either way.
+ * s0, sT, ds0, dsT may be NULL, and s with sa where no backward follows; sT may be s0's memory and ds0 that of dsT; `backward`: 0 or 1. */
 size_t rwkv7_workspace_bytes(int B, int T, int H, int backward);
 int rwkv7_forward_ws(void* stream, int B, int T, int H, int fp32, const float* s0,
                      const void* r, const void* w, const void* k, const void* v, const void* a, const void* b,

@@ -91,6 +91,12 @@ DEVINL Head7 head_of(const Args7c& p, int n) {
     const int bh = p.at + n, b = __builtin_amdgcn_readfirstlane(bh / p.H);
     return {static_cast<size_t>(bh), b, bh - b * p.H};
 }
+// The state of head bh (s0 or dsT) that the first block in the direction of travel starts from.  In blocks it is the copy that rwkv7c_scan leaves
+// in the place of the first block's E: the last block may have written sT (ds0) by then, and that may be the same tensor.
+DEVINL const float* first_state(const Args7c& p, const float* x, size_t bh) {
+    if (x == nullptr) return nullptr;
+    return p.NB > 1 ? p.local + static_cast<size_t>(blockIdx.x) * (p.NB - 1) * 2 * N * N : x + bh * N * N;
+}
 // The chunks of the workgroup's block; false: another workgroup does them.
 struct Part7 { int n, first, chunks; };
 DEVINL bool part_of(const Args7c& p, Part7& x) {
@@ -440,7 +446,7 @@ __global__ __launch_bounds__(NTF, 4) void rwkv7c_fwd(const Args7c args) {
     const size_t tok0 = static_cast<size_t>(b) * p.T + x.first * CL;  // first token row of this block
     if (w < 4) {
         const int all = p.T / CL;
-        const float* const s0 = x.n > 0 ? p.enter + (static_cast<size_t>(blockIdx.x) * (p.NB - 1) + x.n - 1) * N * N : (p.s0 != nullptr ? p.s0 + bh * N * N : nullptr);
+        const float* const s0 = x.n > 0 ? p.enter + (static_cast<size_t>(blockIdx.x) * (p.NB - 1) + x.n - 1) * N * N : first_state(p, p.s0, bh);
         float* const sT = p.sT != nullptr && x.first + x.chunks == all ? p.sT + bh * N * N : nullptr;
         fwd_role_s<F32, KEEP>(S, sb, p, s0, sT, KEEP ? p.s + (bh * all + x.first) * N * N : nullptr, w, tid, tok0, x.chunks, h);
     } else fwd_role_p<F32>(S, sb, p, w - 4, tid & 63, tok0, x.chunks, h);
@@ -629,6 +635,8 @@ __global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
     };
     Block now, next;
     fetch(now);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) p.local[head * (p.NB - 1) * 2 * N * N + o + v * N] = x[v];      // (this thread has these elements of the first E; first_state)
     float bad = 0.f;
     for (int m = 0; m + 1 < p.NB; ++m, to += N * N) {
         if (m + 2 < p.NB) at += 2 * N * N;
@@ -1226,7 +1234,7 @@ __global__ __launch_bounds__(NTB, 3) void rwkv7c_bwd(const Args7c args) {
     // (thread numbers anew: role B has no register to hold one across its loop for the code of the others, which lies behind)
     const auto again = [&]() __attribute__((always_inline)) { return 64 * w + static_cast<int>(lane_again()); };
     if (w >= 8) { bwd_role_p(S, sb, p, again(), w, tok0, nch, p.H, h); return; }
-    const float* const dsT = x.first + nch < all ? p.enter + (static_cast<size_t>(blockIdx.x) * (p.NB - 1) + p.NB - 2 - x.n) * N * N : (p.dsT != nullptr ? p.dsT + bh * N * N : nullptr);
+    const float* const dsT = x.first + nch < all ? p.enter + (static_cast<size_t>(blockIdx.x) * (p.NB - 1) + p.NB - 2 - x.n) * N * N : first_state(p, p.dsT, bh);
     if (w < 4) bwd_role_a(S, sb, p, dsT, p.ds0 != nullptr && x.n == 0 ? p.ds0 + bh * N * N : nullptr, again(), w, nch, tok0, p.H, h);
     else bwd_role_b(S, sb, p, dsT, p.s + (bh * all + x.first) * N * N, tid, w, nch, tok0, p.H, h);
 }

@@ -253,6 +253,27 @@ def test_rwkv7_heads_beyond_a_multiple_of_the_cus(lib, B, H, T, forward, backwar
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,T", [(1, 257, 768), (1, 3, 1024), (2, 64, 4096)])
+def test_rwkv7_states_in_place(lib, B, H, T, dtype):
+    """sT in the memory of s0, ds0 in that of dsT: the bits of separate tensors, also where another block of the head writes what one reads."""
+    n, f32 = [lib.rwkv7_workspace_bytes(B, T, H, i) for i in (0, 1)], int(dtype == torch.float32)
+    assert min(n) > 0
+    s0, x, dy, dsT = _rwkv7(B, T, H, dtype, H)
+    s0, dy, dsT, x = s0.to(DEV), dy.to(DEV), dsT.to(DEV), [t.to(DEV) for t in x]
+    res = []
+    for place in (False, True):
+        a, b = s0.clone(), dsT.clone()
+        sT, ds0 = (a, b) if place else (garbage(a.shape, torch.float32), garbage(b.shape, torch.float32))
+        y, s, sa = garbage((B, T, H * 64), dtype), garbage((B, H, T // 16, 64, 64), torch.float32), garbage((B, T, H, 64), torch.float32)
+        call("rwkv7_forward_ws", y.device, B, T, H, f32, a, *x, y, sT, s, sa, garbage((n[0],), torch.uint8), n[0])
+        d = [garbage((B, T, H * 64), dtype) for _ in range(6)]
+        call("rwkv7_backward_ws", y.device, B, T, H, f32, *x, dy, b, s, sa, ds0, *d, garbage((n[1],), torch.uint8), n[1])
+        res.append([y, sT, s, sa, ds0] + d)
+    same = [torch.equal(g, z) for g, z in zip(*res)]
+    assert all(same), same
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("which", ["a", "k"])
 def test_rwkv7_heads_that_blocks_cannot_carry_are_done_as_a_whole(lib, which, dtype):
     """A NaN among the inputs, and a transition that overflows over a block where the state itself is zero: the bits of a call without a
