@@ -382,9 +382,9 @@ int rwkv_wkv6f_backward_saved(void* stream, int B, int T, int C, int H,
  * stands in for every token's decay in the kernels of rwkv_wkv6f_*, and its gradient is added up over the tokens inside
  * the kernel.  Head size 128: one workgroup holds a whole head; the forward may go without `saved` (nothing is kept then),
  * and the backward needs no more workspace than 4 B C bytes (a multiple of 32 above).  With rwkv_wkv5s_blocks_workspace_bytes (0: no use
- * for it) few long sequences (B H <= 128, or that many beyond a multiple of 256) are cut into blocks of time that are worked on side by side, in
- * the forward by _forward_ws;
- * RWKV_FLAG_WHOLE keeps them whole.  Heads with a decay below e^-9 a step, or one that is no number,
+ * for it) few long sequences (B H <= 128) are cut into blocks of time that are worked on side by side, in the forward by _forward_ws, and so are
+ * those beyond a multiple of 256, up to 128 in the backward and up to 32 in the forward (a workspace that is too small is not used there; with
+ * B H < 256 the forward takes it for an error).  Their results differ from whole sequences' by rounding; RWKV_FLAG_WHOLE keeps all whole.  Heads with a decay below e^-9 a step, or one that is no number,
  * run step by step, at both sizes.  `saved`: 64 KB (size 64: 16 KB, for any layer) per head and 64 tokens, 1.07 GB at B8 T4096
  * C4096 (268 MB at C2048).  Other head sizes, RWKV_FLAG_SWEEPS / RWKV_PASS_* or (size 64)
  * saved = NULL: rwkv_wkv5raw_forward / _backward. */

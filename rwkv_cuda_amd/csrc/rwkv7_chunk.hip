@@ -428,8 +428,9 @@ template <bool F32, bool KEEP> DEVINL void fwd_role_s(SmemCF& S, const lds_t sb,
 // What bounds it: issue and, with KEEP, the writes (half of the states, and it takes 310 us instead of 332; fp32 mode 324 of 372).
 // B8 T1024 C4096, one call, bf16: 398 us with every product on the fp32 matrix instructions, in four waves that did
 // everything in turn between four barriers; 390 in two roles of four waves; 335 with split products but for the tiles, whose 16 fp32
-// instructions a P wave held the vector unit for 512 cycles and took four more planes, twice the exponentials.  That form and this one in
-// alternation on one machine: bf16 355 -> 331 us, 268 -> 241 without KEEP; fp32 mode 386 -> 368, 306 -> 280.
+// instructions a P wave held the vector unit for 512 cycles and took four more planes, twice the exponentials.  That form and the present one
+// in alternation on one machine: bf16 329 -> 309 us, 273 -> 244 without KEEP; fp32 mode 377 -> 368, 310 -> 280 (2 to 4 us of that are
+// exponentials and decays that are rounded once).
 // Not kept: a ninth wave for the inverse (one workgroup a CU then: 502 us); rows asked for two chunks ahead (bf16 without KEEP 242 -> 253).
 // Errors against 64 bits, T1024, fp32 mode, with the tiles on fp32 instructions -> now, 1e-7, at w = 0.5 +- 1, 2 +- 0.5, -3 +- 0.5, -6 +- 0.5, -8 +- 0.5:
 // y 1.38 -> 0.80, 1.44 -> 0.78, 1.18 -> 0.96, 1.23 -> 1.16, 1.30 -> 1.22; sT 0.61 -> 0.55, 0.61 -> 0.56, 0.75 -> 0.69, 1.00 -> 0.96, 1.10 -> 1.04.
@@ -668,12 +669,13 @@ __global__ __launch_bounds__(256) void rwkv7c_scan(const Args7c p) {
 //                channel), scale them, scan the decay gradient and park the results; they run one phase behind the A waves.
 //   waves 8..11 ("P"): fetch the seven input rows and `sa` two chunks ahead, convert them, build the operand planes
 //                (double-buffered), the causal tiles and the inverse.  The finished gradient rows leave LDS-staged, as whole rows, through the A waves.
-// What bounds it: issue.  Over the three phases a SIMD issues 4300 to 4900 cycles of vector and 2900 of matrix instructions, which overlap by
-// a fifth, of some 9000.  B8 T1024 C4096, one call, bf16 mode / fp32 mode, us: 762 / . with fp32 matrix instructions; 626 / 765 with split
+// What bounds it: waits at the barriers, three a chunk, and issue.  Of 9400 cycles a chunk (B8 T1024 C4096, bf16 mode) a SIMD's vector unit has
+// instructions for 5400 and its matrix unit for 2300, which overlap in part: neither is full, the roles wait for each other.  One call, bf16
+// mode / fp32 mode, us: 762 / . with fp32 matrix instructions; 626 / 765 with split
 // products but for the tiles, 11800 cycles a chunk, 5200 of them phase 3, where wave 0 of role A made a tile, an fp32 one and the inverse;
 // 606 / 708 with inputs split once, the tiles with the P waves a phase earlier and what role B waited for with role A; 588 / 642 with one
-// gradient state instead of two and the values that finish a chunk worked out in the phases before, in which role B waited.  First and last
-// form in alternation on one machine.
+// gradient state instead of two and the values that finish a chunk worked out in the phases before, in which role B waited; 564 / 634 now,
+// with planes and an inverse that take fewer cycles; 4 us of that in either mode are exponentials and decays that are rounded once.
 // Errors against 64 bits, T1024, fp32 mode, with the tiles on fp32 instructions -> now, 1e-7, at w = 0.5 +- 1, 2 +- 0.5, -3 +- 0.5, -6 +- 0.5, -8 +- 0.5:
 // ds0 0.82 -> 0.76, 0.84 -> 0.80, 0.82 -> 0.75, 1.05 -> 1.02, 1.15 -> 1.09;
 // dr 1.12 -> 0.90, 1.21 -> 0.88, 1.00 -> 0.97, 1.18 -> 1.14, 1.26 -> 1.20;
@@ -732,7 +734,7 @@ DEVINL LaneB moved(const LaneB& b, lds_t d) {
 // v, dy: four tokens of a channel, and over channels
 template <bool F32> DEVINL auto exact_piece(lds_t a) { if constexpr (F32) return get3(a); else return lds_ld<u32x2>(a); }
 template <bool F32> DEVINL auto exact_tr(uint32_t plane, const Tr& o, int hb) { if constexpr (F32) return get3_tr(plane, o, hb); else return ld_tr16(o, plane, hb); }
-// causal_acc from three-term planes (or, not three, exact ones): rows of the result from a, columns from b; transposed: tokens s along
+// causal_tile with planes chosen at run time, of three terms (or, not three, exact ones): rows of the result from a, columns from b; transposed: tokens s along
 // the rows.  All but the planes' addresses is uniform: the waves that make different tiles share the code.
 DEVINL f32x4 causal_split(const Tr& o, lds_t a, bool a3, lds_t b, bool b3, bool transposed, bool strict, int l16, int g) {
     Sum2 sum = SUM0;
@@ -762,13 +764,19 @@ DEVINL f32x4 causal_split(const Tr& o, lds_t a, bool a3, lds_t b, bool b3, bool 
     return acc;
 }
 
-// Per visit i (chunks in descending order) every wave passes three barriers; role B trails role A by one phase, so that
-// both always have matrix work in the same phase:
-//          phase 1                          | phase 2                                   | phase 3
-//   A:     state parts of dU, dV of (i)      | dU, dW, dV, state update of (i)           | dAB, dAK of (i), both ways; tile, M of (i + 1)
-//   B:     other tile parts, rest of (i - 1) | dY S0, U dS, V dS, dRB, dRK of (i)        | dW S0, state update, dr of (i)
-//   P:     decay sums, U, v, dy (i + 1)      | AR, BK, ES (i + 1)                        | RAW, DWF (i + 1)
-// (the rows of visit i - 1 leave through the A waves)
+// Per visit i (chunks in descending order) every wave passes three barriers; role B finishes a visit in the next one's phase 1, so that all
+// roles always have matrix work in the same phase.  What they do, and what of LDS they read (<) and write (>) between two barriers; (i): the
+// copy of visit i of what has two:
+//     phase 1   A   B E^T, K E^T of i                                                < BK (i), dec (i)                       > DS
+//               B   dA, dB, dK and what is left of i - 1                             < A_ROWS, B_COLS, K_COLS, DWF (i - 1)   > park
+//               P   planes of i + 1                                                  < part                                  > AR, BK, U, V, DY, dec (i + 1)
+//     phase 2   A   dU, dW, dV, the state of i; the tiles dRB, dRK of i to LDS       < MB, AKR, AR, DY, V (i), dec (i)       > DW, R_ROWS, B_COLS and K_COLS (dRB, dRK), parkv (i)
+//               B   dY S0, U E, V E of i; AR, BK of i into registers                 < DS, AR, BK, U, V, DY (i)
+//               P   the causal tiles of i + 1; factors; decays of i + 2              < AR, BK (i + 1)                        > ES, DWF (i + 1), part
+//     phase 3   A   dAB, dAK of i, dRB, dRK of i + 1; rows of i - 1 to memory        < DW, U, V (i), DY, U, V (i + 1), park, parkv (i - 1)   > A_ROWS, B_COLS and K_COLS (dAB, dAK)
+//               B   dW S0, dR of i; the state entering the next chunk asked for      < DW, R_ROWS, ES (i)
+//               P   the inverse and the tiles of i + 1 to LDS; rows of i + 4 asked for                                       > AB, MB, AKR
+// (In visit 0 role B has P at the end of the call to make in phase 1, from U, V, BK and dec of visit 0.)
 
 // ---- role P: elementwise preparation (lane = channel, tokens 4 wp + e) one visit ahead, and the row-wise output stores
 struct Prep7 { uint32_t nx[7][4]; float nsa[4]; };
@@ -1170,7 +1178,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             Pj = pp;
         }
         __syncthreads();
-        // ---------------------------------------------------------------- phase 2: dY S0, U dS, V dS; dRB (q even), dRK, by rows and by columns
+        // ---------------------------------------------------------------- phase 2: dY S0, U E, V E
         auto dy_of = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::DY, two.tr, hb); };
         auto u_of = [&](int hb) __attribute__((always_inline)) { return get3_tr(L::U, two.tr, hb); };
         auto v_of = [&](int hb) __attribute__((always_inline)) { return exact_tr<F32>(L::V, two.tr, hb); };
@@ -1193,7 +1201,7 @@ template <bool F32> DEVINL void bwd_role_b(SmemCB<F32>& S, const lds_t sb, const
             xR = total(pr); xB = total(pb); xK = total(pk);
         }
         __syncthreads();
-        // ---------------------------------------------------------------- phase 3: dW S0; the gradient state
+        // ---------------------------------------------------------------- phase 3: dW S0, dR
         {
             const uint32_t me = lane_again();
             er = lds_ld<f32x4>(sb + copy_of(i) + L::ES + piece2(16 * q + (me & 15), me >> 4));
